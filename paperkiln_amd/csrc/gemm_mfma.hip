@@ -1047,10 +1047,13 @@ void run_plan(const Plan& p, bool tA, bool tB, const GemmArgs& ga, int splits, b
                 launch_geo<GeoSmall>(tA, tB, ga, splits, f32, st);
     }
 }
-bool takes(const void* a, bool tA, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K) {
+bool takes(const void* a, bool tA, int64_t lda, const void* b, bool tB, int64_t ldb, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > (1 << 30) || N > (1 << 30) || K > (1 << 30)) return false;
     if (!aligned16(a) || !aligned16(b)) return false;
-    if (lda % 8 || ldb % 8 || K % 8 || N % 8) return false;
+    if (lda % 8 || ldb % 8 || N % 8) return false;
+    // a contraction that runs along a row of either operand is read in 16-byte chunks; where it is the row index of both
+    // (a weight gradient over the tokens) rows past its end read as zeros and any length goes
+    if (K % 8 && (!tA || tB)) return false;
     if (tA && M % 8) return false;  // A^T is read in 16-byte chunks along M
     return true;
 }
@@ -1075,7 +1078,7 @@ GemmArgs gemm_args(const void* a, int64_t lda, const void* b, int64_t ldb, int64
 // that are not multiples of 8): the caller then uses the library GEMM.
 bool gemm_mfma_bf16(const void* a, bool tA, int64_t lda, const void* b, bool tB, int64_t ldb, void* c, int c_dtype,
                     int64_t M, int64_t N, int64_t K, int64_t ldc, float beta, hipStream_t st, const void* addend) {
-    if (!takes(a, tA, lda, b, ldb, M, N, K) || !aligned16(c) || ldc % 8) return false;
+    if (!takes(a, tA, lda, b, tB, ldb, M, N, K) || !aligned16(c) || ldc % 8) return false;
     if (beta != 0.0f && beta != 1.0f) return false;
     GemmArgs g = gemm_args(a, lda, b, ldb, M, N, K);
     g.c = c;
@@ -1110,7 +1113,7 @@ bool gemm_mfma_bf16(const void* a, bool tA, int64_t lda, const void* b, bool tB,
 // cut), for a caller that adds them itself on the way to where the result goes.
 bool gemm_mfma_bf16_parts(const void* a, bool tA, int64_t lda, const void* b, bool tB, int64_t ldb, int64_t M, int64_t N,
                           int64_t K, hipStream_t st, std::unique_ptr<Buffer>& part, int& nparts) {
-    if (!takes(a, tA, lda, b, ldb, M, N, K)) return false;
+    if (!takes(a, tA, lda, b, tB, ldb, M, N, K)) return false;
     const Plan p = make_plan(tA, tB, M, N, K, lda, ldb, N);
     part.reset(new Buffer(sizeof(float) * static_cast<size_t>(p.S) * M * N));
     GemmArgs g = gemm_args(a, lda, b, ldb, M, N, K);
@@ -1125,7 +1128,7 @@ bool gemm_mfma_bf16_parts(const void* a, bool tA, int64_t lda, const void* b, bo
 // ---- the tied head's cross-entropy inside its logits product ----
 namespace {
 bool head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K) {
-    if (!takes(a, false, lda, b, ldb, M, N, K)) return false;
+    if (!takes(a, false, lda, b, true, ldb, M, N, K)) return false;
     const int64_t ext_max = (int64_t{1} << 30) - 8192;
     return M * lda * 2 < ext_max && N * ldb * 2 < ext_max && lda < (1 << 21) && ldb < (1 << 21) && N < (1 << 20);
 }
@@ -1200,7 +1203,7 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
     const int64_t ext_max = (int64_t{1} << 30) - 8192;
     for (int p = 0; p < count; ++p) {
         const GroupedProduct& q = ps[p];
-        if (!takes(q.a, true, q.lda, q.b, q.ldb, q.M, q.N, K) || !aligned16(q.c) || q.ldc % 4) return false;
+        if (!takes(q.a, true, q.lda, q.b, false, q.ldb, q.M, q.N, K) || !aligned16(q.c) || q.ldc % 4) return false;
         if (K * q.lda * 2 >= ext_max || K * q.ldb * 2 >= ext_max || q.lda >= (1 << 21) || q.ldb >= (1 << 21) || q.ldc >= (1 << 20))
             return false;
         gr.a[p] = static_cast<const uint16_t*>(q.a);
