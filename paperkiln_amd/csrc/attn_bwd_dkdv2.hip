@@ -412,8 +412,9 @@ int launch_geo(const AttnArgs& a_in, hipStream_t st) {
         PK_HIP(hipGetLastError());
         return launch_sink_tail_reduce(a, st);
     }
-    hipLaunchKernelGGL((mfma_dkdv2<D, GF32, false, BNK, BMQ>), dim3(xcd_grid(paired ? (nkb + 1) / 2 : nkb, 1, a.Hkv * a.B)),
-                       dim3(4 * BNK), 0, st, a);
+    const int ids = a.window > 0 && a.sinks > 0 && nkb > 1 ? xcd_grid_block0_first(nkb, a.Hkv * a.B)
+                                                           : xcd_grid(paired ? (nkb + 1) / 2 : nkb, 1, a.Hkv * a.B);
+    hipLaunchKernelGGL((mfma_dkdv2<D, GF32, false, BNK, BMQ>), dim3(ids), dim3(4 * BNK), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }

@@ -113,11 +113,7 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
     // [hfirst, hfirst + nh) of the group and leaves fp32 partial sums for launch_gqa_reduce
     const int hs = a.head_split;
     int blk, rr = 0, kvu;
-    if (a.window > 0 && a.sinks > 0 && nkb > 1) {
-        if (!xcd_map_block0_first(nkb, a.Hkv * a.B, blk, kvu)) return;
-    } else if (!xcd_map(paired ? (nkb + 1) / 2 : nkb, hs, a.Hkv * a.B, blk, rr, kvu)) {
-        return;
-    }
+    if (!xcd_map(paired ? (nkb + 1) / 2 : nkb, hs, a.Hkv * a.B, blk, rr, kvu)) return;
     const int hfirst = rr * rep / hs, nh = (rr + 1) * rep / hs - hfirst;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv;
     const float cexp = a.scale * LOG2E;

@@ -264,17 +264,34 @@ __device__ inline u32x4 dma_rsrc(const void* p, uint32_t bytes) {
 // are given ids that are congruent mod 8: one unit's tensors then live in ONE
 // L2 instead of being fetched into all eight.
 // Launch with grid.x = xcd_grid(nblk, rep, kv_units).
+//
+// Only whole multiples of 8 units divide that way. The kv_units % 8 units left over are dealt block by block over all
+// XCDs instead, ahead of the others (each L2 then fetches their K/V for itself): kept whole, one XCD would have a unit
+// more than the next -- and fewer than 8 units in all would leave the other XCDs idle (one head of 4096 tokens, bf16,
+// head_dim 64, ran its 32 query blocks on the 32 CUs of one XCD; 5 units kept 3 of 8 XCDs idle).
+__host__ __device__ inline int xcd_loose_ids(int nblk, int rep, int kv_units) {  // ids per XCD for the units left over
+    return ((kv_units & 7) * rep * nblk + 7) / 8;
+}
 __host__ __device__ inline int xcd_grid(int nblk, int rep, int kv_units) {
-    return nblk * rep * ((kv_units + 7) / 8) * 8;
+    return (nblk * rep * (kv_units / 8) + xcd_loose_ids(nblk, rep, kv_units)) * 8;
+}
+// The idx-th of the left-over units' blocks, block 0 of every unit and head first; false past their end.
+__device__ inline bool xcd_loose_block(int idx, int nblk, int rep, int kv_units, int& blk, int& r, int& kvu) {
+    const int heads = (kv_units & 7) * rep;
+    blk = idx / heads;
+    r = (idx % heads) % rep;
+    kvu = (kv_units & ~7) + (idx % heads) / rep;
+    return blk < nblk;
 }
 // blk: block index inside the unit (0 = dispatched first); r: query head inside
 // the GQA group; kvu: (batch, KV head) unit. Returns false for padding ids.
 __device__ inline bool xcd_map(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu) {
-    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int xcd = blockIdx.x & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = static_cast<int>(blockIdx.x >> 3) - loose;
+    if (j < 0) return xcd_loose_block((j + loose) * 8 + xcd, nblk, rep, kv_units, blk, r, kvu);
     blk = j % nblk;
     r = (j / nblk) % rep;
     kvu = (j / (nblk * rep)) * 8 + xcd;
-    return kvu < kv_units;
+    return true;
 }
 // The same ids in block-major order: block 0 of every unit and head of an XCD's share first, then every block 1, ...
 // For causal blocks that are NOT paired, block 0 is the heaviest and the work falls linearly with the index, so this
@@ -282,29 +299,47 @@ __device__ inline bool xcd_map(int nblk, int rep, int kv_units, int& blk, int& r
 // the unit-major order above the last units' heavy blocks start late and stretch the tail of the launch
 // (512 unpaired workgroups of 256 queries at B x H = 32, T = 4096 took 232 us against 208 for the smaller kernel).
 __device__ inline bool xcd_map_block_major(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu) {
-    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int per = ((kv_units + 7) / 8) * rep;  // (unit, head) pairs of one XCD
+    const int xcd = blockIdx.x & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = static_cast<int>(blockIdx.x >> 3) - loose;
+    if (j < 0) return xcd_loose_block((j + loose) * 8 + xcd, nblk, rep, kv_units, blk, r, kvu);
+    const int per = (kv_units / 8) * rep;  // (unit, head) pairs of one XCD
     blk = j / per;
     r = (j % per) % rep;
     kvu = ((j % per) / rep) * 8 + xcd;
-    return kvu < kv_units;
+    return true;
 }
 
 // The same mapping with block 0 of EVERY unit dispatched before any other block (rep = 1). With a
 // band mask plus sink keys the workgroup that owns key block 0 walks all query tiles while the others
 // walk a handful; started last it is the tail of the launch, started first it runs beside them.
+// Launch with grid.x = xcd_grid_block0_first(nblk, kv_units).
+__host__ __device__ inline int xcd_grid_block0_first(int nblk, int kv_units) {
+    return (nblk * (kv_units / 8) + ((kv_units & 7) != 0) + ((kv_units & 7) * (nblk - 1) + 7) / 8) * 8;
+}
 __device__ inline bool xcd_map_block0_first(int nblk, int kv_units, int& blk, int& kvu) {
-    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int upx = (kv_units + 7) / 8;  // units per XCD
-    if (j < upx) {
-        blk = 0;
-        kvu = j * 8 + xcd;
-    } else {
-        const int jj = j - upx;
-        blk = 1 + jj % (nblk - 1);
-        kvu = (jj / (nblk - 1)) * 8 + xcd;
+    const int xcd = blockIdx.x & 7, upx = kv_units / 8, left = kv_units & 7;  // whole units per XCD, units left over
+    int j = static_cast<int>(blockIdx.x >> 3);
+    blk = 0;
+    if (left != 0 && j-- == 0) {  // block 0 of the left-over units, one per XCD
+        kvu = (kv_units & ~7) + xcd;
+        return xcd < left;
     }
-    return kvu < kv_units;
+    if (j < upx) {
+        kvu = j * 8 + xcd;
+        return true;
+    }
+    j -= upx;
+    const int loose = (left * (nblk - 1) + 7) / 8;
+    if (j < loose) {
+        const int idx = j * 8 + xcd;
+        if (idx >= left * (nblk - 1)) return false;
+        blk = 1 + idx / left;
+        kvu = (kv_units & ~7) + idx % left;
+        return true;
+    }
+    j -= loose;
+    blk = 1 + j % (nblk - 1);
+    kvu = (j / (nblk - 1)) * 8 + xcd;
+    return true;
 }
 
 // Full-causal work per 128-row block grows linearly with its index, so the forward and dQ kernels
