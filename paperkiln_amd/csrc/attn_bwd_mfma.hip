@@ -269,52 +269,57 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_dq(AttnArgs a) {
 }
 
 template <int D, bool GF32>
-int launch(const AttnArgs& a, int stages, hipStream_t st) {
-    const int64_t rows = static_cast<int64_t>(a.B) * a.Hq * a.T;
-    constexpr int RPB = 256 / (D / 8);
+int launch_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
     // dQ with 8 wavefronts (256 queries) per K/V tile where the paired causal grid still gives every CU two
     // workgroups in turn, as in the forward kernel; 4 wavefronts otherwise.
     const int nb256 = (a.T + 255) / 256;
     const bool wide = D == 128 && a.causal && a.window == 0 && static_cast<int64_t>((nb256 + 1) / 2) * a.Hq * a.B >= 512;
     const int nbq = wide ? nb256 : (a.T + 127) / 128;
     const bool paired = pair_causal_blocks(nbq, a.Hq * a.B, a.causal, a.window);
-    const dim3 dq_grid(xcd_grid(paired ? (nbq + 1) / 2 : nbq, a.Hq / a.Hkv, a.Hkv * a.B));
-    // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote
-    const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
-    const bool dq3 = mfma_dq3_takes(a);  // 64 queries per wavefront, one wavefront per SIMD
-    if (fused) {
-        if (dq3) {
-            if (int rc = launch_mfma_dq3(a, true, st)) return rc;
-        } else if (wide)
-            hipLaunchKernelGGL((mfma_dq<D, GF32, true, 8>), dq_grid, dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL((mfma_dq<D, GF32, true, 4>), dq_grid, dim3(256), 0, st, a);
-        PK_HIP(hipGetLastError());
-    } else if (stages & PK_BWD_DELTA) {
-        hipLaunchKernelGGL((mfma_delta<D>), dim3((rows + RPB - 1) / RPB), dim3(256), 0, st, a);
-        PK_HIP(hipGetLastError());
-    }
-    if (stages & PK_BWD_DKDV) {
-        // without a band: 64 keys per wavefront, one wavefront per SIMD; with one: 32 keys, two per SIMD
-        if (int rc = mfma_dkdv3_takes(a) ? launch_mfma_dkdv3(a, st) : launch_mfma_dkdv2(a, st)) return rc;
-    }
-    if (!fused && (stages & PK_BWD_DQ)) {
-        if (dq3) {
-            if (int rc = launch_mfma_dq3(a, false, st)) return rc;
-        } else if (wide)
-            hipLaunchKernelGGL((mfma_dq<D, GF32, false, 8>), dq_grid, dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL((mfma_dq<D, GF32, false, 4>), dq_grid, dim3(256), 0, st, a);
-        PK_HIP(hipGetLastError());
-    }
+    const dim3 grid(xcd_grid(paired ? (nbq + 1) / 2 : nbq, a.Hq / a.Hkv, a.Hkv * a.B));
+    if (wide && fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, true, 8>), grid, dim3(512), 0, st, a);
+    if (wide && !fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, false, 8>), grid, dim3(512), 0, st, a);
+    if (!wide && fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, true, 4>), grid, dim3(256), 0, st, a);
+    if (!wide && !fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, false, 4>), grid, dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
     return PK_OK;
+}
+template <int D>
+int launch_delta(const AttnArgs& a, hipStream_t st) {
+    constexpr int RPB = 256 / (D / 8);
+    const int64_t rows = static_cast<int64_t>(a.B) * a.Hq * a.T;
+    hipLaunchKernelGGL((mfma_delta<D>), dim3((rows + RPB - 1) / RPB), dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+// Which dQ kernel: wavefronts that split the keys for small launches and for head sizes other than 64 and 128, 64
+// queries per wavefront (one wavefront per SIMD) for long sequences, 32 otherwise.
+int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    if (split_takes_dq(a)) return launch_split_dq(a, fuse_delta, st);
+    if (mfma_dq3_takes(a)) return launch_mfma_dq3(a, fuse_delta, st);
+    if (a.dk_dim == 128) return a.grad_f32 ? launch_dq<128, true>(a, fuse_delta, st) : launch_dq<128, false>(a, fuse_delta, st);
+    return a.grad_f32 ? launch_dq<64, true>(a, fuse_delta, st) : launch_dq<64, false>(a, fuse_delta, st);
 }
 
 }  // namespace
 
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
-    if (a.dk_dim == 128) return a.grad_f32 ? launch<128, true>(a, stages, st) : launch<128, false>(a, stages, st);
-    return a.grad_f32 ? launch<64, true>(a, stages, st) : launch<64, false>(a, stages, st);
+    // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote
+    const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
+    int rc = PK_OK;
+    if (fused)
+        rc = run_dq(a, true, st);
+    else if (stages & PK_BWD_DELTA)
+        rc = a.dk_dim == 128 ? launch_delta<128>(a, st) : a.dk_dim == 64 ? launch_delta<64>(a, st)
+                                                                        : launch_generic_bwd(a, true, PK_BWD_DELTA, st);
+    if (rc) return rc;
+    if (stages & PK_BWD_DKDV) {
+        // split queries as above; without a band: 64 keys per wavefront, one wavefront per SIMD; with one: 32 keys, two
+        // per SIMD
+        rc = split_takes_dkdv(a) ? launch_split_dkdv(a, st) : mfma_dkdv3_takes(a) ? launch_mfma_dkdv3(a, st) : launch_mfma_dkdv2(a, st);
+        if (rc) return rc;
+    }
+    return !fused && (stages & PK_BWD_DQ) ? run_dq(a, false, st) : PK_OK;
 }
 
 }  // namespace pk

@@ -375,10 +375,7 @@ bool aligned16(const void* p, int64_t sb, int64_t st, int64_t sh) {
 
 }  // namespace
 
-// The MFMA kernels take bf16 storage, head_dim 64 or 128, a positive scale
-// (the running max is tracked on raw scores) and 16-byte-aligned rows.
-bool mfma_supported(const AttnArgs& a) {
-    if (a.dk_dim != 64 && a.dk_dim != 128) return false;
+bool bf16_rows_aligned(const AttnArgs& a) {
     if (!(a.scale > 0.0f)) return false;
     if (!aligned16(a.q, a.q_sb, a.q_st, a.q_sh) || !aligned16(a.k, a.k_sb, a.k_st, a.k_sh) ||
         !aligned16(a.v, a.v_sb, a.v_st, a.v_sh) || !aligned16(a.o, a.o_sb, a.o_st, a.o_sh))

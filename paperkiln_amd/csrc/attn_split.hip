@@ -1,0 +1,739 @@
+// bf16 attention (forward, dQ, dK/dV) in workgroups whose wavefronts share the CONTRACTION: KW groups of wavefronts take
+// every KW-th tile of the keys (of the queries for dK/dV) of one block of rows, and their partial results meet in LDS at
+// the end. Mathematics and operand layouts are those of attn_fwd_mfma.hip / attn_bwd_mfma.hip.
+//
+// What bounds it: the other bf16 kernels give a workgroup 128 or 256 rows and let it walk every visible tile alone. With
+// few (batch, head) units or short sequences that is a handful of workgroups on 256 CUs, each a serial chain of tiles of
+// about half a microsecond. Here a block is 32 rows and four wavefronts split its tiles: four times the workgroups, a
+// quarter of the chain, and a sequence of 128 tokens is one tile per wavefront -- one round trip to memory.
+//
+// The same kernels, with wavefronts that own different rows and share the tiles (QW = 4, KW = 1), are the path of every
+// head size that is a multiple of 8 up to 128 but not 64 or 128 (D is the size rounded up to 32; chunks past the real
+// size read as zero and are not stored). P and dS enter their products there as TWO bf16 operands, the rounded value
+// and the remainder (EXACT: 16 significant bits, against 8 in the kernels of head_dim 64 and 128), because these sizes
+// used to run in fp32 arithmetic throughout.
+#include "mfma_common.h"
+#include "pk_internal.h"
+
+namespace pk {
+namespace {
+
+constexpr float LOG2E = 1.4426950408889634f;
+
+// A tile of ROWS rows of a [T, dk] bf16 matrix, moved by G threads: thread t of the group carries the 16-byte chunks
+// t, t + G, ... Rows past T and chunks past dk read as zero.
+template <int D, int G, int ROWS>
+struct Mover {
+    static constexpr int NCH = D / 8, CPT = ROWS * NCH / G;
+    static_assert(CPT >= 1 && ROWS * NCH % G == 0, "every thread moves the same number of chunks");
+    int off[CPT];  // byte offsets inside a tile
+    u32x4 r[CPT];
+    __device__ void init(int t, int64_t st, int dk) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int c = t + G * i, row = c / NCH, ch = c % NCH;
+            off[i] = ch * 8 < dk ? static_cast<int>(row * st + ch * 8) * 2 : static_cast<int>(OUTSIDE);
+        }
+    }
+    __device__ void load(const void* base, int64_t elem_off, int64_t st, int r0, int T, int dk) {
+        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(base, elem_off, st, r0, T, dk);
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) r[i] = tile_load16(rs, off[i]);
+    }
+    __device__ void store(uint16_t* lds, int pitch, int t) const {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int c = t + G * i;
+            *reinterpret_cast<u32x4*>(lds + (c / NCH) * pitch + (c % NCH) * 8) = r[i];
+        }
+    }
+};
+
+// Row `row` of a head as an operand held in registers: chunk kk covers d = 16kk + 8g .. +7; zero past T and past dk.
+template <int D>
+__device__ inline void load_row(const void* base, int64_t off, int64_t st, int row, int T, int dk, int g, bf16x8* out) {
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+        u32x4 z = {0, 0, 0, 0};
+        const int col = kk * 16 + g * 8;
+        if (row < T && col < dk)
+            z = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + off + row * st + col);
+        out[kk] = *reinterpret_cast<bf16x8*>(&z);
+    }
+}
+
+// Elements 8H .. 8H+7 of a C tile as a bf16 k-chunk and what its rounding left over
+template <int H>
+__device__ inline void split_operand(const f32x16& c, bf16x8& hi, bf16x8& lo) {
+    u32x4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x0 = c[8 * H + 2 * i], x1 = c[8 * H + 2 * i + 1];
+        h[i] = pack_bf16(x0, x1);
+        l[i] = pack_bf16(x0 - __uint_as_float(h[i] << 16), x1 - __uint_as_float(h[i] & 0xffff0000u));
+    }
+    hi = *reinterpret_cast<bf16x8*>(&h);
+    lo = *reinterpret_cast<bf16x8*>(&l);
+}
+
+// acc[db] += M^T c for the 32 rows of an LDS tile that start at row0, M the tile (columns 32 db ..), c a C tile whose rows
+// are the tile's rows
+template <int D, bool EXACT>
+__device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, const f32x16& c, f32x16* acc, int lane) {
+    constexpr int DB = D / 32;
+    bf16x8 h0, l0, h1, l1;
+    if (EXACT) {
+        split_operand<0>(c, h0, l0);
+        split_operand<1>(c, h1, l1);
+    } else {
+        h0 = c_to_operand<0>(c);
+        h1 = c_to_operand<1>(c);
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        const bf16x8 m = lds_read_tr_operand(tile, pitch, row0, db * 32, lane);
+        acc[db] = mfma32(m, h0, acc[db]);
+        if (EXACT) acc[db] = mfma32(m, l0, acc[db]);
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        const bf16x8 m = lds_read_tr_operand(tile, pitch, row0 + 16, db * 32, lane);
+        acc[db] = mfma32(m, h1, acc[db]);
+        if (EXACT) acc[db] = mfma32(m, l1, acc[db]);
+    }
+}
+
+// The KW groups' accumulators of N blocks added up: group kg ends up with the sums of blocks kg, kg + KW, ... (in group
+// order, so repeatable). `red` is LDS for KW N KB per row group, free to overwrite when this is called.
+template <int N, int KW>
+__device__ inline void join_groups(f32x16* acc, float* red, int kg, int lane) {
+    if (KW == 1) return;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        if (n % KW == kg) continue;
+        f32x4* p = reinterpret_cast<f32x4*>(red) + ((kg * N + n) * 4) * 64 + lane;
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+            const f32x4 v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
+            p[qd * 64] = v;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        if (n % KW != kg) continue;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const f32x4* p = reinterpret_cast<const f32x4*>(red) + ((k * N + n) * 4) * 64 + lane;
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                f32x4 v;
+                if (k == n % KW)
+                    v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
+                else
+                    v = p[qd * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[qd * 4 + e] += v[e];
+            }
+        }
+        acc[n] = s;
+    }
+}
+
+// One 32 x 32 accumulator block (lane = row of the output, natural column order) scaled and written; columns past dk are
+// not. Both lanes of a pair (c, c + 32) hold the same row and must be active.
+__device__ inline void store_block(bool f32, void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
+    if (f32) {
+        float* row = static_cast<float*>(base) + row_off;
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+            const int col = 32 * db + 8 * qd + 4 * g;
+            const f32x4 v = {acc[qd * 4] * sc, acc[qd * 4 + 1] * sc, acc[qd * 4 + 2] * sc, acc[qd * 4 + 3] * sc};
+            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = v;
+        }
+    } else {
+        uint16_t* row = static_cast<uint16_t*>(base) + row_off;
+#pragma unroll
+        for (int qp = 0; qp < 2; ++qp) {
+            const int lo = qp * 8, hi = qp * 8 + 4;
+            const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo] * sc, acc[lo + 1] * sc),
+                                                             pack_bf16(acc[hi] * sc, acc[hi + 1] * sc), false, false);
+            const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo + 2] * sc, acc[lo + 3] * sc),
+                                                             pack_bf16(acc[hi + 2] * sc, acc[hi + 3] * sc), false, false);
+            const u32x4 v = {r0[0], r1[0], r0[1], r1[1]};
+            const int col = 32 * db + 8 * (2 * qp + g);
+            if (col < dk) *reinterpret_cast<u32x4*>(row + col) = v;
+        }
+    }
+}
+
+// A group of several wavefronts has two tile buffers and one barrier per tile; a group of one wavefront has one buffer and
+// none: a wavefront's LDS operations complete in order, so it overwrites its tile behind its own last read of it.
+template <int QW>
+__device__ inline void tile_barrier() {
+    if (QW > 1)
+        __syncthreads();
+    else
+        __builtin_amdgcn_wave_barrier();
+}
+
+// The tiles of BN keys that queries [q0, q0 + BM) can see, as a list: sink tiles [0, ns), then [lo, hi].
+struct KeyTiles {
+    int ns, lo, n;
+    __device__ KeyTiles(const AttnArgs& a, int q0, int BM, int BN) {
+        const int qmax = min(q0 + BM, a.T) - 1;
+        const int hi = (a.causal ? qmax : a.T - 1) / BN;
+        lo = a.window > 0 ? max(0, q0 + 1 - a.window) / BN : 0;
+        ns = a.window > 0 ? min((a.sinks + BN - 1) / BN, lo) : 0;
+        n = ns + hi - lo + 1;
+    }
+    __device__ int tile(int i) const { return i < ns ? i : lo + i - ns; }
+};
+
+__device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk) {
+    const int rep = a.Hq / a.Hkv;
+    int blk, rr, kvu;
+    // causal blocks without a band: the heaviest blocks of every unit first
+    if (a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
+                                  : !xcd_map(nqb, rep, a.Hkv * a.B, blk, rr, kvu))
+        return false;
+    hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    qblk = nqb - 1 - blk;
+    return true;
+}
+
+// ---- forward: QW groups of 32 queries x KW groups of key tiles of 32 NB keys ----
+template <int D, int QW, int KW, int NB, bool EXACT>
+__global__ __launch_bounds__(64 * QW * KW) void split_fwd(AttnArgs a) {
+    constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW;
+    constexpr int KS = D + 8;                              // row reads conflict-free
+    constexpr int VS = (D / 32) % 2 ? D : D + 32;          // 4-row transposing reads conflict-free
+    constexpr int TILE = BN * (KS + VS), NBUF = QW > 1 ? 2 : 1;
+    constexpr int RED = KW > 1 ? QW * KW * (DB * 1024 + 128) * 2 : 0;  // in uint16
+    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    const int nqb = (a.T + BM - 1) / BM;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, nqb, b, h, hk, qblk)) return;
+    const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
+    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float cexp = a.scale * LOG2E;
+
+    Mover<D, G, BN> mk, mv;
+    mk.init(gt, a.k_st, dk);
+    mv.init(gt, a.v_st, dk);
+    const KeyTiles kt(a, q0, BM, BN);
+    const int iters = (kt.n + KW - 1) / KW;
+    auto fetch = [&](int i) {  // this group's i-th tile (past its last: nothing)
+        const int at = i * KW + kg;
+        if (at < kt.n) {
+            const int r0 = kt.tile(at) * BN;
+            mk.load(a.k, kb, a.k_st, r0, a.T, dk);
+            mv.load(a.v, vb, a.v_st, r0, a.T, dk);
+        }
+    };
+    auto commit = [&](int buf) {
+        uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
+        mk.store(t, KS, gt);
+        mv.store(t + BN * KS, VS, gt);
+    };
+    fetch(0);
+    bf16x8 qreg[KK];
+    load_row<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    f32x16 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+    float m = -1e30f, l = 0.0f;  // the reference's running-max seed, src/ops.cpp:881
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    commit(0);
+    tile_barrier<QW>();
+
+    for (int i = 0; i < iters; ++i) {
+        if (i + 1 < iters) fetch(i + 1);  // in flight during the math
+        const int at = i * KW + kg;
+        const uint16_t* Ks = lds + (i % NBUF * KW + kg) * TILE;
+        const uint16_t* Vs = Ks + BN * KS;
+        const int n0 = at < kt.n ? kt.tile(at) * BN : a.T;
+        f32x16 s[NB];
+        bool live[NB], any = false;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {  // wavefront-uniform: is anything of this 32 x 32 block visible?
+            const int k0 = n0 + nb * 32;
+            live[nb] = k0 < a.T && qlo < a.T && !(a.causal && k0 > qhi) && !(a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks);
+            any = any || live[nb];
+        }
+        if (any) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                if (!live[nb]) continue;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[nb][r] = 0.0f;
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk)
+                    s[nb] = mfma32(lds_read8(Ks + (nb * 32 + c32) * KS + kk * 16 + g * 8), qreg[kk], s[nb]);
+                const int k0 = n0 + nb * 32;
+                const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
+                if (kind != MaskKind::NONE) mask_block(s[nb], kind, vis, k0 + g * 4, -INFINITY);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[nb][r]);
+            }
+            mx = xhalf_max(mx);
+            if (__any(mx > m)) {  // wavefront-uniform
+                const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f((m - mn) * cexp);
+                l *= alpha;
+                m = mn;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+            }
+            const float mc = m * cexp;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                if (!live[nb]) continue;
+                float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[nb][r] = __builtin_amdgcn_exp2f(fmaf(s[nb][r], cexp, -mc));
+                    ps[r & 3] += s[nb][r];
+                }
+                l += (ps[0] + ps[1]) + (ps[2] + ps[3]);  // per-lane partial; the two halves meet below
+                accumulate_tr<D, EXACT>(Vs, VS, nb * 32, s[nb], acc, lane);
+            }
+        }
+        if (i + 1 < iters) commit(i + 1);  // two buffers: last read one iteration ago, before the previous barrier
+        tile_barrier<QW>();
+    }
+
+    l = xhalf_sum(l);
+    if (KW > 1) {
+        if (QW == 1) __syncthreads();  // every group has read its last tile
+        // the groups' running maxima and sums meet, then their accumulators scaled to the common maximum
+        float* red = reinterpret_cast<float*>(lds) + qg * KW * (DB * 1024 + 128);
+        float* ml = red + KW * DB * 1024;
+        ml[kg * 128 + lane] = m;
+        ml[kg * 128 + 64 + lane] = l;
+        __syncthreads();
+        float mt = m, lt = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
+#pragma unroll
+        for (int k = 0; k < KW; ++k) lt += ml[k * 128 + 64 + lane] * __builtin_amdgcn_exp2f((ml[k * 128 + lane] - mt) * cexp);
+        const float alpha = __builtin_amdgcn_exp2f((m - mt) * cexp);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        join_groups<DB, KW>(acc, red, kg, lane);
+        m = mt, l = lt;
+    }
+    if (qi < a.T) {
+        const float inv = 1.0f / l;
+        const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if (KW == 1 || db % KW == kg) store_block(false, a.o, ro, db, g, acc[db], inv, dk);
+        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = m * a.scale + logf(l);
+    }
+}
+
+// ---- dQ (and delta, when asked for with it): the same blocks ----
+template <int D, int QW, int KW, int NB, bool EXACT>
+__global__ __launch_bounds__(64 * QW * KW) void split_dq(AttnArgs a, int fuse_delta) {
+    constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
+    constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
+    constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;  // in uint16
+    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    const int nqb = (a.T + BM - 1) / BM;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, nqb, b, h, hk, qblk)) return;
+    const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
+    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float cexp = a.scale * LOG2E;
+
+    Mover<D, G, BN> mk, mv;
+    mk.init(gt, a.k_st, dk);
+    mv.init(gt, a.v_st, dk);
+    const KeyTiles kt(a, q0, BM, BN);
+    const int iters = (kt.n + KW - 1) / KW;
+    auto fetch = [&](int i) {
+        const int at = i * KW + kg;
+        if (at < kt.n) {
+            const int r0 = kt.tile(at) * BN;
+            mk.load(a.k, kb, a.k_st, r0, a.T, dk);
+            mv.load(a.v, vb, a.v_st, r0, a.T, dk);
+        }
+    };
+    auto commit = [&](int buf) {
+        uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
+        mk.store(t, S, gt);
+        mv.store(t + BN * S, S, gt);
+    };
+    fetch(0);
+    bf16x8 qreg[KK], greg[KK];
+    load_row<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    load_row<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
+    float nlse = 0.0f, dl = 0.0f;
+    if (qi < a.T) nlse = -a.lse[lrow] * LOG2E;
+    if (fuse_delta) {
+        bf16x8 oreg[KK];
+        load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, qi, a.T, dk, g, oreg);
+        float part = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+            const u32x4 ov = *reinterpret_cast<const u32x4*>(&oreg[kk]);
+            const u32x4 gv = *reinterpret_cast<const u32x4*>(&greg[kk]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                part = fmaf(__uint_as_float(ov[i] << 16), __uint_as_float(gv[i] << 16), part);
+                part = fmaf(__uint_as_float(ov[i] & 0xFFFF0000u), __uint_as_float(gv[i] & 0xFFFF0000u), part);
+            }
+        }
+        dl = xhalf_sum(part);
+        if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
+    } else if (qi < a.T) {
+        dl = a.delta[lrow];
+    }
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    f32x16 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+    commit(0);
+    tile_barrier<QW>();
+
+    for (int i = 0; i < iters; ++i) {
+        if (i + 1 < iters) fetch(i + 1);
+        const int at = i * KW + kg;
+        const uint16_t* Ks = lds + (i % NBUF * KW + kg) * TILE;
+        const uint16_t* Vs = Ks + BN * S;
+        const int n0 = at < kt.n ? kt.tile(at) * BN : a.T;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int k0 = n0 + nb * 32;
+            // wavefront-uniform: nothing of this 32 x 32 block is visible
+            if (k0 >= a.T || qlo >= a.T || (a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks))
+                continue;
+            f32x16 s, dp;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.0f;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                s = mfma32(lds_read8(Ks + (nb * 32 + c32) * S + kk * 16 + g * 8), qreg[kk], s);
+                dp = mfma32(lds_read8(Vs + (nb * 32 + c32) * S + kk * 16 + g * 8), greg[kk], dp);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dp[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * (dp[r] - dl);
+            const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
+            if (kind != MaskKind::NONE) mask_block(dp, kind, vis, k0 + g * 4, 0.0f);
+            accumulate_tr<D, EXACT>(Ks, S, nb * 32, dp, acc, lane);
+        }
+        if (i + 1 < iters) commit(i + 1);
+        tile_barrier<QW>();
+    }
+    if (KW > 1 && QW == 1) __syncthreads();  // every group has read its last tile
+    join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane);
+    if (qi < a.T) {
+        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if (KW == 1 || db % KW == kg) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk);
+    }
+}
+
+// ---- dK, dV: QW groups of 32 keys x KW groups of query tiles of 32 NB ----
+// A wavefront owns 32 keys (K and V resident as B operands, lane = key) and both accumulators, so P goes from its
+// exponentials into dV and into dS without leaving the registers. The steps are the query tiles that can see the block,
+// for every query head of the KV head's group in turn.
+template <int D, int QW, int KW, int NB, bool EXACT>
+__global__ __launch_bounds__(64 * QW * KW) void split_dkdv(AttnArgs a) {
+    constexpr int BNK = 32 * QW, BMQ = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
+    constexpr int ROWC = 2 * BMQ * 2;                    // LSE and delta of a tile's rows, in uint16
+    constexpr int TILE = 2 * BMQ * S + ROWC, NBUF = QW > 1 ? 2 : 1;
+    constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
+    const int nkb = (a.T + BNK - 1) / BNK;
+    // hs > 1: the query heads of the group are dealt to hs workgroups (gqa_head_split); this one takes heads
+    // [h0, h0 + nh) of the group and leaves fp32 partial sums for launch_gqa_reduce
+    const int hs = a.head_split;
+    int blk, rr, kvu;
+    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
+    if (a.causal && nkb > 1 ? !xcd_map_block_major(nkb, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nkb, hs, a.Hkv * a.B, blk, rr, kvu))
+        return;
+    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = rr * rep / hs, nh = (rr + 1) * rep / hs - h0;
+    const int k0 = blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
+    const float cexp = a.scale * LOG2E;
+
+    // query tiles that can see keys [k0, k0 + BNK) (paperkiln src/ops.cpp:960-965 inverted)
+    const int khi = min(k0 + BNK, a.T) - 1;
+    const int qt_lo = a.causal ? k0 / BMQ : 0;
+    const int qt_hi = (a.window > 0 && k0 >= a.sinks) ? min(a.T - 1, khi + a.window - 1) / BMQ : (a.T - 1) / BMQ;
+    const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh, iters = (steps + KW - 1) / KW;
+
+    Mover<D, G, BMQ> mq, mg;
+    mq.init(gt, a.q_st, dk);
+    mg.init(gt, a.do_st, dk);
+    float row_r = 0.0f;
+    // steps advance by KW; the (head, tile) of the next fetch is counted up
+    int f_h = kg / nqt, f_t = kg % nqt, c_t = f_t;
+    auto fetch = [&](int i) {
+        if (i * KW + kg < steps) {
+            const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * BMQ;
+            mq.load(a.q, b * a.q_sb + h * a.q_sh, a.q_st, r0, a.T, dk);
+            mg.load(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, r0, a.T, dk);
+            if (gt < 2 * BMQ) {  // LSE in the first BMQ threads, delta in the next; rows past the end are masked
+                const int t = min(r0 + gt % BMQ, a.T - 1);
+                const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + t;
+                row_r = gt < BMQ ? a.lse[lrow] : a.delta[lrow];
+            }
+            f_t += KW;
+            while (f_t >= nqt) f_t -= nqt, ++f_h;
+        }
+    };
+    auto commit = [&](int buf) {
+        uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
+        mq.store(t, S, gt);
+        mg.store(t + BMQ * S, S, gt);
+        if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = gt < BMQ ? -row_r * LOG2E : row_r;
+    };
+    fetch(0);
+    bf16x8 kreg[KK], vreg[KK];
+    load_row<D>(a.k, b * a.k_sb + hk * a.k_sh, a.k_st, kj, a.T, dk, g, kreg);
+    load_row<D>(a.v, b * a.v_sb + hk * a.v_sh, a.v_st, kj, a.T, dk, g, vreg);
+    f32x16 acc[2 * DB];  // dV^T, dK^T
+#pragma unroll
+    for (int n = 0; n < 2 * DB; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.0f;
+    const KeyVis kvis(kj, a.T, a.causal, a.window, a.sinks);
+    commit(0);
+    tile_barrier<QW>();
+
+    for (int i = 0; i < iters; ++i) {
+        if (i + 1 < iters) fetch(i + 1);
+        const uint16_t* Qs = lds + (i % NBUF * KW + kg) * TILE;
+        const uint16_t* Gs = Qs + BMQ * S;
+        const float* rows = reinterpret_cast<const float*>(Qs + 2 * BMQ * S);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int qlo = (qt_lo + c_t) * BMQ + nb * 32, qhi = qlo + 31;
+            // wavefront-uniform: nothing of this 32 x 32 block is visible
+            if (i * KW + kg >= steps || qlo >= a.T || kw0 >= a.T || (a.causal && kw0 > qhi) ||
+                (a.window > 0 && kw0 + 31 + a.window <= qlo && kw0 >= a.sinks))
+                continue;
+            f32x16 s, dp;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.0f;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                s = mfma32(lds_read8(Qs + (nb * 32 + c32) * S + kk * 16 + g * 8), kreg[kk], s);
+                dp = mfma32(lds_read8(Gs + (nb * 32 + c32) * S + kk * 16 + g * 8), vreg[kk], dp);
+            }
+            // lane = key kj; element r = query qlo + (r/4)*8 + 4g + r%4
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                const f32x4 nl = *reinterpret_cast<const f32x4*>(rows + nb * 32 + qd * 8 + g * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[qd * 4 + e] = __builtin_amdgcn_exp2f(fmaf(s[qd * 4 + e], cexp, nl[e]));
+            }
+            const bool full = qhi < a.T && kw0 + 31 < a.T && (!a.causal || kw0 + 31 <= qlo) &&
+                              (a.window == 0 || kw0 + a.window > qhi || kw0 + 31 < a.sinks);
+            if (!full) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = kvis(qlo + (r >> 2) * 8 + g * 4 + (r & 3)) ? s[r] : 0.0f;
+            }
+            accumulate_tr<D, EXACT>(Gs, S, nb * 32, s, acc, lane);
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (dp[qd * 4 + e] - dl[e]);
+            }
+            accumulate_tr<D, EXACT>(Qs, S, nb * 32, dp, acc + DB, lane);
+        }
+        c_t += KW;
+        while (c_t >= nqt) c_t -= nqt;
+        if (i + 1 < iters) commit(i + 1);
+        tile_barrier<QW>();
+    }
+    float* red = reinterpret_cast<float*>(lds) + qg * KW * DB * 1024;
+    if (KW > 1 && QW == 1) __syncthreads();  // every group has read its last tile
+    join_groups<DB, KW>(acc, red, kg, lane);
+    if (KW > 1) __syncthreads();
+    join_groups<DB, KW>(acc + DB, red, kg, lane);
+    if (kj < a.T) {
+        const bool parts = hs > 1;  // partial rows: part[unit][split][dK | dV][T][dk]
+        const int64_t pk = (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+        const int64_t rv = parts ? pk + static_cast<int64_t>(a.T) * dk : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
+        const int64_t rk = parts ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+        void* const dst_v = parts ? a.part : a.dv;
+        void* const dst_k = parts ? a.part : a.dk;
+        const bool f32 = parts || a.grad_f32;
+#pragma unroll
+        for (int n = 0; n < 2 * DB; ++n) {
+            if (KW > 1 && n % DB % KW != kg) continue;
+            if (n < DB)
+                store_block(f32, dst_v, rv, n, g, acc[n], 1.0f, dk);
+            else
+                store_block(f32, dst_k, rk, n - DB, g, acc[n], a.scale, dk);
+        }
+    }
+}
+
+
+// How a launch shares its work out: four wavefronts with 32 rows each (WIDE), or one block of 32 rows whose tiles are
+// split between four or eight wavefronts.
+enum class Form { NONE, WIDE, FOUR, EIGHT };
+
+// Which form, from the number of 32-row blocks of the launch (`blocks`) and the sequence length. A block split between
+// eight wavefronts has the shortest chain but fills half a CU or more, so it wins while the blocks come to about one
+// per CU; between four, up to two or three per CU; beyond that the chip is full either way and rows that share a
+// tile's trip to LDS win. Measured (us, bf16, causal; eight | four | the kernels of head_dim 64 / 128 without a split):
+//   forward, head_dim 64      T 512, 8 heads 7.5 | 8.4 | 11.0;  32 heads 12.1 | 9.0 | 11.3;  64 heads 22 | 14.6 | 11.8
+//                             T 4096, 1 head 21 | 35 | 58;  4 heads 29 | 35 | 58;  8 heads 51 | 51 | 59
+//                             T 1024, 32 heads 26 | 21 | 19;  T 2048, 16 heads 34 | 31 | 32;  T 128, 1 head 5.6 | 5.3 | 5.9
+//   dQ, head_dim 64           T 512, 32 heads 15 | 11 | 17;  T 1024, 32 heads 32 | 25 | 27;  T 4096, 8 heads 60 | 59 | 89
+//   dK/dV, head_dim 64        T 512, 32 heads 16 | 16 | 22;  T 1024, 32 heads 34 | 38 | 33;  T 4096, 4 heads 35 | 50 | 79
+//   forward, head_dim 128     T 512, 8 heads 11 | 12 | 16;  32 heads 18 | 18 | 16;  T 1024, 16 heads 22 | 23 | 26
+//   dQ, head_dim 128          T 512, 8 heads 16 | 14 | 22;  T 2048, 8 heads 41 | 40 | 68;  16 heads 84 | 79 | 72
+//   dK/dV, head_dim 128       T 512, 32 heads - | 24 | 34;  T 2048, 8 heads - | 48 | 66;  16 heads - | 94 | 69
+// From 4096 tokens on head_dim 128 stays with the unsplit kernels whatever the number of units: a
+// unit alone, a unit in a batch and the prefix of a longer sequence are then the same bits, which callers rely on there.
+bool one_kernel_for_any_batch(const AttnArgs& a) { return a.dk_dim == 128 && a.T >= 4096; }
+Form fwd_form(const AttnArgs& a) {
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
+    const bool plain = a.dk_dim == 64 || a.dk_dim == 128;  // the unsplit kernels take these
+    if (one_kernel_for_any_batch(a)) return Form::NONE;
+    if (blocks <= 320) return a.T <= 160 ? Form::FOUR : Form::EIGHT;
+    if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
+    if (blocks <= 600) return a.T >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 ? Form::FOUR : Form::NONE;
+    return blocks <= 1100 && a.T >= 3000 ? Form::EIGHT : Form::NONE;
+}
+Form dq_form(const AttnArgs& a) {
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
+    const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
+    if (one_kernel_for_any_batch(a)) return Form::NONE;
+    // above 96 columns eight wavefronts of this kernel do not fit the registers
+    const Form best = a.dk_dim > 96 || a.T <= 160 ? Form::FOUR : Form::EIGHT;
+    if (blocks <= 320) return best;
+    if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
+    if (blocks <= 600) return a.T >= 1536 ? best : a.dk_dim == 64 || a.T >= 768 ? Form::FOUR : Form::NONE;
+    return blocks <= 1100 && a.dk_dim == 64 && a.T >= 1000 ? Form::FOUR : Form::NONE;
+}
+int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
+Form dkdv_form(const AttnArgs& a) {
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
+    const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
+    if (one_kernel_for_any_batch(a)) return Form::NONE;
+    const Form best = a.dk_dim > 64 || a.T <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
+    if (!plain) return blocks <= 700 ? best : Form::WIDE;
+    if (blocks <= 600) return best;
+    return blocks <= 1100 && a.dk_dim == 64 && a.T >= 2000 ? best : Form::NONE;
+}
+
+template <int D, int QW, int KW, int NB, bool EXACT>
+void run_fwd(const AttnArgs& a, hipStream_t st) {
+    const int nqb = (a.T + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((split_fwd<D, QW, KW, NB, EXACT>), dim3(xcd_grid(nqb, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a);
+}
+template <int D, int QW, int KW, int NB, bool EXACT>
+void run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    const int nqb = (a.T + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((split_dq<D, QW, KW, NB, EXACT>), dim3(xcd_grid(nqb, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a,
+                       fuse_delta ? 1 : 0);
+}
+template <int D, int QW, int KW, int NB, bool EXACT>
+void run_dkdv(const AttnArgs& a, hipStream_t st) {
+    const int nkb = (a.T + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT>), dim3(xcd_grid(nkb, a.head_split, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a);
+}
+
+template <int D, bool EXACT>
+int fwd_of(const AttnArgs& a, Form f, hipStream_t st) {
+    if (f == Form::EIGHT) run_fwd<D, 1, 8, 1, EXACT>(a, st);
+    if (f == Form::FOUR) run_fwd<D, 1, 4, 1, EXACT>(a, st);
+    if constexpr (EXACT)
+        if (f == Form::WIDE) run_fwd<D, 4, 1, 2, EXACT>(a, st);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+template <int D, bool EXACT>
+int dq_of(const AttnArgs& a, Form f, bool fuse_delta, hipStream_t st) {
+    if constexpr (D <= 96)
+        if (f == Form::EIGHT) run_dq<D, 1, 8, 1, EXACT>(a, fuse_delta, st);
+    if (f == Form::FOUR) run_dq<D, 1, 4, 1, EXACT>(a, fuse_delta, st);
+    if constexpr (EXACT)
+        if (f == Form::WIDE) run_dq<D, 4, 1, 2, EXACT>(a, fuse_delta, st);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+template <int D, bool EXACT>
+int dkdv_of(const AttnArgs& a, Form f, hipStream_t st) {
+    if constexpr (D <= 64)
+        if (f == Form::EIGHT) run_dkdv<D, 1, 8, 1, EXACT>(a, st);
+    if (f == Form::FOUR) run_dkdv<D, 1, 4, 1, EXACT>(a, st);
+    if constexpr (EXACT)
+        if (f == Form::WIDE) run_dkdv<D, 4, 1, 2, EXACT>(a, st);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+// f<D, EXACT>() for the instantiation that serves head_dim dk
+#define PK_SPLIT_DISPATCH(call)                        \
+    do {                                               \
+        const int dk = a.dk_dim;                       \
+        if (dk == 64) return call(64, false);          \
+        if (dk == 128) return call(128, false);        \
+        if (dk <= 32) return call(32, true);           \
+        if (dk <= 64) return call(64, true);           \
+        if (dk <= 96) return call(96, true);           \
+        return call(128, true);                        \
+    } while (0)
+
+}  // namespace
+
+bool split_serves(const AttnArgs& a) { return a.dk_dim % 8 == 0 && a.dk_dim <= 128 && bf16_rows_aligned(a); }
+bool split_takes_fwd(const AttnArgs& a) { return fwd_form(a) != Form::NONE; }
+bool split_takes_dq(const AttnArgs& a) { return dq_form(a) != Form::NONE; }
+bool split_takes_dkdv(const AttnArgs& a) { return dkdv_form(a) != Form::NONE; }
+int launch_split_fwd(const AttnArgs& a, hipStream_t st) {
+#define PK_CALL(D, E) fwd_of<D, E>(a, fwd_form(a), st)
+    PK_SPLIT_DISPATCH(PK_CALL);
+#undef PK_CALL
+}
+int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+#define PK_CALL(D, E) dq_of<D, E>(a, dq_form(a), fuse_delta, st)
+    PK_SPLIT_DISPATCH(PK_CALL);
+#undef PK_CALL
+}
+int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
+    a.head_split = dkdv_splits(a);
+    const auto run = [&]() -> int {
+#define PK_CALL(D, E) dkdv_of<D, E>(a, dkdv_form(a), st)
+        PK_SPLIT_DISPATCH(PK_CALL);
+#undef PK_CALL
+    };
+    if (const int rc = run()) return rc;
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
+}
+
+}  // namespace pk

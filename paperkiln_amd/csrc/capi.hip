@@ -170,7 +170,7 @@ int pk_attn_fwd(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k
     const void* used[] = {q->ptr, k->ptr, v->ptr, o->ptr, lse};
     for (const void* p : used) dev_touch(p, stream);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (s->dtype == PK_BF16 && mfma_supported(a)) return launch_mfma_fwd(a, st);
+    if (s->dtype == PK_BF16 && split_serves(a)) return split_takes_fwd(a) ? launch_split_fwd(a, st) : launch_mfma_fwd(a, st);
     if (s->dtype == PK_F32 && f32_mfma_supported(a)) return launch_f32_mfma_fwd(a, st);
     return launch_generic_fwd(a, s->dtype == PK_BF16, st);
 }
@@ -254,7 +254,7 @@ int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
         a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + before_part + (256 - before_part % 256) % 256);
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (s->dtype == PK_BF16 && mfma_supported(a)) return launch_mfma_bwd(a, stages, st);
+    if (s->dtype == PK_BF16 && split_serves(a)) return launch_mfma_bwd(a, stages, st);
     if (s->dtype == PK_F32 && f32_mfma_supported(a)) return launch_f32_mfma_bwd(a, stages, st);
     return launch_generic_bwd(a, s->dtype == PK_BF16, stages, st);
 }

@@ -115,7 +115,7 @@ __host__ inline bool sink_tail_pays(const SinkTail& t, int T, int window, int kv
 // and a second kernel adds the splits in order (no atomics, repeatable). Band-free bf16 kernels only.
 __host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window, int bf16) {
     const int rep = Hq / Hkv;
-    if (!bf16 || rep <= 1 || window != 0 || (dk != 64 && dk != 128)) return 1;
+    if (!bf16 || rep <= 1 || window != 0 || dk % 8 != 0 || dk > 128) return 1;
     const int nkb = (T + 127) / 128;
     const long long wgs = static_cast<long long>(causal ? (nkb + 1) / 2 : nkb) * B * Hkv;
     if (wgs >= 384) return 1;  // at least one and a half workgroups per CU already
@@ -141,8 +141,21 @@ bool f32_mfma_supported(const AttnArgs& a);
 int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
 
+// attn_split.hip: bf16 kernels whose wavefronts split the contraction. They serve every head size that is a multiple of
+// 8 up to 128; at 64 and 128 `split_takes_*` says whether a launch is small enough for them to be ahead of the kernels
+// below, at the other sizes they take everything.
+bool split_serves(const AttnArgs& a);
+bool split_takes_fwd(const AttnArgs& a);
+bool split_takes_dq(const AttnArgs& a);
+bool split_takes_dkdv(const AttnArgs& a);
+int launch_split_fwd(const AttnArgs& a, hipStream_t st);
+int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
+int launch_split_dkdv(const AttnArgs& a, hipStream_t st);
+
 // attn_fwd_mfma.hip / attn_bwd_mfma.hip: bf16 MFMA kernels, head_dim 64 or 128.
-bool mfma_supported(const AttnArgs& a);
+// 16-byte-aligned rows whose stride keeps a tile's byte offsets in 31 bits, and a positive scale (the running max is
+// tracked on raw scores): what every bf16 matrix-core kernel asks of its tensors.
+bool bf16_rows_aligned(const AttnArgs& a);
 int launch_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
 int launch_mfma_dkdv2(const AttnArgs& a, hipStream_t st);

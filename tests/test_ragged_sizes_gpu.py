@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from paperkiln_amd import blockops, synth
+from paperkiln_amd import blockops, ops, synth
 from paperkiln_amd.llama import Llama
 
 pytestmark = pytest.mark.gpu
@@ -32,3 +32,67 @@ def test_bf16_training_on_a_ragged_token_count(tokens, seq):
     finally:
         blockops.set_gemm_backend(before)
         m.close()
+
+
+def exact_attention(q, k, v, d_o, scale, causal, window, sinks):
+    """O, LSE, dQ, dK, dV in float64 (src/ops.cpp:863-1027) of [B,T,H,dk] tensors, K / V heads shared by groups."""
+    q, k, v, d_o = (x.double().permute(0, 2, 1, 3).contiguous() for x in (q, k, v, d_o))
+    B, Hq, T, dk = q.shape
+    rep = Hq // k.shape[1]
+    kx, vx = (x.repeat_interleave(rep, 1) for x in (k, v))
+    i, j = torch.arange(T, device=q.device)[:, None], torch.arange(T, device=q.device)[None, :]
+    vis = (j <= i) if causal else torch.ones(T, T, dtype=torch.bool, device=q.device)
+    if window > 0:
+        vis = vis & ((j + window > i) | (j < sinks))
+    s = (scale * (q @ kx.transpose(2, 3))).masked_fill(~vis, float("-inf"))
+    lse = torch.logsumexp(s, -1)
+    p = torch.exp(s - lse[..., None])
+    o = p @ vx
+    dp = d_o @ vx.transpose(2, 3)
+    ds = scale * p * (dp - (d_o * o).sum(-1, keepdim=True))
+    dq, dkx, dvx = ds @ kx, ds.transpose(2, 3) @ q, p.transpose(2, 3) @ d_o
+    group = lambda x: x.reshape(B, Hq // rep, rep, T, dk).sum(2)  # noqa: E731
+    back = lambda x: x.permute(0, 2, 1, 3)  # noqa: E731
+    return back(o), lse, back(dq), back(group(dkx)), back(group(dvx))
+
+
+def run_attention(B, T, Hq, Hkv, dk, dtype, causal, window, sinks, grad_dtype=torch.float32):
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    q, d_o = (torch.randn((B, T, Hq, dk), generator=gen, device="cuda").to(dtype) for _ in range(2))
+    k, v = (torch.randn((B, T, Hkv, dk), generator=gen, device="cuda").to(dtype) for _ in range(2))
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    got = (o, lse) + ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, grad_dtype=grad_dtype)
+    return got, exact_attention(q, k, v, d_o, scale, causal, window, sinks)
+
+
+def errors(got, want):
+    """Largest difference over the reference's largest value (at least 0.5: a single token has no dQ), per output."""
+    return [float((g.double() - w).abs().max()) / max(float(w.abs().max()), 0.5) for g, w in zip(got, want)]
+
+
+# Workgroups whose wavefronts split the keys or queries: lengths around the 32-row tile, fewer tiles than wavefronts and a
+# remainder after dealing them to four and eight, one head and several, units that do not divide by the 8 XCDs.
+SPLIT_CASES = [(1, 1, 1, 1, True, 0, 0), (1, 33, 1, 1, True, 0, 0), (3, 159, 1, 1, True, 0, 0), (1, 161, 3, 3, False, 0, 0),
+               (1, 300, 5, 5, True, 0, 0), (1, 511, 7, 1, True, 0, 0), (2, 417, 9, 3, True, 0, 0), (1, 700, 2, 2, True, 37, 5),
+               (1, 1100, 1, 1, True, 64, 33)]
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_split_kernels_of_small_launches(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.bfloat16, causal, window, sinks))
+    assert max(e) < 1e-2, e
+
+
+# Head sizes that are no 64 or 128: each multiple of 8 around the padded sizes 32, 64, 96, 128; launches small enough for
+# split tiles and large enough for four rows of wavefronts per tile. P keeps 16 bits there, so fp32 dV is held to 2e-5 where
+# the bf16 operand of head_dim 64 / 128 would leave 4e-3; dQ and dK carry the rounding of the bf16 O in rowsum(dO .* O).
+@pytest.mark.parametrize("dk", [8, 24, 32, 40, 56, 72, 80, 96, 104, 120])
+@pytest.mark.parametrize("case", [(1, 200, 3, 1, True, 0, 0), (2, 77, 4, 2, False, 0, 0), (5, 97, 64, 64, True, 0, 0),
+                                  (9, 130, 28, 28, True, 40, 3)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_head_sizes_between_the_usual_ones(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.bfloat16, causal, window, sinks))
+    assert e[0] < 5e-3 and e[1] < 1e-5 and max(e[2:4]) < 5e-3 and e[4] < 2e-5, e
