@@ -620,44 +620,46 @@ int launch_fwd(const AttnArgs& a, hipStream_t st) {
 }
 
 template <int D>
-int launch_bwd(const AttnArgs& a_in, int stages, hipStream_t st) {
+int launch_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    const int nqb = (a.T + 127) / 128;
+    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
+    const dim3 grid(xcd_grid(paired ? (nqb + 1) / 2 : nqb, a.Hq / a.Hkv, a.Hkv * a.B));
+    if (fuse_delta)
+        hipLaunchKernelGGL((f32_dq<D, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((f32_dq<D, false>), grid, dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+template <int D>
+int launch_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     // a tail step is one wavefront's matrix work, as long as a full step's
     if (!sink_tail_pays(a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0}, a.T, a.window, a.Hkv * a.B, 32, 1, 1.0f))
         a.tail = nullptr;
-    const int nqb = (a.T + 127) / 128;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
-    const dim3 dq_grid(xcd_grid(paired ? (nqb + 1) / 2 : nqb, a.Hq / a.Hkv, a.Hkv * a.B));
-    const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
-    if (fused) {  // dQ forms delta itself and runs first; dK/dV reads what it wrote
-        hipLaunchKernelGGL((f32_dq<D, true>), dq_grid, dim3(256), 0, st, a);
-        PK_HIP(hipGetLastError());
-    } else if (stages & PK_BWD_DELTA) {
-        if (int rc = launch_generic_bwd(a, false, PK_BWD_DELTA, st)) return rc;
-    }
-    if (stages & PK_BWD_DKDV) {
-        const int nch = a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0;
-        const int nkb = (a.T + 127) / 128;
-        const bool paired = a.causal && a.window == 0;
-        const dim3 grid(xcd_grid(paired ? (nkb + 1) / 2 : nkb + nch, 1, a.Hkv * a.B));
-        hipLaunchKernelGGL(f32_dkdv<D>, grid, dim3(512), 0, st, a);
-        PK_HIP(hipGetLastError());
-        if (nch > 0)
-            if (int rc = launch_sink_tail_reduce(a, st)) return rc;
-    }
-    if (!fused && (stages & PK_BWD_DQ)) {
-        hipLaunchKernelGGL((f32_dq<D, false>), dq_grid, dim3(256), 0, st, a);
-        PK_HIP(hipGetLastError());
-    }
-    return PK_OK;
+    const int nch = a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0;
+    const int nkb = (a.T + 127) / 128;
+    const bool paired = a.causal && a.window == 0;
+    hipLaunchKernelGGL(f32_dkdv<D>, dim3(xcd_grid(paired ? (nkb + 1) / 2 : nkb + nch, 1, a.Hkv * a.B)), dim3(512), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return nch > 0 ? launch_sink_tail_reduce(a, st) : PK_OK;
+}
+int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    if (f32_split_takes_dq(a)) return launch_f32_split_dq(a, fuse_delta, st);
+    return a.dk_dim == 32 ? launch_dq<32>(a, fuse_delta, st) : a.dk_dim == 64 ? launch_dq<64>(a, fuse_delta, st)
+                                                                              : launch_dq<128>(a, fuse_delta, st);
+}
+int run_dkdv(const AttnArgs& a, hipStream_t st) {
+    if (f32_split_takes_dkdv(a)) return launch_f32_split_dkdv(a, st);
+    return a.dk_dim == 32 ? launch_dkdv<32>(a, st) : a.dk_dim == 64 ? launch_dkdv<64>(a, st) : launch_dkdv<128>(a, st);
 }
 
 }  // namespace
 
-// fp32 tensors (gradients fp32 as well), head_dim 32 / 64 / 128, a positive scale (the running
+// fp32 tensors (gradients fp32 as well), head_dim 32 / 64 / 128 or what the split kernels serve, a positive scale (the running
 // max is tracked on raw scores) and 16-byte-aligned rows.
 bool f32_mfma_supported(const AttnArgs& a) {
-    if (a.dk_dim != 32 && a.dk_dim != 64 && a.dk_dim != 128) return false;
+    if (a.dk_dim != 32 && a.dk_dim != 64 && a.dk_dim != 128 && !f32_split_serves(a)) return false;
     if (!(a.scale > 0.0f)) return false;
     if (!aligned_f32(a.q, a.q_sb, a.q_st, a.q_sh) || !aligned_f32(a.k, a.k_sb, a.k_st, a.k_sh) ||
         !aligned_f32(a.v, a.v_sb, a.v_st, a.v_sh) || !aligned_f32(a.o, a.o_sb, a.o_st, a.o_sh))
@@ -672,6 +674,7 @@ bool f32_mfma_supported(const AttnArgs& a) {
 }
 
 int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st) {
+    if (f32_split_takes_fwd(a)) return launch_f32_split_fwd(a, st);
     switch (a.dk_dim) {
         case 32: return launch_fwd<32>(a, st);
         case 64: return launch_fwd<64>(a, st);
@@ -680,11 +683,15 @@ int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st) {
 }
 
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
-    switch (a.dk_dim) {
-        case 32: return launch_bwd<32>(a, stages, st);
-        case 64: return launch_bwd<64>(a, stages, st);
-        default: return launch_bwd<128>(a, stages, st);
-    }
+    const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
+    int rc = PK_OK;
+    if (fused)  // dQ forms delta itself and runs first; dK/dV reads what it wrote
+        rc = run_dq(a, true, st);
+    else if (stages & PK_BWD_DELTA)
+        rc = launch_generic_bwd(a, false, PK_BWD_DELTA, st);
+    if (!rc && (stages & PK_BWD_DKDV)) rc = run_dkdv(a, st);
+    if (!rc && !fused && (stages & PK_BWD_DQ)) rc = run_dq(a, false, st);
+    return rc;
 }
 
 }  // namespace pk

@@ -1,0 +1,522 @@
+// fp32 attention (forward, dQ, dK/dV) in workgroups whose wavefronts share the CONTRACTION, the fp32 counterpart of
+// attn_split.hip: one block of 32 rows per workgroup, KW wavefronts that take every KW-th 32-row tile of the other side,
+// each from LDS of its own, results joined at the end. Operand layouts of v_mfma_f32_32x32x2_f32 as in
+// attn_f32_mfma.hip; products and sums are fp32 throughout.
+//
+// What bounds it: a 32 x 32 block is D matrix instructions of 64 clocks per product, so four wavefronts of a CU are bound
+// by the matrix pipe as soon as each has something to do. The kernels of attn_f32_mfma.hip give a workgroup 128 rows and
+// let each wavefront walk every tile: 256 workgroups of very different length at B=4 H=8 T=1024, where the longest is
+// half the launch. Here there are four times as many, a quarter or an eighth as long.
+//
+// They are also the path of every head size that is a multiple of 4 up to 128 but not 32, 64 or 128 (columns padded to
+// D = 32, 64, 96 or 128, zero past the real size and not stored).
+#include "attn_split.h"
+
+namespace pk {
+namespace {
+
+constexpr float LOG2E = 1.4426950408889634f;
+
+__device__ inline f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+__device__ inline int crow(int r, int g) { return (r >> 2) * 8 + 4 * g + (r & 3); }
+
+// A 32-row tile of a [T, dk] fp32 matrix, moved by one wavefront through a buffer resource (rows past T and chunks past
+// dk read as zero) into LDS rows of pitch D + 4: 16-byte row reads of 16 rows then touch all 64 banks once.
+template <int D>
+struct Mover32 {
+    static constexpr int NCH = D / 4, CPT = 32 * NCH / 64, P = D + 4;
+    int off[CPT];
+    u32x4 r[CPT];
+    __device__ void init(int lane, int64_t st, int dk) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int c = lane + 64 * i, row = c / NCH, ch = c % NCH;
+            off[i] = ch * 4 < dk ? static_cast<int>(row * st + ch * 4) * 4 : static_cast<int>(OUTSIDE);
+        }
+    }
+    __device__ void load(const void* base, int64_t elem_off, int64_t st, int r0, int T, int dk) {
+        const int64_t left = ((static_cast<int64_t>(T) - r0 - 1) * st + dk) * 4;  // r0 < T
+        float* p = static_cast<float*>(const_cast<void*>(base)) + elem_off + static_cast<int64_t>(r0) * st;
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc(p, 0, left > 0x7fffffff ? 0x7fffffff : static_cast<int>(left), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) r[i] = tile_load16(rs, off[i]);
+    }
+    __device__ void store(float* lds, int lane) const {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int c = lane + 64 * i;
+            *reinterpret_cast<u32x4*>(lds + (c / NCH) * P + (c % NCH) * 4) = r[i];
+        }
+    }
+};
+
+// Row `row` of a head as an operand: chunk j holds columns 8j + 4g .. +3; zero past T and past dk.
+template <int D>
+__device__ inline void load_row32(const void* base, int64_t off, int64_t st, int row, int T, int dk, int g, f32x4* out) {
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) {
+        const int col = 8 * j + 4 * g;
+        f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (row < T && col < dk) z = *reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + off + row * st + col);
+        out[j] = z;
+    }
+}
+
+// The order inside both products is pinned -- the fragments of the next group of matrix instructions, then this group --
+// so that no fragment is waited for and no more than two groups of them hold registers (left to itself the scheduler
+// reads a whole tile ahead and spills at D = 128).
+//
+// (rows of the tile) . b, contracted over the columns; b from registers, or from an LDS tile of the same layout
+template <int D, typename B>
+__device__ inline f32x16 rows_dot(const float* tile, B b, int c32, int g) {
+    constexpr int NJ = D / 8, P = D + 4;
+    const float* row = tile + c32 * P + 4 * g;
+    f32x16 t;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = 0.0f;
+    f32x4 a = *reinterpret_cast<const f32x4*>(row), bb = b(0);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        f32x4 na = a, nb = bb;
+        if (j + 1 < NJ) {
+            na = *reinterpret_cast<const f32x4*>(row + 8 * (j + 1));
+            nb = b(j + 1);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t = mfma2(a[i], bb[i], t);
+        a = na, bb = nb;
+    }
+    return t;
+}
+// acc[db] += tile^T c: register r of the C tile is the operand of the tile's row crow(r, g)
+template <int D>
+__device__ inline void accumulate_tr32(const float* tile, const f32x16& c, f32x16* acc, int c32, int g) {
+    constexpr int DB = D / 32, P = D + 4;
+    float m[DB], n[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) m[db] = tile[crow(0, g) * P + c32 + 32 * db];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if (r + 1 < 16) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) n[db] = tile[crow(r + 1, g) * P + c32 + 32 * db];
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db) acc[db] = mfma2(m[db], c[r], acc[db]);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) m[db] = n[db];
+    }
+#pragma unroll
+    for (int r = 0; r + 1 < 16; ++r) {
+        __builtin_amdgcn_sched_group_barrier(0x100, DB, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, DB, 0);
+    }
+}
+
+// ---- forward ----
+template <int D, int KW>
+__global__ __launch_bounds__(64 * KW) void f32_split_fwd(AttnArgs a) {
+    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P, RED = KW * (DB * 1024 + 128);
+    __shared__ __attribute__((aligned(16))) float lds[KW * TILE > RED ? KW * TILE : RED];
+    const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk)) return;
+    const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
+    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float cexp = a.scale * LOG2E;
+    float* const Ks = lds + kg * TILE;
+    float* const Vs = Ks + 32 * P;
+
+    Mover32<D> mk, mv;
+    mk.init(lane, a.k_st, dk);
+    mv.init(lane, a.v_st, dk);
+    const KeyTiles kt(a, q0, 32, 32);
+    // one tensor in flight at a time: V of a tile behind its S product, K of the next tile behind the rest
+    if (kg < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(kg) * 32, a.T, dk);
+    f32x4 qreg[D / 8];
+    load_row32<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    f32x16 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+    float m = -1e30f, l = 0.0f;  // the reference's running-max seed, src/ops.cpp:881
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+
+    for (int at = kg; at < kt.n; at += KW) {
+        const int k0 = kt.tile(at) * 32;
+        mk.store(Ks, lane);
+        tile_barrier<1>();
+        mv.load(a.v, vb, a.v_st, k0, a.T, dk);
+        f32x16 s = rows_dot<D>(Ks, [&](int j) { return qreg[j]; }, c32, g);
+        mv.store(Vs, lane);
+        tile_barrier<1>();
+        if (at + KW < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(at + KW) * 32, a.T, dk);
+        if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= q0 && k0 >= a.sinks))) {
+            const MaskKind kind = mask_kind(k0, k0 + 31, q0, qhi, a.T, a.causal, a.window, a.sinks);
+            if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, -INFINITY);
+            float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            mx = xhalf_max(mx);
+            if (__any(mx > m)) {  // wavefront-uniform
+                const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f((m - mn) * cexp);
+                l *= alpha;
+                m = mn;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+            }
+            const float mc = m * cexp;
+            float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, -mc));
+                ps[r & 3] += s[r];
+            }
+            l += (ps[0] + ps[1]) + (ps[2] + ps[3]);  // per-lane partial; the two halves meet below
+            accumulate_tr32<D>(Vs, s, acc, c32, g);
+        }
+        tile_barrier<1>();
+    }
+
+    l = xhalf_sum(l);
+    __syncthreads();  // every wavefront has read its last tile
+    float* ml = lds + KW * DB * 1024;
+    ml[kg * 128 + lane] = m;
+    ml[kg * 128 + 64 + lane] = l;
+    __syncthreads();
+    float mt = m, lt = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
+#pragma unroll
+    for (int k = 0; k < KW; ++k) lt += ml[k * 128 + 64 + lane] * __builtin_amdgcn_exp2f((ml[k * 128 + lane] - mt) * cexp);
+    const float alpha = __builtin_amdgcn_exp2f((m - mt) * cexp);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+    join_groups<DB, KW>(acc, lds, kg, lane);
+    if (qi < a.T) {
+        const float inv = 1.0f / lt;
+        const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if (db % KW == kg) store_block(true, a.o, ro, db, g, acc[db], inv, dk);
+        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = mt * a.scale + logf(lt);
+    }
+}
+
+// ---- dQ (and delta, when asked for with it) ----
+template <int D, int KW>
+__global__ __launch_bounds__(64 * KW) void f32_split_dq(AttnArgs a, int fuse_delta) {
+    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P, RED = KW * DB * 1024;
+    __shared__ __attribute__((aligned(16))) float lds[KW * TILE > RED ? KW * TILE : RED];
+    const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk)) return;
+    const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
+    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float cexp = a.scale * LOG2E;
+    float* const Ks = lds + kg * TILE;
+    float* const Vs = Ks + 32 * P;
+
+    Mover32<D> mk, mv;
+    mk.init(lane, a.k_st, dk);
+    mv.init(lane, a.v_st, dk);
+    const KeyTiles kt(a, q0, 32, 32);
+    // one tensor in flight at a time: V of a tile behind its S product, K of the next tile behind the rest
+    if (kg < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(kg) * 32, a.T, dk);
+    f32x4 qreg[D / 8], greg[D / 8];
+    load_row32<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    load_row32<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
+    float nlse = 0.0f, dl = 0.0f;
+    if (qi < a.T) nlse = -a.lse[lrow] * LOG2E;
+    if (fuse_delta) {
+        f32x4 oreg[D / 8];
+        load_row32<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, qi, a.T, dk, g, oreg);
+        float part = 0.0f;
+#pragma unroll
+        for (int j = 0; j < D / 8; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part = fmaf(oreg[j][i], greg[j][i], part);
+        dl = xhalf_sum(part);
+        if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
+    } else if (qi < a.T) {
+        dl = a.delta[lrow];
+    }
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    f32x16 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+
+    for (int at = kg; at < kt.n; at += KW) {
+        const int k0 = kt.tile(at) * 32;
+        mk.store(Ks, lane);
+        tile_barrier<1>();
+        mv.load(a.v, vb, a.v_st, k0, a.T, dk);
+        f32x16 s = rows_dot<D>(Ks, [&](int j) { return qreg[j]; }, c32, g);
+        mv.store(Vs, lane);
+        tile_barrier<1>();
+        if (at + KW < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(at + KW) * 32, a.T, dk);
+        if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= q0 && k0 >= a.sinks))) {
+            const f32x16 dp = rows_dot<D>(Vs, [&](int j) { return greg[j]; }, c32, g);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * (dp[r] - dl);
+            const MaskKind kind = mask_kind(k0, k0 + 31, q0, qhi, a.T, a.causal, a.window, a.sinks);
+            if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, 0.0f);
+            accumulate_tr32<D>(Ks, s, acc, c32, g);
+        }
+        tile_barrier<1>();
+    }
+    __syncthreads();  // every wavefront has read its last tile
+    join_groups<DB, KW>(acc, lds, kg, lane);
+    if (qi < a.T) {
+        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if (db % KW == kg) store_block(true, a.dq, ro, db, g, acc[db], a.scale, dk);
+    }
+}
+
+// ---- dK, dV: a block of 32 keys, the query tiles (of every query head of the group in turn) split ----
+template <int D, int KW>
+__global__ __launch_bounds__(64 * KW) void f32_split_dkdv(AttnArgs a) {
+    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P + 64, RED = KW * DB * 1024;
+    // K and V of the block stay in LDS, one copy for all wavefronts, where registers are short and the LDS has the room
+    // (at D = 128 for K only)
+    constexpr bool V_LDS = D == 64 || D == 96, K_LDS = V_LDS || D == 128;
+    constexpr int KVB = (K_LDS + V_LDS) * 32 * P;
+    __shared__ __attribute__((aligned(16))) float lds[KVB + (KW * TILE > RED ? KW * TILE : RED)];
+    const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
+    const int nkb = (a.T + 31) / 32;
+    const int hs = a.head_split;  // > 1: this workgroup takes heads [h0, h0 + nh) of the group, see gqa_head_split
+    int blk, rr, kvu;
+    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
+    if (a.causal && nkb > 1 ? !xcd_map_block_major(nkb, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nkb, hs, a.Hkv * a.B, blk, rr, kvu))
+        return;
+    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = rr * rep / hs, nh = (rr + 1) * rep / hs - h0;
+    const int k0 = blk * 32, kj = k0 + c32;
+    const float cexp = a.scale * LOG2E;
+    float* const Qs = lds + KVB + kg * TILE;
+    float* const Gs = Qs + 32 * P;
+    float* const rows = Gs + 32 * P;  // -LSE log2(e) and delta of the tile's rows
+
+    // query tiles that can see keys [k0, k0 + 32) (paperkiln src/ops.cpp:960-965 inverted)
+    const int khi = min(k0 + 32, a.T) - 1;
+    const int qt_lo = a.causal ? k0 / 32 : 0;
+    const int qt_hi = (a.window > 0 && k0 >= a.sinks) ? min(a.T - 1, khi + a.window - 1) / 32 : (a.T - 1) / 32;
+    const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh;
+
+    Mover32<D> mq, mg;
+    mq.init(lane, a.q_st, dk);
+    mg.init(lane, a.do_st, dk);
+    float row_r = 0.0f;
+    int f_h = kg / nqt, f_t = kg % nqt;  // head and tile of the next fetch
+    // one tensor in flight at a time: dO of a tile behind its S product, Q of the next tile behind the rest
+    int c_h = 0, c_r0 = 0;  // query head and first row of the step in hand
+    auto fetch_q = [&]() {
+        const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * 32;
+        mq.load(a.q, b * a.q_sb + h * a.q_sh, a.q_st, r0, a.T, dk);
+        const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(r0 + c32, a.T - 1);  // rows past the end are masked
+        row_r = g == 0 ? a.lse[lrow] : a.delta[lrow];
+        c_h = h, c_r0 = r0;
+        f_t += KW;
+        while (f_t >= nqt) f_t -= nqt, ++f_h;
+    };
+    if (kg < steps) fetch_q();
+    f32x4 kreg[D / 8], vreg[D / 8];
+    if (K_LDS) {
+        for (int c = static_cast<int>(threadIdx.x); c < (K_LDS + V_LDS) * 32 * (D / 4); c += 64 * KW) {
+            const int which = c / (32 * (D / 4)), row = c / (D / 4) % 32, col = c % (D / 4) * 4;
+            const float* src = which == 0 ? static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh + (k0 + row) * a.k_st
+                                          : static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh + (k0 + row) * a.v_st;
+            f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (k0 + row < a.T && col < dk) z = *reinterpret_cast<const f32x4*>(src + col);
+            *reinterpret_cast<f32x4*>(lds + (which * 32 + row) * P + col) = z;
+        }
+        __syncthreads();
+    }
+    if (!K_LDS) load_row32<D>(a.k, b * a.k_sb + hk * a.k_sh, a.k_st, kj, a.T, dk, g, kreg);
+    if (!V_LDS) load_row32<D>(a.v, b * a.v_sb + hk * a.v_sh, a.v_st, kj, a.T, dk, g, vreg);
+    // (rows of a tile) . (K or V rows of the block)
+    auto dot = [&](const float* tile, bool in_lds, const f32x4* reg, const float* shared) {
+        if (in_lds)
+            return rows_dot<D>(tile, [&](int j) { return *reinterpret_cast<const f32x4*>(shared + c32 * P + 8 * j + 4 * g); }, c32, g);
+        return rows_dot<D>(tile, [&](int j) { return reg[j]; }, c32, g);
+    };
+    f32x16 acc[2 * DB];  // dV^T, dK^T
+#pragma unroll
+    for (int n = 0; n < 2 * DB; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.0f;
+    const KeyVis kvis(kj, a.T, a.causal, a.window, a.sinks);
+
+    for (int step = kg; step < steps; step += KW) {
+        const int qlo = c_r0, qhi = qlo + 31;
+        mq.store(Qs, lane);
+        rows[lane] = g == 0 ? -row_r * LOG2E : row_r;
+        tile_barrier<1>();
+        mg.load(a.d_o, b * a.do_sb + c_h * a.do_sh, a.do_st, qlo, a.T, dk);
+        f32x16 s = dot(Qs, K_LDS, kreg, lds);
+        mg.store(Gs, lane);
+        tile_barrier<1>();
+        if (step + KW < steps) fetch_q();
+        if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks))) {
+            // lane = key kj; element r = query qlo + crow(r, g)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                const f32x4 nl = *reinterpret_cast<const f32x4*>(rows + qd * 8 + g * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[qd * 4 + e] = __builtin_amdgcn_exp2f(fmaf(s[qd * 4 + e], cexp, nl[e]));
+            }
+            const bool full = qhi < a.T && k0 + 31 < a.T && (!a.causal || k0 + 31 <= qlo) &&
+                              (a.window == 0 || k0 + a.window > qhi || k0 + 31 < a.sinks);
+            if (!full) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = kvis(qlo + crow(r, g)) ? s[r] : 0.0f;
+            }
+            accumulate_tr32<D>(Gs, s, acc, c32, g);
+            f32x16 dp = dot(Gs, V_LDS, vreg, lds + 32 * P);
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + 32 + qd * 8 + g * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (dp[qd * 4 + e] - dl[e]);
+            }
+            accumulate_tr32<D>(Qs, dp, acc + DB, c32, g);
+        }
+        tile_barrier<1>();
+    }
+    __syncthreads();  // every wavefront has read its last tile
+    join_groups<DB, KW>(acc, lds + KVB, kg, lane);
+    __syncthreads();
+    join_groups<DB, KW>(acc + DB, lds + KVB, kg, lane);
+    if (kj < a.T) {
+        const bool parts = hs > 1;  // partial rows: part[unit][split][dK | dV][T][dk]
+        const int64_t pk = (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+        const int64_t rv = parts ? pk + static_cast<int64_t>(a.T) * dk : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
+        const int64_t rk = parts ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            if (db % KW != kg) continue;
+            store_block(true, parts ? a.part : a.dv, rv, db, g, acc[db], 1.0f, dk);
+            store_block(true, parts ? a.part : a.dk, rk, db, g, acc[DB + db], a.scale, dk);
+        }
+    }
+}
+
+// A block's tiles split between four or eight wavefronts, or not this kernel.
+enum class Form { NONE, FOUR, EIGHT };
+
+// Which form, from the number of 32-row blocks of the launch and the length of a block's chain; the kernels of attn_f32_mfma.hip
+// (128 rows a workgroup) where they are ahead: head_dim 128 once there are about four blocks per CU -- a split block's
+// tiles then cross the L2 four times as often as theirs and hide it behind twice the matrix work only -- and many short
+// sequences. Measured (us, causal; eight | four | 128 rows):
+//   forward, head_dim 64    T 512, 8 heads 15 | 16 | 46;  T 2048, 8 heads 51 | 60 | 168;  B=4 T=1024 H=8 58 | 54 | 88
+//                           B=2 T=4096 H=16 653 | 609 | 656;  B=32 T=128 H=8 28 | 19 | 18
+//   dQ, head_dim 64         T 2048, 8 heads 68 | 84 | 222;  B=4 T=1024 H=8 89 | 79 | 117;  B=2 T=4096 H=16 912 | 833 | 919
+//   dK/dV, head_dim 64      T 512, 8 heads 23 | 25 | 97;  B=4 T=1024 H=8 96 | 105 | 169;  B=8 T=1024 H=16 384 | 423 | 338
+//                           B=2 T=4096 H=16 1130 | 1299 | 1177
+//   head_dim 32             B=4 T=1024 H=8: forward 30 | 31 | 46, dQ 43 | 43 | 64, dK/dV 59 | 53 | 100
+//   head_dim 128            T 512, 8 heads: forward - | 27 | 73, dQ - | 38 | 105, dK/dV - | 55 | 174
+//                           B=4 T=1024 H=8: - | 115 | 146, - | 162 | 204, - | 276 | 306
+//                           B=16 T=512 H=8: - | 152 | 140, - | 220 | 218, - | 381 | 190
+bool has_own_kernel(const AttnArgs& a) { return a.dk_dim == 32 || a.dk_dim == 64 || a.dk_dim == 128; }
+bool many_short(const AttnArgs& a, int64_t blocks) { return a.T <= 160 && blocks > 600; }
+Form query_form(const AttnArgs& a, int64_t short_chain) {  // forward, dQ
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
+    if (has_own_kernel(a) && (many_short(a, blocks) || (a.dk_dim == 128 && blocks > 1200))) return Form::NONE;
+    const int chain = chain_tokens(a);
+    return a.dk_dim <= 64 && ((blocks <= 600 && chain >= 1000) || (blocks <= short_chain && chain >= 256)) ? Form::EIGHT : Form::FOUR;
+}
+Form fwd_form(const AttnArgs& a) { return query_form(a, 200); }
+Form dq_form(const AttnArgs& a) { return query_form(a, 0); }
+int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
+Form dkdv_form(const AttnArgs& a) {
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
+    // where query heads share KV heads the 128-key kernel walks the whole group in one workgroup
+    if (has_own_kernel(a) && a.Hq == a.Hkv) {
+        if (many_short(a, blocks) || (a.dk_dim == 128 && blocks > 1200)) return Form::NONE;
+        if (a.dk_dim == 64 && blocks > 1400 && a.T < 3000) return Form::NONE;
+    }
+    if (a.dk_dim > 64) return Form::FOUR;
+    return a.dk_dim > 32 || (blocks <= 320 && chain_tokens(a) >= 512) ? Form::EIGHT : Form::FOUR;
+}
+
+template <int D, int KW>
+void run_fwd(const AttnArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL((f32_split_fwd<D, KW>), dim3(xcd_grid((a.T + 31) / 32, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(64 * KW), 0, st, a);
+}
+template <int D, int KW>
+void run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    hipLaunchKernelGGL((f32_split_dq<D, KW>), dim3(xcd_grid((a.T + 31) / 32, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(64 * KW), 0, st, a,
+                       fuse_delta ? 1 : 0);
+}
+template <int D, int KW>
+void run_dkdv(const AttnArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL((f32_split_dkdv<D, KW>), dim3(xcd_grid((a.T + 31) / 32, a.head_split, a.Hkv * a.B)), dim3(64 * KW), 0, st, a);
+}
+
+}  // namespace
+
+// a lane's byte offset inside a 32-row tile is kept in 31 bits
+bool f32_split_serves(const AttnArgs& a) {
+    auto ok = [](int64_t st) { return st > 0 && st < (int64_t{1} << 22); };
+    return a.dk_dim % 4 == 0 && a.dk_dim <= 128 && ok(a.q_st) && ok(a.k_st) && ok(a.v_st) && (!a.d_o || ok(a.do_st));
+}
+bool f32_split_takes_fwd(const AttnArgs& a) { return f32_split_serves(a) && fwd_form(a) != Form::NONE; }
+bool f32_split_takes_dq(const AttnArgs& a) { return f32_split_serves(a) && dq_form(a) != Form::NONE; }
+bool f32_split_takes_dkdv(const AttnArgs& a) { return f32_split_serves(a) && dkdv_form(a) != Form::NONE; }
+
+int launch_f32_split_fwd(const AttnArgs& a, hipStream_t st) {
+    const bool eight = fwd_form(a) == Form::EIGHT;
+    if (a.dk_dim <= 32)
+        eight ? run_fwd<32, 8>(a, st) : run_fwd<32, 4>(a, st);
+    else if (a.dk_dim <= 64)
+        eight ? run_fwd<64, 8>(a, st) : run_fwd<64, 4>(a, st);
+    else if (a.dk_dim <= 96)
+        run_fwd<96, 4>(a, st);
+    else
+        run_fwd<128, 4>(a, st);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    const bool eight = dq_form(a) == Form::EIGHT;
+    if (a.dk_dim <= 32)
+        eight ? run_dq<32, 8>(a, fuse_delta, st) : run_dq<32, 4>(a, fuse_delta, st);
+    else if (a.dk_dim <= 64)
+        eight ? run_dq<64, 8>(a, fuse_delta, st) : run_dq<64, 4>(a, fuse_delta, st);
+    else if (a.dk_dim <= 96)
+        run_dq<96, 4>(a, fuse_delta, st);
+    else
+        run_dq<128, 4>(a, fuse_delta, st);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+int launch_f32_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
+    a.head_split = dkdv_splits(a);
+    const bool eight = dkdv_form(a) == Form::EIGHT;
+    if (a.dk_dim <= 32)
+        eight ? run_dkdv<32, 8>(a, st) : run_dkdv<32, 4>(a, st);
+    else if (a.dk_dim <= 64)
+        run_dkdv<64, 8>(a, st);
+    else if (a.dk_dim <= 96)
+        run_dkdv<96, 4>(a, st);
+    else
+        run_dkdv<128, 4>(a, st);
+    PK_HIP(hipGetLastError());
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
+}
+
+}  // namespace pk

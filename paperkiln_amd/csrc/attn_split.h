@@ -1,0 +1,116 @@
+// What the attention kernels whose wavefronts split the contraction share (attn_split.hip: bf16, attn_f32_split.hip:
+// fp32). Accumulator blocks are 32 x 32 C tiles with lane = row of the output and the columns in natural order.
+#pragma once
+#include "mfma_common.h"
+#include "pk_internal.h"
+
+namespace pk {
+namespace {
+
+// The KW groups' accumulators of N blocks added up: group kg ends up with the sums of blocks kg, kg + KW, ... (in group
+// order, so repeatable). `red` is LDS for KW N KB per row group, free to overwrite when this is called.
+template <int N, int KW>
+__device__ inline void join_groups(f32x16* acc, float* red, int kg, int lane) {
+    if (KW == 1) return;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        if (n % KW == kg) continue;
+        f32x4* p = reinterpret_cast<f32x4*>(red) + ((kg * N + n) * 4) * 64 + lane;
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+            const f32x4 v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
+            p[qd * 64] = v;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        if (n % KW != kg) continue;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const f32x4* p = reinterpret_cast<const f32x4*>(red) + ((k * N + n) * 4) * 64 + lane;
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                f32x4 v;
+                if (k == n % KW)
+                    v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
+                else
+                    v = p[qd * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[qd * 4 + e] += v[e];
+            }
+        }
+        acc[n] = s;
+    }
+}
+
+// One 32 x 32 accumulator block (lane = row of the output, natural column order) scaled and written; columns past dk are
+// not. Both lanes of a pair (c, c + 32) hold the same row and must be active.
+__device__ inline void store_block(bool f32, void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
+    if (f32) {
+        float* row = static_cast<float*>(base) + row_off;
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+            const int col = 32 * db + 8 * qd + 4 * g;
+            const f32x4 v = {acc[qd * 4] * sc, acc[qd * 4 + 1] * sc, acc[qd * 4 + 2] * sc, acc[qd * 4 + 3] * sc};
+            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = v;
+        }
+    } else {
+        uint16_t* row = static_cast<uint16_t*>(base) + row_off;
+#pragma unroll
+        for (int qp = 0; qp < 2; ++qp) {
+            const int lo = qp * 8, hi = qp * 8 + 4;
+            const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo] * sc, acc[lo + 1] * sc),
+                                                             pack_bf16(acc[hi] * sc, acc[hi + 1] * sc), false, false);
+            const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo + 2] * sc, acc[lo + 3] * sc),
+                                                             pack_bf16(acc[hi + 2] * sc, acc[hi + 3] * sc), false, false);
+            const u32x4 v = {r0[0], r1[0], r0[1], r1[1]};
+            const int col = 32 * db + 8 * (2 * qp + g);
+            if (col < dk) *reinterpret_cast<u32x4*>(row + col) = v;
+        }
+    }
+}
+
+// A group of several wavefronts has two tile buffers and one barrier per tile; a group of one wavefront has one buffer and
+// none: a wavefront's LDS operations complete in order, so it overwrites its tile behind its own last read of it.
+template <int QW>
+__device__ inline void tile_barrier() {
+    if (QW > 1)
+        __syncthreads();
+    else
+        __builtin_amdgcn_wave_barrier();
+}
+
+// How many tokens of the other side a block of rows walks at most: what its chain of tiles is as long as.
+inline int chain_tokens(const AttnArgs& a) { return a.window > 0 && a.window + 64 < a.T ? a.window + 64 : a.T; }
+
+// The tiles of BN keys that queries [q0, q0 + BM) can see, as a list: sink tiles [0, ns), then [lo, hi].
+struct KeyTiles {
+    int ns, lo, n;
+    __device__ KeyTiles(const AttnArgs& a, int q0, int BM, int BN) {
+        const int qmax = min(q0 + BM, a.T) - 1;
+        const int hi = (a.causal ? qmax : a.T - 1) / BN;
+        lo = a.window > 0 ? max(0, q0 + 1 - a.window) / BN : 0;
+        ns = a.window > 0 ? min((a.sinks + BN - 1) / BN, lo) : 0;
+        n = ns + hi - lo + 1;
+    }
+    __device__ int tile(int i) const { return i < ns ? i : lo + i - ns; }
+};
+
+__device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk) {
+    const int rep = a.Hq / a.Hkv;
+    int blk, rr, kvu;
+    // causal blocks without a band: the heaviest blocks of every unit first
+    if (a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
+                                  : !xcd_map(nqb, rep, a.Hkv * a.B, blk, rr, kvu))
+        return false;
+    hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    qblk = nqb - 1 - blk;
+    return true;
+}
+
+}  // namespace
+}  // namespace pk

@@ -12,8 +12,7 @@
 // size read as zero and are not stored). P and dS enter their products there as TWO bf16 operands, the rounded value
 // and the remainder (EXACT: 16 significant bits, against 8 in the kernels of head_dim 64 and 128), because these sizes
 // used to run in fp32 arithmetic throughout.
-#include "mfma_common.h"
-#include "pk_internal.h"
+#include "attn_split.h"
 
 namespace pk {
 namespace {
@@ -101,108 +100,6 @@ __device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, 
         acc[db] = mfma32(m, h1, acc[db]);
         if (EXACT) acc[db] = mfma32(m, l1, acc[db]);
     }
-}
-
-// The KW groups' accumulators of N blocks added up: group kg ends up with the sums of blocks kg, kg + KW, ... (in group
-// order, so repeatable). `red` is LDS for KW N KB per row group, free to overwrite when this is called.
-template <int N, int KW>
-__device__ inline void join_groups(f32x16* acc, float* red, int kg, int lane) {
-    if (KW == 1) return;
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-        if (n % KW == kg) continue;
-        f32x4* p = reinterpret_cast<f32x4*>(red) + ((kg * N + n) * 4) * 64 + lane;
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-            const f32x4 v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
-            p[qd * 64] = v;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-        if (n % KW != kg) continue;
-        f32x16 s;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-            const f32x4* p = reinterpret_cast<const f32x4*>(red) + ((k * N + n) * 4) * 64 + lane;
-#pragma unroll
-            for (int qd = 0; qd < 4; ++qd) {
-                f32x4 v;
-                if (k == n % KW)
-                    v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
-                else
-                    v = p[qd * 64];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s[qd * 4 + e] += v[e];
-            }
-        }
-        acc[n] = s;
-    }
-}
-
-// One 32 x 32 accumulator block (lane = row of the output, natural column order) scaled and written; columns past dk are
-// not. Both lanes of a pair (c, c + 32) hold the same row and must be active.
-__device__ inline void store_block(bool f32, void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
-    if (f32) {
-        float* row = static_cast<float*>(base) + row_off;
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-            const int col = 32 * db + 8 * qd + 4 * g;
-            const f32x4 v = {acc[qd * 4] * sc, acc[qd * 4 + 1] * sc, acc[qd * 4 + 2] * sc, acc[qd * 4 + 3] * sc};
-            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = v;
-        }
-    } else {
-        uint16_t* row = static_cast<uint16_t*>(base) + row_off;
-#pragma unroll
-        for (int qp = 0; qp < 2; ++qp) {
-            const int lo = qp * 8, hi = qp * 8 + 4;
-            const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo] * sc, acc[lo + 1] * sc),
-                                                             pack_bf16(acc[hi] * sc, acc[hi + 1] * sc), false, false);
-            const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo + 2] * sc, acc[lo + 3] * sc),
-                                                             pack_bf16(acc[hi + 2] * sc, acc[hi + 3] * sc), false, false);
-            const u32x4 v = {r0[0], r1[0], r0[1], r1[1]};
-            const int col = 32 * db + 8 * (2 * qp + g);
-            if (col < dk) *reinterpret_cast<u32x4*>(row + col) = v;
-        }
-    }
-}
-
-// A group of several wavefronts has two tile buffers and one barrier per tile; a group of one wavefront has one buffer and
-// none: a wavefront's LDS operations complete in order, so it overwrites its tile behind its own last read of it.
-template <int QW>
-__device__ inline void tile_barrier() {
-    if (QW > 1)
-        __syncthreads();
-    else
-        __builtin_amdgcn_wave_barrier();
-}
-
-// The tiles of BN keys that queries [q0, q0 + BM) can see, as a list: sink tiles [0, ns), then [lo, hi].
-struct KeyTiles {
-    int ns, lo, n;
-    __device__ KeyTiles(const AttnArgs& a, int q0, int BM, int BN) {
-        const int qmax = min(q0 + BM, a.T) - 1;
-        const int hi = (a.causal ? qmax : a.T - 1) / BN;
-        lo = a.window > 0 ? max(0, q0 + 1 - a.window) / BN : 0;
-        ns = a.window > 0 ? min((a.sinks + BN - 1) / BN, lo) : 0;
-        n = ns + hi - lo + 1;
-    }
-    __device__ int tile(int i) const { return i < ns ? i : lo + i - ns; }
-};
-
-__device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk) {
-    const int rep = a.Hq / a.Hkv;
-    int blk, rr, kvu;
-    // causal blocks without a band: the heaviest blocks of every unit first
-    if (a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
-                                  : !xcd_map(nqb, rep, a.Hkv * a.B, blk, rr, kvu))
-        return false;
-    hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
-    qblk = nqb - 1 - blk;
-    return true;
 }
 
 // ---- forward: QW groups of 32 queries x KW groups of key tiles of 32 NB keys ----
@@ -604,7 +501,7 @@ __global__ __launch_bounds__(64 * QW * KW) void split_dkdv(AttnArgs a) {
 // split between four or eight wavefronts.
 enum class Form { NONE, WIDE, FOUR, EIGHT };
 
-// Which form, from the number of 32-row blocks of the launch (`blocks`) and the sequence length. A block split between
+// Which form, from the number of 32-row blocks of the launch (`blocks`) and the length of a block's chain. A block split between
 // eight wavefronts has the shortest chain but fills half a CU or more, so it wins while the blocks come to about one
 // per CU; between four, up to two or three per CU; beyond that the chip is full either way and rows that share a
 // tile's trip to LDS win. Measured (us, bf16, causal; eight | four | the kernels of head_dim 64 / 128 without a split):
@@ -623,31 +520,31 @@ Form fwd_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;  // the unsplit kernels take these
     if (one_kernel_for_any_batch(a)) return Form::NONE;
-    if (blocks <= 320) return a.T <= 160 ? Form::FOUR : Form::EIGHT;
+    if (blocks <= 320) return chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
     if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
-    if (blocks <= 600) return a.T >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 ? Form::FOUR : Form::NONE;
-    return blocks <= 1100 && a.T >= 3000 ? Form::EIGHT : Form::NONE;
+    if (blocks <= 600) return chain_tokens(a) >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 ? Form::FOUR : Form::NONE;
+    return blocks <= 1100 && chain_tokens(a) >= 3000 ? Form::EIGHT : Form::NONE;
 }
 Form dq_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     if (one_kernel_for_any_batch(a)) return Form::NONE;
     // above 96 columns eight wavefronts of this kernel do not fit the registers
-    const Form best = a.dk_dim > 96 || a.T <= 160 ? Form::FOUR : Form::EIGHT;
+    const Form best = a.dk_dim > 96 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
     if (blocks <= 320) return best;
     if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
-    if (blocks <= 600) return a.T >= 1536 ? best : a.dk_dim == 64 || a.T >= 768 ? Form::FOUR : Form::NONE;
-    return blocks <= 1100 && a.dk_dim == 64 && a.T >= 1000 ? Form::FOUR : Form::NONE;
+    if (blocks <= 600) return chain_tokens(a) >= 1536 ? best : a.dk_dim == 64 || chain_tokens(a) >= 768 ? Form::FOUR : Form::NONE;
+    return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 1000 ? Form::FOUR : Form::NONE;
 }
 int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
 Form dkdv_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     if (one_kernel_for_any_batch(a)) return Form::NONE;
-    const Form best = a.dk_dim > 64 || a.T <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
+    const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
     if (!plain) return blocks <= 700 ? best : Form::WIDE;
     if (blocks <= 600) return best;
-    return blocks <= 1100 && a.dk_dim == 64 && a.T >= 2000 ? best : Form::NONE;
+    return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 2000 ? best : Form::NONE;
 }
 
 template <int D, int QW, int KW, int NB, bool EXACT>

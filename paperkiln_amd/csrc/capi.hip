@@ -101,10 +101,10 @@ size_t tail_bytes(const pk_attn_shape* s) {
     return pad + sink_tail_bytes(s->B * s->Hkv, t.nch, s->dk);
 }
 
-// (GQA, band-free bf16 only) the per-split partial dK / dV of the dK/dV launch, after delta and the sink tail
+// (GQA only) the per-split partial dK / dV of the dK/dV launch, after delta and the sink tail
 int head_split_of(const pk_attn_shape* s) {
     const Mask m = effective_mask(s);
-    return gqa_head_split(s->B, s->T, s->Hq, s->Hkv, s->dk, s->causal != 0, m.window, s->dtype == PK_BF16);
+    return gqa_head_split(s->B, s->T, s->Hq, s->Hkv, s->dk, s->causal != 0, m.window);
 }
 size_t part_bytes(const pk_attn_shape* s) {
     const int hs = head_split_of(s);

@@ -112,12 +112,13 @@ __host__ inline bool sink_tail_pays(const SinkTail& t, int T, int window, int kv
 // fill 64 of 256 CUs. Where the launch would leave CUs idle, the heads of a group are dealt to `hs`
 // workgroups; split r takes heads [r rep / hs, (r + 1) rep / hs), writes its fp32 partial dK and dV to
 //   part[((unit * hs + r) * 2 + {0: dK, 1: dV}) * T + key][head_dim]
-// and a second kernel adds the splits in order (no atomics, repeatable). Band-free bf16 kernels only.
-__host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window, int bf16) {
+// and a second kernel adds the splits in order (no atomics, repeatable). The kernels of attn_split.hip and
+// attn_f32_split.hip split that way, band or not, and mfma_dkdv3 (band-free bf16); the others walk a group in one workgroup.
+__host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window) {
     const int rep = Hq / Hkv;
-    if (!bf16 || rep <= 1 || window != 0 || dk % 8 != 0 || dk > 128) return 1;
+    if (rep <= 1 || dk % 4 != 0 || dk > 128) return 1;
     const int nkb = (T + 127) / 128;
-    const long long wgs = static_cast<long long>(causal ? (nkb + 1) / 2 : nkb) * B * Hkv;
+    const long long wgs = static_cast<long long>(causal && window == 0 ? (nkb + 1) / 2 : nkb) * B * Hkv;
     if (wgs >= 384) return 1;  // at least one and a half workgroups per CU already
     const int hs = static_cast<int>((512 + wgs - 1) / wgs);
     return hs < rep ? hs : rep;
@@ -136,7 +137,17 @@ int launch_sink_tail_reduce(const AttnArgs& a, hipStream_t st);
 int launch_generic_fwd(const AttnArgs& a, bool bf16_in, hipStream_t st);
 int launch_generic_bwd(const AttnArgs& a, bool bf16_in, int stages, hipStream_t st);
 
-// attn_f32_mfma.hip: fp32 tensors on the fp32 matrix instruction, head_dim 32 / 64 / 128.
+// attn_f32_split.hip: fp32 kernels whose wavefronts split the contraction; every head size that is a multiple of 4 up to
+// 128. At 32, 64 and 128 `f32_split_takes_*` says whether they are ahead of the kernels of attn_f32_mfma.hip.
+bool f32_split_serves(const AttnArgs& a);
+bool f32_split_takes_fwd(const AttnArgs& a);
+bool f32_split_takes_dq(const AttnArgs& a);
+bool f32_split_takes_dkdv(const AttnArgs& a);
+int launch_f32_split_fwd(const AttnArgs& a, hipStream_t st);
+int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
+int launch_f32_split_dkdv(const AttnArgs& a, hipStream_t st);
+
+// attn_f32_mfma.hip: fp32 tensors on the fp32 matrix instruction, head sizes that are multiples of 4 up to 128.
 bool f32_mfma_supported(const AttnArgs& a);
 int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);

@@ -96,3 +96,18 @@ def test_head_sizes_between_the_usual_ones(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.bfloat16, causal, window, sinks))
     assert e[0] < 5e-3 and e[1] < 1e-5 and max(e[2:4]) < 5e-3 and e[4] < 2e-5, e
+
+
+# The same of fp32 tensors: head_dim 32 / 64 / 128 in launches small enough for the split kernels (four and eight
+# wavefronts, query heads dealt to several workgroups), and sizes between them at any launch size.
+F32_CASES = [(c, dk) for c in SPLIT_CASES for dk in (32, 64, 128)]
+F32_CASES += [(c, dk) for c in [(1, 200, 3, 1, True, 0, 0), (2, 77, 4, 2, False, 0, 0), (5, 97, 64, 64, True, 0, 0), (9, 130, 28, 28, True, 40, 3)]
+              for dk in (4, 20, 48, 80, 100, 124)]
+F32_CASES += [((1, 1100, 8, 2, True, 0, 0), 64), ((1, 1100, 8, 2, True, 300, 4), 32)]
+
+
+@pytest.mark.parametrize("case,dk", F32_CASES, ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c if isinstance(c, tuple) else f"d{c}")
+def test_fp32_split_kernels(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.float32, causal, window, sinks))
+    assert max(e) < 5e-6, e
