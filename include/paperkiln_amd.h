@@ -184,6 +184,9 @@ int pk_llama_param_info(void* handle, int i, char* name, size_t name_len, int64_
 int pk_llama_set_param(void* handle, int i, const float* host);
 int pk_llama_get_param(void* handle, int i, float* host);
 int pk_llama_get_grad(void* handle, int i, float* host);
+/* Every parameter (grads 0) or gradient (grads 1) at once: hosts[i] takes the i-th, pk_llama_num_params pointers. The
+ * copies are pipelined through pinned staging that the model keeps (at most 16 MiB). */
+int pk_llama_get_all(void* handle, int grads, float* const* hosts);
 /* zero_grad -> forward -> mean cross-entropy -> backward: the step of tools/mtstudio.cpp:456-471.
  * ids/targets are host arrays of n tokens, B = n/seq_len stacked sequences (seq_len 0 = one).
  * checkpoint_blocks: Llama::checkpoint_blocks (llama.hpp:45). fused_head 1 evaluates the tied head

@@ -4,10 +4,13 @@
 // shape of tools/mtstudio.cpp:456-480. The per-block activation checkpoint is
 // the reference's checkpoint() (src/autograd.cpp:68-102) on HBM tensors; its
 // receipt here is bytes from the allocator's high-water mark, not a node count.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "pk_internal.h"
@@ -72,6 +75,7 @@ struct Model {
     // allocation, [1, slab_len] fp32, with every parameter's tensors as views at the same offset:
     // zero_grad, the clip norm and the optimiser step are then one launch each, not one per parameter.
     Tensor pslab, gslab, mslab, vslab;
+    SlabReader reader;
     long t = 0;
     // Pinned staging for what a pass sends up (ids, targets, positions): one host copy and asynchronous transfers
     // instead of three transfers from pageable memory with a wait each. Written only between passes (a pass ends
@@ -314,6 +318,20 @@ int pk_llama_get_grad(void* h, int i, float* host) {
             std::memset(host, 0, sizeof(float) * p->data.numel());
         else
             hip_check(hipMemcpy(host, p->grad.ptr(), sizeof(float) * p->data.numel(), hipMemcpyDeviceToHost), "hipMemcpy");
+    });
+}
+int pk_llama_get_all(void* h, int grads, float* const* hosts) {
+    return with_model(h, [&](Model* m) {
+        if (!hosts) throw Error(PK_ERR_ARGUMENT, "pk_llama_get_all: null argument");
+        const Tensor& slab = grads ? m->gslab : m->pslab;
+        std::vector<SlabReader::Piece> pieces;
+        for (size_t i = 0; i < m->named.size(); ++i) {
+            const Tensor& t = grads ? m->named[i].second->grad : m->named[i].second->data;
+            if (!hosts[i]) throw Error(PK_ERR_ARGUMENT, "pk_llama_get_all: null data");
+            if (t.buf != slab.buf) throw std::runtime_error("a parameter's storage is no longer the model's own");
+            pieces.push_back(SlabReader::Piece{t.off_bytes / static_cast<int64_t>(sizeof(float)), t.numel(), hosts[i]});
+        }
+        m->reader.read(static_cast<const float*>(slab.ptr()), pieces, tape_stream());
     });
 }
 int pk_llama_set_head_chunk(void* h, int64_t rows) {

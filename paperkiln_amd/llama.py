@@ -51,19 +51,16 @@ class Llama:
             a = np.ascontiguousarray(sd[n], np.float32).reshape(self.shapes[i])
             _lib.check(self.L.pk_llama_set_param(self.h, i, a.ctypes.data_as(_f32p)))
 
-    def _get(self, fn):
-        out = {}
-        for i, (n, s) in enumerate(zip(self.names, self.shapes)):
-            a = np.empty(s, np.float32)
-            _lib.check(fn(self.h, i, a.ctypes.data_as(_f32p)))
-            out[n] = a
+    def _get(self, grads):
+        out = {n: np.empty(s, np.float32) for n, s in zip(self.names, self.shapes)}
+        _lib.check(self.L.pk_llama_get_all(self.h, grads, (C.c_void_p * len(out))(*(a.ctypes.data for a in out.values()))))
         return out
 
     def params(self):
-        return self._get(self.L.pk_llama_get_param)
+        return self._get(0)
 
     def grads(self):
-        return self._get(self.L.pk_llama_get_grad)
+        return self._get(1)
 
     def set_head_chunk(self, rows):
         """Rows of the tied head evaluated at a time when fused_head=True (default 2048)."""
