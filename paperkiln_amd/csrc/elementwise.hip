@@ -510,51 +510,88 @@ __global__ void rms_bwd_dw_part8(const uint16_t* dy, const uint16_t* x, const fl
     }
 }
 // dx and the dW partial sums in one pass over dY and x (both are wanted in a training step, and each reads both
-// tensors): a wavefront takes ROWS_PB / 8 rows of its block, two at a time, lane l the columns 8 l .. 8 l + 7 of
-// every 512-column pass (NP passes, C <= 512 NP), keeps its rows' contribution to dW in registers, and the eight
-// wavefronts meet in LDS in a fixed order.
+// tensors): a wavefront takes every eighth row of its block's rows_pb, two at a time, lane l the E columns E l ..
+// of every 64 E-column pass (E = 16 bytes of elements; NP passes, C <= 64 E NP), keeps its rows' contribution to dW in
+// registers, and the eight wavefronts meet in LDS in a fixed order.
 // ADD: dx = addend + (the above), the gradient that reached x along another path (a residual connection), added
-// before the one rounding to bf16.
-template <int NP, bool ADD>
-__global__ void rms_bwd_dx_dw8(const uint16_t* dy, const uint16_t* x, const float* rinv, const float* w,
-                               const uint16_t* addend, uint16_t* dx, float* part, int64_t R, int C) {
-    constexpr int NWV = 8;            // wavefronts per block
+// before the one rounding to the storage type.
+// Bound by the latency of a load and a row reduction where there are few rows: 512 fp32 rows of 128 took 3.1 us for dx,
+// 10.6 us for the dW parts (one thread to a column walked 32 rows) and 2.2 us for the addend as kernels of their own.
+template <typename T>
+struct RowVec;
+template <>
+struct RowVec<uint16_t> {
+    static constexpr int E = 8;
+    float v[E];
+    __device__ void load(const uint16_t* p) {
+        const F8 x = ld8(p, 0);
+#pragma unroll
+        for (int k = 0; k < E; ++k) v[k] = x.v[k];
+    }
+    __device__ void load(const float* p) {
+        const F8 x = ld8(p, 0);
+#pragma unroll
+        for (int k = 0; k < E; ++k) v[k] = x.v[k];
+    }
+    __device__ void store(uint16_t* p) const {
+        F8 x;
+#pragma unroll
+        for (int k = 0; k < E; ++k) x.v[k] = v[k];
+        st8(p, 0, x);
+    }
+};
+template <>
+struct RowVec<float> {
+    static constexpr int E = 4;
+    float v[E];
+    __device__ void load(const float* p) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+        for (int k = 0; k < E; ++k) v[k] = x[k];
+    }
+    __device__ void store(float* p) const { *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]}; }
+};
+template <typename T, int NP, bool ADD>
+__global__ void rms_bwd_dx_dw(const T* dy, const T* x, const float* rinv, const float* w, const T* addend, T* dx, float* part,
+                              int64_t R, int C, int rows_pb) {
+    using V = RowVec<T>;
+    constexpr int NWV = 8, E = V::E;  // wavefronts per block, columns per lane and pass
     extern __shared__ float sh_dw[];  // [NWV - 1][C]: wavefronts 1 .. NWV - 1
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * ROWS_PB, r1 = min(r0 + ROWS_PB, R);
-    F8 acc[NP], ww[NP];
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_pb, r1 = min(r0 + rows_pb, R);
+    V acc[NP], ww[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-        const int j = lane * 8 + p * 512;
+        const int j = (lane + p * 64) * E;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc[p].v[k] = 0.0f;
-        if (j < C) ww[p] = ld8(w, j);
+        for (int k = 0; k < E; ++k) acc[p].v[k] = 0.0f;
+        if (j < C) ww[p].load(w + j);
     }
     // two rows of the wavefront at a time: their loads are in flight together, and so are the two row reductions
     for (int64_t row = r0 + wv; row < r1; row += 2 * NWV) {
         const bool two = row + NWV < r1;
         const int64_t rows[2] = {row, two ? row + NWV : row};
-        F8 g[2][NP], v[2][NP], e[2][ADD ? NP : 1];
+        V g[2][NP], v[2][NP], e[2][ADD ? NP : 1];
         float term[2] = {0.0f, 0.0f};
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const int j = lane * 8 + p * 512;
+                const int j = (lane + p * 64) * E;
                 if (j < C) {
-                    g[q][p] = ld8(dy + rows[q] * C, j);
-                    v[q][p] = ld8(x + rows[q] * C, j);
-                    if (ADD) e[q][p] = ld8(addend + rows[q] * C, j);
+                    g[q][p].load(dy + rows[q] * C + j);
+                    v[q][p].load(x + rows[q] * C + j);
+                    if (ADD) e[q][p].load(addend + rows[q] * C + j);
                 }
             }
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const int j = lane * 8 + p * 512;
+                const int j = (lane + p * 64) * E;
                 if (j < C) {
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) term[q] = fmaf(g[q][p].v[k] * ww[p].v[k], v[q][p].v[k], term[q]);
+                    for (int k = 0; k < E; ++k) term[q] = fmaf(g[q][p].v[k] * ww[p].v[k], v[q][p].v[k], term[q]);
                 }
             }
         term[0] = wave_sum(term[0]);
@@ -565,16 +602,16 @@ __global__ void rms_bwd_dx_dw8(const uint16_t* dy, const uint16_t* x, const floa
             const float ri = rinv[rows[q]], kk = ri * ri * term[q] / static_cast<float>(C);
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const int j = lane * 8 + p * 512;
+                const int j = (lane + p * 64) * E;
                 if (j < C) {
-                    F8 o;
+                    V o;
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) {
+                    for (int k = 0; k < E; ++k) {
                         o.v[k] = ri * (g[q][p].v[k] * ww[p].v[k] - v[q][p].v[k] * kk);
                         if (ADD) o.v[k] += e[q][p].v[k];
                         acc[p].v[k] = fmaf(g[q][p].v[k] * v[q][p].v[k], ri, acc[p].v[k]);
                     }
-                    st8(dx + rows[q] * C, j, o);
+                    o.store(dx + rows[q] * C + j);
                 }
             }
         }
@@ -582,10 +619,10 @@ __global__ void rms_bwd_dx_dw8(const uint16_t* dy, const uint16_t* x, const floa
     if (wv > 0) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const int j = lane * 8 + p * 512;
+            const int j = (lane + p * 64) * E;
             if (j < C) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) sh_dw[(wv - 1) * C + j + k] = acc[p].v[k];
+                for (int k = 0; k < E; ++k) sh_dw[(wv - 1) * C + j + k] = acc[p].v[k];
             }
         }
     }
@@ -593,10 +630,10 @@ __global__ void rms_bwd_dx_dw8(const uint16_t* dy, const uint16_t* x, const floa
     if (wv == 0) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const int j = lane * 8 + p * 512;
+            const int j = (lane + p * 64) * E;
             if (j < C) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
+                for (int k = 0; k < E; ++k) {
                     float t = acc[p].v[k];
 #pragma unroll
                     for (int q = 0; q < NWV - 1; ++q) t += sh_dw[q * C + j + k];
@@ -801,6 +838,51 @@ __global__ void __launch_bounds__(EMB_NT) emb_bwd_runs(const T* dy, const int* s
     *dst = acc;
 }
 
+// The same sums without the sort, for a batch of ids that a workgroup can look through itself: block p leaves if an
+// earlier row has row p's id, and otherwise lists the later rows that have it, in ascending order (each wavefront its own
+// quarter of them), and adds them up. A sort of a few hundred ids is four launches that take 15 us on an idle chip.
+constexpr int EMB_SCAN_MAX = 4096;
+template <typename T>
+__global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, float* dtable, int n, int d) {
+    __shared__ uint16_t rows[NT / 64][EMB_SCAN_MAX / (NT / 64) + 64];
+    __shared__ int count[NT / 64];
+    const int p = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int id = ids[p];
+    bool seen = false;
+#pragma unroll 4
+    for (int q = threadIdx.x; q < p; q += NT) seen = seen | (ids[q] == id);
+    if (__syncthreads_or(seen)) return;
+    const int quarter = ((n - p + NT - 1) / NT) * 64;  // of the rows p .. n - 1, in whole wavefronts
+    const int lo = p + wv * quarter, hi = min(lo + quarter, n);
+    int c = 0;
+#pragma unroll 4
+    for (int q0 = lo; q0 < hi; q0 += 64) {
+        const bool hit = q0 + lane < hi && ids[q0 + lane] == id;
+        const uint64_t m = __ballot(hit);
+        if (hit) rows[wv][c + __popcll(m & ((uint64_t{1} << lane) - 1))] = static_cast<uint16_t>(q0 + lane);
+        c += __popcll(m);
+    }
+    if (lane == 0) count[wv] = c;
+    __syncthreads();
+    for (int col = threadIdx.x; col < d; col += NT) {
+        float* dst = dtable + static_cast<int64_t>(id) * d + col;
+        float acc = *dst;
+        for (int w = 0; w < NT / 64; ++w) {
+            const int end = count[w];
+            int r = 0;
+            for (; r + EMB_ROWS <= end; r += EMB_ROWS) {
+                float v[EMB_ROWS];
+#pragma unroll
+                for (int u = 0; u < EMB_ROWS; ++u) v[u] = ldf(dy, static_cast<int64_t>(rows[w][r + u]) * d + col);
+#pragma unroll
+                for (int u = 0; u < EMB_ROWS; ++u) acc += v[u];
+            }
+            for (; r < end; ++r) acc += ldf(dy, static_cast<int64_t>(rows[w][r]) * d + col);
+        }
+        *dst = acc;
+    }
+}
+
 __device__ inline float block_reduce(float x, bool is_max, float* sh) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
@@ -965,14 +1047,34 @@ __global__ void sumsq_part(const float* x, int64_t n, double* part) {
     }
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
-// CLIP: the gradient is scaled by gs first and the scaled value written back, as ops::clip_grad_norm leaves it
-// (src/ops.cpp:1058-1062), in the same pass instead of one of its own.
-template <bool CLIP>
+// The clip of ops::clip_grad_norm (src/ops.cpp:1047-1062) from the partial sums of squares: the norm in double, what the
+// gradients are to be multiplied by, and the norm itself for the host (pinned memory). It stays on the device: the
+// optimizer step behind it reads it there, where a copy to the host and back between the two left the GPU idle for 35 to
+// 50 us a step.
+__global__ void clip_factor_k(const double* part, int n, float max_norm, float* factor, float* norm_out) {
+    __shared__ double sh[NT];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < n; i += NT) s += part[i];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = NT / 2; o >= 1; o >>= 1) {
+        if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const double total = sqrt(sh[0]), limit = static_cast<double>(max_norm);
+        *factor = total > limit && total > 0.0 ? static_cast<float>(limit / total) : 1.0f;
+        *norm_out = static_cast<float>(total);
+    }
+}
+// clip (if given): the gradient is scaled by *clip first and the scaled value written back, as ops::clip_grad_norm leaves
+// it (src/ops.cpp:1058-1062), in the same pass instead of one of its own.
 __global__ void adamw_k(float* p, float* g, float* m, float* v, float lr, float b1, float b2, float eps, float wd, float c1,
-                        float c2, float gs, int64_t n) {
+                        float c2, const float* clip, int64_t n) {
+    const float gs = clip ? *clip : 1.0f;
     for (int64_t i = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * NT) {
         float gi = g[i];
-        if (CLIP) {
+        if (gs != 1.0f) {
             gi *= gs;
             g[i] = gi;
         }
@@ -984,6 +1086,7 @@ __global__ void adamw_k(float* p, float* g, float* m, float* v, float lr, float 
         p[i] -= lr * (upd + wd * p[i]);
     }
 }
+__global__ void copy_word_k(const uint32_t* src, uint32_t* dst) { *dst = *src; }
 
 void same_shape(const Tensor& a, const Tensor& b, const char* who) {
     if (a.rows != b.rows || a.cols != b.cols) throw std::runtime_error(std::string(who) + ": shape mismatch");
@@ -1189,30 +1292,37 @@ void k_rmsnorm_bwd(const Tensor& dy, const Tensor& x, const float* rinv, const T
     const int C = static_cast<int>(x.cols);
     if (addend && (!dx || addend->rows != x.rows || addend->cols != x.cols || addend->dtype != dx->dtype))
         throw std::runtime_error("rmsnorm backward: the addend must have dx's shape and type");
-    if (dx && dw && x.dtype == PK_BF16 && C % 8 == 0 && C <= 2048 && aligned16p(x.ptr()) && aligned16p(dy.ptr()) &&
-        aligned16p(dx->ptr()) && aligned16p(w.ptr()) && (!addend || aligned16p(addend->ptr()))) {
-        const int nparts = static_cast<int>((x.rows + ROWS_PB - 1) / ROWS_PB);
+    if (dx && dw && C % 8 == 0 && C <= 2048 && aligned16p(x.ptr()) && aligned16p(dy.ptr()) && aligned16p(dx->ptr()) &&
+        aligned16p(w.ptr()) && (!addend || aligned16p(addend->ptr()))) {
+        // one row to a wavefront until that gives every CU a workgroup, four of them beyond: a longer walk down the
+        // rows means fewer partial sums of dW to add afterwards
+        const int rows_pb = x.rows >= 256 * ROWS_PB ? ROWS_PB : x.rows >= 128 * ROWS_PB ? ROWS_PB / 2 : ROWS_PB / 4;
+        const int nparts = static_cast<int>((x.rows + rows_pb - 1) / rows_pb);
         Buffer part(sizeof(float) * static_cast<size_t>(nparts) * C);
         const size_t lds = sizeof(float) * 7 * C;
-        auto launch = [&](auto np) {
-            constexpr int NP = decltype(np)::value;
+        PK_DISPATCH1(T, x.dtype, {
+            auto launch = [&](auto np, auto add) {
+                hipLaunchKernelGGL((rms_bwd_dx_dw<T, decltype(np)::value, decltype(add)::value>), dim3(nparts), dim3(512), lds,
+                                   tape_stream(), static_cast<const T*>(dy.ptr()), static_cast<const T*>(x.ptr()), rinv,
+                                   static_cast<const float*>(w.ptr()), static_cast<const T*>(addend ? addend->ptr() : nullptr),
+                                   static_cast<T*>(dx->ptr()), static_cast<float*>(part.p), x.rows, C, rows_pb);
+            };
+            auto passes = [&](auto add) {
+                const int np = (C + 64 * RowVec<T>::E - 1) / (64 * RowVec<T>::E);
+                if (np <= 1)
+                    launch(std::integral_constant<int, 1>{}, add);
+                else if (np <= 2)
+                    launch(std::integral_constant<int, 2>{}, add);
+                else if (np <= 4)
+                    launch(std::integral_constant<int, 4>{}, add);
+                else
+                    launch(std::integral_constant<int, 8>{}, add);
+            };
             if (addend)
-                hipLaunchKernelGGL((rms_bwd_dx_dw8<NP, true>), dim3(nparts), dim3(512), lds, tape_stream(),
-                                   static_cast<const uint16_t*>(dy.ptr()), static_cast<const uint16_t*>(x.ptr()), rinv,
-                                   static_cast<const float*>(w.ptr()), static_cast<const uint16_t*>(addend->ptr()),
-                                   static_cast<uint16_t*>(dx->ptr()), static_cast<float*>(part.p), x.rows, C);
+                passes(std::true_type{});
             else
-                hipLaunchKernelGGL((rms_bwd_dx_dw8<NP, false>), dim3(nparts), dim3(512), lds, tape_stream(),
-                                   static_cast<const uint16_t*>(dy.ptr()), static_cast<const uint16_t*>(x.ptr()), rinv,
-                                   static_cast<const float*>(w.ptr()), static_cast<const uint16_t*>(nullptr),
-                                   static_cast<uint16_t*>(dx->ptr()), static_cast<float*>(part.p), x.rows, C);
-        };
-        if (C <= 512)
-            launch(std::integral_constant<int, 1>{});
-        else if (C <= 1024)
-            launch(std::integral_constant<int, 2>{});
-        else
-            launch(std::integral_constant<int, 4>{});
+                passes(std::false_type{});
+        })
         post();
         hipLaunchKernelGGL(colsum_parts, dim3((C + 63) / 64), dim3(1024), 0, tape_stream(),
                            static_cast<const float*>(part.p), static_cast<float*>(dw->ptr()), nparts, C);
@@ -1297,6 +1407,12 @@ void k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable) {
     if (dy.rows > (1 << 30)) shape_fail("embedding: more than 2^30 rows");
     const int n = static_cast<int>(dy.rows), d = static_cast<int>(dy.cols);
     const hipStream_t st = tape_stream();
+    if (n <= EMB_SCAN_MAX) {
+        PK_DISPATCH1(T, dy.dtype, hipLaunchKernelGGL((emb_bwd_scan<T>), dim3(n), dim3(NT), 0, st, static_cast<const T*>(dy.ptr()),
+                                                     ids, static_cast<float*>(dtable.ptr()), n, d));
+        post();
+        return;
+    }
     Buffer rows_in(sizeof(int) * n), rows_out(sizeof(int) * n), ids_out(sizeof(int) * n);
     int* const r_in = static_cast<int*>(rows_in.p);
     int* const r_out = static_cast<int*>(rows_out.p);
@@ -1370,16 +1486,20 @@ double k_sumsq_to_host(const Tensor& g) {
     const int nb = k_sumsq_parts(g, static_cast<double*>(part.p));
     return k_sum_f64_to_host(static_cast<const double*>(part.p), nb);
 }
+void k_clip_factor(const double* part_dev, int n, float max_norm, float* factor_dev, float* norm_pinned) {
+    hipLaunchKernelGGL(clip_factor_k, dim3(1), dim3(NT), 0, tape_stream(), part_dev, n, max_norm, factor_dev, norm_pinned);
+    post();
+}
+void k_word_to_pinned(const void* src, void* pinned) {
+    hipLaunchKernelGGL(copy_word_k, dim3(1), dim3(1), 0, tape_stream(), static_cast<const uint32_t*>(src),
+                       static_cast<uint32_t*>(pinned));
+    post();
+}
 void k_adamw(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, float lr, float b1, float b2,
-             float eps, float wd, float c1, float c2, float grad_scale) {
-    if (grad_scale != 1.0f)
-        hipLaunchKernelGGL(adamw_k<true>, ew_grid(p.numel()), dim3(NT), 0, tape_stream(), static_cast<float*>(p.ptr()),
-                           static_cast<float*>(g.ptr()), static_cast<float*>(m.ptr()), static_cast<float*>(v.ptr()), lr, b1,
-                           b2, eps, wd, c1, c2, grad_scale, p.numel());
-    else
-        hipLaunchKernelGGL(adamw_k<false>, ew_grid(p.numel()), dim3(NT), 0, tape_stream(), static_cast<float*>(p.ptr()),
-                           static_cast<float*>(g.ptr()), static_cast<float*>(m.ptr()), static_cast<float*>(v.ptr()), lr, b1,
-                           b2, eps, wd, c1, c2, 1.0f, p.numel());
+             float eps, float wd, float c1, float c2, const float* clip_dev) {
+    hipLaunchKernelGGL(adamw_k, ew_grid(p.numel()), dim3(NT), 0, tape_stream(), static_cast<float*>(p.ptr()),
+                       static_cast<float*>(g.ptr()), static_cast<float*>(m.ptr()), static_cast<float*>(v.ptr()), lr, b1, b2,
+                       eps, wd, c1, c2, clip_dev, p.numel());
     post();
 }
 

@@ -56,6 +56,99 @@ Var make_param(int64_t r, int64_t c, const std::vector<float>& host) {
     return v;
 }
 
+// A device slab read back into many host arrays. One blocking copy per array from pageable memory runs at about
+// 7 GB/s (141 MB of a 35 M parameter model took 20 ms): the runtime copies through its own staging on one thread, and
+// that thread also takes the page faults of freshly allocated arrays. Here the slab comes down in chunks through pinned
+// staging, and several host threads, each with two chunks of its own, copy them out while the next ones arrive (the
+// link moves 141 MB in 2.5 ms, one thread copies it into fresh pages in 10 ms, eight in 2 ms).
+class SlabReader {
+public:
+    static constexpr int64_t CHUNK = int64_t{1} << 18;  // floats: 1 MiB
+    static constexpr int MAX_THREADS = 8;               // so the staging is at most 16 MiB
+    SlabReader() = default;
+    SlabReader(const SlabReader&) = delete;
+    SlabReader& operator=(const SlabReader&) = delete;
+    ~SlabReader() {
+        if (staging_) (void)hipHostFree(staging_);
+    }
+    struct Piece {
+        int64_t begin, count;  // floats of the slab, ascending and disjoint
+        float* host;
+    };
+    void read(const float* slab, const std::vector<Piece>& pieces, hipStream_t stream) {
+        if (pieces.empty()) return;
+        const int64_t total = pieces.back().begin + pieces.back().count, chunks = (total + CHUNK - 1) / CHUNK;
+        // a thread costs about as much to start as it takes to copy a chunk: two chunks or more for each
+        const int hw = std::max(1, static_cast<int>(std::thread::hardware_concurrency()));
+        const int threads = static_cast<int>(std::clamp<int64_t>(chunks / 2, 1, std::min(hw, MAX_THREADS)));
+        reserve(static_cast<size_t>(threads) * 2);
+        int device = 0;
+        hip_check(hipGetDevice(&device), "hipGetDevice");
+        std::vector<std::exception_ptr> failed(threads);
+        auto work = [&](int w) {
+            try {
+                hip_check(hipSetDevice(device), "hipSetDevice");
+                copy_out(slab, pieces, total, chunks, w, threads, stream);
+            } catch (...) {
+                failed[w] = std::current_exception();
+            }
+        };
+        std::vector<std::thread> pool;
+        try {
+            for (int w = 1; w < threads; ++w) pool.emplace_back(work, w);
+        } catch (...) {  // no more threads to be had: their chunks are copied here
+            for (int w = static_cast<int>(pool.size()) + 1; w < threads; ++w) work(w);
+        }
+        work(0);
+        for (auto& t : pool) t.join();
+        for (const auto& e : failed)
+            if (e) std::rethrow_exception(e);
+    }
+
+private:
+    float* staging_ = nullptr;
+    size_t chunks_ = 0;
+    void reserve(size_t chunks) {
+        if (chunks <= chunks_) return;
+        if (staging_) hip_check(hipHostFree(staging_), "hipHostFree");
+        staging_ = nullptr;
+        chunks_ = 0;
+        void* p = nullptr;
+        hip_check(hipHostMalloc(&p, sizeof(float) * CHUNK * chunks, hipHostMallocDefault), "hipHostMalloc");
+        staging_ = static_cast<float*>(p);
+        chunks_ = chunks;
+    }
+    // worker w's share, chunks w, w + threads, ...: the next one is on its way while the present one is copied out
+    void copy_out(const float* slab, const std::vector<Piece>& pieces, int64_t total, int64_t chunks, int w, int threads,
+                  hipStream_t stream) {
+        struct Event {
+            hipEvent_t e = nullptr;
+            Event() { hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate"); }
+            ~Event() { (void)hipEventDestroy(e); }
+        } arrived[2];
+        auto fetch = [&](int64_t c, int slot) {
+            const int64_t n = std::min(CHUNK, total - c * CHUNK);
+            hip_check(hipMemcpyAsync(staging_ + (2 * w + slot) * CHUNK, slab + c * CHUNK, sizeof(float) * n,
+                                     hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+            hip_check(hipEventRecord(arrived[slot].e, stream), "hipEventRecord");
+        };
+        int slot = 0;
+        fetch(w, 0);
+        for (int64_t c = w; c < chunks; c += threads, slot ^= 1) {
+            if (c + threads < chunks) fetch(c + threads, slot ^ 1);
+            hip_check(hipEventSynchronize(arrived[slot].e), "hipEventSynchronize");
+            const float* src = staging_ + (2 * w + slot) * CHUNK;
+            const int64_t lo = c * CHUNK, hi = std::min(lo + CHUNK, total);
+            auto p = std::upper_bound(pieces.begin(), pieces.end(), lo,
+                                      [](int64_t v, const Piece& q) { return v < q.begin + q.count; });
+            for (; p != pieces.end() && p->begin < hi; ++p) {
+                const int64_t from = std::max(lo, p->begin), to = std::min(hi, p->begin + p->count);
+                std::memcpy(p->host + (from - p->begin), src + (from - lo), sizeof(float) * (to - from));
+            }
+        }
+    }
+};
+
 struct Block {
     Var ln1_w, ln2_w, q, k, v, o, gate, up, down;
 };
@@ -357,19 +450,18 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         if (n % sl != 0) shape_fail("ids not a multiple of seq_len");
         k_fill(m->gslab, 0.0f);  // zero_grad: every parameter's gradient is a view of this slab
         // ids, targets and positions (which restart per sequence, llama.cpp:73-76) go up from pinned memory behind
-        // the fill, without a wait
+        // the fill, as one transfer and without a wait
         int* st = m->staging(static_cast<size_t>(3 * n + 1));
         std::memcpy(st, host_ids, sizeof(int) * n);
         std::memcpy(st + n, host_targets, sizeof(int) * n);
         for (int64_t i = 0; i < n; ++i) st[2 * n + i] = static_cast<int>(i % sl);
-        auto up = [&](const int* src) {
-            auto b = std::make_shared<Buffer>(sizeof(int) * n);
-            hip_check(hipMemcpyAsync(b->p, src, sizeof(int) * n, hipMemcpyHostToDevice, tape_stream()), "hipMemcpyAsync");
-            return b;
+        auto sent = std::make_shared<Buffer>(sizeof(int) * 3 * n);
+        hip_check(hipMemcpyAsync(sent->p, st, sizeof(int) * 3 * n, hipMemcpyHostToDevice, tape_stream()), "hipMemcpyAsync");
+        auto third = [&](int k) {  // a view that keeps the whole transfer's memory
+            return std::shared_ptr<Buffer>(new Buffer(static_cast<int*>(sent->p) + k * n, sizeof(int) * n),
+                                           [sent](Buffer* b) { delete b; });
         };
-        auto ids = up(st);
-        auto tg = up(st + n);
-        auto pos_dev = up(st + 2 * n);
+        auto ids = third(0), tg = third(1), pos_dev = third(2);
         // Everything allocated from here on, until backward returns, is activation memory.
         if (compute_dtype() != PK_F32) {  // build the bf16 parameter shadows first: they are not activations
             for (const auto& b : m->blocks) {
@@ -395,7 +487,7 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         if (do_backward) backward(l);
         // the loss comes back into the pinned staging's spare word behind the last kernel: one wait ends the pass
         float* hl = reinterpret_cast<float*>(st + 3 * n);
-        hip_check(hipMemcpyAsync(hl, l->data.ptr(), 4, hipMemcpyDeviceToHost, tape_stream()), "hipMemcpyAsync");
+        k_word_to_pinned(l->data.ptr(), hl);
         hip_check(hipStreamSynchronize(tape_stream()), "hipStreamSynchronize");
         if (stats) stats->peak_activation_bytes = static_cast<int64_t>(dev_peak_bytes() - base);
         *loss = *hl;
@@ -410,25 +502,27 @@ int pk_llama_adamw_step(void* h, float lr, float b1, float b2, float eps, float 
             k_fill(m->mslab, 0.0f);
             k_fill(m->vslab, 0.0f);
         }
-        // ops::clip_grad_norm over the slab (the padding between parameters is zero): double
-        // accumulation as the reference (ops.cpp:1047-1053), one host round trip.
-        double tn = 0.0;
-        float clip = 1.0f;
+        // ops::clip_grad_norm over the slab (the padding between parameters is zero), in double as the reference
+        // (ops.cpp:1047-1053); the AdamW pass applies it, and the norm reaches the host with the wait at the end
+        std::unique_ptr<Buffer> clip;
+        float* const norm = reinterpret_cast<float*>(m->staging(1));
+        *norm = 0.0f;
         if (max_norm > 0.0f) {
             Buffer parts(sizeof(double) * SUMSQ_MAX_PARTS);
+            clip = std::make_unique<Buffer>(sizeof(float));
             const int nb = k_sumsq_parts(m->gslab, static_cast<double*>(parts.p));
-            tn = std::sqrt(k_sum_f64_to_host(static_cast<const double*>(parts.p), nb));
-            if (tn > max_norm && tn > 0.0) clip = static_cast<float>(max_norm / tn);  // applied by the AdamW pass
+            k_clip_factor(static_cast<const double*>(parts.p), nb, max_norm, static_cast<float*>(clip->p), norm);
         }
-        if (total_norm) *total_norm = static_cast<float>(tn);
         ++m->t;
         const float c1 = 1.0f - std::pow(b1, static_cast<float>(m->t));
         const float c2 = 1.0f - std::pow(b2, static_cast<float>(m->t));
         // every parameter of this model receives a gradient each step, so the reference's "skip a
         // parameter that never accumulated" (nn.cpp:309) never applies; padding stays at zero
-        k_adamw(m->pslab, m->gslab, m->mslab, m->vslab, lr, b1, b2, eps, wd, c1, c2, clip);
+        k_adamw(m->pslab, m->gslab, m->mslab, m->vslab, lr, b1, b2, eps, wd, c1, c2,
+                clip ? static_cast<const float*>(clip->p) : nullptr);
         refresh_shadows();  // the bf16 copies of the weights follow them, in one launch
         hip_check(hipStreamSynchronize(tape_stream()), "hipStreamSynchronize");
+        if (total_norm) *total_norm = *norm;
     });
 }
 

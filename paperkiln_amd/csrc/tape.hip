@@ -347,7 +347,7 @@ void backward(const Var& root) {
     Tensor seed = Tensor::make(1, 1, root->data.dtype);
     k_fill(seed, 1.0f);
     const bool fresh = root->grad.empty();
-    root->accumulate(seed);
+    root->accumulate_owned(std::move(seed));
     root->grad_is_unit = fresh;
     run_backward(root);
 }

@@ -61,9 +61,13 @@ double k_sumsq_to_host(const Tensor& g);                               // clip_g
 constexpr int SUMSQ_MAX_PARTS = 1024;
 int k_sumsq_parts(const Tensor& g, double* part_dev);
 double k_sum_f64_to_host(const double* part_dev, int64_t n);
-// grad_scale != 1: g is scaled in place first (the clip of ops::clip_grad_norm), in the same pass
+// What ops::clip_grad_norm multiplies the gradients by (1 where the norm is within max_norm), from those partial sums,
+// left on the device for k_adamw; the norm itself goes to pinned host memory, to be read after a wait for the stream.
+void k_clip_factor(const double* part_dev, int n, float max_norm, float* factor_dev, float* norm_pinned);
+void k_word_to_pinned(const void* src, void* pinned);  // one float for the host, cheaper than a copy
+// clip_dev (may be null): g is scaled in place by *clip_dev first, in the same pass
 void k_adamw(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, float lr, float b1, float b2,
-             float eps, float wd, float c1, float c2, float grad_scale = 1.0f);                 // nn.cpp:301-321
+             float eps, float wd, float c1, float c2, const float* clip_dev = nullptr);         // nn.cpp:301-321
 
 // C[M,N] (+)= op(A) . op(B), row-major, bf16 or fp32 operands, fp32 accumulate
 // (device::gemm, src/device.cpp:91-125). C may be a column slice of a wider
