@@ -241,6 +241,10 @@ __device__ inline void st8(uint16_t* p, int64_t e, const F8& x) {
     const u32x4 r = {pack_bf16(x.v[0], x.v[1]), pack_bf16(x.v[2], x.v[3]), pack_bf16(x.v[4], x.v[5]), pack_bf16(x.v[6], x.v[7])};
     *reinterpret_cast<u32x4*>(p + e) = r;
 }
+__device__ inline void st8(float* p, int64_t e, const F8& x) {
+    *reinterpret_cast<f32x4*>(p + e) = f32x4{x.v[0], x.v[1], x.v[2], x.v[3]};
+    *reinterpret_cast<f32x4*>(p + e + 4) = f32x4{x.v[4], x.v[5], x.v[6], x.v[7]};
+}
 #define PK_EW8_LOOP(i, n8) \
     for (int64_t i = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x; i < (n8); i += static_cast<int64_t>(gridDim.x) * NT)
 template <int OP>
@@ -720,16 +724,18 @@ __global__ void cast_cols_k(const TA* src, TY* dst, int64_t rows, int64_t cols, 
         stf(dst, (i / cols) * ld + off + i % cols, ldf(src, i));
 }
 
-// Many casts of fp32 matrices into column blocks of bf16 matrices as one launch (the refresh of every compute-dtype
-// weight copy after an optimizer step): job j covers blocks [block_begin[j], block_begin[j + 1]), eight elements a thread.
+// Many casts of fp32 matrices into column blocks of bf16 or fp32 matrices as one launch (the refresh of every
+// compute-dtype weight copy after an optimizer step): job j covers blocks [block_begin[j], block_begin[j + 1]), eight
+// elements a thread.
 struct CastJobs {
     static constexpr int MAX = 64;
     int count;
     int block_begin[MAX + 1];
     const float* src[MAX];
-    uint16_t* dst[MAX];
+    void* dst[MAX];
     int rows[MAX], cols[MAX], ld[MAX], off[MAX];
 };
+template <typename TY>
 __global__ void cast_jobs_k(CastJobs jobs) {
     int j = 0;
     while (static_cast<int>(blockIdx.x) >= jobs.block_begin[j + 1]) ++j;
@@ -738,7 +744,7 @@ __global__ void cast_jobs_k(CastJobs jobs) {
     const int64_t i = (static_cast<int64_t>(blockIdx.x) - jobs.block_begin[j]) * NT + threadIdx.x;
     if (i >= n8) return;
     const int64_t e = i * 8, r = e / cols, c = e - r * cols;
-    st8(jobs.dst[j], r * jobs.ld[j] + jobs.off[j] + c, ld8(jobs.src[j], e));
+    st8(static_cast<TY*>(jobs.dst[j]), r * jobs.ld[j] + jobs.off[j] + c, ld8(jobs.src[j], e));
 }
 
 // apply_rope (ops.cpp:497-509 forward, :519-533 backward = rotation by -theta).
@@ -1115,11 +1121,12 @@ void k_cast_cols(const Tensor& src, const Tensor& dst, int64_t col_off) {
                                     dst.cols, col_off)));
     post();
 }
-// dst_k[:, off_k : off_k + cols_k] = bf16(src_k) for every job, one launch per 64 jobs. False, with nothing done,
-// if a job is not an fp32 -> bf16 cast with column counts and offsets that are multiples of 8 (the caller casts one by one).
+// dst_k[:, off_k : off_k + cols_k] = src_k for every job, one launch per 64 jobs. False, with nothing done, if a job is not
+// a cast from fp32 with column counts and offsets that are multiples of 8, or if the destinations' types differ (the caller
+// casts one by one).
 bool k_cast_many(const std::vector<CastJob>& list) {
     for (const CastJob& c : list)
-        if (c.src.dtype != PK_F32 || c.dst.dtype != PK_BF16 || c.src.cols % 8 || c.dst.cols % 8 || c.col_off % 8 ||
+        if (c.src.dtype != PK_F32 || c.dst.dtype != list[0].dst.dtype || c.src.cols % 8 || c.dst.cols % 8 || c.col_off % 8 ||
             c.src.rows != c.dst.rows || c.col_off < 0 || c.col_off + c.src.cols > c.dst.cols ||
             c.src.numel() / 8 > (int64_t{1} << 30) || !aligned16p(c.src.ptr()) || !aligned16p(c.dst.ptr()))
             return false;
@@ -1132,7 +1139,7 @@ bool k_cast_many(const std::vector<CastJob>& list) {
             const int k = jobs.count++;
             jobs.block_begin[k] = blocks;
             jobs.src[k] = static_cast<const float*>(c.src.ptr());
-            jobs.dst[k] = static_cast<uint16_t*>(c.dst.ptr());
+            jobs.dst[k] = c.dst.ptr();
             jobs.rows[k] = static_cast<int>(c.src.rows);
             jobs.cols[k] = static_cast<int>(c.src.cols);
             jobs.ld[k] = static_cast<int>(c.dst.cols);
@@ -1141,7 +1148,8 @@ bool k_cast_many(const std::vector<CastJob>& list) {
         }
         for (int k = jobs.count; k <= CastJobs::MAX; ++k) jobs.block_begin[k] = blocks;
         if (blocks > 0) {
-            hipLaunchKernelGGL(cast_jobs_k, dim3(static_cast<unsigned>(blocks)), dim3(NT), 0, tape_stream(), jobs);
+            PK_DISPATCH1(TY, list[0].dst.dtype, hipLaunchKernelGGL((cast_jobs_k<TY>), dim3(static_cast<unsigned>(blocks)), dim3(NT),
+                                                                   0, tape_stream(), jobs));
             post();
         }
     }
@@ -1533,6 +1541,14 @@ std::atomic<int> g_head_in_product{1};
 void set_head_kernel(int in_product) { g_head_in_product.store(in_product != 0, std::memory_order_relaxed); }
 int head_kernel() { return g_head_in_product.load(std::memory_order_relaxed); }
 
+// Which fp32 products the hand-written kernel gets when they come one by one: those that are over in about the time that
+// the library needs to launch one (2048 x 1000 x 128: 10.4 us against 8.8), and weight gradients over up to 2048 tokens,
+// which it computes faster than the library or level with it at every size measured (1001 x 128 x 2048: 13 us against
+// 27; 512 x 1536 x 2048: 38 against 35); beyond, the library.
+bool gemm_f32_is_ahead(bool tA, int64_t M, int64_t N, int64_t K) {
+    return M * N * K <= (int64_t{1} << 28) || (tA && K <= 2048);
+}
+
 void gemm(const Tensor& A, bool tA, const Tensor& B, bool tB, void* C, int c_dtype, int64_t M, int64_t N, int64_t ldc,
           float beta, int64_t lda) {
     if (lda == 0) lda = A.cols;
@@ -1549,6 +1565,11 @@ void gemm(const Tensor& A, bool tA, const Tensor& B, bool tB, void* C, int c_dty
     if (A.dtype == PK_BF16 && mine &&
         gemm_mfma_bf16(A.ptr(), tA, lda, B.ptr(), tB, B.cols, C, c_dtype, M, N, Ka, ldc, beta, tape_stream()))
         return;
+    if (A.dtype == PK_F32 && c_dtype == PK_F32 && mine && gemm_f32_is_ahead(tA, M, N, Ka)) {
+        const F32Product p{static_cast<const float*>(A.ptr()), lda, static_cast<const float*>(B.ptr()), B.cols,
+                           static_cast<float*>(C), ldc, nullptr, M, N, Ka};
+        if (gemm_f32(&p, 1, tA, tB, beta, tape_stream())) return;
+    }
     // Row-major C = op(A) op(B)  <=>  column-major C^T = op(B)^T op(A)^T.
     const rocblas_datatype ab = A.dtype == PK_F32 ? rocblas_datatype_f32_r : rocblas_datatype_bf16_r;
     const rocblas_datatype ct = c_dtype == PK_F32 ? rocblas_datatype_f32_r : rocblas_datatype_bf16_r;

@@ -1,0 +1,261 @@
+// The fp32 matrix product on the matrix cores (v_mfma_f32_32x32x2_f32): C = op(A) op(B) (+ C or an addend), row-major, up
+// to eight products in one launch.
+//
+// The fp32 matrix rate is a sixteenth of the bf16 one: a wavefront's 32 x 32 block needs 8 bytes a cycle, which L1 and L2
+// deliver without LDS. Fragments are therefore loaded from global memory straight into the layout the instruction reads,
+// two chunks of the contraction ahead of the multiplications, and there is no barrier in the loop. What bounds a small
+// product is latency, and that a projection of a few hundred tokens has 16 to 200 blocks of 32 x 32 for 1024 SIMDs: the
+// wavefronts of a workgroup split the contraction and add their accumulators through LDS at the end, in a fixed order.
+//
+// Against the library, which serves the larger products (GPU time, 512 tokens of width 128): 3.8 us and 3.9 for the
+// fused q/k/v projection, 5.2 and 6.0 for the down projection; but a launch here costs the host 3 us, not 10 to 25, sums
+// an addend on the way out, and takes all the weight gradients of a block together. 2048 tokens of width 512 against
+// 1536 columns: 45 us and 28.
+#include "mfma_common.h"
+#include "tensor.h"
+
+#include <algorithm>
+
+namespace pk {
+namespace {
+
+struct Jobs {
+    static constexpr int MAX = 8;
+    int count;
+    int first[MAX + 1];  // job j's tiles are first[j] .. first[j + 1] - 1
+    const float* a[MAX];
+    const float* b[MAX];
+    float* c[MAX];
+    const float* addend[MAX];
+    int lda[MAX], ldb[MAX], ldc[MAX], M[MAX], N[MAX], K[MAX];
+};
+
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // a row may start at any element
+
+// One chunk of KC steps of the contraction for NBLK blocks of 16 rows (of A) or columns (of B). The instruction takes four
+// steps, one for each 16 lanes. Which four does not matter as long as A and B agree: lanes 16 g .. 16 g + 15 take steps
+// 4 g .. 4 g + 3 of every 16, so that a row of an operand whose steps are adjacent is read 64 bytes at a time, 16 bytes a
+// lane. (With the 32 x 32 instruction, whose two steps leave a lane's 16 bytes alone in their line, the loads kept the
+// CU's address unit busy for twice as long as the multiplications took.)
+// ROWS: element (k, i) is p[k ld + i], otherwise p[i ld + k]. off: the lane's byte offset of step 4 g of a chunk at step 0;
+// k0: the chunk's first step. Everything that changes from load to load is in scalar registers.
+template <bool ROWS, int NBLK, int KC>
+__device__ inline void load_chunk(__amdgpu_buffer_rsrc_t p, int ld, const int (&off)[NBLK], int k0, float (&f)[NBLK][KC / 4]) {
+#pragma unroll
+    for (int s = 0; s < KC / 4; s += 4)
+#pragma unroll
+        for (int b = 0; b < NBLK; ++b) {
+            if (ROWS) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    f[b][s + e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(p, off[b], (k0 + 4 * s + e) * ld * 4, 0));
+            } else {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(p, off[b] + 16 * s, k0 * 4, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[b][s + e] = __uint_as_float(v[e]);
+            }
+        }
+}
+// The same where the contraction is shorter than a chunk: zeros past its end.
+template <bool ROWS, int NBLK, int KC>
+__device__ inline void load_short(const float* p, int64_t ld, const int (&idx)[NBLK], int k0, int K, float (&f)[NBLK][KC / 4]) {
+#pragma unroll
+    for (int b = 0; b < NBLK; ++b)
+#pragma unroll
+        for (int s = 0; s < KC / 4; ++s) {
+            const int at = k0 + 4 * (s & ~3) + (s & 3), k = min(at, K - 1);
+            const float v = ROWS ? p[k * ld + idx[b]] : p[idx[b] * ld + k];
+            f[b][s] = at < K ? v : 0.0f;
+        }
+}
+
+__host__ __device__ inline int64_t extent(int64_t rows, int64_t cols, int64_t ld) { return ((rows - 1) * ld + cols) * 4; }
+__device__ inline int bytes_of(int rows, int cols, int64_t ld) { return static_cast<int>(extent(rows, cols, ld)); }
+
+// A workgroup's tile is MB x NB blocks of 16 x 16; its KW wavefronts split the contraction chunk by chunk.
+template <bool TA, bool TB, int MB, int NB, int KW>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs jobs, const int tiles, const float beta) {
+    constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB, TN = 16 * NB;
+    // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
+    const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (t >= tiles) return;
+    int j = 0;
+    while (t >= jobs.first[j + 1]) ++j;
+    const int M = jobs.M[j], N = jobs.N[j], K = jobs.K[j];
+    const int tn = (N + TN - 1) / TN, m0 = ((t - jobs.first[j]) / tn) * TM, n0 = ((t - jobs.first[j]) % tn) * TN;
+    const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, grp = lane >> 4;
+    const float* const a = jobs.a[j];
+    const float* const b = jobs.b[j];
+    const int64_t lda = jobs.lda[j], ldb = jobs.ldb[j];
+    int row[MB], col[NB];  // rows and columns past the edge read the last one; they are not stored
+#pragma unroll
+    for (int i = 0; i < MB; ++i) row[i] = min(m0 + i * 16 + l16, M - 1);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) col[i] = min(n0 + i * 16 + l16, N - 1);
+
+    f32x4 acc[MB][NB];
+#pragma unroll
+    for (int x = 0; x < MB; ++x)
+#pragma unroll
+        for (int y = 0; y < NB; ++y) acc[x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a), 0, bytes_of(TA ? K : M, TA ? M : K, lda), 0x00020000);
+    const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(b), 0, bytes_of(TB ? N : K, TB ? K : N, ldb), 0x00020000);
+    int oa[MB], ob[NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) oa[i] = static_cast<int>(TA ? 4 * grp * lda + row[i] : row[i] * lda + 4 * grp) * 4;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) ob[i] = static_cast<int>(TB ? col[i] * ldb + 4 * grp : 4 * grp * ldb + col[i]) * 4;
+    float fa[BUFS][MB][KC / 4], fb[BUFS][NB][KC / 4];
+    const int chunks = (K + KC - 1) / KC;
+    auto load = [&](int chunk, int buf) {
+        const int over = max((chunk + 1) * KC - K, 0), k0 = chunk * KC - over;
+        if (over == 0) {
+            load_chunk<TA, MB, KC>(ra, jobs.lda[j], oa, k0, fa[buf]);
+            load_chunk<!TB, NB, KC>(rb, jobs.ldb[j], ob, k0, fb[buf]);
+        } else if (K >= KC) {  // the last chunk, moved back to end where the contraction does: its first steps are done already
+            load_chunk<TA, MB, KC>(ra, jobs.lda[j], oa, k0, fa[buf]);
+            load_chunk<!TB, NB, KC>(rb, jobs.ldb[j], ob, k0, fb[buf]);
+#pragma unroll
+            for (int s = 0; s < KC / 4; ++s) {
+                const bool done = 4 * grp + 4 * (s & ~3) + (s & 3) < over;
+#pragma unroll
+                for (int x = 0; x < MB; ++x) fa[buf][x][s] = done ? 0.0f : fa[buf][x][s];
+#pragma unroll
+                for (int y = 0; y < NB; ++y) fb[buf][y][s] = done ? 0.0f : fb[buf][y][s];
+            }
+        } else {
+            load_short<TA, MB, KC>(a, lda, row, 4 * grp, K, fa[buf]);
+            load_short<!TB, NB, KC>(b, ldb, col, 4 * grp, K, fb[buf]);
+        }
+    };
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int s = 0; s < KC / 4; ++s)
+#pragma unroll
+            for (int x = 0; x < MB; ++x)
+#pragma unroll
+                for (int y = 0; y < NB; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[buf][x][s], fb[buf][y][s], acc[x][y], 0, 0, 0);
+    };
+    const int mine = kw < chunks ? (chunks - kw + KW - 1) / KW : 0;  // chunks kw, kw + KW, ... are this wavefront's
+#pragma unroll
+    for (int u = 0; u < BUFS; ++u)
+        if (u < mine) load(kw + u * KW, u);
+    __builtin_amdgcn_sched_barrier(0);
+    int i = 0;
+    for (; i + BUFS <= mine; i += BUFS) {
+#pragma unroll
+        for (int u = 0; u < BUFS; ++u) {
+            multiply(u);
+            if (i + u + BUFS < mine) load(kw + (i + u + BUFS) * KW, u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < BUFS - 1; ++u)
+        if (i + u < mine) multiply(u);
+
+    const float* const add = jobs.addend[j] ? jobs.addend[j] : beta != 0.0f ? jobs.c[j] : nullptr;
+    float* const out = jobs.c[j];
+    const int64_t ldc = jobs.ldc[j];
+    auto store = [&](int x, int y, f32x4 v) {
+        const int n = n0 + y * 16 + l16;
+        if (n >= N) return;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + x * 16 + 4 * grp + r;
+            if (m < M) {
+                const int64_t o = m * ldc + n;
+                out[o] = add ? add[o] + v[r] : v[r];
+            }
+        }
+    };
+    __shared__ f32x4 part[KW][MB * NB][64];
+#pragma unroll
+    for (int x = 0; x < MB; ++x)
+#pragma unroll
+        for (int y = 0; y < NB; ++y) part[kw][x * NB + y][lane] = acc[x][y];
+    __syncthreads();
+#pragma unroll
+    for (int g0 = 0; g0 < MB * NB; g0 += KW) {
+        const int g = g0 + kw;
+        if (g < MB * NB) {
+            f32x4 s = part[0][g][lane];
+#pragma unroll
+            for (int k = 1; k < KW; ++k) s += part[k][g][lane];
+            store(g / NB, g % NB, s);
+        }
+    }
+}
+
+template <bool TA, bool TB, int MB, int NB, int KW>
+void launch(Jobs& jobs, float beta, hipStream_t st) {
+    constexpr int TM = 16 * MB, TN = 16 * NB;
+    int tiles = 0;
+    for (int j = 0; j < jobs.count; ++j) {
+        jobs.first[j] = tiles;
+        tiles += ((jobs.M[j] + TM - 1) / TM) * ((jobs.N[j] + TN - 1) / TN);
+    }
+    for (int j = jobs.count; j <= Jobs::MAX; ++j) jobs.first[j] = tiles;
+    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
+                       tiles, beta);
+    hip_check(hipGetLastError(), "gemm_f32");
+}
+
+// Which tile: a 32 x 32 one keeps more CUs busy, a 64 x 64 one reads its operands half as often. Measured on projections,
+// heads and weight gradients of 64 to 8192 tokens: with more than 640 of the small tiles (2.5 to a CU) the large one is
+// ahead (2048 x 1000 x 128: 10.4 us against 15.7), except for weight gradients, whose long contraction the small one walks
+// with more wavefronts (512 x 1536 x 8192: 117 us against 152). With a tile or less to a CU, eight wavefronts split the
+// contraction instead of four.
+template <bool TA, bool TB>
+void launch_by_size(Jobs& jobs, float beta, hipStream_t st) {
+    int64_t tiles = 0;
+    int longest = 0;
+    for (int j = 0; j < jobs.count; ++j) {
+        tiles += static_cast<int64_t>((jobs.M[j] + 31) / 32) * ((jobs.N[j] + 31) / 32);
+        longest = std::max(longest, jobs.K[j]);
+    }
+    if (tiles > 640 && (!TA || longest < 256))
+        launch<TA, TB, 4, 4, 4>(jobs, beta, st);
+    else if (tiles <= 256 && longest >= 256)
+        launch<TA, TB, 2, 2, 8>(jobs, beta, st);
+    else
+        launch<TA, TB, 2, 2, 4>(jobs, beta, st);
+}
+
+}  // namespace
+
+bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
+    if (count < 1 || count > Jobs::MAX || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
+    Jobs jobs{};
+    jobs.count = count;
+    for (int j = 0; j < count; ++j) {
+        const F32Product& p = ps[j];
+        const int64_t limit = int64_t{1} << 30;
+        if (p.M <= 0 || p.N <= 0 || p.K <= 0 || p.M > limit || p.N > limit || p.K > limit || p.lda > limit || p.ldb > limit ||
+            p.ldc > limit)
+            return false;
+        if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= int64_t{1} << 31 || extent(tB ? p.N : p.K, tB ? p.K : p.N, p.ldb) >= int64_t{1} << 31)
+            return false;
+        jobs.a[j] = p.a;
+        jobs.b[j] = p.b;
+        jobs.c[j] = p.c;
+        jobs.addend[j] = p.addend;
+        jobs.lda[j] = static_cast<int>(p.lda);
+        jobs.ldb[j] = static_cast<int>(p.ldb);
+        jobs.ldc[j] = static_cast<int>(p.ldc);
+        jobs.M[j] = static_cast<int>(p.M);
+        jobs.N[j] = static_cast<int>(p.N);
+        jobs.K[j] = static_cast<int>(p.K);
+    }
+    if (tA)
+        launch_by_size<true, false>(jobs, beta, st);
+    else if (tB)
+        launch_by_size<false, true>(jobs, beta, st);
+    else
+        launch_by_size<false, false>(jobs, beta, st);
+    return true;
+}
+
+}  // namespace pk

@@ -463,15 +463,14 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         };
         auto ids = third(0), tg = third(1), pos_dev = third(2);
         // Everything allocated from here on, until backward returns, is activation memory.
-        if (compute_dtype() != PK_F32) {  // build the bf16 parameter shadows first: they are not activations
-            for (const auto& b : m->blocks) {
-                prepare_shadow_cat({b.q, b.k, b.v});
-                prepare_shadow(b.o);
-                prepare_shadow_cat({b.gate, b.up});
-                prepare_shadow(b.down);
-            }
-            prepare_shadow(m->embed);
+        // The copies of the parameters that the products read come first: they are not activations.
+        for (const auto& b : m->blocks) {
+            prepare_shadow_cat({b.q, b.k, b.v});
+            prepare_shadow(b.o);
+            prepare_shadow_cat({b.gate, b.up});
+            prepare_shadow(b.down);
         }
+        prepare_shadow(m->embed);
         const size_t base = dev_live_bytes();  // the allocator's host-side counters: nothing to wait for
         dev_reset_peak();
         const size_t live0 = live_variables();

@@ -120,23 +120,31 @@ void flush_weight_gradients() {
     auto& jobs = pending().jobs;
     size_t i = 0;
     while (i < jobs.size()) {
-        // a run of jobs with one token count
+        // a run of jobs of one element type, in bf16 also of one token count
+        const int dtype = jobs[i].x.dtype;
+        const int64_t K = jobs[i].x.rows;
         size_t j = i;
         GroupedProduct gp[8];
-        while (j < jobs.size() && j - i < 8 && jobs[j].x.rows == jobs[i].x.rows) {
+        F32Product fp[8];
+        while (j < jobs.size() && j - i < 8 && jobs[j].x.dtype == dtype && (dtype == PK_F32 || jobs[j].x.rows == K)) {
             const auto& job = jobs[j];
             Tensor& g = job.W->ensure_grad();
-            gp[j - i] = GroupedProduct{job.x.ptr(), job.x.cols,
-                                       static_cast<const char*>(job.dy.ptr()) + job.col0 * static_cast<int64_t>(job.dy.esize()),
-                                       job.dy.cols, static_cast<float*>(g.ptr()), g.cols, job.x.cols, job.ncols};
+            const char* dy = static_cast<const char*>(job.dy.ptr()) + job.col0 * static_cast<int64_t>(job.dy.esize());
+            float* const c = static_cast<float*>(g.ptr());
+            gp[j - i] = GroupedProduct{job.x.ptr(), job.x.cols, dy, job.dy.cols, c, g.cols, job.x.cols, job.ncols};
+            fp[j - i] = F32Product{static_cast<const float*>(job.x.ptr()), job.x.cols, reinterpret_cast<const float*>(dy),
+                                   job.dy.cols, c, g.cols, nullptr, job.x.cols, job.ncols, job.x.rows};
             ++j;
         }
-        const int64_t K = jobs[i].x.rows;
-        if (!gemm_mfma_grouped_tn(gp, static_cast<int>(j - i), K, tape_stream())) {
-            for (size_t k = 0; k < j - i; ++k)
+        const int count = static_cast<int>(j - i);
+        const char* const refused = "a deferred weight-gradient product was refused by the kernel it was queued for";
+        if (dtype == PK_F32) {
+            if (!gemm_f32(fp, count, true, false, 1.0f, tape_stream())) throw std::runtime_error(refused);
+        } else if (!gemm_mfma_grouped_tn(gp, count, K, tape_stream())) {
+            for (int k = 0; k < count; ++k)
                 if (!gemm_mfma_bf16(gp[k].a, true, gp[k].lda, gp[k].b, false, gp[k].ldb, gp[k].c, PK_F32, gp[k].M, gp[k].N, K,
                                     gp[k].ldc, 1.0f, tape_stream()))
-                    throw std::runtime_error("a deferred weight-gradient product was refused by the kernel it was queued for");
+                    throw std::runtime_error(refused);
         }
         i = j;
     }
@@ -144,11 +152,16 @@ void flush_weight_gradients() {
 }
 
 // Whether dW += x^T dy[:, col0 : col0 + ncols] can wait in the queue: a backward pass is running and the product is one
-// the hand-written kernel takes (bf16 operands, fp32 parameter gradient, aligned, a contraction worth grouping).
+// the hand-written kernels take (operands of one type, fp32 parameter gradient; in bf16 aligned, and a contraction worth
+// grouping).
 bool weight_gradient_can_wait(const Tensor& x, const Tensor& dy, int64_t col0, int64_t ncols, const Var& W) {
     if (pending().depth == 0 || gemm_backend() != 1) return false;
-    if (x.dtype != PK_BF16 || dy.dtype != PK_BF16 || !W->is_param || x.rows != dy.rows || x.rows < 2048) return false;
-    if (x.cols % 8 || dy.cols % 8 || col0 % 8 || ncols % 8 || W->data.rows != x.cols || W->data.cols != ncols) return false;
+    if (x.dtype != dy.dtype || !W->is_param || x.rows != dy.rows || W->data.rows != x.cols || W->data.cols != ncols) return false;
+    if (x.dtype == PK_BF16) {
+        if (x.rows < 2048 || x.cols % 8 || dy.cols % 8 || col0 % 8 || ncols % 8) return false;
+    } else if (x.numel() >= (int64_t{1} << 29) || dy.numel() >= (int64_t{1} << 29)) {
+        return false;
+    }
     return W->grad.empty() || W->grad.dtype == PK_F32;
 }
 void hold_weight_gradient(const Tensor& x, const Tensor& dy, int64_t col0, int64_t ncols, const Var& W) {
@@ -433,14 +446,21 @@ Var linear_add(const Var& x, const Var& W, const Var& r, bool result_needed) {
         shape_fail("add: shape mismatch");
     const Tensor& Wc = shadow_of(W);
     Tensor y = Tensor::make(x->data.rows, W->data.cols, x->data.dtype);
-    const bool contiguous = r->data.off_bytes % 16 == 0;
+    auto in_epilogue = [&] {
+        const int64_t M = y.rows, N = y.cols, K = x->data.cols;
+        if (gemm_backend() == 0 || x->data.dtype != Wc.dtype) return false;
+        if (x->data.dtype == PK_BF16)
+            return r->data.off_bytes % 16 == 0 && gemm_mfma_bf16(x->data.ptr(), false, K, Wc.ptr(), false, N, y.ptr(), y.dtype, M,
+                                                                 N, K, N, 1.0f, tape_stream(), r->data.ptr());
+        const F32Product p{static_cast<const float*>(x->data.ptr()), K, static_cast<const float*>(Wc.ptr()), N,
+                           static_cast<float*>(y.ptr()), N, static_cast<const float*>(r->data.ptr()), M, N, K};
+        return gemm_f32_is_ahead(false, M, N, K) && gemm_f32(&p, 1, false, false, 0.0f, tape_stream());
+    };
     // result_needed = false: the caller only wants the node (the last op of a segment that is being re-run for its
     // tape: the backward closure reads x, W and the node's gradient, never the node's value), so nothing is multiplied
     if (!result_needed && grad_enabled()) {
         // y stays as allocated: its shape is what the tape needs
-    } else if (!(x->data.dtype == PK_BF16 && Wc.dtype == PK_BF16 && gemm_backend() != 0 && contiguous &&
-          gemm_mfma_bf16(x->data.ptr(), false, x->data.cols, Wc.ptr(), false, Wc.cols, y.ptr(), y.dtype, y.rows, y.cols,
-                         x->data.cols, y.cols, 1.0f, tape_stream(), r->data.ptr()))) {
+    } else if (!in_epilogue()) {
         gemm(x->data, false, Wc, false, y.ptr(), y.dtype, y.rows, y.cols, y.cols, 0.0f);
         k_add(r->data, y, y);
     }

@@ -17,7 +17,7 @@ void hip_check(hipError_t e, const char* what);  // throws Error(PK_ERR_HIP), as
 void k_fill(const Tensor& y, float v);
 void k_cast(const Tensor& src, const Tensor& dst);                      // dtype conversion / copy
 void k_cast_cols(const Tensor& src, const Tensor& dst, int64_t col_off);
-// many such casts (fp32 -> a column block of a bf16 matrix) as one launch; false = not applicable, nothing done
+// many such casts (fp32 -> a column block of a bf16 or fp32 matrix) as one launch; false = not applicable, nothing done
 struct CastJob {
     Tensor src, dst;
     int64_t col_off;
@@ -99,6 +99,21 @@ struct GroupedProduct {
     int64_t M, N;
 };
 bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStream_t st);
+// gemm_f32.hip: C_p = op(A_p) op(B_p) + (addend_p, or C_p if beta is 1) for up to eight products of one orientation in one
+// launch, fp32 throughout on the matrix cores; any sizes and row pitches. False, with nothing done, if A and B are both
+// transposed or an operand has 2 GiB or more.
+struct F32Product {
+    const float* a;
+    int64_t lda;
+    const float* b;
+    int64_t ldb;
+    float* c;
+    int64_t ldc;
+    const float* addend;  // row pitch ldc; may be null
+    int64_t M, N, K;
+};
+bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st);
+bool gemm_f32_is_ahead(bool tA, int64_t M, int64_t N, int64_t K);  // of the library, for one product of this size
 int64_t gemm_head_spans(int64_t N);
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,

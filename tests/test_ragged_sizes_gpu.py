@@ -111,3 +111,44 @@ def test_fp32_split_kernels(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.float32, causal, window, sinks))
     assert max(e) < 5e-6, e
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 65, 31), (64, 32, 33), (31, 97, 344), (1, 40, 1001), (900, 1030, 70)])
+def test_fp32_products(M, N, K, tA, tB):
+    """The hand-written fp32 GEMM at the edges of its tiles (32 and, from 640 of those on, 64), of its contraction chunks
+    and of the split of the contraction among wavefronts, with and without the sum onto C. Against float64."""
+    import ctypes as C
+
+    from paperkiln_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b = (torch.randn(s, generator=gen, device="cuda") for s in ((K, M) if tA else (M, K), (N, K) if tB else (K, N)))
+    c0 = torch.randn((M, N), generator=gen, device="cuda")
+    want = (a.double().T if tA else a.double()) @ (b.double().T if tB else b.double())
+    for accumulate in (0, 1):
+        c = c0.clone()
+        _lib.check(_lib.lib().pk_op_gemm(C.c_void_p(a.data_ptr()), tA, C.c_void_p(b.data_ptr()), tB, C.c_void_p(c.data_ptr()),
+                                         M, N, K, _lib.PK_F32, _lib.PK_F32, accumulate, None))
+        torch.cuda.synchronize()
+        err = (c.double() - want - accumulate * c0.double()).abs().max()
+        assert err < 4e-7 * (K + 16) ** 0.5 * 4, (accumulate, float(err))
+
+
+@pytest.mark.parametrize("vocab,d,ff,tokens,seq", [(101, 64, 176, 77, 11), (301, 96, 256, 700, 100), (130, 64, 176, 4100, 820)])
+def test_fp32_training_on_ragged_sizes(vocab, d, ff, tokens, seq):
+    """A whole fp32 pass (weight gradients of a block in one launch, residual sums in the products, the embedding's
+    gradient with and without the sort) against the same pass on the library's GEMM."""
+    m = Llama(vocab=vocab, d=d, n_layers=2, n_heads=d // 32, d_ff=ff, compute_dtype="fp32", seed=8)
+    toks = synth.randint(3, tokens + 1, vocab)
+    before = blockops.set_gemm_backend(0)
+    try:
+        want_loss, _ = m.loss_backward(toks[:-1], toks[1:], seq)
+        want = m.grads()
+        blockops.set_gemm_backend(1)
+        for ck in (False, True):
+            loss, _ = m.loss_backward(toks[:-1], toks[1:], seq, checkpoint=ck)
+            assert abs(loss - want_loss) < 1e-5
+            assert rel(m.grads(), want) < 2e-5
+    finally:
+        blockops.set_gemm_backend(before)
+        m.close()
