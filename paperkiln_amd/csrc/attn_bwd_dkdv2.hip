@@ -375,13 +375,16 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
     }
 }
 
-// dK / dV rows [0, sinks) of every (batch, KV head) = the band part plus the chunks, in that order.
+// dK / dV rows [0, sinks) of every (batch, KV head) = the band part plus the chunks, in that order. One element a thread: a
+// unit's rows as a loop of one workgroup were a chain of up to 32 x (nch + 1) dependent loads behind each other.
 template <bool GF32>
 __global__ __launch_bounds__(256) void sink_tail_reduce(AttnArgs a, int nch) {
     const int kvu = blockIdx.x, hk = kvu % a.Hkv, b = kvu / a.Hkv, D = a.dk_dim;
-    for (int idx = threadIdx.x; idx < 2 * a.sinks * D; idx += 256) {
+    const int idx = blockIdx.y * 256 + threadIdx.x;
+    if (idx < 2 * a.sinks * D) {
         const int which = idx / (a.sinks * D), j = (idx / D) % a.sinks, d = idx % D;
         float sum = sink_tail_rows(a.tail, kvu, nch, nch, which, D)[j * D + d];
+#pragma unroll 4
         for (int c = 0; c < nch; ++c) sum += sink_tail_rows(a.tail, kvu, nch, c, which, D)[j * D + d];
         void* dst = which == 0 ? a.dk : a.dv;
         const int64_t at = which == 0 ? b * a.dk_sb + hk * a.dk_sh + j * a.dk_st + d
@@ -432,10 +435,11 @@ int launch(const AttnArgs& a, hipStream_t st) {
 
 int launch_sink_tail_reduce(const AttnArgs& a, hipStream_t st) {
     const int nch = sink_tail(a.T, a.window, a.sinks).nch;
+    const dim3 grid(a.Hkv * a.B, (2 * a.sinks * a.dk_dim + 255) / 256);
     if (a.grad_f32)
-        hipLaunchKernelGGL(sink_tail_reduce<true>, dim3(a.Hkv * a.B), dim3(256), 0, st, a, nch);
+        hipLaunchKernelGGL(sink_tail_reduce<true>, grid, dim3(256), 0, st, a, nch);
     else
-        hipLaunchKernelGGL(sink_tail_reduce<false>, dim3(a.Hkv * a.B), dim3(256), 0, st, a, nch);
+        hipLaunchKernelGGL(sink_tail_reduce<false>, grid, dim3(256), 0, st, a, nch);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }

@@ -582,7 +582,8 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
     }
 }
 
-// dK / dV = the splits' partial sums added in split order; four consecutive head_dim elements per thread
+// dK / dV = the splits' partial sums added in split order, for the sink keys' rows also the chunks of a split tail; four
+// consecutive head_dim elements per thread
 template <bool GF32>
 __global__ __launch_bounds__(256) void gqa_reduce(AttnArgs a) {
     const int D = a.dk_dim, hs = a.head_split;
@@ -599,6 +600,13 @@ __global__ __launch_bounds__(256) void gqa_reduce(AttnArgs a) {
     for (int r = 1; r < hs; ++r) {
         const f32x4 x = *reinterpret_cast<const f32x4*>(src + r * split_stride);
         sum[0] += x[0], sum[1] += x[1], sum[2] += x[2], sum[3] += x[3];
+    }
+    if (a.tail && t < a.sinks) {
+        const int nch = sink_tail(a.T, a.window, a.sinks).nch;
+        for (int c = 0; c < nch; ++c) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(sink_tail_rows(a.tail, kvu, nch, c, which, D) + t * D + d);
+            sum[0] += x[0], sum[1] += x[1], sum[2] += x[2], sum[3] += x[3];
+        }
     }
     void* dst = which == 0 ? a.dk : a.dv;
     const int64_t at = which == 0 ? b * a.dk_sb + hk * a.dk_sh + t * a.dk_st + d : b * a.dv_sb + hk * a.dv_sh + t * a.dv_st + d;

@@ -299,12 +299,17 @@ __global__ __launch_bounds__(64 * KW) void f32_split_dkdv(AttnArgs a) {
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
     const int nkb = (a.T + 31) / 32;
     const int hs = a.head_split;  // > 1: this workgroup takes heads [h0, h0 + nh) of the group, see gqa_head_split
+    // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
+    const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
+    const int nblk = nkb + tl.nch;
     int blk, rr, kvu;
     // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
-    if (a.causal && nkb > 1 ? !xcd_map_block_major(nkb, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nkb, hs, a.Hkv * a.B, blk, rr, kvu))
+    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu))
         return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = rr * rep / hs, nh = (rr + 1) * rep / hs - h0;
-    const int k0 = blk * 32, kj = k0 + c32;
+    const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
+    if (chunk >= 0 && rr > 0) return;
+    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
+    const int k0 = chunk >= 0 ? 0 : blk * 32, kj = k0 + c32;
     const float cexp = a.scale * LOG2E;
     float* const Qs = lds + KVB + kg * TILE;
     float* const Gs = Qs + 32 * P;
@@ -312,8 +317,11 @@ __global__ __launch_bounds__(64 * KW) void f32_split_dkdv(AttnArgs a) {
 
     // query tiles that can see keys [k0, k0 + 32) (paperkiln src/ops.cpp:960-965 inverted)
     const int khi = min(k0 + 32, a.T) - 1;
-    const int qt_lo = a.causal ? k0 / 32 : 0;
-    const int qt_hi = (a.window > 0 && k0 >= a.sinks) ? min(a.T - 1, khi + a.window - 1) / 32 : (a.T - 1) / 32;
+    const int qt_lo = chunk >= 0 ? (tl.q0 + chunk * TAIL_CHUNK) / 32 : a.causal ? k0 / 32 : 0;
+    const int q_end = chunk >= 0 ? min(a.T, tl.q0 + (chunk + 1) * TAIL_CHUNK) - 1
+                      : tl.nch > 0 && k0 == 0 ? tl.q0 - 1
+                      : a.window > 0 && k0 >= a.sinks ? min(a.T - 1, khi + a.window - 1) : a.T - 1;
+    const int qt_hi = q_end / 32;
     const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh;
 
     Mover32<D> mq, mg;
@@ -400,16 +408,25 @@ __global__ __launch_bounds__(64 * KW) void f32_split_dkdv(AttnArgs a) {
     join_groups<DB, KW>(acc, lds + KVB, kg, lane);
     __syncthreads();
     join_groups<DB, KW>(acc + DB, lds + KVB, kg, lane);
-    if (kj < a.T) {
-        const bool parts = hs > 1;  // partial rows: part[unit][split][dK | dV][T][dk]
-        const int64_t pk = (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
-        const int64_t rv = parts ? pk + static_cast<int64_t>(a.T) * dk : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
-        const int64_t rk = parts ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+    // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
+    // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
+    const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1);
+    if (kj < a.T && (chunk < 0 || to_tail)) {
+        const bool parts = hs > 1 && !to_tail;
+        const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
+                                   : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+        const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
+        const bool scratch = parts || to_tail;
+        void* const room = to_tail ? a.tail : a.part;
+        const int64_t rv = scratch ? pv : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
+        const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+        void* const dst_v = scratch ? room : a.dv;
+        void* const dst_k = scratch ? room : a.dk;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             if (db % KW != kg) continue;
-            store_block(true, parts ? a.part : a.dv, rv, db, g, acc[db], 1.0f, dk);
-            store_block(true, parts ? a.part : a.dk, rk, db, g, acc[DB + db], a.scale, dk);
+            store_block(true, dst_v, rv, db, g, acc[db], 1.0f, dk);
+            store_block(true, dst_k, rk, db, g, acc[DB + db], a.scale, dk);
         }
     }
 }
@@ -431,23 +448,43 @@ enum class Form { NONE, FOUR, EIGHT };
 //                           B=4 T=1024 H=8: - | 115 | 146, - | 162 | 204, - | 276 | 306
 //                           B=16 T=512 H=8: - | 152 | 140, - | 220 | 218, - | 381 | 190
 bool has_own_kernel(const AttnArgs& a) { return a.dk_dim == 32 || a.dk_dim == 64 || a.dk_dim == 128; }
-bool many_short(const AttnArgs& a, int64_t blocks) { return a.T <= 160 && blocks > 600; }
-Form query_form(const AttnArgs& a, int64_t short_chain) {  // forward, dQ
-    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
-    if (has_own_kernel(a) && (many_short(a, blocks) || (a.dk_dim == 128 && blocks > 1200))) return Form::NONE;
+// and where all chains are equally long (no mask, or a window; forward, dQ, dK/dV):
+//   head_dim 128, T 600, window 120, 24 heads 33 48 75 | 42 61 77, 38 heads 50 72 113 | 43 63 79;  T 600, no mask, 16 heads
+//   62 86 135 | 92 124 162, 38 heads 95 131 250 | 95 128 167;  T 2400, window 100, 8 heads 49 71 107 | 43 63 79
+//   head_dim 64, T 1200, window 64, 16 heads 16 28 32 | 22 29 35, 24 heads 19 30 44 | 22 30 36, 38 heads 29 44 68 | 37 57 68
+bool query_kernel_is_ahead(const AttnArgs& a, int64_t blocks, bool dq) {
+    if (!has_own_kernel(a)) return false;
     const int chain = chain_tokens(a);
+    if (a.T <= 160 && blocks > 600) return true;
+    if (a.dk_dim == 128) return blocks > (a.T <= 96 ? 300 : even_chains(a) || chain < 400 ? 512 : 1200);
+    return !dq && blocks > 1500 && (a.T <= 200 || (a.dk_dim == 64 && even_chains(a) && chain > 128));
+}
+Form query_form(const AttnArgs& a, bool dq) {  // forward, dQ
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
+    if (query_kernel_is_ahead(a, blocks, dq)) return Form::NONE;
+    const int chain = chain_tokens(a);
+    const int64_t short_chain = dq ? 0 : 200;
     return a.dk_dim <= 64 && ((blocks <= 600 && chain >= 1000) || (blocks <= short_chain && chain >= 256)) ? Form::EIGHT : Form::FOUR;
 }
-Form fwd_form(const AttnArgs& a) { return query_form(a, 200); }
-Form dq_form(const AttnArgs& a) { return query_form(a, 0); }
+Form fwd_form(const AttnArgs& a) { return query_form(a, false); }
+Form dq_form(const AttnArgs& a) { return query_form(a, true); }
 int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
+// The 128-key kernel walks the whole group of query heads in one workgroup: it is behind while those leave CUs idle,
+// however many blocks a split of keys and heads comes to (a group of four, head_dim 128, T 600, window 120: 8 KV heads
+// 252 us against 100, 24 KV heads 256 against 268; T 2400, window 100, 8 KV heads 258 against 356).
+bool key_kernel_is_ahead(const AttnArgs& a, int64_t blocks) {
+    if (!has_own_kernel(a)) return false;
+    const int chain = chain_tokens(a);
+    const int64_t groups = static_cast<int64_t>((a.T + 127) / 128) * a.Hkv * a.B;  // workgroups of the 128-key kernel
+    if (a.dk_dim == 128 && groups >= 100 && chain < 400) return true;
+    if (a.T <= 160) return a.Hq == a.Hkv ? blocks > 600 : groups >= 128;
+    if (a.dk_dim == 128) return a.Hq == a.Hkv ? blocks > (even_chains(a) ? 512 : 1200) : groups >= 112;
+    if (a.dk_dim == 64 && chain <= 160 && even_chains(a) && groups > 192 && groups <= 256) return true;  // one to a CU
+    return a.dk_dim == 64 && a.Hq == a.Hkv && blocks > 1400 && a.T < 3000;
+}
 Form dkdv_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
-    // where query heads share KV heads the 128-key kernel walks the whole group in one workgroup
-    if (has_own_kernel(a) && a.Hq == a.Hkv) {
-        if (many_short(a, blocks) || (a.dk_dim == 128 && blocks > 1200)) return Form::NONE;
-        if (a.dk_dim == 64 && blocks > 1400 && a.T < 3000) return Form::NONE;
-    }
+    if (key_kernel_is_ahead(a, blocks)) return Form::NONE;
     if (a.dk_dim > 64) return Form::FOUR;
     return a.dk_dim > 32 || (blocks <= 320 && chain_tokens(a) >= 512) ? Form::EIGHT : Form::FOUR;
 }
@@ -463,7 +500,7 @@ void run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 }
 template <int D, int KW>
 void run_dkdv(const AttnArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL((f32_split_dkdv<D, KW>), dim3(xcd_grid((a.T + 31) / 32, a.head_split, a.Hkv * a.B)), dim3(64 * KW), 0, st, a);
+    hipLaunchKernelGGL((f32_split_dkdv<D, KW>), dim3(xcd_grid((a.T + 31) / 32 + tail_blocks(a), a.head_split, a.Hkv * a.B)), dim3(64 * KW), 0, st, a);
 }
 
 }  // namespace
@@ -506,6 +543,7 @@ int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 int launch_f32_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     a.head_split = dkdv_splits(a);
+    if (!split_tail_pays(a, a.head_split)) a.tail = nullptr;
     const bool eight = dkdv_form(a) == Form::EIGHT;
     if (a.dk_dim <= 32)
         eight ? run_dkdv<32, 8>(a, st) : run_dkdv<32, 4>(a, st);
@@ -516,7 +554,7 @@ int launch_f32_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     else
         run_dkdv<128, 4>(a, st);
     PK_HIP(hipGetLastError());
-    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
 }
 
 }  // namespace pk

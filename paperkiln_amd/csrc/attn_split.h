@@ -86,6 +86,18 @@ __device__ inline void tile_barrier() {
 
 // How many tokens of the other side a block of rows walks at most: what its chain of tiles is as long as.
 inline int chain_tokens(const AttnArgs& a) { return a.window > 0 && a.window + 64 < a.T ? a.window + 64 : a.T; }
+// Whether all blocks of a launch have about the same chain. Under a full causal mask they do not: the longest are twice the
+// mean and decide when an unsplit launch ends.
+inline bool even_chains(const AttnArgs& a) { return !a.causal || chain_tokens(a) < a.T; }
+// Whether a dK/dV launch deals the queries past the band of the sink keys' block to workgroups of their own (sink_tail): the
+// block's chain through all of them, against the rest of the launch, two workgroups to a CU with a band of queries and about
+// three tiles of overhead each. (fp32, head_dim 64, T 2476, window 64, 4 sinks, 4 heads: 86 us with that chain.)
+inline bool split_tail_pays(const AttnArgs& a, int head_split) {
+    const SinkTail t = sink_tail(a.T, a.window, a.sinks);
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * head_split;
+    return a.tail && t.nch > 0 && a.T - t.q0 > (blocks + 511) / 512 * (a.window + 128);
+}
+inline int tail_blocks(const AttnArgs& a) { return a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0; }
 
 // The tiles of BN keys that queries [q0, q0 + BM) can see, as a list: sink tiles [0, ns), then [lo, hi].
 struct KeyTiles {

@@ -372,18 +372,26 @@ __global__ __launch_bounds__(64 * QW * KW) void split_dkdv(AttnArgs a) {
     // hs > 1: the query heads of the group are dealt to hs workgroups (gqa_head_split); this one takes heads
     // [h0, h0 + nh) of the group and leaves fp32 partial sums for launch_gqa_reduce
     const int hs = a.head_split;
+    // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
+    const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
+    const int nblk = nkb + tl.nch;
     int blk, rr, kvu;
     // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
-    if (a.causal && nkb > 1 ? !xcd_map_block_major(nkb, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nkb, hs, a.Hkv * a.B, blk, rr, kvu))
+    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu))
         return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = rr * rep / hs, nh = (rr + 1) * rep / hs - h0;
-    const int k0 = blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
+    const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
+    if (chunk >= 0 && rr > 0) return;
+    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
+    const int k0 = chunk >= 0 ? 0 : blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
     const float cexp = a.scale * LOG2E;
 
     // query tiles that can see keys [k0, k0 + BNK) (paperkiln src/ops.cpp:960-965 inverted)
     const int khi = min(k0 + BNK, a.T) - 1;
-    const int qt_lo = a.causal ? k0 / BMQ : 0;
-    const int qt_hi = (a.window > 0 && k0 >= a.sinks) ? min(a.T - 1, khi + a.window - 1) / BMQ : (a.T - 1) / BMQ;
+    const int qt_lo = chunk >= 0 ? (tl.q0 + chunk * TAIL_CHUNK) / BMQ : a.causal ? k0 / BMQ : 0;
+    const int q_end = chunk >= 0 ? min(a.T, tl.q0 + (chunk + 1) * TAIL_CHUNK) - 1
+                      : tl.nch > 0 && k0 == 0 ? tl.q0 - 1
+                      : a.window > 0 && k0 >= a.sinks ? min(a.T - 1, khi + a.window - 1) : a.T - 1;
+    const int qt_hi = q_end / BMQ;
     const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh, iters = (steps + KW - 1) / KW;
 
     Mover<D, G, BMQ> mq, mg;
@@ -477,14 +485,21 @@ __global__ __launch_bounds__(64 * QW * KW) void split_dkdv(AttnArgs a) {
     join_groups<DB, KW>(acc, red, kg, lane);
     if (KW > 1) __syncthreads();
     join_groups<DB, KW>(acc + DB, red, kg, lane);
-    if (kj < a.T) {
-        const bool parts = hs > 1;  // partial rows: part[unit][split][dK | dV][T][dk]
-        const int64_t pk = (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
-        const int64_t rv = parts ? pk + static_cast<int64_t>(a.T) * dk : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
-        const int64_t rk = parts ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
-        void* const dst_v = parts ? a.part : a.dv;
-        void* const dst_k = parts ? a.part : a.dk;
-        const bool f32 = parts || a.grad_f32;
+    // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
+    // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
+    const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1);
+    if (kj < a.T && (chunk < 0 || to_tail)) {
+        const bool parts = hs > 1 && !to_tail;
+        const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
+                                   : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+        const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
+        const bool scratch = parts || to_tail;
+        void* const room = to_tail ? a.tail : a.part;
+        const int64_t rv = scratch ? pv : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
+        const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+        void* const dst_v = scratch ? room : a.dv;
+        void* const dst_k = scratch ? room : a.dk;
+        const bool f32 = scratch || a.grad_f32;
 #pragma unroll
         for (int n = 0; n < 2 * DB; ++n) {
             if (KW > 1 && n % DB % KW != kg) continue;
@@ -513,25 +528,37 @@ enum class Form { NONE, WIDE, FOUR, EIGHT };
 //   forward, head_dim 128     T 512, 8 heads 11 | 12 | 16;  32 heads 18 | 18 | 16;  T 1024, 16 heads 22 | 23 | 26
 //   dQ, head_dim 128          T 512, 8 heads 16 | 14 | 22;  T 2048, 8 heads 41 | 40 | 68;  16 heads 84 | 79 | 72
 //   dK/dV, head_dim 128       T 512, 32 heads - | 24 | 34;  T 2048, 8 heads - | 48 | 66;  16 heads - | 94 | 69
+// Where the kernels without a split exist, they win on short chains as soon as the blocks exceed the CUs, on even chains
+// from there on, and always where a chain is a single tile of theirs (us, split | unsplit, forward, dQ, dK/dV):
+//   head_dim 64, T 64, 16 units 5.3 6.6 6.7 | 4.3 5.4 5.7;     T 180, 32 units 6.5 8.5 8.8 | 6.7 9.3 9.5, 64 units 8.0 10.1 15.9 | 6.8 9.4 9.7
+//   T 600, window 128, 16 units 10.5 13.7 15.0 | 9.2 11.2 10.9;  T 929, no mask, 16 units 16.8 20.1 25.0 | 17.5 25.9 28.6
+//   head_dim 128, T 600, window 60, 16 units 12.2 17.8 18.2 | 11.0 13.6 10.5;  T 1100, no mask, 16 units 41 60 72 | 29 43 54
 // From 4096 tokens on head_dim 128 stays with the unsplit kernels whatever the number of units: a
 // unit alone, a unit in a batch and the prefix of a longer sequence are then the same bits, which callers rely on there.
-bool one_kernel_for_any_batch(const AttnArgs& a) { return a.dk_dim == 128 && a.T >= 4096; }
+bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
+    if (a.dk_dim != 64 && a.dk_dim != 128) return false;  // they take these head sizes only
+    if (a.dk_dim == 128 && a.T >= 4096) return true;
+    const int chain = chain_tokens(a);
+    if (blocks <= 256) return false;
+    return chain < 256 || (even_chains(a) && !(a.dk_dim == 64 && chain >= 768 && blocks <= 600));
+}
 Form fwd_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
-    const bool plain = a.dk_dim == 64 || a.dk_dim == 128;  // the unsplit kernels take these
-    if (one_kernel_for_any_batch(a)) return Form::NONE;
-    if (blocks <= 320) return chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
+    const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
+    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= 64)) return Form::NONE;
+    if (blocks <= 256) return chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
     if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
-    if (blocks <= 600) return chain_tokens(a) >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 ? Form::FOUR : Form::NONE;
+    if (blocks <= 600)
+        return chain_tokens(a) >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 && a.causal ? Form::FOUR : Form::NONE;
     return blocks <= 1100 && chain_tokens(a) >= 3000 ? Form::EIGHT : Form::NONE;
 }
 Form dq_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
-    if (one_kernel_for_any_batch(a)) return Form::NONE;
+    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= 64)) return Form::NONE;
     // above 96 columns eight wavefronts of this kernel do not fit the registers
     const Form best = a.dk_dim > 96 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
-    if (blocks <= 320) return best;
+    if (blocks <= 256) return best;
     if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
     if (blocks <= 600) return chain_tokens(a) >= 1536 ? best : a.dk_dim == 64 || chain_tokens(a) >= 768 ? Form::FOUR : Form::NONE;
     return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 1000 ? Form::FOUR : Form::NONE;
@@ -540,7 +567,8 @@ int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
 Form dkdv_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
-    if (one_kernel_for_any_batch(a)) return Form::NONE;
+    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 64) && dkdv_splits(a) == 1))
+        return Form::NONE;
     const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
     if (!plain) return blocks <= 700 ? best : Form::WIDE;
     if (blocks <= 600) return best;
@@ -561,7 +589,7 @@ void run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 template <int D, int QW, int KW, int NB, bool EXACT>
 void run_dkdv(const AttnArgs& a, hipStream_t st) {
     const int nkb = (a.T + 32 * QW - 1) / (32 * QW);
-    hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT>), dim3(xcd_grid(nkb, a.head_split, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a);
+    hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT>), dim3(xcd_grid(nkb + tail_blocks(a), a.head_split, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a);
 }
 
 template <int D, bool EXACT>
@@ -624,13 +652,14 @@ int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     a.head_split = dkdv_splits(a);
+    if (!split_tail_pays(a, a.head_split)) a.tail = nullptr;
     const auto run = [&]() -> int {
 #define PK_CALL(D, E) dkdv_of<D, E>(a, dkdv_form(a), st)
         PK_SPLIT_DISPATCH(PK_CALL);
 #undef PK_CALL
     };
     if (const int rc = run()) return rc;
-    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
 }
 
 }  // namespace pk

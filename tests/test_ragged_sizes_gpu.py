@@ -113,6 +113,18 @@ def test_fp32_split_kernels(case, dk):
     assert max(e) < 5e-6, e
 
 
+# The queries past the sink keys' band dealt to workgroups of their own: one chunk and a short last one, all 32 sink rows,
+# query heads dealt as well, blocks of 32 keys and (bf16, head_dim 48, many of them) of 128.
+@pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 48), (torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float32, 32),
+                                      (torch.float32, 64), (torch.float32, 128)], ids=str)
+@pytest.mark.parametrize("case", [(1, 770, 2, 2, True, 64, 1), (1, 1300, 7, 1, True, 100, 32), (2, 1411, 4, 2, True, 33, 5),
+                                  (9, 1200, 4, 4, True, 40, 16)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_sink_tail_of_the_split_kernels(case, dtype, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, dtype, causal, window, sinks))
+    assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
+
+
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 65, 31), (64, 32, 33), (31, 97, 344), (1, 40, 1001), (900, 1030, 70)])
 def test_fp32_products(M, N, K, tA, tB):
