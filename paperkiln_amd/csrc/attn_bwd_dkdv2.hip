@@ -74,9 +74,7 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
     const int row_lane = lds_row<D>(c32) * S + g * 8;
     const int tr_lane = lds_row<D>(4 * g + ((lane & 15) >> 2)) * S + TrMap<D>::src_col(0, (lane >> 4) & 1, lane & 3);
     const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv;
-    // Full-causal: key block i is seen by T - 128i queries; blocks i and nkb-1-i
-    // are taken back to back so that every workgroup carries the same work.
-    const bool paired = a.causal && a.window == 0;
+    // Full-causal: key block i is seen by T - 128i queries.
     int blk, rr, kvu;
     // Band mask with a few sink keys: the queries past block 0's band are cut into chunks that get
     // workgroups of their own (ids nkb .. nkb + nch - 1 of the unit), see sink_tail.
@@ -85,14 +83,14 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
         if (!xcd_map(nkb + tl.nch, 1, a.Hkv * a.B, blk, rr, kvu)) return;
     } else if (a.window > 0 && a.sinks > 0 && nkb > 1) {
         if (!xcd_map_block0_first(nkb, a.Hkv * a.B, blk, kvu)) return;
-    } else if (!xcd_map(paired ? (nkb + 1) / 2 : nkb, 1, a.Hkv * a.B, blk, rr, kvu)) {
+    } else if (!map_causal_blocks(a, nkb, 1, blk, rr, kvu)) {
         return;
     }
     const int chunk = (TAIL && blk >= nkb) ? blk - nkb : -1;  // >= 0: this workgroup takes a chunk of the sink tail
     if (TAIL && chunk >= 0) blk = 0;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv;
     const float cexp = a.scale * LOG2E;
-    const int npass = (paired && blk != nkb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nkb - 1 - blk) ? 2 : 1;
 
     for (int pass = 0; pass < npass; ++pass) {
         const int kblk = pass == 0 ? blk : nkb - 1 - blk;  // heavy block first
@@ -402,7 +400,7 @@ template <int D, bool GF32, int BNK, int BMQ>
 int launch_geo(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     const int nkb = (a.T + BNK - 1) / BNK;
-    const bool paired = a.causal && a.window == 0;
+    a.paired = pair_causal_blocks(nkb, static_cast<int64_t>(a.Hkv) * a.B, a.causal, a.window, 256);
     SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
     // a tail step keeps two of the eight wavefronts busy but takes as long as a full one (measured)
     if (!sink_tail_pays(tl, a.T, a.window, a.Hkv * a.B, 64, 3, 1.0f)) {
@@ -416,7 +414,7 @@ int launch_geo(const AttnArgs& a_in, hipStream_t st) {
         return launch_sink_tail_reduce(a, st);
     }
     const int ids = a.window > 0 && a.sinks > 0 && nkb > 1 ? xcd_grid_block0_first(nkb, a.Hkv * a.B)
-                                                           : xcd_grid(paired ? (nkb + 1) / 2 : nkb, 1, a.Hkv * a.B);
+                                                           : xcd_grid(a.paired ? (nkb + 1) / 2 : nkb, 1, a.Hkv * a.B);
     hipLaunchKernelGGL((mfma_dkdv2<D, GF32, false, BNK, BMQ>), dim3(ids), dim3(4 * BNK), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;

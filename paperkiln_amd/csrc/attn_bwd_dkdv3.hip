@@ -106,18 +106,16 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
     const int role = w >> 1, khalf = w & 1;
     const int g = lane >> 5, c32 = lane & 31;
     const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv;
-    // Full-causal: key block i is seen by T - 128i queries; blocks i and nkb-1-i
-    // are taken back to back so that every workgroup carries the same work.
-    const bool paired = a.causal && a.window == 0;
+    // Full-causal: key block i is seen by T - 128i queries.
     // hs > 1: the query heads of the group are dealt to hs workgroups (gqa_head_split); this one takes heads
     // [hfirst, hfirst + nh) of the group and leaves fp32 partial sums for launch_gqa_reduce
     const int hs = a.head_split;
     int blk, rr = 0, kvu;
-    if (!xcd_map(paired ? (nkb + 1) / 2 : nkb, hs, a.Hkv * a.B, blk, rr, kvu)) return;
+    if (!map_causal_blocks(a, nkb, hs, blk, rr, kvu)) return;
     const int hfirst = rr * rep / hs, nh = (rr + 1) * rep / hs - hfirst;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv;
     const float cexp = a.scale * LOG2E;
-    const int npass = (paired && blk != nkb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nkb - 1 - blk) ? 2 : 1;
 
     for (int pass = 0; pass < npass; ++pass) {
         const int kblk = pass == 0 ? blk : nkb - 1 - blk;  // heavy block first
@@ -616,12 +614,11 @@ __global__ __launch_bounds__(256) void gqa_reduce(AttnArgs a) {
 template <int D, bool GF32>
 int launch(const AttnArgs& a, hipStream_t st) {
     const int nb128 = (a.T + 127) / 128;
-    const bool paired = a.causal && a.window == 0;
     const int hs = a.part ? a.head_split : 1;
     AttnArgs b = a;
     b.head_split = hs;
-    hipLaunchKernelGGL((mfma_dkdv3<D, GF32>), dim3(xcd_grid(paired ? (nb128 + 1) / 2 : nb128, hs, a.Hkv * a.B)),
-                       dim3(256), 0, st, b);
+    b.paired = pair_causal_blocks(nb128, static_cast<int64_t>(a.Hkv) * a.B * hs, a.causal, a.window, 256);
+    hipLaunchKernelGGL((mfma_dkdv3<D, GF32>), causal_blocks_grid(b, nb128, hs), dim3(256), 0, st, b);
     PK_HIP(hipGetLastError());
     return hs > 1 ? launch_gqa_reduce(b, st) : PK_OK;
 }

@@ -108,14 +108,10 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
     const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
     int blk, rr, kvu;
-    // unpaired causal blocks without a band: heaviest blocks of every unit first
-    if (!paired && a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
-                                             : !xcd_map(paired ? (nqb + 1) / 2 : nqb, rep, a.Hkv * a.B, blk, rr, kvu))
-        return;
+    if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
-    const int npass = (paired && blk != nqb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
     const float cexp = a.scale * LOG2E;
 
     auto lds32 = [](const void* p) { return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p)); };
@@ -519,10 +515,11 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
 }
 
 template <int D, bool GF32>
-int launch(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+int launch(const AttnArgs& a_in, bool fuse_delta, hipStream_t st) {
+    AttnArgs a = a_in;
     const int nqb = (a.T + BM - 1) / BM;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
-    const dim3 grid(xcd_grid(paired ? (nqb + 1) / 2 : nqb, a.Hq / a.Hkv, a.Hkv * a.B));
+    a.paired = pair_causal_blocks(nqb, static_cast<int64_t>(a.Hq) * a.B, a.causal, a.window, 256);
+    const dim3 grid = causal_blocks_grid(a, nqb, a.Hq / a.Hkv);
     if (fuse_delta)
         hipLaunchKernelGGL((mfma_dq3<D, GF32, true>), grid, dim3(256), 0, st, a);
     else

@@ -130,14 +130,10 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_dq(AttnArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
     const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
     int blk, rr, kvu;
-    // unpaired causal blocks without a band: heaviest blocks of every unit first
-    if (!paired && a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
-                                             : !xcd_map(paired ? (nqb + 1) / 2 : nqb, rep, a.Hkv * a.B, blk, rr, kvu))
-        return;
+    if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
-    const int npass = (paired && blk != nqb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int qblk = pass == 0 ? nqb - 1 - blk : blk;
     const int q0 = qblk * BM;
@@ -269,14 +265,16 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_dq(AttnArgs a) {
 }
 
 template <int D, bool GF32>
-int launch_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+int launch_dq(const AttnArgs& a_in, bool fuse_delta, hipStream_t st) {
+    AttnArgs a = a_in;
     // dQ with 8 wavefronts (256 queries) per K/V tile where the paired causal grid still gives every CU two
     // workgroups in turn, as in the forward kernel; 4 wavefronts otherwise.
     const int nb256 = (a.T + 255) / 256;
     const bool wide = D == 128 && a.causal && a.window == 0 && static_cast<int64_t>((nb256 + 1) / 2) * a.Hq * a.B >= 512;
     const int nbq = wide ? nb256 : (a.T + 127) / 128;
-    const bool paired = pair_causal_blocks(nbq, a.Hq * a.B, a.causal, a.window);
-    const dim3 grid(xcd_grid(paired ? (nbq + 1) / 2 : nbq, a.Hq / a.Hkv, a.Hkv * a.B));
+    // as in the forward kernel (16 heads x 1024 x 16, head_dim 64: 76 us singly, 80 paired)
+    a.paired = (D == 128 || nbq <= 2) && pair_causal_blocks(nbq, static_cast<int64_t>(a.Hq) * a.B, a.causal, a.window, wide ? 256 : 512);
+    const dim3 grid = causal_blocks_grid(a, nbq, a.Hq / a.Hkv);
     if (wide && fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, true, 8>), grid, dim3(512), 0, st, a);
     if (wide && !fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, false, 8>), grid, dim3(512), 0, st, a);
     if (!wide && fuse_delta) hipLaunchKernelGGL((mfma_dq<D, GF32, true, 4>), grid, dim3(256), 0, st, a);

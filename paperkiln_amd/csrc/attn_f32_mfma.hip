@@ -79,14 +79,10 @@ __global__ __launch_bounds__(256, 2) void f32_fwd(AttnArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
     const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
-    // Full-causal work per query block grows with its index: a workgroup takes blocks i and
-    // nqb-1-i back to back where the halved grid still fills the chip (pair_causal_blocks), else the
-    // blocks are dispatched singly, heaviest first.
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
     int blk, rr, kvu;
-    if (!xcd_map(paired ? (nqb + 1) / 2 : nqb, rep, a.Hkv * a.B, blk, rr, kvu)) return;
+    if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
-    const int npass = (paired && blk != nqb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int q0 = (pass == 0 ? nqb - 1 - blk : blk) * BM;
     const int qlo = q0 + w * 32, qhi = qlo + 31, qi = qlo + c32;
@@ -219,11 +215,10 @@ __global__ __launch_bounds__(256, 1) void f32_dq(AttnArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
     const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);  // as in the forward
     int blk, rr, kvu;
-    if (!xcd_map(paired ? (nqb + 1) / 2 : nqb, rep, a.Hkv * a.B, blk, rr, kvu)) return;
+    if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
-    const int npass = (paired && blk != nqb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int q0 = (pass == 0 ? nqb - 1 - blk : blk) * BM;
     const int qlo = q0 + w * 32, qhi = qlo + 31, qi = qlo + c32;
@@ -414,14 +409,13 @@ __global__ __launch_bounds__(512, 1) void f32_dkdv(AttnArgs a) {
     const int g = lane >> 5, c32 = lane & 31;
     const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv;
     const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
-    const bool paired = a.causal && a.window == 0;
     int blk0, rr, kvu;
-    if (!xcd_map(paired ? (nkb + 1) / 2 : nkb + tl.nch, 1, a.Hkv * a.B, blk0, rr, kvu)) return;
+    if (!map_causal_blocks(a, nkb + tl.nch, 1, blk0, rr, kvu)) return;
     const int chunk = blk0 >= nkb ? blk0 - nkb : -1;
     if (chunk >= 0) blk0 = 0;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv;
     const float cexp = a.scale * LOG2E;
-    const int npass = (paired && blk0 != nkb - 1 - blk0) ? 2 : 1;
+    const int npass = (a.paired && blk0 != nkb - 1 - blk0) ? 2 : 1;
 
   for (int pass = 0; pass < npass; ++pass) {
     const int kblk = pass == 0 ? blk0 : nkb - 1 - blk0;  // heavy block first
@@ -610,20 +604,22 @@ bool aligned_f32(const void* p, int64_t sb, int64_t st, int64_t sh) {
 }
 
 template <int D>
-int launch_fwd(const AttnArgs& a, hipStream_t st) {
+int launch_fwd(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
     const int nqb = (a.T + 127) / 128;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
-    const dim3 grid(xcd_grid(paired ? (nqb + 1) / 2 : nqb, a.Hq / a.Hkv, a.Hkv * a.B));
+    a.paired = pair_causal_blocks(nqb, static_cast<int64_t>(a.Hq) * a.B, a.causal, a.window, 256);
+    const dim3 grid = causal_blocks_grid(a, nqb, a.Hq / a.Hkv);
     hipLaunchKernelGGL(f32_fwd<D>, grid, dim3(256), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
 
 template <int D>
-int launch_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+int launch_dq(const AttnArgs& a_in, bool fuse_delta, hipStream_t st) {
+    AttnArgs a = a_in;
     const int nqb = (a.T + 127) / 128;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
-    const dim3 grid(xcd_grid(paired ? (nqb + 1) / 2 : nqb, a.Hq / a.Hkv, a.Hkv * a.B));
+    a.paired = pair_causal_blocks(nqb, static_cast<int64_t>(a.Hq) * a.B, a.causal, a.window, 256);
+    const dim3 grid = causal_blocks_grid(a, nqb, a.Hq / a.Hkv);
     if (fuse_delta)
         hipLaunchKernelGGL((f32_dq<D, true>), grid, dim3(256), 0, st, a);
     else
@@ -639,8 +635,8 @@ int launch_dkdv(const AttnArgs& a_in, hipStream_t st) {
         a.tail = nullptr;
     const int nch = a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0;
     const int nkb = (a.T + 127) / 128;
-    const bool paired = a.causal && a.window == 0;
-    hipLaunchKernelGGL(f32_dkdv<D>, dim3(xcd_grid(paired ? (nkb + 1) / 2 : nkb + nch, 1, a.Hkv * a.B)), dim3(512), 0, st, a);
+    a.paired = pair_causal_blocks(nkb, static_cast<int64_t>(a.Hkv) * a.B, a.causal, a.window, 256);
+    hipLaunchKernelGGL(f32_dkdv<D>, causal_blocks_grid(a, nkb + nch, 1), dim3(512), 0, st, a);
     PK_HIP(hipGetLastError());
     return nch > 0 ? launch_sink_tail_reduce(a, st) : PK_OK;
 }

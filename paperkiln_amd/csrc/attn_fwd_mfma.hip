@@ -112,18 +112,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void mfma_fwd(AttnArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
     const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
-    // Full-causal work per query block grows linearly with its index, so a
-    // workgroup takes blocks i and nqb-1-i back to back: every workgroup then
-    // carries the same number of key tiles and the last wave of workgroups
-    // does not idle three quarters of the chip.
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
     int blk, rr, kvu;
-    // unpaired causal blocks without a band: heaviest blocks of every unit first
-    if (!paired && a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
-                                             : !xcd_map(paired ? (nqb + 1) / 2 : nqb, rep, a.Hkv * a.B, blk, rr, kvu))
-        return;
+    if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
-    const int npass = (paired && blk != nqb - 1 - blk) ? 2 : 1;
+    const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int qblk = pass == 0 ? nqb - 1 - blk : blk;
     const int q0 = qblk * BM;
@@ -349,12 +341,14 @@ __global__ __launch_bounds__(64 * NW, OCC) void mfma_fwd(AttnArgs a) {
 }
 
 template <int D, int NQ, int OCC, int NW, bool WIN>
-int launch_win(const AttnArgs& a, hipStream_t st) {
+int launch_win(const AttnArgs& a_in, hipStream_t st) {
     constexpr int BM = 32 * NW * NQ;
-    const int nqb = (a.T + BM - 1) / BM;
-    const bool paired = pair_causal_blocks(nqb, a.Hq * a.B, a.causal, a.window);
-    dim3 grid(xcd_grid(paired ? (nqb + 1) / 2 : nqb, a.Hq / a.Hkv, a.Hkv * a.B));
-    hipLaunchKernelGGL((mfma_fwd<D, NQ, OCC, NW, WIN>), grid, dim3(64 * NW), 0, st, a);
+    const int nqb = (a_in.T + BM - 1) / BM;
+    AttnArgs a = a_in;
+    // head_dim 64 keeps three workgroups or more on a CU and evens out by itself: singly, from three blocks on, is ahead or
+    // level at every size measured (16 heads x 1024 x 16: 55 us against 58)
+    a.paired = (D == 128 || nqb <= 2) && pair_causal_blocks(nqb, static_cast<int64_t>(a.Hq) * a.B, a.causal, a.window, NW == 8 ? 256 : 512);
+    hipLaunchKernelGGL((mfma_fwd<D, NQ, OCC, NW, WIN>), causal_blocks_grid(a, nqb, a.Hq / a.Hkv), dim3(64 * NW), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }

@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pk_internal.h"
+
 namespace pk {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -342,14 +344,26 @@ __device__ inline bool xcd_map_block0_first(int nblk, int kv_units, int& blk, in
     return true;
 }
 
-// Full-causal work per 128-row block grows linearly with its index, so the forward and dQ kernels
-// give a workgroup blocks i and n-1-i back to back: equal work everywhere. That halves the number
-// of workgroups; when the halved grid would not give every CU more than one workgroup (short
-// sequences, few heads) the blocks are dispatched singly, heaviest first, and the hardware
-// balances them (measured: 448 paired workgroups beat 896 single ones by 25 %, 128 paired lose
-// to 256 single by 10 %).
-__host__ __device__ inline bool pair_causal_blocks(int nblk, int units, int causal, int window) {
-    return causal && window == 0 && static_cast<int64_t>((nblk + 1) / 2) * units > 256;
+// Full-causal work per block grows linearly with its index (falls, for key blocks), so a workgroup may take blocks i and
+// n-1-i back to back: equal work everywhere, half the prologues, and the units one after another, so that fewer of them
+// share an L2 at a time. Singly and heaviest first the blocks fill the chip whatever their number. Pairs are ahead (0 to
+// 11 %) where they come to whole rounds of the workgroups that run at a time, `together`; everywhere else they leave part
+// of the chip idle for a round: at head_dim 128 16 heads of 5000 tokens took 145 us (forward) and 280 (dK/dV) paired, 131
+// and 215 singly; 24 heads x 4096 x 2 328 us (dQ) against 291; fp32, 16 heads x 1024 x 6 305, 485, 620 against 249, 377, 481.
+__host__ inline bool pair_causal_blocks(int nblk, int64_t units, int causal, int window, int together) {
+    if (!causal || window != 0) return false;
+    const int64_t pairs = static_cast<int64_t>((nblk + 1) / 2) * units;
+    const double paired = static_cast<double>((pairs + together - 1) / together) * (nblk + 1);  // in units of block 0's work
+    const double singly = 0.5 * nblk * (nblk + 1) * static_cast<double>(units) / together;
+    return paired <= (1.04 + 0.12 / nblk) * singly;  // short sequences: a block's prologue counts for more
+}
+// Which block of which unit a workgroup of such a launch takes; not paired: heaviest blocks of every unit first.
+__device__ inline bool map_causal_blocks(const AttnArgs& a, int nblk, int rep, int& blk, int& rr, int& kvu) {
+    if (!a.paired && a.causal && a.window == 0) return xcd_map_block_major(nblk, rep, a.Hkv * a.B, blk, rr, kvu);
+    return xcd_map(a.paired ? (nblk + 1) / 2 : nblk, rep, a.Hkv * a.B, blk, rr, kvu);
+}
+__host__ inline dim3 causal_blocks_grid(const AttnArgs& a, int nblk, int rep) {
+    return dim3(xcd_grid(a.paired ? (nblk + 1) / 2 : nblk, rep, a.Hkv * a.B));
 }
 
 // Branch-free visibility tests (the reference's two ranges, paperkiln

@@ -39,6 +39,7 @@ struct AttnArgs {
     float* delta;    // bwd scratch: rowsum(dO .* O)   [B,Hq,T]
     float* tail;     // bwd scratch: partial dK/dV rows of the sink keys (see sink_tail), or null
     float* part;     // bwd scratch: per-split partial dK/dV of a GQA group (see gqa_head_split), or null
+    int paired;      // full-causal launches of 128-row blocks and more: two blocks to a workgroup (see pair_causal_blocks)
     int head_split;  // number of workgroups that share the query heads of one KV head in the dK/dV launch (1 = no split)
     int64_t q_sb, q_st, q_sh;
     int64_t k_sb, k_st, k_sh;
