@@ -422,10 +422,22 @@ int launch_geo(const AttnArgs& a_in, hipStream_t st) {
 
 template <int D, bool GF32>
 int launch(const AttnArgs& a, hipStream_t st) {
-    // A band of a few key blocks: the small geometry, two workgroups per CU. Measured at B=4 H=16 T=4096, head_dim 128,
-    // small against large: window 128 0.190 / 0.229 ms, 256 0.190 / 0.223, 512 0.264 / 0.276, 1024 0.404 / 0.387,
-    // 2048 0.623 / 0.565; at head_dim 64 (window 256) 0.142 / 0.134, so only head_dim 128 takes it.
-    if (D == 128 && a.window > 0 && a.window <= 512) return launch_geo<D, GF32, 64, 32>(a, st);
+    // Short sequences and bands of a few key blocks: the small geometry, two workgroups per CU or (head_dim 64) four, which
+    // hides the two memory round trips at the start of each and wastes less of the last tile. Measured, small | large
+    // (us): B=4 H=16 T=4096, head_dim 128, window 128 190 | 229, 512 264 | 276, 1024 404 | 387; 16 heads, no band, T 48 x 170
+    // at head_dim 64 29 | 57, at 128 59 | 82; T 128 x 64 28 | 36 and 52 | 67; T 400 x 20 41 | 49 and 76 | 81; T 900 x 3,
+    // head_dim 64 32 | 26.
+    // At head_dim 64 a wide band has to come with many of its workgroups (3571 tokens, window 315, 8 heads 20 | 16; 2000 x 4,
+    // window 300, 16 heads 56 | 64), sink keys with a narrow one, whose tail then hides the sinks' (16 heads of 500 tokens,
+    // window 100, 4 sinks: x 16 40 | 52, x 6 24 | 23; 2000 x 4, window 300, 16 sinks 74 | 71).
+    const int64_t small = static_cast<int64_t>((a.T + 63) / 64) * a.Hkv * a.B;  // its workgroups
+    const bool narrow = a.window <= 128, many = small >= 1024;
+    const bool ahead = a.window == 0    ? a.T <= 256 || (a.T <= 512 && small >= 256)
+                       : a.window > 512 ? false
+                       : D == 128       ? true
+                       : a.sinks > 0    ? narrow && many
+                                        : narrow || many;
+    if (ahead) return launch_geo<D, GF32, 64, 32>(a, st);
     return launch_geo<D, GF32, 128, 64>(a, st);
 }
 

@@ -632,10 +632,16 @@ bool mfma_dkdv3_takes(const AttnArgs& a) {
     // (0.22 against 0.24 ms at head_dim 128, window 256 + 4 sinks, T 4096): the steps are
     // few, most of them masked, and the workgroup that owns the sink keys alone walks every query tile
     // Short sequences (a workgroup meets a handful of query steps) are left to the 32-key kernel, which is ahead
-    // below T = 512 at head_dim 128 and below T = 1024 at head_dim 64 (measured, B x H = 16 .. 256) -- unless query
-    // heads share KV heads: only this kernel deals the heads of a group to several workgroups.
+    // below T = 512 at head_dim 128 and below T = 1024 at head_dim 64 (measured, B x H = 16 .. 256). Where query heads share
+    // KV heads only this kernel deals the heads of a group to several workgroups, for the price of fp32 partial sums of the
+    // whole of dK and dV: worth it until the 64-key workgroups of the other, which walk a group's heads in turn, come to
+    // about one per CU, or more where each walks many queries (us, this kernel | the other; 16 query heads on 4):
+    //   head_dim 64    T 64 x 62 36 | 13;  T 256 x 31 59 | 44;  T 400 x 10 46 | 52, x 20 79 | 53;  T 500 x 16 69 | 73, x 32 102 | 88
+    //   head_dim 128   T 100 x 20 44 | 23;  T 256 x 15 58 | 37;  T 400 x 5 39 | 55, x 10 71 | 56;  T 500 x 8 63 | 67, x 16 120 | 81
     const int t_min = a.dk_dim == 128 ? 512 : 1024;
-    return (a.dk_dim == 128 || a.dk_dim == 64) && a.window == 0 && (a.T >= t_min || a.Hq > a.Hkv) &&
+    const int64_t groups = static_cast<int64_t>((a.T + 63) / 64) * a.Hkv * a.B;
+    const int64_t enough = a.dk_dim == 128 ? (a.T <= 256 ? 128 : 270) : a.T <= 128 ? 128 : a.T <= 256 ? 240 : a.T <= 448 ? 500 : 1000;
+    return (a.dk_dim == 128 || a.dk_dim == 64) && a.window == 0 && (a.T >= t_min || (a.Hq > a.Hkv && groups < enough)) &&
            reach < (int64_t{1} << 31);
 }
 

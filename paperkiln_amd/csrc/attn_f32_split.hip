@@ -455,9 +455,10 @@ bool has_own_kernel(const AttnArgs& a) { return a.dk_dim == 32 || a.dk_dim == 64
 bool query_kernel_is_ahead(const AttnArgs& a, int64_t blocks, bool dq) {
     if (!has_own_kernel(a)) return false;
     const int chain = chain_tokens(a);
-    if (a.T <= 160 && blocks > 600) return true;
+    if (a.T <= 160 && blocks > (a.T <= 64 ? 256 : dq ? 512 : 600)) return true;
     if (a.dk_dim == 128) return blocks > (a.T <= 96 ? 300 : even_chains(a) || chain < 400 ? 512 : 1200);
-    return !dq && blocks > 1500 && (a.T <= 200 || (a.dk_dim == 64 && even_chains(a) && chain > 128));
+    if (a.T <= 200 && even_chains(a) && blocks > 512) return true;
+    return !dq && blocks > 1500 && (a.T <= 200 || (even_chains(a) && chain > 128));
 }
 Form query_form(const AttnArgs& a, bool dq) {  // forward, dQ
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
@@ -471,16 +472,18 @@ Form dq_form(const AttnArgs& a) { return query_form(a, true); }
 int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
 // The 128-key kernel walks the whole group of query heads in one workgroup: it is behind while those leave CUs idle,
 // however many blocks a split of keys and heads comes to (a group of four, head_dim 128, T 600, window 120: 8 KV heads
-// 252 us against 100, 24 KV heads 256 against 268; T 2400, window 100, 8 KV heads 258 against 356).
+// 252 us against 100, 24 KV heads 256 against 268; T 2400, window 100, 8 KV heads 258 against 356). Causal, every head its own
+// (us, this kernel | the 128-key one): head_dim 128, T 1100, 24 heads 255 | 287, 32 heads 328 | 287; head_dim 64, T 400, 64
+// heads 54 | 65, 96 heads 77 | 66.
 bool key_kernel_is_ahead(const AttnArgs& a, int64_t blocks) {
     if (!has_own_kernel(a)) return false;
     const int chain = chain_tokens(a);
     const int64_t groups = static_cast<int64_t>((a.T + 127) / 128) * a.Hkv * a.B;  // workgroups of the 128-key kernel
-    if (a.dk_dim == 128 && groups >= 100 && chain < 400) return true;
-    if (a.T <= 160) return a.Hq == a.Hkv ? blocks > 600 : groups >= 128;
-    if (a.dk_dim == 128) return a.Hq == a.Hkv ? blocks > (even_chains(a) ? 512 : 1200) : groups >= 112;
+    if (a.dk_dim == 128 && groups >= (a.T <= 64 ? 80 : 100) && chain < 400) return true;
+    if (a.T <= 160) return a.Hq == a.Hkv ? blocks > (a.T <= 64 ? 256 : 600) : groups >= 128;
+    if (a.dk_dim == 128) return a.Hq == a.Hkv ? blocks > (even_chains(a) ? 512 : a.T < 800 ? 800 : 900) : groups >= 112;
     if (a.dk_dim == 64 && chain <= 160 && even_chains(a) && groups > 192 && groups <= 256) return true;  // one to a CU
-    return a.dk_dim == 64 && a.Hq == a.Hkv && blocks > 1400 && a.T < 3000;
+    return a.Hq == a.Hkv && ((a.dk_dim == 64 && blocks > 1400 && a.T < 3000) || (a.T <= 450 && blocks > 1000));
 }
 Form dkdv_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);

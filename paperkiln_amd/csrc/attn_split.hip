@@ -540,6 +540,7 @@ bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
     if (a.dk_dim == 128 && a.T >= 4096) return true;
     const int chain = chain_tokens(a);
     if (blocks <= 256) return false;
+    if ((chain < 512 || a.dk_dim == 128) && blocks > 540) return true;
     return chain < 256 || (even_chains(a) && !(a.dk_dim == 64 && chain >= 768 && blocks <= 600));
 }
 Form fwd_form(const AttnArgs& a) {
@@ -567,7 +568,7 @@ int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
 Form dkdv_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
-    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 64) && dkdv_splits(a) == 1))
+    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 72) && dkdv_splits(a) == 1))
         return Form::NONE;
     const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
     if (!plain) return blocks <= 700 ? best : Form::WIDE;
