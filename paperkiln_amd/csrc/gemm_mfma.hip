@@ -1047,15 +1047,14 @@ void run_plan(const Plan& p, bool tA, bool tB, const GemmArgs& ga, int splits, b
                 launch_geo<GeoSmall>(tA, tB, ga, splits, f32, st);
     }
 }
-bool takes(const void* a, bool tA, int64_t lda, const void* b, bool tB, int64_t ldb, int64_t M, int64_t N, int64_t K) {
+bool takes(const void* a, bool tA, int64_t lda, const void* b, bool tB, int64_t ldb, int64_t M, int64_t N, int64_t K,
+           bool any_n = false) {
     if (M <= 0 || N <= 0 || K <= 0 || M > (1 << 30) || N > (1 << 30) || K > (1 << 30)) return false;
     if (!aligned16(a) || !aligned16(b)) return false;
-    if (lda % 8 || ldb % 8 || N % 8) return false;
+    if (lda % 8 || ldb % 8 || (N % 8 && !any_n)) return false;
     // a contraction that runs along a row of either operand is read in 16-byte chunks; where it is the row index of both
     // (a weight gradient over the tokens) rows past its end read as zeros and any length goes
-    if (K % 8 && (!tA || tB)) return false;
-    if (tA && M % 8) return false;  // A^T is read in 16-byte chunks along M
-    return true;
+    return K % 8 == 0 || (tA && !tB);  // A^T is read in chunks along M, which end inside its rows' pitch
 }
 GemmArgs gemm_args(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K) {
     GemmArgs g;
@@ -1128,7 +1127,7 @@ bool gemm_mfma_bf16_parts(const void* a, bool tA, int64_t lda, const void* b, bo
 // ---- the tied head's cross-entropy inside its logits product ----
 namespace {
 bool head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K) {
-    if (!takes(a, false, lda, b, true, ldb, M, N, K)) return false;
+    if (!takes(a, false, lda, b, true, ldb, M, N, K, true)) return false;
     const int64_t ext_max = (int64_t{1} << 30) - 8192;
     return M * lda * 2 < ext_max && N * ldb * 2 < ext_max && lda < (1 << 21) && ldb < (1 << 21) && N < (1 << 20);
 }
@@ -1146,14 +1145,22 @@ void launch_head(GemmArgs g, const HeadArgs& hd, hipStream_t st) {
 }  // namespace
 
 // 256 x 256 tiles, one workgroup of eight wavefronts per CU (128 x 128 tiles with two workgroups per CU, whose
-// epilogues could overlap each other's matrix work, measured 15 % slower on [2048, 32000] x 512)
+// epilogues could overlap each other's matrix work, measured 15 % slower on [2048, 32000] x 512), unless those are fewer
+// than three quarters of the CUs.
+namespace {
+bool head_small(int64_t M, int64_t N) {
+    return ((M + GeoLarge::BM - 1) / GeoLarge::BM) * ((N + GeoLarge::BN - 1) / GeoLarge::BN) < cu_count() * 3 / 4;
+}
+}  // namespace
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K) {
     return head_takes(a, lda, b, ldb, M, N, K);
 }
-int64_t gemm_head_spans(int64_t N) { return (N + GeoLarge::BN - 1) / GeoLarge::BN * GeoLarge::WGN; }
+int64_t gemm_head_spans(int64_t M, int64_t N) {
+    return head_small(M, N) ? (N + GeoSmall::BN - 1) / GeoSmall::BN * GeoSmall::WGN : (N + GeoLarge::BN - 1) / GeoLarge::BN * GeoLarge::WGN;
+}
 
 // Pass 1 over logits = A B^T (A [M, K] and B [N, K], bf16), which are formed tile by tile and never stored: per row
-// its maximum, 1 / sum exp(z - maximum) and its loss against target[row]. `stats` is scratch of gemm_head_spans(N) * M
+// its maximum, 1 / sum exp(z - maximum) and its loss against target[row]. `stats` is scratch of gemm_head_spans(M, N) * M
 // pairs of floats, `zt` of M floats. False, with nothing done, for operands the kernel does not take.
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,
                     void* stats, float* zt, float* row_max, float* row_inv, float* nll, hipStream_t st) {
@@ -1163,19 +1170,20 @@ bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int6
     hd.target = target;
     hd.stats = static_cast<float2*>(stats);
     hd.zt = zt;
-    launch_head<GeoLarge, 1>(g, hd, st);
+    head_small(M, N) ? launch_head<GeoSmall, 1>(g, hd, st) : launch_head<GeoLarge, 1>(g, hd, st);
     hipLaunchKernelGGL(head_rows, dim3(static_cast<unsigned>((M + 15) / 16)), dim3(256), 0, st, hd.stats, zt,
-                       static_cast<int>(gemm_head_spans(N)), static_cast<int>(M), row_max, row_inv, nll);
+                       static_cast<int>(gemm_head_spans(M, N)), static_cast<int>(M), row_max, row_inv, nll);
     hip_check(hipGetLastError(), "head_rows launch");
     return true;
 }
 
 // Pass 2: the same tiles again, stored as dlogits[M, N] (bf16, row pitch ldc) =
-// (exp(z - row_max) row_inv - [column == target]) gscale (src/ops.cpp:371-374).
+// (exp(z - row_max) row_inv - [column == target]) gscale (src/ops.cpp:371-374). N is a multiple of 8 here: a vocabulary
+// that is not comes padded, and its last columns are what rows of zeros in B give.
 bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
                        const int* target, const float* row_max, const float* row_inv, float gscale, void* dl, int64_t ldc,
                        hipStream_t st) {
-    if (!head_takes(a, lda, b, ldb, M, N, K) || !aligned16(dl) || ldc % 8 || ldc >= (1 << 20)) return false;
+    if (!head_takes(a, lda, b, ldb, M, N, K) || !aligned16(dl) || N % 8 || ldc % 8 || ldc >= (1 << 20)) return false;
     GemmArgs g = gemm_args(a, lda, b, ldb, M, N, K);
     g.c = dl;
     g.ldc = ldc;
@@ -1184,7 +1192,7 @@ bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, i
     hd.row_max = row_max;
     hd.row_inv = row_inv;
     hd.gscale = gscale;
-    launch_head<GeoLarge, 2>(g, hd, st);
+    head_small(M, N) ? launch_head<GeoSmall, 2>(g, hd, st) : launch_head<GeoLarge, 2>(g, hd, st);
     return true;
 }
 
@@ -1196,7 +1204,7 @@ bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, i
 // contractions. False, with nothing done, when an operand is not what the ring kernel takes or the tiles are too few
 // to be worth it (the caller then multiplies them one by one).
 bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStream_t st) {
-    if (count < 2 || count > GROUP_MAX || K < 2048) return false;
+    if (count < 2 || count > GROUP_MAX) return false;
     GroupArgs gr{};
     gr.count = count;
     int tiles = 0;
@@ -1220,8 +1228,9 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
     }
     for (int p = count; p < GROUP_MAX; ++p) gr.tile_end[p] = tiles;
     // worth it from about 3/8 of the CUs busy with whole contractions (measured: 196 tiles x 8192 in 69 us against 132
-    // for the same four products one by one); with more tiles than CUs the 4-wavefront form, two workgroups per CU
-    if (tiles < cu_count() * 3 / 8) return false;
+    // for the same four products one by one), and with any number of tiles where the contraction is short: a product of its
+    // own is 10 us or more there, with a pass over its partial sums, and the grouped launch takes about 0.4 us for 64 tokens
+    if (tiles < cu_count() * 3 / 8 && K > 640 * count) return false;
     GemmArgs g = gemm_args(ps[0].a, ps[0].lda, ps[0].b, ps[0].ldb, ps[0].M, ps[0].N, K);
     g.beta = 1;
     g.splits = 1;

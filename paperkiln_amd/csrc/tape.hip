@@ -51,13 +51,19 @@ TapeContext::Shadows& shadows() {
     return *c.shadows;
 }
 
+int64_t round_up8(int64_t n) { return (n + 7) / 8 * 8; }
+
 const Tensor& shadow_of(const Var& W) {
     const int compute = tape_context().compute;
     if (compute == PK_F32 || W->data.dtype != PK_F32) return W->data;
     auto& map = shadows().single;
     auto it = map.find(W.get());
     if (it == map.end()) {
-        Tensor t = Tensor::make(W->data.rows, W->data.cols, compute);
+        // rows up to a multiple of 8, the last ones zeros: an embedding whose vocabulary is none is multiplied as if it were
+        const int64_t rows = W->data.rows;
+        Tensor t = Tensor::make(round_up8(rows), W->data.cols, compute);
+        if (rows % 8) k_fill(t.row_range(rows, t.rows - rows), 0.0f);
+        t.rows = rows;
         k_cast(W->data, t);
         it = map.emplace(W.get(), std::move(t)).first;
     }
@@ -152,13 +158,12 @@ void flush_weight_gradients() {
 }
 
 // Whether dW += x^T dy[:, col0 : col0 + ncols] can wait in the queue: a backward pass is running and the product is one
-// the hand-written kernels take (operands of one type, fp32 parameter gradient; in bf16 aligned, and a contraction worth
-// grouping).
+// the hand-written kernels take (operands of one type, fp32 parameter gradient; in bf16 aligned).
 bool weight_gradient_can_wait(const Tensor& x, const Tensor& dy, int64_t col0, int64_t ncols, const Var& W) {
     if (pending().depth == 0 || gemm_backend() != 1) return false;
     if (x.dtype != dy.dtype || !W->is_param || x.rows != dy.rows || W->data.rows != x.cols || W->data.cols != ncols) return false;
     if (x.dtype == PK_BF16) {
-        if (x.rows < 2048 || x.cols % 8 || dy.cols % 8 || col0 % 8 || ncols % 8) return false;
+        if (x.cols % 8 || dy.cols % 8 || col0 % 8 || ncols % 8) return false;
     } else if (x.numel() >= (int64_t{1} << 29) || dy.numel() >= (int64_t{1} << 29)) {
         return false;
     }
@@ -880,6 +885,7 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
     // bf16 operands the library's own GEMM takes: the cross-entropy runs inside the logits product, which forms
     // every tile twice (row statistics and loss, then dlogits) instead of storing [rows, V] logits for a row kernel
     bool in_product = h->data.dtype == PK_BF16 && Ec.dtype == PK_BF16 && head_kernel() != 0 && gemm_backend() != 0 &&
+                      (V % 8 == 0 || E->data.dtype == PK_F32) &&  // a bf16 parameter has no padded copy
                       gemm_head_takes(h->data.ptr(), d, Ec.ptr(), d, std::min<int64_t>(N, chunk_rows > 0 ? chunk_rows : 4096), V, d);
     // default chunk: the same scratch either way (4096 rows of bf16 dlogits, or 2048 of fp32 logits: 262 MB at 32000 words)
     if (chunk_rows <= 0) chunk_rows = in_product ? 4096 : 2048;
@@ -890,15 +896,16 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
         Tensor dl;
         int64_t dl_ld = V;
         if (in_product) {
-            Buffer stats(sizeof(float) * 2 * static_cast<size_t>(gemm_head_spans(V)) * rows), rowf(sizeof(float) * 3 * rows);
+            Buffer stats(sizeof(float) * 2 * static_cast<size_t>(gemm_head_spans(rows, V)) * rows), rowf(sizeof(float) * 3 * rows);
             float* zt = static_cast<float*>(rowf.p);
             float* row_max = zt + rows;
             float* row_inv = row_max + rows;
             in_product = gemm_head_rows(hview.ptr(), d, Ec.ptr(), d, rows, V, d, tg + r0, stats.p, zt, row_max, row_inv, nll_r,
                                         tape_stream());
             if (in_product && grads) {
-                dl = Tensor::make(rows, V, PK_BF16);
-                if (!gemm_head_dlogits(hview.ptr(), d, Ec.ptr(), d, rows, V, d, tg + r0, row_max, row_inv, g1, dl.ptr(), V,
+                dl_ld = round_up8(V);  // the columns past V meet rows of zeros in E's padded copy
+                dl = Tensor::make(rows, dl_ld, PK_BF16);
+                if (!gemm_head_dlogits(hview.ptr(), d, Ec.ptr(), d, rows, dl_ld, d, tg + r0, row_max, row_inv, g1, dl.ptr(), dl_ld,
                                        tape_stream()))
                     throw std::runtime_error("linear_cross_entropy: the head's second pass refused what its first took");
             }
@@ -924,8 +931,12 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
                 }
             }
         }
-        if (want_dh)
-            gemm(dl, false, Ec, false, static_cast<char*>(dh1.ptr()) + r0 * d * hes, dh1.dtype, rows, d, d, 0.0f, dl_ld);
+        if (want_dh) {
+            Tensor Ek = Ec;
+            Ek.rows = dl.cols;  // V, or up to a multiple of 8 with the copy's rows of zeros
+            gemm(dl, false, Ek, false, static_cast<char*>(dh1.ptr()) + r0 * d * hes, dh1.dtype, rows, d, d, 0.0f, dl_ld);
+        }
+        dl.cols = V;
         if (want_dE) gemm(dl, true, hview, false, dE1.ptr(), PK_F32, V, d, d, r0 == 0 && !dE_in_place ? 0.0f : 1.0f, dl_ld);
     }
     Tensor out = Tensor::make(1, 1, PK_F32);

@@ -84,7 +84,7 @@ bool gemm_mfma_bf16_parts(const void* a, bool tA, int64_t lda, const void* b, bo
                           int64_t K, hipStream_t st, std::unique_ptr<Buffer>& part, int& nparts);
 // The tied head's cross-entropy inside its logits product A B^T (bf16 [M, K] and [N, K]): the logits are formed tile
 // by tile, twice, and never stored. gemm_head_rows: per row the maximum, 1 / sum exp(z - maximum) and the loss
-// (stats: scratch of gemm_head_spans(N) * M float pairs, zt: of M floats); gemm_head_dlogits: bf16 dlogits.
+// (stats: scratch of gemm_head_spans(M, N) * M float pairs, zt: of M floats); gemm_head_dlogits: bf16 dlogits.
 // Both return false, having done nothing, for operands the kernel does not take.
 // Several weight-gradient products C_p += A_p^T B_p (A_p [K, M_p], B_p [K, N_p] bf16; C_p [M_p, N_p] fp32) that share
 // the contraction length, as one launch of the hand-written kernel. False, with nothing done, where that does not
@@ -114,7 +114,7 @@ struct F32Product {
 };
 bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st);
 bool gemm_f32_is_ahead(bool tA, int64_t M, int64_t N, int64_t K);  // of the library, for one product of this size
-int64_t gemm_head_spans(int64_t N);
+int64_t gemm_head_spans(int64_t M, int64_t N);
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,
                     void* stats, float* zt, float* row_max, float* row_inv, float* nll, hipStream_t st);

@@ -34,6 +34,33 @@ def test_bf16_training_on_a_ragged_token_count(tokens, seq):
         m.close()
 
 
+@pytest.mark.parametrize("vocab,d,ff,layers,tokens,seq", [(301, 64, 176, 2, 77, 11), (1001, 128, 344, 1, 693, 77),
+                                                          (12345, 256, 688, 1, 2600, 650), (17, 64, 176, 1, 64, 0)])
+def test_bf16_training_with_any_vocabulary(vocab, d, ff, layers, tokens, seq):
+    """The tied head's cross-entropy inside its product, with a vocabulary padded to a multiple of 8 (small and large
+    tiles), and the weight gradients of few tokens in one launch. Against the library GEMM, same operands."""
+    m = Llama(vocab=vocab, d=d, n_layers=layers, n_heads=d // 32, d_ff=ff, compute_dtype="bf16", seed=8)
+    toks = synth.randint(3, tokens + 1, vocab)
+    toks[:4] = vocab - 1  # the last word is used, as input and as target
+    before = blockops.set_gemm_backend(0)
+    try:
+        want_loss, _ = m.loss_backward(toks[:-1], toks[1:], seq)
+        want = m.grads()
+        blockops.set_gemm_backend(1)
+        for ck in (False, True):
+            loss, _ = m.loss_backward(toks[:-1], toks[1:], seq, checkpoint=ck)
+            assert abs(loss - want_loss) < 1e-3
+            assert rel(m.grads(), want) < 2e-2
+        assert m.loss_backward(toks[:-1], toks[1:], seq, backward=False)[0] == loss
+        m.adamw_step(1e-3)  # the padded copy is refreshed in place
+        a, _ = m.loss_backward(toks[:-1], toks[1:], seq)
+        blockops.set_gemm_backend(0)
+        assert abs(a - m.loss_backward(toks[:-1], toks[1:], seq)[0]) < 1e-3
+    finally:
+        blockops.set_gemm_backend(before)
+        m.close()
+
+
 def exact_attention(q, k, v, d_o, scale, causal, window, sinks):
     """O, LSE, dQ, dK, dV in float64 (src/ops.cpp:863-1027) of [B,T,H,dk] tensors, K / V heads shared by groups."""
     q, k, v, d_o = (x.double().permute(0, 2, 1, 3).contiguous() for x in (q, k, v, d_o))
