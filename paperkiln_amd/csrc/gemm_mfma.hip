@@ -1077,8 +1077,12 @@ GemmArgs gemm_args(const void* a, int64_t lda, const void* b, int64_t ldb, int64
 // that are not multiples of 8): the caller then uses the library GEMM.
 bool gemm_mfma_bf16(const void* a, bool tA, int64_t lda, const void* b, bool tB, int64_t ldb, void* c, int c_dtype,
                     int64_t M, int64_t N, int64_t K, int64_t ldc, float beta, hipStream_t st, const void* addend) {
-    if (!takes(a, tA, lda, b, tB, ldb, M, N, K) || !aligned16(c) || ldc % 8) return false;
     if (beta != 0.0f && beta != 1.0f) return false;
+    if (g_force_geo < 0 && gemm_small_is_ahead(tA, tB, M, N, K)) {
+        const SmallProduct p{a, lda, b, ldb, c, ldc, addend, M, N, K};
+        if (gemm_small(&p, 1, tA, tB, c_dtype, addend ? 0.0f : beta, st)) return true;
+    }
+    if (!takes(a, tA, lda, b, tB, ldb, M, N, K) || !aligned16(c) || ldc % 8) return false;
     GemmArgs g = gemm_args(a, lda, b, ldb, M, N, K);
     g.c = c;
     g.ldc = ldc;
@@ -1208,6 +1212,7 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
     GroupArgs gr{};
     gr.count = count;
     int tiles = 0;
+    int64_t small = 0;  // tiles of 32 x 32
     const int64_t ext_max = (int64_t{1} << 30) - 8192;
     for (int p = 0; p < count; ++p) {
         const GroupedProduct& q = ps[p];
@@ -1224,9 +1229,16 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
         gr.ldc[p] = static_cast<int>(q.ldc);
         gr.tiles_n[p] = static_cast<int>((q.N + 127) / 128);
         tiles += static_cast<int>((q.M + 127) / 128) * gr.tiles_n[p];
+        small += ((q.M + 31) / 32) * ((q.N + 31) / 32);
         gr.tile_end[p] = tiles;
     }
     for (int p = count; p < GROUP_MAX; ++p) gr.tile_end[p] = tiles;
+    if (g_force_geo < 0 && gemm_small_us(true, false, small, K) < (4.0 + 0.0105 * K) * ((tiles + cu_count() - 1) / cu_count())) {
+        SmallProduct sp[GROUP_MAX];
+        for (int p = 0; p < count; ++p)
+            sp[p] = SmallProduct{ps[p].a, ps[p].lda, ps[p].b, ps[p].ldb, ps[p].c, ps[p].ldc, nullptr, ps[p].M, ps[p].N, K};
+        if (gemm_small(sp, count, true, false, PK_F32, 1.0f, st)) return true;
+    }
     // worth it from about 3/8 of the CUs busy with whole contractions (measured: 196 tiles x 8192 in 69 us against 132
     // for the same four products one by one), and with any number of tiles where the contraction is short: a product of its
     // own is 10 us or more there, with a pass over its partial sums, and the grouped launch takes about 0.4 us for 64 tokens

@@ -1,0 +1,242 @@
+// The bf16 matrix product where it is small: C = op(A) op(B) (+ C or an addend), row-major, up to eight products in one
+// launch, bf16 operands, fp32 accumulation.
+//
+// gemm_mfma.hip feeds 128 x 128 tiles through a ring in LDS. A projection of a few hundred tokens is a handful of those,
+// over a contraction of a few slices, and takes 5 to 8 us of prologue, pipeline fill and strip-wise store, on a
+// fraction of the CUs. Here a workgroup's four or eight wavefronts share a 32 x 32 tile and split its contraction,
+// load their fragments from global memory straight into the layout the instruction reads -- everything a short
+// contraction needs is in flight at once -- and meet once, in LDS, in a fixed order. What bounds it is that one round
+// trip. Operands cross the L2 once per 32 rows, so it is behind as soon as the tiles are many (gemm_small_us).
+#include "mfma_common.h"
+#include "tensor.h"
+
+#include <algorithm>
+
+namespace pk {
+namespace {
+
+struct Jobs {
+    static constexpr int MAX = 8;
+    int count;
+    int first[MAX + 1];  // job j's tiles are first[j] .. first[j + 1] - 1
+    const uint16_t* a[MAX];
+    const uint16_t* b[MAX];
+    void* c[MAX];
+    const void* addend[MAX];
+    int lda[MAX], ldb[MAX], ldc[MAX], M[MAX], N[MAX], K[MAX];
+};
+constexpr int KC = 32;  // steps of the contraction per chunk: one v_mfma_f32_16x16x32_bf16
+
+__host__ __device__ inline int64_t extent(int64_t rows, int64_t cols, int64_t ld) { return ((rows - 1) * ld + cols) * 2; }
+
+// One chunk for two interleaved blocks of 16 rows (of A) or columns (of B): lane l holds of block b row or column
+// 2 (l % 16) + b, steps 8 (l / 16) .. + 7. PAIRS: the steps are rows of the operand, and one dword of a row holds the lane's
+// place in both blocks; otherwise the steps are adjacent, 16 bytes a lane, 64 a row. Interleaved rather than side by side, so
+// that both kinds of operand fit each other and a lane's two columns of C are one dword of bf16.
+template <bool PAIRS>
+struct Chunk {
+    u32x4 raw[2];  // PAIRS: dwords of steps 0-3, 4-7; otherwise the two blocks' fragments
+    __device__ void load(__amdgpu_buffer_rsrc_t p, const int (&off)[2], int k0, int ld) {
+        if (PAIRS) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) raw[e / 4][e % 4] = __builtin_amdgcn_raw_buffer_load_b32(p, off[0], (k0 + e) * ld * 2, 0);
+        } else {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) raw[b] = __builtin_amdgcn_raw_buffer_load_b128(p, off[b], k0 * 2, 0);
+        }
+    }
+    __device__ void clear_first(int n, int grp) {  // zeros for the first n steps of the chunk (an even number if !PAIRS)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int step = 8 * grp + (PAIRS ? 4 * h + e : 2 * e);
+                raw[h][e] = step < n ? 0u : raw[h][e];
+            }
+    }
+    __device__ bf16x8 block(int b) const {
+        u32x4 f = raw[b];
+        if (PAIRS) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)  // steps 2e, 2e + 1 of the low (b = 0) or high halves
+                f[e] = __builtin_amdgcn_perm(raw[e / 2][e % 2 * 2 + 1], raw[e / 2][e % 2 * 2], b == 0 ? 0x05040100u : 0x07060302u);
+        }
+        return *reinterpret_cast<const bf16x8*>(&f);
+    }
+};
+
+template <bool TA, bool TB, bool CF32, int KW>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs jobs, const int tiles, const int accumulate) {
+    constexpr int BUFS = 4;
+    // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
+    const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (t >= tiles) return;
+    int j = 0;
+    while (t >= jobs.first[j + 1]) ++j;
+    const int M = jobs.M[j], N = jobs.N[j], K = jobs.K[j], lda = jobs.lda[j], ldb = jobs.ldb[j];
+    const int tn = (N + 31) / 32, m0 = ((t - jobs.first[j]) / tn) * 32, n0 = ((t - jobs.first[j]) % tn) * 32;
+    const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, grp = lane >> 4;
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(jobs.a[j]), 0,
+                                                      static_cast<int>(extent(TA ? K : M, TA ? M : K, lda)), 0x00020000);
+    const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(jobs.b[j]), 0,
+                                                      static_cast<int>(extent(TB ? N : K, TB ? K : N, ldb)), 0x00020000);
+    int oa[2], ob[2];  // rows and columns past the edge read the last ones; they are not stored
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        oa[b] = TA ? (8 * grp * lda + min(m0 + 2 * l16, M - 2)) * 2 : (min(m0 + 2 * l16 + b, M - 1) * lda + 8 * grp) * 2;
+        ob[b] = TB ? (min(n0 + 2 * l16 + b, N - 1) * ldb + 8 * grp) * 2 : (8 * grp * ldb + min(n0 + 2 * l16, N - 2)) * 2;
+    }
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    Chunk<TA> fa[BUFS];
+    Chunk<!TB> fb[BUFS];
+    const int chunks = (K + KC - 1) / KC;
+    auto load = [&](int chunk, int buf) {
+        // the last chunk of a contraction that is no multiple is moved back to end where that does: its first steps are done
+        const int over = max((chunk + 1) * KC - K, 0), k0 = chunk * KC - over;
+        fa[buf].load(ra, oa, k0, lda);
+        fb[buf].load(rb, ob, k0, ldb);
+        if (over > 0) {
+            fa[buf].clear_first(over, grp);
+            fb[buf].clear_first(over, grp);
+        }
+    };
+    auto multiply = [&](int buf) {
+        const bf16x8 a0 = fa[buf].block(0), a1 = fa[buf].block(1), b0 = fb[buf].block(0), b1 = fb[buf].block(1);
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[0][0], 0, 0, 0);
+        acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[0][1], 0, 0, 0);
+        acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[1][0], 0, 0, 0);
+        acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[1][1], 0, 0, 0);
+    };
+    const int mine = kw < chunks ? (chunks - kw + KW - 1) / KW : 0;  // chunks kw, kw + KW, ... are this wavefront's
+#pragma unroll
+    for (int u = 0; u < BUFS; ++u)
+        if (u < mine) load(kw + u * KW, u);
+    __builtin_amdgcn_sched_barrier(0);
+    int i = 0;
+    for (; i + BUFS <= mine; i += BUFS) {
+#pragma unroll
+        for (int u = 0; u < BUFS; ++u) {
+            multiply(u);
+            if (i + u + BUFS < mine) load(kw + (i + u + BUFS) * KW, u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < BUFS - 1; ++u)
+        if (i + u < mine) multiply(u);
+
+    // lane (l16, grp), register r of block (x, y): row m0 + 2 (4 grp + r) + x, column n0 + 2 l16 + y
+    __shared__ f32x4 part[KW][2][2][64];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) part[kw][x][y][lane] = acc[x][y];
+    __syncthreads();
+    constexpr int RPW = 8 / KW;  // of the 2 x 4 rows a lane holds, each wavefront adds up this many
+    const int n = n0 + 2 * l16;
+    if (n >= N) return;
+    const int64_t ldc = jobs.ldc[j];
+#pragma unroll
+    for (int q = 0; q < RPW; ++q) {
+        const int row = kw * RPW + q, x = row >> 2, r = row & 3;
+        float s0 = reinterpret_cast<const float*>(&part[0][x][0][lane])[r], s1 = reinterpret_cast<const float*>(&part[0][x][1][lane])[r];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) {
+            s0 += reinterpret_cast<const float*>(&part[k][x][0][lane])[r];
+            s1 += reinterpret_cast<const float*>(&part[k][x][1][lane])[r];
+        }
+        const int m = m0 + 2 * (4 * grp + r) + x;
+        if (m >= M) continue;
+        const int64_t o = m * ldc + n;
+        const void* const add = jobs.addend[j] ? jobs.addend[j] : accumulate ? jobs.c[j] : nullptr;
+        if (CF32) {
+            f32x2 v = {s0, s1};
+            if (add) {
+                const f32x2 e = *reinterpret_cast<const f32x2*>(static_cast<const float*>(add) + o);
+                v[0] += e[0], v[1] += e[1];
+            }
+            *reinterpret_cast<f32x2*>(static_cast<float*>(jobs.c[j]) + o) = v;
+        } else {
+            if (add) {
+                const uint32_t e = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(add) + o);
+                s0 += __uint_as_float(e << 16), s1 += __uint_as_float(e & 0xffff0000u);
+            }
+            *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.c[j]) + o) = pack_bf16(s0, s1);
+        }
+    }
+}
+
+template <bool TA, bool TB, bool CF32>
+void launch(Jobs& jobs, bool accumulate, hipStream_t st) {
+    int tiles = 0, longest = 0;
+    for (int j = 0; j < jobs.count; ++j) {
+        jobs.first[j] = tiles;
+        tiles += ((jobs.M[j] + 31) / 32) * ((jobs.N[j] + 31) / 32);
+        longest = std::max(longest, jobs.K[j]);
+    }
+    for (int j = jobs.count; j <= Jobs::MAX; ++j) jobs.first[j] = tiles;
+    const dim3 grid((tiles + 7) / 8 * 8);
+    // eight wavefronts where each still has a few chunks and two workgroups fit every CU
+    if (longest >= 512 && tiles <= 1024)
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 8>), grid, dim3(512), 0, st, jobs, tiles, accumulate ? 1 : 0);
+    else
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 4>), grid, dim3(256), 0, st, jobs, tiles, accumulate ? 1 : 0);
+    hip_check(hipGetLastError(), "gemm_small");
+}
+
+}  // namespace
+
+// Microseconds that this kernel takes, and the ring kernels (one product; several, grouped), as fitted to 250 sizes of 64 to 8192 tokens,
+// widths 64 to 512 and vocabularies of 4000. Here a workgroup is a chain of its contraction's loads, and the launch all
+// its tiles' operands through the L2s, in rounds of 256 tiles; there a tile is a chain of slices, cut up from 2048 on.
+// (512 tokens: 128 x 384 projection 3.1 and 4.6, 344 x 128 3.5 and 6.2, its two gradients 3.8 and 7.5, 4.5 and 8.8;
+// 4096 tokens, 512 x 1536: 30 and 12.)
+double gemm_small_us(bool tA, bool tB, int64_t tiles, int64_t K) {
+    const double chain = tA ? 0.0019 : tB ? 0.0035 : 0.0022, stream = tA ? 1.0e-5 : tB ? 1.3e-5 : 0.9e-5;
+    return 2.8 + std::max(chain * K, static_cast<double>((tiles + 255) / 256 * 256) * (0.0011 + stream * K));
+}
+bool gemm_small_is_ahead(bool tA, bool tB, int64_t M, int64_t N, int64_t K) {
+    const double ring = K >= 2048 ? (tA ? 13.5 : 15.5) : (tA ? 4.0 : 3.6) + 0.0072 * K;
+    return gemm_small_us(tA, tB, ((M + 31) / 32) * ((N + 31) / 32), K) < ring;
+}
+
+bool gemm_small(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st) {
+    if (count < 1 || count > Jobs::MAX || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
+    Jobs jobs{};
+    jobs.count = count;
+    for (int j = 0; j < count; ++j) {
+        const SmallProduct& p = ps[j];
+        const int64_t limit = int64_t{1} << 30;
+        if (p.M < 2 || p.N < 2 || p.K < KC || p.M > limit || p.N > limit || p.K > limit) return false;
+        if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= limit || extent(tB ? p.N : p.K, tB ? p.K : p.N, p.ldb) >= limit) return false;
+        // pairs of columns, and of steps where those are adjacent, are read and written as one
+        auto aligned = [](const void* q, int a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
+        if (p.lda % 2 || p.ldb % 2 || p.ldc % 2 || p.N % 2 || (tA && p.M % 2) || (!(tA && !tB) && p.K % 2)) return false;
+        if (!aligned(p.a, 4) || !aligned(p.b, 4) || !aligned(p.c, 8) || !aligned(p.addend, 8)) return false;
+        jobs.a[j] = static_cast<const uint16_t*>(p.a);
+        jobs.b[j] = static_cast<const uint16_t*>(p.b);
+        jobs.c[j] = p.c;
+        jobs.addend[j] = p.addend;
+        jobs.lda[j] = static_cast<int>(p.lda);
+        jobs.ldb[j] = static_cast<int>(p.ldb);
+        jobs.ldc[j] = static_cast<int>(p.ldc);
+        jobs.M[j] = static_cast<int>(p.M);
+        jobs.N[j] = static_cast<int>(p.N);
+        jobs.K[j] = static_cast<int>(p.K);
+    }
+    const bool f32 = c_dtype == PK_F32, acc = beta != 0.0f;
+    if (tA)
+        f32 ? launch<true, false, true>(jobs, acc, st) : launch<true, false, false>(jobs, acc, st);
+    else if (tB)
+        f32 ? launch<false, true, true>(jobs, acc, st) : launch<false, true, false>(jobs, acc, st);
+    else
+        f32 ? launch<false, false, true>(jobs, acc, st) : launch<false, false, false>(jobs, acc, st);
+    return true;
+}
+
+}  // namespace pk

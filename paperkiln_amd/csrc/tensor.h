@@ -99,6 +99,22 @@ struct GroupedProduct {
     int64_t M, N;
 };
 bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStream_t st);
+// gemm_small.hip: C_p = op(A_p) op(B_p) + (addend_p, or C_p if beta is 1), bf16 operands, C of c_dtype, for up to eight
+// products of one orientation in one launch; for sizes where tiles of 128 x 128 are few. False, with nothing done, for
+// operands it does not take (odd pitches or sizes, both transposed, a contraction below 32, a gigabyte or more).
+struct SmallProduct {
+    const void* a;
+    int64_t lda;
+    const void* b;
+    int64_t ldb;
+    void* c;
+    int64_t ldc;
+    const void* addend;  // C's type and row pitch; may be null
+    int64_t M, N, K;
+};
+bool gemm_small(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st);
+bool gemm_small_is_ahead(bool tA, bool tB, int64_t M, int64_t N, int64_t K);  // of gemm_mfma.hip's tiles, for one product
+double gemm_small_us(bool tA, bool tB, int64_t tiles, int64_t K);               // tiles of 32 x 32, of all products together
 // gemm_f32.hip: C_p = op(A_p) op(B_p) + (addend_p, or C_p if beta is 1) for up to eight products of one orientation in one
 // launch, fp32 throughout on the matrix cores; any sizes and row pitches. False, with nothing done, if A and B are both
 // transposed or an operand has 2 GiB or more.

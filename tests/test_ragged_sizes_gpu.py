@@ -173,6 +173,25 @@ def test_fp32_products(M, N, K, tA, tB):
         assert err < 4e-7 * (K + 16) ** 0.5 * 4, (accumulate, float(err))
 
 
+@pytest.mark.parametrize("c_dtype", [torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K", [(2, 2, 32), (34, 66, 34), (64, 32, 64), (62, 30, 344), (2, 40, 1002), (126, 130, 700), (1000, 64, 66)])
+def test_small_bf16_products(M, N, K, tA, tB, c_dtype):
+    """The bf16 GEMM of few tiles at the edges of those (32), of its contraction chunks (an odd length where both operands
+    have it as rows) and of the split among four and eight wavefronts, with and without the sum onto C."""
+    K += tA
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b = (torch.randn(s, generator=gen, device="cuda").bfloat16() for s in ((K, M) if tA else (M, K), (N, K) if tB else (K, N)))
+    c0 = torch.randn((M, N), generator=gen, device="cuda").to(c_dtype)
+    want = (a.double().T if tA else a.double()) @ (b.double().T if tB else b.double())
+    for out in (None, c0.clone()):
+        got = blockops.matmul(a, b, bool(tA), bool(tB), out_dtype=c_dtype, out=out)
+        torch.cuda.synchronize()
+        exact = want + (0 if out is None else c0.double())
+        err = ((got.double() - exact).abs() - (exact.abs() / 256 if c_dtype == torch.bfloat16 else 0)).max()
+        assert err < 2e-6 * K ** 0.5 * 4, float(err)
+
+
 @pytest.mark.parametrize("vocab,d,ff,tokens,seq", [(101, 64, 176, 77, 11), (301, 96, 256, 700, 100), (130, 64, 176, 4100, 820)])
 def test_fp32_training_on_ragged_sizes(vocab, d, ff, tokens, seq):
     """A whole fp32 pass (weight gradients of a block in one launch, residual sums in the products, the embedding's
