@@ -546,7 +546,7 @@ int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 int launch_f32_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     a.head_split = dkdv_splits(a);
-    if (!split_tail_pays(a, a.head_split)) a.tail = nullptr;
+    if (!split_tail_pays(a, a.head_split, 32)) a.tail = nullptr;
     const bool eight = dkdv_form(a) == Form::EIGHT;
     if (a.dk_dim <= 32)
         eight ? run_dkdv<32, 8>(a, st) : run_dkdv<32, 4>(a, st);

@@ -653,7 +653,7 @@ int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     a.head_split = dkdv_splits(a);
-    if (!split_tail_pays(a, a.head_split)) a.tail = nullptr;
+    if (!split_tail_pays(a, a.head_split, dkdv_form(a) == Form::WIDE ? 128 : 32)) a.tail = nullptr;
     const auto run = [&]() -> int {
 #define PK_CALL(D, E) dkdv_of<D, E>(a, dkdv_form(a), st)
         PK_SPLIT_DISPATCH(PK_CALL);

@@ -118,9 +118,10 @@ __host__ inline bool sink_tail_pays(const SinkTail& t, int T, int window, int kv
 __host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window) {
     const int rep = Hq / Hkv;
     if (rep <= 1 || dk % 4 != 0 || dk > 128) return 1;
-    const int nkb = (T + 127) / 128;
+    // with a band only the 32-key kernels split, and without the split they fill the chip with a quarter of the sequence
+    const int nkb = window > 0 ? (T + 31) / 32 : (T + 127) / 128;
     const long long wgs = static_cast<long long>(causal && window == 0 ? (nkb + 1) / 2 : nkb) * B * Hkv;
-    if (wgs >= 384) return 1;  // at least one and a half workgroups per CU already
+    if (wgs >= (window > 0 ? 96 : 384)) return 1;  // without a band: one and a half workgroups per CU
     const int hs = static_cast<int>((512 + wgs - 1) / wgs);
     return hs < rep ? hs : rep;
 }
