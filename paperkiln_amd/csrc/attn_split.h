@@ -92,7 +92,7 @@ inline bool even_chains(const AttnArgs& a) { return !a.causal || chain_tokens(a)
 // Whether a dK/dV launch deals the queries past the band of the sink keys' block to workgroups of their own (sink_tail): the
 // block's chain through all of them, against the rest of the launch, two workgroups to a CU with a band of queries and about
 // three tiles of overhead each. (fp32, head_dim 64, T 2476, window 64, 4 sinks, 4 heads: 86 us with that chain.)
-// (bf16, head_dim 32, T 4213, window 1224, 16 sinks, 8 heads, blocks of 128 rows: 355 us with it, 151 without.)
+// (bf16, head_dim 32, T 4213, window 1224, 16 sinks, 8 heads, blocks of 128 rows: 355 us with that chain, 146 with the tail dealt out.)
 inline bool split_tail_pays(const AttnArgs& a, int head_split, int block_rows) {
     const SinkTail t = sink_tail(a.T, a.window, a.sinks);
     const int64_t blocks = static_cast<int64_t>((a.T + block_rows - 1) / block_rows) * a.Hkv * a.B * head_split;
