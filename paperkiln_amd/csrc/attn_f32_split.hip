@@ -115,8 +115,10 @@ __device__ inline void accumulate_tr32(const float* tile, const f32x16& c, f32x1
 }
 
 // ---- forward ----
+// The launch bounds ask for the wavefronts that the LDS leaves room for: four to a SIMD at head_dim 32, two at 64 (backward,
+// head_dim 24, T 402 x 22, 16 heads: 204 -> 173 us; head_dim 64, T 731 x 4, 28 heads on 4, window 309: 296 -> 242).
 template <int D, int KW>
-__global__ __launch_bounds__(64 * KW) void f32_split_fwd(AttnArgs a) {
+__global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_fwd(AttnArgs a) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P, RED = KW * (DB * 1024 + 128);
     __shared__ __attribute__((aligned(16))) float lds[KW * TILE > RED ? KW * TILE : RED];
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(64 * KW) void f32_split_fwd(AttnArgs a) {
 
 // ---- dQ (and delta, when asked for with it) ----
 template <int D, int KW>
-__global__ __launch_bounds__(64 * KW) void f32_split_dq(AttnArgs a, int fuse_delta) {
+__global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_dq(AttnArgs a, int fuse_delta) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P, RED = KW * DB * 1024;
     __shared__ __attribute__((aligned(16))) float lds[KW * TILE > RED ? KW * TILE : RED];
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -288,7 +290,7 @@ __global__ __launch_bounds__(64 * KW) void f32_split_dq(AttnArgs a, int fuse_del
 
 // ---- dK, dV: a block of 32 keys, the query tiles (of every query head of the group in turn) split ----
 template <int D, int KW>
-__global__ __launch_bounds__(64 * KW) void f32_split_dkdv(AttnArgs a) {
+__global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) void f32_split_dkdv(AttnArgs a) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P + 64, RED = KW * DB * 1024;
     // K and V of the block stay in LDS, one copy for all wavefronts, where registers are short and the LDS has the room
     // (at D = 128 for K only)

@@ -18,6 +18,10 @@ namespace pk {
 namespace {
 
 constexpr float LOG2E = 1.4426950408889634f;
+// The maximum that P is formed against moves only when a row outgrows it by this many powers of two: some row of 32 finds a
+// new maximum in most tiles, and rescaling costs three instructions per accumulator element. P then reaches 2^6, which its
+// operands and the fp32 sums hold as they hold 1.
+constexpr float LAZY_T = 6.0f;
 
 // A tile of ROWS rows of a [T, dk] bf16 matrix, moved by G threads: thread t of the group carries the 16-byte chunks
 // t, t + G, ... Rows past T and chunks past dk read as zero.
@@ -88,23 +92,32 @@ __device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, 
         h0 = c_to_operand<0>(c);
         h1 = c_to_operand<1>(c);
     }
+    // a product that waits for the one before it takes half as long again: the rounded operand into every block, then the
+    // remainder
+    bf16x8 m[DB];
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-        const bf16x8 m = lds_read_tr_operand(tile, pitch, row0, db * 32, lane);
-        acc[db] = mfma32(m, h0, acc[db]);
-        if (EXACT) acc[db] = mfma32(m, l0, acc[db]);
-    }
+    for (int half = 0; half < 2; ++half) {
+        const bf16x8 h = half ? h1 : h0, l = half ? l1 : l0;
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-        const bf16x8 m = lds_read_tr_operand(tile, pitch, row0 + 16, db * 32, lane);
-        acc[db] = mfma32(m, h1, acc[db]);
-        if (EXACT) acc[db] = mfma32(m, l1, acc[db]);
+        for (int db = 0; db < DB; ++db) {
+            m[db] = lds_read_tr_operand(tile, pitch, row0 + 16 * half, db * 32, lane);
+            acc[db] = mfma32(m[db], h, acc[db]);
+        }
+        if (EXACT)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) acc[db] = mfma32(m[db], l, acc[db]);
     }
 }
 
+// The launch bounds of all three kernels ask for two wavefronts to a SIMD where the registers allow it. Left to itself the
+// compiler kept the accumulators of head sizes above 64 in accumulation registers beside 200 others, one wavefront to a SIMD,
+// whose products, exponentials and LDS reads then took turns; within 256 registers they need no copies either. Forward, B=2
+// T=4096 H=16 (with the alternating products and the lazy maximum below): head_dim 96 261 -> 179 us, 48 166 -> 137, 32 104 ->
+// 93; backward 594 -> 542, 416 -> 360, 313 -> 259.
+
 // ---- forward: QW groups of 32 queries x KW groups of key tiles of 32 NB keys ----
 template <int D, int QW, int KW, int NB, bool EXACT>
-__global__ __launch_bounds__(64 * QW * KW) void split_fwd(AttnArgs a) {
+__global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW;
     constexpr int KS = D + 8;                              // row reads conflict-free
     constexpr int VS = (D / 32) % 2 ? D : D + 32;          // 4-row transposing reads conflict-free
@@ -169,14 +182,31 @@ __global__ __launch_bounds__(64 * QW * KW) void split_fwd(AttnArgs a) {
         }
         if (any) {
             float mx = -INFINITY;
+            bool all = true;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                all = all && live[nb];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[nb][r] = 0.0f;
+            }
+            if (NB > 1 && all) {  // alternating: independent products follow one another
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+                        s[nb] = mfma32(lds_read8(Ks + (nb * 32 + c32) * KS + kk * 16 + g * 8), qreg[kk], s[nb]);
+            } else {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    if (!live[nb]) continue;
+#pragma unroll
+                    for (int kk = 0; kk < KK; ++kk)
+                        s[nb] = mfma32(lds_read8(Ks + (nb * 32 + c32) * KS + kk * 16 + g * 8), qreg[kk], s[nb]);
+                }
+            }
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 if (!live[nb]) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[nb][r] = 0.0f;
-#pragma unroll
-                for (int kk = 0; kk < KK; ++kk)
-                    s[nb] = mfma32(lds_read8(Ks + (nb * 32 + c32) * KS + kk * 16 + g * 8), qreg[kk], s[nb]);
                 const int k0 = n0 + nb * 32;
                 const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
                 if (kind != MaskKind::NONE) mask_block(s[nb], kind, vis, k0 + g * 4, -INFINITY);
@@ -184,7 +214,7 @@ __global__ __launch_bounds__(64 * QW * KW) void split_fwd(AttnArgs a) {
                 for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[nb][r]);
             }
             mx = xhalf_max(mx);
-            if (__any(mx > m)) {  // wavefront-uniform
+            if (__any((mx - m) * cexp > LAZY_T)) {  // wavefront-uniform, rare after the first tiles
                 const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f((m - mn) * cexp);
                 l *= alpha;
                 m = mn;
@@ -245,7 +275,7 @@ __global__ __launch_bounds__(64 * QW * KW) void split_fwd(AttnArgs a) {
 
 // ---- dQ (and delta, when asked for with it): the same blocks ----
 template <int D, int QW, int KW, int NB, bool EXACT>
-__global__ __launch_bounds__(64 * QW * KW) void split_dq(AttnArgs a, int fuse_delta) {
+__global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
     constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;  // in uint16
@@ -357,8 +387,8 @@ __global__ __launch_bounds__(64 * QW * KW) void split_dq(AttnArgs a, int fuse_de
 // A wavefront owns 32 keys (K and V resident as B operands, lane = key) and both accumulators, so P goes from its
 // exponentials into dV and into dS without leaving the registers. The steps are the query tiles that can see the block,
 // for every query head of the KV head's group in turn.
-template <int D, int QW, int KW, int NB, bool EXACT>
-__global__ __launch_bounds__(64 * QW * KW) void split_dkdv(AttnArgs a) {
+template <int D, int QW, int KW, int NB, bool EXACT, int OCC>
+__global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
     constexpr int BNK = 32 * QW, BMQ = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int ROWC = 2 * BMQ * 2;                    // LSE and delta of a tile's rows, in uint16
     constexpr int TILE = 2 * BMQ * S + ROWC, NBUF = QW > 1 ? 2 : 1;
@@ -590,7 +620,14 @@ void run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 template <int D, int QW, int KW, int NB, bool EXACT>
 void run_dkdv(const AttnArgs& a, hipStream_t st) {
     const int nkb = (a.T + 32 * QW - 1) / (32 * QW);
-    hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT>), dim3(xcd_grid(nkb + tail_blocks(a), a.head_split, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a);
+    const dim3 grid(xcd_grid(nkb + tail_blocks(a), a.head_split, a.Hkv * a.B));
+    // Two wavefronts to a SIMD cost head sizes up to 96 a few spilled registers: not while there is a workgroup for each CU at
+    // most (us of a backward, head_dim 80: T 4263, 6 heads, 204 workgroups, one | two 223 | 268; T 1466 x 9, 4 KV heads, 432:
+    // 216 | 201; T 743 x 19, 4 KV heads, 456: 715 | 639).
+    if (D == 96 && QW > 1 && static_cast<int64_t>(nkb) * a.head_split * a.Hkv * a.B > 256)
+        hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT, 2>), grid, dim3(64 * QW * KW), 0, st, a);
+    else
+        hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT, D <= 64 ? 2 : 1>), grid, dim3(64 * QW * KW), 0, st, a);
 }
 
 template <int D, bool EXACT>
