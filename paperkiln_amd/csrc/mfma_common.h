@@ -320,27 +320,30 @@ __host__ __device__ inline int xcd_grid_block0_first(int nblk, int kv_units) {
 __device__ inline bool xcd_map_block0_first(int nblk, int kv_units, int& blk, int& kvu) {
     const int xcd = blockIdx.x & 7, upx = kv_units / 8, left = kv_units & 7;  // whole units per XCD, units left over
     int j = static_cast<int>(blockIdx.x >> 3);
-    blk = 0;
-    if (left != 0 && j-- == 0) {  // block 0 of the left-over units, one per XCD
-        kvu = (kv_units & ~7) + xcd;
-        return xcd < left;
+    if (left != 0) {  // block 0 of the left-over units, one per XCD; the rest of them follows the others' block 0
+        const int loose = (left * (nblk - 1) + 7) / 8;
+        if (j == 0) {
+            blk = 0;
+            kvu = (kv_units & ~7) + xcd;
+            return xcd < left;
+        }
+        --j;
+        if (j >= upx && j < upx + loose) {
+            const int idx = (j - upx) * 8 + xcd;
+            blk = 1 + idx / left;
+            kvu = (kv_units & ~7) + idx % left;
+            return idx < left * (nblk - 1);
+        }
+        if (j >= upx) j -= loose;
     }
     if (j < upx) {
+        blk = 0;
         kvu = j * 8 + xcd;
-        return true;
+    } else {
+        j -= upx;
+        blk = 1 + j % (nblk - 1);
+        kvu = (j / (nblk - 1)) * 8 + xcd;
     }
-    j -= upx;
-    const int loose = (left * (nblk - 1) + 7) / 8;
-    if (j < loose) {
-        const int idx = j * 8 + xcd;
-        if (idx >= left * (nblk - 1)) return false;
-        blk = 1 + idx / left;
-        kvu = (kv_units & ~7) + idx % left;
-        return true;
-    }
-    j -= loose;
-    blk = 1 + j % (nblk - 1);
-    kvu = (j / (nblk - 1)) * 8 + xcd;
     return true;
 }
 
