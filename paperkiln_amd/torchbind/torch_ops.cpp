@@ -148,6 +148,8 @@ struct AttentionBackward : public Node {
 };
 
 Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Mask& m) {
+    for (const Tensor* x : {&q, &k, &v})  // a tangent would be dropped without a word
+        if (x->_fw_grad(0).defined()) throw std::runtime_error("attention: forward-mode differentiation is not implemented");
     auto [o, lse] = forward(q, k, v, m);
     if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) {
         auto node = std::shared_ptr<AttentionBackward>(new AttentionBackward(torch::autograd::collect_next_edges(q, k, v)),

@@ -210,3 +210,11 @@ def test_fp32_training_on_ragged_sizes(vocab, d, ff, tokens, seq):
     finally:
         blockops.set_gemm_backend(before)
         m.close()
+
+
+def test_forward_mode_is_refused():
+    import torch.autograd.forward_ad as fwd
+
+    q, k, v, tangent = (torch.randn(1, 33, 2, 64, device="cuda") for _ in range(4))
+    with fwd.dual_level(), pytest.raises(RuntimeError):
+        ops.attention(fwd.make_dual(q, tangent), k, v, 0.125)
