@@ -573,12 +573,21 @@ bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
     if ((chain < 512 || a.dk_dim == 128) && blocks > 540) return true;
     return chain < 256 || (even_chains(a) && !(a.dk_dim == 64 && chain >= 768 && blocks <= 600));
 }
+// Head sizes other than 64 and 128, FOUR | WIDE. Many short chains of equal length are ahead unsplit from two blocks a CU on
+// (head_dim 80, T 64 x 87, 8 heads, no mask: forward 10.8 | 7.0 us, backward 43 | 28; T 2089, window 20: 16 | 12, 46 | 36), long
+// causal ones stay split for longer, the more so the fewer columns (forward: head_dim 32, T 3201 x 3, 4 heads 30 | 67, T 5179 x
+// 2, 8 heads 91 | 105; head_dim 96, T 1886 x 3, 8 heads 45 | 53, T 4618, 16 heads 148 | 128).
+bool wide_chains(const AttnArgs& a, int64_t blocks) { return a.dk_dim > 32 && even_chains(a) && chain_tokens(a) <= 160 && blocks > 550; }
 Form fwd_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     if (unsplit_is_ahead(a, blocks) || (plain && a.T <= 64)) return Form::NONE;
     if (blocks <= 256) return chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
-    if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
+    if (!plain) {
+        const int chain = chain_tokens(a);
+        const int64_t longest = a.dk_dim <= 32 ? (chain >= (a.causal ? 400 : 2000) ? 2600 : 1100) : (a.causal && chain >= 900 ? 1450 : 1100);
+        return blocks <= longest && !wide_chains(a, blocks) ? Form::FOUR : Form::WIDE;
+    }
     if (blocks <= 600)
         return chain_tokens(a) >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 && a.causal ? Form::FOUR : Form::NONE;
     return blocks <= 1100 && chain_tokens(a) >= 3000 ? Form::EIGHT : Form::NONE;
@@ -590,7 +599,10 @@ Form dq_form(const AttnArgs& a) {
     // above 96 columns eight wavefronts of this kernel do not fit the registers
     const Form best = a.dk_dim > 96 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
     if (blocks <= 256) return best;
-    if (!plain) return blocks <= 1100 ? Form::FOUR : Form::WIDE;
+    if (!plain) {  // T 5395, 8 heads, head_dim 32: a backward of 156 us against 253; T 1169 x 2, 16 heads, 80: 93 against 104
+        const bool far = a.causal && chain_tokens(a) >= (a.dk_dim <= 32 ? 1200 : 900);
+        return blocks <= (!far || a.dk_dim > 96 ? 1100 : a.dk_dim <= 32 ? 2600 : 1250) && !wide_chains(a, blocks) ? Form::FOUR : Form::WIDE;
+    }
     if (blocks <= 600) return chain_tokens(a) >= 1536 ? best : a.dk_dim == 64 || chain_tokens(a) >= 768 ? Form::FOUR : Form::NONE;
     return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 1000 ? Form::FOUR : Form::NONE;
 }
@@ -601,7 +613,11 @@ Form dkdv_form(const AttnArgs& a) {
     if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 72) && dkdv_splits(a) == 1))
         return Form::NONE;
     const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
-    if (!plain) return blocks <= 700 ? best : Form::WIDE;
+    if (!plain) {  // T 2933 x 2, 4 heads, head_dim 96: a backward of 127 us against 157; T 1714 x 2, 8 heads, 32: 52 against 65
+        const bool far = a.causal && chain_tokens(a) >= 1500 && a.dk_dim <= 96;
+        const bool wide = a.dk_dim > 64 && wide_chains(a, blocks);  // at 48, T 239 x 9, 8 KV heads, window 47, WIDE is behind: 31 | 27
+        return blocks <= (!far ? 700 : a.dk_dim <= 32 ? 1600 : 800) && !wide ? best : Form::WIDE;
+    }
     if (blocks <= 600) return best;
     return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 2000 ? best : Form::NONE;
 }
