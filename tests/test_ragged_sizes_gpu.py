@@ -218,3 +218,13 @@ def test_forward_mode_is_refused():
     q, k, v, tangent = (torch.randn(1, 33, 2, 64, device="cuda") for _ in range(4))
     with fwd.dual_level(), pytest.raises(RuntimeError):
         ops.attention(fwd.make_dual(q, tangent), k, v, 0.125)
+
+
+# Either side of the lines between chains that are split and those that are not, head sizes between the usual ones: many long
+# causal chains of few columns, many short ones of equal length.
+@pytest.mark.parametrize("case,dk", [((18, 511, 4, 4, True, 0, 0), 32), ((6, 1446, 4, 2, True, 0, 0), 96), ((36, 114, 4, 2, False, 0, 0), 112),
+                                     ((11, 812, 2, 2, True, 22, 0), 80), ((11, 111, 16, 16, True, 20, 16), 80)], ids=str)
+def test_lines_between_split_and_unsplit_chains(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.bfloat16, causal, window, sinks))
+    assert e[0] < 5e-3 and e[1] < 1e-5 and max(e[2:4]) < 5e-3 and e[4] < 2e-5, e
