@@ -78,6 +78,7 @@ struct HeadArgs {
     const float* row_max;  // pass 2: [M]
     const float* row_inv;  // pass 2: [M], 1 / sum_j exp(z_j - row_max)
     float gscale;          // pass 2
+    int vocab;             // pass 2: columns from here to N only pad the matrix; their dlogits are 0
 };
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -659,6 +660,16 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             for (int j = 0; j < FN; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], LOG2E, -ref));
+            if (hd.vocab < g.N && bl.n0 + BN > hd.vocab) {
+                // wavefront-uniform. The padding's logits are 0, not in the row's maximum: their exponentials overflow where
+                // every real logit lies far below 0, and dh would multiply the infinities with the zero rows that pad B.
+                const int col0 = bl.n0 + wn * FN * 32 + gh * 4;
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (col0 + j * 32 + (r >> 2) * 8 + (r & 3) >= hd.vocab) acc[i][j][r] = 0.0f;
+            }
             if (__builtin_amdgcn_ballot_w64(has) != 0) {  // few wavefronts hold a target column of one of their rows
                 const int at = has ? (tt >> 5) * 16 + ((tt >> 3) & 3) * 4 + (tt & 3) : -1;
 #pragma unroll
@@ -1183,11 +1194,11 @@ bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int6
 
 // Pass 2: the same tiles again, stored as dlogits[M, N] (bf16, row pitch ldc) =
 // (exp(z - row_max) row_inv - [column == target]) gscale (src/ops.cpp:371-374). N is a multiple of 8 here: a vocabulary
-// that is not comes padded, and its last columns are what rows of zeros in B give.
+// that is not comes padded with rows of zeros in B, and the columns from `vocab` on come out 0.
 bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                       const int* target, const float* row_max, const float* row_inv, float gscale, void* dl, int64_t ldc,
-                       hipStream_t st) {
-    if (!head_takes(a, lda, b, ldb, M, N, K) || !aligned16(dl) || N % 8 || ldc % 8 || ldc >= (1 << 20)) return false;
+                       int64_t vocab, const int* target, const float* row_max, const float* row_inv, float gscale, void* dl,
+                       int64_t ldc, hipStream_t st) {
+    if (!head_takes(a, lda, b, ldb, M, N, K) || !aligned16(dl) || N % 8 || vocab > N || ldc % 8 || ldc >= (1 << 20)) return false;
     GemmArgs g = gemm_args(a, lda, b, ldb, M, N, K);
     g.c = dl;
     g.ldc = ldc;
@@ -1196,6 +1207,7 @@ bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, i
     hd.row_max = row_max;
     hd.row_inv = row_inv;
     hd.gscale = gscale;
+    hd.vocab = static_cast<int>(vocab);
     head_small(M, N) ? launch_head<GeoSmall, 2>(g, hd, st) : launch_head<GeoLarge, 2>(g, hd, st);
     return true;
 }

@@ -903,10 +903,10 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
             in_product = gemm_head_rows(hview.ptr(), d, Ec.ptr(), d, rows, V, d, tg + r0, stats.p, zt, row_max, row_inv, nll_r,
                                         tape_stream());
             if (in_product && grads) {
-                dl_ld = round_up8(V);  // the columns past V meet rows of zeros in E's padded copy
+                dl_ld = round_up8(V);  // the columns past V are zeros and meet rows of zeros in E's padded copy
                 dl = Tensor::make(rows, dl_ld, PK_BF16);
-                if (!gemm_head_dlogits(hview.ptr(), d, Ec.ptr(), d, rows, dl_ld, d, tg + r0, row_max, row_inv, g1, dl.ptr(), dl_ld,
-                                       tape_stream()))
+                if (!gemm_head_dlogits(hview.ptr(), d, Ec.ptr(), d, rows, dl_ld, d, V, tg + r0, row_max, row_inv, g1, dl.ptr(),
+                                       dl_ld, tape_stream()))
                     throw std::runtime_error("linear_cross_entropy: the head's second pass refused what its first took");
             }
         }

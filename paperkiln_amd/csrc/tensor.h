@@ -84,7 +84,8 @@ bool gemm_mfma_bf16_parts(const void* a, bool tA, int64_t lda, const void* b, bo
                           int64_t K, hipStream_t st, std::unique_ptr<Buffer>& part, int& nparts);
 // The tied head's cross-entropy inside its logits product A B^T (bf16 [M, K] and [N, K]): the logits are formed tile
 // by tile, twice, and never stored. gemm_head_rows: per row the maximum, 1 / sum exp(z - maximum) and the loss
-// (stats: scratch of gemm_head_spans(M, N) * M float pairs, zt: of M floats); gemm_head_dlogits: bf16 dlogits.
+// (stats: scratch of gemm_head_spans(M, N) * M float pairs, zt: of M floats); gemm_head_dlogits: bf16 dlogits, of which the
+// columns from `vocab` on are 0 (N is the vocabulary padded to a multiple of 8, in the rows of b as well).
 // Both return false, having done nothing, for operands the kernel does not take.
 // Several weight-gradient products C_p += A_p^T B_p (A_p [K, M_p], B_p [K, N_p] bf16; C_p [M_p, N_p] fp32) that share
 // the contraction length, as one launch of the hand-written kernel. False, with nothing done, where that does not
@@ -135,8 +136,8 @@ bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,
                     void* stats, float* zt, float* row_max, float* row_inv, float* nll, hipStream_t st);
 bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                       const int* target, const float* row_max, const float* row_inv, float gscale, void* dl, int64_t ldc,
-                       hipStream_t st);
+                       int64_t vocab, const int* target, const float* row_max, const float* row_inv, float gscale, void* dl,
+                       int64_t ldc, hipStream_t st);
 // Which GEMM serves bf16 operands: 1 (default) and 2 = the hand-written kernel for everything it takes (1 also
 // groups a backward pass's weight-gradient products into shared launches), 0 = the library only. Set from the environment
 // (PK_GEMM=library) or by a caller that wants to compare them.

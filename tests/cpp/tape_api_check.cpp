@@ -302,13 +302,18 @@ void linear_add_case(int dtype, const char* name, int T, int din, int dout, doub
 }
 
 // The chunked tied head with the cross-entropy inside the logits product against the same head through fp32 logits
-// and the row kernel, on logits of a few tens in size (far from the ~0.01 of a freshly initialised model): the
-// in-product path carries the row maximum and the scaling in the exponent of exp2, which is where a large logit
-// would show.
-void head_case() {
-    std::printf("linear_cross_entropy, logits of size ~50: inside the product vs fp32 logits + row kernel\n");
-    const int T = 300, d = 64, V = 1000;
-    const auto hh = draw(static_cast<size_t>(T) * d, 61, 3.0), he = draw(static_cast<size_t>(V) * d, 62, 3.0);
+// and the row kernel, far from the ~0.01 logits of a freshly initialised model: the in-product path carries the row
+// maximum and the scaling in the exponent of exp2, which is where a large logit would show. Logits of a few tens in size
+// (common = 0), or all of them near common * 3: with every real logit far below zero, the zero columns that pad a
+// vocabulary to a multiple of 8 are far above the row's maximum and must not reach the exponential.
+void head_case(int V, float common, const char* name) {
+    std::printf("linear_cross_entropy, vocabulary %d, %s: inside the product vs fp32 logits + row kernel\n", V, name);
+    const int T = 300, d = 64;
+    auto hh = draw(static_cast<size_t>(T) * d, 61, common == 0.0f ? 3.0 : 0.3), he = draw(static_cast<size_t>(V) * d, 62, 3.0);
+    if (common != 0.0f) {
+        for (int i = 0; i < T; ++i) hh[static_cast<size_t>(i) * d] = common;
+        for (int i = 0; i < V; ++i) he[static_cast<size_t>(i) * d] = 3.0f;
+    }
     std::vector<int> target(T);
     for (int i = 0; i < T; ++i) target[i] = (37 * i + 11) % V;
     auto tg = device_ints(target);
@@ -338,7 +343,11 @@ void head_case() {
         }
         return w / std::fmax(size, 1e-30);
     };
-    check(std::isfinite(prod.loss) && prod.loss > 10.0f, "loss is finite and large (the logits are)", prod.loss);
+    bool finite = std::isfinite(prod.loss);
+    for (const std::vector<float>* g : {&prod.gh, &prod.ge})
+        for (float x : *g) finite = finite && std::isfinite(x);
+    check(finite, "loss and gradients are finite", prod.loss);
+    if (common == 0.0f) check(prod.loss > 10.0f, "the loss is large (the logits are)", prod.loss);
     check(std::fabs(prod.loss - rows.loss) <= 2e-5 * rows.loss, "loss", std::fabs(prod.loss - rows.loss));
     check(rel(prod.gh, rows.gh) <= 1.0 / 64, "dh", rel(prod.gh, rows.gh));
     check(rel(prod.ge, rows.ge) <= 1.0 / 64, "dE", rel(prod.ge, rows.ge));
@@ -455,7 +464,8 @@ int main() {
     linear_add_case(PK_F32, "float32 (product, then add)", 40, 24, 16, 1e-6);
     linear_add_case(PK_BF16, "bfloat16, edge tiles", 200, 72, 136, 1.0 / 128);
     linear_add_case(PK_BF16, "bfloat16, long contraction", 300, 1376, 64, 1.0 / 128);
-    head_case();
+    head_case(1000, 0.0f, "logits of size ~50");
+    for (int V : {18, 1002, 50258}) head_case(V, -50.0f, "logits near -150");  // one tile, 128 x 128 tiles, 256 x 256 tiles
     grouped_weight_gradient_case();
     behaviour_case();
     if (g_failures == 0) {
