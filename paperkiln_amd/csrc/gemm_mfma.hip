@@ -321,8 +321,10 @@ __device__ inline TileDesc tile_desc(const uint16_t* base, int64_t ld, int rc0, 
         left = ((rcs - 1) * ld + kspan) * 2;
         d.step = BK * 2;
     } else {  // [k][column]
+        // An odd number of columns (of A^T only) ends in the middle of a dword, which the range check drops whole: the last
+        // row's last element would read as zero. That dword lies inside the row's pitch, a multiple of 8.
         p = reinterpret_cast<const char*>(base + static_cast<int64_t>(k_begin) * ld + rc0);
-        left = ((kspan - 1) * ld + rcs) * 2;
+        left = ((kspan - 1) * ld + rcs + (rcs & 1)) * 2;
         d.step = static_cast<int>(BK * ld * 2);
     }
     const uint64_t a = reinterpret_cast<uint64_t>(p) - BIAS;

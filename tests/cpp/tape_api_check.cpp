@@ -316,6 +316,7 @@ void head_case(int V, float common, const char* name) {
     }
     std::vector<int> target(T);
     for (int i = 0; i < T; ++i) target[i] = (37 * i + 11) % V;
+    for (int i : {127, 255, 299}) target[i] = V - 1;  // the last word's share of each chunk's last row is one of dE's largest
     auto tg = device_ints(target);
     pk::set_compute_dtype(PK_BF16);
     struct Run {
@@ -465,6 +466,7 @@ int main() {
     linear_add_case(PK_BF16, "bfloat16, edge tiles", 200, 72, 136, 1.0 / 128);
     linear_add_case(PK_BF16, "bfloat16, long contraction", 300, 1376, 64, 1.0 / 128);
     head_case(1000, 0.0f, "logits of size ~50");
+    for (int V : {17, 1001}) head_case(V, 0.0f, "logits of size ~50");  // odd: dE contracts over rows that end inside a dword
     for (int V : {18, 1002, 50258}) head_case(V, -50.0f, "logits near -150");  // one tile, 128 x 128 tiles, 256 x 256 tiles
     grouped_weight_gradient_case();
     behaviour_case();
