@@ -76,11 +76,11 @@ int pk_attn_fwd(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k
  * D_i [B,Hq,T] fp32; for a band mask with 1..32 sink keys, room for the
  * partial dK/dV rows of the sink keys (the queries past the band of the first
  * key block may be handed to extra workgroups whose partial sums are added in
- * a fixed order); and, without a band, where query heads share KV heads
- * (Hq > Hkv) on a shape too small to fill the GPU, room for the fp32 partial
- * dK/dV of the workgroups that the heads of a group are dealt to (added in a
- * fixed order as well). Ask with the window and sinks the backward will run
- * with. */
+ * a fixed order); and, where query heads share KV heads (Hq > Hkv) on a
+ * shape that the kernels which deal a group's heads to several workgroups
+ * take, room for the fp32 partial dK/dV of those workgroups (added in a fixed
+ * order as well). Ask with the mask and element type the backward will run
+ * with; scale and grad_dtype make no difference. */
 size_t pk_attn_bwd_workspace_bytes(const pk_attn_shape* s);
 
 /* Backward closure of the same node (src/ops.cpp:902-933, 997-1026),

@@ -614,9 +614,8 @@ __global__ __launch_bounds__(256) void gqa_reduce(AttnArgs a) {
 template <int D, bool GF32>
 int launch(const AttnArgs& a, hipStream_t st) {
     const int nb128 = (a.T + 127) / 128;
-    const int hs = a.part ? a.head_split : 1;
+    const int hs = a.head_split;
     AttnArgs b = a;
-    b.head_split = hs;
     b.paired = pair_causal_blocks(nb128, static_cast<int64_t>(a.Hkv) * a.B * hs, a.causal, a.window, 256);
     hipLaunchKernelGGL((mfma_dkdv3<D, GF32>), causal_blocks_grid(b, nb128, hs), dim3(256), 0, st, b);
     PK_HIP(hipGetLastError());

@@ -680,6 +680,8 @@ int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st) {
     }
 }
 
+bool f32_deals_heads(const AttnArgs& a) { return a.head_split > 1 && f32_split_takes_dkdv(a); }
+
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
     int rc = PK_OK;

@@ -471,7 +471,6 @@ Form query_form(const AttnArgs& a, bool dq) {  // forward, dQ
 }
 Form fwd_form(const AttnArgs& a) { return query_form(a, false); }
 Form dq_form(const AttnArgs& a) { return query_form(a, true); }
-int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
 // The 128-key kernel walks the whole group of query heads in one workgroup: it is behind while those leave CUs idle,
 // however many blocks a split of keys and heads comes to (a group of four, head_dim 128, T 600, window 120: 8 KV heads
 // 252 us against 100, 24 KV heads 256 against 268; T 2400, window 100, 8 KV heads 258 against 356). Causal, every head its own
@@ -488,7 +487,7 @@ bool key_kernel_is_ahead(const AttnArgs& a, int64_t blocks) {
     return a.Hq == a.Hkv && ((a.dk_dim == 64 && blocks > 1400 && a.T < 3000) || (a.T <= 450 && blocks > 1000));
 }
 Form dkdv_form(const AttnArgs& a) {
-    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * a.head_split;
     if (key_kernel_is_ahead(a, blocks)) return Form::NONE;
     if (a.dk_dim > 64) return Form::FOUR;
     return a.dk_dim > 32 || (blocks <= 320 && chain_tokens(a) >= 512) ? Form::EIGHT : Form::FOUR;
@@ -547,7 +546,6 @@ int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 }
 int launch_f32_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
-    a.head_split = dkdv_splits(a);
     if (!split_tail_pays(a, a.head_split, 32)) a.tail = nullptr;
     const bool eight = dkdv_form(a) == Form::EIGHT;
     if (a.dk_dim <= 32)

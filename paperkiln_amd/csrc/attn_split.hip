@@ -606,11 +606,10 @@ Form dq_form(const AttnArgs& a) {
     if (blocks <= 600) return chain_tokens(a) >= 1536 ? best : a.dk_dim == 64 || chain_tokens(a) >= 768 ? Form::FOUR : Form::NONE;
     return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 1000 ? Form::FOUR : Form::NONE;
 }
-int dkdv_splits(const AttnArgs& a) { return a.part ? a.head_split : 1; }
 Form dkdv_form(const AttnArgs& a) {
-    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * dkdv_splits(a);
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * a.head_split;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
-    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 72) && dkdv_splits(a) == 1))
+    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 72) && a.head_split == 1))
         return Form::NONE;
     const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
     if (!plain) {  // T 2933 x 2, 4 heads, head_dim 96: a backward of 127 us against 157; T 1714 x 2, 8 heads, 32: 52 against 65
@@ -705,7 +704,6 @@ int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 }
 int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
-    a.head_split = dkdv_splits(a);
     if (!split_tail_pays(a, a.head_split, dkdv_form(a) == Form::WIDE ? 128 : 32)) a.tail = nullptr;
     const auto run = [&]() -> int {
 #define PK_CALL(D, E) dkdv_of<D, E>(a, dkdv_form(a), st)

@@ -106,9 +106,24 @@ int head_split_of(const pk_attn_shape* s) {
     const Mask m = effective_mask(s);
     return gqa_head_split(s->B, s->T, s->Hq, s->Hkv, s->dk, s->causal != 0, m.window);
 }
+// Whether the dK/dV launch goes to a kernel that splits so, asked of the dispatch itself. Only dimensions, mask and input
+// type of the shape count: the tensors are taken as aligned rows, a positive scale and fp32 gradients as given. Others take
+// the scalar kernels or one that walks a group in one workgroup, so the answer is an upper bound for them.
+bool deals_heads(const pk_attn_shape* s) {
+    AttnArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.B = s->B; a.T = s->T; a.Hq = s->Hq; a.Hkv = s->Hkv; a.dk_dim = s->dk;
+    const Mask m = effective_mask(s);
+    a.causal = s->causal != 0; a.window = m.window; a.sinks = m.sinks;
+    a.scale = 1.0f;
+    a.grad_f32 = 1;
+    a.q_st = a.k_st = a.v_st = a.o_st = a.do_st = a.dq_st = a.dk_st = a.dv_st = s->dk;
+    a.head_split = head_split_of(s);
+    return s->dtype == PK_BF16 ? split_serves(a) && bf16_deals_heads(a) : f32_mfma_supported(a) && f32_deals_heads(a);
+}
 size_t part_bytes(const pk_attn_shape* s) {
     const int hs = head_split_of(s);
-    if (hs <= 1) return 0;
+    if (hs <= 1 || !deals_heads(s)) return 0;
     const size_t before = delta_bytes(s) + tail_bytes(s);
     return (256 - before % 256) % 256 + gqa_part_bytes(s->B * s->Hkv, hs, s->T, s->dk);
 }
@@ -249,9 +264,12 @@ int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
         const size_t db = delta_bytes(s);
         a.tail = reinterpret_cast<float*>(static_cast<char*>(workspace) + db + (256 - db % 256) % 256);
     }
-    if (split_heads && part_bytes(s)) {
-        a.head_split = head_split_of(s);
-        a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + before_part + (256 - before_part % 256) % 256);
+    if (split_heads) {
+        a.head_split = head_split_of(s);  // also where no partial sums follow from it: the dispatch reads it
+        if (part_bytes(s))
+            a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + before_part + (256 - before_part % 256) % 256);
+        else if (s->dtype == PK_BF16 ? split_serves(a) && bf16_deals_heads(a) : f32_mfma_supported(a) && f32_deals_heads(a))
+            return fail(PK_ERR_WORKSPACE, "pk_attn_bwd: the dK/dV kernel of these tensors needs partial sums that its shape was not given");
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (s->dtype == PK_BF16 && split_serves(a)) return launch_mfma_bwd(a, stages, st);

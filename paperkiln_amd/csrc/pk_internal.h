@@ -38,9 +38,9 @@ struct AttnArgs {
     void* dv;
     float* delta;    // bwd scratch: rowsum(dO .* O)   [B,Hq,T]
     float* tail;     // bwd scratch: partial dK/dV rows of the sink keys (see sink_tail), or null
-    float* part;     // bwd scratch: per-split partial dK/dV of a GQA group (see gqa_head_split), or null
+    float* part;     // bwd scratch: per-split partial dK/dV of a GQA group (see gqa_head_split); null where no kernel splits
     int paired;      // full-causal launches of 128-row blocks and more: two blocks to a workgroup (see pair_causal_blocks)
-    int head_split;  // number of workgroups that share the query heads of one KV head in the dK/dV launch (1 = no split)
+    int head_split;  // number of workgroups that share the query heads of one KV head in a dK/dV launch that splits (1 = no split)
     int64_t q_sb, q_st, q_sh;
     int64_t k_sb, k_st, k_sh;
     int64_t v_sb, v_st, v_sh;
@@ -114,7 +114,8 @@ __host__ inline bool sink_tail_pays(const SinkTail& t, int T, int window, int kv
 // workgroups; split r takes heads [r rep / hs, (r + 1) rep / hs), writes its fp32 partial dK and dV to
 //   part[((unit * hs + r) * 2 + {0: dK, 1: dV}) * T + key][head_dim]
 // and a second kernel adds the splits in order (no atomics, repeatable). The kernels of attn_split.hip and
-// attn_f32_split.hip split that way, band or not, and mfma_dkdv3 (band-free bf16); the others walk a group in one workgroup.
+// attn_f32_split.hip split that way, band or not, and mfma_dkdv3 (band-free bf16); the others walk a group in one workgroup,
+// and a launch that goes to them needs no partial sums (bf16_deals_heads, f32_deals_heads).
 __host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window) {
     const int rep = Hq / Hkv;
     if (rep <= 1 || dk % 4 != 0 || dk > 128) return 1;
@@ -153,6 +154,7 @@ int launch_f32_split_dkdv(const AttnArgs& a, hipStream_t st);
 bool f32_mfma_supported(const AttnArgs& a);
 int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
+bool f32_deals_heads(const AttnArgs& a);  // its dK/dV kernel for this launch uses a.head_split and a.part
 
 // attn_split.hip: bf16 kernels whose wavefronts split the contraction. They serve every head size that is a multiple of
 // 8 up to 128; at 64 and 128 `split_takes_*` says whether a launch is small enough for them to be ahead of the kernels
@@ -171,6 +173,7 @@ int launch_split_dkdv(const AttnArgs& a, hipStream_t st);
 bool bf16_rows_aligned(const AttnArgs& a);
 int launch_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
+bool bf16_deals_heads(const AttnArgs& a);  // its dK/dV kernel for this launch uses a.head_split and a.part
 int launch_mfma_dkdv2(const AttnArgs& a, hipStream_t st);
 // attn_bwd_dkdv3.hip: dK / dV with 64 keys per wavefront and hand-fixed register classes (head_dim 64 or 128, no band)
 bool mfma_dkdv3_takes(const AttnArgs& a);

@@ -66,9 +66,11 @@ BWD_DELTA, BWD_DKDV, BWD_DQ, BWD_ALL = 1, 2, 4, 7
 
 def bwd_workspace_bytes(q, k, grad_dtype=None, window=0, sinks=0):
     """Bytes of scratch pk_attn_bwd needs for these shapes and this mask (pk_attn_bwd_workspace_bytes):
-    a band mask with sink keys needs more than the plain causal mask."""
-    sh = _shape(q, k, 1.0, True, window, sinks, grad_dtype or q.dtype)
-    return max(int(_lib.lib().pk_attn_bwd_workspace_bytes(C.byref(sh))), 16)
+    a band mask with sink keys needs more than the plain causal mask. Without a band, enough for either
+    value of ``causal``."""
+    masks = (True,) if window > 0 else (True, False)
+    shapes = [_shape(q, k, 1.0, causal, window, sinks, grad_dtype or q.dtype) for causal in masks]
+    return max([int(_lib.lib().pk_attn_bwd_workspace_bytes(C.byref(sh))) for sh in shapes] + [16])
 
 
 def attn_bwd(q, k, v, o, lse, d_o, scale, causal=True, window=0, sinks=0, grad_dtype=None, out=None,

@@ -43,8 +43,8 @@ def test_argument_errors_do_not_need_a_gpu():
 
 
 def test_backward_workspace_follows_the_mask():
-    """pk_attn_bwd_workspace_bytes: delta [B, Hq, T] fp32 for every mask; without a band, query heads that share KV
-    heads on a grid that would leave CUs idle add the per-split partial dK / dV; a band mask with 1..32 sink keys on a
+    """pk_attn_bwd_workspace_bytes: delta [B, Hq, T] fp32 for every mask; query heads that share KV heads add the
+    per-split partial dK / dV where the kernel of that launch deals them to several workgroups; a band mask with 1..32 sink keys on a
     sequence longer than key block 0's band adds the partial sink rows of a split sink tail
     ((chunks of 512 queries + 1) x {dK, dV} x 32 rows x head_dim fp32 per (batch, KV head), 256-byte aligned)."""
     L = _lib.lib()
@@ -68,6 +68,45 @@ def test_backward_workspace_follows_the_mask():
     assert ws(256, 4, t=q0) == 4 * B * Hq * q0   # the sequence ends with the band: no tail
     odd = 4 * B * Hq * 4001                      # delta not a multiple of 256 bytes: the tail starts aligned
     assert ws(256, 4, t=4001) == odd + (256 - odd % 256) % 256 + 4 * B * Hkv * (-(-(4001 - q0) // 512) + 1) * 2 * 32 * dk
+
+
+def test_partial_sums_are_asked_for_where_a_kernel_writes_them():
+    """Query heads that share KV heads: fp32 partial dK / dV are part of the workspace only where the dK/dV launch goes to
+    a kernel that deals a group's heads to several workgroups; scale and gradient type do not change the answer."""
+    L = _lib.lib()
+
+    def ws(B, T, Hq, Hkv, dk, dtype, causal=1, window=0, scale=0.5, grad=_lib.PK_F32):
+        sh = _lib.AttnShape(B, T, Hq, Hkv, dk, causal, window, 0, scale, dtype, grad)
+        return L.pk_attn_bwd_workspace_bytes(ctypes.byref(sh)) - 4 * B * Hq * T
+
+    f32, bf16 = _lib.PK_F32, _lib.PK_BF16
+    assert ws(4, 4096, 16, 4, 128, f32) == 0     # walked in one workgroup by the 128-key kernel (134 MB otherwise)
+    assert ws(31, 256, 16, 4, 64, bf16) == 0     # by the 32-key kernel (65 MB otherwise)
+    assert ws(1, 700, 14, 2, 256, bf16) == 0     # head sizes of the scalar kernels
+    parts = 4 * 2 * 2 * 4096 * 128 * 16
+    assert ws(4, 4096, 16, 4, 128, bf16) == parts  # 2 splits of 16 units: the 64-key kernel
+    for scale, grad in ((-1.0, f32), (0.0, bf16)):
+        assert ws(4, 4096, 16, 4, 128, bf16, scale=scale, grad=grad) == parts
+    assert ws(1, 256, 14, 2, 64, f32) > 0 and ws(1, 256, 14, 2, 80, bf16, window=64) > 0  # kernels that split the queries
+
+
+def test_workspace_of_the_torch_front_end_fits_both_masks():
+    """ops.bwd_workspace_bytes is not told whether the mask is causal: it has to be enough for either."""
+    import random
+
+    import torch
+
+    from paperkiln_amd import ops
+    L, rng = _lib.lib(), random.Random(5)
+    for _ in range(400):
+        dtype = rng.choice([torch.float32, torch.bfloat16])
+        B, Hkv, rep, dk = rng.randint(1, 40), rng.randint(1, 4), rng.randint(1, 8), rng.choice([32, 64, 80, 128])
+        T = int(2 ** rng.uniform(0, 13))
+        q, k = (torch.empty((B, T, h, dk), dtype=dtype, device="meta") for h in (Hkv * rep, Hkv))
+        code = _lib.PK_F32 if dtype == torch.float32 else _lib.PK_BF16
+        for causal in (0, 1):
+            sh = _lib.AttnShape(B, T, Hkv * rep, Hkv, dk, causal, 0, 0, 0.3, code, code)
+            assert ops.bwd_workspace_bytes(q, k) >= L.pk_attn_bwd_workspace_bytes(ctypes.byref(sh))
 
 
 def test_a_window_that_covers_the_sequence_is_no_band():

@@ -140,6 +140,23 @@ def test_fp32_split_kernels(case, dk):
     assert max(e) < 5e-6, e
 
 
+# Query heads that share KV heads where the launch is one of a kernel that walks the group in one workgroup: the workspace is
+# the row sums alone, and the entry point with the library's own scratch runs the same kernels.
+@pytest.mark.parametrize("case,dtype,dk", [((31, 256, 16, 4, True, 0, 0), torch.bfloat16, 64), ((67, 64, 8, 2, False, 0, 0), torch.bfloat16, 128),
+                                           ((4, 1100, 16, 4, True, 0, 0), torch.float32, 128)], ids=str)
+def test_query_groups_without_partial_sums(case, dtype, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    q, k, v, d_o = (torch.randn((B, T, h, dk), generator=torch.Generator(device="cuda").manual_seed(i), device="cuda").to(dtype)
+                    for i, h in enumerate((Hq, Hkv, Hkv, Hq)))
+    assert ops.bwd_workspace_bytes(q, k) == 4 * B * Hq * T
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal)
+    got = ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal)
+    assert all(torch.equal(a, b) for a, b in zip(got, ops.attn_bwd_static(q, k, v, o, lse, d_o, scale, causal)))
+    e = errors((o, lse) + got, exact_attention(q, k, v, d_o, scale, causal, window, sinks))
+    assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
+
+
 # The queries past the sink keys' band dealt to workgroups of their own: one chunk and a short last one, all 32 sink rows,
 # query heads dealt as well, blocks of 32 keys and (bf16, head_dim 48, many of them) of 128.
 @pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 48), (torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float32, 32),
