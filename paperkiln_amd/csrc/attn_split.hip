@@ -9,15 +9,22 @@
 //
 // The same kernels, with wavefronts that own different rows and share the tiles (QW = 4, KW = 1), are the path of every
 // head size that is a multiple of 8 up to 128 but not 64 or 128 (D is the size rounded up to 32; chunks past the real
-// size read as zero and are not stored). P and dS enter their products there as TWO bf16 operands, the rounded value
-// and the remainder (EXACT: 16 significant bits, against 8 in the kernels of head_dim 64 and 128), because these sizes
-// used to run in fp32 arithmetic throughout.
+// size read as zero and are not stored). Rows that are not aligned run in fp32 arithmetic there (attn_generic.hip), and these
+// are no less exact (EXACT; head_dim 64 and 128 round P and dS to one bf16 operand): P and dS enter their products as several
+// operands, the rounded value and the remainders.
+#include <type_traits>
+
 #include "attn_split.h"
 
 namespace pk {
 namespace {
 
 constexpr float LOG2E = 1.4426950408889634f;
+// How many operands P and dS are (EXACT). Gradients can be fp32: three, all 24 bits; with two their error against float64 was
+// 2.5e-6 of their norm at every size, three leave 2 to 9e-7, the scalar kernels 2e-7 to 1.5e-6 (eleven shapes of 97 to 4096
+// tokens, head_dim 24 to 120). O is bf16 always: with two its error is the scalar kernels' to four digits, with three too.
+// The third costs (us, B=2 T=4096 H=16, dQ and dK/dV): head_dim 32 110 -> 140, 148 -> 195; 96 219 -> 254, 326 -> 409.
+constexpr int FWD_PARTS = 2, BWD_PARTS = 3;
 // The maximum that P is formed against moves only when a row outgrows it by this many powers of two: some row of 32 finds a
 // new maximum in most tiles, and rescaling costs three instructions per accumulator element. P then reaches 2^6, which its
 // operands and the fp32 sums hold as they hold 1.
@@ -65,55 +72,65 @@ __device__ inline void load_row(const void* base, int64_t off, int64_t st, int r
     }
 }
 
-// Elements 8H .. 8H+7 of a C tile as a bf16 k-chunk and what its rounding left over
-template <int H>
-__device__ inline void split_operand(const f32x16& c, bf16x8& hi, bf16x8& lo) {
-    u32x4 h, l;
+// Elements 8H .. 8H+7 of a C tile as N bf16 k-chunks: the rounded values, then what the rounding before left over, rounded.
+// 8 significant bits each and signs of their own: three hold the 24 bits of the fp32 values.
+template <int H, int N>
+__device__ inline void split_operand(const f32x16& c, bf16x8 (&part)[N]) {
+    u32x4 p[N];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float x0 = c[8 * H + 2 * i], x1 = c[8 * H + 2 * i + 1];
-        h[i] = pack_bf16(x0, x1);
-        l[i] = pack_bf16(x0 - __uint_as_float(h[i] << 16), x1 - __uint_as_float(h[i] & 0xffff0000u));
+        float x0 = c[8 * H + 2 * i], x1 = c[8 * H + 2 * i + 1];
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            p[n][i] = pack_bf16(x0, x1);
+            x0 -= __uint_as_float(p[n][i] << 16), x1 -= __uint_as_float(p[n][i] & 0xffff0000u);
+        }
     }
-    hi = *reinterpret_cast<bf16x8*>(&h);
-    lo = *reinterpret_cast<bf16x8*>(&l);
+#pragma unroll
+    for (int n = 0; n < N; ++n) part[n] = *reinterpret_cast<bf16x8*>(&p[n]);
+}
+
+// P of a raw score and the row's LSE (nl: -LSE of the row when EXACT, else -LSE log2 e). EXACT: the difference is formed in one
+// rounding, of the difference; in units of log2 the scale, the LSE and the product would each be rounded at the size of the LSE.
+template <bool EXACT>
+__device__ inline float weight_of(float s, float scale, float cexp, float nl) {
+    return __builtin_amdgcn_exp2f(EXACT ? fmaf(s, scale, nl) * LOG2E : fmaf(s, cexp, nl));
 }
 
 // acc[db] += M^T c for the 32 rows of an LDS tile that start at row0, M the tile (columns 32 db ..), c a C tile whose rows
-// are the tile's rows
-template <int D, bool EXACT>
+// are the tile's rows, as PARTS operands
+template <int D, int PARTS>
 __device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, const f32x16& c, f32x16* acc, int lane) {
     constexpr int DB = D / 32;
-    bf16x8 h0, l0, h1, l1;
-    if (EXACT) {
-        split_operand<0>(c, h0, l0);
-        split_operand<1>(c, h1, l1);
-    } else {
-        h0 = c_to_operand<0>(c);
-        h1 = c_to_operand<1>(c);
-    }
-    // a product that waits for the one before it takes half as long again: the rounded operand into every block, then the
-    // remainder
-    bf16x8 m[DB];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const bf16x8 h = half ? h1 : h0, l = half ? l1 : l0;
+    const auto half = [&](auto hc) {
+        constexpr int H = decltype(hc)::value;
+        bf16x8 part[PARTS];
+        if constexpr (PARTS == 1)
+            part[0] = c_to_operand<H>(c);
+        else
+            split_operand<H>(c, part);
+        // a product that waits for the one before it takes half as long again: the rounded operand into every block, then
+        // the remainders
+        bf16x8 m[DB];
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            m[db] = lds_read_tr_operand(tile, pitch, row0 + 16 * half, db * 32, lane);
-            acc[db] = mfma32(m[db], h, acc[db]);
+            m[db] = lds_read_tr_operand(tile, pitch, row0 + 16 * H, db * 32, lane);
+            acc[db] = mfma32(m[db], part[0], acc[db]);
         }
-        if (EXACT)
 #pragma unroll
-            for (int db = 0; db < DB; ++db) acc[db] = mfma32(m[db], l, acc[db]);
-    }
+        for (int n = 1; n < PARTS; ++n)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) acc[db] = mfma32(m[db], part[n], acc[db]);
+    };
+    half(std::integral_constant<int, 0>{});
+    half(std::integral_constant<int, 1>{});
 }
 
 // The launch bounds of all three kernels ask for two wavefronts to a SIMD where the registers allow it. Left to itself the
 // compiler kept the accumulators of head sizes above 64 in accumulation registers beside 200 others, one wavefront to a SIMD,
 // whose products, exponentials and LDS reads then took turns; within 256 registers they need no copies either. Forward, B=2
 // T=4096 H=16 (with the alternating products and the lazy maximum below): head_dim 96 261 -> 179 us, 48 166 -> 137, 32 104 ->
-// 93; backward 594 -> 542, 416 -> 360, 313 -> 259.
+// 93; backward 594 -> 542, 416 -> 360, 313 -> 259 (with two operands each for P and dS; with three 653, 450, 334).
 
 // ---- forward: QW groups of 32 queries x KW groups of key tiles of 32 NB keys ----
 template <int D, int QW, int KW, int NB, bool EXACT>
@@ -234,7 +251,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
                     ps[r & 3] += s[nb][r];
                 }
                 l += (ps[0] + ps[1]) + (ps[2] + ps[3]);  // per-lane partial; the two halves meet below
-                accumulate_tr<D, EXACT>(Vs, VS, nb * 32, s[nb], acc, lane);
+                accumulate_tr<D, EXACT ? FWD_PARTS : 1>(Vs, VS, nb * 32, s[nb], acc, lane);
             }
         }
         if (i + 1 < iters) commit(i + 1);  // two buffers: last read one iteration ago, before the previous barrier
@@ -315,7 +332,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse
     load_row<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
     const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
     float nlse = 0.0f, dl = 0.0f;
-    if (qi < a.T) nlse = -a.lse[lrow] * LOG2E;
+    if (qi < a.T) nlse = EXACT ? -a.lse[lrow] : -a.lse[lrow] * LOG2E;
     if (fuse_delta) {
         bf16x8 oreg[KK];
         load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, qi, a.T, dk, g, oreg);
@@ -365,10 +382,10 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse
                 dp = mfma32(lds_read8(Vs + (nb * 32 + c32) * S + kk * 16 + g * 8), greg[kk], dp);
             }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) dp[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * (dp[r] - dl);
+            for (int r = 0; r < 16; ++r) dp[r] = weight_of<EXACT>(s[r], a.scale, cexp, nlse) * (dp[r] - dl);
             const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
             if (kind != MaskKind::NONE) mask_block(dp, kind, vis, k0 + g * 4, 0.0f);
-            accumulate_tr<D, EXACT>(Ks, S, nb * 32, dp, acc, lane);
+            accumulate_tr<D, EXACT ? BWD_PARTS : 1>(Ks, S, nb * 32, dp, acc, lane);
         }
         if (i + 1 < iters) commit(i + 1);
         tile_barrier<QW>();
@@ -448,7 +465,7 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
         uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
         mq.store(t, S, gt);
         mg.store(t + BMQ * S, S, gt);
-        if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = gt < BMQ ? -row_r * LOG2E : row_r;
+        if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = gt >= BMQ ? row_r : EXACT ? -row_r : -row_r * LOG2E;
     };
     fetch(0);
     bf16x8 kreg[KK], vreg[KK];
@@ -488,7 +505,7 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
             for (int qd = 0; qd < 4; ++qd) {
                 const f32x4 nl = *reinterpret_cast<const f32x4*>(rows + nb * 32 + qd * 8 + g * 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s[qd * 4 + e] = __builtin_amdgcn_exp2f(fmaf(s[qd * 4 + e], cexp, nl[e]));
+                for (int e = 0; e < 4; ++e) s[qd * 4 + e] = weight_of<EXACT>(s[qd * 4 + e], a.scale, cexp, nl[e]);
             }
             const bool full = qhi < a.T && kw0 + 31 < a.T && (!a.causal || kw0 + 31 <= qlo) &&
                               (a.window == 0 || kw0 + a.window > qhi || kw0 + 31 < a.sinks);
@@ -496,14 +513,14 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] = kvis(qlo + (r >> 2) * 8 + g * 4 + (r & 3)) ? s[r] : 0.0f;
             }
-            accumulate_tr<D, EXACT>(Gs, S, nb * 32, s, acc, lane);
+            accumulate_tr<D, EXACT ? BWD_PARTS : 1>(Gs, S, nb * 32, s, acc, lane);
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
                 const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (dp[qd * 4 + e] - dl[e]);
             }
-            accumulate_tr<D, EXACT>(Qs, S, nb * 32, dp, acc + DB, lane);
+            accumulate_tr<D, EXACT ? BWD_PARTS : 1>(Qs, S, nb * 32, dp, acc + DB, lane);
         }
         c_t += KW;
         while (c_t >= nqt) c_t -= nqt;
@@ -574,8 +591,8 @@ bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
     return chain < 256 || (even_chains(a) && !(a.dk_dim == 64 && chain >= 768 && blocks <= 600));
 }
 // Head sizes other than 64 and 128, FOUR | WIDE. Many short chains of equal length are ahead unsplit from two blocks a CU on
-// (head_dim 80, T 64 x 87, 8 heads, no mask: forward 10.8 | 7.0 us, backward 43 | 28; T 2089, window 20: 16 | 12, 46 | 36), long
-// causal ones stay split for longer, the more so the fewer columns (forward: head_dim 32, T 3201 x 3, 4 heads 30 | 67, T 5179 x
+// (head_dim 80, T 64 x 87, 8 heads, no mask: forward 10.8 | 7.0 us, dQ 27 | 18, dK/dV 47 | 21; T 2089 x 4, window 20: dQ 38 | 29,
+// dK/dV 71 | 33), long causal ones stay split for longer, the more so the fewer columns (forward: head_dim 32, T 3201 x 3, 4 heads 30 | 67, T 5179 x
 // 2, 8 heads 91 | 105; head_dim 96, T 1886 x 3, 8 heads 45 | 53, T 4618, 16 heads 148 | 128).
 bool wide_chains(const AttnArgs& a, int64_t blocks) { return a.dk_dim > 32 && even_chains(a) && chain_tokens(a) <= 160 && blocks > 550; }
 Form fwd_form(const AttnArgs& a) {
@@ -599,7 +616,7 @@ Form dq_form(const AttnArgs& a) {
     // above 96 columns eight wavefronts of this kernel do not fit the registers
     const Form best = a.dk_dim > 96 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
     if (blocks <= 256) return best;
-    if (!plain) {  // T 5395, 8 heads, head_dim 32: a backward of 156 us against 253; T 1169 x 2, 16 heads, 80: 93 against 104
+    if (!plain) {  // FOUR | WIDE: T 5395, 8 heads, head_dim 32: 75 us | 126; T 1169 x 2, 16 heads, 80: 41 | 46
         const bool far = a.causal && chain_tokens(a) >= (a.dk_dim <= 32 ? 1200 : 900);
         return blocks <= (!far || a.dk_dim > 96 ? 1100 : a.dk_dim <= 32 ? 2600 : 1250) && !wide_chains(a, blocks) ? Form::FOUR : Form::WIDE;
     }
@@ -612,9 +629,9 @@ Form dkdv_form(const AttnArgs& a) {
     if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 72) && a.head_split == 1))
         return Form::NONE;
     const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
-    if (!plain) {  // T 2933 x 2, 4 heads, head_dim 96: a backward of 127 us against 157; T 1714 x 2, 8 heads, 32: 52 against 65
+    if (!plain) {  // split | WIDE: T 2933 x 2, 4 heads, head_dim 96: 96 us | 135; T 1714 x 2, 8 heads, 32: 40 | 57
         const bool far = a.causal && chain_tokens(a) >= 1500 && a.dk_dim <= 96;
-        const bool wide = a.dk_dim > 64 && wide_chains(a, blocks);  // at 48, T 239 x 9, 8 KV heads, window 47, WIDE is behind: 31 | 27
+        const bool wide = a.dk_dim > 64 && wide_chains(a, blocks);  // at 48, T 239 x 9, 8 KV heads, window 47, WIDE is behind: 22 | 16
         return blocks <= (!far ? 700 : a.dk_dim <= 32 ? 1600 : 800) && !wide ? best : Form::WIDE;
     }
     if (blocks <= 600) return best;
@@ -637,8 +654,8 @@ void run_dkdv(const AttnArgs& a, hipStream_t st) {
     const int nkb = (a.T + 32 * QW - 1) / (32 * QW);
     const dim3 grid(xcd_grid(nkb + tail_blocks(a), a.head_split, a.Hkv * a.B));
     // Two wavefronts to a SIMD cost head sizes up to 96 a few spilled registers: not while there is a workgroup for each CU at
-    // most (us of a backward, head_dim 80: T 4263, 6 heads, 204 workgroups, one | two 223 | 268; T 1466 x 9, 4 KV heads, 432:
-    // 216 | 201; T 743 x 19, 4 KV heads, 456: 715 | 639).
+    // most (us, head_dim 80, one | two: T 4263, 6 heads, 204 workgroups 193 | 237; 16 heads on 4, T 1466 x 9, 432: 302 | 272,
+    // T 743 x 19, 456: 211 | 185). A few hundred workgroups with one head each are behind with two (4 heads, T 1466 x 9: 78 | 94).
     if (D == 96 && QW > 1 && static_cast<int64_t>(nkb) * a.head_split * a.Hkv * a.B > 256)
         hipLaunchKernelGGL((split_dkdv<D, QW, KW, NB, EXACT, 2>), grid, dim3(64 * QW * KW), 0, st, a);
     else

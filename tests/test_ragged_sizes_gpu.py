@@ -61,8 +61,9 @@ def test_bf16_training_with_any_vocabulary(vocab, d, ff, layers, tokens, seq):
         m.close()
 
 
-def exact_attention(q, k, v, d_o, scale, causal, window, sinks):
-    """O, LSE, dQ, dK, dV in float64 (src/ops.cpp:863-1027) of [B,T,H,dk] tensors, K / V heads shared by groups."""
+def exact_attention(q, k, v, d_o, scale, causal, window, sinks, given_o=None):
+    """O, LSE, dQ, dK, dV in float64 (src/ops.cpp:863-1027) of [B,T,H,dk] tensors, K / V heads shared by groups. given_o: the O
+    whose rowsum(dO .* O) the gradients are formed with, as a backward is given it; the exact O otherwise."""
     q, k, v, d_o = (x.double().permute(0, 2, 1, 3).contiguous() for x in (q, k, v, d_o))
     B, Hq, T, dk = q.shape
     rep = Hq // k.shape[1]
@@ -76,7 +77,8 @@ def exact_attention(q, k, v, d_o, scale, causal, window, sinks):
     p = torch.exp(s - lse[..., None])
     o = p @ vx
     dp = d_o @ vx.transpose(2, 3)
-    ds = scale * p * (dp - (d_o * o).sum(-1, keepdim=True))
+    o_sum = o if given_o is None else given_o.double().permute(0, 2, 1, 3)
+    ds = scale * p * (dp - (d_o * o_sum).sum(-1, keepdim=True))
     dq, dkx, dvx = ds @ kx, ds.transpose(2, 3) @ q, p.transpose(2, 3) @ d_o
     group = lambda x: x.reshape(B, Hq // rep, rep, T, dk).sum(2)  # noqa: E731
     back = lambda x: x.permute(0, 2, 1, 3)  # noqa: E731
@@ -114,8 +116,9 @@ def test_split_kernels_of_small_launches(case, dk):
 
 
 # Head sizes that are no 64 or 128: each multiple of 8 around the padded sizes 32, 64, 96, 128; launches small enough for
-# split tiles and large enough for four rows of wavefronts per tile. P keeps 16 bits there, so fp32 dV is held to 2e-5 where
-# the bf16 operand of head_dim 64 / 128 would leave 4e-3; dQ and dK carry the rounding of the bf16 O in rowsum(dO .* O).
+# split tiles and large enough for four rows of wavefronts per tile. P and dS keep all their bits there, so fp32 dV is held to
+# 2e-5 where the bf16 operand of head_dim 64 / 128 would leave 4e-3; dQ and dK carry the rounding of the bf16 O in
+# rowsum(dO .* O).
 @pytest.mark.parametrize("dk", [8, 24, 32, 40, 56, 72, 80, 96, 104, 120])
 @pytest.mark.parametrize("case", [(1, 200, 3, 1, True, 0, 0), (2, 77, 4, 2, False, 0, 0), (5, 97, 64, 64, True, 0, 0),
                                   (9, 130, 28, 28, True, 40, 3)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
@@ -123,6 +126,26 @@ def test_head_sizes_between_the_usual_ones(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.bfloat16, causal, window, sinks))
     assert e[0] < 5e-3 and e[1] < 1e-5 and max(e[2:4]) < 5e-3 and e[4] < 2e-5, e
+
+
+# ... and against the scalar kernels, which take the same values in rows that are not 16-byte aligned and form P and dS in
+# fp32: with the O that both are given in the exact rowsum too, what is left is fp32 rounding in one order of summation or
+# another, a few 1e-7 of the gradient's norm either way and 2.5e-6 where P or dS lose bits on the way into a product.
+@pytest.mark.parametrize("dk", [8, 24, 40, 80, 96, 120])
+@pytest.mark.parametrize("case", [(1, 200, 3, 1, True, 0, 0), (5, 97, 64, 64, True, 0, 0), (2, 1024, 4, 4, True, 0, 0),
+                                  (9, 130, 28, 28, True, 40, 3)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_gradients_as_exact_as_the_scalar_kernels(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    q, k, v, d_o = (torch.randn((B, T, h, dk), generator=gen, device="cuda").bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    want = exact_attention(q, k, v, d_o, scale, causal, window, sinks, o)[2:]
+    norms = []
+    for view in (lambda x: x, lambda x: torch.nn.functional.pad(x, (0, 1))[..., :dk]):
+        got = ops.attn_bwd(*(view(x) for x in (q, k, v, o)), lse, view(d_o), scale, causal, window, sinks, grad_dtype=torch.float32)
+        norms.append([float((g.double() - w).norm() / w.norm()) for g, w in zip(got, want)])
+    assert all(a < 1.25 * b + 1e-7 for a, b in zip(*norms)), norms
 
 
 # The same of fp32 tensors: head_dim 32 / 64 / 128 in launches small enough for the split kernels (four and eight
