@@ -1548,6 +1548,11 @@ int head_kernel() { return g_head_in_product.load(std::memory_order_relaxed); }
 bool gemm_f32_is_ahead(bool tA, int64_t M, int64_t N, int64_t K) {
     return M * N * K <= (int64_t{1} << 28) || (tA && K <= 2048);
 }
+// Which weight gradients [M, N] over K tokens it gets when a backward pass holds them back and launches up to eight together,
+// which fills the chip that one of them alone leaves half empty. Two blocks, forward and backward, ms, held | one by one by the
+// rule above | this line: width 128, 16384 tokens 1.74 | 1.98 | 1.74; 256, 8192 1.59 | 1.71 | 1.58; 512, 4096 2.01 | 2.10 | 2.00,
+// 6000 2.97 | 3.12 | 2.98, 8192 3.82 | 3.65 | 3.66, 16384 8.23 | 7.74 | 7.84; 1024, 2048 3.59 | 3.53 | 3.51, 8192 12.5 | 12.0 | 12.0.
+bool gemm_f32_held_is_ahead(int64_t M, int64_t N, int64_t K) { return M * N * K <= (int64_t{1} << 32); }
 
 void gemm(const Tensor& A, bool tA, const Tensor& B, bool tB, void* C, int c_dtype, int64_t M, int64_t N, int64_t ldc,
           float beta, int64_t lda) {

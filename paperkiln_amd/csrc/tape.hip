@@ -158,13 +158,14 @@ void flush_weight_gradients() {
 }
 
 // Whether dW += x^T dy[:, col0 : col0 + ncols] can wait in the queue: a backward pass is running and the product is one
-// the hand-written kernels take (operands of one type, fp32 parameter gradient; in bf16 aligned).
+// the hand-written kernels take (operands of one type, fp32 parameter gradient; in bf16 aligned; in fp32 up to the size at
+// which the library is ahead of them).
 bool weight_gradient_can_wait(const Tensor& x, const Tensor& dy, int64_t col0, int64_t ncols, const Var& W) {
     if (pending().depth == 0 || gemm_backend() != 1) return false;
     if (x.dtype != dy.dtype || !W->is_param || x.rows != dy.rows || W->data.rows != x.cols || W->data.cols != ncols) return false;
     if (x.dtype == PK_BF16) {
         if (x.cols % 8 || dy.cols % 8 || col0 % 8 || ncols % 8) return false;
-    } else if (x.numel() >= (int64_t{1} << 29) || dy.numel() >= (int64_t{1} << 29)) {
+    } else if (x.numel() >= (int64_t{1} << 29) || dy.numel() >= (int64_t{1} << 29) || !gemm_f32_held_is_ahead(x.cols, ncols, x.rows)) {
         return false;
     }
     return W->grad.empty() || W->grad.dtype == PK_F32;

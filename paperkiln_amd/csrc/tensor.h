@@ -131,6 +131,7 @@ struct F32Product {
 };
 bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st);
 bool gemm_f32_is_ahead(bool tA, int64_t M, int64_t N, int64_t K);  // of the library, for one product of this size
+bool gemm_f32_held_is_ahead(int64_t M, int64_t N, int64_t K);      // the same for a weight gradient among several
 int64_t gemm_head_spans(int64_t M, int64_t N);
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,

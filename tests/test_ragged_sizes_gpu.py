@@ -232,7 +232,8 @@ def test_small_bf16_products(M, N, K, tA, tB, c_dtype):
         assert err < 2e-6 * K ** 0.5 * 4, float(err)
 
 
-@pytest.mark.parametrize("vocab,d,ff,tokens,seq", [(101, 64, 176, 77, 11), (301, 96, 256, 700, 100), (130, 64, 176, 4100, 820)])
+@pytest.mark.parametrize("vocab,d,ff,tokens,seq", [(101, 64, 176, 77, 11), (301, 96, 256, 700, 100), (130, 64, 176, 4100, 820),
+                                                   (130, 512, 1376, 6200, 775)])  # of the last some are held back, some not
 def test_fp32_training_on_ragged_sizes(vocab, d, ff, tokens, seq):
     """A whole fp32 pass (weight gradients of a block in one launch, residual sums in the products, the embedding's
     gradient with and without the sort) against the same pass on the library's GEMM."""
