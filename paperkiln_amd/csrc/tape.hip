@@ -887,7 +887,9 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
     // every tile twice (row statistics and loss, then dlogits) instead of storing [rows, V] logits for a row kernel
     bool in_product = h->data.dtype == PK_BF16 && Ec.dtype == PK_BF16 && head_kernel() != 0 && gemm_backend() != 0 &&
                       (V % 8 == 0 || E->data.dtype == PK_F32) &&  // a bf16 parameter has no padded copy
-                      gemm_head_takes(h->data.ptr(), d, Ec.ptr(), d, std::min<int64_t>(N, chunk_rows > 0 ? chunk_rows : 4096), V, d);
+                      // both passes: the second runs over the padded vocabulary
+                      gemm_head_takes(h->data.ptr(), d, Ec.ptr(), d, std::min<int64_t>(N, chunk_rows > 0 ? chunk_rows : 4096),
+                                      round_up8(V), d);
     // default chunk: the same scratch either way (4096 rows of bf16 dlogits, or 2048 of fp32 logits: 262 MB at 32000 words)
     if (chunk_rows <= 0) chunk_rows = in_product ? 4096 : 2048;
     for (int64_t r0 = 0; r0 < N; r0 += chunk_rows) {

@@ -468,6 +468,7 @@ int main() {
     head_case(1000, 0.0f, "logits of size ~50");
     for (int V : {17, 1001}) head_case(V, 0.0f, "logits of size ~50");  // odd: dE contracts over rows that end inside a dword
     for (int V : {18, 1002, 50258}) head_case(V, -50.0f, "logits near -150");  // one tile, 128 x 128 tiles, 256 x 256 tiles
+    head_case((1 << 20) - 1, 0.0f, "logits of size ~50");  // past the in-product head's limit when padded: both take the row kernel
     grouped_weight_gradient_case();
     behaviour_case();
     if (g_failures == 0) {
