@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/python_numbers.h>
 
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -134,12 +135,19 @@ struct AttentionBackward : public Node {
 
     explicit AttentionBackward(torch::autograd::edge_list&& next) : Node(std::move(next)) {}
     std::string name() const override { return "AttentionBackward"; }
+    // Backward passes of two threads may share this node, and one that does not keep the graph releases it: under the node's
+    // lock, like every node that holds tensors.
     void release_variables() override {
+        const std::lock_guard<std::mutex> lock(mutex_);
         q.reset_data(), k.reset_data(), v.reset_data(), o.reset_data(), lse.reset_data();
     }
     variable_list apply(variable_list&& in) override {
         const auto self = getptr();
-        const Tensor tq = q.unpack(), tk = k.unpack(), tv = v.unpack(), to = o.unpack(self), tl = lse.unpack();
+        Tensor tq, tk, tv, to, tl;
+        {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            tq = q.unpack(), tk = k.unpack(), tv = v.unpack(), to = o.unpack(self), tl = lse.unpack();
+        }
         Tensor d_o = in[0].defined() ? in[0] : at::zeros_like(to);
         if (d_o.stride(-1) != 1) d_o = d_o.contiguous();
         Grads g = backward(tq, tk, tv, to, tl, d_o, mask, tq.scalar_type(), nullptr, PK_BWD_ALL);

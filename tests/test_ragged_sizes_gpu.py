@@ -261,6 +261,34 @@ def test_forward_mode_is_refused():
         ops.attention(fwd.make_dual(q, tangent), k, v, 0.125)
 
 
+def test_two_threads_differentiate_one_graph():
+    """Backward passes that share a node take its tensors under the node's lock; one of them releases them at the end."""
+    import threading
+
+    q, k, v, d_o = (torch.randn(2, 65, 4, 64, device="cuda", requires_grad=i < 3) for i in range(4))
+    o = ops.attention(q, k, v, 0.125)
+    want = torch.autograd.grad(o, (q, k, v), d_o, retain_graph=True)
+    got, errors = [], []
+
+    def work():
+        try:
+            for _ in range(20):
+                got.append(torch.autograd.grad(o, (q, k, v), d_o, retain_graph=True))
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors and len(got) == 80, errors
+    assert all(torch.equal(a, b) for g in got for a, b in zip(g, want))
+    torch.autograd.grad(o, (q, k, v), d_o)
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(o, (q, k, v), d_o)
+
+
 # Either side of the lines between chains that are split and those that are not, head sizes between the usual ones: many long
 # causal chains of few columns, many short ones of equal length.
 @pytest.mark.parametrize("case,dk", [((18, 511, 4, 4, True, 0, 0), 32), ((6, 1446, 4, 2, True, 0, 0), 96), ((36, 114, 4, 2, False, 0, 0), 112),
