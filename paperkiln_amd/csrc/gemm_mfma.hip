@@ -70,7 +70,9 @@ struct GemmArgs {
 // What the two passes of the tied head's cross-entropy do with a tile of logits instead of storing it (gemm_ring's
 // EPI parameter). Pass 1: per row and per 64-column span of a wavefront, the span's maximum and its sum of
 // exp(z - maximum), to stats[span][row], and the target column's logit to zt[row]. Pass 2: the same tile formed
-// again, turned into dlogits = (exp(z - row_max) row_inv - [column == target]) gscale and stored as bf16.
+// again, turned into dlogits = (exp(z - row_max) row_inv - [column == target]) gscale and stored as bf16. EPI 1 is the first
+// pass, EPI 2 the second, EPI 4 the second over a vocabulary padded to a multiple of 8: its test of the columns keeps 95 scalar
+// registers outside their file, which the whole of pass 2 would pay for (4096 rows x 32000 x 512: 165 -> 169 us).
 struct HeadArgs {
     const int* target;     // [M]
     float2* stats;         // pass 1: [spans][M]
@@ -78,7 +80,7 @@ struct HeadArgs {
     const float* row_max;  // pass 2: [M]
     const float* row_inv;  // pass 2: [M], 1 / sum_j exp(z_j - row_max)
     float gscale;          // pass 2
-    int vocab;             // pass 2: columns from here to N only pad the matrix; their dlogits are 0
+    int vocab;             // EPI 4: columns from here to N only pad the matrix; their dlogits are 0
 };
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -611,17 +613,20 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     };
     // lane (c32, gh) holds, of row (wm FM + i) 32 + c32 of the tile, columns (wn FN + j) 32 + 8 qd + 4 gh + e
+    auto drop_columns = [&](const Block& bl, int from) {  // columns from there on count for nothing
+        const int col0 = bl.n0 + wn * FN * 32 + gh * 4;
+        if (bl.n0 + BN <= from) return;  // wavefront-uniform
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (col0 + j * 32 + (r >> 2) * 8 + (r & 3) >= from) acc[i][j][r] = -INFINITY;
+    };
     auto head_stats = [&](const Block& bl) {  // EPI 1
-        const int span = (bl.n0 / BN) * G::WGN + wn, col0 = bl.n0 + wn * FN * 32 + gh * 4;
-        if (bl.n0 + BN > g.N) {  // wavefront-uniform: columns past the matrix count for nothing
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (col0 + j * 32 + (r >> 2) * 8 + (r & 3) >= g.N) acc[i][j][r] = -INFINITY;
-        }
+        const int span = (bl.n0 / BN) * G::WGN + wn;
+        drop_columns(bl, g.N);
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const int row = bl.m0 + (wm * FM + i) * 32 + c32;
@@ -649,7 +654,10 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             if (has) hd.zt[row] = zt;
         }
     };
-    auto head_dlogits = [&](const Block& bl) {  // EPI 2: the sums become dlogits where they lie
+    auto head_dlogits = [&](const Block& bl) {  // EPI 2, 4: the sums become dlogits where they lie
+        // The padding's logits are 0, not in the row's maximum: their exponentials would overflow where every real logit lies
+        // far below 0, and dh multiply the infinities with the zero rows that pad B.
+        if constexpr (EPI == 4) drop_columns(bl, hd.vocab);
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const int row = bl.m0 + (wm * FM + i) * 32 + c32;
@@ -662,16 +670,6 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             for (int j = 0; j < FN; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], LOG2E, -ref));
-            if (hd.vocab < g.N && bl.n0 + BN > hd.vocab) {
-                // wavefront-uniform. The padding's logits are 0, not in the row's maximum: their exponentials overflow where
-                // every real logit lies far below 0, and dh would multiply the infinities with the zero rows that pad B.
-                const int col0 = bl.n0 + wn * FN * 32 + gh * 4;
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (col0 + j * 32 + (r >> 2) * 8 + (r & 3) >= hd.vocab) acc[i][j][r] = 0.0f;
-            }
             if (__builtin_amdgcn_ballot_w64(has) != 0) {  // few wavefronts hold a target column of one of their rows
                 const int at = has ? (tt >> 5) * 16 + ((tt >> 3) & 3) * 4 + (tt & 3) : -1;
 #pragma unroll
@@ -838,7 +836,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                 if constexpr (EPI == 1) {
                     head_stats(cb);  // nothing goes through the slot, and no store joins the count of loads in flight
                 } else {
-                    if constexpr (EPI == 2) head_dlogits(cb);
+                    if constexpr (EPI == 2 || EPI == 4) head_dlogits(cb);
                     barrier();  // every wavefront has read slot u: it takes the result on its way out
                     store_result(lds + u * SLOT, cb);
                     since_store = 0;
@@ -1210,7 +1208,10 @@ bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, i
     hd.row_inv = row_inv;
     hd.gscale = gscale;
     hd.vocab = static_cast<int>(vocab);
-    head_small(M, N) ? launch_head<GeoSmall, 2>(g, hd, st) : launch_head<GeoLarge, 2>(g, hd, st);
+    if (vocab == N)
+        head_small(M, N) ? launch_head<GeoSmall, 2>(g, hd, st) : launch_head<GeoLarge, 2>(g, hd, st);
+    else
+        head_small(M, N) ? launch_head<GeoSmall, 4>(g, hd, st) : launch_head<GeoLarge, 4>(g, hd, st);
     return true;
 }
 
