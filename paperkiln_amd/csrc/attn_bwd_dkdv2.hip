@@ -396,17 +396,20 @@ __global__ __launch_bounds__(256) void sink_tail_reduce(AttnArgs a, int nch) {
     }
 }
 
+// The sink tail that a launch of this kernel deals out, if any (nch = 0: none). A tail step keeps two of the eight wavefronts
+// busy but takes as long as a full one (measured).
+SinkTail dealt_tail(const AttnArgs& a) {
+    const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
+    return sink_tail_pays(tl, a.T, a.window, a.Hkv * a.B, 64, 3, 1.0f) ? tl : SinkTail{0, 0};
+}
+
 template <int D, bool GF32, int BNK, int BMQ>
 int launch_geo(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
     const int nkb = (a.T + BNK - 1) / BNK;
     a.paired = pair_causal_blocks(nkb, static_cast<int64_t>(a.Hkv) * a.B, a.causal, a.window, 256);
-    SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
-    // a tail step keeps two of the eight wavefronts busy but takes as long as a full one (measured)
-    if (!sink_tail_pays(tl, a.T, a.window, a.Hkv * a.B, 64, 3, 1.0f)) {
-        a.tail = nullptr;
-        tl.nch = 0;
-    }
+    const SinkTail tl = dealt_tail(a);
+    if (tl.nch == 0) a.tail = nullptr;
     if (tl.nch > 0) {
         hipLaunchKernelGGL((mfma_dkdv2<D, GF32, true, BNK, BMQ>), dim3(xcd_grid(nkb + tl.nch, 1, a.Hkv * a.B)), dim3(4 * BNK), 0,
                            st, a);
@@ -420,24 +423,41 @@ int launch_geo(const AttnArgs& a_in, hipStream_t st) {
     return PK_OK;
 }
 
+// Short sequences and bands of a few key blocks: the small geometry, two workgroups per CU or (head_dim 64) four, which
+// hides the two memory round trips at the start of each and wastes less of the last tile. Measured, small | large
+// (us): B=4 H=16 T=4096, head_dim 128, window 128 190 | 229, 512 264 | 276, 1024 404 | 387; 16 heads, no band, T 48 x 170
+// at head_dim 64 29 | 57, at 128 59 | 82; T 128 x 64 28 | 36 and 52 | 67; T 400 x 20 41 | 49 and 76 | 81; T 900 x 3,
+// head_dim 64 32 | 26.
+// The large one is ahead in spite of that where its workgroups, one to a CU, come to one round of the chip, or nearly whole to
+// two, and the small one's do not save a part of them in the last tile: head_dim 64, causal, T 200 x 128 heads 15 | 11, 256 x
+// 128 16 | 12, 512 x 128 29 | 25, 96 x 256 13 | 10, 400 x 64 17 | 15, 320 x 96 15 | 13; no mask, 400 x 128 36 | 30, 512 x 128
+// 40 | 33, 320 x 160 28 | 23, 160 x 256 (a part saved) 20 | 25; one head more in eight and it is behind (512 x 160, causal
+// 33 | 34, 256 x 160 14 | 16). At head_dim 128 only where one round is whole: causal, 256 x 128 22 | 19, 96 x 256 17 | 15.
+// At head_dim 64 a wide band has to come with many of its workgroups (3571 tokens, window 315, 8 heads 20 | 16; 2000 x 4,
+// window 300, 16 heads 56 | 64; 2000 x 2, 16 heads, window 512 48 | 39), sink keys with a narrow one, whose tail then hides the
+// sinks' (16 heads of 500 tokens, window 100, 4 sinks: x 16 40 | 52, x 6 24 | 23; 2000 x 4, window 300, 16 sinks 74 | 71) or is
+// dealt out (64 heads of 2000, window 128, 4 sinks, left whole 76 | 60; window 32, dealt out 53 | 64).
+template <int D>
+bool small_geometry_is_ahead(const AttnArgs& a) {
+    const int64_t units = static_cast<int64_t>(a.Hkv) * a.B;
+    const int64_t small = (a.T + 63) / 64 * units, large = (a.T + 127) / 128 * units;  // workgroups of either
+    if (a.window == 0) {
+        if (a.T > 512 || (a.T > 256 && small < 256)) return false;
+        const bool saves = small * 5 < large * 8;
+        if (D == 128) return saves || large < 240 || large > 256;
+        if (large <= 256) return a.T <= 32;
+        if (large > 512) return true;
+        return a.causal ? !((a.T > 256 && large <= 300) || (a.T > 128 && large > 480 && small == 2 * large)) : saves || large < 450;
+    }
+    if (a.window > 512) return false;
+    if (D == 128) return true;
+    if (a.sinks > 0) return a.window <= 128 && small >= 1024 && (units > 96 || dealt_tail(a).nch > 0);
+    return a.window <= 64 || (a.window <= 128 ? large < 160 || large > 256 : small >= 1100);
+}
+
 template <int D, bool GF32>
 int launch(const AttnArgs& a, hipStream_t st) {
-    // Short sequences and bands of a few key blocks: the small geometry, two workgroups per CU or (head_dim 64) four, which
-    // hides the two memory round trips at the start of each and wastes less of the last tile. Measured, small | large
-    // (us): B=4 H=16 T=4096, head_dim 128, window 128 190 | 229, 512 264 | 276, 1024 404 | 387; 16 heads, no band, T 48 x 170
-    // at head_dim 64 29 | 57, at 128 59 | 82; T 128 x 64 28 | 36 and 52 | 67; T 400 x 20 41 | 49 and 76 | 81; T 900 x 3,
-    // head_dim 64 32 | 26.
-    // At head_dim 64 a wide band has to come with many of its workgroups (3571 tokens, window 315, 8 heads 20 | 16; 2000 x 4,
-    // window 300, 16 heads 56 | 64), sink keys with a narrow one, whose tail then hides the sinks' (16 heads of 500 tokens,
-    // window 100, 4 sinks: x 16 40 | 52, x 6 24 | 23; 2000 x 4, window 300, 16 sinks 74 | 71).
-    const int64_t small = static_cast<int64_t>((a.T + 63) / 64) * a.Hkv * a.B;  // its workgroups
-    const bool narrow = a.window <= 128, many = small >= 1024;
-    const bool ahead = a.window == 0    ? a.T <= 256 || (a.T <= 512 && small >= 256)
-                       : a.window > 512 ? false
-                       : D == 128       ? true
-                       : a.sinks > 0    ? narrow && many
-                                        : narrow || many;
-    if (ahead) return launch_geo<D, GF32, 64, 32>(a, st);
+    if (small_geometry_is_ahead<D>(a)) return launch_geo<D, GF32, 64, 32>(a, st);
     return launch_geo<D, GF32, 128, 64>(a, st);
 }
 

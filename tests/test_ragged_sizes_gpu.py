@@ -163,6 +163,18 @@ def test_fp32_split_kernels(case, dk):
     assert max(e) < 5e-6, e
 
 
+# Either side of the lines between the two geometries of the 32-key dK/dV kernel: one round of the chip and one head more, two
+# nearly whole rounds, and with a band and sink keys whose queries are dealt out or left whole.
+@pytest.mark.parametrize("case,dk", [((32, 200, 8, 8, True, 0, 0), 64), ((33, 200, 4, 4, True, 0, 0), 64), ((16, 200, 8, 8, True, 0, 0), 64),
+                                     ((17, 200, 8, 8, True, 0, 0), 64), ((16, 512, 8, 8, True, 0, 0), 64), ((20, 320, 8, 8, False, 0, 0), 64),
+                                     ((32, 160, 8, 8, False, 0, 0), 64), ((32, 96, 8, 8, True, 0, 0), 128), ((16, 256, 8, 8, True, 0, 0), 128),
+                                     ((8, 300, 8, 8, True, 100, 0), 64), ((10, 1000, 8, 8, True, 64, 4), 64), ((8, 1000, 8, 8, True, 32, 4), 64),
+                                     ((5, 1000, 8, 8, True, 300, 0), 64)], ids=str)
+def test_lines_between_the_dkdv_geometries(case, dk):
+    e = errors(*run_attention(*case[:4], dk, torch.bfloat16, *case[4:]))
+    assert max(e) < 1e-2, e
+
+
 # Query heads that share KV heads where the launch is one of a kernel that walks the group in one workgroup: the workspace is
 # the row sums alone, and the entry point with the library's own scratch runs the same kernels.
 @pytest.mark.parametrize("case,dtype,dk", [((31, 256, 16, 4, True, 0, 0), torch.bfloat16, 64), ((67, 64, 8, 2, False, 0, 0), torch.bfloat16, 128),
