@@ -432,7 +432,8 @@ int launch_geo(const AttnArgs& a_in, hipStream_t st) {
 // two, and the small one's do not save a part of them in the last tile: head_dim 64, causal, T 200 x 128 heads 15 | 11, 256 x
 // 128 16 | 12, 512 x 128 29 | 25, 96 x 256 13 | 10, 400 x 64 17 | 15, 320 x 96 15 | 13; no mask, 400 x 128 36 | 30, 512 x 128
 // 40 | 33, 320 x 160 28 | 23, 160 x 256 (a part saved) 20 | 25; one head more in eight and it is behind (512 x 160, causal
-// 33 | 34, 256 x 160 14 | 16). At head_dim 128 only where one round is whole: causal, 256 x 128 22 | 19, 96 x 256 17 | 15.
+// 33 | 34, 256 x 160 14 | 16). At head_dim 128 only where one round is whole (causal, 256 x 128 22 | 19, 96 x 256 17 | 15) or all
+// chains are as long (no mask, 400 x 48 25 | 22, 480 x 64 29 | 27).
 // At head_dim 64 a wide band has to come with many of its workgroups (3571 tokens, window 315, 8 heads 20 | 16; 2000 x 4,
 // window 300, 16 heads 56 | 64; 2000 x 2, 16 heads, window 512 48 | 39), sink keys with a narrow one, whose tail then hides the
 // sinks' (16 heads of 500 tokens, window 100, 4 sinks: x 16 40 | 52, x 6 24 | 23; 2000 x 4, window 300, 16 sinks 74 | 71) or is
@@ -444,13 +445,14 @@ bool small_geometry_is_ahead(const AttnArgs& a) {
     if (a.window == 0) {
         if (a.T > 512 || (a.T > 256 && small < 256)) return false;
         const bool saves = small * 5 < large * 8;
-        if (D == 128) return saves || large < 240 || large > 256;
+        if (D == 128) return large > 256 || (a.causal || a.T <= 300 ? saves || large < 240 : false);
         if (large <= 256) return a.T <= 32;
         if (large > 512) return true;
         return a.causal ? !((a.T > 256 && large <= 300) || (a.T > 128 && large > 480 && small == 2 * large)) : saves || large < 450;
     }
     if (a.window > 512) return false;
     if (D == 128) return true;
+    if (a.T <= 128 && a.Hq > a.Hkv) return false;  // a group's heads in turn, a step or two of 64 queries each: T 60, 14 on 2 17 | 20
     if (a.sinks > 0) return a.window <= 128 && small >= 1024 && (units > 96 || dealt_tail(a).nch > 0);
     return a.window <= 64 || (a.window <= 128 ? large < 160 || large > 256 : small >= 1100);
 }

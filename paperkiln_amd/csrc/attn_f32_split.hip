@@ -457,7 +457,8 @@ bool has_own_kernel(const AttnArgs& a) { return a.dk_dim == 32 || a.dk_dim == 64
 bool query_kernel_is_ahead(const AttnArgs& a, int64_t blocks, bool dq) {
     if (!has_own_kernel(a)) return false;
     const int chain = chain_tokens(a);
-    if (a.T <= 160 && blocks > (a.T <= 64 ? 256 : dq ? 512 : 600)) return true;
+    if (dq && a.T <= 32) return true;  // one tile, nothing to split: T 30, 16 heads of 128 12.9 us against 17.5, of 64 8.6 and 10.2
+    if (a.T <= 160 && blocks > (a.T <= (dq && a.dk_dim == 128 ? 96 : 64) ? 256 : dq ? 512 : 600)) return true;
     if (a.dk_dim == 128) return blocks > (a.T <= 96 ? 300 : even_chains(a) || chain < 400 ? 512 : 1200);
     if (a.T <= 200 && even_chains(a) && blocks > 512) return true;
     return !dq && blocks > 1500 && (a.T <= 200 || (even_chains(a) && chain > 128));
@@ -480,10 +481,17 @@ bool key_kernel_is_ahead(const AttnArgs& a, int64_t blocks) {
     if (!has_own_kernel(a)) return false;
     const int chain = chain_tokens(a);
     const int64_t groups = static_cast<int64_t>((a.T + 127) / 128) * a.Hkv * a.B;  // workgroups of the 128-key kernel
+    // One tile, nothing to split but the heads of a group: T 26, 8 heads of 128 x 7 14 us against 21, of 64 9.2 and 11.6; groups
+    // of two, 48 of 128 22 and 25; groups of four, 64 of 128 37 and 26, 68 37 and 42.
+    if (a.T <= 32 && (a.Hq <= 2 * a.Hkv || (a.Hq <= 4 * a.Hkv && a.dk_dim >= 64 && groups > 64))) return true;
     if (a.dk_dim == 128 && groups >= (a.T <= 64 ? 80 : 100) && chain < 400) return true;
-    if (a.T <= 160) return a.Hq == a.Hkv ? blocks > (a.T <= 64 ? 256 : 600) : groups >= 128;
+    if (a.T <= 160) return a.Hq == a.Hkv ? blocks > (a.T <= (a.dk_dim > 32 ? 96 : 64) ? 256 : 600) : groups >= 128;
     if (a.dk_dim == 128) return a.Hq == a.Hkv ? blocks > (even_chains(a) ? 512 : a.T < 800 ? 800 : 900) : groups >= 112;
     if (a.dk_dim == 64 && chain <= 160 && even_chains(a) && groups > 192 && groups <= 256) return true;  // one to a CU
+    // groups of heads in causal pairs of 128-key blocks that come to most of a round (T 200, 218 units of two heads 159 | 101, 167,
+    // 252 of four 240 | 151; 401, 128 of two 212 | 136; 500, 88 of four 340 | 292)
+    if (a.dk_dim == 64 && a.Hq > a.Hkv && a.causal && a.window == 0 && a.T <= 512 && (a.T + 127) / 128 % 2 == 0 && groups > 340 && groups <= 512)
+        return true;
     return a.Hq == a.Hkv && ((a.dk_dim == 64 && blocks > 1400 && a.T < 3000) || (a.T <= 450 && blocks > 1000));
 }
 Form dkdv_form(const AttnArgs& a) {

@@ -7,11 +7,15 @@
 // about half a microsecond. Here a block is 32 rows and four wavefronts split its tiles: four times the workgroups, a
 // quarter of the chain, and a sequence of 128 tokens is one tile per wavefront -- one round trip to memory.
 //
+// Which of these kernels a launch takes, or whether it takes one of the others, depends on its number of blocks (fwd_form,
+// dq_form, dkdv_form): the same call gives the same bits every time, but a unit in a batch need not give those it gives alone.
+//
 // The same kernels, with wavefronts that own different rows and share the tiles (QW = 4, KW = 1), are the path of every
 // head size that is a multiple of 8 up to 128 but not 64 or 128 (D is the size rounded up to 32; chunks past the real
 // size read as zero and are not stored). Rows that are not aligned run in fp32 arithmetic there (attn_generic.hip), and these
 // are no less exact (EXACT; head_dim 64 and 128 round P and dS to one bf16 operand): P and dS enter their products as several
 // operands, the rounded value and the remainders.
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_split.h"
@@ -580,8 +584,11 @@ enum class Form { NONE, WIDE, FOUR, EIGHT };
 //   head_dim 64, T 64, 16 units 5.3 6.6 6.7 | 4.3 5.4 5.7;     T 180, 32 units 6.5 8.5 8.8 | 6.7 9.3 9.5, 64 units 8.0 10.1 15.9 | 6.8 9.4 9.7
 //   T 600, window 128, 16 units 10.5 13.7 15.0 | 9.2 11.2 10.9;  T 929, no mask, 16 units 16.8 20.1 25.0 | 17.5 25.9 28.6
 //   head_dim 128, T 600, window 60, 16 units 12.2 17.8 18.2 | 11.0 13.6 10.5;  T 1100, no mask, 16 units 41 60 72 | 29 43 54
-// From 4096 tokens on head_dim 128 stays with the unsplit kernels whatever the number of units: a
-// unit alone, a unit in a batch and the prefix of a longer sequence are then the same bits, which callers rely on there.
+// From 4096 tokens on head_dim 128 stays with the unsplit kernels whatever the number of units. That is not for speed (causal,
+// forward, dQ, dK/dV, us, unsplit | split: 4096 x 1 head 86 118 94 | 32 67 67, 4 heads 88 120 96 | 42 98 80; 8192 x 1 167 223 179
+// | 54 206 126; window 256, 2 heads 17 20 26 | 10 14 31). A unit alone, a unit in a batch and the prefix of a longer sequence are
+// then the same bits (O, LSE and dQ; dK and dV too where every head is its own), which the tests of long sequences compare.
+// Everywhere else the sums' order, and so the last bits, depend on how many blocks a launch has.
 bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
     if (a.dk_dim != 64 && a.dk_dim != 128) return false;  // they take these head sizes only
     if (a.dk_dim == 128 && a.T >= 4096) return true;
@@ -599,20 +606,26 @@ Form fwd_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     if (unsplit_is_ahead(a, blocks) || (plain && a.T <= 64)) return Form::NONE;
-    if (blocks <= 256) return chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
+    // (six tiles on eight wavefronts, T 170, 38 heads of 128: four 8.8 us, eight 9.8, unsplit 9.0)
+    if (blocks <= 256) return chain_tokens(a) <= (plain ? 192 : 160) ? Form::FOUR : Form::EIGHT;
     if (!plain) {
         const int chain = chain_tokens(a);
         const int64_t longest = a.dk_dim <= 32 ? (chain >= (a.causal ? 400 : 2000) ? 2600 : 1100) : (a.causal && chain >= 900 ? 1450 : 1100);
         return blocks <= longest && !wide_chains(a, blocks) ? Form::FOUR : Form::WIDE;
     }
+    // past 512 blocks eight wavefronts a block, two workgroups to a CU, are a second round (no mask, T 1700, 10 heads of 64:
+    // eight 34 us, four 24, unsplit 28; causal, T 850, 19 heads of 128: 25, 17, 24)
     if (blocks <= 600)
-        return chain_tokens(a) >= (a.dk_dim == 64 ? 1536 : 768) ? Form::EIGHT : a.dk_dim == 64 && a.causal ? Form::FOUR : Form::NONE;
+        return chain_tokens(a) >= (a.dk_dim == 64 ? 1536 : 768) ? (blocks <= 512 ? Form::EIGHT : Form::FOUR)
+               : a.dk_dim == 64 && a.causal                    ? Form::FOUR
+                                                               : Form::NONE;
     return blocks <= 1100 && chain_tokens(a) >= 3000 ? Form::EIGHT : Form::NONE;
 }
 Form dq_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
-    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= 64)) return Form::NONE;
+    // (causal, T 80, 77 heads of 128: four wavefronts 10.8 us, unsplit 10.1; T 100 11.0 and 11.6)
+    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.causal ? 96 : 64))) return Form::NONE;
     // above 96 columns eight wavefronts of this kernel do not fit the registers
     const Form best = a.dk_dim > 96 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;
     if (blocks <= 256) return best;
@@ -623,19 +636,37 @@ Form dq_form(const AttnArgs& a) {
     if (blocks <= 600) return chain_tokens(a) >= 1536 ? best : a.dk_dim == 64 || chain_tokens(a) >= 768 ? Form::FOUR : Form::NONE;
     return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 1000 ? Form::FOUR : Form::NONE;
 }
+// Every head its own, head_dim 64 and 128: where the unsplit kernels are ahead of a block split between four wavefronts. At 128
+// one such workgroup fills a CU, so that short chains are behind even in one round (causal, four | unsplit, us: T 80, 77 heads
+// 11.3 | 10.0, T 170, 38 heads 13.6 | 12.5, T 250, 29 heads 14.6 | 15.4), and the blocks of a second round have to be few against
+// the chain (T 300, 38 heads 22 | 18; T 400, 21 heads 19 | 20.5, 34 heads 25 | 21; T 600, 17 heads 26 | 29, 26 heads 30 | 28; T
+// 1000, 16 heads 39 | 40; T 4000, 5 heads 106 | 92). At 64 two do: T 300, 50 heads 11.4 | 13.3, 60 heads 14.6 | 13.2.
+bool short_chains(const AttnArgs& a, int64_t blocks) {
+    const int chain = chain_tokens(a);
+    if (a.dk_dim == 64) return blocks > 512 && chain < 400;
+    if (blocks <= 256) return a.T <= (a.window > 0 ? 250 : 180);
+    return blocks > std::min(512, 256 + std::max(chain - 350, 0) * 2 / 5);
+}
 Form dkdv_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * a.head_split;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
-    if (unsplit_is_ahead(a, blocks) || (plain && a.T <= (a.dk_dim == 128 && a.window > 0 ? 128 : 72) && a.head_split == 1))
+    if (unsplit_is_ahead(a, blocks) || (plain && a.head_split == 1 && (a.T <= 72 || (a.Hq == a.Hkv && short_chains(a, blocks)))))
         return Form::NONE;
+    // a band over two tiles and groups of two: the sum over the dealt heads takes longer than they do (T 40, window 13, four
+    // heads on two: head_dim 64 10.0 us | 8.6, 128 13.2 | 9.8; groups of four 10.4 | 11.7, 13.7 | 14.2)
+    if (plain && a.window > 0 && a.T <= 64 && a.Hq <= 2 * a.Hkv) return Form::NONE;
     const Form best = a.dk_dim > 64 || chain_tokens(a) <= 160 ? Form::FOUR : Form::EIGHT;  // registers, as above
     if (!plain) {  // split | WIDE: T 2933 x 2, 4 heads, head_dim 96: 96 us | 135; T 1714 x 2, 8 heads, 32: 40 | 57
         const bool far = a.causal && chain_tokens(a) >= 1500 && a.dk_dim <= 96;
         const bool wide = a.dk_dim > 64 && wide_chains(a, blocks);  // at 48, T 239 x 9, 8 KV heads, window 47, WIDE is behind: 22 | 16
         return blocks <= (!far ? 700 : a.dk_dim <= 32 ? 1600 : 800) && !wide ? best : Form::WIDE;
     }
-    if (blocks <= 600) return best;
-    return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 2000 ? best : Form::NONE;
+    // at 64 eight wavefronts are ahead in one round only, or nearly so where the causal chains are long (us, eight | four | unsplit:
+    // T 350, 25 heads 16 | 10.4 | 13.9; T 600, 29 heads 25 | 15.5 | 19; T 2200, 13 heads 37 | 34 | 57, 14 heads 55 | 37 | 46;
+    // T 3000, 4 heads 31 | 37 | 63)
+    const Form later = a.dk_dim == 64 && blocks > 256 && !(blocks <= 450 && chain_tokens(a) >= 2000 && !even_chains(a)) ? Form::FOUR : best;
+    if (blocks <= 600) return later;
+    return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 2000 ? later : Form::NONE;
 }
 
 template <int D, int QW, int KW, int NB, bool EXACT>

@@ -175,6 +175,18 @@ def test_lines_between_the_dkdv_geometries(case, dk):
     assert max(e) < 1e-2, e
 
 
+# Either side of the lines between the split kernels and the others at the usual head sizes: the shortest sequences, one and
+# two rounds of blocks, and groups of heads.
+@pytest.mark.parametrize("case,dtype,dk", [(c, torch.bfloat16, d) for c in [(1, 90, 8, 8, True, 0, 0), (2, 177, 9, 9, True, 0, 0), (3, 322, 16, 16, True, 0, 0),
+                                           (2, 350, 13, 13, True, 0, 0), (1, 1700, 10, 10, False, 0, 0), (2, 40, 4, 2, True, 13, 0), (2, 60, 14, 2, True, 20, 2)]
+                                           for d in (64, 128)] +
+                                          [(c, torch.float32, d) for c in [(2, 26, 6, 6, True, 0, 0), (9, 30, 8, 2, False, 0, 0), (24, 32, 6, 3, True, 0, 0),
+                                           (30, 96, 4, 4, True, 0, 0)] for d in (32, 64, 128)] + [((50, 200, 8, 4, True, 0, 0), torch.float32, 64)], ids=str)
+def test_lines_between_split_and_unsplit_launches(case, dtype, dk):
+    e = errors(*run_attention(*case[:4], dk, dtype, *case[4:]))
+    assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
+
+
 # Query heads that share KV heads where the launch is one of a kernel that walks the group in one workgroup: the workspace is
 # the row sums alone, and the entry point with the library's own scratch runs the same kernels.
 @pytest.mark.parametrize("case,dtype,dk", [((31, 256, 16, 4, True, 0, 0), torch.bfloat16, 64), ((67, 64, 8, 2, False, 0, 0), torch.bfloat16, 128),
