@@ -167,8 +167,10 @@ typedef struct pk_llama_config {
 typedef struct pk_llama_stats {
     int64_t live_vars_after_forward;        /* the reference's receipt (tests/test_checkpointing.cpp:46-60) */
     int64_t activation_bytes_after_forward; /* allocator bytes held by the tape between forward and backward */
-    int64_t peak_activation_bytes;          /* high-water mark over forward + backward, parameters, gradients,
-                                               optimizer state and bf16 parameter shadows excluded */
+    int64_t peak_activation_bytes;          /* high-water mark over forward + backward; parameters, gradients,
+                                               optimizer state and the copies of parameters that the products
+                                               read (bf16 ones, and in either type the concatenated q|k|v and
+                                               gate|up weights) excluded */
 } pk_llama_stats;
 
 /* Llama::Llama(cfg, seed): N(0, 0.02) Linear / Embedding weights, unit norm gains.

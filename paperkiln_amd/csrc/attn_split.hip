@@ -587,7 +587,7 @@ enum class Form { NONE, WIDE, FOUR, EIGHT };
 // From 4096 tokens on head_dim 128 stays with the unsplit kernels whatever the number of units. That is not for speed (causal,
 // forward, dQ, dK/dV, us, unsplit | split: 4096 x 1 head 86 118 94 | 32 67 67, 4 heads 88 120 96 | 42 98 80; 8192 x 1 167 223 179
 // | 54 206 126; window 256, 2 heads 17 20 26 | 10 14 31). A unit alone, a unit in a batch and the prefix of a longer sequence are
-// then the same bits (O, LSE and dQ; dK and dV too where every head is its own), which the tests of long sequences compare.
+// then the same bits (O, LSE and dQ), which the tests of long sequences compare.
 // Everywhere else the sums' order, and so the last bits, depend on how many blocks a launch has.
 bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
     if (a.dk_dim != 64 && a.dk_dim != 128) return false;  // they take these head sizes only

@@ -1,7 +1,7 @@
-// The fp32 matrix product on the matrix cores (v_mfma_f32_32x32x2_f32): C = op(A) op(B) (+ C or an addend), row-major, up
+// The fp32 matrix product on the matrix cores (v_mfma_f32_16x16x4_f32): C = op(A) op(B) (+ C or an addend), row-major, up
 // to eight products in one launch.
 //
-// The fp32 matrix rate is a sixteenth of the bf16 one: a wavefront's 32 x 32 block needs 8 bytes a cycle, which L1 and L2
+// The fp32 matrix rate is a sixteenth of the bf16 one: a wavefront's 32 x 32 outputs need 8 bytes a cycle, which L1 and L2
 // deliver without LDS. Fragments are therefore loaded from global memory straight into the layout the instruction reads,
 // two chunks of the contraction ahead of the multiplications, and there is no barrier in the loop. What bounds a small
 // product is latency, and that a projection of a few hundred tokens has 16 to 200 blocks of 32 x 32 for 1024 SIMDs: the

@@ -206,7 +206,7 @@ HEAD_CASES = [
     ("bf16", 4104, 1500, 500, 256, True),        # vocab % 64 != 0: the last 64-column span of a row is partly masked
     ("bf16", 776, 700, 350, 300, True),          # vocab % 256 != 0 and whole spans past the last column
     ("fp32", 1001, 700, 350, 256, False),        # vocab % 4 != 0: the generic row kernel (+ cast in bf16)
-    ("bf16", 1001, 700, 350, 256, True),         # ... which the in-product setting falls back to (vocab % 8 != 0)
+    ("bf16", 1001, 700, 350, 256, True),         # vocab % 8 != 0: the in-product head over columns padded with zeros
     ("fp32", 50257, 600, 300, 256, False),       # vocab > 32768: a row no longer fits the one-pass kernel's registers
     ("bf16", 50257, 600, 300, 256, False),
 ]
