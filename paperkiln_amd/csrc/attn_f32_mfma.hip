@@ -4,7 +4,9 @@
 // 948-995) for fp32 tensors with head_dim 32, 64 or 128. Products and sums are
 // fp32 throughout, so the result stays inside the fp32 contract (max-abs 1e-5
 // against the CPU reference); the scalar kernels of attn_generic.hip remain the
-// path for every other head size and for unaligned rows.
+// path for every other head size and for unaligned rows. Launches with many blocks
+// go to attn_f32x3.hip, small ones to attn_f32_split.hip; what is left here are
+// short sequences of many units.
 //
 // v_mfma_f32_32x32x2_f32 operands (g = lane / 32, c = lane % 32):
 //   A (32 x 2): lane holds A[row c][k = g]          (one float)
@@ -643,11 +645,13 @@ int launch_dkdv(const AttnArgs& a_in, hipStream_t st) {
     return nch > 0 ? launch_sink_tail_reduce(a, st) : PK_OK;
 }
 int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    if (f32x3_takes_dq(a)) return launch_f32x3_dq(a, fuse_delta, st);
     if (f32_split_takes_dq(a)) return launch_f32_split_dq(a, fuse_delta, st);
     return a.dk_dim == 32 ? launch_dq<32>(a, fuse_delta, st) : a.dk_dim == 64 ? launch_dq<64>(a, fuse_delta, st)
                                                                               : launch_dq<128>(a, fuse_delta, st);
 }
 int run_dkdv(const AttnArgs& a, hipStream_t st) {
+    if (f32x3_takes_dkdv(a)) return launch_f32x3_dkdv(a, st);
     if (f32_split_takes_dkdv(a)) return launch_f32_split_dkdv(a, st);
     return a.dk_dim == 32 ? launch_dkdv<32>(a, st) : a.dk_dim == 64 ? launch_dkdv<64>(a, st) : launch_dkdv<128>(a, st);
 }
@@ -672,6 +676,7 @@ bool f32_mfma_supported(const AttnArgs& a) {
 }
 
 int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st) {
+    if (f32x3_takes_fwd(a)) return launch_f32x3_fwd(a, st);
     if (f32_split_takes_fwd(a)) return launch_f32_split_fwd(a, st);
     switch (a.dk_dim) {
         case 32: return launch_fwd<32>(a, st);

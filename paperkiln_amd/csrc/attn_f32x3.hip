@@ -1,0 +1,808 @@
+// fp32 attention (forward, dQ, dK/dV) on the bf16 matrix instruction: every fp32 operand as three bf16 parts.
+//
+// A value is split into the bf16 next to it, the bf16 next to what that leaves, and the rest, which is a bf16 exactly: 8
+// significant bits each with signs of their own hold the 24 of an fp32 value. A product of two such values is nine products
+// of parts, of which the three smallest are at most 2^-26 of the whole and are left out; the other six are exact in
+// fp32 and are added in fp32 by the matrix unit, small ones first. Error of a 32 x 32 product of normal values against
+// float64, of the result's norm: 64 columns 4.6e-8 (v_mfma_f32_32x32x2_f32, which rounds its sum every second
+// column: 1.44e-7), 128 columns 6.1e-8 (2.0e-7). Parts below 2^-126 are lost, so that precision fades for values below 1e-33.
+//
+// What bounds it: the fp32 instruction does 157 TFLOP/s, and the kernels on it (attn_f32_split.hip) stood at 105 to 130; six
+// bf16 products for one take 3/8 of its clocks. Beside them stands the splitting, 5.5 vector instructions an element: a tile
+// is split once, on its way into LDS, for all wavefronts of a workgroup, so a workgroup is QW x 32 rows that share tiles
+// (times KW groups that take every KW-th tile, for launches with few blocks).
+#include <type_traits>
+
+#include "attn_split.h"
+
+namespace pk {
+namespace {
+
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float LAZY_T = 6.0f;  // as in attn_split.hip: the running maximum moves when it is outgrown by 2^6
+
+// A product that is not fused into the sum it enters.
+__device__ inline float mul_rounded(float x, float y) {
+#pragma clang fp contract(off)
+    return x * y;
+}
+
+// Two fp32 values as three packed bf16 pairs. The first part is cut off, not rounded, so that every finite value has one; an
+// infinity leaves no rest, and what it meets becomes NaN.
+__device__ inline void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const uint32_t u0 = __float_as_uint(x0) & 0xffff0000u, u1 = __float_as_uint(x1) & 0xffff0000u;
+    h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // upper halves
+    x0 -= __uint_as_float(u0), x1 -= __uint_as_float(u1);
+    m = pack_bf16(x0, x1);
+    x0 -= __uint_as_float(m << 16), x1 -= __uint_as_float(m & 0xffff0000u);
+    l = pack_bf16(x0, x1);
+}
+
+// Columns and rows as in mfma_common.h (TrMap, lds_row), so that row reads and transposing reads of one plane are both free
+// of bank conflicts at 64 and 128 columns; at 32 and 96 both are in natural order.
+template <int D>
+__device__ constexpr int tr_src_col(int db, int u, int a) {
+    if constexpr (D == 128)
+        return TrMap<128>::src_col(db, u, a);
+    else
+        return 32 * db + 16 * u + 4 * a;
+}
+template <int D>
+__device__ constexpr int tr_col0(int db, int qd, int g) {
+    if constexpr (D == 128)
+        return TrMap<128>::col0(db, qd, g);
+    else
+        return 32 * db + 8 * qd + 4 * g;
+}
+// operand of the 16 rows from row0 on (a multiple of 16), the 32 columns of block db
+template <int D>
+__device__ inline bf16x8 tr_operand(const uint16_t* plane, int row0, int db, int lane) {
+    const int g = lane >> 5, u = (lane >> 4) & 1, j = lane & 15;
+    const uint16_t* p = plane + (row0 + lds_row<D>(4 * g + (j >> 2))) * (D + 8) + tr_src_col<D>(db, u, j & 3);
+    const s16x4 lo = lds_read_tr4(p), hi = lds_read_tr4(p + TR_HI_ROWS<D> * (D + 8));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    s16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return *reinterpret_cast<bf16x8*>(&v);
+}
+// store_block of attn_split.h in this column order, fp32
+template <int D>
+__device__ inline void store_block32(void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
+    float* row = static_cast<float*>(base) + row_off;
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+        const int col = tr_col0<D>(db, qd, g);
+        const f32x4 v = {acc[qd * 4] * sc, acc[qd * 4 + 1] * sc, acc[qd * 4 + 2] * sc, acc[qd * 4 + 3] * sc};
+        if (col < dk) *reinterpret_cast<f32x4*>(row + col) = v;
+    }
+}
+
+// A 32-row tile of a [T, dk] fp32 matrix, moved by G threads (rows past T and chunks past dk read as zero) into three
+// planes of 32 rows of pitch D + 8: 16-byte row reads then touch all banks once.
+template <int D, int G>
+struct Mover3 {
+    static constexpr int NCH = D / 4, CPT = 32 * NCH / G, P = D + 8, PLANE = 32 * P;
+    static_assert(CPT >= 1 && 32 * NCH % G == 0, "every thread moves the same number of chunks");
+    int off[CPT];
+    u32x4 r[CPT];
+    __device__ void init(int t, int64_t st, int dk) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int c = t + G * i, row = c / NCH, ch = c % NCH;
+            off[i] = ch * 4 < dk ? static_cast<int>(row * st + ch * 4) * 4 : static_cast<int>(OUTSIDE);
+        }
+    }
+    __device__ void load(const void* base, int64_t elem_off, int64_t st, int r0, int T, int dk) {
+        const int64_t left = ((static_cast<int64_t>(T) - r0 - 1) * st + dk) * 4;  // r0 < T
+        float* p = static_cast<float*>(const_cast<void*>(base)) + elem_off + static_cast<int64_t>(r0) * st;
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc(p, 0, left > 0x7fffffff ? 0x7fffffff : static_cast<int>(left), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) r[i] = tile_load16(rs, off[i]);
+    }
+    __device__ void store(uint16_t* tile, int t) const {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(&r[i]);
+            uint32_t h[2], m[2], l[2];
+            split2(x[0], x[1], h[0], m[0], l[0]);
+            split2(x[2], x[3], h[1], m[1], l[1]);
+            uint16_t* p = at(tile, t, i);
+            *reinterpret_cast<u32x2*>(p) = u32x2{h[0], h[1]};
+            *reinterpret_cast<u32x2*>(p + PLANE) = u32x2{m[0], m[1]};
+            *reinterpret_cast<u32x2*>(p + 2 * PLANE) = u32x2{l[0], l[1]};
+        }
+    }
+    __device__ static uint16_t* at(uint16_t* tile, int t, int i) {
+        const int c = t + G * i;
+        return tile + lds_row<D>(c / NCH) * P + (c % NCH) * 4;
+    }
+};
+
+// eight values as three operands
+__device__ inline void split8(const float (&x)[8], bf16x8& h, bf16x8& m, bf16x8& l) {
+    u32x4 p[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a, b, c;
+        split2(x[2 * i], x[2 * i + 1], a, b, c);
+        p[0][i] = a, p[1][i] = b, p[2][i] = c;
+    }
+    h = *reinterpret_cast<bf16x8*>(&p[0]);
+    m = *reinterpret_cast<bf16x8*>(&p[1]);
+    l = *reinterpret_cast<bf16x8*>(&p[2]);
+}
+
+// Row `row` of a head as three operands: chunk kk holds columns 16 kk + 8 g .. +7; zero past T and past dk. `dot`, when
+// given, gathers this lane's share of the row's product with a row of `other`.
+template <int D>
+__device__ inline void load_row3(const void* base, int64_t off, int64_t st, int row, int T, int dk, int g, bf16x8 (&out)[3][D / 16],
+                                 const float* other = nullptr, float* dot = nullptr) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+        float x[8];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int col = 16 * kk + 8 * g + 4 * half;
+            f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (row < T && col < dk) {
+                z = *reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + off + row * st + col);
+                if (dot) {
+                    const f32x4 y = *reinterpret_cast<const f32x4*>(other + col);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum = fmaf(y[e], z[e], sum);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[4 * half + e] = z[e];
+        }
+        split8(x, out[0][kk], out[1][kk], out[2][kk]);
+    }
+    if (dot) *dot = sum;
+}
+
+// (rows of the tile) . b over the columns: all small products first, then the large ones on top of their sum
+template <int D>
+__device__ inline f32x16 dot3(const uint16_t* tile, const bf16x8 (&b)[3][D / 16], int c32, int g) {
+    constexpr int P = D + 8, PLANE = 32 * P;
+    const uint16_t* row = tile + lds_row<D>(c32) * P + g * 8;
+    f32x16 t;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+        const bf16x8 h = lds_read8(row + kk * 16), m = lds_read8(row + PLANE + kk * 16), l = lds_read8(row + 2 * PLANE + kk * 16);
+        t = mfma32(l, b[0][kk], t);
+        t = mfma32(h, b[2][kk], t);
+        t = mfma32(m, b[1][kk], t);
+        t = mfma32(m, b[0][kk], t);
+        t = mfma32(h, b[1][kk], t);
+    }
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) t = mfma32(lds_read8(row + kk * 16), b[0][kk], t);
+    return t;
+}
+
+// acc[n] += tile^T c for blocks db0 + n of the columns, c a C tile whose rows are the tile's rows. The tile's product is formed by
+// itself, small products first, and added once: on the accumulator each of the twelve would be rounded at its size.
+template <int D, int NB = D / 32>
+__device__ inline void accumulate3(const uint16_t* tile, const f32x16& c, f32x16* acc, int lane, int db0 = 0) {
+    constexpr int PLANE = 32 * (D + 8);
+    bf16x8 ch[2], cm[2], cl[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const float x[8] = {c[8 * half], c[8 * half + 1], c[8 * half + 2], c[8 * half + 3],
+                            c[8 * half + 4], c[8 * half + 5], c[8 * half + 6], c[8 * half + 7]};
+        split8(x, ch[half], cm[half], cl[half]);
+    }
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+        const int db = min(db0 + n, D / 32 - 1);
+        f32x16 t;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[r] = 0.0f;
+        bf16x8 h[2];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            h[half] = tr_operand<D>(tile, 16 * half, db, lane);
+            const bf16x8 m = tr_operand<D>(tile + PLANE, 16 * half, db, lane), l = tr_operand<D>(tile + 2 * PLANE, 16 * half, db, lane);
+            t = mfma32(l, ch[half], t);
+            t = mfma32(h[half], cl[half], t);
+            t = mfma32(m, cm[half], t);
+            t = mfma32(m, ch[half], t);
+            t = mfma32(h[half], cm[half], t);
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half) t = mfma32(h[half], ch[half], t);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][r] += t[r];
+        if (D == 128) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// m scale + log(l 2^-off): the logarithm of a mantissa and whole powers of two, added in 64 bits (logf of all of l and two sums
+// in 32 bits, each rounded at the size of the result, had 4.2e-8 to 5.8e-8 of it as their error)
+__device__ inline float log_sum(float m, float scale, float off, float l) {
+    const double e = static_cast<double>(__builtin_amdgcn_frexp_expf(l)) - static_cast<double>(off);
+    return static_cast<float>(static_cast<double>(m) * static_cast<double>(scale) + e * 0.69314718055994531 +
+                              static_cast<double>(logf(__builtin_amdgcn_frexp_mantf(l))));
+}
+
+// Tile buffers: two and one barrier a tile where a workgroup is one group, one and two barriers where two groups share the LDS.
+template <int D, int QW, int KW>
+constexpr int BUFS = KW == 1 && (D < 128 || QW > 4) ? 2 : 1;
+
+// ---- forward: QW groups of 32 queries x KW groups of 32-key tiles ----
+template <int D, int QW, int KW>
+__global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
+    constexpr int BM = 32 * QW, DB = D / 32, G = 64 * QW, NBUF = BUFS<D, QW, KW>;
+    constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
+    constexpr int RED = KW > 1 ? QW * KW * (DB * 1024 + 128) * 2 : 0;  // in uint16
+    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, (a.T + BM - 1) / BM, b, h, hk, qblk)) return;
+    const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
+    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float cexp = a.scale * LOG2E;
+
+    Mover3<D, G> mk, mv;
+    mk.init(gt, a.k_st, dk);
+    mv.init(gt, a.v_st, dk);
+    const KeyTiles kt(a, q0, BM, 32);
+    const int iters = (kt.n + KW - 1) / KW;
+    auto fetch = [&](int i) {  // this group's i-th tile (past its last: nothing)
+        const int at = i * KW + kg;
+        if (at < kt.n) {
+            mk.load(a.k, kb, a.k_st, kt.tile(at) * 32, a.T, dk);
+            mv.load(a.v, vb, a.v_st, kt.tile(at) * 32, a.T, dk);
+        }
+    };
+    auto commit = [&](int i) {
+        uint16_t* t = lds + (i % NBUF * KW + kg) * TILE;
+        if (i * KW + kg < kt.n) mk.store(t, gt), mv.store(t + 3 * PLANE, gt);
+    };
+    fetch(0);
+    bf16x8 qreg[3][D / 16];
+    load_row3<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    f32x16 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+    double lsum = 0.0;  // a sequence of tiles is a long chain of additions
+    float m = -1e30f, mc = mul_rounded(m, cexp);  // the reference's running-max seed, src/ops.cpp:881; and m cexp as P is formed against it
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    commit(0);
+    __syncthreads();
+
+    for (int i = 0; i < iters; ++i) {
+        if (i + 1 < iters) fetch(i + 1);  // in flight during the math
+        const int at = i * KW + kg;
+        const uint16_t* Ks = lds + (i % NBUF * KW + kg) * TILE;
+        const int k0 = at < kt.n ? kt.tile(at) * 32 : a.T;
+        // wavefront-uniform: is anything of this 32 x 32 block visible?
+        if (k0 < a.T && qlo < a.T && !(a.causal && k0 > qhi) && !(a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks)) {
+            f32x16 s = dot3<D>(Ks, qreg, c32, g);
+            const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
+            if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, -INFINITY);
+            float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            mx = xhalf_max(mx);
+            if (__any((mx - m) * cexp > LAZY_T)) {  // wavefront-uniform, rare after the first tiles
+                const float mn = fmaxf(m, mx), mcn = mul_rounded(mn, cexp), alpha = __builtin_amdgcn_exp2f(mc - mcn);
+                lsum *= static_cast<double>(alpha);
+                m = mn, mc = mcn;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+            }
+            float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, -mc));
+                ps[r & 3] += s[r];
+            }
+            lsum += static_cast<double>((ps[0] + ps[1]) + (ps[2] + ps[3]));  // per-lane partial; the two halves meet below
+            accumulate3<D>(Ks + 3 * PLANE, s, acc, lane);
+        }
+        if (NBUF == 1) __syncthreads();
+        if (i + 1 < iters) commit(i + 1);  // two buffers: last read one iteration ago, before the previous barrier
+        __syncthreads();
+    }
+
+    float l = xhalf_sum(static_cast<float>(lsum));
+    float off = fmaf(m, cexp, -mc);  // what the rounding of mc left out
+    if (KW > 1) {
+        // the groups' running maxima and sums meet, then their accumulators scaled to the common maximum
+        float* red = reinterpret_cast<float*>(lds) + qg * KW * (DB * 1024 + 128);
+        float* ml = red + KW * DB * 1024;
+        ml[kg * 128 + lane] = m;
+        ml[kg * 128 + 64 + lane] = l;
+        __syncthreads();
+        float mt = m, lt = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const float mk = ml[k * 128 + lane];
+            lt += ml[k * 128 + 64 + lane] * __builtin_amdgcn_exp2f(fmaf(mk - mt, cexp, -fmaf(mk, cexp, -mul_rounded(mk, cexp))));
+        }
+        const float alpha = __builtin_amdgcn_exp2f(fmaf(m - mt, cexp, -off));
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        join_groups<DB, KW>(acc, red, kg, lane);
+        m = mt, l = lt, off = 0.0f;
+    }
+    if (qi < a.T) {
+        const float inv = 1.0f / l;
+        const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if (KW == 1 || db % KW == kg) store_block32<D>(a.o, ro, db, g, acc[db], inv, dk);
+        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = log_sum(m, a.scale, off, l);
+    }
+}
+
+// ---- dQ (and delta, when asked for with it): the same blocks ----
+template <int D, int QW, int KW>
+__global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs a, int fuse_delta) {
+    constexpr int BM = 32 * QW, DB = D / 32, G = 64 * QW, NBUF = BUFS<D, QW, KW>;
+    constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
+    constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;  // in uint16
+    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, (a.T + BM - 1) / BM, b, h, hk, qblk)) return;
+    const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
+    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float cexp = a.scale * LOG2E;
+
+    Mover3<D, G> mk, mv;
+    mk.init(gt, a.k_st, dk);
+    mv.init(gt, a.v_st, dk);
+    const KeyTiles kt(a, q0, BM, 32);
+    const int iters = (kt.n + KW - 1) / KW;
+    auto fetch = [&](int i) {
+        const int at = i * KW + kg;
+        if (at < kt.n) {
+            mk.load(a.k, kb, a.k_st, kt.tile(at) * 32, a.T, dk);
+            mv.load(a.v, vb, a.v_st, kt.tile(at) * 32, a.T, dk);
+        }
+    };
+    auto commit = [&](int i) {
+        uint16_t* t = lds + (i % NBUF * KW + kg) * TILE;
+        if (i * KW + kg < kt.n) mk.store(t, gt), mv.store(t + 3 * PLANE, gt);
+    };
+    fetch(0);
+    bf16x8 qreg[3][D / 16], greg[3][D / 16];
+    load_row3<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
+    float nlse = 0.0f, dl = 0.0f;
+    if (qi < a.T) nlse = -a.lse[lrow] * LOG2E;
+    if (fuse_delta) {
+        float part;
+        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg,
+                     static_cast<const float*>(a.o) + b * a.o_sb + h * a.o_sh + qi * a.o_st, &part);
+        dl = xhalf_sum(part);
+        if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
+    } else {
+        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
+        if (qi < a.T) dl = a.delta[lrow];
+    }
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    f32x16 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+    commit(0);
+    __syncthreads();
+
+    for (int i = 0; i < iters; ++i) {
+        if (i + 1 < iters) fetch(i + 1);
+        const int at = i * KW + kg;
+        const uint16_t* Ks = lds + (i % NBUF * KW + kg) * TILE;
+        const int k0 = at < kt.n ? kt.tile(at) * 32 : a.T;
+        if (k0 < a.T && qlo < a.T && !(a.causal && k0 > qhi) && !(a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks)) {
+            f32x16 s = dot3<D>(Ks, qreg, c32, g);
+            const f32x16 dp = dot3<D>(Ks + 3 * PLANE, greg, c32, g);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * (dp[r] - dl);
+            const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
+            if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, 0.0f);
+            accumulate3<D>(Ks, s, acc, lane);
+        }
+        if (NBUF == 1) __syncthreads();
+        if (i + 1 < iters) commit(i + 1);
+        __syncthreads();
+    }
+    join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane);
+    if (qi < a.T) {
+        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, g, acc[db], a.scale, dk);
+    }
+}
+
+// The two products of a step that need no other go to two sets of wavefronts, as in the other dK/dV kernels: with both
+// sides' resident rows and both accumulators one wavefront needs 320 registers at 128 columns before it has begun. A C
+// tile crosses LDS in fp32, lane by lane as it lies in registers.
+__device__ inline void put_tile(float* buf, const f32x16& t, int lane) {
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd)
+        *reinterpret_cast<f32x4*>(buf + qd * 256 + lane * 4) = f32x4{t[qd * 4], t[qd * 4 + 1], t[qd * 4 + 2], t[qd * 4 + 3]};
+}
+__device__ inline f32x16 get_tile(const float* buf, int lane) {
+    f32x16 t;
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(buf + qd * 256 + lane * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[qd * 4 + e] = v[e];
+    }
+    return t;
+}
+
+// ---- dK, dV: QW groups of 32 keys, the query tiles of every query head of the group in turn ----
+// A step is two phases. First: role 0 S = Q K^T and P, role 1 dP = dO V^T, each half of the next tile's way into LDS. Then, P handed
+// over: role 0 dV^T += dO^T P, role 1 dS = P (dP - delta) and dK^T += Q^T dS.
+template <int D, int QW>
+__global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
+    constexpr int BNK = 32 * QW, DB = D / 32, G = 64 * QW;
+    constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE + 128;  // LSE and delta of a tile's rows behind it
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * TILE];
+    __shared__ __attribute__((aligned(16))) float pbuf[QW * 1024];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int role = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) & (G - 1);
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
+    const int nkb = (a.T + BNK - 1) / BNK;
+    const int hs = a.head_split;  // > 1: this workgroup takes heads [h0, h0 + nh) of the group, see gqa_head_split
+    // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
+    const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
+    const int nblk = nkb + tl.nch;
+    int blk, rr, kvu;
+    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
+    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu))
+        return;
+    const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
+    if (chunk >= 0 && rr > 0) return;
+    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
+    const int k0 = chunk >= 0 ? 0 : blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
+    const float cexp = a.scale * LOG2E;
+
+    // query tiles that can see keys [k0, k0 + BNK) (paperkiln src/ops.cpp:960-965 inverted)
+    const int khi = min(k0 + BNK, a.T) - 1;
+    const int qt_lo = chunk >= 0 ? (tl.q0 + chunk * TAIL_CHUNK) / 32 : a.causal ? k0 / 32 : 0;
+    const int q_end = chunk >= 0 ? min(a.T, tl.q0 + (chunk + 1) * TAIL_CHUNK) - 1
+                      : tl.nch > 0 && k0 == 0 ? tl.q0 - 1
+                      : a.window > 0 && k0 >= a.sinks ? min(a.T - 1, khi + a.window - 1) : a.T - 1;
+    const int qt_hi = q_end / 32;
+    const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh;
+
+    // role 0 moves Q and the rows' LSE, role 1 dO and their delta
+    const void* const src = role == 0 ? a.q : a.d_o;
+    const int64_t s_sb = role == 0 ? a.q_sb : a.do_sb, s_sh = role == 0 ? a.q_sh : a.do_sh, s_st = role == 0 ? a.q_st : a.do_st;
+    const float* const src_rows = role == 0 ? a.lse : a.delta;
+    const float row_sc = role == 0 ? -LOG2E : 1.0f;
+    Mover3<D, G> mv;
+    mv.init(gt, s_st, dk);
+    float row_r = 0.0f;
+    int f_h = 0, f_t = 0;  // the (head, tile) of the next fetch
+    auto fetch = [&]() {
+        const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * 32;
+        mv.load(src, b * s_sb + h * s_sh, s_st, r0, a.T, dk);
+        if (gt < 32) row_r = src_rows[(static_cast<int64_t>(b) * a.Hq + h) * a.T + min(r0 + gt, a.T - 1)];  // rows past the end are masked
+        if (++f_t == nqt) f_t = 0, ++f_h;
+    };
+    auto commit = [&](int i) {
+        uint16_t* t = lds + (i & 1) * TILE;
+        mv.store(t + role * 3 * PLANE, gt);
+        if (gt < 32) reinterpret_cast<float*>(t + 6 * PLANE)[role * 32 + gt] = row_r * row_sc;
+    };
+    fetch();
+    bf16x8 res[3][D / 16];  // K rows for role 0, V rows for role 1
+    load_row3<D>(role == 0 ? a.k : a.v, role == 0 ? b * a.k_sb + hk * a.k_sh : b * a.v_sb + hk * a.v_sh, role == 0 ? a.k_st : a.v_st,
+                 kj, a.T, dk, g, res);
+    f32x16 acc[DB];  // dV^T, dK^T
+#pragma unroll
+    for (int n = 0; n < DB; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.0f;
+    const KeyVis kvis(kj, a.T, a.causal, a.window, a.sinks);
+    commit(0);
+    if (steps > 1) fetch();
+    __syncthreads();
+
+    float* const pb = pbuf + qg * 1024;
+    // one loop for each role: with the role tested inside, every step moves the accumulators at the join
+    const auto loop = [&](auto role_c) {
+        constexpr int ROLE = decltype(role_c)::value;
+        int c_t = 0;
+        for (int i = 0; i < steps; ++i) {
+            const uint16_t* Qs = lds + (i & 1) * TILE;
+            const uint16_t* Gs = Qs + 3 * PLANE;
+            const float* rows = reinterpret_cast<const float*>(Qs + 6 * PLANE);
+            const int qlo = (qt_lo + c_t) * 32, qhi = qlo + 31;
+            if (++c_t == nqt) c_t = 0;
+            // wavefront-uniform, the same for both roles: is anything of this 32 x 32 block visible?
+            const bool live = qlo < a.T && kw0 < a.T && !(a.causal && kw0 > qhi) && !(a.window > 0 && kw0 + 31 + a.window <= qlo && kw0 >= a.sinks);
+            f32x16 t;
+            if (live) t = dot3<D>(ROLE == 0 ? Qs : Gs, res, c32, g);
+            if (ROLE == 0 && live) {
+                // lane = key kj; element r = query qlo + (r/4)*8 + 4g + r%4
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) {
+                    const f32x4 nl = *reinterpret_cast<const f32x4*>(rows + qd * 8 + g * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[qd * 4 + e] = __builtin_amdgcn_exp2f(fmaf(t[qd * 4 + e], cexp, nl[e]));
+                }
+                const bool full = qhi < a.T && kw0 + 31 < a.T && (!a.causal || kw0 + 31 <= qlo) &&
+                                  (a.window == 0 || kw0 + a.window > qhi || kw0 + 31 < a.sinks);
+                if (!full) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) t[r] = kvis(qlo + (r >> 2) * 8 + g * 4 + (r & 3)) ? t[r] : 0.0f;
+                }
+                put_tile(pb, t, lane);
+            }
+            if (i + 1 < steps) {  // the other buffer was last read one step ago, before the previous barrier
+                commit(i + 1);
+                if (i + 2 < steps) fetch();
+            }
+            __syncthreads();
+            if (ROLE == 1 && live) {
+                const f32x16 p = get_tile(pb, lane);
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) {
+                    const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + 32 + qd * 8 + g * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[qd * 4 + e] = p[qd * 4 + e] * (t[qd * 4 + e] - dl[e]);
+                }
+            }
+            if (live) accumulate3<D>(ROLE == 0 ? Gs : Qs, t, acc, lane);
+            __syncthreads();
+        }
+    };
+    if (role == 0)
+        loop(std::integral_constant<int, 0>{});
+    else
+        loop(std::integral_constant<int, 1>{});
+    // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
+    // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
+    const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1);
+    if (kj < a.T && (chunk < 0 || to_tail)) {
+        const bool parts = hs > 1 && !to_tail;
+        const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
+                                   : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+        const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
+        const bool scratch = parts || to_tail;
+        void* const room = to_tail ? a.tail : a.part;
+        const int64_t row = scratch ? (role == 0 ? pv : pk) : role == 0 ? b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st
+                                                                       : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+        void* const dst = scratch ? room : role == 0 ? a.dv : a.dk;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) store_block32<D>(dst, row, db, g, acc[db], role == 0 ? 1.0f : a.scale, dk);
+    }
+}
+
+// ---- dQ above 64 columns: the same two phases ----
+// First: role 0 S = K Q^T and P, role 1 dP - delta, each half of the next tile's way into LDS; both tiles are handed over, and each role
+// forms dS for itself and takes half the columns of dQ^T += K^T dS.
+template <int D>
+__global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta) {
+    constexpr int QW = 4, BM = 32 * QW, DB = D / 32, G = 64 * QW, HB = (DB + 1) / 2;
+    constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * TILE];
+    __shared__ __attribute__((aligned(16))) float cbuf[2][QW * 1024];
+
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int role = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) & (G - 1);
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
+    int b, h, hk, qblk;
+    if (!map_query_block(a, (a.T + BM - 1) / BM, b, h, hk, qblk)) return;
+    const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
+    const float cexp = a.scale * LOG2E;
+
+    // role 0 moves K, role 1 V
+    const void* const src = role == 0 ? a.k : a.v;
+    const int64_t s_off = role == 0 ? b * a.k_sb + hk * a.k_sh : b * a.v_sb + hk * a.v_sh, s_st = role == 0 ? a.k_st : a.v_st;
+    Mover3<D, G> mv;
+    mv.init(gt, s_st, dk);
+    const KeyTiles kt(a, q0, BM, 32);
+    auto fetch = [&](int i) { mv.load(src, s_off, s_st, kt.tile(i) * 32, a.T, dk); };
+    auto commit = [&](int i) { mv.store(lds + (i & 1) * TILE + role * 3 * PLANE, gt); };
+    fetch(0);
+    bf16x8 res[3][D / 16];  // Q rows for role 0, dO rows for role 1
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
+    float row_r = 0.0f;  // -LSE log2(e) for role 0, delta for role 1
+    if (role == 0) {
+        load_row3<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, res);
+        if (qi < a.T) row_r = -a.lse[lrow] * LOG2E;
+    } else if (fuse_delta) {
+        float part;
+        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, res,
+                     static_cast<const float*>(a.o) + b * a.o_sb + h * a.o_sh + qi * a.o_st, &part);
+        row_r = xhalf_sum(part);
+        if (qi < a.T && g == 0) a.delta[lrow] = row_r;
+    } else {
+        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, res);
+        if (qi < a.T) row_r = a.delta[lrow];
+    }
+    const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    f32x16 acc[HB];
+#pragma unroll
+    for (int db = 0; db < HB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+    commit(0);
+    if (kt.n > 1) fetch(1);
+    __syncthreads();
+
+    const auto loop = [&](auto role_c) {
+        constexpr int ROLE = decltype(role_c)::value;
+        for (int i = 0; i < kt.n; ++i) {
+            const uint16_t* Ks = lds + (i & 1) * TILE;
+            const int k0 = kt.tile(i) * 32;
+            const bool live = k0 < a.T && qlo < a.T && !(a.causal && k0 > qhi) && !(a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks);
+            f32x16 t;
+            if (live) {
+                t = dot3<D>(ROLE == 0 ? Ks : Ks + 3 * PLANE, res, c32, g);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) t[r] = ROLE == 0 ? __builtin_amdgcn_exp2f(fmaf(t[r], cexp, row_r)) : t[r] - row_r;
+                const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
+                if (kind != MaskKind::NONE) mask_block(t, kind, vis, k0 + g * 4, 0.0f);
+                put_tile(cbuf[ROLE] + qg * 1024, t, lane);
+            }
+            if (i + 1 < kt.n) {
+                commit(i + 1);
+                if (i + 2 < kt.n) fetch(i + 2);
+            }
+            __syncthreads();
+            if (live) {
+                const f32x16 o = get_tile(cbuf[1 - ROLE] + qg * 1024, lane);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) t[r] *= o[r];
+                accumulate3<D, HB>(Ks, t, acc, lane, ROLE * HB);
+            }
+            __syncthreads();
+        }
+    };
+    if (role == 0)
+        loop(std::integral_constant<int, 0>{});
+    else
+        loop(std::integral_constant<int, 1>{});
+    if (qi < a.T) {
+        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+#pragma unroll
+        for (int db = 0; db < HB; ++db)
+            if (role * HB + db < DB) store_block32<D>(a.dq, ro, role * HB + db, g, acc[db], a.scale, dk);
+    }
+}
+
+// Which form a launch takes, from its number of 32-row blocks and the length of a block's chain; NONE leaves it to the kernels
+// on the fp32 instruction, which split a block's tiles four or eight ways (attn_f32_split.hip) and are ahead while that is what
+// fills the chip. PAIR: 64 rows, two groups of two wavefronts that take every other tile; WIDE: 128 rows (256 at 128 columns).
+// Over 840 random shapes of 100 to 6000 tokens and 100 or more blocks the launches that come here are 1.2 (32 columns) to 1.7
+// (96) times as fast as on the fp32 instruction in the geometric mean. Measured (us, fp32 | PAIR | WIDE; causal unless said):
+//   forward, 64 columns    T 1024 x 4, 8 heads 57 | 42 | 60;   T 4096 x 4, 16 heads 1155 | 814 | 716;  T 2048, 8 heads 48 | 74 | 115
+//   dQ                     80 | 56 | 75;                       1595 | 1077 | 953;                      68 | 89 | 136
+//   dK/dV (64 | 128 keys)  101 | 70 | 79;                      2282 | 1450 | 1390;                     81 | 124 | 146
+//   128 columns            T 4096 x 4, 16 heads: forward 2135 | 2257 | 1374, dQ 3262 | 2140, dK/dV 4240 | 3450 | 3470
+//                          T 2420, 8 heads 146 | 164 | 281;  T 4403, 8 heads 426 | 356 | 526;  no mask, T 1634, 8 heads 151 | 119 | 209
+enum class Form { NONE, PAIR, WIDE };
+
+int64_t blocks_of(const AttnArgs& a, int64_t units) { return static_cast<int64_t>((a.T + 31) / 32) * units; }
+// all blocks about as long as the longest: half the launch is not over before it
+bool level(const AttnArgs& a) { return !a.causal || 2 * chain_tokens(a) <= a.T; }
+
+Form fwd_form(const AttnArgs& a) {
+    const int64_t blocks = blocks_of(a, static_cast<int64_t>(a.Hq) * a.B);
+    if (a.T <= (a.dk_dim > 96 ? 128 : 32)) return Form::NONE;  // one tile to a block, or hardly more
+    if (a.dk_dim <= 32) return blocks < (level(a) ? 800 : 900) ? Form::NONE : blocks < 3000 ? Form::PAIR : Form::WIDE;
+    if (a.dk_dim <= 64) return blocks < (level(a) ? 500 : 700) ? Form::NONE : blocks < 2500 ? Form::PAIR : Form::WIDE;
+    if (a.dk_dim <= 96) return blocks < (level(a) ? 250 : 640) ? Form::NONE : blocks < (level(a) ? 1100 : 2100) ? Form::PAIR : Form::WIDE;
+    if (blocks < (level(a) ? 260 : 700)) return Form::NONE;
+    return blocks < (level(a) ? 1050 : 1500) ? Form::PAIR : Form::WIDE;
+}
+Form dq_form(const AttnArgs& a) {
+    const int64_t blocks = blocks_of(a, static_cast<int64_t>(a.Hq) * a.B);
+    if (a.T <= 32) return Form::NONE;
+    if (a.dk_dim <= 32) return blocks < (level(a) ? 400 : 750) ? Form::NONE : Form::PAIR;
+    if (a.dk_dim <= 64) return blocks < (level(a) ? 300 : 660) ? Form::NONE : blocks < 2500 ? Form::PAIR : Form::WIDE;
+    return blocks < (level(a) ? 260 : chain_tokens(a) < 600 ? 600 : 730) ? Form::NONE : Form::WIDE;
+}
+// The query heads of a group are dealt out where the launch would be on the fp32 instruction, which is what its workspace is sized
+// for (f32_deals_heads): with 64 keys to a workgroup the others have enough of them. The blocks are those of all splits.
+int head_split(const AttnArgs& a) { return f32_deals_heads(a) ? a.head_split : 1; }
+Form dkdv_form(const AttnArgs& a) {
+    const int64_t blocks = blocks_of(a, static_cast<int64_t>(a.Hkv) * a.B * head_split(a));
+    const int chain = chain_tokens(a);
+    // a sink keys' block that walks every query of every head of its group (32 heads on 8, T 1625, window 122: 100 us | 136; T 843 x
+    // 6, window 79: 139 | 206)
+    if (a.window > 0 && a.sinks > 0 && blocks < (a.Hq > a.Hkv ? 2000 : 800)) return Form::NONE;
+    if (a.dk_dim <= 32) return blocks < (level(a) ? (chain < 130 ? 2000 : chain < 400 ? 1000 : 840) : 1250) ? Form::NONE : Form::PAIR;
+    if (a.dk_dim <= 64) return blocks < (!level(a) ? 700 : chain <= 200 ? 400 : 512) ? Form::NONE : Form::PAIR;
+    if (a.dk_dim <= 96) return blocks < (level(a) ? 260 : 600) ? Form::NONE : blocks < (level(a) ? 600 : 900) ? Form::PAIR : Form::WIDE;
+    return blocks < (level(a) ? 260 : 450) ? Form::NONE : Form::PAIR;
+}
+// Whether the queries past the band of the sink keys' block go to workgroups of their own: split_tail_pays, and the pieces, which
+// walk all heads of a group, are shorter than the block's chain through its share of the heads.
+bool tail_pays(const AttnArgs& a, int block_rows) {
+    const SinkTail t = sink_tail(a.T, a.window, a.sinks);
+    const int64_t rep = a.Hq / a.Hkv, share = (rep + a.head_split - 1) / a.head_split, left = a.T - t.q0;
+    return split_tail_pays(a, a.head_split, block_rows) && share * left > rep * (left < TAIL_CHUNK ? left : TAIL_CHUNK);
+}
+
+template <int D, int QW, int KW>
+int run_fwd(const AttnArgs& a, hipStream_t st) {
+    const int nqb = (a.T + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((x3_fwd<D, QW, KW>), dim3(xcd_grid(nqb, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+template <int D, int QW, int KW>
+int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    const int nqb = (a.T + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((x3_dq<D, QW, KW>), dim3(xcd_grid(nqb, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(64 * QW * KW), 0, st, a, fuse_delta ? 1 : 0);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+template <int D>
+int run_dq_wide(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    hipLaunchKernelGGL((x3_dq_wide<D>), dim3(xcd_grid((a.T + 127) / 128, a.Hq / a.Hkv, a.Hkv * a.B)), dim3(512), 0, st, a, fuse_delta ? 1 : 0);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+template <int D, int QW>
+int run_dkdv(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
+    a.head_split = head_split(a);
+    if (!tail_pays(a, 32 * QW)) a.tail = nullptr;
+    const int nkb = (a.T + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((x3_dkdv<D, QW>), dim3(xcd_grid(nkb + tail_blocks(a), a.head_split, a.Hkv * a.B)), dim3(128 * QW), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
+}
+
+}  // namespace
+
+// what the fp32 split kernels ask of their tensors holds for these as well
+bool f32x3_takes_fwd(const AttnArgs& a) { return f32_split_serves(a) && fwd_form(a) != Form::NONE; }
+bool f32x3_takes_dq(const AttnArgs& a) { return f32_split_serves(a) && dq_form(a) != Form::NONE; }
+bool f32x3_takes_dkdv(const AttnArgs& a) { return f32_split_serves(a) && dkdv_form(a) != Form::NONE; }
+
+int launch_f32x3_fwd(const AttnArgs& a, hipStream_t st) {
+    const bool wide = fwd_form(a) == Form::WIDE;
+    if (a.dk_dim <= 32) return wide ? run_fwd<32, 4, 1>(a, st) : run_fwd<32, 2, 2>(a, st);
+    if (a.dk_dim <= 64) return wide ? run_fwd<64, 4, 1>(a, st) : run_fwd<64, 2, 2>(a, st);
+    if (a.dk_dim <= 96) return wide ? run_fwd<96, 4, 1>(a, st) : run_fwd<96, 2, 2>(a, st);
+    if (!wide) return run_fwd<128, 2, 2>(a, st);
+    // 256 rows are mostly cut off by the ends of short sequences and bands (T 230 x 40, 8 heads 90 us, with 128 rows 71)
+    return chain_tokens(a) <= 320 ? run_fwd<128, 4, 1>(a, st) : run_fwd<128, 8, 1>(a, st);
+}
+int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
+    const bool wide = dq_form(a) == Form::WIDE;
+    if (a.dk_dim <= 32) return run_dq<32, 2, 2>(a, fuse_delta, st);
+    if (a.dk_dim <= 64) return wide ? run_dq<64, 4, 1>(a, fuse_delta, st) : run_dq<64, 2, 2>(a, fuse_delta, st);
+    return a.dk_dim <= 96 ? run_dq_wide<96>(a, fuse_delta, st) : run_dq_wide<128>(a, fuse_delta, st);
+}
+int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st) {
+    if (a.dk_dim <= 32) return run_dkdv<32, 2>(a, st);
+    if (a.dk_dim <= 64) return run_dkdv<64, 2>(a, st);
+    if (a.dk_dim <= 96) return dkdv_form(a) == Form::WIDE ? run_dkdv<96, 4>(a, st) : run_dkdv<96, 2>(a, st);
+    return run_dkdv<128, 2>(a, st);
+}
+
+}  // namespace pk

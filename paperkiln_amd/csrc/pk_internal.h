@@ -150,6 +150,15 @@ int launch_f32_split_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_f32_split_dkdv(const AttnArgs& a, hipStream_t st);
 
+// attn_f32x3.hip: fp32 on the bf16 matrix instruction, every value as three bf16 parts; the head sizes and rows that
+// attn_f32_split.hip serves, launches with enough blocks.
+bool f32x3_takes_fwd(const AttnArgs& a);
+bool f32x3_takes_dq(const AttnArgs& a);
+bool f32x3_takes_dkdv(const AttnArgs& a);
+int launch_f32x3_fwd(const AttnArgs& a, hipStream_t st);
+int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
+int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st);
+
 // attn_f32_mfma.hip: fp32 tensors on the fp32 matrix instruction, head sizes that are multiples of 4 up to 128.
 bool f32_mfma_supported(const AttnArgs& a);
 int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st);

@@ -163,6 +163,45 @@ def test_fp32_split_kernels(case, dk):
     assert max(e) < 5e-6, e
 
 
+# fp32 values as three bf16 parts, in launches with the blocks for it: both forms of every kernel, lengths around the 32-row tile
+# and the 64- and 128-row blocks, fewer tiles than groups of wavefronts, padded columns, dealt heads and dealt sink tails. What is
+# left is fp32 rounding: of a score, of its exponential, and once a tile of the sums, a few times 6e-8 of the norm.
+PARTS_CASES = [(20, 161, 11, 11, True, 0, 0), (64, 33, 9, 9, False, 0, 0), (7, 577, 16, 8, True, 0, 0), (13, 511, 16, 16, False, 0, 0),
+               (3, 1100, 16, 4, True, 0, 0), (12, 383, 8, 8, True, 37, 5), (1, 2500, 14, 2, True, 0, 0), (10, 1411, 8, 8, True, 33, 9),
+               (40, 129, 16, 16, True, 0, 0)]
+
+
+@pytest.mark.parametrize("dk", [4, 24, 32, 44, 64, 80, 96, 100, 128])
+@pytest.mark.parametrize("case", PARTS_CASES, ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_fp32_as_three_parts(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    got, want = run_attention(B, T, Hq, Hkv, dk, torch.float32, causal, window, sinks)
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(got, want)]
+    assert max(e) < 1e-6, e
+
+
+def test_fp32_as_three_parts_over_the_range_of_fp32():
+    """Columns of V from 1e-25 to 1e35 (P reaches 2^6 and their sum the number of keys), each exact at its own size; a NaN reaches
+    what it should."""
+    B, T, H, dk = 24, 200, 8, 64
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn((B, T, H, dk), generator=gen, device="cuda") for _ in range(3))
+    size = torch.logspace(-25, 35, dk, device="cuda")
+    v = v * size
+    v[3, 150, 2, 7] = float("nan")
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, _ = ops.attn_fwd(q, k, v, scale)
+    p = torch.softmax((scale * (q.double().permute(0, 2, 1, 3) @ k.double().permute(0, 2, 3, 1).contiguous()))
+                      .masked_fill(torch.ones(T, T, device="cuda").triu(1).bool(), float("-inf")), -1)
+    want = (p @ v.double().nan_to_num(nan=0.0).permute(0, 2, 1, 3).contiguous()).permute(0, 2, 1, 3)
+    bad = torch.isnan(o)
+    assert bad[3, 150:, 2, 7].all() and int(bad.sum()) == int(bad[3, :, 2, 7].sum())
+    good = torch.ones(dk, dtype=torch.bool, device="cuda")
+    good[7] = False
+    d = (o.double() - want).reshape(-1, dk).norm(dim=0) / want.reshape(-1, dk).norm(dim=0)
+    assert float(d[good].max()) < 1e-6, d
+
+
 # Either side of the lines between the two geometries of the 32-key dK/dV kernel: one round of the chip and one head more, two
 # nearly whole rounds, and with a band and sink keys whose queries are dealt out or left whole.
 @pytest.mark.parametrize("case,dk", [((32, 200, 8, 8, True, 0, 0), 64), ((33, 200, 4, 4, True, 0, 0), 64), ((16, 200, 8, 8, True, 0, 0), 64),
