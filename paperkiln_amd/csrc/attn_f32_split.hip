@@ -214,13 +214,17 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
 
 // ---- dQ (and delta, when asked for with it) ----
 template <int D, int KW>
-__global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_dq(AttnArgs a, int fuse_delta) {
-    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P, RED = KW * DB * 1024;
-    __shared__ __attribute__((aligned(16))) float lds[KW * TILE > RED ? KW * TILE : RED];
+constexpr int dq_lds() {  // floats
+    constexpr int TILE = 2 * 32 * (D + 4), RED = KW * (D / 32) * 1024;
+    return KW * TILE > RED ? KW * TILE : RED;
+}
+template <int D, int KW>
+__device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float* lds) {
+    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P;
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
     int b, h, hk, qblk;
-    if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk)) return;
+    if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk, id)) return;
     const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
     const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
     const float cexp = a.scale * LOG2E;
@@ -287,16 +291,32 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
             if (db % KW == kg) store_block(true, a.dq, ro, db, g, acc[db], a.scale, dk);
     }
 }
+template <int D, int KW>
+__global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_dq(AttnArgs a, int fuse_delta) {
+    __shared__ __attribute__((aligned(16))) float lds[dq_lds<D, KW>()];
+    dq_block<D, KW>(a, fuse_delta, static_cast<int>(blockIdx.x), lds);
+}
 
 // ---- dK, dV: a block of 32 keys, the query tiles (of every query head of the group in turn) split ----
+// OWN_DELTA: the rows' delta is formed here, from O and the tile of dO, in the order of dq_block and to the same bits; otherwise
+// it is read.
+//
+// K and V of the block stay in LDS, one copy for all wavefronts, where registers are short and the LDS has the room (at D = 128
+// for K only).
+template <int D>
+constexpr bool V_IN_LDS = D == 64 || D == 96;
+template <int D>
+constexpr bool K_IN_LDS = V_IN_LDS<D> || D == 128;
 template <int D, int KW>
-__global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) void f32_split_dkdv(AttnArgs a) {
-    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P + 64, RED = KW * DB * 1024;
-    // K and V of the block stay in LDS, one copy for all wavefronts, where registers are short and the LDS has the room
-    // (at D = 128 for K only)
-    constexpr bool V_LDS = D == 64 || D == 96, K_LDS = V_LDS || D == 128;
+constexpr int dkdv_lds() {  // floats
+    constexpr int TILE = 2 * 32 * (D + 4) + 64, RED = KW * (D / 32) * 1024;
+    return (K_IN_LDS<D> + V_IN_LDS<D>) * 32 * (D + 4) + (KW * TILE > RED ? KW * TILE : RED);
+}
+template <int D, int KW, bool OWN_DELTA>
+__device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
+    constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P + 64;
+    constexpr bool V_LDS = V_IN_LDS<D>, K_LDS = K_IN_LDS<D>;
     constexpr int KVB = (K_LDS + V_LDS) * 32 * P;
-    __shared__ __attribute__((aligned(16))) float lds[KVB + (KW * TILE > RED ? KW * TILE : RED)];
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
     const int nkb = (a.T + 31) / 32;
@@ -306,7 +326,7 @@ __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) 
     const int nblk = nkb + tl.nch;
     int blk, rr, kvu;
     // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
-    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu))
+    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu, id) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu, id))
         return;
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
@@ -337,7 +357,10 @@ __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) 
         const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * 32;
         mq.load(a.q, b * a.q_sb + h * a.q_sh, a.q_st, r0, a.T, dk);
         const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(r0 + c32, a.T - 1);  // rows past the end are masked
-        row_r = g == 0 ? a.lse[lrow] : a.delta[lrow];
+        if (g == 0)
+            row_r = a.lse[lrow];
+        else if (!OWN_DELTA)
+            row_r = a.delta[lrow];
         c_h = h, c_r0 = r0;
         f_t += KW;
         while (f_t >= nqt) f_t -= nqt, ++f_h;
@@ -373,12 +396,26 @@ __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) 
     for (int step = kg; step < steps; step += KW) {
         const int qlo = c_r0, qhi = qlo + 31;
         mq.store(Qs, lane);
-        rows[lane] = g == 0 ? -row_r * LOG2E : row_r;
+        if (!OWN_DELTA || g == 0) rows[lane] = g == 0 ? -row_r * LOG2E : row_r;
         tile_barrier<1>();
         mg.load(a.d_o, b * a.do_sb + c_h * a.do_sh, a.do_st, qlo, a.T, dk);
+        f32x4 oreg[OWN_DELTA ? D / 8 : 1];
+        if constexpr (OWN_DELTA) load_row32<D>(a.o, b * a.o_sb + c_h * a.o_sh, a.o_st, qlo + c32, a.T, dk, g, oreg);
         f32x16 s = dot(Qs, K_LDS, kreg, lds);
         mg.store(Gs, lane);
         tile_barrier<1>();
+        if constexpr (OWN_DELTA) {
+            float part = 0.0f;
+#pragma unroll
+            for (int j = 0; j < D / 8; ++j) {
+                const f32x4 gv = *reinterpret_cast<const f32x4*>(Gs + c32 * P + 8 * j + 4 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) part = fmaf(oreg[j][i], gv[i], part);
+            }
+            part = xhalf_sum(part);
+            if (g == 1) rows[lane] = part;
+            tile_barrier<1>();
+        }
         if (step + KW < steps) fetch_q();
         if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks))) {
             // lane = key kj; element r = query qlo + crow(r, g)
@@ -431,6 +468,25 @@ __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) 
             store_block(true, dst_k, rk, db, g, acc[DB + db], a.scale, dk);
         }
     }
+}
+template <int D, int KW>
+__global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) void f32_split_dkdv(AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) float lds[dkdv_lds<D, KW>()];
+    dkdv_block<D, KW, false>(a, static_cast<int>(blockIdx.x), lds);
+}
+
+// ---- dK, dV and dQ in one launch ----
+// Two launches of a handful of workgroups each, the second waiting for the first one's delta, are two round trips to memory with
+// most CUs idle. Here blocks 0 .. dkdv_ids - 1 are the dK/dV launch's, which forms its own delta, and the others the dQ launch's.
+template <int D>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_split_bwd(AttnArgs a, int dkdv_ids) {
+    constexpr int Q = dq_lds<D, 4>(), K = dkdv_lds<D, 4>();
+    __shared__ __attribute__((aligned(16))) float lds[Q > K ? Q : K];
+    const int id = static_cast<int>(blockIdx.x);
+    if (id < dkdv_ids)
+        dkdv_block<D, 4, true>(a, id, lds);
+    else
+        dq_block<D, 4>(a, 1, id - dkdv_ids, lds);
 }
 
 // A block's tiles split between four or eight wavefronts, or not this kernel.
@@ -515,6 +571,11 @@ void run_dkdv(const AttnArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((f32_split_dkdv<D, KW>), dim3(xcd_grid((a.T + 31) / 32 + tail_blocks(a), a.head_split, a.Hkv * a.B)), dim3(64 * KW), 0, st, a);
 }
 
+template <int D>
+void run_bwd(const OneLaunch& l, hipStream_t st) {
+    hipLaunchKernelGGL(f32_split_bwd<D>, dim3(l.dkdv_ids + l.dq_ids), dim3(256), 0, st, l.a, l.dkdv_ids);
+}
+
 }  // namespace
 
 // a lane's byte offset inside a 32-row tile is kept in 31 bits
@@ -566,6 +627,35 @@ int launch_f32_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
         run_dkdv<128, 4>(a, st);
     PK_HIP(hipGetLastError());
     return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
+}
+
+// dQ and dK/dV in one launch: while their workgroups find room on the chip together, one to a CU above 32 columns, or nearly do
+// where causal chains are of very different length. Measured, the launches of a backward one after the other | this one (us):
+//   head_dim 32   T 194, 16 heads 19.0 | 13.9;  T 623 x 2, 8 heads 36 | 28;  T 640, 32 heads on 8 50 | 50
+//            64   T 511, 8 heads 41 | 29;  T 872 x 8, 1 head 68 | 46;  T 41 x 7, 8 heads, no mask 21 | 12.6;  T 2931, 4 heads 174 | 181
+//            128  T 370, 16 heads 74 | 68;  no mask: T 56 x 46, 2 heads 41 | 47, T 1179 x 3, 2 heads 233 | 314
+// Over 300 random shapes of up to 1000 blocks it is 1.2 to 1.7 times as fast as they are below these lines.
+bool f32_split_takes_bwd(const AttnArgs& a) {
+    if (!f32_split_serves(a)) return false;
+    const OneLaunch l(a);
+    const int ids = l.dkdv_ids + l.dq_ids;
+    if (a.dk_dim <= 32) return ids <= (even_chains(a) ? 800 : 960);
+    if (ids <= 256) return true;
+    if (a.dk_dim > 96 || a.T <= 32 || chain_tokens(a) > 2600) return false;  // (one tile: T 24 x 104, 2 heads of 64 16.3 | 21.1)
+    return ids <= (even_chains(a) ? 300 : 700);
+}
+int launch_f32_split_bwd(const AttnArgs& a, hipStream_t st) {
+    const OneLaunch l(a);
+    if (a.dk_dim <= 32)
+        run_bwd<32>(l, st);
+    else if (a.dk_dim <= 64)
+        run_bwd<64>(l, st);
+    else if (a.dk_dim <= 96)
+        run_bwd<96>(l, st);
+    else
+        run_bwd<128>(l, st);
+    PK_HIP(hipGetLastError());
+    return l.finish(st);
 }
 
 }  // namespace pk

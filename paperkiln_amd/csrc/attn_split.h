@@ -100,6 +100,22 @@ inline bool split_tail_pays(const AttnArgs& a, int head_split, int block_rows) {
 }
 inline int tail_blocks(const AttnArgs& a) { return a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0; }
 
+// A backward whose dK/dV and dQ blocks of 32 rows go into one launch: the arguments of its dK/dV part, and the two kinds' ids. Heads
+// of a group are dealt out where the workspace holds their partial sums.
+struct OneLaunch {
+    AttnArgs a;
+    int dkdv_ids, dq_ids;
+    explicit OneLaunch(const AttnArgs& args) : a(args) {
+        if (!a.part) a.head_split = 1;
+        if (!split_tail_pays(a, a.head_split, 32)) a.tail = nullptr;
+        const int nblk = (a.T + 31) / 32, units = a.Hkv * a.B;
+        dkdv_ids = xcd_grid(nblk + tail_blocks(a), a.head_split, units);
+        dq_ids = xcd_grid(nblk, a.Hq / a.Hkv, units);
+    }
+    // partial sums, as after a dK/dV launch
+    int finish(hipStream_t st) const { return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK; }
+};
+
 // The tiles of BN keys that queries [q0, q0 + BM) can see, as a list: sink tiles [0, ns), then [lo, hi].
 struct KeyTiles {
     int ns, lo, n;
@@ -113,12 +129,12 @@ struct KeyTiles {
     __device__ int tile(int i) const { return i < ns ? i : lo + i - ns; }
 };
 
-__device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk) {
+__device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk, int id = static_cast<int>(blockIdx.x)) {
     const int rep = a.Hq / a.Hkv;
     int blk, rr, kvu;
     // causal blocks without a band: the heaviest blocks of every unit first
-    if (a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu)
-                                  : !xcd_map(nqb, rep, a.Hkv * a.B, blk, rr, kvu))
+    if (a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu, id)
+                                  : !xcd_map(nqb, rep, a.Hkv * a.B, blk, rr, kvu, id))
         return false;
     hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
     qblk = nqb - 1 - blk;

@@ -101,6 +101,18 @@ __device__ inline float weight_of(float s, float scale, float cexp, float nl) {
     return __builtin_amdgcn_exp2f(EXACT ? fmaf(s, scale, nl) * LOG2E : fmaf(s, cexp, nl));
 }
 
+// sum + the products of eight elements, in order
+__device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
+    const u32x4 xv = *reinterpret_cast<const u32x4*>(&x);
+    const u32x4 yv = *reinterpret_cast<const u32x4*>(&y);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sum = fmaf(__uint_as_float(xv[i] << 16), __uint_as_float(yv[i] << 16), sum);
+        sum = fmaf(__uint_as_float(xv[i] & 0xFFFF0000u), __uint_as_float(yv[i] & 0xFFFF0000u), sum);
+    }
+    return sum;
+}
+
 // acc[db] += M^T c for the 32 rows of an LDS tile that start at row0, M the tile (columns 32 db ..), c a C tile whose rows
 // are the tile's rows, as PARTS operands
 template <int D, int PARTS>
@@ -295,19 +307,22 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
 }
 
 // ---- dQ (and delta, when asked for with it): the same blocks ----
+template <int D, int QW, int KW, int NB>
+constexpr int dq_lds() {  // in uint16
+    constexpr int TILES = (QW > 1 ? 2 : 1) * KW * 2 * 32 * NB * (D + 8), RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
+    return TILES > RED ? TILES : RED;
+}
 template <int D, int QW, int KW, int NB, bool EXACT>
-__global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
+__device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint16_t* lds) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
-    constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;  // in uint16
-    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
     const int nqb = (a.T + BM - 1) / BM;
     int b, h, hk, qblk;
-    if (!map_query_block(a, nqb, b, h, hk, qblk)) return;
+    if (!map_query_block(a, nqb, b, h, hk, qblk, id)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
     const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
     const float cexp = a.scale * LOG2E;
@@ -342,15 +357,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse
         load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, qi, a.T, dk, g, oreg);
         float part = 0.0f;
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            const u32x4 ov = *reinterpret_cast<const u32x4*>(&oreg[kk]);
-            const u32x4 gv = *reinterpret_cast<const u32x4*>(&greg[kk]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                part = fmaf(__uint_as_float(ov[i] << 16), __uint_as_float(gv[i] << 16), part);
-                part = fmaf(__uint_as_float(ov[i] & 0xFFFF0000u), __uint_as_float(gv[i] & 0xFFFF0000u), part);
-            }
-        }
+        for (int kk = 0; kk < KK; ++kk) part = add_products(oreg[kk], greg[kk], part);
         dl = xhalf_sum(part);
         if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
     } else if (qi < a.T) {
@@ -403,18 +410,30 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse
             if (KW == 1 || db % KW == kg) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk);
     }
 }
+template <int D, int QW, int KW, int NB, bool EXACT>
+__global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
+    __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW, NB>()];
+    dq_block<D, QW, KW, NB, EXACT>(a, fuse_delta, static_cast<int>(blockIdx.x), lds);
+}
 
 // ---- dK, dV: QW groups of 32 keys x KW groups of query tiles of 32 NB ----
 // A wavefront owns 32 keys (K and V resident as B operands, lane = key) and both accumulators, so P goes from its
 // exponentials into dV and into dS without leaving the registers. The steps are the query tiles that can see the block,
 // for every query head of the KV head's group in turn.
-template <int D, int QW, int KW, int NB, bool EXACT, int OCC>
-__global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
+//
+// OWN_DELTA (one wavefront to a group, tiles of 32): the rows' delta is formed here, from O and the tile of dO, in the order of
+// dq_block and to the same bits; otherwise it is read.
+template <int D, int QW, int KW, int NB>
+constexpr int dkdv_lds() {  // in uint16; LSE and delta of a tile's rows behind it
+    constexpr int TILES = (QW > 1 ? 2 : 1) * KW * (2 * 32 * NB * (D + 8) + 128 * NB), RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
+    return TILES > RED ? TILES : RED;
+}
+template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA>
+__device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
+    static_assert(!OWN_DELTA || (QW == 1 && NB == 1), "a lane holds the row of O whose row of dO its wavefront has just written");
     constexpr int BNK = 32 * QW, BMQ = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int ROWC = 2 * BMQ * 2;                    // LSE and delta of a tile's rows, in uint16
     constexpr int TILE = 2 * BMQ * S + ROWC, NBUF = QW > 1 ? 2 : 1;
-    constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;
-    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
@@ -428,7 +447,7 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
     const int nblk = nkb + tl.nch;
     int blk, rr, kvu;
     // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
-    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu))
+    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu, id) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu, id))
         return;
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
@@ -449,6 +468,7 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
     mq.init(gt, a.q_st, dk);
     mg.init(gt, a.do_st, dk);
     float row_r = 0.0f;
+    bf16x8 oreg[OWN_DELTA ? KK : 1];
     // steps advance by KW; the (head, tile) of the next fetch is counted up
     int f_h = kg / nqt, f_t = kg % nqt, c_t = f_t;
     auto fetch = [&](int i) {
@@ -459,8 +479,12 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
             if (gt < 2 * BMQ) {  // LSE in the first BMQ threads, delta in the next; rows past the end are masked
                 const int t = min(r0 + gt % BMQ, a.T - 1);
                 const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + t;
-                row_r = gt < BMQ ? a.lse[lrow] : a.delta[lrow];
+                if (gt < BMQ)
+                    row_r = a.lse[lrow];
+                else if (!OWN_DELTA)
+                    row_r = a.delta[lrow];
             }
+            if constexpr (OWN_DELTA) load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, r0 + c32, a.T, dk, g, oreg);
             f_t += KW;
             while (f_t >= nqt) f_t -= nqt, ++f_h;
         }
@@ -469,7 +493,16 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
         uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
         mq.store(t, S, gt);
         mg.store(t + BMQ * S, S, gt);
-        if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = gt >= BMQ ? row_r : EXACT ? -row_r : -row_r * LOG2E;
+        float out = gt >= BMQ ? row_r : EXACT ? -row_r : -row_r * LOG2E;
+        if constexpr (OWN_DELTA) {
+            tile_barrier<1>();
+            float part = 0.0f;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) part = add_products(oreg[kk], lds_read8(t + BMQ * S + c32 * S + kk * 16 + g * 8), part);
+            part = xhalf_sum(part);
+            if (g == 1) out = part;
+        }
+        if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = out;
     };
     fetch(0);
     bf16x8 kreg[KK], vreg[KK];
@@ -561,7 +594,24 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
         }
     }
 }
+template <int D, int QW, int KW, int NB, bool EXACT, int OCC>
+__global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) uint16_t lds[dkdv_lds<D, QW, KW, NB>()];
+    dkdv_block<D, QW, KW, NB, EXACT, false>(a, static_cast<int>(blockIdx.x), lds);
+}
 
+// ---- dK, dV and dQ in one launch, as in attn_f32_split.hip ----
+// Blocks 0 .. dkdv_ids - 1 are the dK/dV launch's, which forms its own delta, and the others the dQ launch's.
+template <int D, bool EXACT>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, int dkdv_ids) {
+    constexpr int Q = dq_lds<D, 1, 4, 1>(), K = dkdv_lds<D, 1, 4, 1>();
+    __shared__ __attribute__((aligned(16))) uint16_t lds[Q > K ? Q : K];
+    const int id = static_cast<int>(blockIdx.x);
+    if (id < dkdv_ids)
+        dkdv_block<D, 1, 4, 1, EXACT, true>(a, id, lds);
+    else
+        dq_block<D, 1, 4, 1, EXACT>(a, 1, id - dkdv_ids, lds);
+}
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE), or one block of 32 rows whose tiles are
 // split between four or eight wavefronts.
@@ -722,6 +772,12 @@ int dkdv_of(const AttnArgs& a, Form f, hipStream_t st) {
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
+template <int D, bool EXACT>
+int bwd_of(const OneLaunch& l, hipStream_t st) {
+    hipLaunchKernelGGL((split_bwd<D, EXACT>), dim3(l.dkdv_ids + l.dq_ids), dim3(256), 0, st, l.a, l.dkdv_ids);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
 // f<D, EXACT>() for the instantiation that serves head_dim dk
 #define PK_SPLIT_DISPATCH(call)                        \
     do {                                               \
@@ -760,6 +816,30 @@ int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     };
     if (const int rc = run()) return rc;
     return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
+}
+
+// dQ and dK/dV in one launch: while their workgroups find room on the chip together, two to a CU up to 64 columns and one above.
+// Measured, the launches of a backward one after the other | this one (us): head_dim 64 T 64, 16 heads 11.1 | 7.0, T 300 x 2, 8 heads 23 | 17;
+// 128 T 128 x 2, 8 heads 16 | 12, T 25 x 8, 1 head 11.0 | 12.3, T 64 x 25, 4 heads, window 18 16 | 22; 96 no mask, T 2000, 4 heads 74 | 87; 24 T 4000,
+// 1 head 53 | 58. Over 460 random shapes of up to 1000 blocks it is 1.15 to 1.6 times as fast as they are below these lines.
+bool split_takes_bwd(const AttnArgs& a) {
+    const OneLaunch l(a);
+    const int ids = l.dkdv_ids + l.dq_ids;
+    if (chain_tokens(a) > 2600) return false;
+    if (a.dk_dim <= 32) return ids <= (even_chains(a) ? 400 : 960);
+    if (a.dk_dim <= 64) return ids <= (a.T <= 32 ? 400 : even_chains(a) ? 640 : 800);  // (one tile: T 31 x 84, 4 heads of 64 10.9 | 13.3)
+    if (a.dk_dim <= 96) return ids <= (even_chains(a) ? 380 : 400);
+    return ids <= 256 && (a.dk_dim < 128 || a.T > 32);
+}
+int launch_split_bwd(const AttnArgs& a, hipStream_t st) {
+    const OneLaunch l(a);
+    const auto run = [&]() -> int {
+#define PK_CALL(D, E) bwd_of<D, E>(l, st)
+        PK_SPLIT_DISPATCH(PK_CALL);
+#undef PK_CALL
+    };
+    if (const int rc = run()) return rc;
+    return l.finish(st);
 }
 
 }  // namespace pk

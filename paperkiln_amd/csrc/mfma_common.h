@@ -287,8 +287,10 @@ __device__ inline bool xcd_loose_block(int idx, int nblk, int rep, int kv_units,
 }
 // blk: block index inside the unit (0 = dispatched first); r: query head inside
 // the GQA group; kvu: (batch, KV head) unit. Returns false for padding ids.
-__device__ inline bool xcd_map(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu) {
-    const int xcd = blockIdx.x & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = static_cast<int>(blockIdx.x >> 3) - loose;
+// id: the workgroup's number in a launch of its own (launches of two kinds of blocks count each kind from 0, the second from a
+// multiple of 8 on).
+__device__ inline bool xcd_map(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu, int id = static_cast<int>(blockIdx.x)) {
+    const int xcd = id & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = (id >> 3) - loose;
     if (j < 0) return xcd_loose_block((j + loose) * 8 + xcd, nblk, rep, kv_units, blk, r, kvu);
     blk = j % nblk;
     r = (j / nblk) % rep;
@@ -300,8 +302,8 @@ __device__ inline bool xcd_map(int nblk, int rep, int kv_units, int& blk, int& r
 // hands the CUs the longest workgroups first whatever the number of units (longest-processing-time order); with
 // the unit-major order above the last units' heavy blocks start late and stretch the tail of the launch
 // (512 unpaired workgroups of 256 queries at B x H = 32, T = 4096 took 232 us against 208 for the smaller kernel).
-__device__ inline bool xcd_map_block_major(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu) {
-    const int xcd = blockIdx.x & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = static_cast<int>(blockIdx.x >> 3) - loose;
+__device__ inline bool xcd_map_block_major(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu, int id = static_cast<int>(blockIdx.x)) {
+    const int xcd = id & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = (id >> 3) - loose;
     if (j < 0) return xcd_loose_block((j + loose) * 8 + xcd, nblk, rep, kv_units, blk, r, kvu);
     const int per = (kv_units / 8) * rep;  // (unit, head) pairs of one XCD
     blk = j / per;

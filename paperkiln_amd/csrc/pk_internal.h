@@ -149,6 +149,8 @@ bool f32_split_takes_dkdv(const AttnArgs& a);
 int launch_f32_split_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_f32_split_dkdv(const AttnArgs& a, hipStream_t st);
+bool f32_split_takes_bwd(const AttnArgs& a);  // dQ (with delta) and dK/dV in one launch
+int launch_f32_split_bwd(const AttnArgs& a, hipStream_t st);
 
 // attn_f32x3.hip: fp32 on the bf16 matrix instruction, every value as three bf16 parts; the head sizes and rows that
 // attn_f32_split.hip serves, launches with enough blocks.
@@ -175,6 +177,8 @@ bool split_takes_dkdv(const AttnArgs& a);
 int launch_split_fwd(const AttnArgs& a, hipStream_t st);
 int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_split_dkdv(const AttnArgs& a, hipStream_t st);
+bool split_takes_bwd(const AttnArgs& a);  // dQ (with delta) and dK/dV in one launch
+int launch_split_bwd(const AttnArgs& a, hipStream_t st);
 
 // attn_fwd_mfma.hip / attn_bwd_mfma.hip: bf16 MFMA kernels, head_dim 64 or 128.
 // 16-byte-aligned rows whose stride keeps a tile's byte offsets in 31 bits, and a positive scale (the running max is

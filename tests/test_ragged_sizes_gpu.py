@@ -202,6 +202,31 @@ def test_fp32_as_three_parts_over_the_range_of_fp32():
     assert float(d[good].max()) < 1e-6, d
 
 
+# dQ and dK/dV in one launch against the two launches of the same call's stages: the forms, and so the order of the sums, may differ,
+# nothing else does. Few tiles and remainders, groups of heads dealt out and not, sink tails, the largest launches that go together.
+@pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 24), (torch.bfloat16, 64), (torch.bfloat16, 96), (torch.bfloat16, 128), (torch.float32, 20),
+                                      (torch.float32, 64), (torch.float32, 96), (torch.float32, 128)], ids=str)
+@pytest.mark.parametrize("case", [(1, 1, 1, 1, True, 0, 0), (3, 33, 2, 1, False, 0, 0), (2, 129, 7, 1, True, 0, 0), (1, 770, 2, 2, True, 64, 1),
+                                  (1, 1300, 7, 1, True, 100, 32), (5, 200, 4, 4, True, 0, 0), (1, 97, 64, 8, True, 0, 0)], ids=str)
+def test_backward_in_one_launch(case, dtype, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    q, k, v, d_o = (torch.randn((B, T, h, dk), generator=gen, device="cuda").to(dtype) for h in (Hq, Hkv, Hkv, Hq))
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    one = ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, grad_dtype=torch.float32)
+    bufs = [torch.empty(x.shape, dtype=torch.float32, device="cuda") for x in (q, k, v)]
+    ws = torch.empty(ops.bwd_workspace_bytes(q, k, torch.float32, window, sinks), dtype=torch.uint8, device="cuda")
+    for stages in (ops.BWD_DELTA | ops.BWD_DQ, ops.BWD_DKDV):
+        ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, grad_dtype=torch.float32, out=(*bufs, ws), stages=stages)
+    # bf16 operands of P and dS at 64 and 128 columns: 2^-9 of a term each, of 4 standard deviations at most
+    tol = 1e-2 if dtype == torch.bfloat16 and dk in (64, 128) else 5e-6
+    for a, b in zip(one, bufs):
+        assert float((a - b).abs().max()) <= tol * max(float(b.abs().max()), 0.5)
+    e = errors((o, lse) + tuple(one), exact_attention(q, k, v, d_o, scale, causal, window, sinks))
+    assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
+
+
 # Either side of the lines between the two geometries of the 32-key dK/dV kernel: one round of the chip and one head more, two
 # nearly whole rounds, and with a band and sink keys whose queries are dealt out or left whole.
 @pytest.mark.parametrize("case,dk", [((32, 200, 8, 8, True, 0, 0), 64), ((33, 200, 4, 4, True, 0, 0), 64), ((16, 200, 8, 8, True, 0, 0), 64),
