@@ -301,7 +301,7 @@ int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 
 }  // namespace
 
-bool bf16_deals_heads(const AttnArgs& a) { return a.head_split > 1 && (split_takes_dkdv(a) || mfma_dkdv3_takes(a)); }
+bool bf16_deals_heads(const AttnArgs& a) { return a.head_split > 1 && (split_deals_heads(a) || mfma_dkdv3_takes(a)); }
 
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote

@@ -129,6 +129,36 @@ struct KeyTiles {
     __device__ int tile(int i) const { return i < ns ? i : lo + i - ns; }
 };
 
+// What of a tile a wavefront's 32 rows see, as comparisons with four numbers formed once: written out for every tile the tests were
+// half the instructions of a loop at 64 columns.
+//
+// Its 32 queries from qlo on against the 32 keys from k0 on: is any pair visible, are all?
+struct KeyRange {
+    int end, band, full_end, full_band, sinks;
+    __device__ KeyRange(const AttnArgs& a, int qlo) {
+        end = qlo >= a.T ? -1 : a.causal ? min(a.T - 1, qlo + 31) : a.T - 1;
+        band = a.window > 0 ? qlo - 30 - a.window : 0;
+        full_end = a.causal ? min(a.T - 32, qlo - 31) : a.T - 32;
+        full_band = a.window > 0 ? qlo + 32 - a.window : 0;
+        sinks = a.window > 0 ? a.sinks : 0;
+    }
+    __device__ bool live(int k0) const { return k0 <= end && (k0 >= band || k0 < sinks); }
+    __device__ bool full(int k0) const { return k0 <= full_end && (k0 >= full_band || k0 + 31 < sinks); }
+};
+// Its 32 keys from k0 on against the 32 queries from qlo on.
+struct QueryRange {
+    int lo, end, full_lo, full_end;
+    __device__ QueryRange(const AttnArgs& a, int k0) {
+        const bool band = a.window > 0;
+        lo = a.causal ? k0 - 31 : 0;
+        end = k0 >= a.T ? -1 : band && k0 >= a.sinks ? min(a.T - 1, k0 + 30 + a.window) : a.T - 1;
+        full_lo = a.causal ? k0 + 31 : 0;
+        full_end = k0 + 31 >= a.T ? -1 : band && k0 + 31 >= a.sinks ? min(a.T - 32, k0 + a.window - 32) : a.T - 32;
+    }
+    __device__ bool live(int qlo) const { return qlo >= lo && qlo <= end; }
+    __device__ bool full(int qlo) const { return qlo >= full_lo && qlo <= full_end; }
+};
+
 __device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk, int id = static_cast<int>(blockIdx.x)) {
     const int rep = a.Hq / a.Hkv;
     int blk, rr, kvu;

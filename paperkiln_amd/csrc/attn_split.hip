@@ -10,8 +10,8 @@
 // Which of these kernels a launch takes, or whether it takes one of the others, depends on its number of blocks (fwd_form,
 // dq_form, dkdv_form): the same call gives the same bits every time, but a unit in a batch need not give those it gives alone.
 //
-// The same kernels, with wavefronts that own different rows and share the tiles (QW = 4, KW = 1), are the path of every
-// head size that is a multiple of 8 up to 128 but not 64 or 128 (D is the size rounded up to 32; chunks past the real
+// The same kernels, with wavefronts that own different rows and share the tiles (QW = 4, KW = 1), are the path of most dQ and dK/dV
+// launches at head_dim 64 (dkdv_form_64) and of every head size that is a multiple of 8 up to 128 but not 64 or 128 (D is the size rounded up to 32; chunks past the real
 // size read as zero and are not stored). Rows that are not aligned run in fp32 arithmetic there (attn_generic.hip), and these
 // are no less exact (EXACT; head_dim 64 and 128 round P and dS to one bf16 operand): P and dS enter their products as several
 // operands, the rounded value and the remainders.
@@ -34,6 +34,13 @@ constexpr int FWD_PARTS = 2, BWD_PARTS = 3;
 // operands and the fp32 sums hold as they hold 1.
 constexpr float LAZY_T = 6.0f;
 
+// Where a row of a tile that serves row reads and transposing reads sits in LDS: at 64 columns in the order that keeps both free
+// of bank conflicts (lds_row, mfma_common.h).
+template <int D>
+__device__ constexpr int tile_row(int r) {
+    return lds_row<D == 64 ? 64 : 128>(r);
+}
+
 // A tile of ROWS rows of a [T, dk] bf16 matrix, moved by G threads: thread t of the group carries the 16-byte chunks
 // t, t + G, ... Rows past T and chunks past dk read as zero.
 template <int D, int G, int ROWS>
@@ -54,11 +61,13 @@ struct Mover {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) r[i] = tile_load16(rs, off[i]);
     }
+    // ORDERED: rows in the order of tile_row
+    template <bool ORDERED>
     __device__ void store(uint16_t* lds, int pitch, int t) const {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
-            const int c = t + G * i;
-            *reinterpret_cast<u32x4*>(lds + (c / NCH) * pitch + (c % NCH) * 8) = r[i];
+            const int c = t + G * i, row = c / NCH;
+            *reinterpret_cast<u32x4*>(lds + (ORDERED ? tile_row<D>(row) : row) * pitch + (c % NCH) * 8) = r[i];
         }
     }
 };
@@ -113,9 +122,14 @@ __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
     return sum;
 }
 
+// Whether dP starts from -delta instead of zero, a subtraction an element less: not where its rounding, one more product at the
+// size of delta, would count (EXACT), nor at 128 columns, where it spilled 30 registers more.
+template <int D, bool EXACT>
+constexpr bool FROM_DELTA = !EXACT && D == 64;
+
 // acc[db] += M^T c for the 32 rows of an LDS tile that start at row0, M the tile (columns 32 db ..), c a C tile whose rows
 // are the tile's rows, as PARTS operands
-template <int D, int PARTS>
+template <int D, int PARTS, bool ORDERED>
 __device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, const f32x16& c, f32x16* acc, int lane) {
     constexpr int DB = D / 32;
     const auto half = [&](auto hc) {
@@ -130,7 +144,8 @@ __device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, 
         bf16x8 m[DB];
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            m[db] = lds_read_tr_operand(tile, pitch, row0 + 16 * H, db * 32, lane);
+            m[db] = ORDERED && D == 64 ? lds_read_tr_operand_perm<64>(tile, pitch, row0 + 16 * H, db, lane)
+                                       : lds_read_tr_operand(tile, pitch, row0 + 16 * H, db * 32, lane);
             acc[db] = mfma32(m[db], part[0], acc[db]);
         }
 #pragma unroll
@@ -183,8 +198,8 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     };
     auto commit = [&](int buf) {
         uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
-        mk.store(t, KS, gt);
-        mv.store(t + BN * KS, VS, gt);
+        mk.template store<false>(t, KS, gt);
+        mv.template store<false>(t + BN * KS, VS, gt);
     };
     fetch(0);
     bf16x8 qreg[KK];
@@ -196,6 +211,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
         for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
     float m = -1e30f, l = 0.0f;  // the reference's running-max seed, src/ops.cpp:881
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    const KeyRange range(a, qlo);
     commit(0);
     tile_barrier<QW>();
 
@@ -209,8 +225,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
         bool live[NB], any = false;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {  // wavefront-uniform: is anything of this 32 x 32 block visible?
-            const int k0 = n0 + nb * 32;
-            live[nb] = k0 < a.T && qlo < a.T && !(a.causal && k0 > qhi) && !(a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks);
+            live[nb] = range.live(n0 + nb * 32);
             any = any || live[nb];
         }
         if (any) {
@@ -241,8 +256,8 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
             for (int nb = 0; nb < NB; ++nb) {
                 if (!live[nb]) continue;
                 const int k0 = n0 + nb * 32;
-                const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
-                if (kind != MaskKind::NONE) mask_block(s[nb], kind, vis, k0 + g * 4, -INFINITY);
+                if (!range.full(k0))
+                    mask_block(s[nb], mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks), vis, k0 + g * 4, -INFINITY);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[nb][r]);
             }
@@ -267,7 +282,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
                     ps[r & 3] += s[nb][r];
                 }
                 l += (ps[0] + ps[1]) + (ps[2] + ps[3]);  // per-lane partial; the two halves meet below
-                accumulate_tr<D, EXACT ? FWD_PARTS : 1>(Vs, VS, nb * 32, s[nb], acc, lane);
+                accumulate_tr<D, EXACT ? FWD_PARTS : 1, false>(Vs, VS, nb * 32, s[nb], acc, lane);
             }
         }
         if (i + 1 < iters) commit(i + 1);  // two buffers: last read one iteration ago, before the previous barrier
@@ -316,6 +331,7 @@ template <int D, int QW, int KW, int NB, bool EXACT>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint16_t* lds) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
+    constexpr bool MINUS_DELTA = FROM_DELTA<D, EXACT> && (QW > 1 || KW == 8);  // not with four: T 1661, 16 heads 21.5 us | 24.5
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
@@ -342,8 +358,8 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint1
     };
     auto commit = [&](int buf) {
         uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
-        mk.store(t, S, gt);
-        mv.store(t + BN * S, S, gt);
+        mk.template store<true>(t, S, gt);
+        mv.template store<true>(t + BN * S, S, gt);
     };
     fetch(0);
     bf16x8 qreg[KK], greg[KK];
@@ -364,6 +380,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint1
         dl = a.delta[lrow];
     }
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
+    const KeyRange range(a, qlo);
     f32x16 acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -381,22 +398,19 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint1
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const int k0 = n0 + nb * 32;
-            // wavefront-uniform: nothing of this 32 x 32 block is visible
-            if (k0 >= a.T || qlo >= a.T || (a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks))
-                continue;
+            if (!range.live(k0)) continue;
             f32x16 s, dp;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.0f;
+            for (int r = 0; r < 16; ++r) s[r] = 0.0f, dp[r] = MINUS_DELTA ? -dl : 0.0f;
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
-                s = mfma32(lds_read8(Ks + (nb * 32 + c32) * S + kk * 16 + g * 8), qreg[kk], s);
-                dp = mfma32(lds_read8(Vs + (nb * 32 + c32) * S + kk * 16 + g * 8), greg[kk], dp);
+                s = mfma32(lds_read8(Ks + (nb * 32 + tile_row<D>(c32)) * S + kk * 16 + g * 8), qreg[kk], s);
+                dp = mfma32(lds_read8(Vs + (nb * 32 + tile_row<D>(c32)) * S + kk * 16 + g * 8), greg[kk], dp);
             }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) dp[r] = weight_of<EXACT>(s[r], a.scale, cexp, nlse) * (dp[r] - dl);
-            const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
-            if (kind != MaskKind::NONE) mask_block(dp, kind, vis, k0 + g * 4, 0.0f);
-            accumulate_tr<D, EXACT ? BWD_PARTS : 1>(Ks, S, nb * 32, dp, acc, lane);
+            for (int r = 0; r < 16; ++r) dp[r] = weight_of<EXACT>(s[r], a.scale, cexp, nlse) * (MINUS_DELTA ? dp[r] : dp[r] - dl);
+            if (!range.full(k0)) mask_block(dp, mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks), vis, k0 + g * 4, 0.0f);
+            accumulate_tr<D, EXACT ? BWD_PARTS : 1, true>(Ks, S, nb * 32, dp, acc, lane);
         }
         if (i + 1 < iters) commit(i + 1);
         tile_barrier<QW>();
@@ -491,16 +505,16 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
     };
     auto commit = [&](int buf) {
         uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
-        mq.store(t, S, gt);
-        mg.store(t + BMQ * S, S, gt);
-        float out = gt >= BMQ ? row_r : EXACT ? -row_r : -row_r * LOG2E;
+        mq.template store<true>(t, S, gt);
+        mg.template store<true>(t + BMQ * S, S, gt);
+        float out = gt >= BMQ ? (FROM_DELTA<D, EXACT> ? -row_r : row_r) : EXACT ? -row_r : -row_r * LOG2E;
         if constexpr (OWN_DELTA) {
             tile_barrier<1>();
             float part = 0.0f;
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) part = add_products(oreg[kk], lds_read8(t + BMQ * S + c32 * S + kk * 16 + g * 8), part);
+            for (int kk = 0; kk < KK; ++kk) part = add_products(oreg[kk], lds_read8(t + BMQ * S + tile_row<D>(c32) * S + kk * 16 + g * 8), part);
             part = xhalf_sum(part);
-            if (g == 1) out = part;
+            if (g == 1) out = FROM_DELTA<D, EXACT> ? -part : part;
         }
         if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = out;
     };
@@ -514,6 +528,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[n][r] = 0.0f;
     const KeyVis kvis(kj, a.T, a.causal, a.window, a.sinks);
+    const QueryRange range(a, kw0);
     commit(0);
     tile_barrier<QW>();
 
@@ -524,19 +539,22 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
         const float* rows = reinterpret_cast<const float*>(Qs + 2 * BMQ * S);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            const int qlo = (qt_lo + c_t) * BMQ + nb * 32, qhi = qlo + 31;
-            // wavefront-uniform: nothing of this 32 x 32 block is visible
-            if (i * KW + kg >= steps || qlo >= a.T || kw0 >= a.T || (a.causal && kw0 > qhi) ||
-                (a.window > 0 && kw0 + 31 + a.window <= qlo && kw0 >= a.sinks))
-                continue;
+            const int qlo = (qt_lo + c_t) * BMQ + nb * 32;
+            if ((KW > 1 && i * KW + kg >= steps) || !range.live(qlo)) continue;
             f32x16 s, dp;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.0f;
+            for (int r = 0; r < 16; ++r) s[r] = 0.0f;
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                s = mfma32(lds_read8(Qs + (nb * 32 + c32) * S + kk * 16 + g * 8), kreg[kk], s);
-                dp = mfma32(lds_read8(Gs + (nb * 32 + c32) * S + kk * 16 + g * 8), vreg[kk], dp);
+            for (int qd = 0; qd < 4; ++qd) {
+                f32x4 dl = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (FROM_DELTA<D, EXACT>) dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = dl[e];
             }
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) s = mfma32(lds_read8(Qs + (nb * 32 + tile_row<D>(c32)) * S + kk * 16 + g * 8), kreg[kk], s);
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) dp = mfma32(lds_read8(Gs + (nb * 32 + tile_row<D>(c32)) * S + kk * 16 + g * 8), vreg[kk], dp);
             // lane = key kj; element r = query qlo + (r/4)*8 + 4g + r%4
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
@@ -544,20 +562,19 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s[qd * 4 + e] = weight_of<EXACT>(s[qd * 4 + e], a.scale, cexp, nl[e]);
             }
-            const bool full = qhi < a.T && kw0 + 31 < a.T && (!a.causal || kw0 + 31 <= qlo) &&
-                              (a.window == 0 || kw0 + a.window > qhi || kw0 + 31 < a.sinks);
-            if (!full) {
+            if (!range.full(qlo)) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] = kvis(qlo + (r >> 2) * 8 + g * 4 + (r & 3)) ? s[r] : 0.0f;
             }
-            accumulate_tr<D, EXACT ? BWD_PARTS : 1>(Gs, S, nb * 32, s, acc, lane);
+            accumulate_tr<D, EXACT ? BWD_PARTS : 1, true>(Gs, S, nb * 32, s, acc, lane);
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
-                const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
+                f32x4 dl = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (!FROM_DELTA<D, EXACT>) dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (dp[qd * 4 + e] - dl[e]);
+                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (FROM_DELTA<D, EXACT> ? dp[qd * 4 + e] : dp[qd * 4 + e] - dl[e]);
             }
-            accumulate_tr<D, EXACT ? BWD_PARTS : 1>(Qs, S, nb * 32, dp, acc + DB, lane);
+            accumulate_tr<D, EXACT ? BWD_PARTS : 1, true>(Qs, S, nb * 32, dp, acc + DB, lane);
         }
         c_t += KW;
         while (c_t >= nqt) c_t -= nqt;
@@ -613,9 +630,50 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, in
         dq_block<D, 1, 4, 1, EXACT>(a, 1, id - dkdv_ids, lds);
 }
 
-// How a launch shares its work out: four wavefronts with 32 rows each (WIDE), or one block of 32 rows whose tiles are
-// split between four or eight wavefronts.
-enum class Form { NONE, WIDE, FOUR, EIGHT };
+// How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of
+// 32 rows whose tiles are split between four or eight wavefronts.
+enum class Form { NONE, WIDE, SHORT, HALF, FOUR, EIGHT };
+
+// head_dim 64, launches that fill the chip: rows owned by wavefronts, against the kernels of the other files. A wavefront that holds
+// K and V of its 32 keys needs no P from another, no ring and one barrier a tile, and at 64 columns two of its workgroups fit
+// a CU where one of the others does (bf16, forward + backward kernels of head_dim 64, us, other | WIDE | HALF):
+//   dK/dV    causal T 512 x 16, 8 heads 25.4 | 21.5 | 22.9;  T 1024 x 8, 8 heads 34 | 31 | 32;  T 2048 x 4, 14 heads on 2 110 | 89 | 89;
+//            T 4096 x 4, 16 heads 327 | 281 | 302;  T 4016, 16 heads 83 | 98 | 100;  T 2378 x 3, 4 heads 34 | 56 | 56
+//            no mask T 777 x 6, 12 heads 49 | 36 | 38;  T 1749, 16 heads 67 | 53 | 66;  T 195 x 57, 2 heads 11.2 | 11.8 | 13.5
+//            window 69, 16 sinks, T 1889, 16 heads 30 | 24 | 24;  window 256, 4 sinks, T 4096 x 4, 16 heads 127 | 120 | 124
+//   dQ       causal T 2048 x 4, 14 heads 64 | 59 | 63;  T 4096 x 4, 16 heads 223 | 212 | 243;  T 3190 x 2, 8 heads 75 | 65 | 66
+//            no mask T 777 x 6, 12 heads 29.8 | 28.1 | 29.7;  window 43, T 1976, few heads (bands of 300 to 1700 blocks) 1.1 times with HALF
+//   forward  window 256, T 4096 x 4, 16 heads 59 | 58 | 65, SHORT 45;  window 128, T 700 x 8, 16 heads 20.5 | 20.1 | 18.1, SHORT 15.8;
+//            without a band the forward of attn_fwd_mfma.hip is ahead
+// Long causal chains of few units stay with 64 keys a wavefront (mfma_dkdv3).
+bool narrow_band(const AttnArgs& a) { return a.window > 0 && a.window <= 512 && chain_tokens(a) < a.T; }
+Form fwd_form_64(const AttnArgs& a) {
+    const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
+    if (!narrow_band(a) || 2 * a.window > a.T) return Form::NONE;
+    return blocks >= 1700 ? Form::SHORT : blocks >= 300 ? Form::HALF : Form::NONE;
+}
+Form dq_form_64(const AttnArgs& a) {
+    const int64_t units = static_cast<int64_t>(a.Hq) * a.B, n = (a.T + 127) / 128;
+    if (chain_tokens(a) < a.T) {
+        const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * units;
+        return narrow_band(a) && a.T >= 256 && blocks >= 300 && blocks < 1700 ? Form::HALF : Form::NONE;
+    }
+    // (without a mask 64 queries a wavefront, mfma_dq3, are ahead from 4096 tokens on: T 5856 x 2, 16 heads 394 | 422)
+    if (!a.causal) return a.T >= 100 && a.T < 4096 && units * n >= (a.T < 1000 ? 200 : 330) ? Form::WIDE : Form::NONE;
+    return a.T >= 256 && units * (n + 1) >= 400 ? Form::WIDE : Form::NONE;
+}
+// splits: how many workgroups share the heads of a group
+Form dkdv_form_64(const AttnArgs& a, int splits) {
+    const int64_t units = static_cast<int64_t>(a.Hkv) * a.B * splits, n = (a.T + 127) / 128;
+    if (a.T <= 64 || (splits > 1 && a.T < 400)) return Form::NONE;
+    if (chain_tokens(a) < a.T) {
+        if (a.sinks > 0) return a.window <= 256 && units * n >= 300 ? Form::HALF : Form::NONE;
+        return 3 * a.window <= 2 * a.T && units * n >= 230 ? Form::HALF : Form::NONE;
+    }
+    if (!a.causal) return a.T > 250 ? (units * n >= 160 ? Form::WIDE : Form::NONE) : units * n >= 440 ? Form::HALF : Form::NONE;
+    if (units * (n + 1) < (a.T >= 2000 ? 560 : 500)) return Form::NONE;  // the longest chains against all there is to do
+    return a.T >= 400 ? Form::WIDE : Form::HALF;
+}
 
 // Which form, from the number of 32-row blocks of the launch (`blocks`) and the length of a block's chain. A block split between
 // eight wavefronts has the shortest chain but fills half a CU or more, so it wins while the blocks come to about one
@@ -653,6 +711,8 @@ bool unsplit_is_ahead(const AttnArgs& a, int64_t blocks) {
 // 2, 8 heads 91 | 105; head_dim 96, T 1886 x 3, 8 heads 45 | 53, T 4618, 16 heads 148 | 128).
 bool wide_chains(const AttnArgs& a, int64_t blocks) { return a.dk_dim > 32 && even_chains(a) && chain_tokens(a) <= 160 && blocks > 550; }
 Form fwd_form(const AttnArgs& a) {
+    if (a.dk_dim == 64)
+        if (const Form f = fwd_form_64(a); f != Form::NONE) return f;
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     if (unsplit_is_ahead(a, blocks) || (plain && a.T <= 64)) return Form::NONE;
@@ -672,6 +732,8 @@ Form fwd_form(const AttnArgs& a) {
     return blocks <= 1100 && chain_tokens(a) >= 3000 ? Form::EIGHT : Form::NONE;
 }
 Form dq_form(const AttnArgs& a) {
+    if (a.dk_dim == 64)
+        if (const Form f = dq_form_64(a); f != Form::NONE) return f;
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hq * a.B;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     // (causal, T 80, 77 heads of 128: four wavefronts 10.8 us, unsplit 10.1; T 100 11.0 and 11.6)
@@ -697,7 +759,7 @@ bool short_chains(const AttnArgs& a, int64_t blocks) {
     if (blocks <= 256) return a.T <= (a.window > 0 ? 250 : 180);
     return blocks > std::min(512, 256 + std::max(chain - 350, 0) * 2 / 5);
 }
-Form dkdv_form(const AttnArgs& a) {
+Form dkdv_small_form(const AttnArgs& a) {
     const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.Hkv * a.B * a.head_split;
     const bool plain = a.dk_dim == 64 || a.dk_dim == 128;
     if (unsplit_is_ahead(a, blocks) || (plain && a.head_split == 1 && (a.T <= 72 || (a.Hq == a.Hkv && short_chains(a, blocks)))))
@@ -717,6 +779,15 @@ Form dkdv_form(const AttnArgs& a) {
     const Form later = a.dk_dim == 64 && blocks > 256 && !(blocks <= 450 && chain_tokens(a) >= 2000 && !even_chains(a)) ? Form::FOUR : best;
     if (blocks <= 600) return later;
     return blocks <= 1100 && a.dk_dim == 64 && chain_tokens(a) >= 2000 ? later : Form::NONE;
+}
+
+// The query heads of a group are dealt out where the kernels below this file's lines, or mfma_dkdv3, would be: the workspace is
+// sized for that.
+int splits_of(const AttnArgs& a) { return bf16_deals_heads(a) ? a.head_split : 1; }
+Form dkdv_form(const AttnArgs& a) {
+    if (a.dk_dim == 64)
+        if (const Form f = dkdv_form_64(a, splits_of(a)); f != Form::NONE) return f;
+    return dkdv_small_form(a);
 }
 
 template <int D, int QW, int KW, int NB, bool EXACT>
@@ -749,6 +820,10 @@ int fwd_of(const AttnArgs& a, Form f, hipStream_t st) {
     if (f == Form::FOUR) run_fwd<D, 1, 4, 1, EXACT>(a, st);
     if constexpr (EXACT)
         if (f == Form::WIDE) run_fwd<D, 4, 1, 2, EXACT>(a, st);
+    if constexpr (!EXACT && D == 64) {
+        if (f == Form::SHORT) run_fwd<D, 4, 1, 1, EXACT>(a, st);
+        if (f == Form::HALF) run_fwd<D, 2, 1, 2, EXACT>(a, st);
+    }
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -757,8 +832,10 @@ int dq_of(const AttnArgs& a, Form f, bool fuse_delta, hipStream_t st) {
     if constexpr (D <= 96)
         if (f == Form::EIGHT) run_dq<D, 1, 8, 1, EXACT>(a, fuse_delta, st);
     if (f == Form::FOUR) run_dq<D, 1, 4, 1, EXACT>(a, fuse_delta, st);
-    if constexpr (EXACT)
+    if constexpr (EXACT || D == 64)
         if (f == Form::WIDE) run_dq<D, 4, 1, 2, EXACT>(a, fuse_delta, st);
+    if constexpr (!EXACT && D == 64)
+        if (f == Form::HALF) run_dq<D, 2, 1, 2, EXACT>(a, fuse_delta, st);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -767,8 +844,10 @@ int dkdv_of(const AttnArgs& a, Form f, hipStream_t st) {
     if constexpr (D <= 64)
         if (f == Form::EIGHT) run_dkdv<D, 1, 8, 1, EXACT>(a, st);
     if (f == Form::FOUR) run_dkdv<D, 1, 4, 1, EXACT>(a, st);
-    if constexpr (EXACT)
+    if constexpr (EXACT || D == 64)
         if (f == Form::WIDE) run_dkdv<D, 4, 1, 2, EXACT>(a, st);
+    if constexpr (!EXACT && D == 64)
+        if (f == Form::HALF) run_dkdv<D, 2, 1, 2, EXACT>(a, st);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -796,6 +875,7 @@ bool split_serves(const AttnArgs& a) { return a.dk_dim % 8 == 0 && a.dk_dim <= 1
 bool split_takes_fwd(const AttnArgs& a) { return fwd_form(a) != Form::NONE; }
 bool split_takes_dq(const AttnArgs& a) { return dq_form(a) != Form::NONE; }
 bool split_takes_dkdv(const AttnArgs& a) { return dkdv_form(a) != Form::NONE; }
+bool split_deals_heads(const AttnArgs& a) { return a.head_split > 1 && dkdv_small_form(a) != Form::NONE; }
 int launch_split_fwd(const AttnArgs& a, hipStream_t st) {
 #define PK_CALL(D, E) fwd_of<D, E>(a, fwd_form(a), st)
     PK_SPLIT_DISPATCH(PK_CALL);
@@ -808,9 +888,11 @@ int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 }
 int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
-    if (!split_tail_pays(a, a.head_split, dkdv_form(a) == Form::WIDE ? 128 : 32)) a.tail = nullptr;
+    const Form f = dkdv_form(a);
+    a.head_split = splits_of(a);
+    if (!split_tail_pays(a, a.head_split, f == Form::WIDE ? 128 : f == Form::HALF ? 64 : 32)) a.tail = nullptr;
     const auto run = [&]() -> int {
-#define PK_CALL(D, E) dkdv_of<D, E>(a, dkdv_form(a), st)
+#define PK_CALL(D, E) dkdv_of<D, E>(a, f, st)
         PK_SPLIT_DISPATCH(PK_CALL);
 #undef PK_CALL
     };
@@ -825,9 +907,10 @@ int launch_split_dkdv(const AttnArgs& a_in, hipStream_t st) {
 bool split_takes_bwd(const AttnArgs& a) {
     const OneLaunch l(a);
     const int ids = l.dkdv_ids + l.dq_ids;
-    if (chain_tokens(a) > 2600) return false;
+    // bands of more than a thousand keys, T 3201, window 1268, 4 heads on 1: 57 | 71
+    if (chain_tokens(a) > (chain_tokens(a) < a.T ? 1024 : 2600)) return false;
     if (a.dk_dim <= 32) return ids <= (even_chains(a) ? 400 : 960);
-    if (a.dk_dim <= 64) return ids <= (a.T <= 32 ? 400 : even_chains(a) ? 640 : 800);  // (one tile: T 31 x 84, 4 heads of 64 10.9 | 13.3)
+    if (a.dk_dim <= 64) return ids <= (a.T <= 64 ? 400 : even_chains(a) ? 640 : 800);  // (one tile: T 31 x 84, 4 heads of 64 10.9 | 13.3)
     if (a.dk_dim <= 96) return ids <= (even_chains(a) ? 380 : 400);
     return ids <= 256 && (a.dk_dim < 128 || a.T > 32);
 }

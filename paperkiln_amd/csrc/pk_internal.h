@@ -168,12 +168,13 @@ int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
 bool f32_deals_heads(const AttnArgs& a);  // its dK/dV kernel for this launch uses a.head_split and a.part
 
 // attn_split.hip: bf16 kernels whose wavefronts split the contraction. They serve every head size that is a multiple of
-// 8 up to 128; at 64 and 128 `split_takes_*` says whether a launch is small enough for them to be ahead of the kernels
-// below, at the other sizes they take everything.
+// 8 up to 128; at 64 and 128 `split_takes_*` says whether a launch is one they are ahead in of the kernels below (small ones, and at 64
+// most dK/dV and dQ), at the other sizes they take everything.
 bool split_serves(const AttnArgs& a);
 bool split_takes_fwd(const AttnArgs& a);
 bool split_takes_dq(const AttnArgs& a);
 bool split_takes_dkdv(const AttnArgs& a);
+bool split_deals_heads(const AttnArgs& a);  // its small launches share the heads of a group between workgroups
 int launch_split_fwd(const AttnArgs& a, hipStream_t st);
 int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_split_dkdv(const AttnArgs& a, hipStream_t st);

@@ -227,6 +227,17 @@ def test_backward_in_one_launch(case, dtype, dk):
     assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
 
 
+# bf16 at head_dim 64 in launches that fill the chip: rows owned by wavefronts, two or four to a workgroup, tiles of 32 and 64; lengths
+# around the tiles and blocks, the shortest that come here, bands with and without sinks (dealt out and left whole), dealt heads, no mask.
+@pytest.mark.parametrize("case", [(16, 512, 8, 8, True, 0, 0), (64, 65, 8, 8, True, 0, 0), (20, 399, 8, 8, True, 0, 0), (2, 2049, 14, 2, True, 0, 0),
+                                  (6, 777, 12, 12, False, 0, 0), (40, 129, 8, 4, False, 0, 0), (3, 1889, 16, 16, True, 69, 16),
+                                  (2, 2500, 16, 16, True, 200, 0), (8, 700, 16, 8, True, 128, 0), (4, 300, 16, 16, True, 33, 3),
+                                  (1, 1100, 32, 32, True, 0, 0)], ids=str)
+def test_rows_owned_by_wavefronts_at_head_dim_64(case):
+    e = errors(*run_attention(*case[:4], 64, torch.bfloat16, *case[4:]))
+    assert max(e) < 1e-2, e
+
+
 # Either side of the lines between the two geometries of the 32-key dK/dV kernel: one round of the chip and one head more, two
 # nearly whole rounds, and with a band and sink keys whose queries are dealt out or left whole.
 @pytest.mark.parametrize("case,dk", [((32, 200, 8, 8, True, 0, 0), 64), ((33, 200, 4, 4, True, 0, 0), 64), ((16, 200, 8, 8, True, 0, 0), 64),
