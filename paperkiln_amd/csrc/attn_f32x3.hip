@@ -183,18 +183,26 @@ __device__ inline f32x16 dot3(const uint16_t* tile, const bf16x8 (&b)[3][D / 16]
     return t;
 }
 
+// a C tile, its rows 0 .. 15 and 16 .. 31, as operands
+struct Parts {
+    bf16x8 h[2], m[2], l[2];
+    __device__ inline explicit Parts(const f32x16& c) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const float x[8] = {c[8 * half], c[8 * half + 1], c[8 * half + 2], c[8 * half + 3],
+                                c[8 * half + 4], c[8 * half + 5], c[8 * half + 6], c[8 * half + 7]};
+            split8(x, h[half], m[half], l[half]);
+        }
+    }
+    __device__ inline Parts() {}
+};
+
 // acc[n] += tile^T c for blocks db0 + n of the columns, c a C tile whose rows are the tile's rows. The tile's product is formed by
 // itself, small products first, and added once: on the accumulator each of the twelve would be rounded at its size.
 template <int D, int NB = D / 32>
-__device__ inline void accumulate3(const uint16_t* tile, const f32x16& c, f32x16* acc, int lane, int db0 = 0) {
+__device__ inline void accumulate3(const uint16_t* tile, const Parts& c, f32x16* acc, int lane, int db0 = 0) {
     constexpr int PLANE = 32 * (D + 8);
-    bf16x8 ch[2], cm[2], cl[2];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const float x[8] = {c[8 * half], c[8 * half + 1], c[8 * half + 2], c[8 * half + 3],
-                            c[8 * half + 4], c[8 * half + 5], c[8 * half + 6], c[8 * half + 7]};
-        split8(x, ch[half], cm[half], cl[half]);
-    }
+    const auto &ch = c.h, &cm = c.m, &cl = c.l;
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
         const int db = min(db0 + n, D / 32 - 1);
@@ -309,7 +317,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
                 ps[r & 3] += s[r];
             }
             lsum += static_cast<double>((ps[0] + ps[1]) + (ps[2] + ps[3]));  // per-lane partial; the two halves meet below
-            accumulate3<D>(Ks + 3 * PLANE, s, acc, lane);
+            accumulate3<D>(Ks + 3 * PLANE, Parts(s), acc, lane);
         }
         if (NBUF == 1) __syncthreads();
         if (i + 1 < iters) commit(i + 1);  // two buffers: last read one iteration ago, before the previous barrier
@@ -421,7 +429,7 @@ __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs 
             for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * (dp[r] - dl);
             const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
             if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, 0.0f);
-            accumulate3<D>(Ks, s, acc, lane);
+            accumulate3<D>(Ks, Parts(s), acc, lane);
         }
         if (NBUF == 1) __syncthreads();
         if (i + 1 < iters) commit(i + 1);
@@ -456,11 +464,15 @@ __device__ inline f32x16 get_tile(const float* buf, int lane) {
 }
 
 // ---- dK, dV: QW groups of 32 keys, the query tiles of every query head of the group in turn ----
-// A step is two phases. First: role 0 S = Q K^T and P, role 1 dP = dO V^T, each half of the next tile's way into LDS. Then, P handed
-// over: role 0 dV^T += dO^T P, role 1 dS = P (dP - delta) and dK^T += Q^T dS.
+// A step is two phases. First: role 0 S = Q K^T and P, role 1 dP = dO V^T. Then, P handed over: role 0 dV^T += dO^T P, role 1 dS =
+// P (dP - delta) and dK^T += Q^T dS. Each moves half of the next tile into LDS, role 1 ahead of its first product and role 0
+// behind its second, so that one splits while the other multiplies: in a SIMD a matrix instruction leaves room for four others, and
+// the loop has six of them for each (T 4096 x 2, 16 heads, head_dim 96, us: 1005 -> 968; head_dim 64, window 256, 4 KV heads, T
+// 4096 x 4: 337 -> 323). At 128 columns there is one wavefront to a SIMD and both do it at the end of the first phase (1777; 1872).
 template <int D, int QW>
 __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
     constexpr int BNK = 32 * QW, DB = D / 32, G = 64 * QW;
+    constexpr bool APART = D < 128;
     constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE + 128;  // LSE and delta of a tile's rows behind it
     __shared__ __attribute__((aligned(16))) uint16_t lds[2 * TILE];
     __shared__ __attribute__((aligned(16))) float pbuf[QW * 1024];
@@ -539,7 +551,16 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
             if (++c_t == nqt) c_t = 0;
             // wavefront-uniform, the same for both roles: is anything of this 32 x 32 block visible?
             const bool live = qlo < a.T && kw0 < a.T && !(a.causal && kw0 > qhi) && !(a.window > 0 && kw0 + 31 + a.window <= qlo && kw0 >= a.sinks);
+            // the other buffer was last read one step ago, before the previous barrier
+            const auto stage = [&]() {
+                if (i + 1 < steps) {
+                    commit(i + 1);
+                    if (i + 2 < steps) fetch();
+                }
+            };
+            if (ROLE == 1 && APART) stage();
             f32x16 t;
+            Parts parts;
             if (live) t = dot3<D>(ROLE == 0 ? Qs : Gs, res, c32, g);
             if (ROLE == 0 && live) {
                 // lane = key kj; element r = query qlo + (r/4)*8 + 4g + r%4
@@ -556,11 +577,9 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
                     for (int r = 0; r < 16; ++r) t[r] = kvis(qlo + (r >> 2) * 8 + g * 4 + (r & 3)) ? t[r] : 0.0f;
                 }
                 put_tile(pb, t, lane);
+                if (APART) parts = Parts(t);
             }
-            if (i + 1 < steps) {  // the other buffer was last read one step ago, before the previous barrier
-                commit(i + 1);
-                if (i + 2 < steps) fetch();
-            }
+            if (!APART) stage();
             __syncthreads();
             if (ROLE == 1 && live) {
                 const f32x16 p = get_tile(pb, lane);
@@ -571,7 +590,9 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
                     for (int e = 0; e < 4; ++e) t[qd * 4 + e] = p[qd * 4 + e] * (t[qd * 4 + e] - dl[e]);
                 }
             }
-            if (live) accumulate3<D>(ROLE == 0 ? Gs : Qs, t, acc, lane);
+            if (live && (ROLE == 1 || !APART)) parts = Parts(t);
+            if (live) accumulate3<D>(ROLE == 0 ? Gs : Qs, parts, acc, lane);
+            if (ROLE == 0 && APART) stage();
             __syncthreads();
         }
     };
@@ -598,8 +619,8 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
 }
 
 // ---- dQ above 64 columns: the same two phases ----
-// First: role 0 S = K Q^T and P, role 1 dP - delta, each half of the next tile's way into LDS; both tiles are handed over, and each role
-// forms dS for itself and takes half the columns of dQ^T += K^T dS.
+// First: role 0 S = K Q^T and P, role 1 dP - delta; both tiles are handed over, and each role forms dS for itself and takes half the
+// columns of dQ^T += K^T dS. The next tile is moved as in x3_dkdv (T 4403, 8 heads, head_dim 128, us: 456 -> 436).
 template <int D>
 __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta) {
     constexpr int QW = 4, BM = 32 * QW, DB = D / 32, G = 64 * QW, HB = (DB + 1) / 2;
@@ -656,6 +677,13 @@ __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta)
             const uint16_t* Ks = lds + (i & 1) * TILE;
             const int k0 = kt.tile(i) * 32;
             const bool live = k0 < a.T && qlo < a.T && !(a.causal && k0 > qhi) && !(a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks);
+            const auto stage = [&]() {
+                if (i + 1 < kt.n) {
+                    commit(i + 1);
+                    if (i + 2 < kt.n) fetch(i + 2);
+                }
+            };
+            if (ROLE == 1) stage();
             f32x16 t;
             if (live) {
                 t = dot3<D>(ROLE == 0 ? Ks : Ks + 3 * PLANE, res, c32, g);
@@ -665,17 +693,14 @@ __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta)
                 if (kind != MaskKind::NONE) mask_block(t, kind, vis, k0 + g * 4, 0.0f);
                 put_tile(cbuf[ROLE] + qg * 1024, t, lane);
             }
-            if (i + 1 < kt.n) {
-                commit(i + 1);
-                if (i + 2 < kt.n) fetch(i + 2);
-            }
             __syncthreads();
             if (live) {
                 const f32x16 o = get_tile(cbuf[1 - ROLE] + qg * 1024, lane);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) t[r] *= o[r];
-                accumulate3<D, HB>(Ks, t, acc, lane, ROLE * HB);
+                accumulate3<D, HB>(Ks, Parts(t), acc, lane, ROLE * HB);
             }
+            if (ROLE == 0) stage();
             __syncthreads();
         }
     };
