@@ -7,8 +7,8 @@
 // product is latency, and that a projection of a few hundred tokens has 16 to 200 blocks of 32 x 32 for 1024 SIMDs: the
 // wavefronts of a workgroup split the contraction and add their accumulators through LDS at the end, in a fixed order.
 //
-// Against the library, which serves the larger products (GPU time, 512 tokens of width 128): 3.8 us and 3.9 for the
-// fused q/k/v projection, 5.2 and 6.0 for the down projection; but a launch here costs the host 3 us, not 10 to 25, sums
+// Against the library, which serves the larger products (GPU time, 512 tokens of width 128): level for the fused
+// q/k/v projection, 4.0 us and 6.0 for the down projection; but a launch here costs the host 3 us, not 10 to 25, sums
 // an addend on the way out, and takes all the weight gradients of a block together. 2048 tokens of width 512 against
 // 1536 columns: 45 us and 28.
 #include "mfma_common.h"
@@ -19,15 +19,20 @@
 namespace pk {
 namespace {
 
+struct Job {
+    const float* a;
+    const float* b;
+    float* c;
+    const float* addend;
+    int lda, ldb, ldc, M, N, K;
+};
+// One product's numbers are found at one place, several products' only once the workgroup knows whose tile it has: a second
+// round trip to the arguments, 0.4 to 0.8 us of the 3.5 to 8 that a small product takes.
+template <int MAX>
 struct Jobs {
-    static constexpr int MAX = 8;
     int count;
     int first[MAX + 1];  // job j's tiles are first[j] .. first[j + 1] - 1
-    const float* a[MAX];
-    const float* b[MAX];
-    float* c[MAX];
-    const float* addend[MAX];
-    int lda[MAX], ldb[MAX], ldc[MAX], M[MAX], N[MAX], K[MAX];
+    Job job[MAX];
 };
 
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // a row may start at any element
@@ -73,20 +78,21 @@ __host__ __device__ inline int64_t extent(int64_t rows, int64_t cols, int64_t ld
 __device__ inline int bytes_of(int rows, int cols, int64_t ld) { return static_cast<int>(extent(rows, cols, ld)); }
 
 // A workgroup's tile is MB x NB blocks of 16 x 16; its KW wavefronts split the contraction chunk by chunk.
-template <bool TA, bool TB, int MB, int NB, int KW>
-__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs jobs, const int tiles, const float beta) {
+template <bool TA, bool TB, int MB, int NB, int KW, int MAX>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta) {
     constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB, TN = 16 * NB;
     // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
     const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (t >= tiles) return;
     int j = 0;
-    while (t >= jobs.first[j + 1]) ++j;
-    const int M = jobs.M[j], N = jobs.N[j], K = jobs.K[j];
+    if constexpr (MAX > 1)
+        while (t >= jobs.first[j + 1]) ++j;
+    const int M = jobs.job[j].M, N = jobs.job[j].N, K = jobs.job[j].K;
     const int tn = (N + TN - 1) / TN, m0 = ((t - jobs.first[j]) / tn) * TM, n0 = ((t - jobs.first[j]) % tn) * TN;
     const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, grp = lane >> 4;
-    const float* const a = jobs.a[j];
-    const float* const b = jobs.b[j];
-    const int64_t lda = jobs.lda[j], ldb = jobs.ldb[j];
+    const float* const a = jobs.job[j].a;
+    const float* const b = jobs.job[j].b;
+    const int64_t lda = jobs.job[j].lda, ldb = jobs.job[j].ldb;
     int row[MB], col[NB];  // rows and columns past the edge read the last one; they are not stored
 #pragma unroll
     for (int i = 0; i < MB; ++i) row[i] = min(m0 + i * 16 + l16, M - 1);
@@ -111,11 +117,11 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs jobs, const 
     auto load = [&](int chunk, int buf) {
         const int over = max((chunk + 1) * KC - K, 0), k0 = chunk * KC - over;
         if (over == 0) {
-            load_chunk<TA, MB, KC>(ra, jobs.lda[j], oa, k0, fa[buf]);
-            load_chunk<!TB, NB, KC>(rb, jobs.ldb[j], ob, k0, fb[buf]);
+            load_chunk<TA, MB, KC>(ra, jobs.job[j].lda, oa, k0, fa[buf]);
+            load_chunk<!TB, NB, KC>(rb, jobs.job[j].ldb, ob, k0, fb[buf]);
         } else if (K >= KC) {  // the last chunk, moved back to end where the contraction does: its first steps are done already
-            load_chunk<TA, MB, KC>(ra, jobs.lda[j], oa, k0, fa[buf]);
-            load_chunk<!TB, NB, KC>(rb, jobs.ldb[j], ob, k0, fb[buf]);
+            load_chunk<TA, MB, KC>(ra, jobs.job[j].lda, oa, k0, fa[buf]);
+            load_chunk<!TB, NB, KC>(rb, jobs.job[j].ldb, ob, k0, fb[buf]);
 #pragma unroll
             for (int s = 0; s < KC / 4; ++s) {
                 const bool done = 4 * grp + 4 * (s & ~3) + (s & 3) < over;
@@ -156,9 +162,9 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs jobs, const 
     for (int u = 0; u < BUFS - 1; ++u)
         if (i + u < mine) multiply(u);
 
-    const float* const add = jobs.addend[j] ? jobs.addend[j] : beta != 0.0f ? jobs.c[j] : nullptr;
-    float* const out = jobs.c[j];
-    const int64_t ldc = jobs.ldc[j];
+    const float* const add = jobs.job[j].addend ? jobs.job[j].addend : beta != 0.0f ? jobs.job[j].c : nullptr;
+    float* const out = jobs.job[j].c;
+    const int64_t ldc = jobs.job[j].ldc;
     auto store = [&](int x, int y, f32x4 v) {
         const int n = n0 + y * 16 + l16;
         if (n >= N) return;
@@ -189,46 +195,53 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs jobs, const 
     }
 }
 
-template <bool TA, bool TB, int MB, int NB, int KW>
-void launch(Jobs& jobs, float beta, hipStream_t st) {
+template <bool TA, bool TB, int MB, int NB, int KW, int MAX>
+void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     constexpr int TM = 16 * MB, TN = 16 * NB;
     int tiles = 0;
     for (int j = 0; j < jobs.count; ++j) {
         jobs.first[j] = tiles;
-        tiles += ((jobs.M[j] + TM - 1) / TM) * ((jobs.N[j] + TN - 1) / TN);
+        tiles += ((jobs.job[j].M + TM - 1) / TM) * ((jobs.job[j].N + TN - 1) / TN);
     }
-    for (int j = jobs.count; j <= Jobs::MAX; ++j) jobs.first[j] = tiles;
-    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
+    for (int j = jobs.count; j <= MAX; ++j) jobs.first[j] = tiles;
+    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, MAX>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
                        tiles, beta);
     hip_check(hipGetLastError(), "gemm_f32");
 }
 
-// Which tile: a 32 x 32 one keeps more CUs busy, a 64 x 64 one reads its operands half as often. Measured on projections,
-// heads and weight gradients of 64 to 8192 tokens: with more than 640 of the small tiles (2.5 to a CU) the large one is
-// ahead (2048 x 1000 x 128: 10.4 us against 15.7), except for weight gradients, whose long contraction the small one walks
-// with more wavefronts (512 x 1536 x 8192: 117 us against 152). With a tile or less to a CU, eight wavefronts split the
-// contraction instead of four.
-template <bool TA, bool TB>
-void launch_by_size(Jobs& jobs, float beta, hipStream_t st) {
+// Which tile, by the number of 32 x 32 ones. A small tile keeps more CUs busy, a large one reads its operands less often. Measured
+// on projections, heads and weight gradients of 64 to 8192 tokens:
+//   More than 640 (2.5 to a CU): 64 x 64 (2048 x 1000 x 128: 10.4 us against 15.7), except for weight gradients, whose long
+//   contraction the small one walks with more wavefronts (512 x 1536 x 8192: 117 us against 152).
+//   Up to 64: 16 x 16, up to 128: 16 x 32, which makes a tile for each CU. A wavefront's loads and products for a chunk are a half or
+//   less (us, 32 x 32 with eight | 16 x 32 | 16 x 16 wavefronts: 512 x 128 x 688, B transposed 7.9 | 6.2 | 5.0; 512 x 128 x 344 5.4 |
+//   4.8 | 4.0; 512 x 256 x 688 7.8 | 6.0 | 6.6; 1024 x 128 x 688, B transposed 7.8 | 6.3 | 6.5).
+//   In between 32 x 32; eight wavefronts split the contraction where it is long and there is a tile or less to a CU. Short
+//   contractions of more tiles than that are over sooner as 16 x 32, for which the last round is half as long (1000 x 576 x
+//   192: 7.7 us against 9.4, 256 x 1376 x 256: 5.8 against 6.8; with B transposed, whose rows those tiles read twice, they are not).
+template <bool TA, bool TB, int MAX>
+void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     int64_t tiles = 0;
     int longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
-        tiles += static_cast<int64_t>((jobs.M[j] + 31) / 32) * ((jobs.N[j] + 31) / 32);
-        longest = std::max(longest, jobs.K[j]);
+        tiles += static_cast<int64_t>((jobs.job[j].M + 31) / 32) * ((jobs.job[j].N + 31) / 32);
+        longest = std::max(longest, jobs.job[j].K);
     }
     if (tiles > 640 && (!TA || longest < 256))
         launch<TA, TB, 4, 4, 4>(jobs, beta, st);
+    else if (tiles <= 64)
+        launch<TA, TB, 1, 1, 4>(jobs, beta, st);
+    else if (tiles <= 128 || (!TA && !TB && tiles > 256 && longest <= 256))
+        launch<TA, TB, 1, 2, 4>(jobs, beta, st);
     else if (tiles <= 256 && longest >= 256)
         launch<TA, TB, 2, 2, 8>(jobs, beta, st);
     else
         launch<TA, TB, 2, 2, 4>(jobs, beta, st);
 }
 
-}  // namespace
-
-bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
-    if (count < 1 || count > Jobs::MAX || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
-    Jobs jobs{};
+template <int MAX>
+bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
+    Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
         const F32Product& p = ps[j];
@@ -238,16 +251,16 @@ bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
             return false;
         if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= int64_t{1} << 31 || extent(tB ? p.N : p.K, tB ? p.K : p.N, p.ldb) >= int64_t{1} << 31)
             return false;
-        jobs.a[j] = p.a;
-        jobs.b[j] = p.b;
-        jobs.c[j] = p.c;
-        jobs.addend[j] = p.addend;
-        jobs.lda[j] = static_cast<int>(p.lda);
-        jobs.ldb[j] = static_cast<int>(p.ldb);
-        jobs.ldc[j] = static_cast<int>(p.ldc);
-        jobs.M[j] = static_cast<int>(p.M);
-        jobs.N[j] = static_cast<int>(p.N);
-        jobs.K[j] = static_cast<int>(p.K);
+        jobs.job[j].a = p.a;
+        jobs.job[j].b = p.b;
+        jobs.job[j].c = p.c;
+        jobs.job[j].addend = p.addend;
+        jobs.job[j].lda = static_cast<int>(p.lda);
+        jobs.job[j].ldb = static_cast<int>(p.ldb);
+        jobs.job[j].ldc = static_cast<int>(p.ldc);
+        jobs.job[j].M = static_cast<int>(p.M);
+        jobs.job[j].N = static_cast<int>(p.N);
+        jobs.job[j].K = static_cast<int>(p.K);
     }
     if (tA)
         launch_by_size<true, false>(jobs, beta, st);
@@ -256,6 +269,13 @@ bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
     else
         launch_by_size<false, false>(jobs, beta, st);
     return true;
+}
+
+}  // namespace
+
+bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
+    if (count < 1 || count > 8 || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
+    return count == 1 ? multiply<1>(ps, count, tA, tB, beta, st) : multiply<8>(ps, count, tA, tB, beta, st);
 }
 
 }  // namespace pk
