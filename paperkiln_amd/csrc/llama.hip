@@ -11,6 +11,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "pk_internal.h"
@@ -310,6 +311,29 @@ int guarded(F&& f) {
     }
 }
 
+// AdamW on every parameter with the copies that the products read. False, with nothing done, where the kernel does not take
+// them (or a parameter has two copies).
+bool adamw_with_copies(const Model& m, float lr, float b1, float b2, float eps, float wd, float c1, float c2, const float* factor) {
+    std::unordered_map<const Variable*, CastJob> copies;
+    for (const ShadowCopy& s : shadow_copies())
+        if (!copies.emplace(s.of, s.job).second) return false;
+    std::vector<AdamWPart> parts;
+    size_t found = 0;
+    for (const auto& kv : m.named) {
+        const Tensor& p = kv.second->data;
+        AdamWPart part{p.off_bytes / static_cast<int64_t>(sizeof(float)), p.numel(), p.cols, Tensor(), 0};
+        const auto it = copies.find(kv.second.get());
+        if (it != copies.end()) {
+            part.copy = it->second.dst;
+            part.col_off = it->second.col_off;
+            ++found;
+        }
+        if (p.buf != m.pslab.buf || kv.second->grad.buf != m.gslab.buf || kv.second->grad.off_bytes != p.off_bytes) return false;
+        parts.push_back(std::move(part));
+    }
+    return found == copies.size() && k_adamw_parts(m.pslab, m.gslab, m.mslab, m.vslab, parts, lr, b1, b2, eps, wd, c1, c2, factor);
+}
+
 Model* model_of(void* handle) {
     if (!handle) throw Error(PK_ERR_ARGUMENT, "null model handle");
     return static_cast<Model*>(handle);
@@ -517,9 +541,11 @@ int pk_llama_adamw_step(void* h, float lr, float b1, float b2, float eps, float 
         const float c2 = 1.0f - std::pow(b2, static_cast<float>(m->t));
         // every parameter of this model receives a gradient each step, so the reference's "skip a
         // parameter that never accumulated" (nn.cpp:309) never applies; padding stays at zero
-        k_adamw(m->pslab, m->gslab, m->mslab, m->vslab, lr, b1, b2, eps, wd, c1, c2,
-                clip ? static_cast<const float*>(clip->p) : nullptr);
-        refresh_shadows();  // the bf16 copies of the weights follow them, in one launch
+        const float* const factor = clip ? static_cast<const float*>(clip->p) : nullptr;
+        if (!adamw_with_copies(*m, lr, b1, b2, eps, wd, c1, c2, factor)) {
+            k_adamw(m->pslab, m->gslab, m->mslab, m->vslab, lr, b1, b2, eps, wd, c1, c2, factor);
+            refresh_shadows();  // the copies of the weights follow them, in one launch
+        }
         hip_check(hipStreamSynchronize(tape_stream()), "hipStreamSynchronize");
         if (total_norm) *total_norm = *norm;
     });

@@ -3,3 +3,12 @@
 // implement it.
 #pragma once
 #include "tensor.h"
+
+namespace pk {
+// The copies that products read of the current context's parameters, each with the parameter it follows.
+struct ShadowCopy {
+    const Variable* of;
+    CastJob job;
+};
+std::vector<ShadowCopy> shadow_copies();
+}  // namespace pk

@@ -36,6 +36,13 @@ struct TapeContext::Pending {
         Var W;
     };
     std::vector<Job> jobs;
+    // Likewise the last step of a norm weight's gradient, the sum over its workgroups' shares: taken together when the
+    // outermost pass ends.
+    struct Sum {
+        HeldSum sum;
+        Var w;
+    };
+    std::vector<Sum> sums;
     int depth = 0;  // run_backward calls in progress
 };
 
@@ -185,6 +192,24 @@ bool defer_weight_gradient(const Tensor& x, const Tensor& dy, int64_t col0, int6
     return true;
 }
 
+void flush_held_sums() {
+    auto& sums = pending().sums;
+    std::vector<HeldSum> held;
+    for (auto& s : sums) {  // asked for again: the weight's gradient may have moved since
+        s.sum.dw = static_cast<float*>(s.w->ensure_grad().ptr());
+        held.push_back(s.sum);
+    }
+    k_add_held(held.data(), static_cast<int>(held.size()));
+    sums.clear();
+}
+void hold_sum(HeldSum&& sum, const Var& w) {
+    auto& sums = pending().sums;
+    bool full = sums.size() == 16;
+    for (const auto& s : sums) full = full || s.w.get() == w.get();  // a weight used twice must not meet itself in one launch
+    if (full) flush_held_sums();
+    sums.push_back(TapeContext::Pending::Sum{std::move(sum), w});
+}
+
 void run_backward(const Var& root) {
     auto& pd = pending();
     ++pd.depth;
@@ -192,8 +217,10 @@ void run_backward(const Var& root) {
         for (Variable* n : backward_order(root))
             if (n->backward_fn && !n->grad.empty()) n->backward_fn();
         flush_weight_gradients();
+        if (pd.depth == 1) flush_held_sums();
     } catch (...) {
         pd.jobs.clear();
+        pd.sums.clear();
         --pd.depth;
         throw;
     }
@@ -270,23 +297,28 @@ void set_compute_dtype(int dtype) {
 }
 int compute_dtype() { return tape_context().compute; }
 void invalidate_shadows() { tape_context().shadows.reset(); }
+std::vector<ShadowCopy> shadow_copies() {
+    std::vector<ShadowCopy> list;
+    const TapeContext& c = tape_context();
+    if (!c.shadows) return list;
+    for (auto& kv : c.shadows->single) list.push_back({kv.first, CastJob{kv.first->data, kv.second, 0}});
+    for (auto& kv : c.shadows->cat) {
+        int64_t off = 0;
+        for (const Variable* w : kv.second.ws) {
+            list.push_back({w, CastJob{w->data, kv.second.t, off}});
+            off += w->data.cols;
+        }
+    }
+    return list;
+}
 // The copies are brought up to date where they lie instead of being dropped and rebuilt at their next use: one
 // launch for all of them (a model's dozens of weights would otherwise each be a cast kernel of a few microseconds
 // after every optimizer step). The parameters they were made from must still be alive.
 void refresh_shadows() {
-    TapeContext& c = tape_context();
-    if (!c.shadows) return;
     std::vector<CastJob> jobs;
-    for (auto& kv : c.shadows->single) jobs.push_back(CastJob{kv.first->data, kv.second, 0});
-    for (auto& kv : c.shadows->cat) {
-        int64_t off = 0;
-        for (const Variable* w : kv.second.ws) {
-            jobs.push_back(CastJob{w->data, kv.second.t, off});
-            off += w->data.cols;
-        }
-    }
+    for (const ShadowCopy& s : shadow_copies()) jobs.push_back(s.job);
     if (jobs.empty()) return;
-    if (!k_cast_many(jobs)) c.shadows.reset();  // not casts the batched kernel takes: rebuilt at their next use
+    if (!k_cast_many(jobs)) tape_context().shadows.reset();  // not casts the batched kernel takes: rebuilt at their next use
 }
 void prepare_shadow(const Var& W) { (void)shadow_of(W); }
 void prepare_shadow_cat(const std::vector<Var>& Ws) { (void)shadow_cat(Ws); }
@@ -656,8 +688,11 @@ Var rmsnorm(const Var& x, const Var& w) {
         // x usually has the residual branch's gradient already: the kernel adds it on the way out (one rounding of
         // the sum instead of two) and the result replaces it, which also leaves a shared tensor untouched
         const bool onto = x->requires_grad && !x->is_param && !x->grad.empty() && x->grad.dtype == dx.dtype;
+        HeldSum held;
         k_rmsnorm_bwd(self->grad, x->data, static_cast<const float*>(rinv->p), w->data, dw,
-                      x->requires_grad ? &dx : nullptr, onto ? &x->grad : nullptr);
+                      x->requires_grad ? &dx : nullptr, onto ? &x->grad : nullptr,
+                      dw && w->is_param && pending().depth > 0 ? &held : nullptr);
+        if (held.part) hold_sum(std::move(held), w);
         if (onto) {
             x->grad = std::move(dx);
             x->grad_shared = false;

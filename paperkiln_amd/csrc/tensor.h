@@ -36,8 +36,15 @@ void k_silu_mul_cat_fwd(const Tensor& gu, const Tensor& y);
 void k_silu_mul_cat_bwd(const Tensor& gu, const Tensor& dy, const Tensor& dgu);
 void k_rmsnorm_fwd(const Tensor& x, const Tensor& w, float eps, const Tensor& y, float* rinv);  // ops.cpp:437-445
 // ops.cpp:447-478; with an addend (dx's shape and type) dx = addend + the gradient through the norm
+// With `held`, dw's sum over the workgroups' shares may be left to do (held->part is set then) for k_add_held, which takes many.
+struct HeldSum {
+    std::shared_ptr<Buffer> part;  // [nparts][cols]
+    int nparts = 0, cols = 0;
+    float* dw = nullptr;           // dw[c] += sum over the parts
+};
 void k_rmsnorm_bwd(const Tensor& dy, const Tensor& x, const float* rinv, const Tensor& w, const Tensor* dw_f32,
-                   const Tensor* dx, const Tensor* addend = nullptr);
+                   const Tensor* dx, const Tensor* addend = nullptr, HeldSum* held = nullptr);
+void k_add_held(const HeldSum* held, int count);  // no two with the same dw
 // apply_rope on a fused [N, 3d] matrix (ops.cpp:481-537): rotates adjacent pairs of the
 // first `rot_heads` heads of the q third and of the k third; inverse = backward.
 void k_rope(const Tensor& x, const int* pos, float theta, int d, int head_dim, int rot_heads, bool inverse,
@@ -68,6 +75,15 @@ void k_word_to_pinned(const void* src, void* pinned);  // one float for the host
 // clip_dev (may be null): g is scaled in place by *clip_dev first, in the same pass
 void k_adamw(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, float lr, float b1, float b2,
              float eps, float wd, float c1, float c2, const float* clip_dev = nullptr);         // nn.cpp:301-321
+// The same over parts of the slabs, each of which may have a copy that is written with it: element e of the part to column
+// col_off + e % cols of row e / cols. False, with nothing done, for parts that are not whole groups of four.
+struct AdamWPart {
+    int64_t at, count, cols;
+    Tensor copy;
+    int64_t col_off;
+};
+bool k_adamw_parts(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, const std::vector<AdamWPart>& parts, float lr,
+                   float b1, float b2, float eps, float wd, float c1, float c2, const float* clip_dev);
 
 // C[M,N] (+)= op(A) . op(B), row-major, bf16 or fp32 operands, fp32 accumulate
 // (device::gemm, src/device.cpp:91-125). C may be a column slice of a wider

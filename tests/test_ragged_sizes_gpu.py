@@ -61,6 +61,32 @@ def test_bf16_training_with_any_vocabulary(vocab, d, ff, layers, tokens, seq):
         m.close()
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("vocab,d,ff,layers", [(130, 64, 176, 8), (37, 12, 20, 1), (37, 6, 10, 1)])
+def test_optimiser_step_writes_the_copies(vocab, d, ff, layers, dtype):
+    """AdamW with the products' copies of the parameters written in the same pass: more parameters than one launch takes, sizes
+    that are no multiple of 8, and of 4 (two passes). Against float64; and a model made from the result has the same loss.
+    An update's terms are each within their rounding of 1: 1e-5 of the rate, and the sum's own."""
+    m = Llama(vocab=vocab, d=d, n_layers=layers, n_heads=1, d_ff=ff, compute_dtype=dtype, seed=8)
+    toks = synth.randint(3, 65, vocab)
+    m1 = {k: np.zeros(v.shape) for k, v in m.params().items()}
+    m2 = {k: np.zeros(v.shape) for k, v in m1.items()}
+    for t in (1, 2):
+        m.loss_backward(toks[:-1], toks[1:], 32)
+        g, p = m.grads(), m.params()
+        norm = m.adamw_step(1e-2, max_norm=0.5)
+        for k, now in m.params().items():
+            gk = g[k].astype(np.float64) * min(1.0, 0.5 / norm)
+            m1[k], m2[k] = 0.9 * m1[k] + 0.1 * gk, 0.999 * m2[k] + 0.001 * gk * gk
+            step = m1[k] / (1 - 0.9 ** t) / (np.sqrt(m2[k] / (1 - 0.999 ** t)) + 1e-8) + 0.01 * p[k]
+            assert (np.abs(now - (p[k] - 1e-2 * step)) <= 1e-2 * 1e-5 + 2e-7 * np.abs(now)).all(), (k, t)
+    fresh = Llama(vocab=vocab, d=d, n_layers=layers, n_heads=1, d_ff=ff, compute_dtype=dtype, seed=9)
+    fresh.set_params(m.params())
+    assert fresh.loss_backward(toks[:-1], toks[1:], 32)[0] == m.loss_backward(toks[:-1], toks[1:], 32)[0]
+    m.close()
+    fresh.close()
+
+
 def exact_attention(q, k, v, d_o, scale, causal, window, sinks, given_o=None):
     """O, LSE, dQ, dK, dV in float64 (src/ops.cpp:863-1027) of [B,T,H,dk] tensors, K / V heads shared by groups. given_o: the O
     whose rowsum(dO .* O) the gradients are formed with, as a backward is given it; the exact O otherwise."""
