@@ -232,6 +232,9 @@ Var scale(const Var& x, float s);                   // ops.cpp:843-861
 Var silu(const Var& x);                             // ops.cpp:404-424
 Var silu_mul(const Var& gate, const Var& up);        // mul(silu(gate), up) as one node (llama.cpp:55-58)
 Var silu_mul_cat(const Var& gate_up);                // the same on the halves of one [N, 2*d_ff] projection [gate | up]
+// r + (silu(x gate) .* (x up)) down: a Llama block's MLP and residual (llama.cpp:55-59) as one node, the gated product formed in the
+// projections beside it. result_needed as in linear_add.
+Var gated_mlp(const Var& x, const Var& gate, const Var& up, const Var& down, const Var& r, bool result_needed = true);
 Var rmsnorm(const Var& x, const Var& w);            // ops.cpp:426-479, eps fixed at 1e-5 (:435)
 // ops::apply_rope on the fused [N, 3d] matrix (ops.cpp:481-537). rot_heads = 1 is the
 // reference as written (only the first head of q and of k is rotated, :498-499 with the

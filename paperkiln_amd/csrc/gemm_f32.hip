@@ -24,8 +24,12 @@ struct Job {
     const float* b;
     float* c;
     const float* addend;
+    float* gu;  // the gated forms' [M, 2 N] matrix [gate | up]
     int lda, ldb, ldc, M, N, K;
 };
+// What becomes of a tile. GATE: B is [gate | up], N columns each, and a tile is the same columns of both: C = silu(gate) up, and both
+// of them to gu if it is given. GATE_GRAD: the product is C's gradient d for the gate and up in gu: C is [M, 2 N] and gets theirs.
+enum class End { PLAIN, GATE, GATE_GRAD };
 // One product's numbers are found at one place, several products' only once the workgroup knows whose tile it has: a second
 // round trip to the arguments, 0.4 to 0.8 us of the 3.5 to 8 that a small product takes.
 template <int MAX>
@@ -78,9 +82,10 @@ __host__ __device__ inline int64_t extent(int64_t rows, int64_t cols, int64_t ld
 __device__ inline int bytes_of(int rows, int cols, int64_t ld) { return static_cast<int>(extent(rows, cols, ld)); }
 
 // A workgroup's tile is MB x NB blocks of 16 x 16; its KW wavefronts split the contraction chunk by chunk.
-template <bool TA, bool TB, int MB, int NB, int KW, int MAX>
+template <bool TA, bool TB, int MB, int NB, int KW, int MAX, End END>
 __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta) {
-    constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB, TN = 16 * NB;
+    constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB;
+    constexpr int HALF = END == End::GATE ? NB / 2 : NB, TN = 16 * HALF;  // blocks of columns of C
     // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
     const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (t >= tiles) return;
@@ -97,7 +102,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 #pragma unroll
     for (int i = 0; i < MB; ++i) row[i] = min(m0 + i * 16 + l16, M - 1);
 #pragma unroll
-    for (int i = 0; i < NB; ++i) col[i] = min(n0 + i * 16 + l16, N - 1);
+    for (int i = 0; i < NB; ++i) col[i] = min(n0 + i % HALF * 16 + l16, N - 1) + (i >= HALF ? N : 0);
 
     f32x4 acc[MB][NB];
 #pragma unroll
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
         for (int y = 0; y < NB; ++y) acc[x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a), 0, bytes_of(TA ? K : M, TA ? M : K, lda), 0x00020000);
-    const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(b), 0, bytes_of(TB ? N : K, TB ? K : N, ldb), 0x00020000);
+    const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(b), 0, bytes_of(TB ? N : K, TB ? K : END == End::GATE ? 2 * N : N, ldb), 0x00020000);
     int oa[MB], ob[NB];
 #pragma unroll
     for (int i = 0; i < MB; ++i) oa[i] = static_cast<int>(TA ? 4 * grp * lda + row[i] : row[i] * lda + 4 * grp) * 4;
@@ -173,7 +178,26 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
             const int m = m0 + x * 16 + 4 * grp + r;
             if (m < M) {
                 const int64_t o = m * ldc + n;
-                out[o] = add ? add[o] + v[r] : v[r];
+                if constexpr (END == End::GATE_GRAD)
+                    gated_grad(jobs.job[j].gu[o], jobs.job[j].gu[o + N], v[r], out[o], out[o + N]);
+                else
+                    out[o] = add ? add[o] + v[r] : v[r];
+            }
+        }
+    };
+    auto store_gated = [&](int x, int y, f32x4 gate, f32x4 up) {
+        float* const gu = jobs.job[j].gu;
+        const int n = n0 + y * 16 + l16;
+        if (n >= N) return;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + x * 16 + 4 * grp + r;
+            if (m < M) {
+                out[m * ldc + n] = gated(gate[r], up[r]);
+                if (gu) {
+                    gu[m * ldc * 2 + n] = gate[r];
+                    gu[m * ldc * 2 + N + n] = up[r];
+                }
             }
         }
     };
@@ -184,27 +208,35 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
         for (int y = 0; y < NB; ++y) part[kw][x * NB + y][lane] = acc[x][y];
     __syncthreads();
 #pragma unroll
-    for (int g0 = 0; g0 < MB * NB; g0 += KW) {
+    for (int g0 = 0; g0 < MB * HALF; g0 += KW) {
         const int g = g0 + kw;
-        if (g < MB * NB) {
-            f32x4 s = part[0][g][lane];
+        if (g < MB * HALF) {
+            const int at = g / HALF * NB + g % HALF;
+            f32x4 s = part[0][at][lane];
 #pragma unroll
-            for (int k = 1; k < KW; ++k) s += part[k][g][lane];
-            store(g / NB, g % NB, s);
+            for (int k = 1; k < KW; ++k) s += part[k][at][lane];
+            if constexpr (END == End::GATE) {
+                f32x4 up = part[0][at + HALF][lane];
+#pragma unroll
+                for (int k = 1; k < KW; ++k) up += part[k][at + HALF][lane];
+                store_gated(g / HALF, g % HALF, s, up);
+            } else {
+                store(g / HALF, g % HALF, s);
+            }
         }
     }
 }
 
-template <bool TA, bool TB, int MB, int NB, int KW, int MAX>
+template <bool TA, bool TB, int MB, int NB, int KW, End END, int MAX>
 void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
-    constexpr int TM = 16 * MB, TN = 16 * NB;
+    constexpr int TM = 16 * MB, TN = 16 * (END == End::GATE ? NB / 2 : NB);
     int tiles = 0;
     for (int j = 0; j < jobs.count; ++j) {
         jobs.first[j] = tiles;
         tiles += ((jobs.job[j].M + TM - 1) / TM) * ((jobs.job[j].N + TN - 1) / TN);
     }
     for (int j = jobs.count; j <= MAX; ++j) jobs.first[j] = tiles;
-    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, MAX>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
+    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, MAX, END>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
                        tiles, beta);
     hip_check(hipGetLastError(), "gemm_f32");
 }
@@ -219,28 +251,28 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
 //   In between 32 x 32; eight wavefronts split the contraction where it is long and there is a tile or less to a CU. Short
 //   contractions of more tiles than that are over sooner as 16 x 32, for which the last round is half as long (1000 x 576 x
 //   192: 7.7 us against 9.4, 256 x 1376 x 256: 5.8 against 6.8; with B transposed, whose rows those tiles read twice, they are not).
-template <bool TA, bool TB, int MAX>
+template <bool TA, bool TB, End END, int MAX>
 void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     int64_t tiles = 0;
     int longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
-        tiles += static_cast<int64_t>((jobs.job[j].M + 31) / 32) * ((jobs.job[j].N + 31) / 32);
+        tiles += static_cast<int64_t>((jobs.job[j].M + 31) / 32) * ((jobs.job[j].N * (END == End::GATE ? 2 : 1) + 31) / 32);
         longest = std::max(longest, jobs.job[j].K);
     }
     if (tiles > 640 && (!TA || longest < 256))
-        launch<TA, TB, 4, 4, 4>(jobs, beta, st);
-    else if (tiles <= 64)
-        launch<TA, TB, 1, 1, 4>(jobs, beta, st);
+        launch<TA, TB, 4, 4, 4, END>(jobs, beta, st);
+    else if (tiles <= 64 && END != End::GATE)
+        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END>(jobs, beta, st);
     else if (tiles <= 128 || (!TA && !TB && tiles > 256 && longest <= 256))
-        launch<TA, TB, 1, 2, 4>(jobs, beta, st);
+        launch<TA, TB, 1, 2, 4, END>(jobs, beta, st);
     else if (tiles <= 256 && longest >= 256)
-        launch<TA, TB, 2, 2, 8>(jobs, beta, st);
+        launch<TA, TB, 2, 2, 8, END>(jobs, beta, st);
     else
-        launch<TA, TB, 2, 2, 4>(jobs, beta, st);
+        launch<TA, TB, 2, 2, 4, END>(jobs, beta, st);
 }
 
 template <int MAX>
-bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
+bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st, End end = End::PLAIN, float* gu = nullptr) {
     Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
@@ -249,12 +281,13 @@ bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
         if (p.M <= 0 || p.N <= 0 || p.K <= 0 || p.M > limit || p.N > limit || p.K > limit || p.lda > limit || p.ldb > limit ||
             p.ldc > limit)
             return false;
-        if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= int64_t{1} << 31 || extent(tB ? p.N : p.K, tB ? p.K : p.N, p.ldb) >= int64_t{1} << 31)
+        if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= int64_t{1} << 31 || extent(tB ? p.N : p.K, tB ? p.K : end == End::GATE ? 2 * p.N : p.N, p.ldb) >= int64_t{1} << 31)
             return false;
         jobs.job[j].a = p.a;
         jobs.job[j].b = p.b;
         jobs.job[j].c = p.c;
         jobs.job[j].addend = p.addend;
+        jobs.job[j].gu = gu;
         jobs.job[j].lda = static_cast<int>(p.lda);
         jobs.job[j].ldb = static_cast<int>(p.ldb);
         jobs.job[j].ldc = static_cast<int>(p.ldc);
@@ -262,12 +295,17 @@ bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
         jobs.job[j].N = static_cast<int>(p.N);
         jobs.job[j].K = static_cast<int>(p.K);
     }
+    if constexpr (MAX == 1) {
+        if (end == End::GATE) launch_by_size<false, false, End::GATE>(jobs, beta, st);
+        if (end == End::GATE_GRAD) launch_by_size<false, true, End::GATE_GRAD>(jobs, beta, st);
+        if (end != End::PLAIN) return true;
+    }
     if (tA)
-        launch_by_size<true, false>(jobs, beta, st);
+        launch_by_size<true, false, End::PLAIN>(jobs, beta, st);
     else if (tB)
-        launch_by_size<false, true>(jobs, beta, st);
+        launch_by_size<false, true, End::PLAIN>(jobs, beta, st);
     else
-        launch_by_size<false, false>(jobs, beta, st);
+        launch_by_size<false, false, End::PLAIN>(jobs, beta, st);
     return true;
 }
 
@@ -276,6 +314,14 @@ bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
 bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
     if (count < 1 || count > 8 || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
     return count == 1 ? multiply<1>(ps, count, tA, tB, beta, st) : multiply<8>(ps, count, tA, tB, beta, st);
+}
+bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    const F32Product p{x, K, w, 2 * N, h, N, nullptr, M, N, K};
+    return multiply<1>(&p, 1, false, false, 0.0f, st, End::GATE, gu);
+}
+bool gemm_f32_gated_grad(const float* dy, const float* w, const float* gu, float* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    const F32Product p{dy, K, w, K, dgu, 2 * N, nullptr, M, N, K};
+    return multiply<1>(&p, 1, false, true, 0.0f, st, End::GATE_GRAD, const_cast<float*>(gu));
 }
 
 }  // namespace pk

@@ -341,26 +341,31 @@ __device__ inline void wait_loads_then_barrier() {
     static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
+// GATED: the operand is [gate | up] of `half` columns each, and the tile holds, in 32-column blocks in turn, the same columns of both:
+// a wavefront's two blocks of results are then a gate's and an up's, lane by lane. Column (of gate) a chunk begins at, from the
+// tile's first on, and bytes from the tile's first to the chunk:
+__device__ inline int gated_column(int c) { return (c >> 3) * 32 + (c & 3) * 8; }
+__device__ inline uint32_t gated_bytes(int c, int half) { return (gated_column(c) + (c & 4 ? half : 0)) * 2u; }
 // lane offsets of a wavefront's loads of one operand's slice, for a tile in the matrix's interior (every column there,
 // every slice whole)
-template <typename O>
-__device__ inline void lane_offsets(uint32_t (&off)[O::PER], int w, int lane, int64_t ld) {
+template <typename O, bool GATED = false>
+__device__ inline void lane_offsets(uint32_t (&off)[O::PER], int w, int lane, int64_t ld, int half = 0) {
 #pragma unroll
     for (int j = 0; j < O::PER; ++j) {
         const int u = (w * O::PER + j) * 64 + lane, r = u / O::CPR, c = O::swz(r, u % O::CPR);
-        off[j] = static_cast<uint32_t>(r) * static_cast<uint32_t>(ld) * 2u + c * 16u + BIAS - j * 1024u;
+        off[j] = static_cast<uint32_t>(r) * static_cast<uint32_t>(ld) * 2u + (GATED ? gated_bytes(c, half) : c * 16u) + BIAS - j * 1024u;
     }
 }
 // ... and with the chunks that must not be read sent outside the buffer: columns past the matrix's edge of a
 // [k][column] operand (every slice of an edge tile), chunks past the contraction's end in the last, partial slice of
 // a [row][k] operand (they are the next row's)
-template <typename O, bool TR>
+template <typename O, bool TR, bool GATED = false>
 __device__ inline void lane_offsets_masked(uint32_t (&off)[O::PER], const uint32_t (&whole)[O::PER], int w, int lane, int rc0,
                                            int rc_count, int ktail) {
 #pragma unroll
     for (int j = 0; j < O::PER; ++j) {
         const int u = (w * O::PER + j) * 64 + lane, r = u / O::CPR, c = O::swz(r, u % O::CPR);
-        const bool ok = TR ? rc0 + c * 8 < rc_count : (ktail == 0 || c * 8 < ktail);
+        const bool ok = TR ? rc0 + (GATED ? gated_column(c) : c * 8) < rc_count : (ktail == 0 || c * 8 < ktail);
         off[j] = ok ? whole[j] : OUTSIDE;
     }
 }
@@ -394,14 +399,20 @@ __global__ __launch_bounds__(G::NTHR, NS * (RingOp<TA, G::BM, G::NTHR / 64>::BYT
 void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     static_assert(EPI == 0 || EPI == 3 || (G::KS == 1 && !CF32), "the head's epilogues: one wavefront set, bf16 result");
     constexpr bool GROUPED = EPI == 3;
+    // A gated product's ends. 5, 6: B is [gate | up], N columns each; C = silu(gate) up, and (5) both of them to D, [M, 2 N]. 7: the
+    // product is the gradient of C for the gate and up in D; C is [M, 2 N] and gets theirs.
+    constexpr bool GATE = EPI == 5 || EPI == 6, GATE_GRAD = EPI == 7;
+    static_assert(!GATE || (!TB && G::FN == 2), "a wavefront holds a block of gate and one of up");
     constexpr int BM = G::BM, BN = G::BN, NTHR = G::NTHR, FM = G::FM, FN = G::FN, NW = NTHR / 64;
     using OA = RingOp<TA, BM, NW>;
     using OB = RingOp<!TB, BN, NW>;
     using ST = TileStore<G, CF32>;
     constexpr int SLOT = OA::BYTES + OB::BYTES, PERTOT = OA::PER + OB::PER;
+    constexpr int BNC = GATE ? BN / 2 : BN;  // columns of C per tile
+    constexpr int NST = EPI == 5 ? ST::NST / 2 * 3 : EPI == 6 ? ST::NST / 2 : EPI == 7 ? ST::NST * 2 : ST::NST;
     static_assert(NS >= 2 && NS * SLOT <= 160 * 1024, "the ring must fit the LDS");
     static_assert(ST::BYTES <= SLOT, "an epilogue strip must fit one ring slot");
-    static_assert((NS - 2) * PERTOT + ST::NST < 64, "memory operations in flight must fit the counter");
+    static_assert((NS - 2) * PERTOT + NST < 64, "memory operations in flight must fit the counter");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * SLOT];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int KS = G::KS, NWQ = G::WGM * G::WGN, KPW = BK / 16 / KS;  // k-chunks of a slice per wavefront
@@ -436,7 +447,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             }
             const int tm = t / tiles_n;
             bl.m0 = tm * BM;
-            bl.n0 = (t - tm * tiles_n) * BN;
+            bl.n0 = (t - tm * tiles_n) * BNC;
             bl.z = z;
             bl.p = p;
             bl.k_begin = z * g.k_per_split;
@@ -462,7 +473,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     uint32_t offa[OA::PER], offb[OB::PER], offa_c[OA::PER], offb_c[OB::PER];
     if (!GROUPED) {  // a grouped launch forms them per tile: the row pitches are the problem's
         lane_offsets<OA>(offa, w, lane, g.lda);
-        lane_offsets<OB>(offb, w, lane, g.ldb);
+        lane_offsets<OB, GATE>(offb, w, lane, g.ldb, g.N);
     }
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
     const uint32_t dst_a = lds0 + w * OA::PER * 1024u, dst_b = lds0 + OA::BYTES + w * OB::PER * 1024u;
@@ -487,7 +498,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             lane_offsets<OB>(offb, w, lane, fp.ldb);
         }
         da = tile_desc<TA>(fp.a, fp.lda, fb.m0, fp.M, fb.k_begin, fb.k_end);
-        db = tile_desc<!TB>(fp.b, fp.ldb, fb.n0, fp.N, fb.k_begin, fb.k_end);
+        db = tile_desc<!TB>(fp.b, fp.ldb, fb.n0, GATE ? 2 * fp.N : fp.N, fb.k_begin, fb.k_end);
         // the masked lane offsets: used by every slice of a [k][column] operand, by the last slice of a [row][k] one
         if (TA ? fb.m0 + BM > fp.M : f_ktail != 0)
             lane_offsets_masked<OA, TA>(offa_c, offa, w, lane, fb.m0, fp.M, f_ktail);
@@ -495,8 +506,8 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
             for (int j = 0; j < OA::PER; ++j) offa_c[j] = offa[j];
         }
-        if (!TB ? fb.n0 + BN > fp.N : f_ktail != 0)
-            lane_offsets_masked<OB, !TB>(offb_c, offb, w, lane, fb.n0, fp.N, f_ktail);
+        if (!TB ? fb.n0 + BNC > fp.N : f_ktail != 0)
+            lane_offsets_masked<OB, !TB, GATE>(offb_c, offb, w, lane, fb.n0, fp.N, f_ktail);
         else {
 #pragma unroll
             for (int j = 0; j < OB::PER; ++j) offb_c[j] = offb[j];
@@ -679,6 +690,91 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             }
         }
     };
+    // The ends of gated products, strip by strip as below. Gate, up and the gradient count as they are stored, rounded.
+    const auto lo = [](uint32_t v) { return __uint_as_float(v << 16); };
+    const auto hi = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
+    auto write_strip = [&](uint16_t* cs, int i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                const u32x2 v = {pack_bf16(acc[i][j][qd * 4], acc[i][j][qd * 4 + 1]), pack_bf16(acc[i][j][qd * 4 + 2], acc[i][j][qd * 4 + 3])};
+                *reinterpret_cast<u32x2*>(cs + (wm * 32 + c32) * ST::CP + (wn * FN + j) * 32 + qd * 8 + gh * 4) = v;
+            }
+    };
+    // descriptor of a [M, ld] matrix from the tile's first element on, `cols` columns from there to the last row's end
+    auto tile_rsrc = [&](const void* base, const Block& bl, int64_t ld, int64_t cols) -> u32x4 {
+        const uint64_t a = reinterpret_cast<uint64_t>(static_cast<const uint16_t*>(base) + bl.m0 * ld + bl.n0);
+        const int64_t left = ((g.M - bl.m0 - 1) * ld + cols) * 2;
+        return u32x4{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32) & 0xffffu, left > 0x7ffffff0 ? 0x7ffffff0u : static_cast<uint32_t>(left),
+                     0x00020000u};
+    };
+    auto store_gated = [&](uint8_t* strip, const Block& bl) {
+        constexpr int GPR = ST::CPR / 2;  // chunks of gate in a strip row; each with its chunk of up four further on
+        static_assert(NTHR % GPR == 0 && ST::SR * GPR % NTHR == 0, "one chunk column per thread, whole rounds of rows");
+        const int q = static_cast<int>(threadIdx.x) % GPR, cg = (q >> 2) * 8 + (q & 3), col = gated_column(cg);
+        const u32x4 to_c = tile_rsrc(g.c, bl, g.N, g.N - bl.n0), to_d = tile_rsrc(g.d, bl, 2 * g.N, 2 * g.N - bl.n0);
+        const uint32_t mask = bl.n0 + col < g.N ? 0u : OUTSIDE;
+        uint16_t* const cs = reinterpret_cast<uint16_t*>(strip);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            write_strip(cs, i);
+            __syncthreads();
+            const uint32_t soff = static_cast<uint32_t>(i * 32) * g.N * 2u;
+#pragma unroll
+            for (int k = 0; k < ST::SR * GPR / NTHR; ++k) {
+                const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / GPR, trow = (srow >> 5) * FM * 32 + (srow & 31);
+                const u32x4 gate = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + cg * 8),
+                            up = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + cg * 8 + 32);
+                u32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = pack_bf16(gated(lo(gate[e]), lo(up[e])), gated(hi(gate[e]), hi(up[e])));
+                const uint32_t row = static_cast<uint32_t>(trow) * g.N * 2u;
+                store16(v, (row + col * 2) | mask, to_c, soff);
+                if constexpr (EPI == 5) {
+                    store16(gate, (2 * row + col * 2) | mask, to_d, 2 * soff);
+                    store16(up, (2 * row + col * 2) | mask, to_d, 2 * soff + g.N * 2u);
+                }
+            }
+            __syncthreads();
+        }
+    };
+    auto store_gated_grad = [&](uint8_t* strip, const Block& bl) {
+        const u32x4 to_c = tile_rsrc(g.c, bl, 2 * g.N, 2 * g.N - bl.n0), gu = tile_rsrc(g.d, bl, 2 * g.N, 2 * g.N - bl.n0);
+        const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(static_cast<const uint16_t*>(g.d) + static_cast<int64_t>(bl.m0) * 2 * g.N + bl.n0), 0, static_cast<int>(gu[2]), 0x00020000);
+        const uint32_t mask = bl.n0 + st_ch * 8 < g.N ? 0u : OUTSIDE;
+        uint16_t* const cs = reinterpret_cast<uint16_t*>(strip);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const uint32_t soff = static_cast<uint32_t>(i * 32) * g.N * 4u, up_at = soff + g.N * 2u;
+            u32x4 gate[ST::PER_PHASE], up[ST::PER_PHASE];  // on their way while the strip is written
+#pragma unroll
+            for (int k = 0; k < ST::PER_PHASE; ++k) {
+                gate[k] = __builtin_amdgcn_raw_buffer_load_b128(from, static_cast<int>(coff[k] | mask), static_cast<int>(soff), 0);
+                up[k] = __builtin_amdgcn_raw_buffer_load_b128(from, static_cast<int>(coff[k] | mask), static_cast<int>(up_at), 0);
+            }
+            write_strip(cs, i);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < ST::PER_PHASE; ++k) {
+                const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / ST::CPR;
+                const u32x4 d = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + st_ch * 8);
+                u32x4 dg, du;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float a[2], b[2];
+                    gated_grad(lo(gate[k][e]), lo(up[k][e]), lo(d[e]), a[0], b[0]);
+                    gated_grad(hi(gate[k][e]), hi(up[k][e]), hi(d[e]), a[1], b[1]);
+                    dg[e] = pack_bf16(a[0], a[1]);
+                    du[e] = pack_bf16(b[0], b[1]);
+                }
+                store16(dg, coff[k] | mask, to_c, soff);
+                store16(du, coff[k] | mask, to_c, up_at);
+            }
+            __syncthreads();
+        }
+    };
     // the tile's result, through the ring slot `strip` (which every wavefront has finished reading)
     auto store_result = [&](uint8_t* strip, const Block& bl) {
         if (KS == 2) {  // set 1 hands its sums to set 0, half of them at a time: [wavefront][16-byte group][lane]
@@ -797,7 +893,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             // -- the loads of NS - 2 later slices and, for the NS - 1 slices asked for before the last tile's
             // stores, those stores (memory operations complete in order).
             if (since_store < NS - 1)
-                wait_loads<(NS - 2) * PERTOT + ST::NST>();
+                wait_loads<(NS - 2) * PERTOT + NST>();
             else
                 wait_loads<(NS - 2) * PERTOT>();
             since_store = min(since_store + 1, NS);
@@ -838,7 +934,12 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                 } else {
                     if constexpr (EPI == 2 || EPI == 4) head_dlogits(cb);
                     barrier();  // every wavefront has read slot u: it takes the result on its way out
-                    store_result(lds + u * SLOT, cb);
+                    if constexpr (GATE)
+                        store_gated(lds + u * SLOT, cb);
+                    else if constexpr (GATE_GRAD)
+                        store_gated_grad(lds + u * SLOT, cb);
+                    else
+                        store_result(lds + u * SLOT, cb);
                     since_store = 0;
                 }
                 cv = next_block(cv + stride, cb);
@@ -1212,6 +1313,58 @@ bool gemm_head_dlogits(const void* a, int64_t lda, const void* b, int64_t ldb, i
         head_small(M, N) ? launch_head<GeoSmall, 2>(g, hd, st) : launch_head<GeoLarge, 2>(g, hd, st);
     else
         head_small(M, N) ? launch_head<GeoSmall, 4>(g, hd, st) : launch_head<GeoLarge, 4>(g, hd, st);
+    return true;
+}
+
+// ---- SwiGLU inside the products beside it ----
+// The gate|up projection's two halves meet in the tile that forms them, and the down projection's dX becomes the two halves'
+// gradients where it is formed: no pass reads [tokens, 2 d_ff] to write [tokens, d_ff] or the other way round, and a forward
+// pass that keeps nothing for a backward one does not write gate and up at all (8192 tokens, d_ff 1376: those passes are 14 us
+// and 21; the 35 M parameter model's step with checkpointing, which makes 18 of them, 5.26 -> 5.08 ms). Whole contractions on
+// the two-slot ring.
+namespace {
+template <typename G, bool TB, int EPI>
+void launch_gated_form(GemmArgs g, hipStream_t st) {
+    constexpr int BNC = EPI == 7 ? G::BN : G::BN / 2;
+    g.tiles_m = (g.M + G::BM - 1) / G::BM;
+    g.tiles_n = (g.N + BNC - 1) / BNC;
+    const int64_t vblocks = (static_cast<int64_t>(g.tiles_m) * g.tiles_n + 7) / 8 * 8, slots = cu_count() / 8 * 8 * (G::BM > 128 ? 1 : 2);
+    hipLaunchKernelGGL((gemm_ring<G, false, TB, false, 2, true, EPI>), dim3(static_cast<unsigned>(std::min(vblocks, slots))), dim3(G::NTHR), 0,
+                       st, g, HeadArgs{}, GroupArgs{});
+    hip_check(hipGetLastError(), "gemm_ring (gated) launch");
+}
+// the plan of the product by itself, where it is one of the two forms that are built
+bool gated_plan(bool tB, int64_t M, int64_t cols, int64_t K, int64_t ldb, int64_t pitch, bool& large) {
+    const Plan p = make_plan(false, tB, M, cols, K, K, ldb, pitch);
+    large = p.large;
+    return g_force_geo < 0 && p.S == 1 && (p.ring == 8 || (p.ring == 6 && K <= 768)) && M * pitch * 2 < (int64_t{1} << 31) - 4096;
+}
+}  // namespace
+// h = silu(x gate) .* (x up) for w = [gate | up], N columns each; [x gate | x up] to gu unless that is null.
+bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    if (g_force_geo < 0 && gemm_small_is_ahead(false, false, M, 2 * N, K) && gemm_small_gated(x, w, gu, h, M, N, K, st)) return true;
+    bool large;
+    if (N % 8 || !takes(x, false, K, w, false, 2 * N, M, 2 * N, K) || !aligned16(h) || !aligned16(gu) || !gated_plan(false, M, 2 * N, K, 2 * N, 2 * N, large))
+        return false;
+    GemmArgs g = gemm_args(x, K, w, 2 * N, M, N, K);
+    g.c = h;
+    g.d = gu;
+    if (gu)
+        large ? launch_gated_form<GeoLarge, false, 5>(g, st) : launch_gated_form<GeoSmall, false, 5>(g, st);
+    else
+        large ? launch_gated_form<GeoLarge, false, 6>(g, st) : launch_gated_form<GeoSmall, false, 6>(g, st);
+    return true;
+}
+// d = dy w^T, the gradient of silu(gate) .* up; dgu = [d gate | d up] for gu = [gate | up], N columns each. w is [N, K].
+bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    if (g_force_geo < 0 && gemm_small_is_ahead(false, true, M, N, K) && gemm_small_gated_grad(dy, w, gu, dgu, M, N, K, st)) return true;
+    bool large;
+    if (!takes(dy, false, K, w, true, K, M, N, K) || !aligned16(gu) || !aligned16(dgu) || !gated_plan(true, M, N, K, K, 2 * N, large)) return false;
+    GemmArgs g = gemm_args(dy, K, w, K, M, N, K);
+    g.c = dgu;
+    g.d = gu;
+    g.ldc = 2 * N;
+    large ? launch_gated_form<GeoLarge, true, 7>(g, st) : launch_gated_form<GeoSmall, true, 7>(g, st);
     return true;
 }
 

@@ -20,8 +20,10 @@ struct Job {
     const uint16_t* b;
     void* c;
     const void* addend;
+    uint16_t* gu;  // as in gemm_f32.hip
     int lda, ldb, ldc, M, N, K;
 };
+enum class End { PLAIN, GATE, GATE_GRAD };
 // as in gemm_f32.hip: one product's numbers are found without a second round trip to the arguments (512 x 384 x 128 4.2 -> 3.3 us,
 // 512 x 128 x 344 4.7 -> 3.6, 2048 x 128 x 128 4.0 -> 3.4)
 template <int MAX>
@@ -70,9 +72,9 @@ struct Chunk {
     }
 };
 
-template <bool TA, bool TB, bool CF32, int KW, int MAX>
+template <bool TA, bool TB, bool CF32, int KW, int MAX, End END>
 __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs, const int tiles, const int accumulate) {
-    constexpr int BUFS = 4;
+    constexpr int BUFS = 4, NC = END == End::GATE ? 2 : 1;  // NC: columns of gate and of up, or of one matrix
     // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
     const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (t >= tiles) return;
@@ -85,38 +87,51 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(jobs.job[j].a), 0,
                                                       static_cast<int>(extent(TA ? K : M, TA ? M : K, lda)), 0x00020000);
     const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(jobs.job[j].b), 0,
-                                                      static_cast<int>(extent(TB ? N : K, TB ? K : N, ldb)), 0x00020000);
+                                                      static_cast<int>(extent(TB ? N : K, TB ? K : N * NC, ldb)), 0x00020000);
     int oa[2], ob[2];  // rows and columns past the edge read the last ones; they are not stored
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         oa[b] = TA ? (8 * grp * lda + min(m0 + 2 * l16, M - 2)) * 2 : (min(m0 + 2 * l16 + b, M - 1) * lda + 8 * grp) * 2;
         ob[b] = TB ? (min(n0 + 2 * l16 + b, N - 1) * ldb + 8 * grp) * 2 : (8 * grp * ldb + min(n0 + 2 * l16, N - 2)) * 2;
     }
-    f32x4 acc[2][2];
+    f32x4 acc[NC][2][2];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[c][x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int oc[NC][2];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) oc[c][b] = ob[b] + c * N * 2;
 
     Chunk<TA> fa[BUFS];
-    Chunk<!TB> fb[BUFS];
+    Chunk<!TB> fb[BUFS][NC];
     const int chunks = (K + KC - 1) / KC;
     auto load = [&](int chunk, int buf) {
         // the last chunk of a contraction that is no multiple is moved back to end where that does: its first steps are done
         const int over = max((chunk + 1) * KC - K, 0), k0 = chunk * KC - over;
         fa[buf].load(ra, oa, k0, lda);
-        fb[buf].load(rb, ob, k0, ldb);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) fb[buf][c].load(rb, oc[c], k0, ldb);
         if (over > 0) {
             fa[buf].clear_first(over, grp);
-            fb[buf].clear_first(over, grp);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) fb[buf][c].clear_first(over, grp);
         }
     };
     auto multiply = [&](int buf) {
-        const bf16x8 a0 = fa[buf].block(0), a1 = fa[buf].block(1), b0 = fb[buf].block(0), b1 = fb[buf].block(1);
-        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[1][1], 0, 0, 0);
+        const bf16x8 a0 = fa[buf].block(0), a1 = fa[buf].block(1);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const bf16x8 b0 = fb[buf][c].block(0), b1 = fb[buf][c].block(1);
+            acc[c][0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[c][0][0], 0, 0, 0);
+            acc[c][0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[c][0][1], 0, 0, 0);
+            acc[c][1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[c][1][0], 0, 0, 0);
+            acc[c][1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[c][1][1], 0, 0, 0);
+        }
     };
     const int mine = kw < chunks ? (chunks - kw + KW - 1) / KW : 0;  // chunks kw, kw + KW, ... are this wavefront's
 #pragma unroll
@@ -137,11 +152,13 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
         if (i + u < mine) multiply(u);
 
     // lane (l16, grp), register r of block (x, y): row m0 + 2 (4 grp + r) + x, column n0 + 2 l16 + y
-    __shared__ f32x4 part[KW][2][2][64];
+    __shared__ f32x4 part[KW][NC][2][2][64];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) part[kw][x][y][lane] = acc[x][y];
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) part[kw][c][x][y][lane] = acc[c][x][y];
     __syncthreads();
     constexpr int RPW = 8 / KW;  // of the 2 x 4 rows a lane holds, each wavefront adds up this many
     const int n = n0 + 2 * l16;
@@ -150,15 +167,39 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
         const int row = kw * RPW + q, x = row >> 2, r = row & 3;
-        float s0 = reinterpret_cast<const float*>(&part[0][x][0][lane])[r], s1 = reinterpret_cast<const float*>(&part[0][x][1][lane])[r];
+        auto sum = [&](int c, int y) {
+            float s = reinterpret_cast<const float*>(&part[0][c][x][y][lane])[r];
 #pragma unroll
-        for (int k = 1; k < KW; ++k) {
-            s0 += reinterpret_cast<const float*>(&part[k][x][0][lane])[r];
-            s1 += reinterpret_cast<const float*>(&part[k][x][1][lane])[r];
-        }
+            for (int k = 1; k < KW; ++k) s += reinterpret_cast<const float*>(&part[k][c][x][y][lane])[r];
+            return s;
+        };
+        float s0 = sum(0, 0), s1 = sum(0, 1);
         const int m = m0 + 2 * (4 * grp + r) + x;
         if (m >= M) continue;
         const int64_t o = m * ldc + n;
+        // gate, up and their product's gradient count as they are stored, rounded
+        const auto lo = [](uint32_t v) { return __uint_as_float(v << 16); };
+        const auto hi = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
+        if constexpr (END == End::GATE) {
+            const uint32_t gate = pack_bf16(s0, s1), up = pack_bf16(sum(1, 0), sum(1, 1));
+            *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o) =
+                pack_bf16(gated(lo(gate), lo(up)), gated(hi(gate), hi(up)));
+            if (uint16_t* const gu = jobs.job[j].gu) {
+                *reinterpret_cast<uint32_t*>(gu + m * ldc * 2 + n) = gate;
+                *reinterpret_cast<uint32_t*>(gu + m * ldc * 2 + N + n) = up;
+            }
+            continue;
+        }
+        if constexpr (END == End::GATE_GRAD) {
+            const uint32_t d = pack_bf16(s0, s1), gate = *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o),
+                           up = *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o + N);
+            float dg[2], du[2];
+            gated_grad(lo(gate), lo(up), lo(d), dg[0], du[0]);
+            gated_grad(hi(gate), hi(up), hi(d), dg[1], du[1]);
+            *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o) = pack_bf16(dg[0], dg[1]);
+            *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o + N) = pack_bf16(du[0], du[1]);
+            continue;
+        }
         const void* const add = jobs.job[j].addend ? jobs.job[j].addend : accumulate ? jobs.job[j].c : nullptr;
         if (CF32) {
             f32x2 v = {s0, s1};
@@ -177,7 +218,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
     }
 }
 
-template <bool TA, bool TB, bool CF32, int MAX>
+template <bool TA, bool TB, bool CF32, End END = End::PLAIN, int MAX>
 void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st) {
     int tiles = 0, longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
@@ -189,9 +230,9 @@ void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st) {
     const dim3 grid((tiles + 7) / 8 * 8);
     // eight wavefronts where each still has a few chunks and two workgroups fit every CU
     if (longest >= 512 && tiles <= 1024)
-        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 8, MAX>), grid, dim3(512), 0, st, jobs, tiles, accumulate ? 1 : 0);
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 8, MAX, END>), grid, dim3(512), 0, st, jobs, tiles, accumulate ? 1 : 0);
     else
-        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 4, MAX>), grid, dim3(256), 0, st, jobs, tiles, accumulate ? 1 : 0);
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 4, MAX, END>), grid, dim3(256), 0, st, jobs, tiles, accumulate ? 1 : 0);
     hip_check(hipGetLastError(), "gemm_small");
 }
 
@@ -213,22 +254,24 @@ bool gemm_small_is_ahead(bool tA, bool tB, int64_t M, int64_t N, int64_t K) {
 
 namespace {
 template <int MAX>
-bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st) {
+bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st, End end = End::PLAIN,
+              void* gu = nullptr) {
     Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
         const SmallProduct& p = ps[j];
         const int64_t limit = int64_t{1} << 30;
         if (p.M < 2 || p.N < 2 || p.K < KC || p.M > limit || p.N > limit || p.K > limit) return false;
-        if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= limit || extent(tB ? p.N : p.K, tB ? p.K : p.N, p.ldb) >= limit) return false;
+        if (extent(tA ? p.K : p.M, tA ? p.M : p.K, p.lda) >= limit || extent(tB ? p.N : p.K, tB ? p.K : end == End::GATE ? 2 * p.N : p.N, p.ldb) >= limit) return false;
         // pairs of columns, and of steps where those are adjacent, are read and written as one
         auto aligned = [](const void* q, int a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
         if (p.lda % 2 || p.ldb % 2 || p.ldc % 2 || p.N % 2 || (tA && p.M % 2) || (!(tA && !tB) && p.K % 2)) return false;
-        if (!aligned(p.a, 4) || !aligned(p.b, 4) || !aligned(p.c, 8) || !aligned(p.addend, 8)) return false;
+        if (!aligned(p.a, 4) || !aligned(p.b, 4) || !aligned(p.c, 8) || !aligned(p.addend, 8) || !aligned(gu, 4)) return false;
         jobs.job[j].a = static_cast<const uint16_t*>(p.a);
         jobs.job[j].b = static_cast<const uint16_t*>(p.b);
         jobs.job[j].c = p.c;
         jobs.job[j].addend = p.addend;
+        jobs.job[j].gu = static_cast<uint16_t*>(gu);
         jobs.job[j].lda = static_cast<int>(p.lda);
         jobs.job[j].ldb = static_cast<int>(p.ldb);
         jobs.job[j].ldc = static_cast<int>(p.ldc);
@@ -237,6 +280,11 @@ bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, 
         jobs.job[j].K = static_cast<int>(p.K);
     }
     const bool f32 = c_dtype == PK_F32, acc = beta != 0.0f;
+    if constexpr (MAX == 1) {
+        if (end == End::GATE) launch<false, false, false, End::GATE>(jobs, acc, st);
+        if (end == End::GATE_GRAD) launch<false, true, false, End::GATE_GRAD>(jobs, acc, st);
+        if (end != End::PLAIN) return true;
+    }
     if (tA)
         f32 ? launch<true, false, true>(jobs, acc, st) : launch<true, false, false>(jobs, acc, st);
     else if (tB)
@@ -250,6 +298,14 @@ bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, 
 bool gemm_small(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st) {
     if (count < 1 || count > 8 || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
     return count == 1 ? multiply<1>(ps, count, tA, tB, c_dtype, beta, st) : multiply<8>(ps, count, tA, tB, c_dtype, beta, st);
+}
+bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    const SmallProduct p{x, K, w, 2 * N, h, N, nullptr, M, N, K};
+    return multiply<1>(&p, 1, false, false, PK_BF16, 0.0f, st, End::GATE, gu);
+}
+bool gemm_small_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    const SmallProduct p{dy, K, w, K, dgu, 2 * N, nullptr, M, N, K};
+    return multiply<1>(&p, 1, false, true, PK_BF16, 0.0f, st, End::GATE_GRAD, const_cast<void*>(gu));
 }
 
 }  // namespace pk

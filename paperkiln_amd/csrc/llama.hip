@@ -279,7 +279,7 @@ struct Model {
         Var h2 = ops::rmsnorm(x1, b.ln2_w);
         // re-run at backward time, the block's own output is not needed again (the gradient arrives from outside): the
         // down projection is recorded but not multiplied
-        return ops::linear_add(ops::silu_mul_cat(ops::linear_cat(h2, {b.gate, b.up})), b.down, x1, !recomputing());
+        return ops::gated_mlp(h2, b.gate, b.up, b.down, x1, !recomputing());
     }
 
     // Llama::forward (llama.cpp:71-89) up to the final norm; positions restart per sequence.

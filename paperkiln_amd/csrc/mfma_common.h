@@ -259,6 +259,14 @@ __device__ inline u32x4 dma_rsrc(const void* p, uint32_t bytes) {
     return r;
 }
 
+// silu(g) u and its two derivatives times d (ops.cpp:404-423 with :76-83), for kernels that end or begin at a gated product
+__device__ inline float gated(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
+__device__ inline void gated_grad(float g, float u, float d, float& dg, float& du) {
+    const float s = 1.0f / (1.0f + expf(-g));
+    du = d * (g * s);
+    dg = (d * u) * (s * (1.0f + g * (1.0f - s)));
+}
+
 // XCD-aware workgroup -> tile mapping. The 256 CUs sit in 8 XCDs, each with
 // its own 4 MB L2, and consecutive workgroup ids go round-robin over the XCDs.
 // Every block of a (batch, KV head) unit re-reads that unit's K/V (or Q/dO),

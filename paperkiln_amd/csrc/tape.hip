@@ -474,6 +474,66 @@ Var linear(const Var& x, const Var& W) {
     });
 }
 
+namespace {
+// y = r + x W, the sum in the product's epilogue where the hand-written kernels take the operands
+void add_product(const Tensor& r, const Tensor& x, const Tensor& W, const Tensor& y) {
+    auto in_epilogue = [&] {
+        const int64_t M = y.rows, N = y.cols, K = x.cols;
+        if (gemm_backend() == 0 || x.dtype != W.dtype) return false;
+        if (x.dtype == PK_BF16)
+            return r.off_bytes % 16 == 0 && gemm_mfma_bf16(x.ptr(), false, K, W.ptr(), false, N, y.ptr(), y.dtype, M, N, K, N, 1.0f,
+                                                           tape_stream(), r.ptr());
+        const F32Product p{static_cast<const float*>(x.ptr()), K, static_cast<const float*>(W.ptr()), N,
+                           static_cast<float*>(y.ptr()), N, static_cast<const float*>(r.ptr()), M, N, K};
+        return gemm_f32_is_ahead(false, M, N, K) && gemm_f32(&p, 1, false, false, 0.0f, tape_stream());
+    };
+    if (in_epilogue()) return;
+    gemm(x, false, W, false, y.ptr(), y.dtype, y.rows, y.cols, y.cols, 0.0f);
+    k_add(r, y, y);
+}
+// the gradients of such a node: x's, then W's and r's
+void product_gradient(Variable* self) {
+    const Var& x = self->parents[0];
+    Tensor dx = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
+    gemm(self->grad, false, shadow_of(self->parents[1]), true, dx.ptr(), dx.dtype, dx.rows, dx.cols, dx.cols, 0.0f);
+    x->accumulate_owned(std::move(dx));
+}
+void product_weight_gradients(Variable* self) {
+    const Var& x = self->parents[0];
+    const Var& W = self->parents[1];
+    const Var& r = self->parents[2];
+    bool held = false;  // a held-back product still reads this node's gradient
+    if (W->requires_grad) {
+        held = defer_weight_gradient(x->data, self->grad, 0, W->data.cols, W);
+        if (!held) {
+            Tensor& g = W->ensure_grad();
+            gemm(x->data, true, self->grad, false, g.ptr(), g.dtype, g.rows, g.cols, g.cols, 1.0f);
+        }
+    }
+    if (r->requires_grad) {
+        const bool was_shared = self->grad_shared;  // the products above have read it; r takes the tensor itself
+        self->grad_shared = false;
+        r->accumulate_owned(std::move(self->grad), was_shared || held);
+    }
+}
+// For y = r + (silu(gate) .* up) W: the gradient of [gate | up] out of the product that forms the gated one's. False, with nothing
+// done, where the kernels do not take it.
+bool gated_gradient_in_product(const Tensor& dy, const Var& W, const Var& both) {
+    const Tensor& Wc = shadow_of(W);
+    const Tensor& gu = both->data;
+    const int64_t M = gu.rows, N = gu.cols / 2, K = dy.cols;
+    if (gemm_backend() == 0 || dy.dtype != gu.dtype || Wc.dtype != gu.dtype || !both->requires_grad) return false;
+    if (gu.dtype == PK_F32 && !gemm_f32_is_ahead(false, M, N, K)) return false;
+    Tensor d = Tensor::make(M, 2 * N, gu.dtype);
+    if (gu.dtype == PK_BF16 ? !gemm_mfma_gated_grad(dy.ptr(), Wc.ptr(), gu.ptr(), d.ptr(), M, N, K, tape_stream())
+                            : !gemm_f32_gated_grad(static_cast<const float*>(dy.ptr()), static_cast<const float*>(Wc.ptr()),
+                                                   static_cast<const float*>(gu.ptr()), static_cast<float*>(d.ptr()), M, N, K, tape_stream()))
+        return false;
+    both->accumulate_owned(std::move(d));
+    return true;
+}
+}  // namespace
+
 // y = r + x W: a Linear whose output joins a residual stream (o_proj and the MLP's down projection,
 // llama.cpp:47-59), the sum formed in the product's epilogue where the library's own GEMM takes the operands (one
 // rounding of r + x W instead of two, and no pass over y and r afterwards), by an add otherwise. One node with
@@ -484,48 +544,55 @@ Var linear_add(const Var& x, const Var& W, const Var& r, bool result_needed) {
         shape_fail("add: shape mismatch");
     const Tensor& Wc = shadow_of(W);
     Tensor y = Tensor::make(x->data.rows, W->data.cols, x->data.dtype);
-    auto in_epilogue = [&] {
-        const int64_t M = y.rows, N = y.cols, K = x->data.cols;
-        if (gemm_backend() == 0 || x->data.dtype != Wc.dtype) return false;
-        if (x->data.dtype == PK_BF16)
-            return r->data.off_bytes % 16 == 0 && gemm_mfma_bf16(x->data.ptr(), false, K, Wc.ptr(), false, N, y.ptr(), y.dtype, M,
-                                                                 N, K, N, 1.0f, tape_stream(), r->data.ptr());
-        const F32Product p{static_cast<const float*>(x->data.ptr()), K, static_cast<const float*>(Wc.ptr()), N,
-                           static_cast<float*>(y.ptr()), N, static_cast<const float*>(r->data.ptr()), M, N, K};
-        return gemm_f32_is_ahead(false, M, N, K) && gemm_f32(&p, 1, false, false, 0.0f, tape_stream());
-    };
     // result_needed = false: the caller only wants the node (the last op of a segment that is being re-run for its
     // tape: the backward closure reads x, W and the node's gradient, never the node's value), so nothing is multiplied
-    if (!result_needed && grad_enabled()) {
-        // y stays as allocated: its shape is what the tape needs
-    } else if (!in_epilogue()) {
-        gemm(x->data, false, Wc, false, y.ptr(), y.dtype, y.rows, y.cols, y.cols, 0.0f);
-        k_add(r->data, y, y);
-    }
+    // and y stays as allocated: its shape is what the tape needs
+    if (result_needed || !grad_enabled()) add_product(r->data, x->data, Wc, y);
     return record(std::move(y), {x, W, r}, [](Variable* self) {
-        const Var& x = self->parents[0];
-        const Var& W = self->parents[1];
-        const Var& r = self->parents[2];
-        if (x->requires_grad) {
-            Tensor dx = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
-            gemm(self->grad, false, shadow_of(W), true, dx.ptr(), dx.dtype, dx.rows, dx.cols, dx.cols, 0.0f);
-            x->accumulate_owned(std::move(dx));
-        }
-        bool held = false;  // a held-back product still reads this node's gradient
-        if (W->requires_grad) {
-            held = defer_weight_gradient(x->data, self->grad, 0, W->data.cols, W);
-            if (!held) {
-                Tensor& g = W->ensure_grad();
-                gemm(x->data, true, self->grad, false, g.ptr(), g.dtype, g.rows, g.cols, g.cols, 1.0f);
-            }
-        }
-        if (r->requires_grad) {
-            const bool was_shared = self->grad_shared;  // the products above have read it; r takes the tensor itself
-            self->grad_shared = false;
-            r->accumulate_owned(std::move(self->grad), was_shared || held);
-        }
+        if (self->parents[0]->requires_grad) product_gradient(self);
+        product_weight_gradients(self);
     });
 }
+
+namespace {
+// the gradients of y = x [W_0 | W_1 | ...] for that of y
+void cat_gradients(const Var& x, const std::vector<Var>& Ws, const Tensor& dy) {
+    const int n = static_cast<int>(Ws.size());
+    if (x->requires_grad) {  // dX = dY [W_0 | W_1 | ...]^T
+        Tensor dx = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
+        gemm(dy, false, shadow_cat(Ws), true, dx.ptr(), dx.dtype, dx.rows, dx.cols, dx.cols, 0.0f);
+        x->accumulate_owned(std::move(dx));
+    }
+    bool any = false;
+    for (const Var& W : Ws) any = any || W->requires_grad;
+    if (any) {  // held back, one product per weight, if every one of them can wait
+        bool all = true;
+        const int64_t d = Ws[0]->data.cols;
+        for (int k = 0; k < n; ++k)
+            all = all && (!Ws[k]->requires_grad || weight_gradient_can_wait(x->data, dy, k * d, d, Ws[k]));
+        if (all) {
+            for (int k = 0; k < n; ++k)
+                if (Ws[k]->requires_grad) hold_weight_gradient(x->data, dy, k * d, d, Ws[k]);
+            any = false;
+        }
+    }
+    if (any) {  // dW_k += X^T dY[:, block k]
+        float* dst[4] = {nullptr, nullptr, nullptr, nullptr};
+        std::vector<Tensor> unused;
+        for (int k = 0; k < n; ++k) {
+            if (Ws[k]->requires_grad) {
+                Tensor& g = Ws[k]->ensure_grad();
+                if (g.dtype != PK_F32) throw std::runtime_error("linear_cat: weight gradients must be fp32");
+                dst[k] = static_cast<float*>(g.ptr());
+            } else {
+                unused.push_back(Tensor::make(Ws[k]->data.rows, Ws[k]->data.cols, PK_F32));
+                dst[k] = static_cast<float*>(unused.back().ptr());
+            }
+        }
+        gemm_tn_split(x->data, dy, dst, n, 1.0f);
+    }
+}
+}  // namespace
 
 // y = x [W_0 | W_1 | ...]: several Linear layers that read the same input (q/k/v projections,
 // gate/up projections) as ONE GEMM against the column-wise concatenation of their weights, which
@@ -541,42 +608,8 @@ Var linear_cat(const Var& x, const std::vector<Var>& Ws) {
     gemm(x->data, false, shadow_cat(Ws), false, y.ptr(), y.dtype, N, n * d, n * d, 0.0f);
     std::vector<Var> parents{x};
     parents.insert(parents.end(), Ws.begin(), Ws.end());
-    return record(std::move(y), std::move(parents), [n](Variable* self) {
-        const Var& x = self->parents[0];
-        const std::vector<Var> Ws(self->parents.begin() + 1, self->parents.end());
-        if (x->requires_grad) {  // dX = dY [W_0 | W_1 | ...]^T
-            Tensor dx = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
-            gemm(self->grad, false, shadow_cat(Ws), true, dx.ptr(), dx.dtype, dx.rows, dx.cols, dx.cols, 0.0f);
-            x->accumulate_owned(std::move(dx));
-        }
-        bool any = false;
-        for (const Var& W : Ws) any = any || W->requires_grad;
-        if (any) {  // held back, one product per weight, if every one of them can wait
-            bool all = true;
-            const int64_t d = Ws[0]->data.cols;
-            for (int k = 0; k < n; ++k)
-                all = all && (!Ws[k]->requires_grad || weight_gradient_can_wait(x->data, self->grad, k * d, d, Ws[k]));
-            if (all) {
-                for (int k = 0; k < n; ++k)
-                    if (Ws[k]->requires_grad) hold_weight_gradient(x->data, self->grad, k * d, d, Ws[k]);
-                any = false;
-            }
-        }
-        if (any) {  // dW_k += X^T dY[:, block k]
-            float* dst[4] = {nullptr, nullptr, nullptr, nullptr};
-            std::vector<Tensor> unused;
-            for (int k = 0; k < n; ++k) {
-                if (Ws[k]->requires_grad) {
-                    Tensor& g = Ws[k]->ensure_grad();
-                    if (g.dtype != PK_F32) throw std::runtime_error("linear_cat: weight gradients must be fp32");
-                    dst[k] = static_cast<float*>(g.ptr());
-                } else {
-                    unused.push_back(Tensor::make(Ws[k]->data.rows, Ws[k]->data.cols, PK_F32));
-                    dst[k] = static_cast<float*>(unused.back().ptr());
-                }
-            }
-            gemm_tn_split(x->data, self->grad, dst, n, 1.0f);
-        }
+    return record(std::move(y), std::move(parents), [](Variable* self) {
+        cat_gradients(self->parents[0], std::vector<Var>(self->parents.begin() + 1, self->parents.end()), self->grad);
     });
 }
 
@@ -661,16 +694,60 @@ Var silu_mul(const Var& gate, const Var& up) {
     });
 }
 
+namespace {
+void silu_mul_cat_backward(Variable* self) {
+    const Var& gu = self->parents[0];
+    if (!gu->requires_grad) return;
+    Tensor dgu = Tensor::make(gu->data.rows, gu->data.cols, gu->data.dtype);
+    k_silu_mul_cat_bwd(gu->data, self->grad, dgu);
+    gu->accumulate_owned(std::move(dgu));
+}
+}  // namespace
+
 Var silu_mul_cat(const Var& gu) {
     if (gu->data.cols % 2 != 0) shape_fail("mul: shape mismatch");
     Tensor y = Tensor::make(gu->data.rows, gu->data.cols / 2, gu->data.dtype);
     k_silu_mul_cat_fwd(gu->data, y);
-    return record(std::move(y), {gu}, [](Variable* self) {
-        const Var& gu = self->parents[0];
-        if (!gu->requires_grad) return;
-        Tensor dgu = Tensor::make(gu->data.rows, gu->data.cols, gu->data.dtype);
-        k_silu_mul_cat_bwd(gu->data, self->grad, dgu);
-        gu->accumulate_owned(std::move(dgu));
+    return record(std::move(y), {gu}, silu_mul_cat_backward);
+}
+
+Var gated_mlp(const Var& x, const Var& gate, const Var& up, const Var& down, const Var& r, bool result_needed) {
+    const int64_t N = x->data.rows, ff = gate->data.cols, in = x->data.cols;
+    const int dtype = x->data.dtype;
+    if (gate->data.rows != in || up->data.rows != in || up->data.cols != ff || down->data.rows != ff)
+        shape_fail("matmul: inner dimensions disagree");
+    if (r->data.rows != N || r->data.cols != down->data.cols || r->data.dtype != dtype) shape_fail("add: shape mismatch");
+    // gate and up are kept where a backward pass will ask for them
+    const bool keep = grad_enabled() && (x->requires_grad || gate->requires_grad || up->requires_grad);
+    const Tensor& Wgu = shadow_cat({gate, up});
+    Tensor h = Tensor::make(N, ff, dtype), gu;
+    if (keep) gu = Tensor::make(N, 2 * ff, dtype);
+    const auto in_product = [&] {
+        if (gemm_backend() == 0 || Wgu.dtype != dtype) return false;
+        if (dtype == PK_BF16) return gemm_mfma_gated(x->data.ptr(), Wgu.ptr(), keep ? gu.ptr() : nullptr, h.ptr(), N, ff, in, tape_stream());
+        return gemm_f32_is_ahead(false, N, 2 * ff, in) &&
+               gemm_f32_gated(static_cast<const float*>(x->data.ptr()), static_cast<const float*>(Wgu.ptr()),
+                              keep ? static_cast<float*>(gu.ptr()) : nullptr, static_cast<float*>(h.ptr()), N, ff, in, tape_stream());
+    };
+    if (!in_product()) {
+        if (!keep) gu = Tensor::make(N, 2 * ff, dtype);
+        gemm(x->data, false, Wgu, false, gu.ptr(), dtype, N, 2 * ff, 2 * ff, 0.0f);
+        k_silu_mul_cat_fwd(gu, h);
+    }
+    Tensor y = Tensor::make(N, down->data.cols, dtype);
+    if (result_needed || !grad_enabled()) add_product(r->data, h, shadow_of(down), y);
+
+    // three nodes, as the ops by themselves would leave them
+    Var both;
+    if (keep)
+        both = record(std::move(gu), {x, gate, up}, [](Variable* self) {
+            cat_gradients(self->parents[0], {self->parents[1], self->parents[2]}, self->grad);
+        });
+    Var gated = keep ? record(std::move(h), {both}, silu_mul_cat_backward) : make_var(std::move(h), false);
+    return record(std::move(y), {gated, down, r}, [](Variable* self) {
+        const Var& gated = self->parents[0];
+        if (gated->requires_grad && !gated_gradient_in_product(self->grad, self->parents[1], gated->parents[0])) product_gradient(self);
+        product_weight_gradients(self);
     });
 }
 

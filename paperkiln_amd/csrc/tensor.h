@@ -148,6 +148,15 @@ struct F32Product {
 bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st);
 bool gemm_f32_is_ahead(bool tA, int64_t M, int64_t N, int64_t K);  // of the library, for one product of this size
 bool gemm_f32_held_is_ahead(int64_t M, int64_t N, int64_t K);      // the same for a weight gradient among several
+// SwiGLU inside the products beside it, row-major without gaps. *_gated: h [M, N] = silu(x gate) .* (x up) for x [M, K] and
+// w = [gate | up] [K, 2 N], and [x gate | x up] to gu unless that is null. *_gated_grad: d = dy w^T (dy [M, K], w [N, K]) is
+// the gradient of silu(gate) .* up; that of gu = [gate | up] goes to dgu. False, with nothing done, for what they do not take.
+bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_f32_gated_grad(const float* dy, const float* w, const float* gu, float* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_small_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
 int64_t gemm_head_spans(int64_t M, int64_t N);
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,

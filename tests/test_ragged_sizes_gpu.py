@@ -61,6 +61,21 @@ def test_bf16_training_with_any_vocabulary(vocab, d, ff, layers, tokens, seq):
         m.close()
 
 
+@pytest.mark.parametrize("d,ff,tokens,seq", [(64, 40, 33, 11), (96, 200, 1300, 130), (256, 1000, 2050, 410), (512, 1368, 700, 350),
+                                             (64, 4104, 8200, 820), (800, 304, 8200, 820)])
+def test_bf16_gated_product_in_its_projections(d, ff, tokens, seq):
+    """SwiGLU in the gate|up projection and in the down projection's dX, with and without gate and up being kept, against the passes
+    of their own beside the library's products: the kernel of few tiles, 128 x 128 and 256 x 256 tiles, a d_ff that ends inside
+    one, and a contraction (800) too long for the form, which takes those passes."""
+    test_bf16_training_with_any_vocabulary(130, d, ff, 1, tokens, seq)
+
+
+@pytest.mark.parametrize("d,ff,tokens,seq", [(64, 20, 33, 11), (64, 344, 2100, 420), (256, 250, 400, 100), (288, 256, 800, 100), (128, 90, 500, 100)])
+def test_fp32_gated_product_in_its_projections(d, ff, tokens, seq):
+    """The same in fp32, with each of its tiles."""
+    test_fp32_training_on_ragged_sizes(130, d, ff, tokens, seq)
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("vocab,d,ff,layers", [(130, 64, 176, 8), (37, 12, 20, 1), (37, 6, 10, 1)])
 def test_optimiser_step_writes_the_copies(vocab, d, ff, layers, dtype):
