@@ -1161,6 +1161,13 @@ __global__ void adamw_parts_k(AdamWParts ps, float* p, float* g, float* m, float
         *reinterpret_cast<u32x2*>(to) = u32x2{four[0] | static_cast<uint32_t>(four[1]) << 16, four[2] | static_cast<uint32_t>(four[3]) << 16};
     }
 }
+// What a training pass begins with, in one launch: its gradients cleared, and the host's n words fetched from pinned memory (first,
+// so that the link's round trip passes behind the clearing; a copy by the runtime is a kernel of its own of 4 us and more).
+__global__ void begin_pass_k(f32x4* clear, int64_t n4, const int* pinned, int* to, int64_t n) {
+    const int64_t first = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x, stride = static_cast<int64_t>(gridDim.x) * NT;
+    for (int64_t i = first; i < n; i += stride) to[i] = pinned[i];
+    for (int64_t i = first; i < n4; i += stride) clear[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+}
 __global__ void copy_word_k(const uint32_t* src, uint32_t* dst) { *dst = *src; }
 
 void same_shape(const Tensor& a, const Tensor& b, const char* who) {
@@ -1582,6 +1589,14 @@ double k_sumsq_to_host(const Tensor& g) {
 }
 void k_clip_factor(const double* part_dev, int n, float max_norm, float* factor_dev, float* norm_pinned) {
     hipLaunchKernelGGL(clip_factor_k, dim3(1), dim3(NT), 0, tape_stream(), part_dev, n, max_norm, factor_dev, norm_pinned);
+    post();
+}
+void k_begin_pass(const Tensor& clear, const int* pinned, int* to, int64_t n) {
+    const int64_t n4 = clear.numel() / 4;
+    if (clear.dtype != PK_F32 || clear.numel() % 4 || !aligned16p(clear.ptr())) throw std::runtime_error("begin_pass: whole 16-byte groups");
+    const int64_t blocks = std::min<int64_t>((std::max(n4, n) + NT - 1) / NT, 16384);
+    hipLaunchKernelGGL(begin_pass_k, dim3(static_cast<unsigned>(std::max<int64_t>(blocks, 1))), dim3(NT), 0, tape_stream(),
+                       static_cast<f32x4*>(clear.ptr()), n4, pinned, to, n);
     post();
 }
 void k_word_to_pinned(const void* src, void* pinned) {

@@ -472,15 +472,14 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         m->checkpoint_blocks = checkpoint_blocks != 0;
         const int64_t sl = seq_len == 0 ? n : seq_len;
         if (n % sl != 0) shape_fail("ids not a multiple of seq_len");
-        k_fill(m->gslab, 0.0f);  // zero_grad: every parameter's gradient is a view of this slab
-        // ids, targets and positions (which restart per sequence, llama.cpp:73-76) go up from pinned memory behind
-        // the fill, as one transfer and without a wait
+        // ids, targets and positions (which restart per sequence, llama.cpp:73-76) go up from pinned memory without a wait, with
+        // zero_grad: every parameter's gradient is a view of one slab
         int* st = m->staging(static_cast<size_t>(3 * n + 1));
         std::memcpy(st, host_ids, sizeof(int) * n);
         std::memcpy(st + n, host_targets, sizeof(int) * n);
         for (int64_t i = 0; i < n; ++i) st[2 * n + i] = static_cast<int>(i % sl);
         auto sent = std::make_shared<Buffer>(sizeof(int) * 3 * n);
-        hip_check(hipMemcpyAsync(sent->p, st, sizeof(int) * 3 * n, hipMemcpyHostToDevice, tape_stream()), "hipMemcpyAsync");
+        k_begin_pass(m->gslab, st, static_cast<int*>(sent->p), 3 * n);
         auto third = [&](int k) {  // a view that keeps the whole transfer's memory
             return std::shared_ptr<Buffer>(new Buffer(static_cast<int*>(sent->p) + k * n, sizeof(int) * n),
                                            [sent](Buffer* b) { delete b; });

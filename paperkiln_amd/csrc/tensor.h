@@ -71,6 +71,7 @@ double k_sum_f64_to_host(const double* part_dev, int64_t n);
 // What ops::clip_grad_norm multiplies the gradients by (1 where the norm is within max_norm), from those partial sums,
 // left on the device for k_adamw; the norm itself goes to pinned host memory, to be read after a wait for the stream.
 void k_clip_factor(const double* part_dev, int n, float max_norm, float* factor_dev, float* norm_pinned);
+void k_begin_pass(const Tensor& clear, const int* pinned, int* to, int64_t n);  // clear = 0 (fp32), to[i] = pinned[i]
 void k_word_to_pinned(const void* src, void* pinned);  // one float for the host, cheaper than a copy
 // clip_dev (may be null): g is scaled in place by *clip_dev first, in the same pass
 void k_adamw(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, float lr, float b1, float b2,
