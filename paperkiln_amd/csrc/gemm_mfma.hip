@@ -1373,8 +1373,30 @@ bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* d
 // [M_p, N_p] fp32 with row pitch ldc, one contraction length K for all. The products of a layer's backward pass
 // (X^T dY per weight, K = every token) are each a few dozen 128 x 128 tiles: alone each would cut its contraction into
 // slices to fill the chip and add the partial products afterwards; together their tiles fill it with whole
-// contractions. False, with nothing done, when an operand is not what the ring kernel takes or the tiles are too few
+// contractions; narrow layers' tiles do not, and then the launch cuts the common contraction and a second one adds the
+// slices. False, with nothing done, when an operand is not what the ring kernel takes or the tiles are too few
 // to be worth it (the caller then multiplies them one by one).
+namespace {
+struct GroupSums {
+    int count;
+    int end[GROUP_MAX];  // groups of four elements of problems 0 .. p
+    float* c[GROUP_MAX];
+    int N[GROUP_MAX], ldc[GROUP_MAX];
+};
+// C_p += the slices' partial products, part[s][problem after problem][M_p][N_p], added in slice order
+__global__ void sum_group(const float* part, int nparts, GroupSums gs) {
+    const int n4 = gs.end[gs.count - 1];
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n4; i += static_cast<int>(gridDim.x) * 256) {
+        int p = 0;
+        while (i >= gs.end[p]) ++p;
+        const int e = (i - (p > 0 ? gs.end[p - 1] : 0)) * 4, N = gs.N[p];
+        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k = 0; k < nparts; ++k) s += *reinterpret_cast<const f32x4*>(part + (static_cast<int64_t>(k) * n4 + i) * 4);
+        f32x4* const d = reinterpret_cast<f32x4*>(gs.c[p] + static_cast<int64_t>(e / N) * gs.ldc[p] + e % N);
+        *d += s;
+    }
+}
+}  // namespace
 bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStream_t st) {
     if (count < 2 || count > GROUP_MAX) return false;
     GroupArgs gr{};
@@ -1401,7 +1423,17 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
         gr.tile_end[p] = tiles;
     }
     for (int p = count; p < GROUP_MAX; ++p) gr.tile_end[p] = tiles;
-    if (g_force_geo < 0 && gemm_small_us(true, false, small, K) < (4.0 + 0.0105 * K) * ((tiles + cu_count() - 1) / cu_count())) {
+    // Slices of the contraction: as many as give every CU a (tile, slice), none shorter than 512. Microseconds of whole contractions and
+    // of slices with their sum, against the kernel of few tiles (a block's weights of width 192, d_ff 512, 5940 tokens: 36.2 us
+    // there, 17.5 + 4.9 in six slices; width 128, d_ff 344, 6754 tokens 24.5 and 12.3 + 5.9).
+    int64_t elements = 0;
+    for (int p = 0; p < count; ++p) elements += ps[p].M * ps[p].N;
+    int S = static_cast<int>(std::min<int64_t>({cu_count() / tiles, K / 512, 16}));
+    const int kps = S > 1 ? static_cast<int>(((K + S - 1) / S + BK - 1) / BK * BK) : static_cast<int>(K);
+    if (S > 1) S = static_cast<int>((K + kps - 1) / kps);
+    const double whole = (4.0 + 0.0105 * K) * ((tiles + cu_count() - 1) / cu_count());
+    const double sliced = S > 1 && elements < (int64_t{1} << 28) ? 7.5 + 0.0105 * kps + elements * (8.0 * S + 8.0) / 4.5e6 : 1e30;
+    if (g_force_geo < 0 && gemm_small_us(true, false, small, K) < std::min(whole, sliced)) {
         SmallProduct sp[GROUP_MAX];
         for (int p = 0; p < count; ++p)
             sp[p] = SmallProduct{ps[p].a, ps[p].lda, ps[p].b, ps[p].ldb, ps[p].c, ps[p].ldc, nullptr, ps[p].M, ps[p].N, K};
@@ -1410,11 +1442,39 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
     // worth it from about 3/8 of the CUs busy with whole contractions (measured: 196 tiles x 8192 in 69 us against 132
     // for the same four products one by one), and with any number of tiles where the contraction is short: a product of its
     // own is 10 us or more there, with a pass over its partial sums, and the grouped launch takes about 0.4 us for 64 tokens
-    if (tiles < cu_count() * 3 / 8 && K > 640 * count) return false;
+    const bool slices = g_force_geo < 0 && sliced < whole;
+    if (!slices && tiles < cu_count() * 3 / 8 && K > 640 * count) return false;
     GemmArgs g = gemm_args(ps[0].a, ps[0].lda, ps[0].b, ps[0].ldb, ps[0].M, ps[0].N, K);
     g.beta = 1;
     g.splits = 1;
     g.tiles_m = g.tiles_n = 0;
+    if (slices) {
+        Buffer part(sizeof(float) * static_cast<size_t>(S) * elements);
+        GroupSums gs{};
+        gs.count = count;
+        int64_t at = 0;
+        for (int p = 0; p < count; ++p) {
+            gs.c[p] = ps[p].c;
+            gs.N[p] = gr.N[p];
+            gs.ldc[p] = gr.ldc[p];
+            gr.c[p] = static_cast<float*>(part.p) + at;
+            gr.ldc[p] = gr.N[p];
+            at += ps[p].M * ps[p].N;
+            gs.end[p] = static_cast<int>(at / 4);
+        }
+        g.beta = 0;
+        g.splits = S;
+        g.k_per_split = kps;
+        g.part_stride = elements;
+        const int64_t vblocks = (static_cast<int64_t>(tiles) * S + 7) / 8 * 8;
+        hipLaunchKernelGGL((gemm_ring<GeoSmallK2, true, false, true, 4, true, 3>),
+                           dim3(static_cast<unsigned>(std::min<int64_t>(vblocks, cu_count() / 8 * 8))), dim3(GeoSmallK2::NTHR), 0, st, g, HeadArgs{}, gr);
+        hip_check(hipGetLastError(), "gemm_ring (grouped) launch");
+        hipLaunchKernelGGL(sum_group, dim3(static_cast<unsigned>(std::min<int64_t>((elements / 4 + 255) / 256, 4096))), dim3(256), 0, st,
+                           static_cast<const float*>(part.p), S, gs);
+        hip_check(hipGetLastError(), "sum_group launch");
+        return true;
+    }
     const int64_t vblocks = (static_cast<int64_t>(tiles) + 7) / 8 * 8;
     if (tiles <= cu_count()) {
         const unsigned gx = static_cast<unsigned>(std::min<int64_t>(vblocks, cu_count() / 8 * 8));

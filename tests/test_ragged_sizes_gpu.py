@@ -70,6 +70,13 @@ def test_bf16_gated_product_in_its_projections(d, ff, tokens, seq):
     test_bf16_training_with_any_vocabulary(130, d, ff, 1, tokens, seq)
 
 
+@pytest.mark.parametrize("d,ff,tokens,seq", [(192, 512, 5940, 135), (128, 344, 6754, 614), (96, 200, 3001, 3001), (64, 176, 16380, 819), (64, 40, 1024, 128)])
+def test_bf16_weight_gradients_in_slices(d, ff, tokens, seq):
+    """A narrow block's weight gradients over many tokens: one launch whose contraction is cut, the last slice shorter, and its sum; the
+    last case has too few tokens for two slices of 512 to pay."""
+    test_bf16_training_with_any_vocabulary(130, d, ff, 2, tokens, seq)
+
+
 @pytest.mark.parametrize("d,ff,tokens,seq", [(64, 20, 33, 11), (64, 344, 2100, 420), (256, 250, 400, 100), (288, 256, 800, 100), (128, 90, 500, 100)])
 def test_fp32_gated_product_in_its_projections(d, ff, tokens, seq):
     """The same in fp32, with each of its tiles."""
