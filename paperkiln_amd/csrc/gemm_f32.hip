@@ -244,7 +244,10 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
 // Which tile, by the number of 32 x 32 ones. A small tile keeps more CUs busy, a large one reads its operands less often. Measured
 // on projections, heads and weight gradients of 64 to 8192 tokens:
 //   More than 640 (2.5 to a CU): 64 x 64 (2048 x 1000 x 128: 10.4 us against 15.7), except for weight gradients, whose long
-//   contraction the small one walks with more wavefronts (512 x 1536 x 8192: 117 us against 152).
+//   contraction the small ones walk with more wavefronts (512 x 1536 x 8192: 117 us against 152). Theirs are 32 x 64, which cross
+//   the L2 three times for every four of 32 x 32, where they come to rounds that are full enough: above 768 (us, 32 x 32 | 32 x 64: 2048 x
+//   1536 x 1224 90 | 70, 896 x 896 x 1144 29 | 24, 1536 x 1152 x 1776 73 | 69; 512 x 1376 x 8192, 688 tiles, 134 | 150), and
+//   where they make one a CU, with eight wavefronts (768 x 576 x 6232 65 | 58, 640 x 640 x 896 13.2 | 11.7, 700 x 700 x 3000 37 | 29).
 //   Up to 64: 16 x 16, up to 128: 16 x 32, which makes a tile for each CU. A wavefront's loads and products for a chunk are a half or
 //   less (us, 32 x 32 with eight | 16 x 32 | 16 x 16 wavefronts: 512 x 128 x 688, B transposed 7.9 | 6.2 | 5.0; 512 x 128 x 344 5.4 |
 //   4.8 | 4.0; 512 x 256 x 688 7.8 | 6.0 | 6.6; 1024 x 128 x 688, B transposed 7.8 | 6.3 | 6.5).
@@ -261,6 +264,10 @@ void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     }
     if (tiles > 640 && (!TA || longest < 256))
         launch<TA, TB, 4, 4, 4, END>(jobs, beta, st);
+    else if (TA && longest >= 256 && tiles > 768)
+        launch<TA, TB, 2, 4, 4, END>(jobs, beta, st);
+    else if (TA && longest >= 256 && tiles > 320 && tiles <= 512)
+        launch<TA, TB, 2, 4, 8, END>(jobs, beta, st);
     else if (tiles <= 64 && END != End::GATE)
         launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END>(jobs, beta, st);
     else if (tiles <= 128 || (!TA && !TB && tiles > 256 && longest <= 256))

@@ -361,10 +361,11 @@ def test_fp32_products(M, N, K, tA, tB):
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
-@pytest.mark.parametrize("M,N,K", [(256, 255, 31), (257, 250, 129), (511, 241, 300), (513, 225, 255), (529, 240, 257), (500, 530, 256), (495, 545, 261)])
+@pytest.mark.parametrize("M,N,K", [(256, 255, 31), (257, 250, 129), (511, 241, 300), (513, 225, 255), (529, 240, 257), (500, 530, 256), (495, 545, 261),
+                                   (700, 580, 257), (900, 1030, 300)])
 def test_fp32_products_of_each_tile(M, N, K, tA, tB):
     """The same around the numbers of 32 x 32 tiles (64, 128, 256) and the lengths (256) at which its tile changes: 16 x 16,
-    16 x 32 and 32 x 32 with four and eight wavefronts. The bound: a sum of K products of standard normal numbers, each partial
+    16 x 32 and 32 x 32 with four and eight wavefronts, and for weight gradients 32 x 64 with each. The bound: a sum of K products of standard normal numbers, each partial
     sum rounded with a standard deviation of 2.4e-8 of its size sqrt(k), is off by 1.7e-8 K; five times that is below it
     up to K = 350."""
     test_fp32_products(M, N, K, tA, tB)
