@@ -361,14 +361,27 @@ def test_fp32_products(M, N, K, tA, tB):
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
-@pytest.mark.parametrize("M,N,K", [(256, 255, 31), (257, 250, 129), (511, 241, 300), (513, 225, 255), (529, 240, 257), (500, 530, 256), (495, 545, 261),
-                                   (700, 580, 257), (900, 1030, 300)])
+@pytest.mark.parametrize("M,N,K", [(256, 255, 31), (257, 250, 129), (511, 241, 300), (513, 225, 255), (529, 240, 257), (500, 530, 256), (495, 545, 261)])
 def test_fp32_products_of_each_tile(M, N, K, tA, tB):
     """The same around the numbers of 32 x 32 tiles (64, 128, 256) and the lengths (256) at which its tile changes: 16 x 16,
-    16 x 32 and 32 x 32 with four and eight wavefronts, and for weight gradients 32 x 64 with each. The bound: a sum of K products of standard normal numbers, each partial
+    16 x 32 and 32 x 32 with four and eight wavefronts. The bound: a sum of K products of standard normal numbers, each partial
     sum rounded with a standard deviation of 2.4e-8 of its size sqrt(k), is off by 1.7e-8 K; five times that is below it
     up to K = 350."""
     test_fp32_products(M, N, K, tA, tB)
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 580, 257), (900, 1030, 300), (513, 640, 1001)])
+def test_fp32_weight_gradients_of_wide_tiles(M, N, K):
+    """Weight gradients in tiles of 32 x 64, with four and eight wavefronts. The bound: a wavefront's chain is at most 126 sums, each
+    rounded with a standard deviation of 0.58 of 2^-24 of a partial sum, which is about a tenth of the sum of the terms' magnitudes
+    and seldom a third; five times sqrt(126) 0.58 / 3 of that is below 11."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b, c0 = (torch.randn(s, generator=gen, device="cuda") for s in ((K, M), (K, N), (M, N)))
+    for out in (None, c0.clone()):
+        got = blockops.matmul(a, b, trans_a=True, out=out)
+        base = 0 if out is None else c0.double()
+        room = 11 * 2.0 ** -24 * (a.abs().double().T @ b.abs().double() + (0 if out is None else c0.abs().double()))
+        assert ((got.double() - (a.double().T @ b.double() + base)).abs() <= room).all()
 
 
 @pytest.mark.parametrize("c_dtype", [torch.bfloat16, torch.float32], ids=str)
