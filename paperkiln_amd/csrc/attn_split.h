@@ -93,10 +93,15 @@ inline bool even_chains(const AttnArgs& a) { return !a.causal || chain_tokens(a)
 // block's chain through all of them, against the rest of the launch, two workgroups to a CU with a band of queries and about
 // three tiles of overhead each. (fp32, head_dim 64, T 2476, window 64, 4 sinks, 4 heads: 86 us with that chain.)
 // (bf16, head_dim 32, T 4213, window 1224, 16 sinks, 8 heads, blocks of 128 rows: 355 us with that chain, 146 with the tail dealt out.)
+// Where the heads of a group are dealt out a piece still walks all of them, the block its share: no use if that is no shorter (us, with
+// pieces | without: bf16, head_dim 128, T 615, 7 heads on one, window 25 64 | 24; T 517 x 2, window 68 47 | 26; fp32, head_dim 64, T 636,
+// 28 heads on 4, window 21 130 | 37; T 527 x 3, 7 on one 99 | 33).
 inline bool split_tail_pays(const AttnArgs& a, int head_split, int block_rows) {
     const SinkTail t = sink_tail(a.T, a.window, a.sinks);
     const int64_t blocks = static_cast<int64_t>((a.T + block_rows - 1) / block_rows) * a.Hkv * a.B * head_split;
-    return a.tail && t.nch > 0 && a.T - t.q0 > (blocks + 511) / 512 * (a.window + 128);
+    const int64_t left = a.T - t.q0, rep = a.Hq / a.Hkv, share = (rep + head_split - 1) / head_split;
+    return a.tail && t.nch > 0 && left > (blocks + 511) / 512 * (a.window + 128) &&
+           (share == rep || share * left > rep * (left < TAIL_CHUNK ? left : TAIL_CHUNK));
 }
 inline int tail_blocks(const AttnArgs& a) { return a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0; }
 

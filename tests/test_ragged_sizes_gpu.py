@@ -339,6 +339,17 @@ def test_sink_tail_of_the_split_kernels(case, dtype, dk):
     assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
 
 
+@pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float32, 64), (torch.float32, 48)], ids=str)
+@pytest.mark.parametrize("case", [(1, 615, 7, 1, 25, 16), (1, 636, 28, 4, 21, 16), (1, 1300, 14, 2, 114, 1), (3, 300, 7, 1, 20, 4)],
+                         ids=lambda c: "B%d_T%d_H%d_%d_w%d_s%d" % c)
+def test_sink_keys_of_groups_dealt_out(case, dtype, dk):
+    """Query heads of a group dealt to several workgroups under a band with sinks: whether the sink keys' block walks its heads' tail
+    itself or pieces of it go to others. Bounds as in the test above."""
+    B, T, Hq, Hkv, window, sinks = case
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, dtype, True, window, sinks))
+    assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
+
+
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 65, 31), (64, 32, 33), (31, 97, 344), (1, 40, 1001), (900, 1030, 70)])
 def test_fp32_products(M, N, K, tA, tB):
