@@ -104,7 +104,7 @@ size_t tail_bytes(const pk_attn_shape* s) {
 // (GQA only) the per-split partial dK / dV of the dK/dV launch, after delta and the sink tail
 int head_split_of(const pk_attn_shape* s) {
     const Mask m = effective_mask(s);
-    return gqa_head_split(s->B, s->T, s->Hq, s->Hkv, s->dk, s->causal != 0, m.window);
+    return gqa_head_split(s->B, s->T, s->Hq, s->Hkv, s->dk, s->causal != 0, m.window, m.sinks, s->dtype == PK_BF16);
 }
 // Whether the dK/dV launch goes to a kernel that splits so, asked of the dispatch itself. Only dimensions, mask and input
 // type of the shape count: the tensors are taken as aligned rows, a positive scale and fp32 gradients as given. Others take

@@ -107,6 +107,20 @@ __host__ inline bool sink_tail_pays(const SinkTail& t, int T, int window, int kv
                        ((128 + window) / step + prologue);
     return chain > rest;
 }
+// Launches under a band with 96 to 400 blocks of 32 keys fill the chip undealt; the block of the sink keys is then the longest chain,
+// whole or as pieces that walk every head of the group for up to TAIL_CHUNK queries. Dealt to `hs` workgroups its chain is that of its
+// share of the heads, and fp32 launches deal where that is seven tenths of a piece's at most (us, undealt | dealt: head_dim 128, T 1265,
+// 28 heads on 4, window 613 1047 | 344; T 994 x 2, window 45 545 | 267; 80, T 913 x 5, 7 on one, window 343 363 | 129; 64, T 1122 x 3,
+// window 108 119 | 59; past the line: 64, T 2970 x 2, 8 on 2, window 39 93 | 139; 48, T 2692 x 4, 7 on one, window 98 161 | 226). In
+// bf16 the unsplit kernels take most such shapes, without the deal, and are ahead in half of them (64, T 1986 x 3, 7 on one 39 | 69).
+__host__ __device__ inline int sink_head_split(int B, int T, int Hq, int Hkv, int window, int sinks) {
+    const SinkTail t = sink_tail(T, window, sinks);
+    const long long wgs = static_cast<long long>((T + 31) / 32) * B * Hkv, rep = Hq / Hkv, left = T - t.q0;
+    if (t.nch == 0 || left < (rep == 2 ? 512 : 256) || wgs >= 400) return 1;  // 32, T 478, 32 heads on 16, window 41: 20.8 | 22.2
+    const long long hs = 1600 / wgs < rep ? 1600 / wgs : rep;
+    const long long piece = rep * (left < TAIL_CHUNK ? left : TAIL_CHUNK);
+    return (rep + hs - 1) / hs * left * 10 <= piece * 7 ? static_cast<int>(hs) : 1;
+}
 // GQA head split. One dK/dV workgroup owns 128 keys of one (batch, KV head) and walks the query tiles of every
 // query head of the group in turn, so a launch has ceil(T/128) * B * Hkv workgroups (half that when causal
 // blocks are paired) however many query heads there are: 14 query heads on 2 KV heads at B = 4, T = 2048
@@ -116,13 +130,14 @@ __host__ inline bool sink_tail_pays(const SinkTail& t, int T, int window, int kv
 // and a second kernel adds the splits in order (no atomics, repeatable). The kernels of attn_split.hip and
 // attn_f32_split.hip split that way, band or not, and mfma_dkdv3 (band-free bf16); the others walk a group in one workgroup,
 // and a launch that goes to them needs no partial sums (bf16_deals_heads, f32_deals_heads).
-__host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window) {
+__host__ __device__ inline int gqa_head_split(int B, int T, int Hq, int Hkv, int dk, int causal, int window, int sinks, bool bf16) {
     const int rep = Hq / Hkv;
     if (rep <= 1 || dk % 4 != 0 || dk > 128) return 1;
     // with a band only the 32-key kernels split, and without the split they fill the chip with a quarter of the sequence
     const int nkb = window > 0 ? (T + 31) / 32 : (T + 127) / 128;
     const long long wgs = static_cast<long long>(causal && window == 0 ? (nkb + 1) / 2 : nkb) * B * Hkv;
-    if (wgs >= (window > 0 ? 96 : 384)) return 1;  // without a band: one and a half workgroups per CU
+    if (window > 0 && wgs >= 96) return bf16 ? 1 : sink_head_split(B, T, Hq, Hkv, window, sinks);
+    if (wgs >= 384) return 1;  // without a band: one and a half workgroups per CU
     const int hs = static_cast<int>((512 + wgs - 1) / wgs);
     return hs < rep ? hs : rep;
 }

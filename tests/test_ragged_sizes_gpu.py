@@ -350,6 +350,14 @@ def test_sink_keys_of_groups_dealt_out(case, dtype, dk):
     assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
 
 
+@pytest.mark.parametrize("B,T,Hq,Hkv,dk,window,sinks", [(1, 3050, 7, 1, 64, 1700, 32), (3, 1122, 7, 1, 64, 108, 4), (2, 540, 28, 4, 128, 27, 1),
+                                                        (5, 913, 7, 1, 80, 343, 1), (1, 600, 32, 8, 32, 70, 16), (12, 1055, 4, 1, 128, 33, 4)])
+def test_fp32_groups_dealt_out_for_their_sink_keys(B, T, Hq, Hkv, dk, window, sinks):
+    """Launches that fill the chip undealt, from 96 to 400 blocks of 32 keys. Bound as in the test above."""
+    e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.float32, True, window, sinks))
+    assert max(e) < 5e-6, e
+
+
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 65, 31), (64, 32, 33), (31, 97, 344), (1, 40, 1001), (900, 1030, 70)])
 def test_fp32_products(M, N, K, tA, tB):
