@@ -98,7 +98,13 @@ int pk_attn_bwd(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k
  * events: PK_BWD_DELTA (row sums D_i = sum_d O*dO into the workspace),
  * PK_BWD_DKDV (needs DELTA done), PK_BWD_DQ (needs DELTA done). On the
  * matrix-core paths DELTA | DQ in one call is a single kernel (dQ forms D_i for its own
- * rows and writes them), and pk_attn_bwd == that kernel followed by DKDV.
+ * rows and writes them). pk_attn_bwd is that kernel followed by DKDV, or, where both
+ * are a handful of workgroups, one launch of them together, whose sums may be taken in
+ * another order than those of the parts.
+ * dQ may lie where O does and dK and dV where K and V do, element for element: the
+ * kernels then run one after the other, dQ first, and a workgroup reads its rows of
+ * what it overwrites before it writes them. Results that overlap inputs in any other
+ * way are undefined.
  * The reference has no counterpart: its closure is a single host function
  * (src/ops.cpp:902-933). */
 enum { PK_BWD_DELTA = 1, PK_BWD_DKDV = 2, PK_BWD_DQ = 4, PK_BWD_ALL = 7 };

@@ -306,7 +306,7 @@ bool bf16_deals_heads(const AttnArgs& a) { return a.head_split > 1 && (split_dea
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
-    if (stages == PK_BWD_ALL && split_takes_bwd(a)) return launch_split_bwd(a, st);
+    if (stages == PK_BWD_ALL && !a.in_place && split_takes_bwd(a)) return launch_split_bwd(a, st);
     int rc = PK_OK;
     if (fused)
         rc = run_dq(a, true, st);

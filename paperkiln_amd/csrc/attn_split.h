@@ -105,7 +105,8 @@ inline bool split_tail_pays(const AttnArgs& a, int head_split, int block_rows) {
 }
 inline int tail_blocks(const AttnArgs& a) { return a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0; }
 
-// A backward whose dK/dV and dQ blocks of 32 rows go into one launch: the arguments of its dK/dV part, and the two kinds' ids. Heads
+// A backward whose dK/dV and dQ blocks of 32 rows go into one launch (no gradient where an input is, AttnArgs::in_place: each kind of block
+// reads what the other's would overwrite): the arguments of its dK/dV part, and the two kinds' ids. Heads
 // of a group are dealt out where the workspace holds their partial sums.
 struct OneLaunch {
     AttnArgs a;

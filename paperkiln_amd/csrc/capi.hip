@@ -132,6 +132,18 @@ int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
                const pk_tensor4* o, const float* lse, const pk_tensor4* d_o, const pk_tensor4* dq, const pk_tensor4* dk,
                const pk_tensor4* dv, void* workspace, size_t workspace_bytes, int stages, bool split_heads, void* stream);
 
+// The bytes from the first element of a tensor to past its last.
+struct Extent {
+    uintptr_t lo, hi;
+    Extent(const pk_tensor4* t, int B, int T, int H, int dk, int dtype) {
+        const int64_t es = dtype == PK_F32 ? 4 : 2, ends[] = {(B - 1) * t->stride_b, (T - 1) * t->stride_t, (H - 1) * t->stride_h};
+        int64_t first = 0, last = dk;
+        for (const int64_t e : ends) (e < 0 ? first : last) += e;
+        lo = reinterpret_cast<uintptr_t>(t->ptr) + first * es, hi = reinterpret_cast<uintptr_t>(t->ptr) + last * es;
+    }
+    bool meets(const Extent& o) const { return lo < o.hi && o.lo < hi; }
+};
+
 void fill_common(AttnArgs& a, const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
                  const pk_tensor4* v, const pk_tensor4* o) {
     std::memset(&a, 0, sizeof a);
@@ -257,6 +269,11 @@ int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
     a.dq = dq->ptr; a.dq_sb = dq->stride_b; a.dq_st = dq->stride_t; a.dq_sh = dq->stride_h;
     a.dk = dk->ptr; a.dk_sb = dk->stride_b; a.dk_st = dk->stride_t; a.dk_sh = dk->stride_h;
     a.dv = dv->ptr; a.dv_sb = dv->stride_b; a.dv_st = dv->stride_t; a.dv_sh = dv->stride_h;
+    const Extent in[] = {{q, s->B, s->T, s->Hq, s->dk, s->dtype},   {k, s->B, s->T, s->Hkv, s->dk, s->dtype}, {v, s->B, s->T, s->Hkv, s->dk, s->dtype},
+                         {o, s->B, s->T, s->Hq, s->dk, s->dtype},   {d_o, s->B, s->T, s->Hq, s->dk, s->dtype}},
+                 out[] = {{dq, s->B, s->T, s->Hq, s->dk, s->grad_dtype}, {dk, s->B, s->T, s->Hkv, s->dk, s->grad_dtype}, {dv, s->B, s->T, s->Hkv, s->dk, s->grad_dtype}};
+    for (const Extent& x : in)
+        for (const Extent& y : out) a.in_place = a.in_place || x.meets(y);
     const void* used[] = {q->ptr, k->ptr, v->ptr, o->ptr, lse, d_o->ptr, dq->ptr, dk->ptr, dv->ptr, workspace};
     for (const void* p : used) dev_touch(p, stream);
     a.delta = static_cast<float*>(workspace);

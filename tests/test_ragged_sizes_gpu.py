@@ -275,6 +275,28 @@ def test_backward_in_one_launch(case, dtype, dk):
     assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
 
 
+# A training loop that keeps no tensors it can do without: dQ where O was, dK and dV where K and V were. Small launches and large ones,
+# groups of heads dealt out, dealt sink tails, head sizes of every kernel family. The same bits as dQ and then dK/dV into buffers of
+# their own, which read what they read in this order.
+@pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 24), (torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float32, 20), (torch.float32, 64),
+                                      (torch.float32, 128)], ids=str)
+@pytest.mark.parametrize("case", [(1, 97, 4, 4, True, 0, 0), (2, 129, 7, 1, True, 0, 0), (1, 770, 2, 2, True, 64, 1), (3, 200, 4, 4, False, 0, 0),
+                                  (4, 1024, 8, 8, True, 0, 0), (16, 512, 8, 4, True, 0, 0), (8, 700, 16, 16, True, 100, 4)], ids=str)
+def test_gradients_in_the_place_of_inputs(case, dtype, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    q, k, v, d_o = (torch.randn((B, T, h, dk), generator=gen, device="cuda").to(dtype) for h in (Hq, Hkv, Hkv, Hq))
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    want = [torch.empty_like(x) for x in (q, k, v)]
+    ws = torch.empty(ops.bwd_workspace_bytes(q, k, window=window, sinks=sinks), dtype=torch.uint8, device="cuda")
+    for stages in (ops.BWD_DELTA | ops.BWD_DQ, ops.BWD_DKDV):
+        ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, out=(*want, ws), stages=stages)
+    got = ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, out=(o, k, v, ws))
+    assert all(a.data_ptr() == b.data_ptr() for a, b in zip(got, (o, k, v)))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 # bf16 at head_dim 64 in launches that fill the chip: rows owned by wavefronts, two or four to a workgroup, tiles of 32 and 64; lengths
 # around the tiles and blocks, the shortest that come here, bands with and without sinks (dealt out and left whole), dealt heads, no mask.
 @pytest.mark.parametrize("case", [(16, 512, 8, 8, True, 0, 0), (64, 65, 8, 8, True, 0, 0), (20, 399, 8, 8, True, 0, 0), (2, 2049, 14, 2, True, 0, 0),
