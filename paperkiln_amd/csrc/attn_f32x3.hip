@@ -28,7 +28,7 @@ __device__ inline float mul_rounded(float x, float y) {
 }
 
 // Two fp32 values as three packed bf16 pairs. The first part is cut off, not rounded, so that every finite value has one; an
-// infinity leaves no rest, and what it meets becomes NaN.
+// infinity leaves no rest and makes NaN of what it meets; rows that this reaches are formed again (below).
 __device__ inline void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
     const uint32_t u0 = __float_as_uint(x0) & 0xffff0000u, u1 = __float_as_uint(x1) & 0xffff0000u;
     h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // upper halves
@@ -236,6 +236,143 @@ __device__ inline float log_sum(float m, float scale, float off, float l) {
                               static_cast<double>(logf(__builtin_amdgcn_frexp_mantf(l))));
 }
 
+// ---- rows that are formed again ----
+// An infinity leaves no rest (it is inf, NaN, NaN), and products with weights of up to 2^6 or a long row's sum can leave fp32 where the
+// mean does not. All of these end in results that are not finite, and such rows are formed once more from the tensors themselves, one
+// key or query after the other as the scalar kernels do, over the visible ones only and with sums in 64 bits. A wavefront does this for
+// the rows it is about to store, whose accumulators then hold them; its lanes are the rows of the other side, 64 at a time, and then
+// the columns.
+
+// The kernel's arguments (AttnArgs is the first of them), read from memory where this is called: as the ones that the kernel has read
+// they would be held in scalar registers through its loop, which spilled 50 of them in dK/dV.
+__device__ inline AttnArgs arguments_again() {
+    uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(at));
+    return *(const AttnArgs*)(const __attribute__((address_space(4))) void*)at;
+}
+// Bit r: one of the results of row r (a lane of either half each) is not finite. ok: the lane's row exists and is stored; NB blocks,
+// of which this wavefront has every `step`-th from `first` on.
+template <int NB>
+__device__ inline uint32_t rows_not_finite(const f32x16* acc, bool ok, int first = 0, int step = 1) {
+    float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // stays 0 under finite values
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+        if (step == 1 || n % step == first)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[r & 3] = fmaf(acc[n][r], 0.0f, z[r & 3]);
+    const uint64_t lanes = __ballot(ok && !((z[0] + z[1]) + (z[2] + z[3]) == 0.0f));
+    return static_cast<uint32_t>(lanes | lanes >> 32);
+}
+__device__ inline float dot_exact(const float* x, const float* y, int dk) {
+    double sum = 0.0;
+#pragma unroll 1
+    for (int c = 0; c < dk; c += 4) {
+        const f32x4 u = *reinterpret_cast<const f32x4*>(x + c), v = *reinterpret_cast<const f32x4*>(y + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum += static_cast<double>(u[e]) * static_cast<double>(v[e]);
+    }
+    return static_cast<float>(sum);
+}
+// sum[0], sum[1] += weight(i) rows[i][lane], rows[i][lane + 64] over i in [i0, i1), 64 weights at a time, one to a lane; weight(i, w)
+// is false for an i that has none.
+template <class Weight>
+__device__ inline void add_weighted_rows(int i0, int i1, const float* rows, int64_t st, int dk, int lane, double (&sum)[2], Weight weight) {
+#pragma unroll 1
+    for (int base = i0; base < i1; base += 64) {
+        float w = 0.0f;
+        const bool has = base + lane < i1 && weight(base + lane, w);
+#pragma unroll 1
+        for (uint64_t left = __ballot(has); left != 0; left &= left - 1) {
+            const int at = __builtin_ctzll(left);
+            const double x = static_cast<double>(__shfl(w, at));
+            const float* row = rows + (base + at) * st;
+            if (lane < dk) sum[0] += x * static_cast<double>(row[lane]);
+            if (lane + 64 < dk) sum[1] += x * static_cast<double>(row[lane + 64]);
+        }
+    }
+}
+// Where a wavefront's row crosses LDS: the end of the kernel's, past the RED elements in which groups may still be joining their sums
+template <int D, int WAVES, int RED, int N>
+__device__ inline float* row_room(uint16_t (&lds)[N], int w) {
+    static_assert(N >= RED + 2 * WAVES * D, "room for a row a wavefront");
+    return reinterpret_cast<float*>(lds + N - 2 * WAVES * D) + w * D;
+}
+// A row of results, column by lane, into accumulators whose row it is
+template <int D, int NB>
+__device__ inline void put_row(float* buf, const double (&x)[2], int row, f32x16* acc, int lane, int db0 = 0) {
+    const int g = lane >> 5, c32 = lane & 31;
+    if (lane < D) buf[lane] = static_cast<float>(x[0]);
+    if (lane + 64 < D) buf[lane + 64] = static_cast<float>(x[1]);
+    tile_barrier<1>();
+    if (c32 == row) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            if (db0 + n >= D / 32) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[n][r] = buf[tr_col0<D>(db0 + n, r >> 2, g) + (r & 3)];
+        }
+    }
+    tile_barrier<1>();
+}
+// O and LSE of query qi
+__device__ inline void exact_o(const AttnArgs& a, int b, int h, int hk, int qi, int lane, double (&o)[2], float& lse) {
+    const float* q = static_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh + qi * a.q_st;
+    const float* k = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
+    const float* v = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
+    const int end = a.causal ? qi + 1 : a.T;
+    const auto visible = [&](int kj) { return pk_visible(qi, kj, a.T, a.causal, a.window, a.sinks); };
+    float m = -1e30f;
+    for (int kj = lane; kj < end; kj += 64)
+        if (visible(kj)) m = fmaxf(m, dot_exact(q, k + kj * a.k_st, a.dk_dim));
+#pragma unroll
+    for (int i = 32; i >= 1; i >>= 1) m = fmaxf(m, __shfl_xor(m, i));
+    double l = 0.0;
+    o[0] = o[1] = 0.0;
+    add_weighted_rows(0, end, v, a.v_st, a.dk_dim, lane, o, [&](int kj, float& w) {
+        if (!visible(kj)) return false;
+        w = __builtin_amdgcn_exp2f((dot_exact(q, k + kj * a.k_st, a.dk_dim) - m) * (a.scale * LOG2E));
+        l += static_cast<double>(w);
+        return true;
+    });
+#pragma unroll
+    for (int i = 32; i >= 1; i >>= 1) l += __shfl_xor(l, i);
+    o[0] /= l, o[1] /= l;
+    lse = log_sum(m, a.scale, 0.0f, static_cast<float>(l));
+}
+// dQ of query qi without its factor `scale`
+__device__ inline void exact_dq(const AttnArgs& a, int b, int h, int hk, int qi, float delta, int lane, double (&dq)[2]) {
+    const float* q = static_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh + qi * a.q_st;
+    const float* d_o = static_cast<const float*>(a.d_o) + b * a.do_sb + h * a.do_sh + qi * a.do_st;
+    const float* k = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
+    const float* v = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
+    const float nlse = -a.lse[lrow] * LOG2E;
+    dq[0] = dq[1] = 0.0;
+    add_weighted_rows(0, a.causal ? qi + 1 : a.T, k, a.k_st, a.dk_dim, lane, dq, [&](int kj, float& w) {
+        if (!pk_visible(qi, kj, a.T, a.causal, a.window, a.sinks)) return false;
+        const float p = __builtin_amdgcn_exp2f(fmaf(dot_exact(q, k + kj * a.k_st, a.dk_dim), a.scale * LOG2E, nlse));
+        w = p * (dot_exact(d_o, v + kj * a.v_st, a.dk_dim) - delta);
+        return true;
+    });
+}
+// dV (key_grad false) or dK without its factor `scale` of key kj, over queries [q0, q1) of heads [h0, h0 + nh)
+__device__ inline void exact_dkdv(const AttnArgs& a, bool key_grad, int b, int hk, int h0, int nh, int q0, int q1, int kj, int lane, double (&out)[2]) {
+    const float* k = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh + kj * a.k_st;
+    const float* v = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh + kj * a.v_st;
+    out[0] = out[1] = 0.0;
+    for (int h = h0; h < h0 + nh; ++h) {
+        const float* q = static_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh;
+        const float* d_o = static_cast<const float*>(a.d_o) + b * a.do_sb + h * a.do_sh;
+        const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T;
+        add_weighted_rows(q0, q1, key_grad ? q : d_o, key_grad ? a.q_st : a.do_st, a.dk_dim, lane, out, [&](int qi, float& w) {
+            if (!pk_visible(qi, kj, a.T, a.causal, a.window, a.sinks)) return false;
+            w = __builtin_amdgcn_exp2f(fmaf(dot_exact(q + qi * a.q_st, k, a.dk_dim), a.scale * LOG2E, -a.lse[lrow + qi] * LOG2E));
+            if (key_grad) w *= dot_exact(d_o + qi * a.do_st, v, a.dk_dim) - a.delta[lrow + qi];
+            return true;
+        });
+    }
+}
+
 // Tile buffers: two and one barrier a tile where a workgroup is one group, one and two barriers where two groups share the LDS.
 template <int D, int QW, int KW>
 constexpr int BUFS = KW == 1 && (D < 128 || QW > 4) ? 2 : 1;
@@ -349,13 +486,22 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
         join_groups<DB, KW>(acc, red, kg, lane);
         m = mt, l = lt, off = 0.0f;
     }
+    float inv = 1.0f / l, lse = log_sum(m, a.scale, off, l);
+    for (uint32_t again = rows_not_finite<DB>(acc, qi < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
+        const int row = __builtin_ctz(again);
+        double x[2];
+        float row_lse;
+        exact_o(arguments_again(), b, h, hk, qlo + row, lane, x, row_lse);
+        put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, lane);
+        if (c32 == row) inv = 1.0f, lse = row_lse;
+    }
+    if (a.in_place) __syncthreads();  // every row has been read
     if (qi < a.T) {
-        const float inv = 1.0f / l;
         const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
             if (KW == 1 || db % KW == kg) store_block32<D>(a.o, ro, db, g, acc[db], inv, dk);
-        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = log_sum(m, a.scale, off, l);
+        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = lse;
     }
 }
 
@@ -436,6 +582,13 @@ __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs 
         __syncthreads();
     }
     join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane);
+    for (uint32_t again = rows_not_finite<DB>(acc, qi < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
+        const int row = __builtin_ctz(again);
+        double x[2];
+        exact_dq(arguments_again(), b, h, hk, qlo + row, __shfl(dl, row), lane, x);
+        put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, lane);
+    }
+    if (a.in_place) __syncthreads();  // every row has been read
     if (qi < a.T) {
         const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
 #pragma unroll
@@ -602,8 +755,15 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
         loop(std::integral_constant<int, 1>{});
     // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
     // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
-    const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1);
-    if (kj < a.T && (chunk < 0 || to_tail)) {
+    const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1), stored = kj < a.T && (chunk < 0 || to_tail);
+    for (uint32_t again = rows_not_finite<DB>(acc, stored); __builtin_expect(again != 0, 0); again &= again - 1) {
+        const int row = __builtin_ctz(again);
+        double x[2];
+        exact_dkdv(arguments_again(), role == 1, b, hk, hk * rep + h0, nh, qt_lo * 32, q_end + 1, kw0 + row, lane, x);
+        put_row<D, DB>(row_room<D, 2 * QW, 0>(lds, w), x, row, acc, lane);
+    }
+    if (a.in_place) __syncthreads();  // every row has been read
+    if (stored) {
         const bool parts = hs > 1 && !to_tail;
         const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
                                    : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
@@ -708,6 +868,14 @@ __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta)
         loop(std::integral_constant<int, 0>{});
     else
         loop(std::integral_constant<int, 1>{});
+    // (role 1's last block is a copy of the one before where their number is odd; the rows' delta has been in memory since the first barrier)
+    for (uint32_t again = rows_not_finite<HB>(acc, qi < a.T); __builtin_expect(again != 0, 0); again &= again - 1) {
+        const int row = __builtin_ctz(again);
+        double x[2];
+        exact_dq(arguments_again(), b, h, hk, qlo + row, a.delta[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qlo + row], lane, x);
+        put_row<D, HB>(row_room<D, 2 * QW, 0>(lds, w), x, row, acc, lane, role * HB);
+    }
+    if (a.in_place) __syncthreads();  // every row has been read
     if (qi < a.T) {
         const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
 #pragma unroll

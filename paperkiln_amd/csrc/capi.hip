@@ -194,6 +194,9 @@ int pk_attn_fwd(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k
     AttnArgs a;
     fill_common(a, s, q, k, v, o);
     a.lse = lse;
+    const Extent eq(q, s->B, s->T, s->Hq, s->dk, s->dtype), ek(k, s->B, s->T, s->Hkv, s->dk, s->dtype), ev(v, s->B, s->T, s->Hkv, s->dk, s->dtype),
+        eo(o, s->B, s->T, s->Hq, s->dk, s->dtype);
+    a.in_place = eo.meets(eq) || eo.meets(ek) || eo.meets(ev);
     const void* used[] = {q->ptr, k->ptr, v->ptr, o->ptr, lse};
     for (const void* p : used) dev_touch(p, stream);
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -52,7 +52,7 @@ struct AttnArgs {
     int B, T, Hq, Hkv, dk_dim;
     int causal, window, sinks;
     int grad_f32; // dq/dk/dv element type: 1 = fp32, 0 = bf16
-    int in_place; // bwd: a gradient lies where an input does (or between its rows)
+    int in_place; // O (bwd: a gradient) lies where an input does, or between its rows
     float scale;
 };
 

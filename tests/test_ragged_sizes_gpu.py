@@ -250,6 +250,67 @@ def test_fp32_as_three_parts_over_the_range_of_fp32():
     assert float(d[good].max()) < 1e-6, d
 
 
+def seen(T, key, causal, window, sinks):
+    """Which queries see `key`, as a mask over [B, T, H, dk] tensors."""
+    i = torch.arange(T, device="cuda")
+    vis = (i >= key) if causal else torch.ones_like(i, dtype=torch.bool)
+    if window > 0 and key >= sinks:
+        vis = vis & (i < key + window)
+    return vis.view(1, T, 1, 1)
+
+
+# launches that take the three-part kernels: both forms, every padded head size, a band, groups of heads
+RANGE_CASES = [((24, 200, 8, 8, True, 0, 0), 64), ((5, 4096, 4, 4, True, 0, 0), 64), ((13, 511, 16, 8, False, 0, 0), 96), ((12, 383, 8, 8, True, 37, 5), 32),
+               ((20, 161, 11, 11, True, 0, 0), 128), ((7, 577, 16, 8, True, 0, 0), 44)]
+
+
+@pytest.mark.parametrize("case,dk", RANGE_CASES, ids=str)
+def test_three_parts_keep_infinities(case, dk):
+    """The reference's arithmetic over the visible keys (src/ops.cpp:879-932). A key whose scores are all -inf has no weight, and only dQ
+    shows it, in the column where it is infinite: 0 times inf. An infinite value makes its column of O infinite in the rows that see it
+    and in no others. Finite results to the bound of the test above."""
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    q, k, v, d_o = (torch.randn((B, T, h, dk), generator=gen, device="cuda") for h in (Hq, Hkv, Hkv, Hq))
+    q[..., 1] = -q[..., 1].abs() - 0.1
+    key, scale = T // 3, float(np.float32(1.0 / np.sqrt(dk)))
+    sees = seen(T, key, causal, window, sinks)
+    k_inf, k_zero = k.clone(), k.clone()
+    k_inf[:, key, :, 1], k_zero[:, key] = float("inf"), 0.0
+    o, lse = ops.attn_fwd(q, k_inf, v, scale, causal, window, sinks)
+    got = [o, lse, *ops.attn_bwd(q, k_inf, v, o, lse, d_o, scale, causal, window, sinks)]
+    want = list(exact_attention(q, k_inf, v, d_o, scale, causal, window, sinks))
+    want[2] = torch.where(sees, want[2], exact_attention(q, k_zero, v, d_o, scale, causal, window, sinks)[2])
+    assert torch.equal(torch.isnan(got[2][..., 1]), sees[..., 0].expand(B, T, Hq))
+    got[2], want[2] = (torch.where(sees & (torch.arange(dk, device="cuda") == 1), 0.0, x) for x in (got[2], want[2]))
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(got, want)]
+    assert max(e) < 1e-6, e
+
+    v_inf, v_zero = v.clone(), v.clone()
+    v_inf[:, key, :, 3], v_zero[:, key, :, 3] = float("inf"), 0.0
+    o, lse = ops.attn_fwd(q, k, v_inf, scale, causal, window, sinks)
+    want = exact_attention(q, k, v_zero, d_o, scale, causal, window, sinks)
+    there = sees & (torch.arange(dk, device="cuda") == 3)
+    assert bool((o == float("inf")).eq(there).all())
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip((torch.where(there, 0.0, o), lse), (torch.where(there, 0.0, want[0]), want[1]))]
+    assert max(e) < 1e-6, e
+
+
+@pytest.mark.parametrize("case,dk", RANGE_CASES, ids=str)
+def test_three_parts_hold_what_the_weights_keep_in_range(case, dk):
+    """Values up to the largest of fp32: O is a weighted mean of them, whatever their sum under weights of up to 2^6 would be, and
+    values past the largest bf16 have no rounded first part. Bound as above."""
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    q, k, d_o = (torch.randn((B, T, h, dk), generator=gen, device="cuda") for h in (Hq, Hkv, Hq))
+    v = torch.rand((B, T, Hkv, dk), generator=gen, device="cuda") * 3.4e38
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, _ = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    want = exact_attention(q, k, v * 2.0 ** -40, d_o, scale, causal, window, sinks)[0]
+    e = float((o.double() * 2.0 ** -40 - want).norm() / want.norm())
+    assert e < 1e-6, e
+
+
 # dQ and dK/dV in one launch against the two launches of the same call's stages: the forms, and so the order of the sums, may differ,
 # nothing else does. Few tiles and remainders, groups of heads dealt out and not, sink tails, the largest launches that go together.
 @pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 24), (torch.bfloat16, 64), (torch.bfloat16, 96), (torch.bfloat16, 128), (torch.float32, 20),
