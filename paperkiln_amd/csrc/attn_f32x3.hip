@@ -2,10 +2,12 @@
 //
 // A value is split into the bf16 next to it, the bf16 next to what that leaves, and the rest, which is a bf16 exactly: 8
 // significant bits each with signs of their own hold the 24 of an fp32 value. A product of two such values is nine products
-// of parts, of which the three smallest are at most 2^-26 of the whole and are left out; the other six are exact in
-// fp32 and are added in fp32 by the matrix unit, small ones first. Error of a 32 x 32 product of normal values against
-// float64, of the result's norm: 64 columns 4.6e-8 (v_mfma_f32_32x32x2_f32, which rounds its sum every second
-// column: 1.44e-7), 128 columns 6.1e-8 (2.0e-7). Parts below 2^-126 are lost, so that precision fades for values below 1e-33.
+// of parts, of which the three smallest are at most 2^-24 of the whole (2^-8 times 2^-17, twice; 5e-9 in the mean square) and are
+// left out; the other six are exact in fp32 and are added in fp32 by the matrix unit, small ones first. Error of scores against
+// float64, of the result's norm (in brackets v_mfma_f32_32x32x2_f32, which rounds its sum every second column): 1 column
+// 3.5e-8 (4.0e-8), 4 3.2e-8 (4.9e-8), 16 3.4e-8 (8.2e-8), 64 4.6e-8 (1.4e-7). A single product is off by 1.44e-7 at most, where
+// both factors are just above a power of two, and by 1.3e-7 elsewhere and on the fp32 instruction. Parts below 2^-126 are lost, so
+// that precision fades for values below 1e-33.
 //
 // What bounds it: the fp32 instruction does 157 TFLOP/s, and the kernels on it (attn_f32_split.hip) stood at 105 to 130; six
 // bf16 products for one take 3/8 of its clocks. Beside them stands the splitting, 5.5 vector instructions an element: a tile
@@ -27,12 +29,11 @@ __device__ inline float mul_rounded(float x, float y) {
     return x * y;
 }
 
-// Two fp32 values as three packed bf16 pairs. The first part is cut off, not rounded, so that every finite value has one; an
-// infinity leaves no rest and makes NaN of what it meets; rows that this reaches are formed again (below).
+// Two fp32 values as three packed bf16 pairs, each part rounded: a part cut off leaves a rest of up to 2^-7 of the value instead of
+// 2^-8, and the products left out are then up to 2^-22 of the whole (measured: 2.0e-7, rounded 5.0e-8), for as many instructions.
 __device__ inline void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
-    const uint32_t u0 = __float_as_uint(x0) & 0xffff0000u, u1 = __float_as_uint(x1) & 0xffff0000u;
-    h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // upper halves
-    x0 -= __uint_as_float(u0), x1 -= __uint_as_float(u1);
+    h = pack_bf16(x0, x1);
+    x0 -= __uint_as_float(h << 16), x1 -= __uint_as_float(h & 0xffff0000u);
     m = pack_bf16(x0, x1);
     x0 -= __uint_as_float(m << 16), x1 -= __uint_as_float(m & 0xffff0000u);
     l = pack_bf16(x0, x1);
@@ -237,8 +238,8 @@ __device__ inline float log_sum(float m, float scale, float off, float l) {
 }
 
 // ---- rows that are formed again ----
-// An infinity leaves no rest (it is inf, NaN, NaN), and products with weights of up to 2^6 or a long row's sum can leave fp32 where the
-// mean does not. All of these end in results that are not finite, and such rows are formed once more from the tensors themselves, one
+// An infinity leaves no rest (it is inf, NaN, NaN), a value past the largest bf16 rounds to one, and products with weights of up to 2^6
+// or a long row's sum can leave fp32 where the mean does not. All of these end in results that are not finite, and such rows are formed once more from the tensors themselves, one
 // key or query after the other as the scalar kernels do, over the visible ones only and with sums in 64 bits. A wavefront does this for
 // the rows it is about to store, whose accumulators then hold them; its lanes are the rows of the other side, 64 at a time, and then
 // the columns.

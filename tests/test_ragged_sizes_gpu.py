@@ -311,6 +311,21 @@ def test_three_parts_hold_what_the_weights_keep_in_range(case, dk):
     assert e < 1e-6, e
 
 
+def test_three_parts_round_single_products_as_fp32_does():
+    """Scores of one product each, and rows that see one key (a window of one): LSE is that product. A product of three parts leaves out
+    2^-8 x 2^-17 of it twice and 2^-34; the sum of the others is off by a unit of its last place at most, 2^-23. The factors are near
+    the powers of two, where what is left out weighs most (general ones on the fp32 instruction: 1.3e-7)."""
+    B, T, H, dk = 4, 1024, 8, 64
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.zeros((B, T, H, dk), device="cuda") for _ in range(3))
+    q[..., 5] = (1 + 0.1 * torch.rand((B, T, H), generator=gen, device="cuda")) * 1024
+    k[..., 5] = -(1 + 0.1 * torch.rand((B, T, H), generator=gen, device="cuda")) * 1024
+    _, lse = ops.attn_fwd(q, k, v, 1.0, True, 1, 0)
+    want = (q[..., 5].double() * k[..., 5].double()).permute(0, 2, 1)
+    e = float(((lse.double() - want) / want).abs().max())
+    assert e <= (3 + 2.0 ** -9) * 2.0 ** -24, e
+
+
 # dQ and dK/dV in one launch against the two launches of the same call's stages: the forms, and so the order of the sums, may differ,
 # nothing else does. Few tiles and remainders, groups of heads dealt out and not, sink tails, the largest launches that go together.
 @pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 24), (torch.bfloat16, 64), (torch.bfloat16, 96), (torch.bfloat16, 128), (torch.float32, 20),
