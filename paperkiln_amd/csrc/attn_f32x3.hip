@@ -6,8 +6,8 @@
 // left out; the other six are exact in fp32 and are added in fp32 by the matrix unit, small ones first. Error of scores against
 // float64, of the result's norm (in brackets v_mfma_f32_32x32x2_f32, which rounds its sum every second column): 1 column
 // 3.5e-8 (4.0e-8), 4 3.2e-8 (4.9e-8), 16 3.4e-8 (8.2e-8), 64 4.6e-8 (1.4e-7). A single product is off by 1.44e-7 at most, where
-// both factors are just above a power of two, and by 1.3e-7 elsewhere and on the fp32 instruction. Parts below 2^-126 are lost, so
-// that precision fades for values below 1e-33.
+// both factors are just above a power of two, and by 1.3e-7 elsewhere and on the fp32 instruction. Parts below 2^-126 are lost:
+// rows_to_redo.
 //
 // What bounds it: the fp32 instruction does 157 TFLOP/s, and the kernels on it (attn_f32_split.hip) stood at 105 to 130; six
 // bf16 products for one take 3/8 of its clocks. Beside them stands the splitting, 5.5 vector instructions an element: a tile
@@ -239,10 +239,14 @@ __device__ inline float log_sum(float m, float scale, float off, float l) {
 
 // ---- rows that are formed again ----
 // An infinity leaves no rest (it is inf, NaN, NaN), a value past the largest bf16 rounds to one, and products with weights of up to 2^6
-// or a long row's sum can leave fp32 where the mean does not. All of these end in results that are not finite, and such rows are formed once more from the tensors themselves, one
-// key or query after the other as the scalar kernels do, over the visible ones only and with sums in 64 bits. A wavefront does this for
-// the rows it is about to store, whose accumulators then hold them; its lanes are the rows of the other side, 64 at a time, and then
-// the columns.
+// or a long row's sum can leave fp32 where the mean does not. All of these end in results that are not finite, and such rows are
+// formed once more from the tensors themselves, one key or query after the other as the scalar kernels do, over the visible ones only
+// and with sums in 64 bits. A wavefront does this for the rows it is about to store, whose accumulators then hold them; its lanes are
+// the rows of the other side, 64 at a time, and then the columns. What the test costs where it finds nothing, over 24 shapes: forward
+// 0.998, dQ 1.006, dK/dV 1.009 of the time without it.
+//
+// The last parts of values below 1e-33 are below the range of bf16. Beside others they do not count, and where everything is that
+// small the results are: rows of a wavefront whose results are all below 2^-96, and not all zero, are formed again as well.
 
 // The kernel's arguments (AttnArgs is the first of them), read from memory where this is called: as the ones that the kernel has read
 // they would be held in scalar registers through its loop, which spilled 50 of them in dK/dV.
@@ -251,17 +255,21 @@ __device__ inline AttnArgs arguments_again() {
     asm volatile("" : "+s"(at));
     return *(const AttnArgs*)(const __attribute__((address_space(4))) void*)at;
 }
-// Bit r: one of the results of row r (a lane of either half each) is not finite. ok: the lane's row exists and is stored; NB blocks,
-// of which this wavefront has every `step`-th from `first` on.
+// The lane once more, without a register that holds it through the loop
+__device__ inline int lane_again() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+// Bit r: row r (a lane of either half each) is one of those. ok: the lane's row exists and is stored; NB blocks, of which this
+// wavefront has every `step`-th from `first` on; sc: the factor they are stored with, or a power of two or so from it.
 template <int NB>
-__device__ inline uint32_t rows_not_finite(const f32x16* acc, bool ok, int first = 0, int step = 1) {
-    float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // stays 0 under finite values
+__device__ inline uint32_t rows_to_redo(const f32x16* acc, float sc, bool ok, int first = 0, int step = 1) {
+    float z[4] = {0.0f, 0.0f, 0.0f, 0.0f}, top[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // z stays 0 under finite values
 #pragma unroll
     for (int n = 0; n < NB; ++n)
         if (step == 1 || n % step == first)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) z[r & 3] = fmaf(acc[n][r], 0.0f, z[r & 3]);
-    const uint64_t lanes = __ballot(ok && !((z[0] + z[1]) + (z[2] + z[3]) == 0.0f));
+            for (int r = 0; r < 16; ++r) z[r & 3] = fmaf(acc[n][r], 0.0f, z[r & 3]), top[r & 3] = fmaxf(top[r & 3], fabsf(acc[n][r]));
+    const float t = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
+    uint64_t lanes = __ballot(ok && !((z[0] + z[1]) + (z[2] + z[3]) == 0.0f));
+    if (__ballot(ok && t * sc >= 0x1p-96f) == 0) lanes |= __ballot(ok && t > 0.0f);
     return static_cast<uint32_t>(lanes | lanes >> 32);
 }
 __device__ inline float dot_exact(const float* x, const float* y, int dk) {
@@ -462,47 +470,48 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
         __syncthreads();
     }
 
+    const int le = lane_again(), ge = le >> 5, ce = le & 31, qe = qlo + ce;
     float l = xhalf_sum(static_cast<float>(lsum));
     float off = fmaf(m, cexp, -mc);  // what the rounding of mc left out
     if (KW > 1) {
         // the groups' running maxima and sums meet, then their accumulators scaled to the common maximum
         float* red = reinterpret_cast<float*>(lds) + qg * KW * (DB * 1024 + 128);
         float* ml = red + KW * DB * 1024;
-        ml[kg * 128 + lane] = m;
-        ml[kg * 128 + 64 + lane] = l;
+        ml[kg * 128 + le] = m;
+        ml[kg * 128 + 64 + le] = l;
         __syncthreads();
         float mt = m, lt = 0.0f;
 #pragma unroll
-        for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
+        for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + le]);
 #pragma unroll
         for (int k = 0; k < KW; ++k) {
-            const float mk = ml[k * 128 + lane];
-            lt += ml[k * 128 + 64 + lane] * __builtin_amdgcn_exp2f(fmaf(mk - mt, cexp, -fmaf(mk, cexp, -mul_rounded(mk, cexp))));
+            const float mk = ml[k * 128 + le];
+            lt += ml[k * 128 + 64 + le] * __builtin_amdgcn_exp2f(fmaf(mk - mt, cexp, -fmaf(mk, cexp, -mul_rounded(mk, cexp))));
         }
         const float alpha = __builtin_amdgcn_exp2f(fmaf(m - mt, cexp, -off));
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
-        join_groups<DB, KW>(acc, red, kg, lane);
+        join_groups<DB, KW>(acc, red, kg, le);
         m = mt, l = lt, off = 0.0f;
     }
     float inv = 1.0f / l, lse = log_sum(m, a.scale, off, l);
-    for (uint32_t again = rows_not_finite<DB>(acc, qi < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
+    for (uint32_t again = rows_to_redo<DB>(acc, inv, qe < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
         const int row = __builtin_ctz(again);
         double x[2];
         float row_lse;
-        exact_o(arguments_again(), b, h, hk, qlo + row, lane, x, row_lse);
-        put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, lane);
-        if (c32 == row) inv = 1.0f, lse = row_lse;
+        exact_o(arguments_again(), b, h, hk, qlo + row, le, x, row_lse);
+        put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, le);
+        if (ce == row) inv = 1.0f, lse = row_lse;
     }
     if (a.in_place) __syncthreads();  // every row has been read
-    if (qi < a.T) {
-        const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+    if (qe < a.T) {
+        const int64_t ro = b * a.o_sb + h * a.o_sh + qe * a.o_st;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
-            if (KW == 1 || db % KW == kg) store_block32<D>(a.o, ro, db, g, acc[db], inv, dk);
-        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = lse;
+            if (KW == 1 || db % KW == kg) store_block32<D>(a.o, ro, db, ge, acc[db], inv, dk);
+        if (ge == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qe] = lse;
     }
 }
 
@@ -582,19 +591,20 @@ __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs 
         if (i + 1 < iters) commit(i + 1);
         __syncthreads();
     }
-    join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane);
-    for (uint32_t again = rows_not_finite<DB>(acc, qi < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
+    const int le = lane_again(), ge = le >> 5, qe = qlo + (le & 31);
+    join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, le);
+    for (uint32_t again = rows_to_redo<DB>(acc, 1.0f, qe < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
         const int row = __builtin_ctz(again);
         double x[2];
-        exact_dq(arguments_again(), b, h, hk, qlo + row, __shfl(dl, row), lane, x);
-        put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, lane);
+        exact_dq(arguments_again(), b, h, hk, qlo + row, __shfl(dl, row), le, x);
+        put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, le);
     }
     if (a.in_place) __syncthreads();  // every row has been read
-    if (qi < a.T) {
-        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+    if (qe < a.T) {
+        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qe * a.dq_st;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
-            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, g, acc[db], a.scale, dk);
+            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, ge, acc[db], a.scale, dk);
     }
 }
 
@@ -757,7 +767,7 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
     // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
     // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
     const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1), stored = kj < a.T && (chunk < 0 || to_tail);
-    for (uint32_t again = rows_not_finite<DB>(acc, stored); __builtin_expect(again != 0, 0); again &= again - 1) {
+    for (uint32_t again = rows_to_redo<DB>(acc, 1.0f, stored); __builtin_expect(again != 0, 0); again &= again - 1) {
         const int row = __builtin_ctz(again);
         double x[2];
         exact_dkdv(arguments_again(), role == 1, b, hk, hk * rep + h0, nh, qt_lo * 32, q_end + 1, kw0 + row, lane, x);
@@ -869,19 +879,20 @@ __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta)
         loop(std::integral_constant<int, 0>{});
     else
         loop(std::integral_constant<int, 1>{});
+    const int le = lane_again(), ge = le >> 5, qe = qlo + (le & 31);
     // (role 1's last block is a copy of the one before where their number is odd; the rows' delta has been in memory since the first barrier)
-    for (uint32_t again = rows_not_finite<HB>(acc, qi < a.T); __builtin_expect(again != 0, 0); again &= again - 1) {
+    for (uint32_t again = rows_to_redo<HB>(acc, 1.0f, qe < a.T); __builtin_expect(again != 0, 0); again &= again - 1) {
         const int row = __builtin_ctz(again);
         double x[2];
-        exact_dq(arguments_again(), b, h, hk, qlo + row, a.delta[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qlo + row], lane, x);
-        put_row<D, HB>(row_room<D, 2 * QW, 0>(lds, w), x, row, acc, lane, role * HB);
+        exact_dq(arguments_again(), b, h, hk, qlo + row, a.delta[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qlo + row], le, x);
+        put_row<D, HB>(row_room<D, 2 * QW, 0>(lds, w), x, row, acc, le, role * HB);
     }
     if (a.in_place) __syncthreads();  // every row has been read
-    if (qi < a.T) {
-        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+    if (qe < a.T) {
+        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qe * a.dq_st;
 #pragma unroll
         for (int db = 0; db < HB; ++db)
-            if (role * HB + db < DB) store_block32<D>(a.dq, ro, role * HB + db, g, acc[db], a.scale, dk);
+            if (role * HB + db < DB) store_block32<D>(a.dq, ro, role * HB + db, ge, acc[db], a.scale, dk);
     }
 }
 

@@ -326,6 +326,21 @@ def test_three_parts_round_single_products_as_fp32_does():
     assert e <= (3 + 2.0 ** -9) * 2.0 ** -24, e
 
 
+@pytest.mark.parametrize("tiny", ["v", "d_o", "k"])
+@pytest.mark.parametrize("case,dk", RANGE_CASES, ids=str)
+def test_three_parts_of_tiny_tensors(case, dk, tiny):
+    """Values below 1e-33, whose last parts are below the range of bf16: results as exact as of others. Bound as above."""
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    x = {n: torch.randn((B, T, h, dk), generator=gen, device="cuda") for n, h in (("q", Hq), ("k", Hkv), ("v", Hkv), ("d_o", Hq))}
+    x[tiny] *= 2.0 ** -120
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(x["q"], x["k"], x["v"], scale, causal, window, sinks)
+    got = (o, lse, *ops.attn_bwd(x["q"], x["k"], x["v"], o, lse, x["d_o"], scale, causal, window, sinks))
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(got, exact_attention(x["q"], x["k"], x["v"], x["d_o"], scale, causal, window, sinks))]
+    assert max(e) < 1e-6, e
+
+
 # dQ and dK/dV in one launch against the two launches of the same call's stages: the forms, and so the order of the sums, may differ,
 # nothing else does. Few tiles and remainders, groups of heads dealt out and not, sink tails, the largest launches that go together.
 @pytest.mark.parametrize("dtype,dk", [(torch.bfloat16, 24), (torch.bfloat16, 64), (torch.bfloat16, 96), (torch.bfloat16, 128), (torch.float32, 20),
