@@ -81,8 +81,10 @@ __device__ inline void load_short(const float* p, int64_t ld, const int (&idx)[N
 __host__ __device__ inline int64_t extent(int64_t rows, int64_t cols, int64_t ld) { return ((rows - 1) * ld + cols) * 4; }
 __device__ inline int bytes_of(int rows, int cols, int64_t ld) { return static_cast<int>(extent(rows, cols, ld)); }
 
-// A workgroup's tile is MB x NB blocks of 16 x 16; its KW wavefronts split the contraction chunk by chunk.
-template <bool TA, bool TB, int MB, int NB, int KW, int MAX, End END>
+// A workgroup's tile is MB x NB blocks of 16 x 16; its KW wavefronts split the contraction chunk by chunk. SUMS 2: a wavefront has two
+// sums, of every other step of a chunk, so that four wavefronts' chains of additions, with which a sum's error grows, are as short
+// as eight wavefronts' (at the sizes named below no slower: 4.69 us | 4.68, 3.78 | 3.80, 5.72 | 5.75, 5.87 | 5.88 with one | two).
+template <bool TA, bool TB, int MB, int NB, int KW, int SUMS, int MAX, End END>
 __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta) {
     constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB;
     constexpr int HALF = END == End::GATE ? NB / 2 : NB, TN = 16 * HALF;  // blocks of columns of C
@@ -104,11 +106,13 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 #pragma unroll
     for (int i = 0; i < NB; ++i) col[i] = min(n0 + i % HALF * 16 + l16, N - 1) + (i >= HALF ? N : 0);
 
-    f32x4 acc[MB][NB];
+    f32x4 acc[SUMS][MB][NB];
 #pragma unroll
-    for (int x = 0; x < MB; ++x)
+    for (int i = 0; i < SUMS; ++i)
 #pragma unroll
-        for (int y = 0; y < NB; ++y) acc[x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int x = 0; x < MB; ++x)
+#pragma unroll
+            for (int y = 0; y < NB; ++y) acc[i][x][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a), 0, bytes_of(TA ? K : M, TA ? M : K, lda), 0x00020000);
     const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(b), 0, bytes_of(TB ? N : K, TB ? K : END == End::GATE ? 2 * N : N, ldb), 0x00020000);
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
             for (int x = 0; x < MB; ++x)
 #pragma unroll
                 for (int y = 0; y < NB; ++y)
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[buf][x][s], fb[buf][y][s], acc[x][y], 0, 0, 0);
+                    acc[s % SUMS][x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[buf][x][s], fb[buf][y][s], acc[s % SUMS][x][y], 0, 0, 0);
     };
     const int mine = kw < chunks ? (chunks - kw + KW - 1) / KW : 0;  // chunks kw, kw + KW, ... are this wavefront's
 #pragma unroll
@@ -205,7 +209,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 #pragma unroll
     for (int x = 0; x < MB; ++x)
 #pragma unroll
-        for (int y = 0; y < NB; ++y) part[kw][x * NB + y][lane] = acc[x][y];
+        for (int y = 0; y < NB; ++y) part[kw][x * NB + y][lane] = SUMS > 1 ? acc[0][x][y] + acc[SUMS - 1][x][y] : acc[0][x][y];
     __syncthreads();
 #pragma unroll
     for (int g0 = 0; g0 < MB * HALF; g0 += KW) {
@@ -227,7 +231,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
     }
 }
 
-template <bool TA, bool TB, int MB, int NB, int KW, End END, int MAX>
+template <bool TA, bool TB, int MB, int NB, int KW, End END, int SUMS = 1, int MAX>
 void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     constexpr int TM = 16 * MB, TN = 16 * (END == End::GATE ? NB / 2 : NB);
     int tiles = 0;
@@ -236,7 +240,7 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
         tiles += ((jobs.job[j].M + TM - 1) / TM) * ((jobs.job[j].N + TN - 1) / TN);
     }
     for (int j = jobs.count; j <= MAX; ++j) jobs.first[j] = tiles;
-    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, MAX, END>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
+    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, SUMS, MAX, END>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
                        tiles, beta);
     hip_check(hipGetLastError(), "gemm_f32");
 }
@@ -248,7 +252,7 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
 //   the L2 three times for every four of 32 x 32, where they come to rounds that are full enough: above 768 (us, 32 x 32 | 32 x 64: 2048 x
 //   1536 x 1224 90 | 70, 896 x 896 x 1144 29 | 24, 1536 x 1152 x 1776 73 | 69; 512 x 1376 x 8192, 688 tiles, 134 | 150), and
 //   where they make one a CU, with eight wavefronts (768 x 576 x 6232 65 | 58, 640 x 640 x 896 13.2 | 11.7, 700 x 700 x 3000 37 | 29).
-//   Up to 64: 16 x 16, up to 128: 16 x 32, which makes a tile for each CU. A wavefront's loads and products for a chunk are a half or
+//   Up to 64: 16 x 16, up to 128: 16 x 32, which makes a tile for each CU, in two sums a wavefront. A wavefront's loads and products for a chunk are a half or
 //   less (us, 32 x 32 with eight | 16 x 32 | 16 x 16 wavefronts: 512 x 128 x 688, B transposed 7.9 | 6.2 | 5.0; 512 x 128 x 344 5.4 |
 //   4.8 | 4.0; 512 x 256 x 688 7.8 | 6.0 | 6.6; 1024 x 128 x 688, B transposed 7.8 | 6.3 | 6.5).
 //   In between 32 x 32; eight wavefronts split the contraction where it is long and there is a tile or less to a CU. Short
@@ -269,8 +273,10 @@ void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     else if (TA && longest >= 256 && tiles > 320 && tiles <= 512)
         launch<TA, TB, 2, 4, 8, END>(jobs, beta, st);
     else if (tiles <= 64 && END != End::GATE)
-        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END>(jobs, beta, st);
-    else if (tiles <= 128 || (!TA && !TB && tiles > 256 && longest <= 256))
+        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END, 2>(jobs, beta, st);
+    else if (tiles <= 128)
+        launch<TA, TB, 1, 2, 4, END, 2>(jobs, beta, st);
+    else if (!TA && !TB && tiles > 256 && longest <= 256)
         launch<TA, TB, 1, 2, 4, END>(jobs, beta, st);
     else if (tiles <= 256 && longest >= 256)
         launch<TA, TB, 2, 2, 8, END>(jobs, beta, st);

@@ -516,6 +516,20 @@ def test_fp32_weight_gradients_of_wide_tiles(M, N, K):
         assert ((got.double() - (a.double().T @ b.double() + base)).abs() <= room).all()
 
 
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("M,N", [(256, 256), (512, 256)])  # up to 64 tiles of 32 x 32, up to 128
+def test_long_fp32_products_are_split_eight_ways(M, N, tA, tB):
+    """A chain loses terms below half a unit of its sum's last place: with 1 as the first term and 0.9 x 2^-27 ever after (four of them
+    in an instruction) the chain that holds the 1 loses all of its others, the K / 8 of one chain of eight, and the chains' sums and
+    the rows past a chunk's end are rounded once each."""
+    K = 2048
+    a, b = (torch.ones(s, device="cuda") for s in ((K, M) if tA else (M, K), (N, K) if tB else (K, N)))
+    (a if tA else a.T)[1:] = 0.9 * 2.0 ** -27
+    c = blockops.matmul(a, b, bool(tA), bool(tB))
+    want = 1 + (K - 1) * 0.9 * 2.0 ** -27
+    assert float((c.double() - want).abs().max()) <= (K // 8 + 32) * 0.9 * 2.0 ** -27 + 8 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("c_dtype", [torch.bfloat16, torch.float32], ids=str)
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("M,N,K", [(2, 2, 32), (34, 66, 34), (64, 32, 64), (62, 30, 344), (2, 40, 1002), (126, 130, 700), (1000, 64, 66)])
