@@ -728,7 +728,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                             up = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + cg * 8 + 32);
                 u32x4 v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = pack_bf16(gated_bf16(lo(gate[e]), lo(up[e])), gated_bf16(hi(gate[e]), hi(up[e])));
+                for (int e = 0; e < 4; ++e) v[e] = pack_bf16(gated(lo(gate[e]), lo(up[e])), gated(hi(gate[e]), hi(up[e])));
                 const uint32_t row = static_cast<uint32_t>(trow) * g.N * 2u;
                 store16(v, (row + col * 2) | mask, to_c, soff);
                 if constexpr (EPI == 5) {
@@ -764,8 +764,8 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float a[2], b[2];
-                    gated_grad_bf16(lo(gate[k][e]), lo(up[k][e]), lo(d[e]), a[0], b[0]);
-                    gated_grad_bf16(hi(gate[k][e]), hi(up[k][e]), hi(d[e]), a[1], b[1]);
+                    gated_grad(lo(gate[k][e]), lo(up[k][e]), lo(d[e]), a[0], b[0]);
+                    gated_grad(hi(gate[k][e]), hi(up[k][e]), hi(d[e]), a[1], b[1]);
                     dg[e] = pack_bf16(a[0], a[1]);
                     du[e] = pack_bf16(b[0], b[1]);
                 }

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
         if constexpr (END == End::GATE) {
             const uint32_t gate = pack_bf16(s0, s1), up = pack_bf16(sum(1, 0), sum(1, 1));
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o) =
-                pack_bf16(gated_bf16(lo(gate), lo(up)), gated_bf16(hi(gate), hi(up)));
+                pack_bf16(gated(lo(gate), lo(up)), gated(hi(gate), hi(up)));
             if (uint16_t* const gu = jobs.job[j].gu) {
                 *reinterpret_cast<uint32_t*>(gu + m * ldc * 2 + n) = gate;
                 *reinterpret_cast<uint32_t*>(gu + m * ldc * 2 + N + n) = up;
@@ -194,8 +194,8 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
             const uint32_t d = pack_bf16(s0, s1), gate = *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o),
                            up = *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o + N);
             float dg[2], du[2];
-            gated_grad_bf16(lo(gate), lo(up), lo(d), dg[0], du[0]);
-            gated_grad_bf16(hi(gate), hi(up), hi(d), dg[1], du[1]);
+            gated_grad(lo(gate), lo(up), lo(d), dg[0], du[0]);
+            gated_grad(hi(gate), hi(up), hi(d), dg[1], du[1]);
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o) = pack_bf16(dg[0], dg[1]);
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o + N) = pack_bf16(du[0], du[1]);
             continue;

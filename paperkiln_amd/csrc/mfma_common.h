@@ -267,26 +267,6 @@ __device__ inline void gated_grad(float g, float u, float d, float& dg, float& d
     dg = (d * u) * (s * (1.0f + g * (1.0f - s)));
 }
 
-// The same for results that are rounded to bf16, in half the instructions: expf and a division are some 25, and the epilogue of a
-// tile is made of little else. The exponent is formed in two parts and the reciprocal refined once. Largest error of the sigmoid
-// 1.27e-7 against 1.18e-7; over every bf16 gate within 60 of 0 and every mantissa of up, 1 bf16 product of 4.4 million and 2 gradients
-// come out on the other side of a tie, and the error against float64 is the same to ten digits. (Past 87, where the exponential
-// would leave fp32, it stays at its value there.) The 35 M parameter model's step: 4.66 -> 4.61 ms.
-__device__ inline float sigmoid_for_bf16(float g) {
-    constexpr float L = 1.44269502162933349609375f, L_REST = 1.925963033500011079e-8f;  // log2(e)
-    const float c = __builtin_amdgcn_fmed3f(g, -87.0f, 87.0f), hi = -c * L, lo = fmaf(-c, L_REST, fmaf(-c, L, -hi));
-    float e = __builtin_amdgcn_exp2f(hi);
-    e = fmaf(e, lo * 0.693147180559945f, e);
-    const float d = 1.0f + e, r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-__device__ inline float gated_bf16(float g, float u) { return g * sigmoid_for_bf16(g) * u; }
-__device__ inline void gated_grad_bf16(float g, float u, float d, float& dg, float& du) {
-    const float s = sigmoid_for_bf16(g);
-    du = d * (g * s);
-    dg = (d * u) * (s * (1.0f + g * (1.0f - s)));
-}
-
 // XCD-aware workgroup -> tile mapping. The 256 CUs sit in 8 XCDs, each with
 // its own 4 MB L2, and consecutive workgroup ids go round-robin over the XCDs.
 // Every block of a (batch, KV head) unit re-reads that unit's K/V (or Q/dO),

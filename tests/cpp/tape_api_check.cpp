@@ -407,6 +407,57 @@ void grouped_weight_gradient_case() {
     pk::set_compute_dtype(PK_F32);
 }
 
+// gated_mlp against the ops by themselves where the gate's sigmoid vanishes: gates of -85 and less, whose silu is scaled back by a
+// power of two. bf16 gates and results, each rounded once either way: one unit of theirs, and zero where the ops give zero.
+void vanishing_gates_case(int T, int d) {
+    std::printf("gated_mlp, bfloat16, gates of -85 to -30000, [%d, %d]\n", T, d);
+    const float gates[] = {-85.0f, -86.0f, -87.0f, -87.5f, -88.0f, -88.5f, -89.0f, -95.0f, -104.0f, -200.0f, -1000.0f, -30000.0f};
+    const size_t n = static_cast<size_t>(d) * d;
+    std::vector<float> hx(static_cast<size_t>(T) * d, 0.0f), hg(n, 0.0f), hu(n, 0.0f), hd(n, 0.0f), hr(static_cast<size_t>(T) * d, 0.0f);
+    for (int i = 0; i < T; ++i) hx[static_cast<size_t>(i) * d] = 1.0f;
+    for (int j = 0; j < d; ++j) {
+        hg[j] = gates[j % 12];
+        hu[j] = 1.0f;
+        hd[static_cast<size_t>(j) * d + j] = std::ldexp(1.0f, 110);
+    }
+    std::vector<int> target(T);
+    for (int i = 0; i < T; ++i) target[i] = i % d;
+    auto tg = device_ints(target);
+    pk::set_compute_dtype(PK_BF16);
+    struct Run {
+        std::vector<float> y, gg, gu;
+    };
+    auto run = [&](bool fused) {
+        pk::Var x = pk::make_var(pk::upload(hx.data(), T, d, PK_BF16), true), r = pk::make_var(pk::upload(hr.data(), T, d, PK_BF16), true);
+        pk::Var w[3];
+        const std::vector<float>* h[] = {&hg, &hu, &hd};
+        for (int k = 0; k < 3; ++k) {
+            w[k] = pk::make_var(pk::upload(h[k]->data(), d, d), true);
+            w[k]->is_param = true;
+        }
+        pk::Var y = fused ? pk::ops::gated_mlp(x, w[0], w[1], w[2], r)
+                          : pk::ops::linear_add(pk::ops::silu_mul(pk::ops::linear(x, w[0]), pk::ops::linear(x, w[1])), w[2], r);
+        Run out;
+        out.y = host(y->data);
+        pk::backward(pk::ops::cross_entropy(y, tg));
+        out.gg = host(w[0]->grad);
+        out.gu = host(w[1]->grad);
+        pk::invalidate_shadows();
+        return out;
+    };
+    const Run two = run(false), one = run(true);
+    auto off = [](const std::vector<float>& a, const std::vector<float>& b, size_t count) {  // largest difference in units of b's last place
+        double w = 0.0;
+        for (size_t i = 0; i < count; ++i)
+            if (a[i] != b[i]) w = std::fmax(w, std::fabs(static_cast<double>(a[i]) - b[i]) / std::fmax(std::fabs(b[i]) / 128.0, 1e-38));
+        return w;
+    };
+    check(off(one.y, two.y, one.y.size()) <= 1.0, "silu(gate) up", off(one.y, two.y, one.y.size()));
+    check(off(one.gg, two.gg, d) <= 2.0, "dgate", off(one.gg, two.gg, d));  // d is rounded too
+    check(off(one.gu, two.gu, d) <= 2.0, "dup", off(one.gu, two.gu, d));
+    pk::set_compute_dtype(PK_F32);
+}
+
 void behaviour_case() {
     std::printf("tape behaviour and errors\n");
     const auto h = draw(8 * 4, 31, 1.0);
@@ -470,6 +521,8 @@ int main() {
     for (int V : {18, 1002, 50258}) head_case(V, -50.0f, "logits near -150");  // one tile, 128 x 128 tiles, 256 x 256 tiles
     head_case((1 << 20) - 1, 0.0f, "logits of size ~50");  // past the in-product head's limit when padded: both take the row kernel
     grouped_weight_gradient_case();
+    vanishing_gates_case(16, 64);  // small tiles
+    vanishing_gates_case(4096, 512);
     behaviour_case();
     if (g_failures == 0) {
         std::printf("tape_api_check PASSED\n");
