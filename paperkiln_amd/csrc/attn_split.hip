@@ -122,8 +122,10 @@ __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
     return sum;
 }
 
-// Whether dP starts from -delta instead of zero, a subtraction an element less: not where its rounding, one more product at the
-// size of delta, would count (EXACT), nor at 128 columns, where it spilled 30 registers more.
+// Whether dP starts from -delta instead of zero, a subtraction an element less: dQ 1.6 %, dK/dV 2.5 % over 17 shapes. The sum is then
+// rounded at delta's size four times instead of once, which dS, one bf16 operand there, does not show: errors of dQ and dK against
+// float64 are 1.63e-3 to 1.79e-3 of their norms and the same to four digits either way over 28 inputs, V with a mean of 30 standard
+// deviations among them. Not where P and dS keep all their bits (EXACT), nor at 128 columns, where it spilled 30 registers more.
 template <int D, bool EXACT>
 constexpr bool FROM_DELTA = !EXACT && D == 64;
 
