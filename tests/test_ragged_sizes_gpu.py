@@ -388,6 +388,37 @@ def test_gradients_in_the_place_of_inputs(case, dtype, dk):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+# As a model calls them: q, k and v are slices of one projection, of every other sequence of a longer batch, dO is a transposed view and
+# the gradients go into slices of one buffer. The same kernels as of contiguous tensors, so the same bits: three parts, one launch for
+# the backward, wavefronts that own their rows at head_dim 64.
+@pytest.mark.parametrize("case,dtype,dk", [((24, 200, 8, 8, True, 0, 0), torch.float32, 64), ((13, 511, 16, 8, False, 0, 0), torch.float32, 96),
+                                           ((12, 383, 8, 8, True, 37, 5), torch.float32, 32), ((20, 161, 11, 11, True, 0, 0), torch.float32, 128),
+                                           ((3, 1100, 16, 4, True, 0, 0), torch.float32, 44)] +
+                         [((2, 129, 7, 1, True, 0, 0), t, d) for t, d in [(torch.bfloat16, 24), (torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float32, 20),
+                                                                          (torch.float32, 64), (torch.float32, 128)]] +
+                         [((1, 770, 2, 2, True, 64, 1), t, 64) for t in (torch.bfloat16, torch.float32)] +
+                         [(c, torch.bfloat16, 64) for c in [(16, 512, 8, 8, True, 0, 0), (6, 777, 12, 12, False, 0, 0), (3, 1889, 16, 16, True, 69, 16),
+                                                            (2, 2049, 14, 2, True, 0, 0), (8, 700, 16, 8, True, 128, 0)]], ids=str)
+def test_strided_tensors_give_the_bits_of_contiguous_ones(case, dtype, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
+    q, k, v = cut(torch.randn((2 * B, T, Hq + 2 * Hkv, dk), generator=gen, device="cuda").to(dtype)[::2])
+    d_o = torch.randn((B, Hq, T, dk), generator=gen, device="cuda").to(dtype).permute(0, 2, 1, 3)
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    ws = torch.empty(ops.bwd_workspace_bytes(q, k, window=window, sinks=sinks), dtype=torch.uint8, device="cuda")
+    results = []
+    for view in (lambda x: x, lambda x: x.contiguous()):
+        a = [view(x) for x in (q, k, v)]
+        o, lse = ops.attn_fwd(*a, scale, causal, window, sinks)
+        out = [view(x) for x in cut(torch.full((B, T, Hq + 2 * Hkv, dk), float("nan"), device="cuda").to(dtype))]
+        results.append((o, lse, *ops.attn_bwd(*a, o, lse, view(d_o), scale, causal, window, sinks, out=(*out, ws))))
+    assert not q.is_contiguous() and not d_o.is_contiguous()
+    assert all(torch.equal(x, y) for x, y in zip(*results))
+    e = errors(results[0], exact_attention(q, k, v, d_o, scale, causal, window, sinks))
+    assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
+
+
 # bf16 at head_dim 64 in launches that fill the chip: rows owned by wavefronts, two or four to a workgroup, tiles of 32 and 64; lengths
 # around the tiles and blocks, the shortest that come here, bands with and without sinks (dealt out and left whole), dealt heads, no mask.
 @pytest.mark.parametrize("case", [(16, 512, 8, 8, True, 0, 0), (64, 65, 8, 8, True, 0, 0), (20, 399, 8, 8, True, 0, 0), (2, 2049, 14, 2, True, 0, 0),
