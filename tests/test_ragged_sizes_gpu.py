@@ -259,9 +259,10 @@ def seen(T, key, causal, window, sinks):
     return vis.view(1, T, 1, 1)
 
 
-# launches that take the three-part kernels: both forms, every padded head size, a band, groups of heads
+# launches that take the three-part kernels: both forms, every padded head size, bands, a dealt sink tail, groups of heads, dealt out too
 RANGE_CASES = [((24, 200, 8, 8, True, 0, 0), 64), ((5, 4096, 4, 4, True, 0, 0), 64), ((13, 511, 16, 8, False, 0, 0), 96), ((12, 383, 8, 8, True, 37, 5), 32),
-               ((20, 161, 11, 11, True, 0, 0), 128), ((7, 577, 16, 8, True, 0, 0), 44)]
+               ((20, 161, 11, 11, True, 0, 0), 128), ((7, 577, 16, 8, True, 0, 0), 44), ((10, 1411, 8, 8, True, 33, 9), 64), ((1, 2500, 14, 2, True, 0, 0), 64),
+               ((3, 1100, 16, 4, True, 0, 0), 100)]
 
 
 @pytest.mark.parametrize("case,dk", RANGE_CASES, ids=str)
@@ -273,7 +274,7 @@ def test_three_parts_keep_infinities(case, dk):
     gen = torch.Generator(device="cuda").manual_seed(T + dk)
     q, k, v, d_o = (torch.randn((B, T, h, dk), generator=gen, device="cuda") for h in (Hq, Hkv, Hkv, Hq))
     q[..., 1] = -q[..., 1].abs() - 0.1
-    key, scale = T // 3, float(np.float32(1.0 / np.sqrt(dk)))
+    key, scale = 1 if sinks > 1 else T // 3, float(np.float32(1.0 / np.sqrt(dk)))
     sees = seen(T, key, causal, window, sinks)
     k_inf, k_zero = k.clone(), k.clone()
     k_inf[:, key, :, 1], k_zero[:, key] = float("inf"), 0.0
