@@ -268,8 +268,8 @@ int pk_op_gemm(const void* a, int trans_a, const void* b, int trans_b, void* c, 
  * reference's tiled kernel, src/cuda_resident.cu:141-171) for everything it takes (16-byte aligned rows, sizes that
  * are multiples of 8) -- measured on the MI355X it is ahead of rocBLAS or level with it on every Linear product of a
  * d = 512 block and of a 32000-word tied head -- in the form it picks per shape, rocBLAS for the rest; and the
- * weight-gradient products X^T dY of a backward pass over 2048 tokens or more are held back and multiplied several
- * at a time as one grouped launch. 2: the same kernel, every product on its own. 0: rocBLAS for everything, as for
+ * weight-gradient products X^T dY of a backward pass are held back and multiplied several at a time as one grouped
+ * launch. 2: the same kernel, every product on its own. 0: rocBLAS for everything, as for
  * fp32 operands. Measurement settings, all like 2 but with one form forced: 3 / 4 the register-staged
  * kernel with 128 x 128 / 256 x 256 tiles; 5, 6, 7 the LDS-ring kernel with 128 x 128 tiles and 4, 2, 3 ring slots;
  * 8 the ring kernel with 256 x 256 tiles; 9, 10, 11 the ring kernel with 128 x 128 tiles shared by two wavefront sets
