@@ -282,6 +282,35 @@ int launch_dq(const AttnArgs& a_in, bool fuse_delta, hipStream_t st) {
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
+// Any head size, LPR lanes a row and 16 bytes a lane at a time
+template <bool BF16, int LPR>
+__global__ __launch_bounds__(256) void row_delta(AttnArgs a) {
+    constexpr int W = BF16 ? 8 : 4;
+    const int sub = threadIdx.x % LPR;
+    const int blocks = (a.T + 256 / LPR - 1) / (256 / LPR), hb = blockIdx.x / blocks;
+    const int row = (blockIdx.x % blocks) * (256 / LPR) + static_cast<int>(threadIdx.x) / LPR;
+    const int h = hb % a.Hq, b = hb / a.Hq;
+    float s = 0.0f;
+    if (row < a.T) {
+        const int64_t oo = b * a.o_sb + h * a.o_sh + row * a.o_st, go = b * a.do_sb + h * a.do_sh + row * a.do_st;
+        for (int c = sub * W; c < a.dk_dim; c += LPR * W) {
+            const u32x4 ov = *reinterpret_cast<const u32x4*>(static_cast<const char*>(a.o) + (oo + c) * (BF16 ? 2 : 4));
+            const u32x4 gv = *reinterpret_cast<const u32x4*>(static_cast<const char*>(a.d_o) + (go + c) * (BF16 ? 2 : 4));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (BF16) {
+                    s = fmaf(__uint_as_float(ov[i] << 16), __uint_as_float(gv[i] << 16), s);
+                    s = fmaf(__uint_as_float(ov[i] & 0xFFFF0000u), __uint_as_float(gv[i] & 0xFFFF0000u), s);
+                } else {
+                    s = fmaf(__uint_as_float(ov[i]), __uint_as_float(gv[i]), s);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int o = LPR / 2; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (row < a.T && sub == 0) a.delta[static_cast<int64_t>(hb) * a.T + row] = s;
+}
 template <int D>
 int launch_delta(const AttnArgs& a, hipStream_t st) {
     constexpr int RPB = 256 / (D / 8);
@@ -303,6 +332,22 @@ int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 
 bool bf16_deals_heads(const AttnArgs& a) { return a.head_split > 1 && (split_deals_heads(a) || mfma_dkdv3_takes(a)); }
 
+int launch_row_delta(const AttnArgs& a, bool bf16, hipStream_t st) {
+    const int lanes = bf16 ? (a.dk_dim > 64 ? 16 : a.dk_dim > 32 ? 8 : 4) : a.dk_dim > 32 ? 16 : 8;
+    const dim3 grid((a.T + 256 / lanes - 1) / (256 / lanes) * a.Hq * a.B);
+    if (bf16 && lanes == 16)
+        hipLaunchKernelGGL((row_delta<true, 16>), grid, dim3(256), 0, st, a);
+    else if (bf16 && lanes == 8)
+        hipLaunchKernelGGL((row_delta<true, 8>), grid, dim3(256), 0, st, a);
+    else if (bf16)
+        hipLaunchKernelGGL((row_delta<true, 4>), grid, dim3(256), 0, st, a);
+    else if (lanes == 16)
+        hipLaunchKernelGGL((row_delta<false, 16>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((row_delta<false, 8>), grid, dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);

@@ -690,6 +690,7 @@ bool f32_deals_heads(const AttnArgs& a) { return a.head_split > 1 && f32_split_t
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
     int rc = PK_OK;
+    if (stages == PK_BWD_ALL && !a.in_place && f32x3_takes_bwd(a)) return launch_f32x3_bwd(a, st);
     if (stages == PK_BWD_ALL && !a.in_place && f32_split_takes_bwd(a)) return launch_f32_split_bwd(a, st);
     if (fused)  // dQ forms delta itself and runs first; dK/dV reads what it wrote
         rc = run_dq(a, true, st);

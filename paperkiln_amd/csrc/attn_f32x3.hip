@@ -545,17 +545,19 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
 
 // ---- dQ (and delta, when asked for with it): the same blocks ----
 template <int D, int QW, int KW>
-__global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs a, int fuse_delta) {
+constexpr int dq_lds() {  // in uint16
+    constexpr int TILES = BUFS<D, QW, KW> * KW * 6 * Mover3<D, 64 * QW>::PLANE, RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
+    return TILES > RED ? TILES : RED;
+}
+template <int D, int QW, int KW, int N>
+__device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h, int hk, int qblk, uint16_t (&lds)[N]) {
     constexpr int BM = 32 * QW, DB = D / 32, G = 64 * QW, NBUF = BUFS<D, QW, KW>;
     constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
     constexpr int RED = KW > 1 ? QW * KW * DB * 2048 : 0;  // in uint16
-    __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF * KW * TILE > RED ? NBUF * KW * TILE : RED];
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
-    int b, h, hk, qblk;
-    if (!map_query_block(a, (a.T + BM - 1) / BM, b, h, hk, qblk)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
     const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
     const float cexp = a.scale * LOG2E;
@@ -635,6 +637,12 @@ __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs 
             if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, ge, acc[db], a.scale, dk);
     }
 }
+template <int D, int QW, int KW>
+__global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs a, int fuse_delta) {
+    __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW>()];
+    int b, h, hk, qblk;
+    if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW>(a, fuse_delta, b, h, hk, qblk, lds);
+}
 
 // The two products of a step that need no other go to two sets of wavefronts, as in the other dK/dV kernels: with both
 // sides' resident rows and both accumulators one wavefront needs 320 registers at 128 columns before it has begun. A C
@@ -662,12 +670,12 @@ __device__ inline f32x16 get_tile(const float* buf, int lane) {
 // the loop has six of them for each (T 4096 x 2, 16 heads, head_dim 96, us: 1005 -> 968; head_dim 64, window 256, 4 KV heads, T
 // 4096 x 4: 337 -> 323). At 128 columns there is one wavefront to a SIMD and both do it at the end of the first phase (1777; 1872).
 template <int D, int QW>
-__global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
+constexpr int DKDV_TILE = 6 * Mover3<D, 64 * QW>::PLANE + 128;  // in uint16; LSE and delta of a tile's rows behind it
+template <int D, int QW, int N>
+__device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, uint16_t (&lds)[N], float* pbuf) {
     constexpr int BNK = 32 * QW, DB = D / 32, G = 64 * QW;
     constexpr bool APART = D < 128;
-    constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE + 128;  // LSE and delta of a tile's rows behind it
-    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * TILE];
-    __shared__ __attribute__((aligned(16))) float pbuf[QW * 1024];
+    constexpr int PLANE = Mover3<D, G>::PLANE, TILE = DKDV_TILE<D, QW>;
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int role = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) & (G - 1);
@@ -676,11 +684,6 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
     const int hs = a.head_split;  // > 1: this workgroup takes heads [h0, h0 + nh) of the group, see gqa_head_split
     // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
     const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
-    const int nblk = nkb + tl.nch;
-    int blk, rr, kvu;
-    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
-    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu))
-        return;
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
@@ -815,6 +818,30 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
 #pragma unroll
         for (int db = 0; db < DB; ++db) store_block32<D>(dst, row, db, g, acc[db], role == 0 ? 1.0f : a.scale, dk);
     }
+}
+template <int D, int QW>
+__global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * DKDV_TILE<D, QW>];
+    __shared__ __attribute__((aligned(16))) float pbuf[QW * 1024];
+    const int nblk = (a.T + 32 * QW - 1) / (32 * QW) + (a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0);
+    int blk, rr, kvu;
+    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
+    if (a.causal && nblk > 1 ? xcd_map_block_major(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu)
+                             : xcd_map(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu))
+        dkdv_block<D, QW>(a, blk, rr, kvu, lds, pbuf);
+}
+
+// ---- dK, dV and dQ in one launch, delta read (f32x3_takes_bwd) ----
+template <int D>
+__global__ __launch_bounds__(256, 2) void x3_bwd(AttnArgs a) {
+    constexpr int Q = dq_lds<D, 2, 2>(), K = 2 * DKDV_TILE<D, 2>, N = Q > K + 4096 ? Q : K + 4096;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[N];
+    const JoinedBlocks jb(a, 64);
+    int rank, r, kvu;
+    if (!jb.map(a, rank, r, kvu)) return;
+    if (r < a.head_split) return dkdv_block<D, 2>(a, rank, r, kvu, lds, reinterpret_cast<float*>(lds + K));
+    const int hk = kvu % a.Hkv;
+    dq_block<D, 2, 2>(a, 0, kvu / a.Hkv, hk * (a.Hq / a.Hkv) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // ---- dQ above 64 columns: the same two phases ----
@@ -1009,6 +1036,17 @@ int run_dkdv(const AttnArgs& a_in, hipStream_t st) {
     return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
 }
 
+template <int D>
+int run_bwd(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
+    a.head_split = head_split(a);
+    a.tail = nullptr;
+    if (const int rc = launch_row_delta(a, false, st)) return rc;
+    hipLaunchKernelGGL((x3_bwd<D>), dim3(JoinedBlocks(a, 64).grid(a)), dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
+}
+
 }  // namespace
 
 // what the fp32 split kernels ask of their tensors holds for these as well
@@ -1031,6 +1069,24 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
     if (a.dk_dim <= 64) return wide ? run_dq<64, 4, 1>(a, fuse_delta, st) : run_dq<64, 2, 2>(a, fuse_delta, st);
     return a.dk_dim <= 96 ? run_dq_wide<96>(a, fuse_delta, st) : run_dq_wide<128>(a, fuse_delta, st);
 }
+// dQ and dK/dV in one launch behind one of delta: while either alone is about one round of the chip, its longest chains of tiles are as
+// long as the launch and half of the chip waits for them; together one's chains run beside the other's. Over some rounds it is the same
+// work with a pass over O and dO more. In 64-row blocks of queries, one after the other (or on the fp32 instruction) | joined, us, causal
+// unless said:
+//   64 columns   T 1024 x 4, 8 heads (512) 122 | 110;   T 313 x 4, 16 heads (320) 73 | 36;   T 836 x 2, 8 heads (224) 84 | 65;
+//                T 1841, 8 heads (232) 132 | 117;   T 360 x 3, 8 heads (144) 39 | 32;   no mask, T 777 x 4, 12 heads (624) 208 | 176
+//     below      T 963, 4 heads (64) 50 | 66;   T 894 x 4, 2 heads (112) 45 | 60;   T 3305, 4 heads on 2 (208) 197 | 202
+//     above      T 5833, 8 heads (736) 688 | 710;   T 1024 x 8, 16 heads (2048) 351 | 362;   T 4096 x 4, 16 heads (4096) 2417 | 2562
+//   32 columns   T 1037 x 2, 8 heads (272) 62 | 50;   T 181 x 13, 16 heads (624) 42 | 29;   no mask, T 1639, 8 heads (208) 109 | 88
+//     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
+bool f32x3_takes_bwd(const AttnArgs& a) {
+    if (!f32_split_serves(a) || a.dk_dim > 64 || a.window > 0 || a.T <= 32) return false;
+    const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
+    if (a.dk_dim <= 32) return !a.causal ? q >= 180 && q <= 440 : q >= (a.T <= 130 ? 104 : a.T <= 600 ? 190 : 260) && q <= 640;
+    if (!a.causal) return q >= 120 && q <= 960;
+    return q >= (a.T <= 600 ? 140 : a.T <= 2000 ? 180 : 260) && q <= (a.T <= 1500 ? 1100 : 700);
+}
+int launch_f32x3_bwd(const AttnArgs& a, hipStream_t st) { return a.dk_dim <= 32 ? run_bwd<32>(a, st) : run_bwd<64>(a, st); }
 int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st) {
     if (a.dk_dim <= 32) return run_dkdv<32, 2>(a, st);
     if (a.dk_dim <= 64) return run_dkdv<64, 2>(a, st);

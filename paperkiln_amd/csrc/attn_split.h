@@ -122,6 +122,18 @@ struct OneLaunch {
     int finish(hipStream_t st) const { return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK; }
 };
 
+// The same for blocks of more rows, which read delta: blocks of `rows` keys and blocks of as many queries by rank, the longest of either
+// first. A rank of a (batch, KV head) unit is a block of keys for each share of the group's heads, then one of queries for each head.
+struct JoinedBlocks {
+    int ranks, each;
+    __host__ __device__ JoinedBlocks(const AttnArgs& a, int rows) : ranks((a.T + rows - 1) / rows), each(a.head_split + a.Hq / a.Hkv) {}
+    __host__ int grid(const AttnArgs& a) const { return xcd_grid(ranks, each, a.Hkv * a.B); }
+    // r: the share of the heads whose dK, dV (r < a.head_split), or the head (the others) whose dQ this workgroup forms
+    __device__ bool map(const AttnArgs& a, int& rank, int& r, int& kvu) const {
+        return a.causal && ranks > 1 ? xcd_map_block_major(ranks, each, a.Hkv * a.B, rank, r, kvu) : xcd_map(ranks, each, a.Hkv * a.B, rank, r, kvu);
+    }
+};
+
 // The tiles of BN keys that queries [q0, q0 + BM) can see, as a list: sink tiles [0, ns), then [lo, hi].
 struct KeyTiles {
     int ns, lo, n;

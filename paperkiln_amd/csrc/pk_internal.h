@@ -176,6 +176,10 @@ bool f32x3_takes_dkdv(const AttnArgs& a);
 int launch_f32x3_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st);
+bool f32x3_takes_bwd(const AttnArgs& a);  // dQ and dK/dV in one launch, behind one of delta
+int launch_f32x3_bwd(const AttnArgs& a, hipStream_t st);
+// delta = rowsum(dO .* O) by itself, aligned rows of any head size; attn_bwd_mfma.hip
+int launch_row_delta(const AttnArgs& a, bool bf16, hipStream_t st);
 
 // attn_f32_mfma.hip: fp32 tensors on the fp32 matrix instruction, head sizes that are multiples of 4 up to 128.
 bool f32_mfma_supported(const AttnArgs& a);

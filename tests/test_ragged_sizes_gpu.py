@@ -367,6 +367,27 @@ def test_backward_in_one_launch(case, dtype, dk):
     assert max(e) < (1e-2 if dtype == torch.bfloat16 else 5e-6), e
 
 
+# fp32 blocks of 64 keys and of 64 queries in one launch behind one of delta: one row past a block and a tile, more ranks than heads, groups
+# whose heads are dealt out, units that do not divide by the 8 XCDs, the shortest chains and the most blocks that go together.
+@pytest.mark.parametrize("dk", [4, 32, 44, 64])
+@pytest.mark.parametrize("case", [(18, 33, 16, 16, True, 0, 0), (7, 65, 16, 8, True, 0, 0), (9, 129, 14, 2, True, 0, 0), (2, 641, 13, 13, True, 0, 0),
+                                  (5, 577, 8, 8, False, 0, 0), (1, 2113, 8, 2, True, 0, 0), (40, 257, 3, 3, True, 0, 0)], ids=str)
+def test_fp32_backward_of_joined_blocks(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
+    q, k, v = cut(torch.randn((B, T, Hq + 2 * Hkv, dk), generator=gen, device="cuda"))
+    d_o = torch.randn((B, Hq, T, dk), generator=gen, device="cuda").permute(0, 2, 1, 3)
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    one = ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks)
+    again = ops.attn_bwd(*(x.contiguous() for x in (q, k, v)), o, lse, d_o.contiguous(), scale, causal, window, sinks)
+    assert all(torch.equal(x, y) for x, y in zip(one, again))
+    want = exact_attention(q, k, v, d_o, scale, causal, window, sinks)[2:]
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(one, want)]
+    assert max(e) < 1e-6, e  # as test_fp32_as_three_parts
+
+
 # A training loop that keeps no tensors it can do without: dQ where O was, dK and dV where K and V were. Small launches and large ones,
 # groups of heads dealt out, dealt sink tails, head sizes of every kernel family. The same bits as dQ and then dK/dV into buffers of
 # their own, which read what they read in this order.
