@@ -351,6 +351,7 @@ int launch_row_delta(const AttnArgs& a, bool bf16, hipStream_t st) {
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
+    if (stages == PK_BWD_ALL && !a.in_place && split_takes_joined(a)) return launch_split_joined(a, st);
     if (stages == PK_BWD_ALL && !a.in_place && split_takes_bwd(a)) return launch_split_bwd(a, st);
     int rc = PK_OK;
     if (fused)

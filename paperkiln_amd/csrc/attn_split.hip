@@ -110,6 +110,12 @@ __device__ inline float weight_of(float s, float scale, float cexp, float nl) {
     return __builtin_amdgcn_exp2f(EXACT ? fmaf(s, scale, nl) * LOG2E : fmaf(s, cexp, nl));
 }
 
+// x of another lane of the same sixteen, by the DPP control word
+template <int CTRL>
+__device__ inline float lane_swapped(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
+
 // sum + the products of eight elements, in order
 __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
     const u32x4 xv = *reinterpret_cast<const u32x4*>(&x);
@@ -330,7 +336,7 @@ constexpr int dq_lds() {  // in uint16
     return TILES > RED ? TILES : RED;
 }
 template <int D, int QW, int KW, int NB, bool EXACT>
-__device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint16_t* lds) {
+__device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h, int hk, int qblk, uint16_t* lds) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
     constexpr bool MINUS_DELTA = FROM_DELTA<D, EXACT> && (QW > 1 || KW == 8);  // not with four: T 1661, 16 heads 21.5 us | 24.5
@@ -338,9 +344,6 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint1
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
-    const int nqb = (a.T + BM - 1) / BM;
-    int b, h, hk, qblk;
-    if (!map_query_block(a, nqb, b, h, hk, qblk, id)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
     const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
     const float cexp = a.scale * LOG2E;
@@ -429,7 +432,16 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, uint1
 template <int D, int QW, int KW, int NB, bool EXACT>
 __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
     __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW, NB>()];
-    dq_block<D, QW, KW, NB, EXACT>(a, fuse_delta, static_cast<int>(blockIdx.x), lds);
+    int b, h, hk, qblk;
+    if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW, NB, EXACT>(a, fuse_delta, b, h, hk, qblk, lds);
+}
+
+// The block of `rows` keys of a workgroup, or its piece of a dealt sink tail (past the blocks); rr: its share of the group's heads
+__device__ inline bool map_key_block(const AttnArgs& a, int rows, int& blk, int& rr, int& kvu, int id = static_cast<int>(blockIdx.x)) {
+    const int nblk = (a.T + rows - 1) / rows + (a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0);
+    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
+    return a.causal && nblk > 1 ? xcd_map_block_major(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu, id)
+                                : xcd_map(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu, id);
 }
 
 // ---- dK, dV: QW groups of 32 keys x KW groups of query tiles of 32 NB ----
@@ -437,16 +449,18 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse
 // exponentials into dV and into dS without leaving the registers. The steps are the query tiles that can see the block,
 // for every query head of the KV head's group in turn.
 //
-// OWN_DELTA (one wavefront to a group, tiles of 32): the rows' delta is formed here, from O and the tile of dO, in the order of
-// dq_block and to the same bits; otherwise it is read.
+// OWN_DELTA: the rows' delta is formed here, from O and the tile of dO; otherwise it is read. Of one wavefront to a group and tiles of 32 in the
+// order of dq_block and to the same bits; else a thread's chunks of both, then the lanes that hold a row.
 template <int D, int QW, int KW, int NB>
 constexpr int dkdv_lds() {  // in uint16; LSE and delta of a tile's rows behind it
     constexpr int TILES = (QW > 1 ? 2 : 1) * KW * (2 * 32 * NB * (D + 8) + 128 * NB), RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
     return TILES > RED ? TILES : RED;
 }
 template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA>
-__device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
-    static_assert(!OWN_DELTA || (QW == 1 && NB == 1), "a lane holds the row of O whose row of dO its wavefront has just written");
+__device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, uint16_t* lds) {
+    // a lane holds the row of O whose row of dO its wavefront has just written; or the chunks of O beside its chunks of dO
+    static_assert(!OWN_DELTA || (QW == 1 && NB == 1) || (QW > 1 && (D == 32 || D == 64)), "a row's chunks are in 4 or 8 neighbouring lanes");
+    constexpr bool BY_ROW = OWN_DELTA && QW == 1, BY_CHUNK = OWN_DELTA && QW > 1;
     constexpr int BNK = 32 * QW, BMQ = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int ROWC = 2 * BMQ * 2;                    // LSE and delta of a tile's rows, in uint16
     constexpr int TILE = 2 * BMQ * S + ROWC, NBUF = QW > 1 ? 2 : 1;
@@ -460,11 +474,6 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
     const int hs = a.head_split;
     // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
     const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
-    const int nblk = nkb + tl.nch;
-    int blk, rr, kvu;
-    // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
-    if (a.causal && nblk > 1 ? !xcd_map_block_major(nblk, hs, a.Hkv * a.B, blk, rr, kvu, id) : !xcd_map(nblk, hs, a.Hkv * a.B, blk, rr, kvu, id))
-        return;
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
     const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
@@ -484,7 +493,9 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
     mq.init(gt, a.q_st, dk);
     mg.init(gt, a.do_st, dk);
     float row_r = 0.0f;
-    bf16x8 oreg[OWN_DELTA ? KK : 1];
+    bf16x8 oreg[BY_ROW ? KK : 1];
+    typename std::conditional<BY_CHUNK, Mover<D, G, BMQ>, int>::type mo;
+    if constexpr (BY_CHUNK) mo.init(gt, a.o_st, dk);
     // steps advance by KW; the (head, tile) of the next fetch is counted up
     int f_h = kg / nqt, f_t = kg % nqt, c_t = f_t;
     auto fetch = [&](int i) {
@@ -500,7 +511,8 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
                 else if (!OWN_DELTA)
                     row_r = a.delta[lrow];
             }
-            if constexpr (OWN_DELTA) load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, r0 + c32, a.T, dk, g, oreg);
+            if constexpr (BY_CHUNK) mo.load(a.o, b * a.o_sb + h * a.o_sh, a.o_st, r0, a.T, dk);
+            if constexpr (BY_ROW) load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, r0 + c32, a.T, dk, g, oreg);
             f_t += KW;
             while (f_t >= nqt) f_t -= nqt, ++f_h;
         }
@@ -510,7 +522,18 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
         mq.template store<true>(t, S, gt);
         mg.template store<true>(t + BMQ * S, S, gt);
         float out = gt >= BMQ ? (FROM_DELTA<D, EXACT> ? -row_r : row_r) : EXACT ? -row_r : -row_r * LOG2E;
-        if constexpr (OWN_DELTA) {
+        if constexpr (BY_CHUNK) {
+#pragma unroll
+            for (int i = 0; i < Mover<D, G, BMQ>::CPT; ++i) {
+                float part = add_products(*reinterpret_cast<const bf16x8*>(&mo.r[i]), *reinterpret_cast<const bf16x8*>(&mg.r[i]), 0.0f);
+                part += lane_swapped<0xB1>(part);  // lane ^ 1
+                part += lane_swapped<0x4E>(part);  // lane ^ 2
+                if (D == 64) part += lane_swapped<0x141>(part);  // the other four of eight
+                if (gt % (D / 8) == 0) reinterpret_cast<float*>(t + 2 * BMQ * S)[BMQ + (gt + G * i) / (D / 8)] = FROM_DELTA<D, EXACT> ? -part : part;
+            }
+            if (gt >= BMQ) return;
+        }
+        if constexpr (BY_ROW) {
             tile_barrier<1>();
             float part = 0.0f;
 #pragma unroll
@@ -616,7 +639,8 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, uint16_t* lds) {
 template <int D, int QW, int KW, int NB, bool EXACT, int OCC>
 __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t lds[dkdv_lds<D, QW, KW, NB>()];
-    dkdv_block<D, QW, KW, NB, EXACT, false>(a, static_cast<int>(blockIdx.x), lds);
+    int blk, rr, kvu;
+    if (map_key_block(a, 32 * QW, blk, rr, kvu)) dkdv_block<D, QW, KW, NB, EXACT, false>(a, blk, rr, kvu, lds);
 }
 
 // ---- dK, dV and dQ in one launch, as in attn_f32_split.hip ----
@@ -626,10 +650,28 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, in
     constexpr int Q = dq_lds<D, 1, 4, 1>(), K = dkdv_lds<D, 1, 4, 1>();
     __shared__ __attribute__((aligned(16))) uint16_t lds[Q > K ? Q : K];
     const int id = static_cast<int>(blockIdx.x);
-    if (id < dkdv_ids)
-        dkdv_block<D, 1, 4, 1, EXACT, true>(a, id, lds);
-    else
-        dq_block<D, 1, 4, 1, EXACT>(a, 1, id - dkdv_ids, lds);
+    int blk, rr, kvu, b, h, hk, qblk;
+    if (id < dkdv_ids) {
+        if (map_key_block(a, 32, blk, rr, kvu, id)) dkdv_block<D, 1, 4, 1, EXACT, true>(a, blk, rr, kvu, lds);
+    } else if (map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk, id - dkdv_ids)) {
+        dq_block<D, 1, 4, 1, EXACT>(a, 1, b, h, hk, qblk, lds);
+    }
+}
+
+// ---- the same of wavefronts that own their rows (split_takes_joined) ----
+// dK/dV forms delta from the chunks of O beside those of dO while it moves a tile (up to 64 columns, whose chunks are in 4 or 8 neighbouring
+// lanes; above, it is read): a launch of delta before this one cost 4 us more, of 13 to 60.
+template <int D, bool EXACT>
+__global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
+    constexpr bool OWN_DELTA = D <= 64;
+    constexpr int Q = dq_lds<D, 4, 1, 2>(), K = dkdv_lds<D, 4, 1, 2>();
+    __shared__ __attribute__((aligned(16))) uint16_t lds[Q > K ? Q : K];
+    const JoinedBlocks jb(a, 128);
+    int rank, r, kvu;
+    if (!jb.map(a, rank, r, kvu)) return;
+    if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA>(a, rank, r, kvu, lds);
+    const int hk = kvu % a.Hkv;
+    dq_block<D, 4, 1, 2, EXACT>(a, OWN_DELTA, kvu / a.Hkv, hk * (a.Hq / a.Hkv) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of
@@ -915,6 +957,49 @@ bool split_takes_bwd(const AttnArgs& a) {
     if (a.dk_dim <= 64) return ids <= (a.T <= 64 ? 400 : even_chains(a) ? 640 : 800);  // (one tile: T 31 x 84, 4 heads of 64 10.9 | 13.3)
     if (a.dk_dim <= 96) return ids <= (even_chains(a) ? 380 : 400);
     return ids <= 256 && (a.dk_dim < 128 || a.T > 32);
+}
+// Blocks of 128 keys and of 128 queries in one launch, no band. Where either launch by itself is a round of the chip or less, its longest chains
+// last as long as it does; together one's run beside the other's, and rows that share a tile's trip to LDS do half of the work there that blocks
+// of 32 do. `u` blocks of queries, `n` to a head. Measured, one after the other (or in blocks of 32) | joined, us:
+//   64 columns     T 470 x 8, 8 heads (u 256) 31 | 21;  T 923 x 7, 4 heads (224) 48 | 33;  T 1104 x 2, 16 heads on 8 (288) 67 | 46;  T 150 x 4, 16
+//                  heads (128) 15.4 | 11.0;  T 1024 x 8, 8 heads (512) 57 | 52;  T 4945, 8 heads (312) 190 | 138;  no mask, T 423 x 14, 2 heads (112) 30 | 19
+//     below        T 1066, 16 heads on 4 (144) 38 | 39;  T 1982, 8 on 4 (128) 51 | 61;  T 3520, 8 heads (224) 82 | 94;  no mask, T 3347, 4 on 1 (108) 90 | 114
+//     above        T 1182 x 8, 8 heads (640) 69 | 75;  T 2048 x 4, 14 heads on 2 (896) 149 | 153;  no mask, T 777 x 6, 12 heads (504) 65 | 69
+//   32, 48         T 148 x 58, 2 heads of 48 (232) 21 | 13;  T 486 x 3, 16 heads on 4 (192) 34 | 26;  T 1746, 32 on 8 of 48 (448) 127 | 111
+//     below, above T 961, 16 heads (128) 29 | 35;  T 1715, 14 on 2 of 48 (196) 72 | 79;  T 1951, 32 on 16 (512) 106 | 110
+//   80, 96 (delta in a launch of its own)  T 49 x 131, 2 heads (262) 37 | 21;  T 393 x 7, 14 on 2 (392) 70 | 56;  T 2515, 14 on 2 (280) 217 | 173
+//     below, above T 1110, 16 heads (144) 63 | 69;  T 2573, 8 on 4 (168) 125 | 157;  T 129 x 15, 16 on 8 (480) 40 | 44
+bool split_takes_joined(const AttnArgs& a) {
+    if (a.dk_dim > 96 || a.window > 0 || a.T <= 32) return false;
+    const int64_t n = (a.T + 127) / 128, u = n * a.Hq * a.B;
+    if (a.dk_dim == 64)
+        return a.causal ? u >= (n == 1 ? 60 : n <= 4 ? 104 : n <= 12 ? 150 : n <= 17 ? 200 : 290) && u <= (n <= 2 ? 440 : 560)
+                        : u >= (n == 1 ? 60 : n <= 8 ? 110 : 150) && u <= 300;
+    if (a.dk_dim < 64)
+        return a.causal ? n <= 16 && u >= (n == 1 ? 60 : n <= 2 ? 112 : n <= 7 ? 190 : 300) && u <= 450
+                        : n <= 12 && u >= (n == 1 ? 60 : n <= 6 ? 84 : 200) && u <= 300;
+    return u >= (n == 1 ? 80 : n <= 5 ? 150 : n <= 12 ? 190 : 232) && u <= 440;
+}
+template <int D, bool EXACT>
+int joined_of(const AttnArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL((split_joined<D, EXACT>), dim3(JoinedBlocks(a, 128).grid(a)), dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return PK_OK;
+}
+int launch_split_joined(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
+    a.head_split = splits_of(a);
+    a.tail = nullptr;
+    if (a.dk_dim > 64)
+        if (const int rc = launch_row_delta(a, true, st)) return rc;
+    const auto run = [&]() -> int {
+        if (a.dk_dim == 64) return joined_of<64, false>(a, st);
+        if (a.dk_dim <= 32) return joined_of<32, true>(a, st);
+        if (a.dk_dim <= 64) return joined_of<64, true>(a, st);
+        return joined_of<96, true>(a, st);
+    };
+    if (const int rc = run()) return rc;
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
 }
 int launch_split_bwd(const AttnArgs& a, hipStream_t st) {
     const OneLaunch l(a);

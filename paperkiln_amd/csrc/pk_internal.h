@@ -200,6 +200,8 @@ int launch_split_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_split_dkdv(const AttnArgs& a, hipStream_t st);
 bool split_takes_bwd(const AttnArgs& a);  // dQ (with delta) and dK/dV in one launch
 int launch_split_bwd(const AttnArgs& a, hipStream_t st);
+bool split_takes_joined(const AttnArgs& a);  // the same of blocks of 128 rows
+int launch_split_joined(const AttnArgs& a, hipStream_t st);
 
 // attn_fwd_mfma.hip / attn_bwd_mfma.hip: bf16 MFMA kernels, head_dim 64 or 128.
 // 16-byte-aligned rows whose stride keeps a tile's byte offsets in 31 bits, and a positive scale (the running max is

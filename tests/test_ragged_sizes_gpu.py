@@ -388,6 +388,30 @@ def test_fp32_backward_of_joined_blocks(case, dk):
     assert max(e) < 1e-6, e  # as test_fp32_as_three_parts
 
 
+# bf16 blocks of 128 keys and of 128 queries in one launch: one tile and one row past it, one row past a block, rows past the end in the last
+# tile that delta is formed of, groups whose heads are dealt out, units that do not divide by the 8 XCDs; O a view as the others are.
+@pytest.mark.parametrize("dk", [8, 32, 40, 64, 80, 96])
+@pytest.mark.parametrize("case", [(17, 33, 16, 16, True, 0, 0), (9, 65, 16, 8, True, 0, 0), (13, 129, 8, 8, False, 0, 0), (11, 193, 14, 2, True, 0, 0),
+                                  (5, 577, 9, 3, True, 0, 0), (2, 1025, 16, 4, True, 0, 0), (3, 700, 9, 9, False, 0, 0)], ids=str)
+def test_bf16_backward_of_joined_blocks(case, dk):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
+    q, k, v = cut(torch.randn((B, T, Hq + 2 * Hkv, dk), generator=gen, device="cuda").bfloat16())
+    d_o = torch.randn((B, Hq, T, dk), generator=gen, device="cuda").bfloat16().permute(0, 2, 1, 3)
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    o_view = torch.full((B, T, 2 * Hq, dk), float("nan"), device="cuda").bfloat16()[:, :, :Hq]
+    o_view.copy_(o)
+    one = ops.attn_bwd(q, k, v, o_view, lse, d_o, scale, causal, window, sinks, grad_dtype=torch.float32)
+    again = ops.attn_bwd(*(x.contiguous() for x in (q, k, v, o)), lse, d_o.contiguous(), scale, causal, window, sinks, grad_dtype=torch.float32)
+    assert all(torch.equal(x, y) for x, y in zip(one, again))
+    want = exact_attention(q, k, v, d_o, scale, causal, window, sinks, o)[2:]
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(one, want)]
+    # 64 columns: P and dS as one bf16 operand, 2^-9 of a term; the others keep all their bits
+    assert max(e) < (4e-3 if dk == 64 else 2e-6), e
+
+
 # A training loop that keeps no tensors it can do without: dQ where O was, dK and dV where K and V were. Small launches and large ones,
 # groups of heads dealt out, dealt sink tails, head sizes of every kernel family. The same bits as dQ and then dK/dV into buffers of
 # their own, which read what they read in this order.
