@@ -1078,10 +1078,13 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 //     below      T 963, 4 heads (64) 50 | 66;   T 894 x 4, 2 heads (112) 45 | 60;   T 3305, 4 heads on 2 (208) 197 | 202
 //     above      T 5833, 8 heads (736) 688 | 710;   T 1024 x 8, 16 heads (2048) 351 | 362;   T 4096 x 4, 16 heads (4096) 2417 | 2562
 //   32 columns   T 1037 x 2, 8 heads (272) 62 | 50;   T 181 x 13, 16 heads (624) 42 | 29;   no mask, T 1639, 8 heads (208) 109 | 88
+//   bands, every head its own: 48, T 165 x 6, 8 heads, window 86 (144) 36 | 20;   T 4383, 8 heads, 26 (552) 51 | 42;   T 975 x 13, 2 heads of 64, 408,
+//     1 sink (416) 109 | 79;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
 //     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
 bool f32x3_takes_bwd(const AttnArgs& a) {
-    if (!f32_split_serves(a) || a.dk_dim > 64 || a.window > 0 || a.T <= 32) return false;
+    if (!f32_split_serves(a) || a.dk_dim > 64 || a.T <= 32) return false;
     const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
+    if (a.window > 0) return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= 300) && q >= (a.dk_dim <= 32 ? 130 : 100) && q <= 800;
     if (a.dk_dim <= 32) return !a.causal ? q >= 180 && q <= 440 : q >= (a.T <= 130 ? 104 : a.T <= 600 ? 190 : 260) && q <= 640;
     if (!a.causal) return q >= 120 && q <= 960;
     return q >= (a.T <= 600 ? 140 : a.T <= 2000 ? 180 : 260) && q <= (a.T <= 1500 ? 1100 : 700);

@@ -958,7 +958,7 @@ bool split_takes_bwd(const AttnArgs& a) {
     if (a.dk_dim <= 96) return ids <= (even_chains(a) ? 380 : 400);
     return ids <= 256 && (a.dk_dim < 128 || a.T > 32);
 }
-// Blocks of 128 keys and of 128 queries in one launch, no band. Where either launch by itself is a round of the chip or less, its longest chains
+// Blocks of 128 keys and of 128 queries in one launch. Where either launch by itself is a round of the chip or less, its longest chains
 // last as long as it does; together one's run beside the other's, and rows that share a tile's trip to LDS do half of the work there that blocks
 // of 32 do. `u` blocks of queries, `n` to a head. Measured, one after the other (or in blocks of 32) | joined, us:
 //   64 columns     T 470 x 8, 8 heads (u 256) 31 | 21;  T 923 x 7, 4 heads (224) 48 | 33;  T 1104 x 2, 16 heads on 8 (288) 67 | 46;  T 150 x 4, 16
@@ -969,9 +969,14 @@ bool split_takes_bwd(const AttnArgs& a) {
 //     below, above T 961, 16 heads (128) 29 | 35;  T 1715, 14 on 2 of 48 (196) 72 | 79;  T 1951, 32 on 16 (512) 106 | 110
 //   80, 96 (delta in a launch of its own)  T 49 x 131, 2 heads (262) 37 | 21;  T 393 x 7, 14 on 2 (392) 70 | 56;  T 2515, 14 on 2 (280) 217 | 173
 //     below, above T 1110, 16 heads (144) 63 | 69;  T 2573, 8 on 4 (168) 125 | 157;  T 129 x 15, 16 on 8 (480) 40 | 44
+//   bands, every head its own  64: T 651 x 2, 8 heads, window 235 (96) 26 | 17;  T 4247, 8 heads, 336 (272) 36 | 32;  T 159 x 7, 16 on 8 23 | 18
+//     not          T 1128, 16 heads, 178, 1 sink, whose block is walked whole (144) 33 | 42;  T 1777, 16 on 8 44 | 116;  T 211 x 8, 4 heads (64) 11 | 14
 bool split_takes_joined(const AttnArgs& a) {
-    if (a.dk_dim > 96 || a.window > 0 || a.T <= 32) return false;
+    if (a.dk_dim > 96 || a.T <= 32) return false;
     const int64_t n = (a.T + 127) / 128, u = n * a.Hq * a.B;
+    if (a.window > 0)
+        return a.Hq == a.Hkv && (a.sinks == 0 || a.T <= 600) &&
+               (a.dk_dim == 64 ? u >= (chain_tokens(a) <= 1024 ? 84 : 150) && u <= 450 : u >= 190 && u <= 390);
     if (a.dk_dim == 64)
         return a.causal ? u >= (n == 1 ? 60 : n <= 4 ? 104 : n <= 12 ? 150 : n <= 17 ? 200 : 290) && u <= (n <= 2 ? 440 : 560)
                         : u >= (n == 1 ? 60 : n <= 8 ? 110 : 150) && u <= 300;

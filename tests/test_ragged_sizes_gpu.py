@@ -371,7 +371,8 @@ def test_backward_in_one_launch(case, dtype, dk):
 # whose heads are dealt out, units that do not divide by the 8 XCDs, the shortest chains and the most blocks that go together.
 @pytest.mark.parametrize("dk", [4, 32, 44, 64])
 @pytest.mark.parametrize("case", [(18, 33, 16, 16, True, 0, 0), (7, 65, 16, 8, True, 0, 0), (9, 129, 14, 2, True, 0, 0), (2, 641, 13, 13, True, 0, 0),
-                                  (5, 577, 8, 8, False, 0, 0), (1, 2113, 8, 2, True, 0, 0), (40, 257, 3, 3, True, 0, 0)], ids=str)
+                                  (5, 577, 8, 8, False, 0, 0), (1, 2113, 8, 2, True, 0, 0), (40, 257, 3, 3, True, 0, 0), (6, 321, 9, 9, True, 33, 17),
+                                  (1, 1100, 11, 11, True, 100, 0)], ids=str)
 def test_fp32_backward_of_joined_blocks(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     gen = torch.Generator(device="cuda").manual_seed(T + dk)
@@ -392,7 +393,8 @@ def test_fp32_backward_of_joined_blocks(case, dk):
 # tile that delta is formed of, groups whose heads are dealt out, units that do not divide by the 8 XCDs; O a view as the others are.
 @pytest.mark.parametrize("dk", [8, 32, 40, 64, 80, 96])
 @pytest.mark.parametrize("case", [(17, 33, 16, 16, True, 0, 0), (9, 65, 16, 8, True, 0, 0), (13, 129, 8, 8, False, 0, 0), (11, 193, 14, 2, True, 0, 0),
-                                  (5, 577, 9, 3, True, 0, 0), (2, 1025, 16, 4, True, 0, 0), (3, 700, 9, 9, False, 0, 0)], ids=str)
+                                  (5, 577, 9, 3, True, 0, 0), (2, 1025, 16, 4, True, 0, 0), (3, 700, 9, 9, False, 0, 0), (9, 321, 9, 9, True, 33, 17),
+                                  (2, 1100, 12, 12, True, 100, 0)], ids=str)
 def test_bf16_backward_of_joined_blocks(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     gen = torch.Generator(device="cuda").manual_seed(T + dk)
