@@ -22,13 +22,13 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "attn_bwd_dq.h"
 #include "mfma_common.h"
 #include "pk_internal.h"
 
 namespace pk {
 namespace {
 
-constexpr float LOG2E = 1.4426950408889634f;
 // Two geometries. 128 keys per workgroup (8 wavefronts, 64-query steps, one workgroup per CU) is the general one.
 // With a narrow band a key block meets only a handful of query steps, and the fixed costs of a workgroup -- resident
 // rows, first tiles, pipeline fill, epilogue -- weigh as much as its steps; there a workgroup takes 64 keys with 4
@@ -47,22 +47,35 @@ __device__ inline void store4g(void* base, int64_t idx, float x0, float x1, floa
     }
 }
 
+template <int D, int BMQ>
+using Ring = uint16_t[2][3][BMQ * (D + 8)];  // [Q | dO][ring slot]
+template <int BNK, int BMQ>
+using Weights = uint16_t[2][BMQ / 32][BNK / 32][2 * 64 * 8];  // [step parity][query block][key block][half][lane][8]
+template <int BMQ>
+using Rows = float[3][BMQ];
+// x of another lane of the same sixteen, by the DPP control word
+template <int CTRL>
+__device__ inline float lane_swapped(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
+
+// A workgroup's blocks of BNK keys, by its number in the launch; JOINED: the block jblk of unit jkvu.
 // TAIL: the launch carries the extra workgroups of a split sink tail (a separate instantiation, so
 // that the plain causal kernel keeps its register budget)
-template <int D, bool GF32, bool TAIL, int BNK, int BMQ>
-__global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
+// JOINED: delta is formed here, from the chunks of O beside those of dO, while a tile is moved, and the heads of a group may be dealt to
+// a.head_split workgroups of which this is the rr-th (gqa_head_split); otherwise delta is read and all heads are walked.
+template <int D, bool GF32, bool TAIL, int BNK, int BMQ, bool JOINED>
+__device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weights<BNK, BMQ>& Pbuf, Rows<BMQ>& nlse_s, Rows<BMQ>& dl_s,
+                                    int jblk = 0, int jkvu = 0, int share = 0) {
     constexpr int KK = D / 16, DB = D / 32;
     constexpr int NTHR = 4 * BNK, NKB = BNK / 32, NQB = BMQ / 32;  // threads; 32-key blocks; 32-query blocks per step
     constexpr int S = D + 8;            // tile row pitch (elements): 16-byte row reads conflict-free
     constexpr int NCH = D / 8;          // 16-byte chunks per row
     constexpr int CPT = BMQ * NCH / NTHR;  // chunks per thread per tensor per step
     static_assert(CPT >= 1 && BMQ * NCH % NTHR == 0, "every thread stages the same number of chunks");
-    __shared__ __attribute__((aligned(16))) uint16_t tiles[2][3][BMQ * S];  // [Q | dO][ring slot]
+    static_assert(!JOINED || NCH == 8 || NCH == 16, "a row's chunks are in 8 or 16 neighbouring lanes");
     uint16_t (*const Qs)[BMQ * S] = tiles[0];
     uint16_t (*const dOs)[BMQ * S] = tiles[1];
-    __shared__ __attribute__((aligned(16))) uint16_t Pbuf[2][NQB][NKB][2 * 64 * 8];  // [step parity][query block][key block][half][lane][8]
-    __shared__ __attribute__((aligned(16))) float nlse_s[3][BMQ];            // -LSE * log2(e)
-    __shared__ __attribute__((aligned(16))) float dl_s[3][BMQ];
 
     const int lane = threadIdx.x & 63;
     // the wavefront index as a scalar: every test on it becomes a scalar branch
@@ -73,13 +86,14 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
     // (row c32, column 8g) and a transposing read as lds_read_tr_operand_perm lays it out.
     const int row_lane = lds_row<D>(c32) * S + g * 8;
     const int tr_lane = lds_row<D>(4 * g + ((lane & 15) >> 2)) * S + TrMap<D>::src_col(0, (lane >> 4) & 1, lane & 3);
-    const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv;
+    const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv, hs = JOINED ? a.head_split : 1;
     // Full-causal: key block i is seen by T - 128i queries.
-    int blk, rr, kvu;
+    int blk = jblk, rr = share, kvu = jkvu;
     // Band mask with a few sink keys: the queries past block 0's band are cut into chunks that get
     // workgroups of their own (ids nkb .. nkb + nch - 1 of the unit), see sink_tail.
     const SinkTail tl = TAIL ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
-    if (TAIL) {
+    if (JOINED) {
+    } else if (TAIL) {
         if (!xcd_map(nkb + tl.nch, 1, a.Hkv * a.B, blk, rr, kvu)) return;
     } else if (a.window > 0 && a.sinks > 0 && nkb > 1) {
         if (!xcd_map_block0_first(nkb, a.Hkv * a.B, blk, kvu)) return;
@@ -88,9 +102,9 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
     }
     const int chunk = (TAIL && blk >= nkb) ? blk - nkb : -1;  // >= 0: this workgroup takes a chunk of the sink tail
     if (TAIL && chunk >= 0) blk = 0;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv;
+    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = JOINED ? rr * rep / hs : 0, nh = JOINED ? (rr + 1) * rep / hs - h0 : rep;
     const float cexp = a.scale * LOG2E;
-    const int npass = (a.paired && blk != nkb - 1 - blk) ? 2 : 1;
+    const int npass = (!JOINED && a.paired && blk != nkb - 1 - blk) ? 2 : 1;
 
     for (int pass = 0; pass < npass; ++pass) {
         const int kblk = pass == 0 ? blk : nkb - 1 - blk;  // heavy block first
@@ -126,15 +140,15 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
             qt_hi = tl.q0 / BMQ - 1;  // the band part of block 0 ends where the chunks begin, whatever the block size
         }
         const int nqt = qt_hi - qt_lo + 1;
-        const int steps = nqt * rep;
+        const int steps = nqt * nh;
 
-        u32x4 qr[CPT], gr[CPT];
+        u32x4 qr[CPT], gr[CPT], orow[JOINED ? CPT : 1];
         float lse_r = 0.0f, dl_r = 0.0f;
         // Steps are fetched in order, so the (head, query tile) of the next fetch is counted up, not divided out of
         // the step number, and a thread's position inside a tile (row tid / NCH + RPI i, chunk tid % NCH) is formed once.
         // (Tile positions as scalar bases plus per-thread 32-bit offsets, as the 64-key kernel keeps them, take a
         // third of the vector instructions out of the staging and measured no faster here, slower at head_dim 64.)
-        int f_h = hk * rep, f_qt = 0;
+        int f_h = hk * rep + h0, f_qt = 0;
         const int frow = static_cast<int>(threadIdx.x) / NCH, fch = static_cast<int>(threadIdx.x) % NCH;
         constexpr int RPI = NTHR / NCH;  // tile rows between a thread's consecutive chunks
         auto fetch = [&]() {  // global -> registers, rows past the end clamped
@@ -146,12 +160,14 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
                 const int t = min(q0 + frow + RPI * i, a.T - 1);
                 qr[i] = *reinterpret_cast<const u32x4*>(qb + t * a.q_st);
                 gr[i] = *reinterpret_cast<const u32x4*>(gb + t * a.do_st);
+                if (JOINED)
+                    orow[i] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.o) + b * a.o_sb + f_h * a.o_sh + fch * 8 + t * a.o_st);
             }
             if (threadIdx.x < BMQ) {
                 const int t = min(q0 + static_cast<int>(threadIdx.x), a.T - 1);
                 const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + f_h) * a.T + t;
                 lse_r = a.lse[lrow];  // scaled when it is stored: arithmetic on it here would wait for every load just issued
-                dl_r = a.delta[lrow];
+                if (!JOINED) dl_r = a.delta[lrow];
             }
             const bool wrap = f_qt + 1 == nqt;
             f_qt = wrap ? 0 : f_qt + 1;
@@ -169,10 +185,23 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
                 const int row = c / NCH, ch = c % NCH;
                 *reinterpret_cast<u32x4*>(Qs[slot] + lds_row<D>(row) * S + ch * 8) = qr[i];
                 *reinterpret_cast<u32x4*>(dOs[slot] + lds_row<D>(row) * S + ch * 8) = gr[i];
+                if (JOINED) {
+                    float part = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        part = fmaf(__uint_as_float(orow[i][e] << 16), __uint_as_float(gr[i][e] << 16), part);
+                        part = fmaf(__uint_as_float(orow[i][e] & 0xFFFF0000u), __uint_as_float(gr[i][e] & 0xFFFF0000u), part);
+                    }
+                    part += lane_swapped<0xB1>(part);   // lane ^ 1
+                    part += lane_swapped<0x4E>(part);   // lane ^ 2
+                    part += lane_swapped<0x141>(part);  // the other four of eight
+                    if (NCH == 16) part += lane_swapped<0x140>(part);  // the other eight of sixteen
+                    if (ch == 0) dl_s[slot][row] = part;
+                }
             }
             if (tid < BMQ) {
                 nlse_s[slot][tid] = -lse_r * LOG2E;
-                dl_s[slot][tid] = dl_r;
+                if (!JOINED) dl_s[slot][tid] = dl_r;
             }
         };
         // wavefront-uniform: is anything of (query block qb of the step at query tile `qt`) x (this key block) visible?
@@ -347,7 +376,18 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
                     store4g<true>(rows, TrMap<D>::col0(db, qd, g), acc[db][qd * 4] * sc, acc[db][qd * 4 + 1] * sc,
                                   acc[db][qd * 4 + 2] * sc, acc[db][qd * 4 + 3] * sc);
         }
-        if (kj < a.T && chunk < 0 && !(piece && kj < a.sinks)) {
+        if (JOINED && hs > 1) {  // partial sums of this share of the heads, for launch_gqa_reduce
+            if (kj < a.T) {
+                const int64_t row = ((static_cast<int64_t>(kvu) * hs + rr) * 2 + (rl == 0 ? 1 : 0)) * a.T + kj;
+                const float sc = rl == 0 ? 1.0f : a.scale;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int qd = 0; qd < 4; ++qd)
+                        store4g<true>(a.part, row * D + TrMap<D>::col0(db, qd, g), acc[db][qd * 4] * sc, acc[db][qd * 4 + 1] * sc,
+                                      acc[db][qd * 4 + 2] * sc, acc[db][qd * 4 + 3] * sc);
+            }
+        } else if (kj < a.T && chunk < 0 && !(piece && kj < a.sinks)) {
             void* dst = rl == 0 ? a.dv : a.dk;
             const int64_t ob = rl == 0 ? b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st
                                          : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
@@ -371,6 +411,43 @@ __global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
             run_role(std::integral_constant<int, 1>{});
         __syncthreads();  // the next pass refills the ring
     }
+}
+template <int D, bool GF32, bool TAIL, int BNK, int BMQ>
+__global__ __launch_bounds__(4 * BNK, 2) void mfma_dkdv2(AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) Ring<D, BMQ> tiles;
+    __shared__ __attribute__((aligned(16))) Weights<BNK, BMQ> Pbuf;
+    __shared__ __attribute__((aligned(16))) Rows<BMQ> nlse_s;  // -LSE * log2(e)
+    __shared__ __attribute__((aligned(16))) Rows<BMQ> dl_s;
+    dkdv2_blocks<D, GF32, TAIL, BNK, BMQ, false>(a, tiles, Pbuf, nlse_s, dl_s);
+}
+
+// ---- dQ and dK/dV at head_dim 128 in one launch: blocks of 64 keys and of 128 queries (joined_takes_bwd) ----
+// By rank: two blocks of keys for each share of the group's heads and one of queries for each head. Under a band every unit's block of sink keys comes first, then
+// a unit's blocks along its band; else the longest of every unit.
+template <bool GF32>
+__global__ __launch_bounds__(256, 2) void joined_bwd(AttnArgs a) {
+    __shared__ union {
+        struct {
+            __attribute__((aligned(16))) Ring<128, 32> tiles;
+            __attribute__((aligned(16))) Weights<64, 32> p;
+            __attribute__((aligned(16))) Rows<32> nlse, delta;
+        } k;
+        __attribute__((aligned(16))) uint16_t q[DQ_LDS<128, 4>];
+    } lds;
+    const int nkb = (a.T + 63) / 64, ranks = (a.T + 127) / 128, rep = a.Hq / a.Hkv, keys = 2 * a.head_split, each = keys + rep;
+    int rank, r, kvu, at;
+    if (a.window > 0) {
+        if (!xcd_map_block0_first(ranks * each, a.Hkv * a.B, at, kvu)) return;
+        rank = at / each, r = at % each;
+    } else if (a.causal && ranks > 1 ? !xcd_map_block_major(ranks, each, a.Hkv * a.B, rank, r, kvu)
+                                     : !xcd_map(ranks, each, a.Hkv * a.B, rank, r, kvu)) {
+        return;
+    }
+    const int hk = kvu % a.Hkv;
+    if (r >= keys)
+        dq_block<128, GF32, true, 4>(a, kvu / a.Hkv, hk * rep + r - keys, hk, a.window > 0 ? rank : ranks - 1 - rank, lds.q);
+    else if (2 * rank + r % 2 < nkb)
+        dkdv2_blocks<128, GF32, false, 64, 32, true>(a, lds.k.tiles, lds.k.p, lds.k.nlse, lds.k.delta, 2 * rank + r % 2, kvu, r / 2);
 }
 
 // dK / dV rows [0, sinks) of every (batch, KV head) = the band part plus the chunks, in that order. One element a thread: a
@@ -476,6 +553,40 @@ int launch_sink_tail_reduce(const AttnArgs& a, hipStream_t st) {
     return PK_OK;
 }
 
+// Where either launch by itself is a round of the chip or less, its longest chains last as long as it does, and together one's run beside the
+// other's; dK/dV forms delta while it moves its tiles, 20 vector instructions a 16-byte chunk. From 4096 tokens on without a band the launches
+// stay apart, which keeps dQ's bits whatever the number of units. In 64-row blocks of queries (q), one after the other | joined, us:
+//   causal     T 222 x 5, 16 heads (320) 27 | 20;  T 79 x 18, 4 heads (144) 18 | 11;  T 571 x 2, 8 heads (144) 41 | 32;  T 1792, 16 heads (448) 111 | 101;
+//              T 307 x 4, 16 on 8 (320) 48 | 35;  T 739, 28 on 4 (336) 67 | 54;  T 2531, 7 on one (280) 152 | 134
+//     not      T 609 x 6, 1 head (60) 25 | 34;  T 1423, 8 heads (184) 64 | 74;  T 3991, 4 on 2 (252) 175 | 191;  T 2422 x 3, 8 heads (912) 164 | 200
+//   no mask    T 54 x 10, 8 heads (80) 14.5 | 8.5;  T 1061 x 4, 2 heads (136) 88 | 59;  T 2309, 8 heads (296) 172 | 140;  T 611, 28 on 4 (280) 70 | 52
+//     not      T 1229, 4 heads (80) 54 | 67;  T 352 x 16, 4 heads (384) 40 | 42;  T 1461 x 3, 7 on one (483) 136 | 175
+//   band       T 559 x 4, 8 heads, 71 (288) 30 | 20;  T 140 x 11, 8 heads, 27, 1 sink (264) 24 | 16;  T 1317, 16 on 8, 123 (336) 36 | 28
+//     not      with sinks in long sequences, whose block is walked whole (T 1409, 16 heads, 325 (368) 59 | 87; T 394, 28 on 4, 74 (196) 126 | 145);
+//              T 59 x 29, 16 heads (464) 24 | 29;  T 2839, 14 on 2, 154 (630) 57 | 89
+bool joined_takes_bwd(const AttnArgs& a) {
+    if (a.dk_dim != 128) return false;
+    const bool groups = a.Hq > a.Hkv;
+    const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
+    if (a.window > 0)
+        return a.window <= 512 && (a.sinks == 0 || a.T <= (groups ? 160 : 700)) && q >= (groups ? 76 : 52) && q <= (a.T <= 64 ? 320 : 600);
+    if (a.T >= 4096) return false;
+    if (a.T <= 130) return q >= 56 && q <= 500;
+    if (!a.causal) return q >= 120 && q <= 340;
+    return a.T <= 800 ? q >= 140 && q <= 600 : q >= (a.T <= 2600 ? 260 : 320) && q <= 500;
+}
+int launch_joined_bwd(const AttnArgs& a_in, hipStream_t st) {
+    AttnArgs a = a_in;
+    if (!bf16_deals_heads(a)) a.head_split = 1;
+    const int ranks = (a.T + 127) / 128, each = 2 * a.head_split + a.Hq / a.Hkv;
+    const dim3 grid(a.window > 0 ? xcd_grid_block0_first(ranks * each, a.Hkv * a.B) : xcd_grid(ranks, each, a.Hkv * a.B));
+    if (a.grad_f32)
+        hipLaunchKernelGGL(joined_bwd<true>, grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(joined_bwd<false>, grid, dim3(256), 0, st, a);
+    PK_HIP(hipGetLastError());
+    return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
+}
 int launch_mfma_dkdv2(const AttnArgs& a, hipStream_t st) {
     if (a.dk_dim == 128) return a.grad_f32 ? launch<128, true>(a, st) : launch<128, false>(a, st);
     return a.grad_f32 ? launch<64, true>(a, st) : launch<64, false>(a, st);

@@ -211,6 +211,8 @@ int launch_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
 bool bf16_deals_heads(const AttnArgs& a);  // its dK/dV kernel for this launch uses a.head_split and a.part
 int launch_mfma_dkdv2(const AttnArgs& a, hipStream_t st);
+bool joined_takes_bwd(const AttnArgs& a);  // attn_bwd_dkdv2.hip: dQ (with delta) and dK/dV in one launch, head_dim 128
+int launch_joined_bwd(const AttnArgs& a, hipStream_t st);
 // attn_bwd_dkdv3.hip: dK / dV with 64 keys per wavefront and hand-fixed register classes (head_dim 64 or 128, no band)
 bool mfma_dkdv3_takes(const AttnArgs& a);
 int launch_mfma_dkdv3(const AttnArgs& a, hipStream_t st);

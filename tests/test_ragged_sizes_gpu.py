@@ -414,6 +414,30 @@ def test_bf16_backward_of_joined_blocks(case, dk):
     assert max(e) < (4e-3 if dk == 64 else 2e-6), e
 
 
+# The same at head_dim 128, blocks of 64 keys and of 128 queries: one row past a tile and past either block, an odd number of blocks of keys,
+# bands with and without sinks, both gradient types.
+@pytest.mark.parametrize("grad", [torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("case", [(9, 33, 9, 9, True, 0, 0), (11, 65, 5, 5, False, 0, 0), (13, 129, 9, 9, True, 0, 0), (4, 577, 7, 7, True, 0, 0), (3, 700, 6, 6, False, 0, 0),
+                                  (1, 1793, 12, 12, True, 0, 0), (6, 321, 9, 9, True, 33, 17), (1, 4200, 3, 3, True, 100, 0), (3, 161, 28, 4, True, 0, 0),
+                                  (1, 700, 14, 2, False, 0, 0), (2, 450, 16, 4, True, 60, 0)], ids=str)
+def test_bf16_backward_of_joined_blocks_at_128(case, grad):
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
+    q, k, v = cut(torch.randn((B, T, Hq + 2 * Hkv, 128), generator=gen, device="cuda").bfloat16())
+    d_o = torch.randn((B, Hq, T, 128), generator=gen, device="cuda").bfloat16().permute(0, 2, 1, 3)
+    scale = float(np.float32(1.0 / np.sqrt(128)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    o_view = torch.full((B, T, 2 * Hq, 128), float("nan"), device="cuda").bfloat16()[:, :, :Hq]
+    o_view.copy_(o)
+    one = ops.attn_bwd(q, k, v, o_view, lse, d_o, scale, causal, window, sinks, grad_dtype=grad)
+    again = ops.attn_bwd(*(x.contiguous() for x in (q, k, v, o)), lse, d_o.contiguous(), scale, causal, window, sinks, grad_dtype=grad)
+    assert all(torch.equal(x, y) for x, y in zip(one, again))
+    want = exact_attention(q, k, v, d_o, scale, causal, window, sinks, o)[2:]
+    e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(one, want)]
+    assert max(e) < 4e-3, e  # P and dS as one bf16 operand, and the gradient's own rounding
+
+
 # A training loop that keeps no tensors it can do without: dQ where O was, dK and dV where K and V were. Small launches and large ones,
 # groups of heads dealt out, dealt sink tails, head sizes of every kernel family. The same bits as dQ and then dK/dV into buffers of
 # their own, which read what they read in this order.
