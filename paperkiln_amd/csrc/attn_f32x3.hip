@@ -833,7 +833,7 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
 
 // ---- dK, dV and dQ in one launch, delta read (f32x3_takes_bwd) ----
 template <int D>
-__global__ __launch_bounds__(256, 2) void x3_bwd(AttnArgs a) {
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
     constexpr int Q = dq_lds<D, 2, 2>(), K = 2 * DKDV_TILE<D, 2>, N = Q > K + 4096 ? Q : K + 4096;
     __shared__ __attribute__((aligned(16))) uint16_t lds[N];
     const JoinedBlocks jb(a, 64);
@@ -1078,18 +1078,26 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 //     below      T 963, 4 heads (64) 50 | 66;   T 894 x 4, 2 heads (112) 45 | 60;   T 3305, 4 heads on 2 (208) 197 | 202
 //     above      T 5833, 8 heads (736) 688 | 710;   T 1024 x 8, 16 heads (2048) 351 | 362;   T 4096 x 4, 16 heads (4096) 2417 | 2562
 //   32 columns   T 1037 x 2, 8 heads (272) 62 | 50;   T 181 x 13, 16 heads (624) 42 | 29;   no mask, T 1639, 8 heads (208) 109 | 88
+//   128 columns, one workgroup to a CU   T 270 x 3, 16 heads (240) 122 | 58;   T 1796, 2 heads (58) 240 | 196;   T 2132, 8 heads (272) 393 | 280;
+//                no mask, T 710, 8 heads (96) 127 | 90;   above: T 440 x 19, 4 heads (532) 146 | 158;   no mask, T 1010 x 14, 2 heads (448) 353 | 388
+//   96 columns   T 241 x 10, 4 heads (160) 52 | 33;   T 936, 16 heads of 80 (240) 131 | 97;   below, above: T 2413, 4 heads of 80 (152) 184 | 210;   T 2309 x 2,
+//                8 heads (592) 421 | 499
 //   bands, every head its own: 48, T 165 x 6, 8 heads, window 86 (144) 36 | 20;   T 4383, 8 heads, 26 (552) 51 | 42;   T 975 x 13, 2 heads of 64, 408,
 //     1 sink (416) 109 | 79;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
 //     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
 bool f32x3_takes_bwd(const AttnArgs& a) {
-    if (!f32_split_serves(a) || a.dk_dim > 64 || a.T <= 32) return false;
+    if (!f32_split_serves(a) || a.T <= 32) return false;
     const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
-    if (a.window > 0) return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= 300) && q >= (a.dk_dim <= 32 ? 130 : 100) && q <= 800;
+    if (a.window > 0)
+        return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= (a.dk_dim > 96 ? 600 : 300)) &&
+               q >= (a.dk_dim <= 32 ? 130 : a.dk_dim <= 64 ? 100 : a.dk_dim <= 96 ? 88 : 40) && q <= (a.dk_dim <= 64 ? 800 : 420);
+    if (a.dk_dim > 96) return q >= 40 && q <= (a.causal ? 420 : a.T <= 130 ? 200 : 260);
+    if (a.dk_dim > 64) return q >= (a.causal && a.T > 300 && a.T <= 2600 ? 170 : 88) && q <= (a.causal ? 330 : 300);
     if (a.dk_dim <= 32) return !a.causal ? q >= 180 && q <= 440 : q >= (a.T <= 130 ? 104 : a.T <= 600 ? 190 : 260) && q <= 640;
     if (!a.causal) return q >= 120 && q <= 960;
     return q >= (a.T <= 600 ? 140 : a.T <= 2000 ? 180 : 260) && q <= (a.T <= 1500 ? 1100 : 700);
 }
-int launch_f32x3_bwd(const AttnArgs& a, hipStream_t st) { return a.dk_dim <= 32 ? run_bwd<32>(a, st) : run_bwd<64>(a, st); }
+int launch_f32x3_bwd(const AttnArgs& a, hipStream_t st) { return a.dk_dim <= 32 ? run_bwd<32>(a, st) : a.dk_dim <= 64 ? run_bwd<64>(a, st) : a.dk_dim <= 96 ? run_bwd<96>(a, st) : run_bwd<128>(a, st); }
 int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st) {
     if (a.dk_dim <= 32) return run_dkdv<32, 2>(a, st);
     if (a.dk_dim <= 64) return run_dkdv<64, 2>(a, st);

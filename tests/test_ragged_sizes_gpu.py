@@ -369,7 +369,7 @@ def test_backward_in_one_launch(case, dtype, dk):
 
 # fp32 blocks of 64 keys and of 64 queries in one launch behind one of delta: one row past a block and a tile, more ranks than heads, groups
 # whose heads are dealt out, units that do not divide by the 8 XCDs, the shortest chains and the most blocks that go together.
-@pytest.mark.parametrize("dk", [4, 32, 44, 64])
+@pytest.mark.parametrize("dk", [4, 32, 44, 64, 80, 96, 100, 128])
 @pytest.mark.parametrize("case", [(18, 33, 16, 16, True, 0, 0), (7, 65, 16, 8, True, 0, 0), (9, 129, 14, 2, True, 0, 0), (2, 641, 13, 13, True, 0, 0),
                                   (5, 577, 8, 8, False, 0, 0), (1, 2113, 8, 2, True, 0, 0), (40, 257, 3, 3, True, 0, 0), (6, 321, 9, 9, True, 33, 17),
                                   (1, 1100, 11, 11, True, 100, 0)], ids=str)
