@@ -86,7 +86,7 @@ __device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weig
     // (row c32, column 8g) and a transposing read as lds_read_tr_operand_perm lays it out.
     const int row_lane = lds_row<D>(c32) * S + g * 8;
     const int tr_lane = lds_row<D>(4 * g + ((lane & 15) >> 2)) * S + TrMap<D>::src_col(0, (lane >> 4) & 1, lane & 3);
-    const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv, hs = JOINED ? a.head_split : 1;
+    const int nkb = (a.T + BNK - 1) / BNK, rep = quotient(a.Hq, a.Hkv), hs = JOINED ? a.head_split : 1;
     // Full-causal: key block i is seen by T - 128i queries.
     int blk = jblk, rr = share, kvu = jkvu;
     // Band mask with a few sink keys: the queries past block 0's band are cut into chunks that get
@@ -102,7 +102,7 @@ __device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weig
     }
     const int chunk = (TAIL && blk >= nkb) ? blk - nkb : -1;  // >= 0: this workgroup takes a chunk of the sink tail
     if (TAIL && chunk >= 0) blk = 0;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = JOINED ? rr * rep / hs : 0, nh = JOINED ? (rr + 1) * rep / hs - h0 : rep;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h0 = JOINED ? quotient(rr * rep, hs) : 0, nh = JOINED ? quotient((rr + 1) * rep, hs) - h0 : rep;
     const float cexp = a.scale * LOG2E;
     const int npass = (!JOINED && a.paired && blk != nkb - 1 - blk) ? 2 : 1;
 
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(256, 2) void joined_bwd(AttnArgs a) {
         } k;
         __attribute__((aligned(16))) uint16_t q[DQ_LDS<128, 4>];
     } lds;
-    const int nkb = (a.T + 63) / 64, ranks = (a.T + 127) / 128, rep = a.Hq / a.Hkv, keys = 2 * a.head_split, each = keys + rep;
+    const int nkb = (a.T + 63) / 64, ranks = (a.T + 127) / 128, rep = quotient(a.Hq, a.Hkv), keys = 2 * a.head_split, each = keys + rep;
     int rank, r, kvu, at;
     if (a.window > 0) {
         if (!xcd_map_block0_first(ranks * each, a.Hkv * a.B, at, kvu)) return;
@@ -443,9 +443,9 @@ __global__ __launch_bounds__(256, 2) void joined_bwd(AttnArgs a) {
                                      : !xcd_map(ranks, each, a.Hkv * a.B, rank, r, kvu)) {
         return;
     }
-    const int hk = kvu % a.Hkv;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
     if (r >= keys)
-        dq_block<128, GF32, true, 4>(a, kvu / a.Hkv, hk * rep + r - keys, hk, a.window > 0 ? rank : ranks - 1 - rank, lds.q);
+        dq_block<128, GF32, true, 4>(a, b, hk * rep + r - keys, hk, a.window > 0 ? rank : ranks - 1 - rank, lds.q);
     else if (2 * rank + r % 2 < nkb)
         dkdv2_blocks<128, GF32, false, 64, 32, true>(a, lds.k.tiles, lds.k.p, lds.k.nlse, lds.k.delta, 2 * rank + r % 2, kvu, r / 2);
 }

@@ -107,10 +107,10 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
-    const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
+    const int nqb = (a.T + BM - 1) / BM, rep = quotient(a.Hq, a.Hkv);
     int blk, rr, kvu;
     if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h = hk * rep + rr;
     const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
     const float cexp = a.scale * LOG2E;
 

@@ -59,12 +59,12 @@ __global__ __launch_bounds__(256) void mfma_delta(AttnArgs a) {
 template <int D, bool GF32, bool FUSE_DELTA, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void mfma_dq(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t lds[DQ_LDS<D, NW>];
-    const int nqb = (a.T + 32 * NW - 1) / (32 * NW), rep = a.Hq / a.Hkv;
+    const int nqb = (a.T + 32 * NW - 1) / (32 * NW), rep = quotient(a.Hq, a.Hkv);
     int blk, rr, kvu;
     if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
-    const int hk = kvu % a.Hkv, npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
     for (int pass = 0; pass < npass; ++pass) {
-        dq_block<D, GF32, FUSE_DELTA, NW>(a, kvu / a.Hkv, hk * rep + rr, hk, pass == 0 ? nqb - 1 - blk : blk, lds);
+        dq_block<D, GF32, FUSE_DELTA, NW>(a, b, hk * rep + rr, hk, pass == 0 ? nqb - 1 - blk : blk, lds);
         __syncthreads();  // the next pass refills the tile buffers
     }
 }

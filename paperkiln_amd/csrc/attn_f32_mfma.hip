@@ -80,10 +80,10 @@ __global__ __launch_bounds__(256, 2) void f32_fwd(AttnArgs a) {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
-    const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
+    const int nqb = (a.T + BM - 1) / BM, rep = quotient(a.Hq, a.Hkv);
     int blk, rr, kvu;
     if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h = hk * rep + rr;
     const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int q0 = (pass == 0 ? nqb - 1 - blk : blk) * BM;
@@ -218,10 +218,10 @@ __global__ __launch_bounds__(256, D == 32 ? 3 : D == 64 ? 2 : 1) void f32_dq(Att
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
-    const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
+    const int nqb = (a.T + BM - 1) / BM, rep = quotient(a.Hq, a.Hkv);
     int blk, rr, kvu;
     if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h = hk * rep + rr;
     const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int q0 = (pass == 0 ? nqb - 1 - blk : blk) * BM;
@@ -411,13 +411,13 @@ __global__ __launch_bounds__(512, 1) void f32_dkdv(AttnArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int role = w >> 2, kbw = w & 3;
     const int g = lane >> 5, c32 = lane & 31;
-    const int nkb = (a.T + BNK - 1) / BNK, rep = a.Hq / a.Hkv;
+    const int nkb = (a.T + BNK - 1) / BNK, rep = quotient(a.Hq, a.Hkv);
     const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
     int blk0, rr, kvu;
     if (!map_causal_blocks(a, nkb + tl.nch, 1, blk0, rr, kvu)) return;
     const int chunk = blk0 >= nkb ? blk0 - nkb : -1;
     if (chunk >= 0) blk0 = 0;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
     const float cexp = a.scale * LOG2E;
     const int npass = (a.paired && blk0 != nkb - 1 - blk0) ? 2 : 1;
 

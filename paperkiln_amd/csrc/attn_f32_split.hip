@@ -20,6 +20,20 @@ constexpr float LOG2E = 1.4426950408889634f;
 __device__ inline f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 __device__ inline int crow(int r, int g) { return (r >> 2) * 8 + 4 * g + (r & 3); }
 
+// A head's first element. The value is formed here and kept: left to itself the compiler reads the arguments again, a round trip through the
+// scalar cache each, wherever the next tensor is addressed -- seven times before the first product.
+__device__ inline const float* head_of(const void* base, int64_t sb, int b, int64_t sh, int h) {
+    const float* p = static_cast<const float*>(base) + (b * sb + h * sh);
+    asm volatile("" : "+s"(p));
+    return p;
+}
+// rows r0 .. T - 1 of a head; r0 < T. Whatever lies past them reads as zero.
+__device__ inline __amdgpu_buffer_rsrc_t rows_from(const float* head, int st, int r0, int T, int dk) {
+    const int64_t left = (static_cast<int64_t>(T - r0 - 1) * st + dk) * 4;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(head) + static_cast<int64_t>(r0) * st, 0,
+                                             left > 0x7fffffff ? 0x7fffffff : static_cast<int>(left), 0x00020000);
+}
+
 // A 32-row tile of a [T, dk] fp32 matrix, moved by one wavefront through a buffer resource (rows past T and chunks past
 // dk read as zero) into LDS rows of pitch D + 4: 16-byte row reads of 16 rows then touch all 64 banks once.
 template <int D>
@@ -27,18 +41,15 @@ struct Mover32 {
     static constexpr int NCH = D / 4, CPT = 32 * NCH / 64, P = D + 4;
     int off[CPT];
     u32x4 r[CPT];
-    __device__ void init(int lane, int64_t st, int dk) {
+    __device__ void init(int lane, int st, int dk) {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int c = lane + 64 * i, row = c / NCH, ch = c % NCH;
-            off[i] = ch * 4 < dk ? static_cast<int>(row * st + ch * 4) * 4 : static_cast<int>(OUTSIDE);
+            off[i] = ch * 4 < dk ? (row * st + ch * 4) * 4 : static_cast<int>(OUTSIDE);
         }
     }
-    __device__ void load(const void* base, int64_t elem_off, int64_t st, int r0, int T, int dk) {
-        const int64_t left = ((static_cast<int64_t>(T) - r0 - 1) * st + dk) * 4;  // r0 < T
-        float* p = static_cast<float*>(const_cast<void*>(base)) + elem_off + static_cast<int64_t>(r0) * st;
-        const __amdgpu_buffer_rsrc_t rs =
-            __builtin_amdgcn_make_buffer_rsrc(p, 0, left > 0x7fffffff ? 0x7fffffff : static_cast<int>(left), 0x00020000);
+    __device__ void load(const float* head, int st, int r0, int T, int dk) {
+        const __amdgpu_buffer_rsrc_t rs = rows_from(head, st, r0, T, dk);
 #pragma unroll
         for (int i = 0; i < CPT; ++i) r[i] = tile_load16(rs, off[i]);
     }
@@ -51,14 +62,27 @@ struct Mover32 {
     }
 };
 
-// Row `row` of a head as an operand: chunk j holds columns 8j + 4g .. +3; zero past T and past dk.
+// Row r0 + c32 of a head as an operand: chunk j holds columns 8j + 4g .. +3; zero past T and past dk.
 template <int D>
-__device__ inline void load_row32(const void* base, int64_t off, int64_t st, int row, int T, int dk, int g, f32x4* out) {
+__device__ inline void load_row32(const float* head, int st, int r0, int T, int dk, int c32, int g, f32x4* out) {
+    const __amdgpu_buffer_rsrc_t rs = rows_from(head, st, r0, T, dk);
+    const int row = c32 * st * 4 + 16 * g;
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) {
+        const u32x4 v = tile_load16(rs, 8 * j + 4 * g < dk ? row + 32 * j : static_cast<int>(OUTSIDE));
+        out[j] = *reinterpret_cast<const f32x4*>(&v);
+    }
+}
+
+// The same of a tensor with any row stride (O's is not asked about). The branch around each load keeps it where it is written: free to move, the
+// scheduler holds the row through the products before its use (backward, 128 columns, T 300, 4 heads: 46.5 us | 52.6; 32, T 2900, 4 heads 86 | 96).
+template <int D>
+__device__ inline void load_row_of_o(const float* head, int64_t st, int row, int T, int dk, int g, f32x4* out) {
 #pragma unroll
     for (int j = 0; j < D / 8; ++j) {
         const int col = 8 * j + 4 * g;
         f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (row < T && col < dk) z = *reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + off + row * st + col);
+        if (row < T && col < dk) z = *reinterpret_cast<const f32x4*>(head + row * st + col);
         out[j] = z;
     }
 }
@@ -114,6 +138,51 @@ __device__ inline void accumulate_tr32(const float* tile, const f32x16& c, f32x1
     }
 }
 
+// The KW wavefronts' accumulators of N blocks added up, in wavefront order: the 4 N quads of eight columns are dealt out, one to each wavefront
+// in turn, so that all of them add and store (block by block, three of four wavefronts watch one at 32 columns). `red`: 1024 N KW floats of LDS,
+// free to overwrite. `out` takes (block, quad, sum). weights(), asked for behind the barrier: what wavefront k's part is multiplied by, or nullptr.
+template <int N, int KW, typename W, typename F>
+__device__ inline void join_quads(const f32x16* acc, float* red, int kg, int lane, W weights, F out) {
+    constexpr int ITEMS = 4 * N;
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+            const f32x4 v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
+            *(reinterpret_cast<f32x4*>(red) + (kg * ITEMS + n * 4 + qd) * 64 + lane) = v;
+        }
+    __syncthreads();
+    const float* const weight = weights();
+#pragma unroll
+    for (int i = 0; i < (ITEMS + KW - 1) / KW; ++i) {
+        const int item = i * KW + kg;
+        if (ITEMS % KW != 0 && item >= ITEMS) break;
+        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const f32x4 v = *(reinterpret_cast<const f32x4*>(red) + (k * ITEMS + item) * 64 + lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = weight ? fmaf(v[e], weight[k], s[e]) : s[e] + v[e];
+        }
+        out(item / 4, item % 4, s);
+    }
+}
+// a quad of a lane's output row
+__device__ inline void store_quad(void* base, int64_t row_off, int db, int qd, int g, const f32x4& v, float sc, int dk) {
+    const int col = 32 * db + 8 * qd + 4 * g;
+    const f32x4 o = {v[0] * sc, v[1] * sc, v[2] * sc, v[3] * sc};
+    if (col < dk) *reinterpret_cast<f32x4*>(static_cast<float*>(base) + row_off + col) = o;
+}
+
+// Both tensors of a wavefront's next tile on their way together, or one behind the other's product. Where chains are a tile or two, as in
+// most launches of these kernels, the second trip to memory is a fifth of the launch. Above 64 columns the registers do not hold both; dQ and
+// dK/dV take it at 32 columns in one launch (by themselves they run four and three wavefronts to a SIMD; at 64 T 512, 8 heads is 28.0 us | 29.5).
+//
+// With it, the addresses formed once (head_of) and all wavefronts in the join, T 128 x 2, 4 heads of 32: forward 5.6 -> 4.9 us, backward 9.7 -> 8.5; T 2900,
+// 4 heads 37.7 -> 37.2, 99.9 -> 86.1; 128 columns, T 300, 4 heads 21.2 -> 20.6, 55.2 -> 46.5; 96, no mask, T 700, 4 heads 29.5 -> 28.1, 56.1 -> 56.5.
+template <int D>
+constexpr bool BOTH_AHEAD = D <= 64;
+
 // ---- forward ----
 // The launch bounds ask for the wavefronts that the LDS leaves room for: four to a SIMD at head_dim 32, two at 64 (backward,
 // head_dim 24, T 402 x 22, 16 heads: 204 -> 173 us; head_dim 64, T 731 x 4, 28 heads on 4, window 309: 296 -> 242).
@@ -126,19 +195,20 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
     int b, h, hk, qblk;
     if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk)) return;
     const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
-    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float *const kh = head_of(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of(a.v, a.v_sb, b, a.v_sh, hk), *const qh = head_of(a.q, a.q_sb, b, a.q_sh, h);
+    const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
     float* const Ks = lds + kg * TILE;
     float* const Vs = Ks + 32 * P;
 
     Mover32<D> mk, mv;
-    mk.init(lane, a.k_st, dk);
-    mv.init(lane, a.v_st, dk);
+    mk.init(lane, k_st, dk);
+    mv.init(lane, v_st, dk);
     const KeyTiles kt(a, q0, 32, 32);
-    // one tensor in flight at a time: V of a tile behind its S product, K of the next tile behind the rest
-    if (kg < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(kg) * 32, a.T, dk);
+    if (kg < kt.n) mk.load(kh, k_st, kt.tile(kg) * 32, a.T, dk);
     f32x4 qreg[D / 8];
-    load_row32<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    load_row32<D>(qh, static_cast<int>(a.q_st), q0, a.T, dk, c32, g, qreg);
+    if (BOTH_AHEAD<D> && kg < kt.n) mv.load(vh, v_st, kt.tile(kg) * 32, a.T, dk);
     f32x16 acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -151,11 +221,14 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
         const int k0 = kt.tile(at) * 32;
         mk.store(Ks, lane);
         tile_barrier<1>();
-        mv.load(a.v, vb, a.v_st, k0, a.T, dk);
+        if (!BOTH_AHEAD<D>) mv.load(vh, v_st, k0, a.T, dk);
         f32x16 s = rows_dot<D>(Ks, [&](int j) { return qreg[j]; }, c32, g);
         mv.store(Vs, lane);
         tile_barrier<1>();
-        if (at + KW < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(at + KW) * 32, a.T, dk);
+        if (at + KW < kt.n) {
+            mk.load(kh, k_st, kt.tile(at + KW) * 32, a.T, dk);
+            if (BOTH_AHEAD<D>) mv.load(vh, v_st, kt.tile(at + KW) * 32, a.T, dk);
+        }
         if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= q0 && k0 >= a.sinks))) {
             const MaskKind kind = mask_kind(k0, k0 + 31, q0, qhi, a.T, a.causal, a.window, a.sinks);
             if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, -INFINITY);
@@ -190,26 +263,21 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
     float* ml = lds + KW * DB * 1024;
     ml[kg * 128 + lane] = m;
     ml[kg * 128 + 64 + lane] = l;
-    __syncthreads();
-    float mt = m, lt = 0.0f;
+    const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+    float mt = m, lt = 0.0f, weight[KW];
+    join_quads<DB, KW>(acc, lds, kg, lane, [&]() {
 #pragma unroll
-    for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
+        for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
 #pragma unroll
-    for (int k = 0; k < KW; ++k) lt += ml[k * 128 + 64 + lane] * __builtin_amdgcn_exp2f((ml[k * 128 + lane] - mt) * cexp);
-    const float alpha = __builtin_amdgcn_exp2f((m - mt) * cexp);
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
-    join_groups<DB, KW>(acc, lds, kg, lane);
-    if (qi < a.T) {
-        const float inv = 1.0f / lt;
-        const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-            if (db % KW == kg) store_block(true, a.o, ro, db, g, acc[db], inv, dk);
-        if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = mt * a.scale + logf(lt);
-    }
+        for (int k = 0; k < KW; ++k) {
+            weight[k] = __builtin_amdgcn_exp2f((ml[k * 128 + lane] - mt) * cexp);
+            lt += ml[k * 128 + 64 + lane] * weight[k];
+        }
+        return weight;
+    }, [&](int db, int qd, const f32x4& v) {
+        if (qi < a.T) store_quad(a.o, ro, db, qd, g, v, 1.0f / lt, dk);
+    });
+    if (qi < a.T && g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = mt * a.scale + logf(lt);
 }
 
 // ---- dQ (and delta, when asked for with it) ----
@@ -218,7 +286,7 @@ constexpr int dq_lds() {  // floats
     constexpr int TILE = 2 * 32 * (D + 4), RED = KW * (D / 32) * 1024;
     return KW * TILE > RED ? KW * TILE : RED;
 }
-template <int D, int KW>
+template <int D, int KW, bool BOTH>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float* lds) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P;
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -226,26 +294,29 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
     int b, h, hk, qblk;
     if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk, id)) return;
     const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
-    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float *const kh = head_of(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of(a.v, a.v_sb, b, a.v_sh, hk), *const qh = head_of(a.q, a.q_sb, b, a.q_sh, h);
+    const float *const gh = head_of(a.d_o, a.do_sb, b, a.do_sh, h), *const oh = head_of(a.o, a.o_sb, b, a.o_sh, h);
+    const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
     float* const Ks = lds + kg * TILE;
     float* const Vs = Ks + 32 * P;
 
     Mover32<D> mk, mv;
-    mk.init(lane, a.k_st, dk);
-    mv.init(lane, a.v_st, dk);
+    mk.init(lane, k_st, dk);
+    mv.init(lane, v_st, dk);
     const KeyTiles kt(a, q0, 32, 32);
-    // one tensor in flight at a time: V of a tile behind its S product, K of the next tile behind the rest
-    if (kg < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(kg) * 32, a.T, dk);
+    if (kg < kt.n) mk.load(kh, k_st, kt.tile(kg) * 32, a.T, dk);
     f32x4 qreg[D / 8], greg[D / 8];
-    load_row32<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
-    load_row32<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
-    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
-    float nlse = 0.0f, dl = 0.0f;
-    if (qi < a.T) nlse = -a.lse[lrow] * LOG2E;
+    load_row32<D>(qh, static_cast<int>(a.q_st), q0, a.T, dk, c32, g, qreg);
+    if (BOTH && kg < kt.n) mv.load(vh, v_st, kt.tile(kg) * 32, a.T, dk);
+    load_row32<D>(gh, static_cast<int>(a.do_st), q0, a.T, dk, c32, g, greg);
+    // everything is asked for before anything is waited for
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(qi, a.T - 1);
+    const float lse = a.lse[lrow];
+    float dl = 0.0f;
     if (fuse_delta) {
         f32x4 oreg[D / 8];
-        load_row32<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, qi, a.T, dk, g, oreg);
+        load_row_of_o<D>(oh, a.o_st, qi, a.T, dk, g, oreg);
         float part = 0.0f;
 #pragma unroll
         for (int j = 0; j < D / 8; ++j)
@@ -253,9 +324,10 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
             for (int i = 0; i < 4; ++i) part = fmaf(oreg[j][i], greg[j][i], part);
         dl = xhalf_sum(part);
         if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
-    } else if (qi < a.T) {
+    } else {
         dl = a.delta[lrow];
     }
+    const float nlse = -lse * LOG2E;
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
     f32x16 acc[DB];
 #pragma unroll
@@ -267,11 +339,14 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
         const int k0 = kt.tile(at) * 32;
         mk.store(Ks, lane);
         tile_barrier<1>();
-        mv.load(a.v, vb, a.v_st, k0, a.T, dk);
+        if (!BOTH) mv.load(vh, v_st, k0, a.T, dk);
         f32x16 s = rows_dot<D>(Ks, [&](int j) { return qreg[j]; }, c32, g);
         mv.store(Vs, lane);
         tile_barrier<1>();
-        if (at + KW < kt.n) mk.load(a.k, kb, a.k_st, kt.tile(at + KW) * 32, a.T, dk);
+        if (at + KW < kt.n) {
+            mk.load(kh, k_st, kt.tile(at + KW) * 32, a.T, dk);
+            if (BOTH) mv.load(vh, v_st, kt.tile(at + KW) * 32, a.T, dk);
+        }
         if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= q0 && k0 >= a.sinks))) {
             const f32x16 dp = rows_dot<D>(Vs, [&](int j) { return greg[j]; }, c32, g);
 #pragma unroll
@@ -283,18 +358,15 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
         tile_barrier<1>();
     }
     __syncthreads();  // every wavefront has read its last tile
-    join_groups<DB, KW>(acc, lds, kg, lane);
-    if (qi < a.T) {
-        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-            if (db % KW == kg) store_block(true, a.dq, ro, db, g, acc[db], a.scale, dk);
-    }
+    const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+    join_quads<DB, KW>(acc, lds, kg, lane, []() -> const float* { return nullptr; }, [&](int db, int qd, const f32x4& v) {
+        if (qi < a.T) store_quad(a.dq, ro, db, qd, g, v, a.scale, dk);
+    });
 }
 template <int D, int KW>
 __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_dq(AttnArgs a, int fuse_delta) {
     __shared__ __attribute__((aligned(16))) float lds[dq_lds<D, KW>()];
-    dq_block<D, KW>(a, fuse_delta, static_cast<int>(blockIdx.x), lds);
+    dq_block<D, KW, false>(a, fuse_delta, static_cast<int>(blockIdx.x), lds);
 }
 
 // ---- dK, dV: a block of 32 keys, the query tiles (of every query head of the group in turn) split ----
@@ -309,16 +381,17 @@ template <int D>
 constexpr bool K_IN_LDS = V_IN_LDS<D> || D == 128;
 template <int D, int KW>
 constexpr int dkdv_lds() {  // floats
-    constexpr int TILE = 2 * 32 * (D + 4) + 64, RED = KW * (D / 32) * 1024;
+    constexpr int TILE = 2 * 32 * (D + 4) + 64, RED = 2 * KW * (D / 32) * 1024;
     return (K_IN_LDS<D> + V_IN_LDS<D>) * 32 * (D + 4) + (KW * TILE > RED ? KW * TILE : RED);
 }
 template <int D, int KW, bool OWN_DELTA>
 __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P + 64;
+    constexpr bool BOTH = D == 32 && OWN_DELTA;
     constexpr bool V_LDS = V_IN_LDS<D>, K_LDS = K_IN_LDS<D>;
     constexpr int KVB = (K_LDS + V_LDS) * 32 * P;
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = quotient(a.Hq, a.Hkv);
     const int nkb = (a.T + 31) / 32;
     const int hs = a.head_split;  // > 1: this workgroup takes heads [h0, h0 + nh) of the group, see gqa_head_split
     // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
@@ -330,7 +403,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
         return;
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h0 = chunk >= 0 ? 0 : quotient(rr * rep, hs), nh = chunk >= 0 ? rep : quotient((rr + 1) * rep, hs) - h0;
     const int k0 = chunk >= 0 ? 0 : blk * 32, kj = k0 + c32;
     const float cexp = a.scale * LOG2E;
     float* const Qs = lds + KVB + kg * TILE;
@@ -346,22 +419,32 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     const int qt_hi = q_end / 32;
     const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh;
 
+    const int q_st = static_cast<int>(a.q_st), g_st = static_cast<int>(a.do_st);
+    const float *const kh = head_of(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of(a.v, a.v_sb, b, a.v_sh, hk);
+    // of the first query head in hand; the others follow at q_sh, ...
+    const float *const q0h = head_of(a.q, a.q_sb, b, a.q_sh, hk * rep + h0), *const g0h = head_of(a.d_o, a.do_sb, b, a.do_sh, hk * rep + h0),
+                *const o0h = head_of(a.o, a.o_sb, b, a.o_sh, hk * rep + h0);
     Mover32<D> mq, mg;
-    mq.init(lane, a.q_st, dk);
-    mg.init(lane, a.do_st, dk);
+    mq.init(lane, q_st, dk);
+    mg.init(lane, g_st, dk);
     float row_r = 0.0f;
-    int f_h = kg / nqt, f_t = kg % nqt;  // head and tile of the next fetch
-    // one tensor in flight at a time: dO of a tile behind its S product, Q of the next tile behind the rest
-    int c_h = 0, c_r0 = 0;  // query head and first row of the step in hand
+    int f_h = 0, f_t = kg;  // head and tile of the next fetch
+    while (f_t >= nqt) f_t -= nqt, ++f_h;
+    int c_h = 0, c_r0 = 0;  // query head (from h0 on) and first row of the step in hand
+    f32x4 oreg[OWN_DELTA ? D / 8 : 1];
+    auto fetch_g = [&]() {
+        mg.load(g0h + c_h * a.do_sh, g_st, c_r0, a.T, dk);
+        if constexpr (OWN_DELTA) load_row_of_o<D>(o0h + c_h * a.o_sh, a.o_st, c_r0 + c32, a.T, dk, g, oreg);
+    };
     auto fetch_q = [&]() {
-        const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * 32;
-        mq.load(a.q, b * a.q_sb + h * a.q_sh, a.q_st, r0, a.T, dk);
-        const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(r0 + c32, a.T - 1);  // rows past the end are masked
+        const int r0 = (qt_lo + f_t) * 32;
+        mq.load(q0h + f_h * a.q_sh, q_st, r0, a.T, dk);
+        const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + hk * rep + h0 + f_h) * a.T + min(r0 + c32, a.T - 1);  // rows past the end are masked
         if (g == 0)
             row_r = a.lse[lrow];
         else if (!OWN_DELTA)
             row_r = a.delta[lrow];
-        c_h = h, c_r0 = r0;
+        c_h = f_h, c_r0 = r0;
         f_t += KW;
         while (f_t >= nqt) f_t -= nqt, ++f_h;
     };
@@ -370,16 +453,16 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     if (K_LDS) {
         for (int c = static_cast<int>(threadIdx.x); c < (K_LDS + V_LDS) * 32 * (D / 4); c += 64 * KW) {
             const int which = c / (32 * (D / 4)), row = c / (D / 4) % 32, col = c % (D / 4) * 4;
-            const float* src = which == 0 ? static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh + (k0 + row) * a.k_st
-                                          : static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh + (k0 + row) * a.v_st;
+            const float* src = which == 0 ? kh + (k0 + row) * a.k_st : vh + (k0 + row) * a.v_st;
             f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
             if (k0 + row < a.T && col < dk) z = *reinterpret_cast<const f32x4*>(src + col);
             *reinterpret_cast<f32x4*>(lds + (which * 32 + row) * P + col) = z;
         }
         __syncthreads();
     }
-    if (!K_LDS) load_row32<D>(a.k, b * a.k_sb + hk * a.k_sh, a.k_st, kj, a.T, dk, g, kreg);
-    if (!V_LDS) load_row32<D>(a.v, b * a.v_sb + hk * a.v_sh, a.v_st, kj, a.T, dk, g, vreg);
+    if (!K_LDS) load_row32<D>(kh, static_cast<int>(a.k_st), k0, a.T, dk, c32, g, kreg);
+    if (!V_LDS) load_row32<D>(vh, static_cast<int>(a.v_st), k0, a.T, dk, c32, g, vreg);
+    if (BOTH && kg < steps) fetch_g();
     // (rows of a tile) . (K or V rows of the block)
     auto dot = [&](const float* tile, bool in_lds, const f32x4* reg, const float* shared) {
         if (in_lds)
@@ -398,9 +481,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
         mq.store(Qs, lane);
         if (!OWN_DELTA || g == 0) rows[lane] = g == 0 ? -row_r * LOG2E : row_r;
         tile_barrier<1>();
-        mg.load(a.d_o, b * a.do_sb + c_h * a.do_sh, a.do_st, qlo, a.T, dk);
-        f32x4 oreg[OWN_DELTA ? D / 8 : 1];
-        if constexpr (OWN_DELTA) load_row32<D>(a.o, b * a.o_sb + c_h * a.o_sh, a.o_st, qlo + c32, a.T, dk, g, oreg);
+        if (!BOTH) fetch_g();
         f32x16 s = dot(Qs, K_LDS, kreg, lds);
         mg.store(Gs, lane);
         tile_barrier<1>();
@@ -416,7 +497,10 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
             if (g == 1) rows[lane] = part;
             tile_barrier<1>();
         }
-        if (step + KW < steps) fetch_q();
+        if (step + KW < steps) {
+            fetch_q();
+            if (BOTH) fetch_g();
+        }
         if (!((a.causal && k0 > qhi) || (a.window > 0 && k0 + 31 + a.window <= qlo && k0 >= a.sinks))) {
             // lane = key kj; element r = query qlo + crow(r, g)
 #pragma unroll
@@ -444,30 +528,22 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
         tile_barrier<1>();
     }
     __syncthreads();  // every wavefront has read its last tile
-    join_groups<DB, KW>(acc, lds + KVB, kg, lane);
-    __syncthreads();
-    join_groups<DB, KW>(acc + DB, lds + KVB, kg, lane);
     // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
     // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
     const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1);
-    if (kj < a.T && (chunk < 0 || to_tail)) {
-        const bool parts = hs > 1 && !to_tail;
-        const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
-                                   : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
-        const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
-        const bool scratch = parts || to_tail;
-        void* const room = to_tail ? a.tail : a.part;
-        const int64_t rv = scratch ? pv : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
-        const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
-        void* const dst_v = scratch ? room : a.dv;
-        void* const dst_k = scratch ? room : a.dk;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            if (db % KW != kg) continue;
-            store_block(true, dst_v, rv, db, g, acc[db], 1.0f, dk);
-            store_block(true, dst_k, rk, db, g, acc[DB + db], a.scale, dk);
-        }
-    }
+    const bool parts = hs > 1 && !to_tail;
+    const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
+                               : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+    const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
+    const bool scratch = parts || to_tail, mine = kj < a.T && (chunk < 0 || to_tail);
+    void* const room = to_tail ? a.tail : a.part;
+    const int64_t rv = scratch ? pv : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
+    const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+    void* const dst_v = scratch ? room : a.dv;
+    void* const dst_k = scratch ? room : a.dk;
+    join_quads<2 * DB, KW>(acc, lds + KVB, kg, lane, []() -> const float* { return nullptr; }, [&](int n, int qd, const f32x4& v) {
+        if (mine) store_quad(n < DB ? dst_v : dst_k, n < DB ? rv : rk, n < DB ? n : n - DB, qd, g, v, n < DB ? 1.0f : a.scale, dk);
+    });
 }
 template <int D, int KW>
 __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) void f32_split_dkdv(AttnArgs a) {
@@ -486,7 +562,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_split_bwd(AttnArgs a
     if (id < dkdv_ids)
         dkdv_block<D, 4, true>(a, id, lds);
     else
-        dq_block<D, 4>(a, 1, id - dkdv_ids, lds);
+        dq_block<D, 4, D == 32>(a, 1, id - dkdv_ids, lds);
 }
 
 // A block's tiles split between four or eight wavefronts, or not this kernel.

@@ -679,14 +679,14 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int role = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) & (G - 1);
-    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = quotient(a.Hq, a.Hkv);
     const int nkb = (a.T + BNK - 1) / BNK;
     const int hs = a.head_split;  // > 1: this workgroup takes heads [h0, h0 + nh) of the group, see gqa_head_split
     // the sink keys' queries past their block's band go to workgroups of their own, blocks nkb .. nkb + nch - 1
     const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h0 = chunk >= 0 ? 0 : quotient(rr * rep, hs), nh = chunk >= 0 ? rep : quotient((rr + 1) * rep, hs) - h0;
     const int k0 = chunk >= 0 ? 0 : blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
     const float cexp = a.scale * LOG2E;
 
@@ -840,8 +840,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
     int rank, r, kvu;
     if (!jb.map(a, rank, r, kvu)) return;
     if (r < a.head_split) return dkdv_block<D, 2>(a, rank, r, kvu, lds, reinterpret_cast<float*>(lds + K));
-    const int hk = kvu % a.Hkv;
-    dq_block<D, 2, 2>(a, 0, kvu / a.Hkv, hk * (a.Hq / a.Hkv) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
+    dq_block<D, 2, 2>(a, 0, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // ---- dQ above 64 columns: the same two phases ----

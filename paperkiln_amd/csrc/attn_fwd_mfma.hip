@@ -111,10 +111,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void mfma_fwd(AttnArgs a) {
     // the wavefront index as a scalar: every test on it becomes a scalar branch
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, c32 = lane & 31;
-    const int nqb = (a.T + BM - 1) / BM, rep = a.Hq / a.Hkv;
+    const int nqb = (a.T + BM - 1) / BM, rep = quotient(a.Hq, a.Hkv);
     int blk, rr, kvu;
     if (!map_causal_blocks(a, nqb, rep, blk, rr, kvu)) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h = hk * rep + rr;
     const int npass = (a.paired && blk != nqb - 1 - blk) ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
     const int qblk = pass == 0 ? nqb - 1 - blk : blk;

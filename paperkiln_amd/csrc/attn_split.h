@@ -99,7 +99,7 @@ inline bool even_chains(const AttnArgs& a) { return !a.causal || chain_tokens(a)
 inline bool split_tail_pays(const AttnArgs& a, int head_split, int block_rows) {
     const SinkTail t = sink_tail(a.T, a.window, a.sinks);
     const int64_t blocks = static_cast<int64_t>((a.T + block_rows - 1) / block_rows) * a.Hkv * a.B * head_split;
-    const int64_t left = a.T - t.q0, rep = a.Hq / a.Hkv, share = (rep + head_split - 1) / head_split;
+    const int64_t left = a.T - t.q0, rep = quotient(a.Hq, a.Hkv), share = (rep + head_split - 1) / head_split;
     return a.tail && t.nch > 0 && left > (blocks + 511) / 512 * (a.window + 128) &&
            (share == rep || share * left > rep * (left < TAIL_CHUNK ? left : TAIL_CHUNK));
 }
@@ -126,7 +126,7 @@ struct OneLaunch {
 // first. A rank of a (batch, KV head) unit is a block of keys for each share of the group's heads, then one of queries for each head.
 struct JoinedBlocks {
     int ranks, each;
-    __host__ __device__ JoinedBlocks(const AttnArgs& a, int rows) : ranks((a.T + rows - 1) / rows), each(a.head_split + a.Hq / a.Hkv) {}
+    __host__ __device__ JoinedBlocks(const AttnArgs& a, int rows) : ranks((a.T + rows - 1) / rows), each(a.head_split + quotient(a.Hq, a.Hkv)) {}
     __host__ int grid(const AttnArgs& a) const { return xcd_grid(ranks, each, a.Hkv * a.B); }
     // r: the share of the heads whose dK, dV (r < a.head_split), or the head (the others) whose dQ this workgroup forms
     __device__ bool map(const AttnArgs& a, int& rank, int& r, int& kvu) const {
@@ -178,13 +178,13 @@ struct QueryRange {
 };
 
 __device__ inline bool map_query_block(const AttnArgs& a, int nqb, int& b, int& h, int& hk, int& qblk, int id = static_cast<int>(blockIdx.x)) {
-    const int rep = a.Hq / a.Hkv;
+    const int rep = quotient(a.Hq, a.Hkv);
     int blk, rr, kvu;
     // causal blocks without a band: the heaviest blocks of every unit first
     if (a.causal && a.window == 0 ? !xcd_map_block_major(nqb, rep, a.Hkv * a.B, blk, rr, kvu, id)
                                   : !xcd_map(nqb, rep, a.Hkv * a.B, blk, rr, kvu, id))
         return false;
-    hk = kvu % a.Hkv, b = kvu / a.Hkv, h = hk * rep + rr;
+    b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h = hk * rep + rr;
     qblk = nqb - 1 - blk;
     return true;
 }

@@ -467,7 +467,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
-    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = a.Hq / a.Hkv;
+    const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim, rep = quotient(a.Hq, a.Hkv);
     const int nkb = (a.T + BNK - 1) / BNK;
     // hs > 1: the query heads of the group are dealt to hs workgroups (gqa_head_split); this one takes heads
     // [h0, h0 + nh) of the group and leaves fp32 partial sums for launch_gqa_reduce
@@ -476,7 +476,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     const SinkTail tl = a.tail ? sink_tail(a.T, a.window, a.sinks) : SinkTail{0, 0};
     const int chunk = blk - nkb;  // >= 0: a piece of the tail, for all query heads of the group
     if (chunk >= 0 && rr > 0) return;
-    const int hk = kvu % a.Hkv, b = kvu / a.Hkv, h0 = chunk >= 0 ? 0 : rr * rep / hs, nh = chunk >= 0 ? rep : (rr + 1) * rep / hs - h0;
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h0 = chunk >= 0 ? 0 : quotient(rr * rep, hs), nh = chunk >= 0 ? rep : quotient((rr + 1) * rep, hs) - h0;
     const int k0 = chunk >= 0 ? 0 : blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
     const float cexp = a.scale * LOG2E;
 
@@ -670,8 +670,8 @@ __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     int rank, r, kvu;
     if (!jb.map(a, rank, r, kvu)) return;
     if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA>(a, rank, r, kvu, lds);
-    const int hk = kvu % a.Hkv;
-    dq_block<D, 4, 1, 2, EXACT>(a, OWN_DELTA, kvu / a.Hkv, hk * (a.Hq / a.Hkv) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
+    dq_block<D, 4, 1, 2, EXACT>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of

@@ -267,6 +267,9 @@ __device__ inline void gated_grad(float g, float u, float d, float& dg, float& d
     dg = (d * u) * (s * (1.0f + g * (1.0f - s)));
 }
 
+// n / d where neither is negative: a division of signed numbers is a third longer, and a workgroup divides three to five times before its first load
+__host__ __device__ inline int quotient(int n, int d) { return static_cast<int>(static_cast<unsigned>(n) / static_cast<unsigned>(d)); }
+
 // XCD-aware workgroup -> tile mapping. The 256 CUs sit in 8 XCDs, each with
 // its own 4 MB L2, and consecutive workgroup ids go round-robin over the XCDs.
 // Every block of a (batch, KV head) unit re-reads that unit's K/V (or Q/dO),
@@ -288,9 +291,10 @@ __host__ __device__ inline int xcd_grid(int nblk, int rep, int kv_units) {
 // The idx-th of the left-over units' blocks, block 0 of every unit and head first; false past their end.
 __device__ inline bool xcd_loose_block(int idx, int nblk, int rep, int kv_units, int& blk, int& r, int& kvu) {
     const int heads = (kv_units & 7) * rep;
-    blk = idx / heads;
-    r = (idx % heads) % rep;
-    kvu = (kv_units & ~7) + (idx % heads) / rep;
+    blk = quotient(idx, heads);
+    const int at = idx - blk * heads, unit = quotient(at, rep);
+    r = at - unit * rep;
+    kvu = (kv_units & ~7) + unit;
     return blk < nblk;
 }
 // blk: block index inside the unit (0 = dispatched first); r: query head inside
@@ -300,9 +304,10 @@ __device__ inline bool xcd_loose_block(int idx, int nblk, int rep, int kv_units,
 __device__ inline bool xcd_map(int nblk, int rep, int kv_units, int& blk, int& r, int& kvu, int id = static_cast<int>(blockIdx.x)) {
     const int xcd = id & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = (id >> 3) - loose;
     if (j < 0) return xcd_loose_block((j + loose) * 8 + xcd, nblk, rep, kv_units, blk, r, kvu);
-    blk = j % nblk;
-    r = (j / nblk) % rep;
-    kvu = (j / (nblk * rep)) * 8 + xcd;
+    const int head = quotient(j, nblk), unit = quotient(head, rep);
+    blk = j - head * nblk;
+    r = head - unit * rep;
+    kvu = unit * 8 + xcd;
     return true;
 }
 // The same ids in block-major order: block 0 of every unit and head of an XCD's share first, then every block 1, ...
@@ -314,9 +319,10 @@ __device__ inline bool xcd_map_block_major(int nblk, int rep, int kv_units, int&
     const int xcd = id & 7, loose = xcd_loose_ids(nblk, rep, kv_units), j = (id >> 3) - loose;
     if (j < 0) return xcd_loose_block((j + loose) * 8 + xcd, nblk, rep, kv_units, blk, r, kvu);
     const int per = (kv_units / 8) * rep;  // (unit, head) pairs of one XCD
-    blk = j / per;
-    r = (j % per) % rep;
-    kvu = ((j % per) / rep) * 8 + xcd;
+    blk = quotient(j, per);
+    const int at = j - blk * per, unit = quotient(at, rep);
+    r = at - unit * rep;
+    kvu = unit * 8 + xcd;
     return true;
 }
 
@@ -340,8 +346,9 @@ __device__ inline bool xcd_map_block0_first(int nblk, int kv_units, int& blk, in
         --j;
         if (j >= upx && j < upx + loose) {
             const int idx = (j - upx) * 8 + xcd;
-            blk = 1 + idx / left;
-            kvu = (kv_units & ~7) + idx % left;
+            const int at = quotient(idx, left);
+            blk = 1 + at;
+            kvu = (kv_units & ~7) + idx - at * left;
             return idx < left * (nblk - 1);
         }
         if (j >= upx) j -= loose;
@@ -351,8 +358,9 @@ __device__ inline bool xcd_map_block0_first(int nblk, int kv_units, int& blk, in
         kvu = j * 8 + xcd;
     } else {
         j -= upx;
-        blk = 1 + j % (nblk - 1);
-        kvu = (j / (nblk - 1)) * 8 + xcd;
+        const int unit = quotient(j, nblk - 1);
+        blk = 1 + j - unit * (nblk - 1);
+        kvu = unit * 8 + xcd;
     }
     return true;
 }
