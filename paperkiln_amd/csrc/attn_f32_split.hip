@@ -20,13 +20,6 @@ constexpr float LOG2E = 1.4426950408889634f;
 __device__ inline f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 __device__ inline int crow(int r, int g) { return (r >> 2) * 8 + 4 * g + (r & 3); }
 
-// A head's first element. The value is formed here and kept: left to itself the compiler reads the arguments again, a round trip through the
-// scalar cache each, wherever the next tensor is addressed -- seven times before the first product.
-__device__ inline const float* head_of(const void* base, int64_t sb, int b, int64_t sh, int h) {
-    const float* p = static_cast<const float*>(base) + (b * sb + h * sh);
-    asm volatile("" : "+s"(p));
-    return p;
-}
 // rows r0 .. T - 1 of a head; r0 < T. Whatever lies past them reads as zero.
 __device__ inline __amdgpu_buffer_rsrc_t rows_from(const float* head, int st, int r0, int T, int dk) {
     const int64_t left = (static_cast<int64_t>(T - r0 - 1) * st + dk) * 4;
@@ -138,35 +131,6 @@ __device__ inline void accumulate_tr32(const float* tile, const f32x16& c, f32x1
     }
 }
 
-// The KW wavefronts' accumulators of N blocks added up, in wavefront order: the 4 N quads of eight columns are dealt out, one to each wavefront
-// in turn, so that all of them add and store (block by block, three of four wavefronts watch one at 32 columns). `red`: 1024 N KW floats of LDS,
-// free to overwrite. `out` takes (block, quad, sum). weights(), asked for behind the barrier: what wavefront k's part is multiplied by, or nullptr.
-template <int N, int KW, typename W, typename F>
-__device__ inline void join_quads(const f32x16* acc, float* red, int kg, int lane, W weights, F out) {
-    constexpr int ITEMS = 4 * N;
-#pragma unroll
-    for (int n = 0; n < N; ++n)
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-            const f32x4 v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
-            *(reinterpret_cast<f32x4*>(red) + (kg * ITEMS + n * 4 + qd) * 64 + lane) = v;
-        }
-    __syncthreads();
-    const float* const weight = weights();
-#pragma unroll
-    for (int i = 0; i < (ITEMS + KW - 1) / KW; ++i) {
-        const int item = i * KW + kg;
-        if (ITEMS % KW != 0 && item >= ITEMS) break;
-        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-            const f32x4 v = *(reinterpret_cast<const f32x4*>(red) + (k * ITEMS + item) * 64 + lane);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) s[e] = weight ? fmaf(v[e], weight[k], s[e]) : s[e] + v[e];
-        }
-        out(item / 4, item % 4, s);
-    }
-}
 // a quad of a lane's output row
 __device__ inline void store_quad(void* base, int64_t row_off, int db, int qd, int g, const f32x4& v, float sc, int dk) {
     const int col = 32 * db + 8 * qd + 4 * g;
@@ -195,7 +159,7 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
     int b, h, hk, qblk;
     if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk)) return;
     const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
-    const float *const kh = head_of(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of(a.v, a.v_sb, b, a.v_sh, hk), *const qh = head_of(a.q, a.q_sb, b, a.q_sh, h);
+    const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk), *const qh = head_of<float>(a.q, a.q_sb, b, a.q_sh, h);
     const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
     float* const Ks = lds + kg * TILE;
@@ -265,7 +229,7 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
     ml[kg * 128 + 64 + lane] = l;
     const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
     float mt = m, lt = 0.0f, weight[KW];
-    join_quads<DB, KW>(acc, lds, kg, lane, [&]() {
+    join_shares<DB, KW, 1>(acc, lds, kg, lane, [&]() {
 #pragma unroll
         for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
 #pragma unroll
@@ -274,8 +238,8 @@ __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_sp
             lt += ml[k * 128 + 64 + lane] * weight[k];
         }
         return weight;
-    }, [&](int db, int qd, const f32x4& v) {
-        if (qi < a.T) store_quad(a.o, ro, db, qd, g, v, 1.0f / lt, dk);
+    }, [&](int db, int qd, const f32x4 (&v)[1]) {
+        if (qi < a.T) store_quad(a.o, ro, db, qd, g, v[0], 1.0f / lt, dk);
     });
     if (qi < a.T && g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = mt * a.scale + logf(lt);
 }
@@ -294,8 +258,8 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
     int b, h, hk, qblk;
     if (!map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk, id)) return;
     const int q0 = qblk * 32, qhi = q0 + 31, qi = q0 + c32;
-    const float *const kh = head_of(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of(a.v, a.v_sb, b, a.v_sh, hk), *const qh = head_of(a.q, a.q_sb, b, a.q_sh, h);
-    const float *const gh = head_of(a.d_o, a.do_sb, b, a.do_sh, h), *const oh = head_of(a.o, a.o_sb, b, a.o_sh, h);
+    const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk), *const qh = head_of<float>(a.q, a.q_sb, b, a.q_sh, h);
+    const float *const gh = head_of<float>(a.d_o, a.do_sb, b, a.do_sh, h), *const oh = head_of<float>(a.o, a.o_sb, b, a.o_sh, h);
     const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
     float* const Ks = lds + kg * TILE;
@@ -359,8 +323,8 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
     }
     __syncthreads();  // every wavefront has read its last tile
     const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
-    join_quads<DB, KW>(acc, lds, kg, lane, []() -> const float* { return nullptr; }, [&](int db, int qd, const f32x4& v) {
-        if (qi < a.T) store_quad(a.dq, ro, db, qd, g, v, a.scale, dk);
+    join_shares<DB, KW, 1>(acc, lds, kg, lane, no_weights, [&](int db, int qd, const f32x4 (&v)[1]) {
+        if (qi < a.T) store_quad(a.dq, ro, db, qd, g, v[0], a.scale, dk);
     });
 }
 template <int D, int KW>
@@ -420,10 +384,10 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh;
 
     const int q_st = static_cast<int>(a.q_st), g_st = static_cast<int>(a.do_st);
-    const float *const kh = head_of(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of(a.v, a.v_sb, b, a.v_sh, hk);
+    const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk);
     // of the first query head in hand; the others follow at q_sh, ...
-    const float *const q0h = head_of(a.q, a.q_sb, b, a.q_sh, hk * rep + h0), *const g0h = head_of(a.d_o, a.do_sb, b, a.do_sh, hk * rep + h0),
-                *const o0h = head_of(a.o, a.o_sb, b, a.o_sh, hk * rep + h0);
+    const float *const q0h = head_of<float>(a.q, a.q_sb, b, a.q_sh, hk * rep + h0), *const g0h = head_of<float>(a.d_o, a.do_sb, b, a.do_sh, hk * rep + h0),
+                *const o0h = head_of<float>(a.o, a.o_sb, b, a.o_sh, hk * rep + h0);
     Mover32<D> mq, mg;
     mq.init(lane, q_st, dk);
     mg.init(lane, g_st, dk);
@@ -541,8 +505,8 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
     void* const dst_v = scratch ? room : a.dv;
     void* const dst_k = scratch ? room : a.dk;
-    join_quads<2 * DB, KW>(acc, lds + KVB, kg, lane, []() -> const float* { return nullptr; }, [&](int n, int qd, const f32x4& v) {
-        if (mine) store_quad(n < DB ? dst_v : dst_k, n < DB ? rv : rk, n < DB ? n : n - DB, qd, g, v, n < DB ? 1.0f : a.scale, dk);
+    join_shares<2 * DB, KW, 1>(acc, lds + KVB, kg, lane, no_weights, [&](int n, int qd, const f32x4 (&v)[1]) {
+        if (mine) store_quad(n < DB ? dst_v : dst_k, n < DB ? rv : rk, n < DB ? n : n - DB, qd, g, v[0], n < DB ? 1.0f : a.scale, dk);
     });
 }
 template <int D, int KW>

@@ -47,6 +47,54 @@ __device__ inline void join_groups(f32x16* acc, float* red, int kg, int lane) {
     }
 }
 
+// The same where all wavefronts add and store: every block is four quads of eight columns (four to a lane), the shares of Q quads are dealt out
+// to the KW wavefronts in turn (block by block, three of four watch one at 32 columns). `red`: 1024 N KW floats of LDS, free to overwrite. out takes
+// (block, first quad, sums); weights(), asked for behind the barrier: what wavefront k's part is multiplied by, or nullptr.
+template <int N, int KW, int Q, typename W, typename F>
+__device__ inline void join_shares(const f32x16* acc, float* red, int kg, int lane, W weights, F out) {
+    constexpr int QUADS = 4 * N, ITEMS = QUADS / Q;
+    f32x4* const all = reinterpret_cast<f32x4*>(red) + lane;
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+            const f32x4 v = {acc[n][qd * 4], acc[n][qd * 4 + 1], acc[n][qd * 4 + 2], acc[n][qd * 4 + 3]};
+            all[(kg * QUADS + n * 4 + qd) * 64] = v;
+        }
+    __syncthreads();
+    const float* const weight = weights();
+#pragma unroll
+    for (int i = 0; i < (ITEMS + KW - 1) / KW; ++i) {
+        const int item = i * KW + kg;
+        if (ITEMS % KW != 0 && item >= ITEMS) break;
+        f32x4 s[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            s[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int k = 0; k < KW; ++k) {
+                const f32x4 v = all[(k * QUADS + item * Q + q) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[q][e] = weight ? fmaf(v[e], weight[k], s[q][e]) : s[q][e] + v[e];
+            }
+        }
+        out(item * Q / 4, item * Q % 4, s);
+    }
+}
+__device__ inline const float* no_weights() { return nullptr; }
+
+// A head's first element. The value is formed here and kept: left to itself the compiler reads the arguments again, a round trip through the
+// scalar cache each, wherever the next tensor is addressed -- seven times before the first product.
+// With it, LSE asked for with the rest and all wavefronts in the join, bf16 launches of short chains, us: T 128, 4 heads of 64 forward 5.4 -> 4.8,
+// backward 8.0 -> 7.7; T 200, 4 heads of 128 8.5 -> 7.0, 15.6 -> 14.9; T 90 x 2, 4 heads of 32 backward 7.8 -> 6.5; T 1000 x 2, 8 heads of 80
+// 48.6 -> 46.2; 96 columns, T 400, 4 heads 8.7 -> 7.8, 19.4 -> 16.6. Long chains level, backward at 64 columns 1 to 2 % ahead.
+template <typename T>
+__device__ inline const T* head_of(const void* base, int64_t sb, int b, int64_t sh, int h) {
+    const T* p = static_cast<const T*>(base) + (b * sb + h * sh);
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // One 32 x 32 accumulator block (lane = row of the output, natural column order) scaled and written; columns past dk are
 // not. Both lanes of a pair (c, c + 32) hold the same row and must be active.
 __device__ inline void store_block(bool f32, void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
@@ -71,6 +119,25 @@ __device__ inline void store_block(bool f32, void* base, int64_t row_off, int db
             const int col = 32 * db + 8 * (2 * qp + g);
             if (col < dk) *reinterpret_cast<u32x4*>(row + col) = v;
         }
+    }
+}
+
+// Quads qd and qd + 1 (even, odd) of such a block
+__device__ inline void store_half(bool f32, void* base, int64_t row_off, int db, int qd, int g, const f32x4 (&v)[2], float sc, int dk) {
+    if (f32) {
+        float* row = static_cast<float*>(base) + row_off;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int col = 32 * db + 8 * (qd + q) + 4 * g;
+            const f32x4 o = {v[q][0] * sc, v[q][1] * sc, v[q][2] * sc, v[q][3] * sc};
+            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = o;
+        }
+    } else {
+        const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(v[0][0] * sc, v[0][1] * sc), pack_bf16(v[1][0] * sc, v[1][1] * sc), false, false);
+        const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(v[0][2] * sc, v[0][3] * sc), pack_bf16(v[1][2] * sc, v[1][3] * sc), false, false);
+        const u32x4 o = {r0[0], r1[0], r0[1], r1[1]};
+        const int col = 32 * db + 8 * (qd + g);
+        if (col < dk) *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(base) + row_off + col) = o;
     }
 }
 

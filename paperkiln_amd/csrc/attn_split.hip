@@ -49,15 +49,15 @@ struct Mover {
     static_assert(CPT >= 1 && ROWS * NCH % G == 0, "every thread moves the same number of chunks");
     int off[CPT];  // byte offsets inside a tile
     u32x4 r[CPT];
-    __device__ void init(int t, int64_t st, int dk) {
+    __device__ void init(int t, int st, int dk) {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int c = t + G * i, row = c / NCH, ch = c % NCH;
-            off[i] = ch * 8 < dk ? static_cast<int>(row * st + ch * 8) * 2 : static_cast<int>(OUTSIDE);
+            off[i] = ch * 8 < dk ? (row * st + ch * 8) * 2 : static_cast<int>(OUTSIDE);
         }
     }
-    __device__ void load(const void* base, int64_t elem_off, int64_t st, int r0, int T, int dk) {
-        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(base, elem_off, st, r0, T, dk);
+    __device__ void load(const uint16_t* head, int st, int r0, int T, int dk) {
+        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(head, 0, st, r0, T, dk);
 #pragma unroll
         for (int i = 0; i < CPT; ++i) r[i] = tile_load16(rs, off[i]);
     }
@@ -72,16 +72,28 @@ struct Mover {
     }
 };
 
-// Row `row` of a head as an operand held in registers: chunk kk covers d = 16kk + 8g .. +7; zero past T and past dk.
-template <int D>
-__device__ inline void load_row(const void* base, int64_t off, int64_t st, int row, int T, int dk, int g, bf16x8* out) {
+// Row r0 + c32 of a head as an operand held in registers: chunk kk covers d = 16kk + 8g .. +7; zero past T and past dk. BRANCH: under a
+// condition instead of through a buffer, which keeps the loads where they are written. In the long loops of P and dS in several parts the scheduler
+// needs that (forward, us, buffer | branch: 96 columns, T 1500 x 4, 8 heads 44.0 | 41.6; 48, T 4000 x 2, window 500 27.2 | 26.1; backward 79.7 | 77.1, but
+// 96 columns 111.5 | 113.8; 80, no mask, T 2000 x 4 286 | 291); at 64 columns the buffer is ahead (T 4096 x 2, 8 heads 154 | 156), and where chains are short.
+template <int D, bool BRANCH>
+__device__ inline void load_row(const uint16_t* head, int st, int r0, int T, int dk, int c32, int g, bf16x8* out) {
+    if constexpr (BRANCH) {
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) {
+            u32x4 z = {0, 0, 0, 0};
+            const int col = kk * 16 + g * 8;
+            if (r0 + c32 < T && col < dk) z = *reinterpret_cast<const u32x4*>(head + static_cast<int64_t>(r0 + c32) * st + col);
+            out[kk] = *reinterpret_cast<bf16x8*>(&z);
+        }
+        return;
+    }
+    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(head, 0, st, r0, T, dk);
+    const int row = (c32 * st + g * 8) * 2;
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) {
-        u32x4 z = {0, 0, 0, 0};
-        const int col = kk * 16 + g * 8;
-        if (row < T && col < dk)
-            z = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + off + row * st + col);
-        out[kk] = *reinterpret_cast<bf16x8*>(&z);
+        const u32x4 v = tile_load16(rs, kk * 16 + g * 8 < dk ? row + 32 * kk : static_cast<int>(OUTSIDE));
+        out[kk] = *reinterpret_cast<const bf16x8*>(&v);
     }
 }
 
@@ -188,20 +200,22 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     int b, h, hk, qblk;
     if (!map_query_block(a, nqb, b, h, hk, qblk)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
-    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const uint16_t *const kh = head_of<uint16_t>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<uint16_t>(a.v, a.v_sb, b, a.v_sh, hk),
+                   *const qh = head_of<uint16_t>(a.q, a.q_sb, b, a.q_sh, h);
+    const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
 
     Mover<D, G, BN> mk, mv;
-    mk.init(gt, a.k_st, dk);
-    mv.init(gt, a.v_st, dk);
+    mk.init(gt, k_st, dk);
+    mv.init(gt, v_st, dk);
     const KeyTiles kt(a, q0, BM, BN);
     const int iters = (kt.n + KW - 1) / KW;
     auto fetch = [&](int i) {  // this group's i-th tile (past its last: nothing)
         const int at = i * KW + kg;
         if (at < kt.n) {
             const int r0 = kt.tile(at) * BN;
-            mk.load(a.k, kb, a.k_st, r0, a.T, dk);
-            mv.load(a.v, vb, a.v_st, r0, a.T, dk);
+            mk.load(kh, k_st, r0, a.T, dk);
+            mv.load(vh, v_st, r0, a.T, dk);
         }
     };
     auto commit = [&](int buf) {
@@ -211,7 +225,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     };
     fetch(0);
     bf16x8 qreg[KK];
-    load_row<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    load_row<D, EXACT && (QW > 1)>(qh, static_cast<int>(a.q_st), qlo, a.T, dk, c32, g, qreg);
     f32x16 acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -298,33 +312,34 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     }
 
     l = xhalf_sum(l);
-    if (KW > 1) {
+    const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+    if constexpr (KW > 1) {
         if (QW == 1) __syncthreads();  // every group has read its last tile
-        // the groups' running maxima and sums meet, then their accumulators scaled to the common maximum
+        // the groups' running maxima and sums meet with their accumulators, each scaled to the common maximum
         float* red = reinterpret_cast<float*>(lds) + qg * KW * (DB * 1024 + 128);
         float* ml = red + KW * DB * 1024;
         ml[kg * 128 + lane] = m;
         ml[kg * 128 + 64 + lane] = l;
-        __syncthreads();
-        float mt = m, lt = 0.0f;
+        float mt = m, lt = 0.0f, weight[KW];
+        join_shares<DB, KW, 2>(acc, red, kg, lane, [&]() {
 #pragma unroll
-        for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
+            for (int k = 0; k < KW; ++k) mt = fmaxf(mt, ml[k * 128 + lane]);
 #pragma unroll
-        for (int k = 0; k < KW; ++k) lt += ml[k * 128 + 64 + lane] * __builtin_amdgcn_exp2f((ml[k * 128 + lane] - mt) * cexp);
-        const float alpha = __builtin_amdgcn_exp2f((m - mt) * cexp);
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
-        join_groups<DB, KW>(acc, red, kg, lane);
+            for (int k = 0; k < KW; ++k) {
+                weight[k] = __builtin_amdgcn_exp2f((ml[k * 128 + lane] - mt) * cexp);
+                lt += ml[k * 128 + 64 + lane] * weight[k];
+            }
+            return weight;
+        }, [&](int db, int qd, const f32x4 (&v)[2]) {
+            if (qi < a.T) store_half(false, a.o, ro, db, qd, g, v, 1.0f / lt, dk);
+        });
         m = mt, l = lt;
     }
     if (qi < a.T) {
         const float inv = 1.0f / l;
-        const int64_t ro = b * a.o_sb + h * a.o_sh + qi * a.o_st;
+        if (KW == 1)
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-            if (KW == 1 || db % KW == kg) store_block(false, a.o, ro, db, g, acc[db], inv, dk);
+            for (int db = 0; db < DB; ++db) store_block(false, a.o, ro, db, g, acc[db], inv, dk);
         if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = m * a.scale + logf(l);
     }
 }
@@ -345,20 +360,22 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
-    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const uint16_t *const kh = head_of<uint16_t>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<uint16_t>(a.v, a.v_sb, b, a.v_sh, hk),
+                   *const qh = head_of<uint16_t>(a.q, a.q_sb, b, a.q_sh, h);
+    const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
 
     Mover<D, G, BN> mk, mv;
-    mk.init(gt, a.k_st, dk);
-    mv.init(gt, a.v_st, dk);
+    mk.init(gt, k_st, dk);
+    mv.init(gt, v_st, dk);
     const KeyTiles kt(a, q0, BM, BN);
     const int iters = (kt.n + KW - 1) / KW;
     auto fetch = [&](int i) {
         const int at = i * KW + kg;
         if (at < kt.n) {
             const int r0 = kt.tile(at) * BN;
-            mk.load(a.k, kb, a.k_st, r0, a.T, dk);
-            mv.load(a.v, vb, a.v_st, r0, a.T, dk);
+            mk.load(kh, k_st, r0, a.T, dk);
+            mv.load(vh, v_st, r0, a.T, dk);
         }
     };
     auto commit = [&](int buf) {
@@ -368,22 +385,24 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     };
     fetch(0);
     bf16x8 qreg[KK], greg[KK];
-    load_row<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
-    load_row<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
-    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
-    float nlse = 0.0f, dl = 0.0f;
-    if (qi < a.T) nlse = EXACT ? -a.lse[lrow] : -a.lse[lrow] * LOG2E;
+    load_row<D, EXACT && (QW > 1) && D <= 64>(qh, static_cast<int>(a.q_st), qlo, a.T, dk, c32, g, qreg);
+    load_row<D, EXACT && (QW > 1) && D <= 64>(head_of<uint16_t>(a.d_o, a.do_sb, b, a.do_sh, h), static_cast<int>(a.do_st), qlo, a.T, dk, c32, g, greg);
+    // everything is asked for before anything is waited for
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(qi, a.T - 1);
+    const float lse = a.lse[lrow];
+    float dl = 0.0f;
     if (fuse_delta) {
         bf16x8 oreg[KK];
-        load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, qi, a.T, dk, g, oreg);
+        load_row<D, EXACT && (QW > 1) && D <= 64>(head_of<uint16_t>(a.o, a.o_sb, b, a.o_sh, h), static_cast<int>(a.o_st), qlo, a.T, dk, c32, g, oreg);
         float part = 0.0f;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) part = add_products(oreg[kk], greg[kk], part);
         dl = xhalf_sum(part);
         if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
-    } else if (qi < a.T) {
+    } else {
         dl = a.delta[lrow];
     }
+    const float nlse = EXACT ? -lse : -lse * LOG2E;
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
     const KeyRange range(a, qlo);
     f32x16 acc[DB];
@@ -421,13 +440,14 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
         tile_barrier<QW>();
     }
     if (KW > 1 && QW == 1) __syncthreads();  // every group has read its last tile
-    join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane);
-    if (qi < a.T) {
-        const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+    const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
+    if constexpr (KW > 1)
+        join_shares<DB, KW, 2>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane, no_weights, [&](int db, int qd, const f32x4 (&v)[2]) {
+            if (qi < a.T) store_half(a.grad_f32 != 0, a.dq, ro, db, qd, g, v, a.scale, dk);
+        });
+    else if (qi < a.T)
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-            if (KW == 1 || db % KW == kg) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk);
-    }
+        for (int db = 0; db < DB; ++db) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk);
 }
 template <int D, int QW, int KW, int NB, bool EXACT>
 __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
@@ -451,9 +471,13 @@ __device__ inline bool map_key_block(const AttnArgs& a, int rows, int& blk, int&
 //
 // OWN_DELTA: the rows' delta is formed here, from O and the tile of dO; otherwise it is read. Of one wavefront to a group and tiles of 32 in the
 // order of dq_block and to the same bits; else a thread's chunks of both, then the lanes that hold a row.
+//
+// dV and dK are joined together up to 64 columns; above, the LDS for both would keep a second workgroup off the CU.
+template <int D>
+constexpr bool JOIN_BOTH = D <= 64;
 template <int D, int QW, int KW, int NB>
 constexpr int dkdv_lds() {  // in uint16; LSE and delta of a tile's rows behind it
-    constexpr int TILES = (QW > 1 ? 2 : 1) * KW * (2 * 32 * NB * (D + 8) + 128 * NB), RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
+    constexpr int TILES = (QW > 1 ? 2 : 1) * KW * (2 * 32 * NB * (D + 8) + 128 * NB), RED = KW > 1 ? QW * KW * (D / 32) * (JOIN_BOTH<D> ? 4096 : 2048) : 0;
     return TILES > RED ? TILES : RED;
 }
 template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA>
@@ -489,30 +513,37 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     const int qt_hi = q_end / BMQ;
     const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh, iters = (steps + KW - 1) / KW;
 
+    const int q_st = static_cast<int>(a.q_st), g_st = static_cast<int>(a.do_st), o_st = static_cast<int>(a.o_st);
+    // the first query head's; the others follow at q_sh, ...
+    const uint16_t *const q0h = head_of<uint16_t>(a.q, a.q_sb, b, a.q_sh, hk * rep + h0), *const g0h = head_of<uint16_t>(a.d_o, a.do_sb, b, a.do_sh, hk * rep + h0),
+                   *const o0h = head_of<uint16_t>(a.o, a.o_sb, b, a.o_sh, hk * rep + h0), *const kh = head_of<uint16_t>(a.k, a.k_sb, b, a.k_sh, hk),
+                   *const vh = head_of<uint16_t>(a.v, a.v_sb, b, a.v_sh, hk);
     Mover<D, G, BMQ> mq, mg;
-    mq.init(gt, a.q_st, dk);
-    mg.init(gt, a.do_st, dk);
+    mq.init(gt, q_st, dk);
+    mg.init(gt, g_st, dk);
     float row_r = 0.0f;
     bf16x8 oreg[BY_ROW ? KK : 1];
     typename std::conditional<BY_CHUNK, Mover<D, G, BMQ>, int>::type mo;
-    if constexpr (BY_CHUNK) mo.init(gt, a.o_st, dk);
+    if constexpr (BY_CHUNK) mo.init(gt, o_st, dk);
     // steps advance by KW; the (head, tile) of the next fetch is counted up
-    int f_h = kg / nqt, f_t = kg % nqt, c_t = f_t;
+    int f_h = 0, f_t = kg;
+    while (f_t >= nqt) f_t -= nqt, ++f_h;
+    int c_t = f_t;
     auto fetch = [&](int i) {
         if (i * KW + kg < steps) {
-            const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * BMQ;
-            mq.load(a.q, b * a.q_sb + h * a.q_sh, a.q_st, r0, a.T, dk);
-            mg.load(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, r0, a.T, dk);
+            const int r0 = (qt_lo + f_t) * BMQ;
+            mq.load(q0h + f_h * a.q_sh, q_st, r0, a.T, dk);
+            mg.load(g0h + f_h * a.do_sh, g_st, r0, a.T, dk);
             if (gt < 2 * BMQ) {  // LSE in the first BMQ threads, delta in the next; rows past the end are masked
                 const int t = min(r0 + gt % BMQ, a.T - 1);
-                const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + t;
+                const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + hk * rep + h0 + f_h) * a.T + t;
                 if (gt < BMQ)
                     row_r = a.lse[lrow];
                 else if (!OWN_DELTA)
                     row_r = a.delta[lrow];
             }
-            if constexpr (BY_CHUNK) mo.load(a.o, b * a.o_sb + h * a.o_sh, a.o_st, r0, a.T, dk);
-            if constexpr (BY_ROW) load_row<D>(a.o, b * a.o_sb + h * a.o_sh, a.o_st, r0 + c32, a.T, dk, g, oreg);
+            if constexpr (BY_CHUNK) mo.load(o0h + f_h * a.o_sh, o_st, r0, a.T, dk);
+            if constexpr (BY_ROW) load_row<D, EXACT && (QW > 1) && D <= 64>(o0h + f_h * a.o_sh, o_st, r0, a.T, dk, c32, g, oreg);
             f_t += KW;
             while (f_t >= nqt) f_t -= nqt, ++f_h;
         }
@@ -545,8 +576,8 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     };
     fetch(0);
     bf16x8 kreg[KK], vreg[KK];
-    load_row<D>(a.k, b * a.k_sb + hk * a.k_sh, a.k_st, kj, a.T, dk, g, kreg);
-    load_row<D>(a.v, b * a.v_sb + hk * a.v_sh, a.v_st, kj, a.T, dk, g, vreg);
+    load_row<D, EXACT && (QW > 1) && D <= 64>(kh, static_cast<int>(a.k_st), kw0, a.T, dk, c32, g, kreg);
+    load_row<D, EXACT && (QW > 1) && D <= 64>(vh, static_cast<int>(a.v_st), kw0, a.T, dk, c32, g, vreg);
     f32x16 acc[2 * DB];  // dV^T, dK^T
 #pragma unroll
     for (int n = 0; n < 2 * DB; ++n)
@@ -606,29 +637,34 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
         if (i + 1 < iters) commit(i + 1);
         tile_barrier<QW>();
     }
-    float* red = reinterpret_cast<float*>(lds) + qg * KW * DB * 1024;
     if (KW > 1 && QW == 1) __syncthreads();  // every group has read its last tile
-    join_groups<DB, KW>(acc, red, kg, lane);
-    if (KW > 1) __syncthreads();
-    join_groups<DB, KW>(acc + DB, red, kg, lane);
     // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
     // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
     const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1);
-    if (kj < a.T && (chunk < 0 || to_tail)) {
-        const bool parts = hs > 1 && !to_tail;
-        const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
-                                   : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
-        const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
-        const bool scratch = parts || to_tail;
-        void* const room = to_tail ? a.tail : a.part;
-        const int64_t rv = scratch ? pv : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
-        const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
-        void* const dst_v = scratch ? room : a.dv;
-        void* const dst_k = scratch ? room : a.dk;
-        const bool f32 = scratch || a.grad_f32;
+    const bool parts = hs > 1 && !to_tail;
+    const int64_t pk = to_tail ? ((static_cast<int64_t>(kvu) * (tl.nch + 1) + (chunk >= 0 ? chunk : tl.nch)) * 64 + kj) * dk
+                               : (static_cast<int64_t>(kvu) * hs + rr) * 2 * a.T * dk + static_cast<int64_t>(kj) * dk;
+    const int64_t pv = pk + static_cast<int64_t>(to_tail ? 32 : a.T) * dk;
+    const bool scratch = parts || to_tail, mine = kj < a.T && (chunk < 0 || to_tail);
+    void* const room = to_tail ? a.tail : a.part;
+    const int64_t rv = scratch ? pv : b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st;
+    const int64_t rk = scratch ? pk : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
+    void* const dst_v = scratch ? room : a.dv;
+    void* const dst_k = scratch ? room : a.dk;
+    const bool f32 = scratch || a.grad_f32;
+    if constexpr (KW > 1) {
+        constexpr int N = JOIN_BOTH<D> ? 2 * DB : DB;
+#pragma unroll
+        for (int n0 = 0; n0 < 2 * DB; n0 += N) {
+            if (n0 > 0) __syncthreads();
+            join_shares<N, KW, 2>(acc + n0, reinterpret_cast<float*>(lds) + qg * KW * N * 1024, kg, lane, no_weights, [&](int n, int qd, const f32x4 (&v)[2]) {
+                const bool is_v = n0 + n < DB;
+                if (mine) store_half(f32, is_v ? dst_v : dst_k, is_v ? rv : rk, is_v ? n : n0 + n - DB, qd, g, v, is_v ? 1.0f : a.scale, dk);
+            });
+        }
+    } else if (mine) {
 #pragma unroll
         for (int n = 0; n < 2 * DB; ++n) {
-            if (KW > 1 && n % DB % KW != kg) continue;
             if (n < DB)
                 store_block(f32, dst_v, rv, n, g, acc[n], 1.0f, dk);
             else
