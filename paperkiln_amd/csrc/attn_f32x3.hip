@@ -85,16 +85,16 @@ struct Mover3 {
     static_assert(CPT >= 1 && 32 * NCH % G == 0, "every thread moves the same number of chunks");
     int off[CPT];
     u32x4 r[CPT];
-    __device__ void init(int t, int64_t st, int dk) {
+    __device__ void init(int t, int st, int dk) {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int c = t + G * i, row = c / NCH, ch = c % NCH;
-            off[i] = ch * 4 < dk ? static_cast<int>(row * st + ch * 4) * 4 : static_cast<int>(OUTSIDE);
+            off[i] = ch * 4 < dk ? (row * st + ch * 4) * 4 : static_cast<int>(OUTSIDE);
         }
     }
-    __device__ void load(const void* base, int64_t elem_off, int64_t st, int r0, int T, int dk) {
-        const int64_t left = ((static_cast<int64_t>(T) - r0 - 1) * st + dk) * 4;  // r0 < T
-        float* p = static_cast<float*>(const_cast<void*>(base)) + elem_off + static_cast<int64_t>(r0) * st;
+    __device__ void load(const float* head, int st, int r0, int T, int dk) {
+        const int64_t left = (static_cast<int64_t>(T - r0 - 1) * st + dk) * 4;  // r0 < T
+        float* p = const_cast<float*>(head) + static_cast<int64_t>(r0) * st;
         const __amdgpu_buffer_rsrc_t rs =
             __builtin_amdgcn_make_buffer_rsrc(p, 0, left > 0x7fffffff ? 0x7fffffff : static_cast<int>(left), 0x00020000);
 #pragma unroll
@@ -133,34 +133,41 @@ __device__ inline void split8(const float (&x)[8], bf16x8& h, bf16x8& m, bf16x8&
     l = *reinterpret_cast<bf16x8*>(&p[2]);
 }
 
-// Row `row` of a head as three operands: chunk kk holds columns 16 kk + 8 g .. +7; zero past T and past dk. `dot`, when
-// given, gathers this lane's share of the row's product with a row of `other`.
+// Row `row` of a head, all of it on its way before any of it is split: chunk 2 kk + half holds columns 16 kk + 8 g + 4 half .. +3; zero past T and past dk.
+// A chunk split, or multiplied into delta, where it is loaded waits there, a trip to memory for each of D / 8 chunks: T 241 x 10, 4 heads of 96 forward
+// 18.4 -> 15.9 us; T 1037 x 2, 8 heads of 32 19.5 -> 18.7; dQ and dK/dV in one launch, T 836 x 2, 8 heads of 64 64.8 -> 58.7; long chains level.
 template <int D>
-__device__ inline void load_row3(const void* base, int64_t off, int64_t st, int row, int T, int dk, int g, bf16x8 (&out)[3][D / 16],
-                                 const float* other = nullptr, float* dot = nullptr) {
-    float sum = 0.0f;
+struct Row {
+    f32x4 x[D / 8];
+    __device__ void load(const float* head, int64_t st, int row, int T, int dk, int g) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-        float x[8];
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int col = 16 * kk + 8 * g + 4 * half;
+        for (int j = 0; j < D / 8; ++j) {
+            const int col = 16 * (j / 2) + 8 * g + 4 * (j % 2);
             f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (row < T && col < dk) {
-                z = *reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + off + row * st + col);
-                if (dot) {
-                    const f32x4 y = *reinterpret_cast<const f32x4*>(other + col);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sum = fmaf(y[e], z[e], sum);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[4 * half + e] = z[e];
+            if (row < T && col < dk) z = *reinterpret_cast<const f32x4*>(head + row * st + col);
+            x[j] = z;
         }
-        split8(x, out[0][kk], out[1][kk], out[2][kk]);
     }
-    if (dot) *dot = sum;
-}
+    // as three operands: chunk kk holds columns 16 kk + 8 g .. +7
+    __device__ void split(bf16x8 (&out)[3][D / 16]) const {
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = x[2 * kk + e / 4][e % 4];
+            split8(v, out[0][kk], out[1][kk], out[2][kk]);
+        }
+    }
+    // this lane's share of the product with another row
+    __device__ float dot(const Row& o) const {
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < D / 8; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = fmaf(o.x[j][e], x[j][e], sum);
+        return sum;
+    }
+};
 
 // (rows of the tile) . b over the columns: all small products first, then the large ones on top of their sum
 template <int D>
@@ -428,19 +435,21 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
     int b, h, hk, qblk;
     if (!map_query_block(a, (a.T + BM - 1) / BM, b, h, hk, qblk)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
-    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk),
+                *const qh = head_of<float>(a.q, a.q_sb, b, a.q_sh, h);
+    const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
 
     Mover3<D, G> mk, mv;
-    mk.init(gt, a.k_st, dk);
-    mv.init(gt, a.v_st, dk);
+    mk.init(gt, k_st, dk);
+    mv.init(gt, v_st, dk);
     const KeyTiles kt(a, q0, BM, 32);
     const int iters = (kt.n + KW - 1) / KW;
     auto fetch = [&](int i) {  // this group's i-th tile (past its last: nothing)
         const int at = i * KW + kg;
         if (at < kt.n) {
-            mk.load(a.k, kb, a.k_st, kt.tile(at) * 32, a.T, dk);
-            mv.load(a.v, vb, a.v_st, kt.tile(at) * 32, a.T, dk);
+            mk.load(kh, k_st, kt.tile(at) * 32, a.T, dk);
+            mv.load(vh, v_st, kt.tile(at) * 32, a.T, dk);
         }
     };
     auto commit = [&](int i) {
@@ -449,7 +458,11 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
     };
     fetch(0);
     bf16x8 qreg[3][D / 16];
-    load_row3<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
+    {
+        Row<D> q;
+        q.load(qh, a.q_st, qi, a.T, dk, g);
+        q.split(qreg);
+    }
     f32x16 acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -559,19 +572,21 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
     const int g = lane >> 5, c32 = lane & 31, dk = a.dk_dim;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
-    const int64_t kb = b * a.k_sb + hk * a.k_sh, vb = b * a.v_sb + hk * a.v_sh;
+    const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk),
+                *const qh = head_of<float>(a.q, a.q_sb, b, a.q_sh, h);
+    const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
 
     Mover3<D, G> mk, mv;
-    mk.init(gt, a.k_st, dk);
-    mv.init(gt, a.v_st, dk);
+    mk.init(gt, k_st, dk);
+    mv.init(gt, v_st, dk);
     const KeyTiles kt(a, q0, BM, 32);
     const int iters = (kt.n + KW - 1) / KW;
     auto fetch = [&](int i) {
         const int at = i * KW + kg;
         if (at < kt.n) {
-            mk.load(a.k, kb, a.k_st, kt.tile(at) * 32, a.T, dk);
-            mv.load(a.v, vb, a.v_st, kt.tile(at) * 32, a.T, dk);
+            mk.load(kh, k_st, kt.tile(at) * 32, a.T, dk);
+            mv.load(vh, v_st, kt.tile(at) * 32, a.T, dk);
         }
     };
     auto commit = [&](int i) {
@@ -580,20 +595,25 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     };
     fetch(0);
     bf16x8 qreg[3][D / 16], greg[3][D / 16];
-    load_row3<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, qreg);
-    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
-    float nlse = 0.0f, dl = 0.0f;
-    if (qi < a.T) nlse = -a.lse[lrow] * LOG2E;
-    if (fuse_delta) {
-        float part;
-        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg,
-                     static_cast<const float*>(a.o) + b * a.o_sb + h * a.o_sh + qi * a.o_st, &part);
-        dl = xhalf_sum(part);
-        if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
-    } else {
-        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, greg);
-        if (qi < a.T) dl = a.delta[lrow];
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(qi, a.T - 1);
+    float dl = 0.0f;
+    const float lse = a.lse[lrow];
+    {
+        Row<D> q, d_o;
+        q.load(qh, a.q_st, qi, a.T, dk, g);
+        d_o.load(head_of<float>(a.d_o, a.do_sb, b, a.do_sh, h), a.do_st, qi, a.T, dk, g);
+        if (fuse_delta) {
+            Row<D> o;
+            o.load(head_of<float>(a.o, a.o_sb, b, a.o_sh, h), a.o_st, qi, a.T, dk, g);
+            dl = xhalf_sum(d_o.dot(o));
+            if (qi < a.T && g == 0 && kg == 0) a.delta[lrow] = dl;
+        } else {
+            dl = a.delta[lrow];
+        }
+        q.split(qreg);
+        d_o.split(greg);
     }
+    const float nlse = -lse * LOG2E;
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
     f32x16 acc[DB];
 #pragma unroll
@@ -700,8 +720,9 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     const int nqt = qt_hi - qt_lo + 1, steps = nqt * nh;
 
     // role 0 moves Q and the rows' LSE, role 1 dO and their delta
-    const void* const src = role == 0 ? a.q : a.d_o;
-    const int64_t s_sb = role == 0 ? a.q_sb : a.do_sb, s_sh = role == 0 ? a.q_sh : a.do_sh, s_st = role == 0 ? a.q_st : a.do_st;
+    const int64_t s_sh = role == 0 ? a.q_sh : a.do_sh;
+    const int s_st = static_cast<int>(role == 0 ? a.q_st : a.do_st);
+    const float* const src = head_of<float>(role == 0 ? a.q : a.d_o, role == 0 ? a.q_sb : a.do_sb, b, s_sh, hk * rep + h0);  // the first query head's
     const float* const src_rows = role == 0 ? a.lse : a.delta;
     const float row_sc = role == 0 ? -LOG2E : 1.0f;
     Mover3<D, G> mv;
@@ -709,9 +730,9 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     float row_r = 0.0f;
     int f_h = 0, f_t = 0;  // the (head, tile) of the next fetch
     auto fetch = [&]() {
-        const int h = hk * rep + h0 + f_h, r0 = (qt_lo + f_t) * 32;
-        mv.load(src, b * s_sb + h * s_sh, s_st, r0, a.T, dk);
-        if (gt < 32) row_r = src_rows[(static_cast<int64_t>(b) * a.Hq + h) * a.T + min(r0 + gt, a.T - 1)];  // rows past the end are masked
+        const int r0 = (qt_lo + f_t) * 32;
+        mv.load(src + f_h * s_sh, s_st, r0, a.T, dk);
+        if (gt < 32) row_r = src_rows[(static_cast<int64_t>(b) * a.Hq + hk * rep + h0 + f_h) * a.T + min(r0 + gt, a.T - 1)];  // rows past the end are masked
         if (++f_t == nqt) f_t = 0, ++f_h;
     };
     auto commit = [&](int i) {
@@ -721,8 +742,11 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     };
     fetch();
     bf16x8 res[3][D / 16];  // K rows for role 0, V rows for role 1
-    load_row3<D>(role == 0 ? a.k : a.v, role == 0 ? b * a.k_sb + hk * a.k_sh : b * a.v_sb + hk * a.v_sh, role == 0 ? a.k_st : a.v_st,
-                 kj, a.T, dk, g, res);
+    {
+        Row<D> kv;
+        kv.load(head_of<float>(role == 0 ? a.k : a.v, role == 0 ? a.k_sb : a.v_sb, b, role == 0 ? a.k_sh : a.v_sh, hk), role == 0 ? a.k_st : a.v_st, kj, a.T, dk, g);
+        kv.split(res);
+    }
     f32x16 acc[DB];  // dV^T, dK^T
 #pragma unroll
     for (int n = 0; n < DB; ++n)
@@ -863,29 +887,29 @@ __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta)
     const float cexp = a.scale * LOG2E;
 
     // role 0 moves K, role 1 V
-    const void* const src = role == 0 ? a.k : a.v;
-    const int64_t s_off = role == 0 ? b * a.k_sb + hk * a.k_sh : b * a.v_sb + hk * a.v_sh, s_st = role == 0 ? a.k_st : a.v_st;
+    const float* const src = head_of<float>(role == 0 ? a.k : a.v, role == 0 ? a.k_sb : a.v_sb, b, role == 0 ? a.k_sh : a.v_sh, hk);
+    const int s_st = static_cast<int>(role == 0 ? a.k_st : a.v_st);
     Mover3<D, G> mv;
     mv.init(gt, s_st, dk);
     const KeyTiles kt(a, q0, BM, 32);
-    auto fetch = [&](int i) { mv.load(src, s_off, s_st, kt.tile(i) * 32, a.T, dk); };
+    auto fetch = [&](int i) { mv.load(src, s_st, kt.tile(i) * 32, a.T, dk); };
     auto commit = [&](int i) { mv.store(lds + (i & 1) * TILE + role * 3 * PLANE, gt); };
     fetch(0);
     bf16x8 res[3][D / 16];  // Q rows for role 0, dO rows for role 1
-    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + qi;
-    float row_r = 0.0f;  // -LSE log2(e) for role 0, delta for role 1
-    if (role == 0) {
-        load_row3<D>(a.q, b * a.q_sb + h * a.q_sh, a.q_st, qi, a.T, dk, g, res);
-        if (qi < a.T) row_r = -a.lse[lrow] * LOG2E;
-    } else if (fuse_delta) {
-        float part;
-        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, res,
-                     static_cast<const float*>(a.o) + b * a.o_sb + h * a.o_sh + qi * a.o_st, &part);
-        row_r = xhalf_sum(part);
-        if (qi < a.T && g == 0) a.delta[lrow] = row_r;
-    } else {
-        load_row3<D>(a.d_o, b * a.do_sb + h * a.do_sh, a.do_st, qi, a.T, dk, g, res);
-        if (qi < a.T) row_r = a.delta[lrow];
+    const int64_t lrow = (static_cast<int64_t>(b) * a.Hq + h) * a.T + min(qi, a.T - 1);
+    // -LSE log2(e) for role 0, delta for role 1
+    float row_r = role == 0 ? a.lse[lrow] : fuse_delta ? 0.0f : a.delta[lrow];
+    {
+        Row<D> r;
+        r.load(head_of<float>(role == 0 ? a.q : a.d_o, role == 0 ? a.q_sb : a.do_sb, b, role == 0 ? a.q_sh : a.do_sh, h), role == 0 ? a.q_st : a.do_st, qi, a.T, dk, g);
+        if (role == 1 && fuse_delta) {
+            Row<D> o;
+            o.load(head_of<float>(a.o, a.o_sb, b, a.o_sh, h), a.o_st, qi, a.T, dk, g);
+            row_r = xhalf_sum(r.dot(o));
+            if (qi < a.T && g == 0) a.delta[lrow] = row_r;
+        }
+        if (role == 0) row_r = -row_r * LOG2E;
+        r.split(res);
     }
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
     f32x16 acc[HB];
