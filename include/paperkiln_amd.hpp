@@ -163,6 +163,7 @@ public:
     // grad's storage is also another Variable's grad (both parents of an add take the same tensor): it is read-only
     // until own_grad() has given this Variable a copy of its own. accumulate(), ensure_grad() and zero_grad() do so.
     bool grad_shared = false;
+    Tensor one;  // a [1,1] node's kernel may have left a 1 beside its result: what backward() seeds it with (else it writes one)
     // grad is exactly 1: backward() seeded this [1,1] root and nothing has been added since (lets a scalar loss's
     // backward skip reading its upstream gradient back from the device). Code that writes grad directly clears it.
     bool grad_is_unit = false;

@@ -656,14 +656,14 @@ struct ColSums {
         int nparts, C;
     } job[MAX];
 };
-__global__ void colsum_parts(ColSums sums) {
-    const float* const part = sums.job[blockIdx.y].part;
-    float* const dw = sums.job[blockIdx.y].dw;
-    const int nparts = sums.job[blockIdx.y].nparts, C = sums.job[blockIdx.y].C;
-    // 64 columns x 16 groups of parts per block (1024 threads: each walks a sixteenth of the
-    // parts, the walk being a chain of dependent loads); the groups meet in a fixed order
-    __shared__ float sh[16][64];
-    const int col = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;
+// COLS columns x 16 groups of parts per workgroup (each thread walks a sixteenth of the parts, the walk being a chain of
+// dependent loads); the groups meet in a fixed order
+template <int COLS>
+__device__ void colsum_block(const ColSums::Job& job, int block, float (&sh)[16][COLS]) {
+    const float* const part = job.part;
+    float* const dw = job.dw;
+    const int nparts = job.nparts, C = job.C;
+    const int at = threadIdx.x & (COLS - 1), col = block * COLS + at, grp = threadIdx.x / COLS;
     float s = 0.0f;
     if (col < C) {
         int p = grp;
@@ -674,13 +674,17 @@ __global__ void colsum_parts(ColSums sums) {
         }
         for (; p < nparts; p += 16) s += part[static_cast<int64_t>(p) * C + col];
     }
-    sh[grp][threadIdx.x & 63] = s;
+    sh[grp][at] = s;
     __syncthreads();
     if (grp == 0 && col < C) {
         float t = 0.0f;
-        for (int q = 0; q < 16; ++q) t += sh[q][threadIdx.x];
+        for (int q = 0; q < 16; ++q) t += sh[q][at];
         dw[col] += t;
     }
+}
+__global__ void colsum_parts(ColSums sums) {
+    __shared__ float sh[16][64];
+    colsum_block<64>(sums.job[blockIdx.y], blockIdx.x, sh);
 }
 // dst[i] = beta * dst[i] + sum_s part[s][i], parts added in index order
 template <typename T>
@@ -859,9 +863,16 @@ __global__ void __launch_bounds__(EMB_NT) emb_bwd_runs(const T* dy, const int* s
 // The same sums without the sort, for a batch of ids that a workgroup can look through itself: block p leaves if an
 // earlier row has row p's id, and otherwise lists the later rows that have it, in ascending order (each wavefront its own
 // quarter of them), and adds them up. A sort of a few hundred ids is four launches that take 15 us on an idle chip.
+// Workgroups n, n + 1, ... take the held sums, `per` to each: a launch of their own is 2.5 us and what lies between two.
 constexpr int EMB_SCAN_MAX = 4096;
 template <typename T>
-__global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, float* dtable, int n, int d) {
+__global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, float* dtable, int n, int d, ColSums sums, int per) {
+    static_assert(NT == 256, "16 columns x 16 groups of parts");
+    if (static_cast<int>(blockIdx.x) >= n) {
+        __shared__ float sh[16][16];
+        const int at = blockIdx.x - n, job = at / per;
+        return colsum_block<16>(sums.job[job], at - job * per, sh);
+    }
     __shared__ uint16_t rows[NT / 64][EMB_SCAN_MAX / (NT / 64) + 64];
     __shared__ int count[NT / 64];
     const int p = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1020,7 +1031,7 @@ __global__ void sum_f32_k(const float* x, int64_t n, double* out) {
 }
 // mean of n floats, accumulated in double and rounded to float once: what the host does with
 // k_sum_f32_to_host's result, without the round trip
-__global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, float* out) {
+__global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, float* out, int with_one, float* pinned) {
     // thread t takes the elements sum_f32_k's thread t % NT takes, a quarter of them: the NT partial sums are formed
     // from four pieces each and then added in sum_f32_k's tree
     __shared__ double sh[1024];
@@ -1035,7 +1046,12 @@ __global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, fl
         if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = static_cast<float>(sh[0] / static_cast<double>(n));
+    if (threadIdx.x == 0) {
+        const float mean = static_cast<float>(sh[0] / static_cast<double>(n));
+        out[0] = mean;
+        if (with_one) out[1] = 1.0f;
+        if (pinned) *pinned = mean;
+    }
 }
 __global__ void sumsq_part(const float* x, int64_t n, double* part) {
     __shared__ double sh[NT];
@@ -1069,8 +1085,7 @@ __global__ void sumsq_part(const float* x, int64_t n, double* part) {
 // gradients are to be multiplied by, and the norm itself for the host (pinned memory). It stays on the device: the
 // optimizer step behind it reads it there, where a copy to the host and back between the two left the GPU idle for 35 to
 // 50 us a step.
-__global__ void clip_factor_k(const double* part, int n, float max_norm, float* factor, float* norm_out) {
-    __shared__ double sh[NT];
+__device__ float clip_of(const double* part, int n, float max_norm, double (&sh)[NT], float* norm) {
     double s = 0.0;
     for (int i = threadIdx.x; i < n; i += NT) s += part[i];
     sh[threadIdx.x] = s;
@@ -1079,11 +1094,14 @@ __global__ void clip_factor_k(const double* part, int n, float max_norm, float* 
         if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const double total = sqrt(sh[0]), limit = static_cast<double>(max_norm);
-        *factor = total > limit && total > 0.0 ? static_cast<float>(limit / total) : 1.0f;
-        *norm_out = static_cast<float>(total);
-    }
+    const double total = sqrt(sh[0]), limit = static_cast<double>(max_norm);
+    if (norm && threadIdx.x == 0) *norm = static_cast<float>(total);
+    return total > limit && total > 0.0 ? static_cast<float>(limit / total) : 1.0f;
+}
+__global__ void clip_factor_k(const double* part, int n, float max_norm, float* factor, float* norm_out) {
+    __shared__ double sh[NT];
+    const float f = clip_of(part, n, max_norm, sh, norm_out);
+    if (threadIdx.x == 0) *factor = f;
 }
 __device__ inline void adamw_one(float& p, float g, float& m, float& v, float lr, float b1, float b2, float eps, float wd, float c1, float c2) {
     m = b1 * m + (1.0f - b1) * g;
@@ -1122,15 +1140,23 @@ struct AdamWParts {
         int count, cols, ld, off;
     } part[MAX];
 };
-template <typename TY>
+//
+// OWN_CLIP: every workgroup forms the clip's factor from the partial sums itself, block 0 writes the norm. Up to 1024 workgroups that costs
+// less than a launch before this one (0.46 M parameters: 2.8 us and the gap between two against 1 us).
+template <typename TY, bool OWN_CLIP>
 __global__ void adamw_parts_k(AdamWParts ps, float* p, float* g, float* m, float* v, float lr, float b1, float b2, float eps, float wd,
-                              float c1, float c2, const float* clip) {
+                              float c1, float c2, Clip cl) {
+    float own = 1.0f;
+    if constexpr (OWN_CLIP) {
+        __shared__ double sh[NT];
+        own = clip_of(cl.part_dev, cl.n, cl.max_norm, sh, blockIdx.x == 0 ? cl.norm_pinned : nullptr);
+    }
     const int block = static_cast<int>(blockIdx.x);
     const int j = __builtin_popcountll(__builtin_amdgcn_ballot_w64(block >= ps.begin[threadIdx.x & 63])) - 1;
     const AdamWParts::Part part = ps.part[j];
     const int e = ((block - ps.begin[j]) * NT + static_cast<int>(threadIdx.x)) * 4;
     if (e >= part.count) return;
-    const float gs = clip ? *clip : 1.0f;
+    const float gs = OWN_CLIP ? own : cl.factor ? *cl.factor : 1.0f;
     const int64_t i = part.at + e;
     auto at = [&](float* s) -> f32x4& { return *reinterpret_cast<f32x4*>(s + i); };
     f32x4 gi = at(g), mi = at(m), vi = at(v), pi = at(p);
@@ -1168,7 +1194,24 @@ __global__ void begin_pass_k(f32x4* clear, int64_t n4, const int* pinned, int* t
     for (int64_t i = first; i < n; i += stride) to[i] = pinned[i];
     for (int64_t i = first; i < n4; i += stride) clear[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 }
+// The same with the gather of the tokens' embeddings, ids straight from pinned memory: a launch and a dependent trip to memory less for
+// batches whose ids' way over the link fits into the time of the clearing. A thread gathers four columns.
+template <typename T>
+__global__ void begin_pass_rows(f32x4* clear, int64_t n4, const int* pinned, int* to, int64_t n, const float* table, T* y, int64_t quads, int d4) {
+    const int64_t first = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x, stride = static_cast<int64_t>(gridDim.x) * NT;
+    const int row = static_cast<int>(first) / d4, c = (static_cast<int>(first) - row * d4) * 4;
+    const int id = first < quads ? pinned[row] : 0;  // quads threads or more are launched
+    for (int64_t i = first; i < n; i += stride) to[i] = pinned[i];
+    for (int64_t i = first; i < n4; i += stride) clear[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (first >= quads) return;
+    const f32x4 v = *reinterpret_cast<const f32x4*>(table + static_cast<int64_t>(id) * (d4 * 4) + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) stf(y, first * 4 + e, v[e]);
+}
 __global__ void copy_word_k(const uint32_t* src, uint32_t* dst) { *dst = *src; }
+
+// quads of embeddings up to which a pass's first launch gathers them
+constexpr int64_t BEGIN_GATHERS = int64_t{1} << 17;
 
 void same_shape(const Tensor& a, const Tensor& b, const char* who) {
     if (a.rows != b.rows || a.cols != b.cols) throw std::runtime_error(std::string(who) + ": shape mismatch");
@@ -1504,15 +1547,22 @@ void k_embedding_fwd(const Tensor& table, const int* ids, const Tensor& y) {
                                                 y.rows, static_cast<int>(y.cols)));
     post();
 }
-void k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable) {
+bool k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable, const HeldSum* held, int count) {
     if (dy.rows > (1 << 30)) shape_fail("embedding: more than 2^30 rows");
     const int n = static_cast<int>(dy.rows), d = static_cast<int>(dy.cols);
     const hipStream_t st = tape_stream();
     if (n <= EMB_SCAN_MAX) {
-        PK_DISPATCH1(T, dy.dtype, hipLaunchKernelGGL((emb_bwd_scan<T>), dim3(n), dim3(NT), 0, st, static_cast<const T*>(dy.ptr()),
-                                                     ids, static_cast<float*>(dtable.ptr()), n, d));
+        ColSums sums{};
+        int per = 1;
+        const bool with = held && count <= ColSums::MAX;
+        for (int k = 0; with && k < count; ++k) {
+            sums.job[k] = {static_cast<const float*>(held[k].part->p), held[k].dw, held[k].nparts, held[k].cols};
+            per = std::max(per, (held[k].cols + 15) / 16);
+        }
+        PK_DISPATCH1(T, dy.dtype, hipLaunchKernelGGL((emb_bwd_scan<T>), dim3(n + (with ? count * per : 0)), dim3(NT), 0, st,
+                                                     static_cast<const T*>(dy.ptr()), ids, static_cast<float*>(dtable.ptr()), n, d, sums, per));
         post();
-        return;
+        return with;
     }
     Buffer rows_in(sizeof(int) * n), rows_out(sizeof(int) * n), ids_out(sizeof(int) * n);
     int* const r_in = static_cast<int*>(rows_in.p);
@@ -1527,6 +1577,7 @@ void k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable) {
                                                  static_cast<const T*>(dy.ptr()), i_out, r_out,
                                                  static_cast<float*>(dtable.ptr()), n, d));
     post();
+    return false;
 }
 void k_ce_rows(const Tensor& logits, const int* targets, float gscale, float* nll_rows) {
     PK_DISPATCH1(T, logits.dtype, hipLaunchKernelGGL((ce_rows<T>), dim3(logits.rows), dim3(NT), 0, tape_stream(),
@@ -1552,9 +1603,9 @@ bool k_ce_rows_once(const Tensor& logits, const int* targets, float gscale, floa
     post();
     return true;
 }
-void k_mean_f32(const float* x, int64_t n, const Tensor& out) {
-    if (out.dtype != PK_F32 || out.rows * out.cols != 1) throw std::runtime_error("mean: the result is one float");
-    hipLaunchKernelGGL(mean_f32_k, dim3(1), dim3(1024), 0, tape_stream(), x, n, static_cast<float*>(out.ptr()));
+void k_mean_f32(const float* x, int64_t n, const Tensor& out, float* pinned) {
+    if (out.dtype != PK_F32 || out.rows != 1 || out.cols < 1 || out.cols > 2) throw std::runtime_error("mean: the result is one float, or it and a 1");
+    hipLaunchKernelGGL(mean_f32_k, dim3(1), dim3(1024), 0, tape_stream(), x, n, static_cast<float*>(out.ptr()), out.cols == 2 ? 1 : 0, pinned);
     post();
 }
 double k_sum_f32_to_host(const float* x, int64_t n) {
@@ -1591,13 +1642,23 @@ void k_clip_factor(const double* part_dev, int n, float max_norm, float* factor_
     hipLaunchKernelGGL(clip_factor_k, dim3(1), dim3(NT), 0, tape_stream(), part_dev, n, max_norm, factor_dev, norm_pinned);
     post();
 }
-void k_begin_pass(const Tensor& clear, const int* pinned, int* to, int64_t n) {
+bool k_begin_pass(const Tensor& clear, const int* pinned, int* to, int64_t n, const Tensor& table, const Tensor& y) {
     const int64_t n4 = clear.numel() / 4;
     if (clear.dtype != PK_F32 || clear.numel() % 4 || !aligned16p(clear.ptr())) throw std::runtime_error("begin_pass: whole 16-byte groups");
-    const int64_t blocks = std::min<int64_t>((std::max(n4, n) + NT - 1) / NT, 16384);
+    const int64_t quads = y.numel() / 4, blocks = std::min<int64_t>((std::max(n4, n) + NT - 1) / NT, 16384);
+    const bool gather = quads <= BEGIN_GATHERS && y.cols % 4 == 0 && table.dtype == PK_F32 && table.cols == y.cols && aligned16p(table.ptr());
+    if (gather) {
+        const unsigned grid = static_cast<unsigned>(std::max<int64_t>(blocks, (quads + NT - 1) / NT));
+        PK_DISPATCH1(T, y.dtype, hipLaunchKernelGGL((begin_pass_rows<T>), dim3(grid), dim3(NT), 0, tape_stream(), static_cast<f32x4*>(clear.ptr()), n4,
+                                                    pinned, to, n, static_cast<const float*>(table.ptr()), static_cast<T*>(y.ptr()), quads,
+                                                    static_cast<int>(y.cols / 4)));
+        post();
+        return true;
+    }
     hipLaunchKernelGGL(begin_pass_k, dim3(static_cast<unsigned>(std::max<int64_t>(blocks, 1))), dim3(NT), 0, tape_stream(),
                        static_cast<f32x4*>(clear.ptr()), n4, pinned, to, n);
     post();
+    return false;
 }
 void k_word_to_pinned(const void* src, void* pinned) {
     hipLaunchKernelGGL(copy_word_k, dim3(1), dim3(1), 0, tape_stream(), static_cast<const uint32_t*>(src),
@@ -1613,7 +1674,7 @@ void k_adamw(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v,
 }
 
 bool k_adamw_parts(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, const std::vector<AdamWPart>& parts, float lr,
-                   float b1, float b2, float eps, float wd, float c1, float c2, const float* clip_dev) {
+                   float b1, float b2, float eps, float wd, float c1, float c2, const Clip& clip) {
     int dtype = PK_F32;
     for (const AdamWPart& q : parts) {
         if (q.count % 4 || q.at % 4 || q.count > (int64_t{1} << 30)) return false;
@@ -1627,6 +1688,10 @@ bool k_adamw_parts(const Tensor& p, const Tensor& g, const Tensor& m, const Tens
         if (!q.copy.empty() && q.copy.dtype != dtype) return false;
     for (const Tensor* t : {&p, &g, &m, &v})
         if (t->dtype != PK_F32 || !aligned16p(t->ptr())) return false;
+    int64_t groups = 0;
+    for (const AdamWPart& q : parts) groups += (q.count / 4 + NT - 1) / NT;
+    const bool own_clip = clip.part_dev && groups > 0 && groups <= 1024 && parts.size() <= AdamWParts::MAX;
+    if (clip.part_dev && !own_clip) k_clip_factor(clip.part_dev, clip.n, clip.max_norm, clip.factor, clip.norm_pinned);
     size_t done = 0;
     while (done < parts.size()) {
         AdamWParts ps{};
@@ -1640,10 +1705,17 @@ bool k_adamw_parts(const Tensor& p, const Tensor& g, const Tensor& m, const Tens
         }
         for (int k = n; k <= AdamWParts::MAX; ++k) ps.begin[k] = blocks;
         if (blocks == 0) continue;
-        PK_DISPATCH1(TY, dtype, hipLaunchKernelGGL((adamw_parts_k<TY>), dim3(static_cast<unsigned>(blocks)), dim3(NT), 0, tape_stream(),
-                                                   ps, static_cast<float*>(p.ptr()), static_cast<float*>(g.ptr()),
-                                                   static_cast<float*>(m.ptr()), static_cast<float*>(v.ptr()), lr, b1, b2, eps, wd, c1,
-                                                   c2, clip_dev));
+        const auto launch = [&](auto own) {
+            constexpr bool OWN = decltype(own)::value;
+            PK_DISPATCH1(TY, dtype, hipLaunchKernelGGL((adamw_parts_k<TY, OWN>), dim3(static_cast<unsigned>(blocks)), dim3(NT), 0, tape_stream(),
+                                                       ps, static_cast<float*>(p.ptr()), static_cast<float*>(g.ptr()),
+                                                       static_cast<float*>(m.ptr()), static_cast<float*>(v.ptr()), lr, b1, b2, eps, wd, c1,
+                                                       c2, clip));
+        };
+        if (own_clip)
+            launch(std::true_type{});
+        else
+            launch(std::false_type{});
         post();
     }
     return true;

@@ -284,9 +284,8 @@ struct Model {
         return ops::gated_mlp(h2, b.gate, b.up, b.down, x1, !recomputing());
     }
 
-    // Llama::forward (llama.cpp:71-89) up to the final norm; positions restart per sequence.
-    Var hidden(const std::shared_ptr<Buffer>& ids, const std::shared_ptr<Buffer>& pos_dev, int64_t n, int64_t seq_len) const {
-        Var h = ops::embedding(embed, ids, n);
+    // Llama::forward (llama.cpp:71-89) from the embedded tokens up to the final norm; positions restart per sequence.
+    Var hidden(Var h, const std::shared_ptr<Buffer>& pos_dev, int64_t seq_len) const {
         for (const Block& blk : blocks) {
             if (checkpoint_blocks && grad_enabled()) {
                 const Block* bp = &blk;
@@ -315,7 +314,7 @@ int guarded(F&& f) {
 
 // AdamW on every parameter with the copies that the products read. False, with nothing done, where the kernel does not take
 // them (or a parameter has two copies).
-bool adamw_with_copies(const Model& m, float lr, float b1, float b2, float eps, float wd, float c1, float c2, const float* factor) {
+bool adamw_with_copies(const Model& m, float lr, float b1, float b2, float eps, float wd, float c1, float c2, const Clip& clip) {
     std::unordered_map<const Variable*, CastJob> copies;
     for (const ShadowCopy& s : shadow_copies())
         if (!copies.emplace(s.of, s.job).second) return false;
@@ -333,7 +332,7 @@ bool adamw_with_copies(const Model& m, float lr, float b1, float b2, float eps, 
         if (p.buf != m.pslab.buf || kv.second->grad.buf != m.gslab.buf || kv.second->grad.off_bytes != p.off_bytes) return false;
         parts.push_back(std::move(part));
     }
-    return found == copies.size() && k_adamw_parts(m.pslab, m.gslab, m.mslab, m.vslab, parts, lr, b1, b2, eps, wd, c1, c2, factor);
+    return found == copies.size() && k_adamw_parts(m.pslab, m.gslab, m.mslab, m.vslab, parts, lr, b1, b2, eps, wd, c1, c2, clip);
 }
 
 Model* model_of(void* handle) {
@@ -481,7 +480,6 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         std::memcpy(st + n, host_targets, sizeof(int) * n);
         for (int64_t i = 0; i < n; ++i) st[2 * n + i] = static_cast<int>(i % sl);
         auto sent = std::make_shared<Buffer>(sizeof(int) * 3 * n);
-        k_begin_pass(m->gslab, st, static_cast<int*>(sent->p), 3 * n);
         auto third = [&](int k) {  // a view that keeps the whole transfer's memory
             return std::shared_ptr<Buffer>(new Buffer(static_cast<int*>(sent->p) + k * n, sizeof(int) * n),
                                            [sent](Buffer* b) { delete b; });
@@ -499,8 +497,13 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         const size_t base = dev_live_bytes();  // the allocator's host-side counters: nothing to wait for
         dev_reset_peak();
         const size_t live0 = live_variables();
-        Var hid = m->hidden(ids, pos_dev, n, seq_len);
-        Var l = fused_head ? ops::linear_cross_entropy(hid, m->embed, tg, m->head_chunk_rows, do_backward != 0)
+        Tensor rows = Tensor::make(n, m->cfg.d, compute_dtype());
+        if (!k_begin_pass(m->gslab, st, static_cast<int*>(sent->p), 3 * n, m->embed->data, rows))
+            k_embedding_fwd(m->embed->data, static_cast<const int*>(ids->p), rows);
+        Var hid = m->hidden(ops::embedding_of(m->embed, ids, std::move(rows)), pos_dev, seq_len);
+        // the loss comes back into the pinned staging's spare word; one wait behind the last kernel ends the pass
+        float* hl = reinterpret_cast<float*>(st + 3 * n);
+        Var l = fused_head ? ops::linear_cross_entropy_to(hid, m->embed, tg, m->head_chunk_rows, do_backward != 0, hl)
                            : ops::cross_entropy(ops::matmul_nt(hid, m->embed), tg);
         hid.reset();
         // the allocator's counters move when the host allocates and frees, not when the GPU gets there: no wait here
@@ -509,9 +512,7 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
             stats->activation_bytes_after_forward = static_cast<int64_t>(dev_live_bytes() - base);
         }
         if (do_backward) backward(l);
-        // the loss comes back into the pinned staging's spare word behind the last kernel: one wait ends the pass
-        float* hl = reinterpret_cast<float*>(st + 3 * n);
-        k_word_to_pinned(l->data.ptr(), hl);
+        if (!fused_head) k_word_to_pinned(l->data.ptr(), hl);
         hip_check(hipStreamSynchronize(tape_stream()), "hipStreamSynchronize");
         if (stats) stats->peak_activation_bytes = static_cast<int64_t>(dev_peak_bytes() - base);
         *loss = *hl;
@@ -528,23 +529,23 @@ int pk_llama_adamw_step(void* h, float lr, float b1, float b2, float eps, float 
         }
         // ops::clip_grad_norm over the slab (the padding between parameters is zero), in double as the reference
         // (ops.cpp:1047-1053); the AdamW pass applies it, and the norm reaches the host with the wait at the end
-        std::unique_ptr<Buffer> clip;
+        std::unique_ptr<Buffer> scratch;
         float* const norm = reinterpret_cast<float*>(m->staging(1));
         *norm = 0.0f;
+        Clip clip;
         if (max_norm > 0.0f) {
-            Buffer parts(sizeof(double) * SUMSQ_MAX_PARTS);
-            clip = std::make_unique<Buffer>(sizeof(float));
-            const int nb = k_sumsq_parts(m->gslab, static_cast<double*>(parts.p));
-            k_clip_factor(static_cast<const double*>(parts.p), nb, max_norm, static_cast<float*>(clip->p), norm);
+            scratch = std::make_unique<Buffer>(sizeof(double) * (SUMSQ_MAX_PARTS + 1));
+            double* const parts = static_cast<double*>(scratch->p);
+            clip = Clip{parts, k_sumsq_parts(m->gslab, parts), max_norm, reinterpret_cast<float*>(parts + SUMSQ_MAX_PARTS), norm};
         }
         ++m->t;
         const float c1 = 1.0f - std::pow(b1, static_cast<float>(m->t));
         const float c2 = 1.0f - std::pow(b2, static_cast<float>(m->t));
         // every parameter of this model receives a gradient each step, so the reference's "skip a
         // parameter that never accumulated" (nn.cpp:309) never applies; padding stays at zero
-        const float* const factor = clip ? static_cast<const float*>(clip->p) : nullptr;
-        if (!adamw_with_copies(*m, lr, b1, b2, eps, wd, c1, c2, factor)) {
-            k_adamw(m->pslab, m->gslab, m->mslab, m->vslab, lr, b1, b2, eps, wd, c1, c2, factor);
+        if (!adamw_with_copies(*m, lr, b1, b2, eps, wd, c1, c2, clip)) {
+            if (clip.part_dev) k_clip_factor(clip.part_dev, clip.n, clip.max_norm, clip.factor, clip.norm_pinned);
+            k_adamw(m->pslab, m->gslab, m->mslab, m->vslab, lr, b1, b2, eps, wd, c1, c2, clip.factor);
             refresh_shadows();  // the copies of the weights follow them, in one launch
         }
         hip_check(hipStreamSynchronize(tape_stream()), "hipStreamSynchronize");

@@ -192,15 +192,18 @@ bool defer_weight_gradient(const Tensor& x, const Tensor& dy, int64_t col0, int6
     return true;
 }
 
-void flush_held_sums() {
-    auto& sums = pending().sums;
+std::vector<HeldSum> held_sums() {
     std::vector<HeldSum> held;
-    for (auto& s : sums) {  // asked for again: the weight's gradient may have moved since
+    for (auto& s : pending().sums) {  // asked for again: the weight's gradient may have moved since
         s.sum.dw = static_cast<float*>(s.w->ensure_grad().ptr());
         held.push_back(s.sum);
     }
+    return held;
+}
+void flush_held_sums() {
+    const std::vector<HeldSum> held = held_sums();
     k_add_held(held.data(), static_cast<int>(held.size()));
-    sums.clear();
+    pending().sums.clear();
 }
 void hold_sum(HeldSum&& sum, const Var& w) {
     auto& sums = pending().sums;
@@ -395,8 +398,12 @@ Var record(Tensor result, std::vector<Var> parents, std::function<void(Variable*
 void backward(const Var& root) {
     if (root->data.rows != 1 || root->data.cols != 1)
         throw std::runtime_error("backward: root must be a [1,1] scalar (compose with mean/sum)");
-    Tensor seed = Tensor::make(1, 1, root->data.dtype);
-    k_fill(seed, 1.0f);
+    Tensor seed = std::move(root->one);
+    root->one = Tensor();
+    if (seed.empty()) {
+        seed = Tensor::make(1, 1, root->data.dtype);
+        k_fill(seed, 1.0f);
+    }
     const bool fresh = root->grad.empty();
     root->accumulate_owned(std::move(seed));
     root->grad_is_unit = fresh;
@@ -809,10 +816,16 @@ Var apply_rope(const Var& qkv, const std::shared_ptr<Buffer>& pos, float theta, 
 Var embedding(const Var& table, const std::shared_ptr<Buffer>& ids, int64_t n) {
     Tensor y = Tensor::make(n, table->data.cols, compute_dtype());
     k_embedding_fwd(table->data, static_cast<const int*>(ids->p), y);
-    return record(std::move(y), {table}, [ids](Variable* self) {
+    return embedding_of(table, ids, std::move(y));
+}
+Var embedding_of(const Var& table, const std::shared_ptr<Buffer>& ids, Tensor rows) {
+    return record(std::move(rows), {table}, [ids](Variable* self) {
         const Var& t = self->parents[0];
         if (!t->requires_grad) return;
-        k_embedding_bwd(self->grad, static_cast<const int*>(ids->p), t->ensure_grad());  // scatter-add, ops.cpp:338-347
+        // a model's embedding is the last node of a pass: the sums held until then go with it
+        std::vector<HeldSum> held = held_sums();
+        if (k_embedding_bwd(self->grad, static_cast<const int*>(ids->p), t->ensure_grad(), held.data(), static_cast<int>(held.size())))
+            pending().sums.clear();
     });
 }
 
@@ -968,6 +981,10 @@ Var cross_entropy(const Var& logits, const std::shared_ptr<Buffer>& targets) {
 
 Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffer>& targets, int64_t chunk_rows,
                          bool loss_is_root) {
+    return linear_cross_entropy_to(h, E, targets, chunk_rows, loss_is_root, nullptr);
+}
+Var linear_cross_entropy_to(const Var& h, const Var& E, const std::shared_ptr<Buffer>& targets, int64_t chunk_rows, bool loss_is_root,
+                            float* pinned) {
     const int64_t N = h->data.rows, V = E->data.rows, d = h->data.cols;
     if (d != E->data.cols) shape_fail("matmul: inner dimensions disagree");
     const int* tg = static_cast<const int*>(targets->p);
@@ -1054,10 +1071,13 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
         dl.cols = V;
         if (want_dE) gemm(dl, true, hview, false, dE1.ptr(), PK_F32, V, d, d, r0 == 0 && !dE_in_place ? 0.0f : 1.0f, dl_ld);
     }
-    Tensor out = Tensor::make(1, 1, PK_F32);
-    k_mean_f32(static_cast<const float*>(nll.p), N, out);  // the loss stays on the device: no wait in mid-step
+    Tensor out = Tensor::make(1, 2, PK_F32);
+    k_mean_f32(static_cast<const float*>(nll.p), N, out, pinned);  // the loss stays on the device: no wait in mid-step
+    out.cols = 1;
+    Tensor one = out;
+    one.off_bytes += sizeof(float);
     if (dE_in_place) dE1 = Tensor();
-    return record(std::move(out), {h, E}, [dh1, dE1, dE_in_place](Variable* self) mutable {
+    Var loss = record(std::move(out), {h, E}, [dh1, dE1, dE_in_place](Variable* self) mutable {
         const Var& h = self->parents[0];
         const Var& E = self->parents[1];
         const float g = upstream_scalar(self);  // upstream gradient of the scalar loss
@@ -1078,6 +1098,8 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
         dh1 = Tensor();
         dE1 = Tensor();
     });
+    loss->one = std::move(one);
+    return loss;
 }
 
 double clip_grad_norm(const std::vector<Var>& params, float max_norm) {

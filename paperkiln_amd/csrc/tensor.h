@@ -51,7 +51,8 @@ void k_rope(const Tensor& x, const int* pos, float theta, int d, int head_dim, i
             const Tensor& y);
 void k_rope_inplace(const Tensor& x, const int* pos, float theta, int d, int head_dim, int rot_heads, bool inverse);
 void k_embedding_fwd(const Tensor& table_f32, const int* ids, const Tensor& y);       // ops.cpp:329-337
-void k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable_f32);     // scatter-add, ops.cpp:338-347
+// scatter-add, ops.cpp:338-347; held sums (no two with the same dw) may ride along: true if they did
+bool k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable_f32, const HeldSum* held = nullptr, int count = 0);
 // Row-wise softmax cross-entropy on a block of logits (ops.cpp:350-376): writes
 // dlogits = (P - onehot) * gscale in place and the per-row nll (fp32) with the
 // reference's max(p, 1e-12) clamp.
@@ -61,7 +62,8 @@ void k_ce_rows(const Tensor& logits, const int* targets, float gscale, float* nl
 bool k_ce_rows_once(const Tensor& logits, const int* targets, float gscale, float* nll_rows, const Tensor* dl,
                     int64_t dl_ld = 0);  // dl_ld: row pitch of dl in its own elements (0 = cols)
 double k_sum_f32_to_host(const float* x, int64_t n);                   // double accumulation, ops.cpp:360-367
-void k_mean_f32(const float* x, int64_t n, const Tensor& out);         // the same sum / n into a [1,1] float, no host round trip
+// the same sum / n into a float, no host round trip; a 1 behind it ([1,2] out), and the mean to pinned host memory if given
+void k_mean_f32(const float* x, int64_t n, const Tensor& out, float* pinned = nullptr);
 double k_sumsq_to_host(const Tensor& g);                               // clip_grad_norm's sum, ops.cpp:1046-1052
 // The same in two halves, so that many gradients cost one host round trip: per-block partial sums (at most
 // SUMSQ_MAX_PARTS doubles) into device memory, then one copy and a host sum over all of them.
@@ -71,7 +73,16 @@ double k_sum_f64_to_host(const double* part_dev, int64_t n);
 // What ops::clip_grad_norm multiplies the gradients by (1 where the norm is within max_norm), from those partial sums,
 // left on the device for k_adamw; the norm itself goes to pinned host memory, to be read after a wait for the stream.
 void k_clip_factor(const double* part_dev, int n, float max_norm, float* factor_dev, float* norm_pinned);
-void k_begin_pass(const Tensor& clear, const int* pinned, int* to, int64_t n);  // clear = 0 (fp32), to[i] = pinned[i]
+// the same asked for with the optimiser step; factor: room for it
+struct Clip {
+    const double* part_dev = nullptr;  // null: no clip
+    int n = 0;
+    float max_norm = 0.0f;
+    float* factor = nullptr;
+    float* norm_pinned = nullptr;
+};
+// clear = 0 (fp32), to[i] = pinned[i]; for a batch of few tokens with y = table[pinned[0 .. y.rows - 1]] in the same launch: true if so
+bool k_begin_pass(const Tensor& clear, const int* pinned, int* to, int64_t n, const Tensor& table, const Tensor& y);
 void k_word_to_pinned(const void* src, void* pinned);  // one float for the host, cheaper than a copy
 // clip_dev (may be null): g is scaled in place by *clip_dev first, in the same pass
 void k_adamw(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, float lr, float b1, float b2,
@@ -84,7 +95,7 @@ struct AdamWPart {
     int64_t col_off;
 };
 bool k_adamw_parts(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, const std::vector<AdamWPart>& parts, float lr,
-                   float b1, float b2, float eps, float wd, float c1, float c2, const float* clip_dev);
+                   float b1, float b2, float eps, float wd, float c1, float c2, const Clip& clip);
 
 // C[M,N] (+)= op(A) . op(B), row-major, bf16 or fp32 operands, fp32 accumulate
 // (device::gemm, src/device.cpp:91-125). C may be a column slice of a wider

@@ -109,6 +109,31 @@ def test_optimiser_step_writes_the_copies(vocab, d, ff, layers, dtype):
     fresh.close()
 
 
+@pytest.mark.parametrize("dtype,tol", [("fp32", 1e-5), ("bf16", 1e-2)])
+@pytest.mark.parametrize("vocab", [512, 4000])
+def test_first_and_last_launch_of_a_pass(vocab, dtype, tol):
+    """2048 tokens of 256 columns are gathered in the launch that begins a pass, 2064 are not; 0.4 M parameters form the clip's factor in
+    the optimiser's workgroups, 1.3 M in a launch before. A batch is the mean of its parts (another order of sums; in bf16 dlogits
+    rounded at another scale, 2^-9 of each), the norm that of the gradients read back."""
+    m = Llama(vocab=vocab, d=256, n_layers=1, n_heads=4, d_ff=64, compute_dtype=dtype, seed=5)
+    toks = synth.randint(11, 2065, vocab)
+    parts = [(0, 2048), (2048, 2064)]
+    loss, grads = 0.0, None
+    for lo, hi in parts:
+        w = (hi - lo) / 2064
+        one = m.loss_backward(toks[lo:hi], toks[lo + 1:hi + 1], 16)[0]
+        loss, g = loss + w * one, m.grads()
+        grads = {k: w * g[k].astype(np.float64) + (grads[k] if grads else 0.0) for k in g}
+    whole = m.loss_backward(toks[:2064], toks[1:2065], 16)[0]
+    assert abs(whole - loss) < 1e-5 * loss
+    g = m.grads()
+    assert rel(g, grads) < tol
+    norm = m.adamw_step(1e-3, max_norm=1e-3)
+    assert abs(norm - np.sqrt(sum((x.astype(np.float64) ** 2).sum() for x in g.values()))) < 1e-6 * norm
+    assert rel({k: x * (norm / 1e-3) for k, x in m.grads().items()}, g) < 1e-6  # scaled where they lie
+    m.close()
+
+
 def exact_attention(q, k, v, d_o, scale, causal, window, sinks, given_o=None):
     """O, LSE, dQ, dK, dV in float64 (src/ops.cpp:863-1027) of [B,T,H,dk] tensors, K / V heads shared by groups. given_o: the O
     whose rowsum(dO .* O) the gradients are formed with, as a backward is given it; the exact O otherwise."""
