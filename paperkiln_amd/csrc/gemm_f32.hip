@@ -88,6 +88,8 @@ template <bool TA, bool TB, int MB, int NB, int KW, int SUMS, int MAX, End END>
 __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta) {
     constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB;
     constexpr int HALF = END == End::GATE ? NB / 2 : NB, TN = 16 * HALF;  // blocks of columns of C
+    constexpr int ITEMS = (MB * HALF + KW - 1) / KW;                      // blocks that a wavefront adds up and stores
+    constexpr bool EARLY = END != End::GATE && ITEMS == 1;
     // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
     const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (t >= tiles) return;
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
     if constexpr (MAX > 1)
         while (t >= jobs.first[j + 1]) ++j;
     const int M = jobs.job[j].M, N = jobs.job[j].N, K = jobs.job[j].K;
-    const int tn = (N + TN - 1) / TN, m0 = ((t - jobs.first[j]) / tn) * TM, n0 = ((t - jobs.first[j]) % tn) * TN;
+    const int tn = (N + TN - 1) / TN, at_row = quotient(t - jobs.first[j], tn), m0 = at_row * TM, n0 = (t - jobs.first[j] - at_row * tn) * TN;
     const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, grp = lane >> 4;
     const float* const a = jobs.job[j].a;
     const float* const b = jobs.job[j].b;
@@ -157,6 +159,31 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 #pragma unroll
     for (int u = 0; u < BUFS; ++u)
         if (u < mine) load(kw + u * KW, u);
+    // what the tile meets on its way out is asked for behind the first chunks, not when the contraction is over: a trip to memory of the 4 to 6 us
+    // of a small product (with a residual, us: 512 x 128 x 128 and 344 4.5 -> 4.0, 1024 x 256 x 256 and 688 6.9 -> 6.0; gate and up, 512 x 344 x 128 6.3 ->
+    // 5.2). Tiles of several blocks to a wavefront ask block by block, but for whole blocks (gate and up, 1024 x 688 x 256 17.3 -> 14.6; 392 tiles of weight
+    // gradients 27.0 -> 25.3): held over the loop those blocks cost it registers (28.0).
+    const float* const add = jobs.job[j].addend ? jobs.job[j].addend : beta != 0.0f ? jobs.job[j].c : nullptr;
+    const int64_t ldc = jobs.job[j].ldc;
+    f32x4 met[EARLY ? ITEMS : 1][END == End::GATE_GRAD ? 2 : 1];
+    auto meet = [&](int x, int y, f32x4 (&v)[END == End::GATE_GRAD ? 2 : 1]) {
+        const int n = min(n0 + y * 16 + l16, N - 1);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t o = min(m0 + x * 16 + 4 * grp + r, M - 1) * ldc + n;
+            if constexpr (END == End::GATE_GRAD)
+                v[0][r] = jobs.job[j].gu[o], v[1][r] = jobs.job[j].gu[o + N];
+            else
+                v[0][r] = add[o];
+        }
+    };
+    if constexpr (EARLY)
+        if (END == End::GATE_GRAD || add)
+#pragma unroll
+            for (int q = 0; q < ITEMS; ++q) {
+                const int g = min(q * KW + kw, MB * HALF - 1);
+                meet(g / HALF, g % HALF, met[q]);
+            }
     __builtin_amdgcn_sched_barrier(0);
     int i = 0;
     for (; i + BUFS <= mine; i += BUFS) {
@@ -171,10 +198,8 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
     for (int u = 0; u < BUFS - 1; ++u)
         if (i + u < mine) multiply(u);
 
-    const float* const add = jobs.job[j].addend ? jobs.job[j].addend : beta != 0.0f ? jobs.job[j].c : nullptr;
     float* const out = jobs.job[j].c;
-    const int64_t ldc = jobs.job[j].ldc;
-    auto store = [&](int x, int y, f32x4 v) {
+    auto store = [&](int x, int y, f32x4 v, const f32x4 (&e)[END == End::GATE_GRAD ? 2 : 1]) {
         const int n = n0 + y * 16 + l16;
         if (n >= N) return;
 #pragma unroll
@@ -183,9 +208,9 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
             if (m < M) {
                 const int64_t o = m * ldc + n;
                 if constexpr (END == End::GATE_GRAD)
-                    gated_grad(jobs.job[j].gu[o], jobs.job[j].gu[o + N], v[r], out[o], out[o + N]);
+                    gated_grad(e[0][r], e[1][r], v[r], out[o], out[o + N]);
                 else
-                    out[o] = add ? add[o] + v[r] : v[r];
+                    out[o] = add ? e[0][r] + v[r] : v[r];
             }
         }
     };
@@ -225,7 +250,9 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
                 for (int k = 1; k < KW; ++k) up += part[k][at + HALF][lane];
                 store_gated(g / HALF, g % HALF, s, up);
             } else {
-                store(g / HALF, g % HALF, s);
+                if constexpr (!EARLY)
+                    if (END == End::GATE_GRAD || add) meet(g / HALF, g % HALF, met[0]);
+                store(g / HALF, g % HALF, s, met[EARLY ? g0 / KW : 0]);
             }
         }
     }

@@ -82,7 +82,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
     if constexpr (MAX > 1)
         while (t >= jobs.first[j + 1]) ++j;
     const int M = jobs.job[j].M, N = jobs.job[j].N, K = jobs.job[j].K, lda = jobs.job[j].lda, ldb = jobs.job[j].ldb;
-    const int tn = (N + 31) / 32, m0 = ((t - jobs.first[j]) / tn) * 32, n0 = ((t - jobs.first[j]) % tn) * 32;
+    const int tn = (N + 31) / 32, at_row = quotient(t - jobs.first[j], tn), m0 = at_row * 32, n0 = (t - jobs.first[j] - at_row * tn) * 32;
     const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, grp = lane >> 4;
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(jobs.job[j].a), 0,
                                                       static_cast<int>(extent(TA ? K : M, TA ? M : K, lda)), 0x00020000);
@@ -137,6 +137,23 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
 #pragma unroll
     for (int u = 0; u < BUFS; ++u)
         if (u < mine) load(kw + u * KW, u);
+    // what the tile meets on its way out, asked for behind the first chunks as in gemm_f32.hip
+    constexpr int RPW = 8 / KW;  // of the 2 x 4 rows a lane holds, each wavefront adds up this many
+    const void* const add = jobs.job[j].addend ? jobs.job[j].addend : accumulate ? jobs.job[j].c : nullptr;
+    const int64_t ldc = jobs.job[j].ldc;
+    u32x2 met[RPW];
+    if (END == End::GATE_GRAD || (END == End::PLAIN && add))
+#pragma unroll
+        for (int q = 0; q < RPW; ++q) {
+            const int row = kw * RPW + q;
+            const int64_t o = min(m0 + 2 * (4 * grp + (row & 3)) + (row >> 2), M - 1) * ldc + min(n0 + 2 * l16, N - 2);
+            if (END == End::GATE_GRAD)
+                met[q] = u32x2{*reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o), *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o + N)};
+            else if (CF32)
+                met[q] = *reinterpret_cast<const u32x2*>(static_cast<const float*>(add) + o);
+            else
+                met[q] = u32x2{*reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(add) + o), 0};
+        }
     __builtin_amdgcn_sched_barrier(0);
     int i = 0;
     for (; i + BUFS <= mine; i += BUFS) {
@@ -160,10 +177,8 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
 #pragma unroll
             for (int y = 0; y < 2; ++y) part[kw][c][x][y][lane] = acc[c][x][y];
     __syncthreads();
-    constexpr int RPW = 8 / KW;  // of the 2 x 4 rows a lane holds, each wavefront adds up this many
     const int n = n0 + 2 * l16;
     if (n >= N) return;
-    const int64_t ldc = jobs.job[j].ldc;
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
         const int row = kw * RPW + q, x = row >> 2, r = row & 3;
@@ -191,8 +206,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
             continue;
         }
         if constexpr (END == End::GATE_GRAD) {
-            const uint32_t d = pack_bf16(s0, s1), gate = *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o),
-                           up = *reinterpret_cast<const uint32_t*>(jobs.job[j].gu + o + N);
+            const uint32_t d = pack_bf16(s0, s1), gate = met[q][0], up = met[q][1];
             float dg[2], du[2];
             gated_grad(lo(gate), lo(up), lo(d), dg[0], du[0]);
             gated_grad(hi(gate), hi(up), hi(d), dg[1], du[1]);
@@ -200,17 +214,13 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o + N) = pack_bf16(du[0], du[1]);
             continue;
         }
-        const void* const add = jobs.job[j].addend ? jobs.job[j].addend : accumulate ? jobs.job[j].c : nullptr;
         if (CF32) {
             f32x2 v = {s0, s1};
-            if (add) {
-                const f32x2 e = *reinterpret_cast<const f32x2*>(static_cast<const float*>(add) + o);
-                v[0] += e[0], v[1] += e[1];
-            }
+            if (add) v[0] += __uint_as_float(met[q][0]), v[1] += __uint_as_float(met[q][1]);
             *reinterpret_cast<f32x2*>(static_cast<float*>(jobs.job[j].c) + o) = v;
         } else {
             if (add) {
-                const uint32_t e = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(add) + o);
+                const uint32_t e = met[q][0];
                 s0 += __uint_as_float(e << 16), s1 += __uint_as_float(e & 0xffff0000u);
             }
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o) = pack_bf16(s0, s1);
