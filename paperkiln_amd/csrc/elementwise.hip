@@ -343,9 +343,22 @@ __global__ void ew_silu_mul_bwd(const T* gate, const T* up, const T* dy, T* dgat
     }
 }
 
+// x of another lane of the same sixteen, by the DPP control word
+template <int CTRL>
+__device__ inline float lane_moved(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
+// x of all lanes added up, halves first (lane ^ 32, 16, 8, 4, 2, 1): in registers, where six exchanges through the LDS unit are 0.3 us. All lanes
+// of the wavefront are active. From the third step on the sums repeat every 16, 8, ... lanes, so a rotation is an exchange.
 __device__ inline float wave_sum(float x) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o, 64);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    x += lane_moved<0x128>(x);  // rotated by 8
+    x += lane_moved<0x124>(x);  // by 4
+    x += lane_moved<0x4E>(x);   // lane ^ 2
+    x += lane_moved<0xB1>(x);   // lane ^ 1
     return x;
 }
 
@@ -365,6 +378,31 @@ __global__ void rms_fwd(const T* x, const float* w, float eps, T* y, float* rinv
     const float ri = 1.0f / sqrtf(ss + eps);
     if (lane == 0) rinv[row] = ri;
     for (int j = lane; j < C; j += 64) stf(y + row * C, j, ldf(xr, j) * ri * w[j]);
+}
+// The same to the same bits with the row and w held in registers, all of both on their way together (C <= 64 NP): the loop above makes
+// a trip to memory every 64 columns and reads the row twice. 1024 rows of 256 4.4 -> 3.2 us, 2100 of 512 6.8 -> 4.7.
+template <int NP>
+__global__ void rms_fwd_reg(const float* x, const float* w, float eps, float* y, float* rinv, int64_t R, int C) {
+    const int lane = threadIdx.x & 63;
+    const int64_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= R) return;
+    float v[NP], g[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int j = min(lane + 64 * p, C - 1);
+        v[p] = x[row * C + j];
+        g[p] = w[j];
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+        if (lane + 64 * p < C) ss = fmaf(v[p], v[p], ss);
+    ss = wave_sum(ss) / static_cast<float>(C);
+    const float ri = 1.0f / sqrtf(ss + eps);
+    if (lane == 0) rinv[row] = ri;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+        if (lane + 64 * p < C) y[row * C + lane + 64 * p] = v[p] * ri * g[p];
 }
 // dx = rinv * (dY*w - x * rinv^2 * sum_j(dY*w*x) / C)
 template <typename T>
@@ -588,6 +626,7 @@ __global__ void rms_bwd_dx_dw(const T* dy, const T* x, const float* rinv, const 
                     if (ADD) e[q][p].load(addend + rows[q] * C + j);
                 }
             }
+        const float inv[2] = {rinv[rows[0]], rinv[rows[1]]};
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -603,7 +642,7 @@ __global__ void rms_bwd_dx_dw(const T* dy, const T* x, const float* rinv, const 
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             if (q == 1 && !two) break;  // wavefront-uniform: an odd row count leaves the second row out
-            const float ri = rinv[rows[q]], kk = ri * ri * term[q] / static_cast<float>(C);
+            const float ri = inv[q], kk = ri * ri * term[q] / static_cast<float>(C);
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
                 const int j = (lane + p * 64) * E;
@@ -1406,6 +1445,23 @@ void k_rmsnorm_fwd(const Tensor& x, const Tensor& w, float eps, const Tensor& y,
         else
             hipLaunchKernelGGL(rms_fwd8, dim3((x.rows + 3) / 4), dim3(NT), 0, tape_stream(), static_cast<const uint16_t*>(x.ptr()),
                                static_cast<const float*>(w.ptr()), eps, static_cast<uint16_t*>(y.ptr()), rinv, x.rows, C);
+        post();
+        return;
+    }
+    if (x.dtype == PK_F32 && x.cols <= 1024) {
+        auto launch = [&](auto np) {
+            hipLaunchKernelGGL((rms_fwd_reg<decltype(np)::value>), dim3((x.rows + 3) / 4), dim3(256), 0, tape_stream(),
+                               static_cast<const float*>(x.ptr()), static_cast<const float*>(w.ptr()), eps, static_cast<float*>(y.ptr()), rinv,
+                               x.rows, static_cast<int>(x.cols));
+        };
+        if (x.cols <= 128)
+            launch(std::integral_constant<int, 2>{});
+        else if (x.cols <= 256)
+            launch(std::integral_constant<int, 4>{});
+        else if (x.cols <= 512)
+            launch(std::integral_constant<int, 8>{});
+        else
+            launch(std::integral_constant<int, 16>{});
         post();
         return;
     }
