@@ -152,6 +152,7 @@ constexpr bool BOTH_AHEAD = D <= 64;
 // head_dim 24, T 402 x 22, 16 heads: 204 -> 173 us; head_dim 64, T 731 x 4, 28 heads on 4, window 309: 296 -> 242).
 template <int D, int KW>
 __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_fwd(AttnArgs a) {
+    all_arguments(a);
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P, RED = KW * (DB * 1024 + 128);
     __shared__ __attribute__((aligned(16))) float lds[KW * TILE > RED ? KW * TILE : RED];
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -329,6 +330,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
 }
 template <int D, int KW>
 __global__ __launch_bounds__(64 * KW, D <= 32 ? 4 : D <= 64 ? 2 : 1) void f32_split_dq(AttnArgs a, int fuse_delta) {
+    all_arguments(a);
     __shared__ __attribute__((aligned(16))) float lds[dq_lds<D, KW>()];
     dq_block<D, KW, false>(a, fuse_delta, static_cast<int>(blockIdx.x), lds);
 }
@@ -511,6 +513,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
 }
 template <int D, int KW>
 __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) void f32_split_dkdv(AttnArgs a) {
+    all_arguments(a);
     __shared__ __attribute__((aligned(16))) float lds[dkdv_lds<D, KW>()];
     dkdv_block<D, KW, false>(a, static_cast<int>(blockIdx.x), lds);
 }
@@ -520,6 +523,7 @@ __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) 
 // most CUs idle. Here blocks 0 .. dkdv_ids - 1 are the dK/dV launch's, which forms its own delta, and the others the dQ launch's.
 template <int D>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_split_bwd(AttnArgs a, int dkdv_ids) {
+    all_arguments(a);
     constexpr int Q = dq_lds<D, 4>(), K = dkdv_lds<D, 4>();
     __shared__ __attribute__((aligned(16))) float lds[Q > K ? Q : K];
     const int id = static_cast<int>(blockIdx.x);

@@ -424,6 +424,7 @@ constexpr int BUFS = KW == 1 && (D < 128 || QW > 4) ? 2 : 1;
 // ---- forward: QW groups of 32 queries x KW groups of 32-key tiles ----
 template <int D, int QW, int KW>
 __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
+    if (KW > 1) all_arguments(a);
     constexpr int BM = 32 * QW, DB = D / 32, G = 64 * QW, NBUF = BUFS<D, QW, KW>;
     constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
     constexpr int RED = KW > 1 ? QW * KW * (DB * 1024 + 128) * 2 : 0;  // in uint16
@@ -659,6 +660,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
 }
 template <int D, int QW, int KW>
 __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs a, int fuse_delta) {
+    all_arguments(a);
     __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW>()];
     int b, h, hk, qblk;
     if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW>(a, fuse_delta, b, h, hk, qblk, lds);
@@ -845,6 +847,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 }
 template <int D, int QW>
 __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
+    all_arguments(a);
     __shared__ __attribute__((aligned(16))) uint16_t lds[2 * DKDV_TILE<D, QW>];
     __shared__ __attribute__((aligned(16))) float pbuf[QW * 1024];
     const int nblk = (a.T + 32 * QW - 1) / (32 * QW) + (a.tail ? sink_tail(a.T, a.window, a.sinks).nch : 0);
@@ -858,6 +861,7 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
 // ---- dK, dV and dQ in one launch, delta read (f32x3_takes_bwd) ----
 template <int D>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
+    all_arguments(a);
     constexpr int Q = dq_lds<D, 2, 2>(), K = 2 * DKDV_TILE<D, 2>, N = Q > K + 4096 ? Q : K + 4096;
     __shared__ __attribute__((aligned(16))) uint16_t lds[N];
     const JoinedBlocks jb(a, 64);
@@ -873,6 +877,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
 // columns of dQ^T += K^T dS. The next tile is moved as in x3_dkdv (T 4403, 8 heads, head_dim 128, us: 456 -> 436).
 template <int D>
 __global__ __launch_bounds__(512, 2) void x3_dq_wide(AttnArgs a, int fuse_delta) {
+    all_arguments(a);
     constexpr int QW = 4, BM = 32 * QW, DB = D / 32, G = 64 * QW, HB = (DB + 1) / 2;
     constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
     __shared__ __attribute__((aligned(16))) uint16_t lds[2 * TILE];

@@ -186,6 +186,7 @@ __device__ inline void accumulate_tr(const uint16_t* tile, int pitch, int row0, 
 // ---- forward: QW groups of 32 queries x KW groups of key tiles of 32 NB keys ----
 template <int D, int QW, int KW, int NB, bool EXACT>
 __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
+    if (KW > 1 || !EXACT) all_arguments(a);
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW;
     constexpr int KS = D + 8;                              // row reads conflict-free
     constexpr int VS = (D / 32) % 2 ? D : D + 32;          // 4-row transposing reads conflict-free
@@ -451,6 +452,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
 }
 template <int D, int QW, int KW, int NB, bool EXACT>
 __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
+    all_arguments(a);
     __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW, NB>()];
     int b, h, hk, qblk;
     if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW, NB, EXACT>(a, fuse_delta, b, h, hk, qblk, lds);
@@ -674,6 +676,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 }
 template <int D, int QW, int KW, int NB, bool EXACT, int OCC>
 __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
+    all_arguments(a);
     __shared__ __attribute__((aligned(16))) uint16_t lds[dkdv_lds<D, QW, KW, NB>()];
     int blk, rr, kvu;
     if (map_key_block(a, 32 * QW, blk, rr, kvu)) dkdv_block<D, QW, KW, NB, EXACT, false>(a, blk, rr, kvu, lds);
@@ -683,6 +686,7 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
 // Blocks 0 .. dkdv_ids - 1 are the dK/dV launch's, which forms its own delta, and the others the dQ launch's.
 template <int D, bool EXACT>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, int dkdv_ids) {
+    all_arguments(a);
     constexpr int Q = dq_lds<D, 1, 4, 1>(), K = dkdv_lds<D, 1, 4, 1>();
     __shared__ __attribute__((aligned(16))) uint16_t lds[Q > K ? Q : K];
     const int id = static_cast<int>(blockIdx.x);
@@ -699,6 +703,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, in
 // lanes; above, it is read): a launch of delta before this one cost 4 us more, of 13 to 60.
 template <int D, bool EXACT>
 __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
+    all_arguments(a);
     constexpr bool OWN_DELTA = D <= 64;
     constexpr int Q = dq_lds<D, 4, 1, 2>(), K = dkdv_lds<D, 4, 1, 2>();
     __shared__ __attribute__((aligned(16))) uint16_t lds[Q > K ? Q : K];
