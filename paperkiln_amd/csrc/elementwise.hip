@@ -1084,7 +1084,7 @@ __global__ void sum_f32_k(const float* x, int64_t n, double* out) {
 }
 // mean of n floats, accumulated in double and rounded to float once: what the host does with
 // k_sum_f32_to_host's result, without the round trip
-__global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, float* out, int with_one, float* pinned) {
+__global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, float* out, float* one, float* pinned) {
     // thread t takes the elements sum_f32_k's thread t % NT takes, a quarter of them: the NT partial sums are formed
     // from four pieces each and then added in sum_f32_k's tree
     __shared__ double sh[1024];
@@ -1101,8 +1101,8 @@ __global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, fl
     }
     if (threadIdx.x == 0) {
         const float mean = static_cast<float>(sh[0] / static_cast<double>(n));
-        out[0] = mean;
-        if (with_one) out[1] = 1.0f;
+        *out = mean;
+        if (one) *one = 1.0f;
         if (pinned) *pinned = mean;
     }
 }
@@ -1685,9 +1685,10 @@ bool k_ce_rows_once(const Tensor& logits, const int* targets, float gscale, floa
     post();
     return true;
 }
-void k_mean_f32(const float* x, int64_t n, const Tensor& out, float* pinned) {
-    if (out.dtype != PK_F32 || out.rows != 1 || out.cols < 1 || out.cols > 2) throw std::runtime_error("mean: the result is one float, or it and a 1");
-    hipLaunchKernelGGL(mean_f32_k, dim3(1), dim3(1024), 0, tape_stream(), x, n, static_cast<float*>(out.ptr()), out.cols == 2 ? 1 : 0, pinned);
+void k_mean_f32(const float* x, int64_t n, const Tensor& out, const Tensor* one, float* pinned) {
+    if (out.dtype != PK_F32 || out.rows * out.cols != 1) throw std::runtime_error("mean: the result is one float");
+    hipLaunchKernelGGL(mean_f32_k, dim3(1), dim3(1024), 0, tape_stream(), x, n, static_cast<float*>(out.ptr()),
+                       one ? static_cast<float*>(one->ptr()) : nullptr, pinned);
     post();
 }
 double k_sum_f32_to_host(const float* x, int64_t n) {

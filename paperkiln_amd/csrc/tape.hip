@@ -1071,11 +1071,8 @@ Var linear_cross_entropy_to(const Var& h, const Var& E, const std::shared_ptr<Bu
         dl.cols = V;
         if (want_dE) gemm(dl, true, hview, false, dE1.ptr(), PK_F32, V, d, d, r0 == 0 && !dE_in_place ? 0.0f : 1.0f, dl_ld);
     }
-    Tensor out = Tensor::make(1, 2, PK_F32);
-    k_mean_f32(static_cast<const float*>(nll.p), N, out, pinned);  // the loss stays on the device: no wait in mid-step
-    out.cols = 1;
-    Tensor one = out;
-    one.off_bytes += sizeof(float);
+    Tensor out = Tensor::make(1, 1, PK_F32), one = Tensor::make(1, 1, PK_F32);  // one: backward() hands it over whole
+    k_mean_f32(static_cast<const float*>(nll.p), N, out, &one, pinned);  // the loss stays on the device: no wait in mid-step
     if (dE_in_place) dE1 = Tensor();
     Var loss = record(std::move(out), {h, E}, [dh1, dE1, dE_in_place](Variable* self) mutable {
         const Var& h = self->parents[0];
