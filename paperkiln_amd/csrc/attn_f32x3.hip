@@ -1113,12 +1113,15 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 //                8 heads (592) 421 | 499
 //   bands, every head its own: 48, T 165 x 6, 8 heads, window 86 (144) 36 | 20;   T 4383, 8 heads, 26 (552) 51 | 42;   T 975 x 13, 2 heads of 64, 408,
 //     1 sink (416) 109 | 79;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
+//     whose sink keys' block is walked for up to 600 queries more while there are blocks enough beside it: 64, T 419 x 6, 8 heads, 40, 1 sink (336) 51 | 38;
+//     T 426 x 14, 4 heads, 36, 4 (392) 76 | 39;  48, T 1140 x 11, 2 heads, 556 (396) 119 | 83;  96, T 707 x 10, 2 heads, 321, 1 (240) 102 | 76;  not: 64,
+//     T 962, 8 heads, 331, 16 (128) 58 | 66;  T 934, 12 heads of 48, 396, 1 (180) 64.7 | 65.3; over 36 random shapes 0.83 of the time
 //     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
 bool f32x3_takes_bwd(const AttnArgs& a) {
     if (!f32_split_serves(a) || a.T <= 32) return false;
     const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
     if (a.window > 0)
-        return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= (a.dk_dim > 96 ? 600 : 300)) &&
+        return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= (a.dk_dim > 64 || q >= 200 ? 600 : 300)) &&
                q >= (a.dk_dim <= 32 ? 130 : a.dk_dim <= 64 ? 100 : a.dk_dim <= 96 ? 88 : 40) && q <= (a.dk_dim <= 64 ? 800 : 420);
     if (a.dk_dim > 96) return q >= 40 && q <= (a.causal ? 420 : a.T <= 130 ? 200 : 260);
     if (a.dk_dim > 64) return q >= (a.causal && a.T > 300 && a.T <= 2600 ? 170 : 88) && q <= (a.causal ? 330 : 300);

@@ -397,7 +397,7 @@ def test_backward_in_one_launch(case, dtype, dk):
 @pytest.mark.parametrize("dk", [4, 32, 44, 64, 80, 96, 100, 128])
 @pytest.mark.parametrize("case", [(18, 33, 16, 16, True, 0, 0), (7, 65, 16, 8, True, 0, 0), (9, 129, 14, 2, True, 0, 0), (2, 641, 13, 13, True, 0, 0),
                                   (5, 577, 8, 8, False, 0, 0), (1, 2113, 8, 2, True, 0, 0), (40, 257, 3, 3, True, 0, 0), (6, 321, 9, 9, True, 33, 17),
-                                  (1, 1100, 11, 11, True, 100, 0)], ids=str)
+                                  (1, 1100, 11, 11, True, 100, 0), (8, 471, 6, 6, True, 91, 4)], ids=str)
 def test_fp32_backward_of_joined_blocks(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     gen = torch.Generator(device="cuda").manual_seed(T + dk)
