@@ -1115,7 +1115,7 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 //     1 sink (416) 109 | 79;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
 //     whose sink keys' block is walked for up to 600 queries more while there are blocks enough beside it: 64, T 419 x 6, 8 heads, 40, 1 sink (336) 51 | 38;
 //     T 426 x 14, 4 heads, 36, 4 (392) 76 | 39;  48, T 1140 x 11, 2 heads, 556 (396) 119 | 83;  96, T 707 x 10, 2 heads, 321, 1 (240) 102 | 76;  not: 64,
-//     T 962, 8 heads, 331, 16 (128) 58 | 66;  T 934, 12 heads of 48, 396, 1 (180) 64.7 | 65.3; over 36 random shapes 0.83 of the time
+//     T 962, 8 heads, 331, 16 (128) 58 | 66;  T 934, 12 heads of 48, 396, 1 (180) 64.7 | 65.3; over 36 random shapes 0.86 of the time
 //     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
 bool f32x3_takes_bwd(const AttnArgs& a) {
     if (!f32_split_serves(a) || a.T <= 32) return false;
