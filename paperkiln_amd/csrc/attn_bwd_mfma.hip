@@ -153,12 +153,15 @@ int launch_row_delta(const AttnArgs& a, bool bf16, hipStream_t st) {
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
+Bwd bwd_of_bf16(const AttnArgs& a) {
+    if (joined_takes_bwd(a)) return Bwd::JOINED;
+    return split_takes_joined(a) ? Bwd::SPLIT_JOINED : split_takes_bwd(a) ? Bwd::SPLIT : Bwd::APART;
+}
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     // delta and dQ asked for together: dQ forms delta itself and runs first, dK/dV reads what it wrote
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
-    if (stages == PK_BWD_ALL && !a.in_place && joined_takes_bwd(a)) return launch_joined_bwd(a, st);
-    if (stages == PK_BWD_ALL && !a.in_place && split_takes_joined(a)) return launch_split_joined(a, st);
-    if (stages == PK_BWD_ALL && !a.in_place && split_takes_bwd(a)) return launch_split_bwd(a, st);
+    const Bwd form = stages == PK_BWD_ALL && !a.in_place ? bwd_of_bf16(a) : Bwd::APART;
+    if (form != Bwd::APART) return form == Bwd::JOINED ? launch_joined_bwd(a, st) : form == Bwd::SPLIT ? launch_split_bwd(a, st) : launch_split_joined(a, st);
     int rc = PK_OK;
     if (fused)
         rc = run_dq(a, true, st);

@@ -687,11 +687,15 @@ int launch_f32_mfma_fwd(const AttnArgs& a, hipStream_t st) {
 
 bool f32_deals_heads(const AttnArgs& a) { return a.head_split > 1 && f32_split_takes_dkdv(a); }
 
+Bwd bwd_of_f32(const AttnArgs& a) {
+    if (f32x3_takes_bwd(a)) return f32x3_bwd_keeps_all(a) ? Bwd::F32_PARTS_ALL : Bwd::F32_PARTS;
+    return f32_split_takes_bwd(a) ? Bwd::F32_SPLIT : Bwd::APART;
+}
 int launch_f32_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st) {
     const bool fused = (stages & PK_BWD_DELTA) && (stages & PK_BWD_DQ);
     int rc = PK_OK;
-    if (stages == PK_BWD_ALL && !a.in_place && f32x3_takes_bwd(a)) return launch_f32x3_bwd(a, st);
-    if (stages == PK_BWD_ALL && !a.in_place && f32_split_takes_bwd(a)) return launch_f32_split_bwd(a, st);
+    const Bwd form = stages == PK_BWD_ALL && !a.in_place ? bwd_of_f32(a) : Bwd::APART;
+    if (form != Bwd::APART) return form == Bwd::F32_SPLIT ? launch_f32_split_bwd(a, st) : launch_f32x3_bwd(a, st);
     if (fused)  // dQ forms delta itself and runs first; dK/dV reads what it wrote
         rc = run_dq(a, true, st);
     else if (stages & PK_BWD_DELTA)

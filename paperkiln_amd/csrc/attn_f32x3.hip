@@ -6,8 +6,8 @@
 // left out; the other six are exact in fp32 and are added in fp32 by the matrix unit, small ones first. Error of scores against
 // float64, of the result's norm (in brackets v_mfma_f32_32x32x2_f32, which rounds its sum every second column): 1 column
 // 3.5e-8 (4.0e-8), 4 3.2e-8 (4.9e-8), 16 3.4e-8 (8.2e-8), 64 4.6e-8 (1.4e-7). A single product is off by 1.44e-7 at most, where
-// both factors are just above a power of two, and by 1.3e-7 elsewhere and on the fp32 instruction. Parts below 2^-126 are lost:
-// rows_to_redo.
+// both factors are just above a power of two, and by 1.3e-7 elsewhere and on the fp32 instruction. Parts below 2^-133, the smallest bf16,
+// are lost, and with them bits of values below 2^-109: rows_to_redo, UP.
 //
 // What bounds it: the fp32 instruction does 157 TFLOP/s, and the kernels on it (attn_f32_split.hip) stood at 105 to 130; six
 // bf16 products for one take 3/8 of its clocks. Beside them stands the splitting, 5.5 vector instructions an element: a tile
@@ -22,6 +22,19 @@ namespace {
 
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LAZY_T = 6.0f;  // as in attn_split.hip: the running maximum moves when it is outgrown by 2^6
+
+// Bits of values below 2^-109 do not count beside ordinary ones, but they show in a column that is all as small and where a large partner
+// makes the product ordinary (a column of K at 2^-120 under one of Q at 2^120: dQ off by 3.6e-5). Launches that hold what the fp32
+// instruction does (ALL: f32x3_takes_bwd) split everything at 2^24 times its size, at which the last bit of the smallest fp32 value is a part that
+// is kept. Powers of two change no other bit and leave with factors that are there anyway: scores (2^48) with the exponent's, dP with the
+// subtraction of delta, gradients (2^48) when they are stored. What leaves fp32 at that size (values from 2^104 on, products and gradients from
+// 2^80) ends in results that are not finite. A multiplication an element moved and one for each of P: T 313 x 4, 16 heads of 64, backward
+// 35.1 -> 36.4 us (71 on the fp32 instruction); T 2132, 8 heads of 128 278 -> 291 (394); T 241 x 10, 4 heads of 96 33.0 -> 34.1 (52); T 1037 x
+// 2, 8 heads of 32 49.7 -> 51.4 (62).
+template <bool ALL>
+constexpr float UP = ALL ? 0x1p24f : 1.0f;
+template <bool ALL>
+constexpr float DOWN = 1.0f / UP<ALL>;
 
 // A product that is not fused into the sum it enters.
 __device__ inline float mul_rounded(float x, float y) {
@@ -79,7 +92,7 @@ __device__ inline void store_block32(void* base, int64_t row_off, int db, int g,
 
 // A 32-row tile of a [T, dk] fp32 matrix, moved by G threads (rows past T and chunks past dk read as zero) into three
 // planes of 32 rows of pitch D + 8: 16-byte row reads then touch all banks once.
-template <int D, int G>
+template <int D, int G, bool ALL = false>
 struct Mover3 {
     static constexpr int NCH = D / 4, CPT = 32 * NCH / G, P = D + 8, PLANE = 32 * P;
     static_assert(CPT >= 1 && 32 * NCH % G == 0, "every thread moves the same number of chunks");
@@ -105,8 +118,8 @@ struct Mover3 {
         for (int i = 0; i < CPT; ++i) {
             const f32x4 x = *reinterpret_cast<const f32x4*>(&r[i]);
             uint32_t h[2], m[2], l[2];
-            split2(x[0], x[1], h[0], m[0], l[0]);
-            split2(x[2], x[3], h[1], m[1], l[1]);
+            split2(x[0] * UP<ALL>, x[1] * UP<ALL>, h[0], m[0], l[0]);
+            split2(x[2] * UP<ALL>, x[3] * UP<ALL>, h[1], m[1], l[1]);
             uint16_t* p = at(tile, t, i);
             *reinterpret_cast<u32x2*>(p) = u32x2{h[0], h[1]};
             *reinterpret_cast<u32x2*>(p + PLANE) = u32x2{m[0], m[1]};
@@ -149,12 +162,13 @@ struct Row {
         }
     }
     // as three operands: chunk kk holds columns 16 kk + 8 g .. +7
+    template <bool ALL = false>
     __device__ void split(bf16x8 (&out)[3][D / 16]) const {
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) {
             float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = x[2 * kk + e / 4][e % 4];
+            for (int e = 0; e < 8; ++e) v[e] = x[2 * kk + e / 4][e % 4] * UP<ALL>;
             split8(v, out[0][kk], out[1][kk], out[2][kk]);
         }
     }
@@ -253,8 +267,9 @@ __device__ inline float log_sum(float m, float scale, float off, float l) {
 // 1.000, dQ 1.005, dK/dV 1.013 of the time without it. Rows that are NaN end at the first 64 scores with one (T 4096 x 4, 16 heads, 64
 // columns, forward 0.8 ms: 1.1 where all is NaN, 7.5 with one key that is), rows beside an infinity are walked to the end (45 to 56 ms).
 //
-// The last parts of values below 1e-33 are below the range of bf16. Beside others they do not count, and where everything is that
-// small the results are: rows of a wavefront whose results are all below 2^-96, and not all zero, are formed again as well.
+// The last parts of values below 2^-109 are below the range of bf16. Beside others they do not count, and where everything is that
+// small the results are: rows of a wavefront whose results are all below 2^-96, and not all zero, are formed again as well (not where ALL
+// of fp32's range is split without loss).
 
 // The kernel's arguments (AttnArgs is the first of them), read from memory where this is called: as the ones that the kernel has read
 // they would be held in scalar registers through its loop, which spilled 50 of them in dK/dV.
@@ -267,7 +282,7 @@ __device__ inline AttnArgs arguments_again() {
 __device__ inline int lane_again() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 // Bit r: row r (a lane of either half each) is one of those. ok: the lane's row exists and is stored; NB blocks, of which this
 // wavefront has every `step`-th from `first` on; sc: the factor they are stored with, or a power of two or so from it.
-template <int NB>
+template <int NB, bool ALL = false>
 __device__ inline uint32_t rows_to_redo(const f32x16* acc, float sc, bool ok, int first = 0, int step = 1) {
     float z[4] = {0.0f, 0.0f, 0.0f, 0.0f}, top[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // z stays 0 under finite values
 #pragma unroll
@@ -277,7 +292,7 @@ __device__ inline uint32_t rows_to_redo(const f32x16* acc, float sc, bool ok, in
             for (int r = 0; r < 16; ++r) z[r & 3] = fmaf(acc[n][r], 0.0f, z[r & 3]), top[r & 3] = fmaxf(top[r & 3], fabsf(acc[n][r]));
     const float t = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
     uint64_t lanes = __ballot(ok && !((z[0] + z[1]) + (z[2] + z[3]) == 0.0f));
-    if (__ballot(ok && t * sc >= 0x1p-96f) == 0) lanes |= __ballot(ok && t > 0.0f);
+    if (!ALL && __ballot(ok && t * sc >= 0x1p-96f) == 0) lanes |= __ballot(ok && t > 0.0f);
     return static_cast<uint32_t>(lanes | lanes >> 32);
 }
 __device__ inline float dot_exact(const float* x, const float* y, int dk) {
@@ -563,7 +578,7 @@ constexpr int dq_lds() {  // in uint16
     constexpr int TILES = BUFS<D, QW, KW> * KW * 6 * Mover3<D, 64 * QW>::PLANE, RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
     return TILES > RED ? TILES : RED;
 }
-template <int D, int QW, int KW, int N>
+template <int D, int QW, int KW, bool ALL, int N>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h, int hk, int qblk, uint16_t (&lds)[N]) {
     constexpr int BM = 32 * QW, DB = D / 32, G = 64 * QW, NBUF = BUFS<D, QW, KW>;
     constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
@@ -576,9 +591,9 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk),
                 *const qh = head_of<float>(a.q, a.q_sb, b, a.q_sh, h);
     const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
-    const float cexp = a.scale * LOG2E;
+    const float cexp = a.scale * LOG2E * (DOWN<ALL> * DOWN<ALL>);
 
-    Mover3<D, G> mk, mv;
+    Mover3<D, G, ALL> mk, mv;
     mk.init(gt, k_st, dk);
     mv.init(gt, v_st, dk);
     const KeyTiles kt(a, q0, BM, 32);
@@ -611,10 +626,10 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
         } else {
             dl = a.delta[lrow];
         }
-        q.split(qreg);
-        d_o.split(greg);
+        q.template split<ALL>(qreg);
+        d_o.template split<ALL>(greg);
     }
-    const float nlse = -lse * LOG2E;
+    const float nlse = -lse * LOG2E, dl_up = dl * UP<ALL>;
     const QueryVis vis(qi, a.T, a.causal, a.window, a.sinks);
     f32x16 acc[DB];
 #pragma unroll
@@ -633,7 +648,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
             f32x16 s = dot3<D>(Ks, qreg, c32, g);
             const f32x16 dp = dot3<D>(Ks + 3 * PLANE, greg, c32, g);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * (dp[r] - dl);
+            for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cexp, nlse)) * fmaf(dp[r], DOWN<ALL>, -dl_up);
             const MaskKind kind = mask_kind(k0, k0 + 31, qlo, qhi, a.T, a.causal, a.window, a.sinks);
             if (kind != MaskKind::NONE) mask_block(s, kind, vis, k0 + g * 4, 0.0f);
             accumulate3<D>(Ks, Parts(s), acc, lane);
@@ -644,18 +659,21 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     }
     const int le = lane_again(), ge = le >> 5, qe = qlo + (le & 31);
     join_groups<DB, KW>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, le);
-    for (uint32_t again = rows_to_redo<DB>(acc, 1.0f, qe < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
+    float sc = a.scale * (DOWN<ALL> * DOWN<ALL>);
+    for (uint32_t again = rows_to_redo<DB, ALL>(acc, 1.0f, qe < a.T, kg, KW); __builtin_expect(again != 0, 0); again &= again - 1) {
         const int row = __builtin_ctz(again);
         double x[2];
-        exact_dq(arguments_again(), b, h, hk, qlo + row, __shfl(dl, row), le, x);
+        // (of ALL, delta is as it is only in memory)
+        exact_dq(arguments_again(), b, h, hk, qlo + row, ALL ? a.delta[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qlo + row] : __shfl(dl, row), le, x);
         put_row<D, DB>(row_room<D, QW * KW, RED>(lds, w), x, row, acc, le);
+        if (ALL && (le & 31) == row) sc = a.scale;
     }
     if (a.in_place) __syncthreads();  // every row has been read
     if (qe < a.T) {
         const int64_t ro = b * a.dq_sb + h * a.dq_sh + qe * a.dq_st;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
-            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, ge, acc[db], a.scale, dk);
+            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, ge, acc[db], sc, dk);
     }
 }
 template <int D, int QW, int KW>
@@ -663,7 +681,7 @@ __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs 
     all_arguments(a);
     __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW>()];
     int b, h, hk, qblk;
-    if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW>(a, fuse_delta, b, h, hk, qblk, lds);
+    if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW, false>(a, fuse_delta, b, h, hk, qblk, lds);
 }
 
 // The two products of a step that need no other go to two sets of wavefronts, as in the other dK/dV kernels: with both
@@ -693,7 +711,7 @@ __device__ inline f32x16 get_tile(const float* buf, int lane) {
 // 4096 x 4: 337 -> 323). At 128 columns there is one wavefront to a SIMD and both do it at the end of the first phase (1777; 1872).
 template <int D, int QW>
 constexpr int DKDV_TILE = 6 * Mover3<D, 64 * QW>::PLANE + 128;  // in uint16; LSE and delta of a tile's rows behind it
-template <int D, int QW, int N>
+template <int D, int QW, bool ALL, int N>
 __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, uint16_t (&lds)[N], float* pbuf) {
     constexpr int BNK = 32 * QW, DB = D / 32, G = 64 * QW;
     constexpr bool APART = D < 128;
@@ -710,7 +728,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     if (chunk >= 0 && rr > 0) return;
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv, h0 = chunk >= 0 ? 0 : quotient(rr * rep, hs), nh = chunk >= 0 ? rep : quotient((rr + 1) * rep, hs) - h0;
     const int k0 = chunk >= 0 ? 0 : blk * BNK, kw0 = k0 + qg * 32, kj = kw0 + c32;
-    const float cexp = a.scale * LOG2E;
+    const float cexp = a.scale * LOG2E * (DOWN<ALL> * DOWN<ALL>);
 
     // query tiles that can see keys [k0, k0 + BNK) (paperkiln src/ops.cpp:960-965 inverted)
     const int khi = min(k0 + BNK, a.T) - 1;
@@ -726,8 +744,8 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     const int s_st = static_cast<int>(role == 0 ? a.q_st : a.do_st);
     const float* const src = head_of<float>(role == 0 ? a.q : a.d_o, role == 0 ? a.q_sb : a.do_sb, b, s_sh, hk * rep + h0);  // the first query head's
     const float* const src_rows = role == 0 ? a.lse : a.delta;
-    const float row_sc = role == 0 ? -LOG2E : 1.0f;
-    Mover3<D, G> mv;
+    const float row_sc = role == 0 ? -LOG2E : UP<ALL>;
+    Mover3<D, G, ALL> mv;
     mv.init(gt, s_st, dk);
     float row_r = 0.0f;
     int f_h = 0, f_t = 0;  // the (head, tile) of the next fetch
@@ -747,7 +765,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     {
         Row<D> kv;
         kv.load(head_of<float>(role == 0 ? a.k : a.v, role == 0 ? a.k_sb : a.v_sb, b, role == 0 ? a.k_sh : a.v_sh, hk), role == 0 ? a.k_st : a.v_st, kj, a.T, dk, g);
-        kv.split(res);
+        kv.template split<ALL>(res);
     }
     f32x16 acc[DB];  // dV^T, dK^T
 #pragma unroll
@@ -798,6 +816,8 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                     for (int r = 0; r < 16; ++r) t[r] = kvis(qlo + (r >> 2) * 8 + g * 4 + (r & 3)) ? t[r] : 0.0f;
                 }
                 put_tile(pb, t, lane);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) t[r] *= UP<ALL>;
                 if (APART) parts = Parts(t);
             }
             if (!APART) stage();
@@ -808,7 +828,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                 for (int qd = 0; qd < 4; ++qd) {
                     const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + 32 + qd * 8 + g * 4);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) t[qd * 4 + e] = p[qd * 4 + e] * (t[qd * 4 + e] - dl[e]);
+                    for (int e = 0; e < 4; ++e) t[qd * 4 + e] = p[qd * 4 + e] * fmaf(t[qd * 4 + e], DOWN<ALL>, -dl[e]);
                 }
             }
             if (live && (ROLE == 1 || !APART)) parts = Parts(t);
@@ -824,11 +844,13 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     // partial rows: the sink keys' of a split tail (and, unless the group's heads are split too, of the block's own band) go to
     // tail[unit][piece][dK | dV][32][dk], the others of a split group to part[unit][split][dK | dV][T][dk]
     const bool to_tail = tl.nch > 0 && k0 == 0 && kj < a.sinks && (chunk >= 0 || hs == 1), stored = kj < a.T && (chunk < 0 || to_tail);
-    for (uint32_t again = rows_to_redo<DB>(acc, 1.0f, stored); __builtin_expect(again != 0, 0); again &= again - 1) {
+    float sc = (role == 0 ? 1.0f : a.scale) * (DOWN<ALL> * DOWN<ALL>);
+    for (uint32_t again = rows_to_redo<DB, ALL>(acc, 1.0f, stored); __builtin_expect(again != 0, 0); again &= again - 1) {
         const int row = __builtin_ctz(again);
         double x[2];
         exact_dkdv(arguments_again(), role == 1, b, hk, hk * rep + h0, nh, qt_lo * 32, q_end + 1, kw0 + row, lane, x);
         put_row<D, DB>(row_room<D, 2 * QW, 0>(lds, w), x, row, acc, lane);
+        if (ALL && c32 == row) sc = role == 0 ? 1.0f : a.scale;
     }
     if (a.in_place) __syncthreads();  // every row has been read
     if (stored) {
@@ -842,7 +864,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                                                                        : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
         void* const dst = scratch ? room : role == 0 ? a.dv : a.dk;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) store_block32<D>(dst, row, db, g, acc[db], role == 0 ? 1.0f : a.scale, dk);
+        for (int db = 0; db < DB; ++db) store_block32<D>(dst, row, db, g, acc[db], sc, dk);
     }
 }
 template <int D, int QW>
@@ -855,11 +877,11 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
     // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
     if (a.causal && nblk > 1 ? xcd_map_block_major(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu)
                              : xcd_map(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu))
-        dkdv_block<D, QW>(a, blk, rr, kvu, lds, pbuf);
+        dkdv_block<D, QW, false>(a, blk, rr, kvu, lds, pbuf);
 }
 
 // ---- dK, dV and dQ in one launch, delta read (f32x3_takes_bwd) ----
-template <int D>
+template <int D, bool ALL>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
     all_arguments(a);
     constexpr int Q = dq_lds<D, 2, 2>(), K = 2 * DKDV_TILE<D, 2>, N = Q > K + 4096 ? Q : K + 4096;
@@ -867,9 +889,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
     const JoinedBlocks jb(a, 64);
     int rank, r, kvu;
     if (!jb.map(a, rank, r, kvu)) return;
-    if (r < a.head_split) return dkdv_block<D, 2>(a, rank, r, kvu, lds, reinterpret_cast<float*>(lds + K));
+    if (r < a.head_split) return dkdv_block<D, 2, ALL>(a, rank, r, kvu, lds, reinterpret_cast<float*>(lds + K));
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
-    dq_block<D, 2, 2>(a, 0, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    dq_block<D, 2, 2, ALL>(a, 0, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // ---- dQ above 64 columns: the same two phases ----
@@ -1071,7 +1093,11 @@ int run_bwd(const AttnArgs& a_in, hipStream_t st) {
     a.head_split = head_split(a);
     a.tail = nullptr;
     if (const int rc = launch_row_delta(a, false, st)) return rc;
-    hipLaunchKernelGGL((x3_bwd<D>), dim3(JoinedBlocks(a, 64).grid(a)), dim3(256), 0, st, a);
+    const dim3 grid(JoinedBlocks(a, 64).grid(a));
+    if (f32x3_bwd_keeps_all(a_in))
+        hipLaunchKernelGGL((x3_bwd<D, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((x3_bwd<D, false>), grid, dim3(256), 0, st, a);
     PK_HIP(hipGetLastError());
     return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
 }
@@ -1102,23 +1128,27 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 // long as the launch and half of the chip waits for them; together one's chains run beside the other's. Over some rounds it is the same
 // work with a pass over O and dO more. In 64-row blocks of queries, one after the other (or on the fp32 instruction) | joined, us, causal
 // unless said:
-//   64 columns   T 1024 x 4, 8 heads (512) 122 | 110;   T 313 x 4, 16 heads (320) 73 | 36;   T 836 x 2, 8 heads (224) 84 | 65;
-//                T 1841, 8 heads (232) 132 | 117;   T 360 x 3, 8 heads (144) 39 | 32;   no mask, T 777 x 4, 12 heads (624) 208 | 176
+//   64 columns   T 1024 x 4, 8 heads (512) 122 | 110;   T 313 x 4, 16 heads (320) 73 | 36;   T 836 x 2, 8 heads (224) 81 | 61;
+//                T 1841, 8 heads (232) 136 | 120;   T 360 x 3, 8 heads (144) 38 | 31;   no mask, T 777 x 4, 12 heads (624) 210 | 177
 //     below      T 963, 4 heads (64) 50 | 66;   T 894 x 4, 2 heads (112) 45 | 60;   T 3305, 4 heads on 2 (208) 197 | 202
 //     above      T 5833, 8 heads (736) 688 | 710;   T 1024 x 8, 16 heads (2048) 351 | 362;   T 4096 x 4, 16 heads (4096) 2417 | 2562
-//   32 columns   T 1037 x 2, 8 heads (272) 62 | 50;   T 181 x 13, 16 heads (624) 42 | 29;   no mask, T 1639, 8 heads (208) 109 | 88
-//   128 columns, one workgroup to a CU   T 270 x 3, 16 heads (240) 122 | 58;   T 1796, 2 heads (58) 240 | 196;   T 2132, 8 heads (272) 393 | 280;
-//                no mask, T 710, 8 heads (96) 127 | 90;   above: T 440 x 19, 4 heads (532) 146 | 158;   no mask, T 1010 x 14, 2 heads (448) 353 | 388
-//   96 columns   T 241 x 10, 4 heads (160) 52 | 33;   T 936, 16 heads of 80 (240) 131 | 97;   below, above: T 2413, 4 heads of 80 (152) 184 | 210;   T 2309 x 2,
+//   32 columns   T 1037 x 2, 8 heads (272) 62 | 51;   T 181 x 13, 16 heads (624) 42 | 29;   no mask, T 1639, 8 heads (208) 109 | 85
+//   128 columns, one workgroup to a CU   T 270 x 3, 16 heads (240) 122 | 58;   T 1796, 2 heads (58) 244 | 200;   T 2132, 8 heads (272) 393 | 291;
+//                no mask, T 710, 8 heads (96) 129 | 91;   above: T 440 x 19, 4 heads (532) 146 | 158;   no mask, T 1010 x 14, 2 heads (448) 353 | 388
+//   96 columns   T 241 x 10, 4 heads (160) 52 | 34;   T 936, 16 heads of 80 (240) 130 | 96;   below, above: T 2413, 4 heads of 80 (152) 184 | 210;   T 2309 x 2,
 //                8 heads (592) 421 | 499
-//   bands, every head its own: 48, T 165 x 6, 8 heads, window 86 (144) 36 | 20;   T 4383, 8 heads, 26 (552) 51 | 42;   T 975 x 13, 2 heads of 64, 408,
-//     1 sink (416) 109 | 79;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
-//     whose sink keys' block is walked for up to 600 queries more while there are blocks enough beside it: 64, T 419 x 6, 8 heads, 40, 1 sink (336) 51 | 38;
-//     T 426 x 14, 4 heads, 36, 4 (392) 76 | 39;  48, T 1140 x 11, 2 heads, 556 (396) 119 | 83;  96, T 707 x 10, 2 heads, 321, 1 (240) 102 | 76;  not: 64,
+//   bands, every head its own: 48, T 165 x 6, 8 heads, window 86 (144) 35 | 19;   T 4383, 8 heads, 26 (552) 51 | 41;   T 975 x 13, 2 heads of 64, 408,
+//     1 sink (416) 107 | 74;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
+//     whose sink keys' block is walked for up to 600 queries more while there are blocks enough beside it: 64, T 419 x 6, 8 heads, 40, 1 sink (336) 54 | 40;
+//     T 426 x 14, 4 heads, 36, 4 (392) 78 | 40;  48, T 1140 x 11, 2 heads, 556 (396) 126 | 85;  96, T 707 x 10, 2 heads, 321, 1 (240) 107 | 76;  not: 64,
 //     T 962, 8 heads, 331, 16 (128) 58 | 66;  T 934, 12 heads of 48, 396, 1 (180) 64.7 | 65.3; over 36 random shapes 0.86 of the time
 //     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
+//
+// Where one of the two by itself would be on the fp32 instruction, values keep all the bits that they have there (UP). Scores from 2^80 on are
+// out of range then: at the smallest scale that is 2^40 in the exponent, whose last place is 2^17.
+bool f32x3_bwd_keeps_all(const AttnArgs& a) { return dq_form(a) == Form::NONE || dkdv_form(a) == Form::NONE || f32_split_takes_bwd(a); }
 bool f32x3_takes_bwd(const AttnArgs& a) {
-    if (!f32_split_serves(a) || a.T <= 32) return false;
+    if (!f32_split_serves(a) || a.T <= 32 || (a.scale < 0x1p-40f && f32x3_bwd_keeps_all(a))) return false;
     const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
     if (a.window > 0)
         return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= (a.dk_dim > 64 || q >= 200 ? 600 : 300)) &&

@@ -106,10 +106,9 @@ int head_split_of(const pk_attn_shape* s) {
     const Mask m = effective_mask(s);
     return gqa_head_split(s->B, s->T, s->Hq, s->Hkv, s->dk, s->causal != 0, m.window, m.sinks, s->dtype == PK_BF16);
 }
-// Whether the dK/dV launch goes to a kernel that splits so, asked of the dispatch itself. Only dimensions, mask and input
-// type of the shape count: the tensors are taken as aligned rows, a positive scale and fp32 gradients as given. Others take
-// the scalar kernels or one that walks a group in one workgroup, so the answer is an upper bound for them.
-bool deals_heads(const pk_attn_shape* s) {
+// What the dispatch is asked about a shape: only its dimensions, mask and input type count, the tensors are taken as aligned rows, a
+// positive scale and fp32 gradients as given.
+AttnArgs aligned_rows(const pk_attn_shape* s) {
     AttnArgs a;
     std::memset(&a, 0, sizeof a);
     a.B = s->B; a.T = s->T; a.Hq = s->Hq; a.Hkv = s->Hkv; a.dk_dim = s->dk;
@@ -119,6 +118,12 @@ bool deals_heads(const pk_attn_shape* s) {
     a.grad_f32 = 1;
     a.q_st = a.k_st = a.v_st = a.o_st = a.do_st = a.dq_st = a.dk_st = a.dv_st = s->dk;
     a.head_split = head_split_of(s);
+    return a;
+}
+// Whether the dK/dV launch goes to a kernel that splits so. Other tensors take the scalar kernels or one that walks a group in one
+// workgroup, so the answer is an upper bound for them.
+bool deals_heads(const pk_attn_shape* s) {
+    const AttnArgs a = aligned_rows(s);
     return s->dtype == PK_BF16 ? split_serves(a) && bf16_deals_heads(a) : f32_mfma_supported(a) && f32_deals_heads(a);
 }
 size_t part_bytes(const pk_attn_shape* s) {
@@ -245,6 +250,14 @@ int pk_attn_bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_ten
                        const pk_tensor4* dv, void* workspace, size_t workspace_bytes, int stages,
                        void* stream) {
     return bwd_stages(s, q, k, v, o, lse, d_o, dq, dk, dv, workspace, workspace_bytes, stages, true, stream);
+}
+
+int pk_bwd_of_shape(const pk_attn_shape* s) {
+    AttnArgs a = aligned_rows(s);
+    static float room;  // asked for by its presence alone
+    if (tail_bytes(s)) a.tail = &room;
+    if (s->dtype == PK_BF16) return split_serves(a) ? static_cast<int>(bwd_of_bf16(a)) : -1;
+    return f32_mfma_supported(a) ? static_cast<int>(bwd_of_f32(a)) : -1;
 }
 
 }  // extern "C"

@@ -177,6 +177,7 @@ int launch_f32x3_fwd(const AttnArgs& a, hipStream_t st);
 int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st);
 int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st);
 bool f32x3_takes_bwd(const AttnArgs& a);  // dQ and dK/dV in one launch, behind one of delta
+bool f32x3_bwd_keeps_all(const AttnArgs& a);  // where that launch holds the whole range of fp32, as the instruction does
 int launch_f32x3_bwd(const AttnArgs& a, hipStream_t st);
 // delta = rowsum(dO .* O) by itself, aligned rows of any head size; attn_bwd_mfma.hip
 int launch_row_delta(const AttnArgs& a, bool bf16, hipStream_t st);
@@ -209,6 +210,14 @@ int launch_split_joined(const AttnArgs& a, hipStream_t st);
 bool bf16_rows_aligned(const AttnArgs& a);
 int launch_mfma_fwd(const AttnArgs& a, hipStream_t st);
 int launch_mfma_bwd(const AttnArgs& a, int stages, hipStream_t st);
+
+// How dQ and dK/dV are launched when a backward is asked for as a whole and no gradient lies where an input does: one launch after the other, or
+// one of both (launch_split_bwd, launch_split_joined, launch_joined_bwd; launch_f32_split_bwd, launch_f32x3_bwd in its two forms).
+enum class Bwd { APART, SPLIT, SPLIT_JOINED, JOINED, F32_SPLIT, F32_PARTS, F32_PARTS_ALL };
+Bwd bwd_of_bf16(const AttnArgs& a);
+Bwd bwd_of_f32(const AttnArgs& a);
+// The same of a shape with aligned rows, as a number; -1 for one that the scalar kernels take. For tests.
+extern "C" int pk_bwd_of_shape(const pk_attn_shape* s);
 bool bf16_deals_heads(const AttnArgs& a);  // its dK/dV kernel for this launch uses a.head_split and a.part
 int launch_mfma_dkdv2(const AttnArgs& a, hipStream_t st);
 bool joined_takes_bwd(const AttnArgs& a);  // attn_bwd_dkdv2.hip: dQ (with delta) and dK/dV in one launch, head_dim 128

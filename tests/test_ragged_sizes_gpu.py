@@ -1,10 +1,12 @@
 """GPU tests at the sizes where the kernels' edges lie: token counts, vocabularies, head sizes and sequence lengths that
 are no multiple of a tile, a chunk or a wavefront."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from paperkiln_amd import blockops, ops, synth
+from paperkiln_amd import _lib, blockops, ops, synth
 from paperkiln_amd.llama import Llama
 
 pytestmark = pytest.mark.gpu
@@ -156,6 +158,14 @@ def exact_attention(q, k, v, d_o, scale, causal, window, sinks, given_o=None):
     group = lambda x: x.reshape(B, Hq // rep, rep, T, dk).sum(2)  # noqa: E731
     back = lambda x: x.permute(0, 2, 1, 3)  # noqa: E731
     return back(o), lse, back(dq), back(group(dkx)), back(group(dvx))
+
+
+def bwd_form(case, dk, dtype):
+    """Which launch takes a whole backward of these sizes."""
+    B, T, Hq, Hkv, causal, window, sinks = case
+    code = _lib.PK_F32 if dtype == torch.float32 else _lib.PK_BF16
+    form = _lib.lib().pk_bwd_of_shape(ctypes.byref(_lib.AttnShape(B, T, Hq, Hkv, dk, int(causal), window, sinks, 1.0, code, code)))
+    return "SCALAR" if form < 0 else ("APART", "SPLIT", "SPLIT_JOINED", "JOINED", "F32_SPLIT", "F32_PARTS", "F32_PARTS_ALL")[form]
 
 
 def run_attention(B, T, Hq, Hkv, dk, dtype, causal, window, sinks, grad_dtype=torch.float32):
@@ -364,6 +374,36 @@ def test_three_parts_of_tiny_tensors(case, dk, tiny):
     o, lse = ops.attn_fwd(x["q"], x["k"], x["v"], scale, causal, window, sinks)
     got = (o, lse, *ops.attn_bwd(x["q"], x["k"], x["v"], o, lse, x["d_o"], scale, causal, window, sinks))
     e = [float((g.double() - w).norm() / w.norm()) for g, w in zip(got, exact_attention(x["q"], x["k"], x["v"], x["d_o"], scale, causal, window, sinks))]
+    assert max(e) < 1e-6, e
+
+
+# Launches of the whole backward in three parts where dQ or dK/dV by itself would be on the fp32 instruction: every padded head size, masked
+# and not, bands, groups of heads, dealt out too
+WHOLE_RANGE_CASES = [((12, 383, 8, 8, True, 37, 5), 32), ((5, 577, 8, 8, False, 0, 0), 20), ((4, 313, 16, 16, True, 0, 0), 64), ((7, 65, 16, 8, True, 0, 0), 44),
+                     ((6, 321, 9, 9, True, 33, 17), 80), ((1, 710, 8, 8, False, 0, 0), 96), ((2, 641, 13, 13, True, 0, 0), 128),
+                     ((1, 2113, 8, 2, True, 0, 0), 100), ((1, 710, 8, 8, False, 0, 0), 128)]
+
+
+@pytest.mark.parametrize("tensors", ["kq", "q", "k", "v", "d_o"])
+@pytest.mark.parametrize("case,dk", WHOLE_RANGE_CASES, ids=str)
+def test_joined_parts_hold_columns_of_every_size(case, dk, tensors):
+    """Columns from 2^-120 to 2^20 of one tensor, or one of K at 2^-120 whose scores one of Q at 2^120 makes ordinary: every column of every
+    gradient exact at its own size, from the O and LSE of float64. Bound as of test_fp32_as_three_parts."""
+    assert bwd_form(case, dk, torch.float32) == "F32_PARTS_ALL"
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    x = {n: torch.randn((B, T, h, dk), generator=gen, device="cuda") for n, h in (("q", Hq), ("k", Hkv), ("v", Hkv), ("d_o", Hq))}
+    if tensors == "kq":
+        x["q"][..., 2] *= 2.0 ** 120
+        x["k"][..., 2] *= 2.0 ** -120
+    else:
+        x[tensors] *= 2.0 ** torch.linspace(-120, 20 if tensors in ("v", "d_o") else 0, dk, device="cuda").round()
+        x["d_o"] *= 1.0 if tensors in ("v", "d_o") else 2.0 ** 20  # dQ and dK at 2^-120 of it are in fp32's range
+    args = (x["q"], x["k"], x["v"], x["d_o"], float(np.float32(1.0 / np.sqrt(dk))), causal, window, sinks)
+    o, lse = (t.float().contiguous() for t in exact_attention(*args)[:2])
+    got = ops.attn_bwd(*args[:3], o, lse, *args[3:])
+    columns = lambda t: t.double().reshape(-1, dk).norm(dim=0)  # noqa: E731
+    e = [float((columns(g.double() - w) / columns(w)).max()) for g, w in zip(got, exact_attention(*args, o)[2:])]
     assert max(e) < 1e-6, e
 
 
