@@ -143,7 +143,10 @@ __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
 // Whether dP starts from -delta instead of zero, a subtraction an element less: dQ 1.6 %, dK/dV 2.5 % over 17 shapes. The sum is then
 // rounded at delta's size four times instead of once, which dS, one bf16 operand there, does not show: errors of dQ and dK against
 // float64 are 1.63e-3 to 1.79e-3 of their norms and the same to four digits either way over 28 inputs, V with a mean of 30 standard
-// deviations among them. Not where P and dS keep all their bits (EXACT), nor at 128 columns, where it spilled 30 registers more.
+// deviations among them. Not where P and dS keep all their bits (EXACT), nor at 128 columns, where it spilled 30 registers more; dQ not where
+// four wavefronts share the tiles (T 1661, 16 heads 21.5 us | 24.5), nor in the joined launch, whose sizes came from that form: where V is the same
+// in every row dS is zero and dQ the rounding of dP alone, two to three times as much from -delta (joined launch from zero, us: T 512 x 16, 8 heads
+// 34.4 -> 34.3, T 470 x 8, 8 heads 20.4 -> 20.7, T 1024 x 8 50.3 -> 51.2, T 4945 133.3 -> 135.8).
 template <int D, bool EXACT>
 constexpr bool FROM_DELTA = !EXACT && D == 64;
 
@@ -351,11 +354,10 @@ constexpr int dq_lds() {  // in uint16
     constexpr int TILES = (QW > 1 ? 2 : 1) * KW * 2 * 32 * NB * (D + 8), RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
     return TILES > RED ? TILES : RED;
 }
-template <int D, int QW, int KW, int NB, bool EXACT>
+template <int D, int QW, int KW, int NB, bool EXACT, bool MINUS_DELTA = FROM_DELTA<D, EXACT> && (QW > 1 || KW == 8)>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h, int hk, int qblk, uint16_t* lds) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
-    constexpr bool MINUS_DELTA = FROM_DELTA<D, EXACT> && (QW > 1 || KW == 8);  // not with four: T 1661, 16 heads 21.5 us | 24.5
 
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = w / QW, qg = w % QW, gt = static_cast<int>(threadIdx.x) - kg * G;
@@ -712,7 +714,7 @@ __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     if (!jb.map(a, rank, r, kvu)) return;
     if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA>(a, rank, r, kvu, lds);
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
-    dq_block<D, 4, 1, 2, EXACT>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    dq_block<D, 4, 1, 2, EXACT, false>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of
