@@ -74,8 +74,9 @@ struct Mover {
 
 // Row r0 + c32 of a head as an operand held in registers: chunk kk covers d = 16kk + 8g .. +7; zero past T and past dk. BRANCH: under a
 // condition instead of through a buffer, which keeps the loads where they are written. In the long loops of P and dS in several parts the scheduler
-// needs that (forward, us, buffer | branch: 96 columns, T 1500 x 4, 8 heads 44.0 | 41.6; 48, T 4000 x 2, window 500 27.2 | 26.1; backward 79.7 | 77.1, but
-// 96 columns 111.5 | 113.8; 80, no mask, T 2000 x 4 286 | 291); at 64 columns the buffer is ahead (T 4096 x 2, 8 heads 154 | 156), and where chains are short.
+// needs that (forward, us, buffer | branch: 96 columns, T 1500 x 4, 8 heads 44.0 | 41.6, T 2500, 4 heads 24.8 | 23.5; 48, T 4000 x 2, window 500 27.2 | 26.1; backward
+// 79.7 | 77.1, but 96 columns 111.5 | 113.8; 80, no mask, T 2000 x 4 286 | 291); in the backward at 64 columns the buffer is ahead (T 4096 x 2, 8 heads 154 | 156), and
+// in the forward at 128 (T 200, 4 heads 6.8 | 7.2).
 template <int D, bool BRANCH>
 __device__ inline void load_row(const uint16_t* head, int st, int r0, int T, int dk, int c32, int g, bf16x8* out) {
     if constexpr (BRANCH) {
@@ -204,8 +205,10 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     int b, h, hk, qblk;
     if (!map_query_block(a, nqb, b, h, hk, qblk)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
-    const uint16_t *const kh = head_of<uint16_t>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<uint16_t>(a.v, a.v_sb, b, a.v_sh, hk),
-                   *const qh = head_of<uint16_t>(a.q, a.q_sb, b, a.q_sh, h);
+    // plain addresses: formed with head_of, and Q's row through a buffer, the loops of long chains and of bands were behind (us: 96 columns, T 5637, 2
+    // heads 48 | 53; T 4000, 3 heads 35 | 40; 64, T 980 x 10, 16 heads, window 41, 16 sinks 23.6 | 25.4; T 4096 x 4, 16 heads, window 256 45.3 | 48.1)
+    const uint16_t *const kh = static_cast<const uint16_t*>(a.k) + (b * a.k_sb + hk * a.k_sh), *const vh = static_cast<const uint16_t*>(a.v) + (b * a.v_sb + hk * a.v_sh),
+                   *const qh = static_cast<const uint16_t*>(a.q) + (b * a.q_sb + h * a.q_sh);
     const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
 
@@ -229,7 +232,7 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
     };
     fetch(0);
     bf16x8 qreg[KK];
-    load_row<D, EXACT && (QW > 1)>(qh, static_cast<int>(a.q_st), qlo, a.T, dk, c32, g, qreg);
+    load_row<D, (QW > 1) || (EXACT && D <= 96)>(qh, static_cast<int>(a.q_st), qlo, a.T, dk, c32, g, qreg);
     f32x16 acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)

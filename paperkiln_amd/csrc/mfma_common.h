@@ -274,7 +274,8 @@ __host__ __device__ inline int quotient(int n, int d) { return static_cast<int>(
 // waits one after the other before a workgroup's first load; here they are one.
 // us, as they are used | at once: T 512 x 16, 8 heads of 64 forward 13.6 | 13.4, backward 36.1 | 33.8; T 1024 x 8 20.5 | 19.9, 51.6 | 48.8; T 128, 4 heads
 // backward 7.8 | 7.25; fp32, T 128 x 2, 4 heads of 32 4.95 | 4.8, 8.5 | 8.1. Not in the long kernels of 128 columns, nor where rows are a wavefront's own and
-// the loop is P in two parts: registers of the loop went to it (96 columns, T 1500 x 4 41.6 | 42.1; 128, T 4096 x 4 278 | 285).
+// the loop is P in two parts: registers of the loop went to it (96 columns, T 1500 x 4 41.6 | 42.1; 128, T 4096 x 4 278 | 285), nor
+// in the unsplit forward under a band (64, T 54 x 81, 4 heads, window 42 5.3 | 5.7).
 __device__ inline void all_arguments(const AttnArgs& a) {
     asm volatile("" ::"s"(a.q), "s"(a.q_sb), "s"(a.k_sb), "s"(a.do_sb), "s"(a.dk_st), "s"(a.T), "s"(a.scale));
 }
