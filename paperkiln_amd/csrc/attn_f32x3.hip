@@ -451,8 +451,10 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void x3_fwd(AttnArgs a) {
     int b, h, hk, qblk;
     if (!map_query_block(a, (a.T + BM - 1) / BM, b, h, hk, qblk)) return;
     const int q0 = qblk * BM, qlo = q0 + qg * 32, qhi = qlo + 31, qi = qlo + c32;
-    const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk),
-                *const qh = head_of<float>(a.q, a.q_sb, b, a.q_sh, h);
+    // plain addresses, as in split_fwd (us, with head_of | so: 128 columns, T 3473, 8 heads 241 | 231; T 492 x 33, 2 heads 62.4 | 59.4; 64, T 300 x 16, 8
+    // heads 21.7 | 19.9; T 1024 x 4 40.8 | 40.2)
+    const float *const kh = static_cast<const float*>(a.k) + (b * a.k_sb + hk * a.k_sh), *const vh = static_cast<const float*>(a.v) + (b * a.v_sb + hk * a.v_sh),
+                *const qh = static_cast<const float*>(a.q) + (b * a.q_sb + h * a.q_sh);
     const int k_st = static_cast<int>(a.k_st), v_st = static_cast<int>(a.v_st);
     const float cexp = a.scale * LOG2E;
 

@@ -88,7 +88,7 @@ __device__ inline const float* no_weights() { return nullptr; }
 // With it, LSE asked for with the rest and all wavefronts in the join, bf16 launches of short chains, us: T 128, 4 heads of 64 forward 5.4 -> 4.8,
 // backward 8.0 -> 7.7; T 200, 4 heads of 128 8.5 -> 7.0, 15.6 -> 14.9; T 90 x 2, 4 heads of 32 backward 7.8 -> 6.5; T 1000 x 2, 8 heads of 80
 // 48.6 -> 46.2; 96 columns, T 400, 4 heads 8.7 -> 7.8, 19.4 -> 16.6. Long chains level, backward at 64 columns 1 to 2 % ahead; not in
-// the bf16 forward (split_fwd).
+// the forwards of bf16 and of three parts (split_fwd, x3_fwd).
 template <typename T>
 __device__ inline const T* head_of(const void* base, int64_t sb, int b, int64_t sh, int h) {
     const T* p = static_cast<const T*>(base) + (b * sb + h * sh);
