@@ -560,19 +560,25 @@ int launch_sink_tail_reduce(const AttnArgs& a, hipStream_t st) {
 //              T 307 x 4, 16 on 8 (320) 48 | 35;  T 739, 28 on 4 (336) 67 | 54;  T 2531, 7 on one (280) 152 | 134
 //     not      T 609 x 6, 1 head (60) 25 | 34;  T 1423, 8 heads (184) 64 | 74;  T 3991, 4 on 2 (252) 175 | 191;  T 2422 x 3, 8 heads (912) 164 | 200
 //   no mask    T 54 x 10, 8 heads (80) 14.5 | 8.5;  T 1061 x 4, 2 heads (136) 88 | 59;  T 2309, 8 heads (296) 172 | 140;  T 611, 28 on 4 (280) 70 | 52
-//     not      T 1229, 4 heads (80) 54 | 67;  T 352 x 16, 4 heads (384) 40 | 42;  T 1461 x 3, 7 on one (483) 136 | 175
+//     not      T 1229, 4 heads (80) 54 | 67;  T 352 x 16, 4 heads (384) 40 | 42;  T 1461 x 3, 7 on one (483) 136 | 175;  T 2006, 4 heads (128), where
+//              blocks of 32 rows are a round 70 | 100;  T 62 x 11, 32 on 16 (352) 20 | 24;  T 49 x 69, 4 on 2 (276) 18 | 22
 //   band       T 559 x 4, 8 heads, 71 (288) 30 | 20;  T 140 x 11, 8 heads, 27, 1 sink (264) 24 | 16;  T 1317, 16 on 8, 123 (336) 36 | 28
 //     not      with sinks in long sequences, whose block is walked whole (T 1409, 16 heads, 325 (368) 59 | 87; T 394, 28 on 4, 74 (196) 126 | 145);
-//              T 59 x 29, 16 heads (464) 24 | 29;  T 2839, 14 on 2, 154 (630) 57 | 89
+//              T 59 x 29, 16 heads (464) 24 | 29;  T 2839, 14 on 2, 154 (630) 57 | 89;  few blocks: T 1702, 2 heads, 73 (54) 11.6 | 16.0;  T 1758, 4 on 2,
+//              386 (112) 40 | 45;  groups of more than two whose heads are not dealt out, whose blocks of keys walk them all: T 3396, 7 on one, 477 (378)
+//              92 | 162;  T 372 x 2, 16 on 4, 219 (192) 41 | 54;  T 168 x 4, 16 on 4, 17 (192) 22 | 23;  a tail of sinks beside few blocks: T 697, 8
+//              heads, 181, 4 (88) 26 | 37;  and in long sequences a second round of 512 workgroups: T 3220, 8 heads, 305 (408) 46.7 | 48.4
 bool joined_takes_bwd(const AttnArgs& a) {
     if (a.dk_dim != 128) return false;
     const bool groups = a.Hq > a.Hkv;
     const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
     if (a.window > 0)
-        return a.window <= 512 && (a.sinks == 0 || a.T <= (groups ? 160 : 700)) && q >= (groups ? 76 : 52) && q <= (a.T <= 64 ? 320 : 600);
+        return a.window <= 512 && (a.Hq <= 2 * a.Hkv || bf16_deals_heads(a)) &&
+               (a.sinks == 0 || (groups ? a.T <= 160 : a.T <= 700 && (a.T - a.window <= 300 || q >= 200))) &&
+               q >= (groups ? (a.window > 200 ? 120 : 76) : a.T <= 130 ? 52 : 70) && q <= (a.T <= 64 || a.T > 1000 ? 320 : 600);
     if (a.T >= 4096) return false;
-    if (a.T <= 130) return q >= 56 && q <= 500;
-    if (!a.causal) return q >= 120 && q <= 340;
+    if (a.T <= 130) return q >= 56 && q <= (a.T > 64 || !groups ? 500 : a.Hq == 2 * a.Hkv ? 270 : 340);
+    if (!a.causal) return q >= 130 && q <= 330;
     return a.T <= 800 ? q >= 140 && q <= 600 : q >= (a.T <= 2600 ? 260 : 320) && q <= 500;
 }
 int launch_joined_bwd(const AttnArgs& a_in, hipStream_t st) {

@@ -1136,14 +1136,23 @@ int launch_f32x3_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 //     above      T 5833, 8 heads (736) 688 | 710;   T 1024 x 8, 16 heads (2048) 351 | 362;   T 4096 x 4, 16 heads (4096) 2417 | 2562
 //   32 columns   T 1037 x 2, 8 heads (272) 62 | 51;   T 181 x 13, 16 heads (624) 42 | 29;   no mask, T 1639, 8 heads (208) 109 | 85
 //   128 columns, one workgroup to a CU   T 270 x 3, 16 heads (240) 122 | 58;   T 1796, 2 heads (58) 244 | 200;   T 2132, 8 heads (272) 393 | 291;
-//                no mask, T 710, 8 heads (96) 129 | 91;   above: T 440 x 19, 4 heads (532) 146 | 158;   no mask, T 1010 x 14, 2 heads (448) 353 | 388
+//                no mask, T 710, 8 heads (96) 129 | 91;   above: T 440 x 19, 4 heads (532) 146 | 158;   T 87 x 51, 4 on one (408) 57 | 66;
+//                no mask, T 1010 x 14, 2 heads (448) 353 | 388;   T 44 x 99, 2 heads (198) 30 | 33
 //   96 columns   T 241 x 10, 4 heads (160) 52 | 34;   T 936, 16 heads of 80 (240) 130 | 96;   below, above: T 2413, 4 heads of 80 (152) 184 | 210;   T 2309 x 2,
-//                8 heads (592) 421 | 499
+//                8 heads (592) 421 | 499;   from 2600 tokens on, where the launch of both on the fp32 instruction ends, from 88 blocks on (0.86 of the time over
+//                81 shapes): T 3300 x 2, 1 head of 80 (104) 323 | 277;   T 6000, 1 head (94) 575 | 494;   no mask, above: T 44 x 99, 2 heads (198) 24 | 27;
+//                T 312 x 15, 4 on 2 (300) 81 | 94
+//   no mask, 512 workgroups there at once at 64 columns: up to 256 blocks of either kind are one round instead of two, up to 384 two that are full, from 540
+//     on one round less than apart (T 4549 x 3, 2 heads (432) 643 | 732);   with groups the blocks of keys are the longer ones: T 3183, 8 on 2 (400) 452 | 533;
+//     T 2003, 16 on 4 (512) 344 | 382;   32 columns, T 3353, 8 on 4 (424) 308 | 365
 //   bands, every head its own: 48, T 165 x 6, 8 heads, window 86 (144) 35 | 19;   T 4383, 8 heads, 26 (552) 51 | 41;   T 975 x 13, 2 heads of 64, 408,
 //     1 sink (416) 107 | 74;   not: T 1238, 16 heads of 32, 204, 4 sinks, whose block is walked whole (320) 46 | 64;   T 2377, 8 on 2 of 64 (304) 89 | 118
 //     whose sink keys' block is walked for up to 600 queries more while there are blocks enough beside it: 64, T 419 x 6, 8 heads, 40, 1 sink (336) 54 | 40;
 //     T 426 x 14, 4 heads, 36, 4 (392) 78 | 40;  48, T 1140 x 11, 2 heads, 556 (396) 126 | 85;  96, T 707 x 10, 2 heads, 321, 1 (240) 107 | 76;  not: 64,
-//     T 962, 8 heads, 331, 16 (128) 58 | 66;  T 934, 12 heads of 48, 396, 1 (180) 64.7 | 65.3; over 36 random shapes 0.86 of the time
+//     T 962, 8 heads, 331, 16 (128) 58 | 66;  T 934, 12 heads of 48, 396, 1 (180) 64.7 | 65.3;  80, T 654, 8 heads, 180, 16 (88) 49 | 65;  128, T 490 x
+//     3, 2 heads, 99, 16 (48) 42 | 67;  32, T 137 x 3, 16 heads, 27, 16 (144) 11.6 | 14.9;  T 1554, 8 heads, 1017, 4 (200) 57 | 75
+//     long bands: 32, T 4127, 2 heads, 966 (130) 37 | 50;  T 1204, 8 heads, 574 (152) 29 | 34;  above, 64, T 4520, 8 heads, 1279 (568) 226 | 241;  96,
+//     T 3220, 8 heads, 305 (408) 99 | 131;  T 4790, 4 heads, 74 (300) 59 | 67
 //     below      T 1460, 8 heads (184) 56 | 65;   above   T 3072, 16 heads on 4 (768) 243 | 249;   no mask, T 3830, 8 on 2 (480) 371 | 423
 //
 // Where one of the two by itself would be on the fp32 instruction, values keep all the bits that they have there (UP). Scores from 2^80 on are
@@ -1152,14 +1161,19 @@ bool f32x3_bwd_keeps_all(const AttnArgs& a) { return dq_form(a) == Form::NONE ||
 bool f32x3_takes_bwd(const AttnArgs& a) {
     if (!f32_split_serves(a) || a.T <= 32 || (a.scale < 0x1p-40f && f32x3_bwd_keeps_all(a))) return false;
     const int64_t q = static_cast<int64_t>((a.T + 63) / 64) * a.Hq * a.B;
-    if (a.window > 0)
-        return a.Hq == a.Hkv && (a.sinks == 0 || a.T - a.window <= (a.dk_dim > 64 || q >= 200 ? 600 : 300)) &&
-               q >= (a.dk_dim <= 32 ? 130 : a.dk_dim <= 64 ? 100 : a.dk_dim <= 96 ? 88 : 40) && q <= (a.dk_dim <= 64 ? 800 : 420);
-    if (a.dk_dim > 96) return q >= 40 && q <= (a.causal ? 420 : a.T <= 130 ? 200 : 260);
-    if (a.dk_dim > 64) return q >= (a.causal && a.T > 300 && a.T <= 2600 ? 170 : 88) && q <= (a.causal ? 330 : 300);
-    if (a.dk_dim <= 32) return !a.causal ? q >= 180 && q <= 440 : q >= (a.T <= 130 ? 104 : a.T <= 600 ? 190 : 260) && q <= 640;
-    if (!a.causal) return q >= 120 && q <= 960;
-    return q >= (a.T <= 600 ? 140 : a.T <= 2000 ? 180 : 260) && q <= (a.T <= 1500 ? 1100 : 700);
+    const bool groups = a.Hq > a.Hkv;
+    if (a.window > 0) {
+        const int chain = chain_tokens(a), tail = a.sinks > 0 ? a.T - a.window : 0;
+        return !groups && tail <= (q >= (a.dk_dim <= 32 ? 260 : 200) ? 600 : 300) &&
+               q >= (a.dk_dim <= 32 ? (chain > 400 || tail > 100 ? 200 : 130) : a.dk_dim <= 64 ? 100 : a.dk_dim <= 96 ? 88 : 50) &&
+               q <= (a.dk_dim <= 64 ? (chain > 1000 ? 500 : chain > 400 ? 700 : 800) : a.T > 2500 || a.window < 32 ? 290 : 420);
+    }
+    if (a.dk_dim > 96) return q >= 40 && q <= (a.causal ? (a.T <= 130 ? 300 : 420) : a.T <= 64 ? 130 : a.T <= 130 ? 200 : 260);
+    if (a.dk_dim > 64) return q >= (a.causal && a.T > 300 && a.T <= 2600 ? 170 : 88) && q <= (a.causal ? 330 : a.T <= 100 ? 120 : 290);
+    if (a.dk_dim <= 32)
+        return !a.causal ? q >= 180 && q <= (groups && a.T >= 800 ? 390 : 440) : q >= (a.T <= 130 ? 116 : a.T <= 600 ? 190 : 260) && q <= 640;
+    if (!a.causal) return q >= 124 && q <= 960 && (a.T < 1000 || (groups ? q <= 300 : q <= 384 || q >= 540));
+    return q >= (a.T <= 600 ? 140 : a.T <= 2000 ? 180 : 260) && q <= (a.T <= 1500 ? 1000 : 700);
 }
 int launch_f32x3_bwd(const AttnArgs& a, hipStream_t st) { return a.dk_dim <= 32 ? run_bwd<32>(a, st) : a.dk_dim <= 64 ? run_bwd<64>(a, st) : a.dk_dim <= 96 ? run_bwd<96>(a, st) : run_bwd<128>(a, st); }
 int launch_f32x3_dkdv(const AttnArgs& a, hipStream_t st) {

@@ -1016,20 +1016,26 @@ bool split_takes_bwd(const AttnArgs& a) {
 //   80, 96 (delta in a launch of its own)  T 49 x 131, 2 heads (262) 37 | 21;  T 393 x 7, 14 on 2 (392) 70 | 56;  T 2515, 14 on 2 (280) 217 | 173
 //     below, above T 1110, 16 heads (144) 63 | 69;  T 2573, 8 on 4 (168) 125 | 157;  T 129 x 15, 16 on 8 (480) 40 | 44
 //   bands, every head its own  64: T 651 x 2, 8 heads, window 235 (96) 26 | 17;  T 4247, 8 heads, 336 (272) 36 | 32;  T 159 x 7, 16 on 8 23 | 18
-//     not          T 1128, 16 heads, 178, 1 sink, whose block is walked whole (144) 33 | 42;  T 1777, 16 on 8 44 | 116;  T 211 x 8, 4 heads (64) 11 | 14
+//     not          T 1128, 16 heads, 178, 1 sink, whose block is walked whole (144) 33 | 42;  T 1777, 16 on 8 44 | 116;  T 211 x 8, 4 heads (64) 11 | 14;
+//                  32 columns under long bands: T 3810, 8 heads, 1771 (240) 76 | 90;  T 2632, 16 heads, 1403 (336) 79 | 84
+//   past 512 workgroups, which are there at once, both kinds share a second round: 64, T 4950, 8 heads, window 25 (312) 18.4 | 21.2;  no mask, T 4433,
+//     8 on 4 (280) 256 | 290;  96, no mask, T 222 x 53, 4 heads (424) 49 | 56;  T 37 x 49, 8 heads (392) 19 | 22;  and with groups, whose blocks of keys
+//     walk all heads: T 3156, 16 on 4 (400) 423 | 525;  T 1424, 16 on 4 (192) 128 | 135
 bool split_takes_joined(const AttnArgs& a) {
     if (a.dk_dim > 96 || a.T <= 32) return false;
     const int64_t n = (a.T + 127) / 128, u = n * a.Hq * a.B;
     if (a.window > 0)
         return a.Hq == a.Hkv && (a.sinks == 0 || a.T <= 600) &&
-               (a.dk_dim == 64 ? u >= (chain_tokens(a) <= 1024 ? 84 : 150) && u <= 450 : u >= 190 && u <= 390);
+               (a.dk_dim == 64 ? u >= (chain_tokens(a) <= 1024 ? 84 : 150) && u <= (a.T > 2500 && a.window < 128 ? 256 : 450)
+                               : chain_tokens(a) <= 1024 && u >= 190 && u <= 390);
     if (a.dk_dim == 64)
         return a.causal ? u >= (n == 1 ? 60 : n <= 4 ? 104 : n <= 12 ? 150 : n <= 17 ? 200 : 290) && u <= (n <= 2 ? 440 : 560)
-                        : u >= (n == 1 ? 60 : n <= 8 ? 110 : 150) && u <= 300;
+                        : u >= (n == 1 ? 60 : n <= 8 ? 110 : n <= 32 ? 150 : 170) && u <= (n <= 32 ? 300 : 256);
     if (a.dk_dim < 64)
         return a.causal ? n <= 16 && u >= (n == 1 ? 60 : n <= 2 ? 112 : n <= 7 ? 190 : 300) && u <= 450
                         : n <= 12 && u >= (n == 1 ? 60 : n <= 6 ? 84 : 200) && u <= 300;
-    return u >= (n == 1 ? 80 : n <= 5 ? 150 : n <= 12 ? 190 : 232) && u <= 440;
+    if (!a.causal && n > 8 && a.Hq > a.Hkv) return false;
+    return u >= (n == 1 ? 80 : n <= 5 ? 150 : n <= 12 ? 200 : 232) && u <= (a.causal ? 420 : a.T <= 64 ? 380 : 400);
 }
 template <int D, bool EXACT>
 int joined_of(const AttnArgs& a, hipStream_t st) {
