@@ -138,14 +138,10 @@ int run_dq(const AttnArgs& a, bool fuse_delta, hipStream_t st) {
 bool bf16_deals_heads(const AttnArgs& a) { return a.head_split > 1 && (split_deals_heads(a) || mfma_dkdv3_takes(a)); }
 
 int launch_row_delta(const AttnArgs& a, bool bf16, hipStream_t st) {
-    const int lanes = bf16 ? (a.dk_dim > 64 ? 16 : a.dk_dim > 32 ? 8 : 4) : a.dk_dim > 32 ? 16 : 8;
+    const int lanes = bf16 || a.dk_dim > 32 ? 16 : 8;
     const dim3 grid((a.T + 256 / lanes - 1) / (256 / lanes) * a.Hq * a.B);
-    if (bf16 && lanes == 16)
+    if (bf16)  // asked for above 64 columns
         hipLaunchKernelGGL((row_delta<true, 16>), grid, dim3(256), 0, st, a);
-    else if (bf16 && lanes == 8)
-        hipLaunchKernelGGL((row_delta<true, 8>), grid, dim3(256), 0, st, a);
-    else if (bf16)
-        hipLaunchKernelGGL((row_delta<true, 4>), grid, dim3(256), 0, st, a);
     else if (lanes == 16)
         hipLaunchKernelGGL((row_delta<false, 16>), grid, dim3(256), 0, st, a);
     else
