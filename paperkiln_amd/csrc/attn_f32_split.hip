@@ -389,7 +389,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     const float *const kh = head_of<float>(a.k, a.k_sb, b, a.k_sh, hk), *const vh = head_of<float>(a.v, a.v_sb, b, a.v_sh, hk);
     // of the first query head in hand; the others follow at q_sh, ...
     const float *const q0h = head_of<float>(a.q, a.q_sb, b, a.q_sh, hk * rep + h0), *const g0h = head_of<float>(a.d_o, a.do_sb, b, a.do_sh, hk * rep + h0),
-                *const o0h = head_of<float>(a.o, a.o_sb, b, a.o_sh, hk * rep + h0);
+                *const o0h = OWN_DELTA ? head_of<float>(a.o, a.o_sb, b, a.o_sh, hk * rep + h0) : nullptr;
     Mover32<D> mq, mg;
     mq.init(lane, q_st, dk);
     mg.init(lane, g_st, dk);

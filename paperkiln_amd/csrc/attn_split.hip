@@ -523,7 +523,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
     const int q_st = static_cast<int>(a.q_st), g_st = static_cast<int>(a.do_st), o_st = static_cast<int>(a.o_st);
     // the first query head's; the others follow at q_sh, ...
     const uint16_t *const q0h = head_of<uint16_t>(a.q, a.q_sb, b, a.q_sh, hk * rep + h0), *const g0h = head_of<uint16_t>(a.d_o, a.do_sb, b, a.do_sh, hk * rep + h0),
-                   *const o0h = head_of<uint16_t>(a.o, a.o_sb, b, a.o_sh, hk * rep + h0), *const kh = head_of<uint16_t>(a.k, a.k_sb, b, a.k_sh, hk),
+                   *const o0h = OWN_DELTA ? head_of<uint16_t>(a.o, a.o_sb, b, a.o_sh, hk * rep + h0) : nullptr, *const kh = head_of<uint16_t>(a.k, a.k_sb, b, a.k_sh, hk),
                    *const vh = head_of<uint16_t>(a.v, a.v_sb, b, a.v_sh, hk);
     Mover<D, G, BMQ> mq, mg;
     mq.init(gt, q_st, dk);
