@@ -53,11 +53,6 @@ template <int BNK, int BMQ>
 using Weights = uint16_t[2][BMQ / 32][BNK / 32][2 * 64 * 8];  // [step parity][query block][key block][half][lane][8]
 template <int BMQ>
 using Rows = float[3][BMQ];
-// x of another lane of the same sixteen, by the DPP control word
-template <int CTRL>
-__device__ inline float lane_swapped(float x) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
-}
 
 // A workgroup's blocks of BNK keys, by its number in the launch; JOINED: the block jblk of unit jkvu.
 // TAIL: the launch carries the extra workgroups of a split sink tail (a separate instantiation, so
@@ -192,10 +187,10 @@ __device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weig
                         part = fmaf(__uint_as_float(orow[i][e] << 16), __uint_as_float(gr[i][e] << 16), part);
                         part = fmaf(__uint_as_float(orow[i][e] & 0xFFFF0000u), __uint_as_float(gr[i][e] & 0xFFFF0000u), part);
                     }
-                    part += lane_swapped<0xB1>(part);   // lane ^ 1
-                    part += lane_swapped<0x4E>(part);   // lane ^ 2
-                    part += lane_swapped<0x141>(part);  // the other four of eight
-                    if (NCH == 16) part += lane_swapped<0x140>(part);  // the other eight of sixteen
+                    part += lane_moved<0xB1>(part);   // lane ^ 1
+                    part += lane_moved<0x4E>(part);   // lane ^ 2
+                    part += lane_moved<0x141>(part);  // the other four of eight
+                    if (NCH == 16) part += lane_moved<0x140>(part);  // the other eight of sixteen
                     if (ch == 0) dl_s[slot][row] = part;
                 }
             }

@@ -123,12 +123,6 @@ __device__ inline float weight_of(float s, float scale, float cexp, float nl) {
     return __builtin_amdgcn_exp2f(EXACT ? fmaf(s, scale, nl) * LOG2E : fmaf(s, cexp, nl));
 }
 
-// x of another lane of the same sixteen, by the DPP control word
-template <int CTRL>
-__device__ inline float lane_swapped(float x) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
-}
-
 // sum + the products of eight elements, in order
 __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
     const u32x4 xv = *reinterpret_cast<const u32x4*>(&x);
@@ -564,9 +558,9 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 #pragma unroll
             for (int i = 0; i < Mover<D, G, BMQ>::CPT; ++i) {
                 float part = add_products(*reinterpret_cast<const bf16x8*>(&mo.r[i]), *reinterpret_cast<const bf16x8*>(&mg.r[i]), 0.0f);
-                part += lane_swapped<0xB1>(part);  // lane ^ 1
-                part += lane_swapped<0x4E>(part);  // lane ^ 2
-                if (D == 64) part += lane_swapped<0x141>(part);  // the other four of eight
+                part += lane_moved<0xB1>(part);  // lane ^ 1
+                part += lane_moved<0x4E>(part);  // lane ^ 2
+                if (D == 64) part += lane_moved<0x141>(part);  // the other four of eight
                 if (gt % (D / 8) == 0) reinterpret_cast<float*>(t + 2 * BMQ * S)[BMQ + (gt + G * i) / (D / 8)] = FROM_DELTA<D, EXACT> ? -part : part;
             }
             if (gt >= BMQ) return;

@@ -343,11 +343,6 @@ __global__ void ew_silu_mul_bwd(const T* gate, const T* up, const T* dy, T* dgat
     }
 }
 
-// x of another lane of the same sixteen, by the DPP control word
-template <int CTRL>
-__device__ inline float lane_moved(float x) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
-}
 // x of all lanes added up, halves first (lane ^ 32, 16, 8, 4, 2, 1): in registers, where six exchanges through the LDS unit are 0.3 us. All lanes
 // of the wavefront are active. From the third step on the sums repeat every 16, 8, ... lanes, so a rotation is an exchange.
 __device__ inline float wave_sum(float x) {

@@ -44,6 +44,11 @@ __device__ inline float xhalf_sum(float x) {
     auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// x of another lane of the same sixteen, by the DPP control word
+template <int CTRL>
+__device__ inline float lane_moved(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
 
 // Two fp32 -> packed bf16 (v_cvt_pk_bf16_f32, round to nearest even).
 __device__ inline uint32_t pack_bf16(float lo, float hi) {
