@@ -298,6 +298,15 @@ def seen(T, key, causal, window, sinks):
 RANGE_CASES = [((24, 200, 8, 8, True, 0, 0), 64), ((5, 4096, 4, 4, True, 0, 0), 64), ((13, 511, 16, 8, False, 0, 0), 96), ((12, 383, 8, 8, True, 37, 5), 32),
                ((20, 161, 11, 11, True, 0, 0), 128), ((7, 577, 16, 8, True, 0, 0), 44), ((10, 1411, 8, 8, True, 33, 9), 64), ((1, 2500, 14, 2, True, 0, 0), 64),
                ((3, 1100, 16, 4, True, 0, 0), 100)]
+# ... and the joined launch of the backward above 64 columns
+RANGE_CASES += [((3, 577, 8, 8, False, 0, 0), 96), ((4, 640, 8, 8, True, 0, 0), 96), ((6, 321, 9, 9, True, 33, 17), 96),
+                ((3, 577, 8, 8, False, 0, 0), 128), ((2, 577, 19, 19, True, 0, 0), 128), ((6, 321, 9, 9, True, 33, 17), 128)]
+
+
+def test_range_cases_reach_every_form_of_the_backward():
+    forms = {(bwd_form(case, dk, torch.float32), max(32, (dk + 31) // 32 * 32), case[4]) for case, dk in RANGE_CASES}
+    assert {f[:2] for f in forms} >= {("APART", d) for d in (64, 96, 128)} | {("F32_PARTS", d) for d in (64, 96, 128)} | {("F32_PARTS_ALL", d) for d in (32, 96, 128)}
+    assert {("F32_PARTS", 96, False), ("F32_PARTS", 128, False)} <= forms
 
 
 @pytest.mark.parametrize("case,dk", RANGE_CASES, ids=str)
@@ -437,9 +446,12 @@ def test_backward_in_one_launch(case, dtype, dk):
 @pytest.mark.parametrize("dk", [4, 32, 44, 64, 80, 96, 100, 128])
 @pytest.mark.parametrize("case", [(18, 33, 16, 16, True, 0, 0), (7, 65, 16, 8, True, 0, 0), (9, 129, 14, 2, True, 0, 0), (2, 641, 13, 13, True, 0, 0),
                                   (5, 577, 8, 8, False, 0, 0), (1, 2113, 8, 2, True, 0, 0), (40, 257, 3, 3, True, 0, 0), (6, 321, 9, 9, True, 33, 17),
-                                  (1, 1100, 11, 11, True, 100, 0), (8, 471, 6, 6, True, 91, 4)], ids=str)
+                                  (1, 1100, 11, 11, True, 100, 0), (8, 471, 6, 6, True, 91, 4), (7, 129, 14, 2, True, 0, 0), (3, 577, 8, 8, False, 0, 0),
+                                  (20, 257, 3, 3, True, 0, 0)], ids=str)
 def test_fp32_backward_of_joined_blocks(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
+    past = dk > 64 and case[:2] in ((9, 129), (5, 577), (40, 257))  # the sizes past the last one that goes together
+    assert bwd_form(case, dk, torch.float32).startswith("APART" if past else "F32_PARTS")
     gen = torch.Generator(device="cuda").manual_seed(T + dk)
     cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
     q, k, v = cut(torch.randn((B, T, Hq + 2 * Hkv, dk), generator=gen, device="cuda"))
@@ -459,9 +471,11 @@ def test_fp32_backward_of_joined_blocks(case, dk):
 @pytest.mark.parametrize("dk", [8, 32, 40, 64, 80, 96])
 @pytest.mark.parametrize("case", [(17, 33, 16, 16, True, 0, 0), (9, 65, 16, 8, True, 0, 0), (13, 129, 8, 8, False, 0, 0), (11, 193, 14, 2, True, 0, 0),
                                   (5, 577, 9, 3, True, 0, 0), (2, 1025, 16, 4, True, 0, 0), (3, 700, 9, 9, False, 0, 0), (9, 321, 9, 9, True, 33, 17),
-                                  (2, 1100, 12, 12, True, 100, 0)], ids=str)
+                                  (2, 1100, 12, 12, True, 100, 0), (1, 1025, 36, 9, True, 0, 0), (4, 700, 9, 9, False, 0, 0)], ids=str)
 def test_bf16_backward_of_joined_blocks(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
+    below = (dk < 64 and case[:2] == (2, 1025)) or (dk > 64 and case[:2] == (3, 700))  # sizes below the first one that goes together
+    assert bwd_form(case, dk, torch.bfloat16) == ("APART" if below else "SPLIT_JOINED")
     gen = torch.Generator(device="cuda").manual_seed(T + dk)
     cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
     q, k, v = cut(torch.randn((B, T, Hq + 2 * Hkv, dk), generator=gen, device="cuda").bfloat16())
@@ -501,9 +515,10 @@ def test_joined_blocks_round_dp_as_the_launches_do(case):
 @pytest.mark.parametrize("grad", [torch.bfloat16, torch.float32], ids=str)
 @pytest.mark.parametrize("case", [(9, 33, 9, 9, True, 0, 0), (11, 65, 5, 5, False, 0, 0), (13, 129, 9, 9, True, 0, 0), (4, 577, 7, 7, True, 0, 0), (3, 700, 6, 6, False, 0, 0),
                                   (1, 1793, 12, 12, True, 0, 0), (6, 321, 9, 9, True, 33, 17), (1, 4200, 3, 3, True, 100, 0), (3, 161, 28, 4, True, 0, 0),
-                                  (1, 700, 14, 2, False, 0, 0), (2, 450, 16, 4, True, 60, 0)], ids=str)
+                                  (1, 700, 14, 2, False, 0, 0), (2, 450, 16, 4, True, 60, 0), (1, 450, 16, 4, True, 60, 0), (2, 450, 8, 4, True, 60, 0)], ids=str)
 def test_bf16_backward_of_joined_blocks_at_128(case, grad):
     B, T, Hq, Hkv, causal, window, sinks = case
+    assert bwd_form(case, 128, torch.bfloat16) == ("APART" if case[:3] == (2, 450, 16) else "JOINED")  # (its group of four is not dealt out)
     gen = torch.Generator(device="cuda").manual_seed(T)
     cut = lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:])  # noqa: E731
     q, k, v = cut(torch.randn((B, T, Hq + 2 * Hkv, 128), generator=gen, device="cuda").bfloat16())
