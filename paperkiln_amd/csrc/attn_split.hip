@@ -139,9 +139,9 @@ __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
 // rounded at delta's size four times instead of once, which dS, one bf16 operand there, does not show: errors of dQ and dK against
 // float64 are 1.63e-3 to 1.79e-3 of their norms and the same to four digits either way over 28 inputs, V with a mean of 30 standard
 // deviations among them. Not where P and dS keep all their bits (EXACT), nor at 128 columns, where it spilled 30 registers more; dQ not where
-// four wavefronts share the tiles (T 1661, 16 heads 21.5 us | 24.5), nor in the joined launch, whose sizes came from that form: where V is the same
-// in every row dS is zero and dQ the rounding of dP alone, two to three times as much from -delta (joined launch from zero, us: T 512 x 16, 8 heads
-// 34.4 -> 34.3, T 470 x 8, 8 heads 20.4 -> 20.7, T 1024 x 8 50.3 -> 51.2, T 4945 133.3 -> 135.8).
+// four wavefronts share the tiles (T 1661, 16 heads 21.5 us | 24.5), nor in the joined launch for sizes whose dQ by itself is not: where V is the
+// same in every row dS is zero and dQ the rounding of dP alone, two to three times as much from -delta (joined launch, from -delta | from zero, us:
+// T 470 x 8, 8 heads 20.1 | 20.4, T 1024 x 8 50.1 | 50.9, T 1661, 16 heads 45.5 | 46.4).
 template <int D, bool EXACT>
 constexpr bool FROM_DELTA = !EXACT && D == 64;
 
@@ -700,7 +700,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, in
 // ---- the same of wavefronts that own their rows (split_takes_joined) ----
 // dK/dV forms delta from the chunks of O beside those of dO while it moves a tile (up to 64 columns, whose chunks are in 4 or 8 neighbouring
 // lanes; above, it is read): a launch of delta before this one cost 4 us more, of 13 to 60.
-template <int D, bool EXACT>
+template <int D, bool EXACT, bool MINUS_DELTA>
 __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     all_arguments(a);
     constexpr bool OWN_DELTA = D <= 64;
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     if (!jb.map(a, rank, r, kvu)) return;
     if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA>(a, rank, r, kvu, lds);
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
-    dq_block<D, 4, 1, 2, EXACT, false>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    dq_block<D, 4, 1, 2, EXACT, MINUS_DELTA>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of
@@ -1031,9 +1031,9 @@ bool split_takes_joined(const AttnArgs& a) {
     if (!a.causal && n > 8 && a.Hq > a.Hkv) return false;
     return u >= (n == 1 ? 80 : n <= 5 ? 150 : n <= 12 ? 200 : 232) && u <= (a.causal ? 420 : a.T <= 64 ? 380 : 400);
 }
-template <int D, bool EXACT>
+template <int D, bool EXACT, bool MINUS_DELTA = false>
 int joined_of(const AttnArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL((split_joined<D, EXACT>), dim3(JoinedBlocks(a, 128).grid(a)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((split_joined<D, EXACT, MINUS_DELTA>), dim3(JoinedBlocks(a, 128).grid(a)), dim3(256), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -1044,7 +1044,10 @@ int launch_split_joined(const AttnArgs& a_in, hipStream_t st) {
     if (a.dk_dim > 64)
         if (const int rc = launch_row_delta(a, true, st)) return rc;
     const auto run = [&]() -> int {
-        if (a.dk_dim == 64) return joined_of<64, false>(a, st);
+        if (a.dk_dim == 64) {
+            const Form alone = dq_form(a);
+            return alone == Form::NONE || alone == Form::FOUR ? joined_of<64, false>(a, st) : joined_of<64, false, true>(a, st);
+        }
         if (a.dk_dim <= 32) return joined_of<32, true>(a, st);
         if (a.dk_dim <= 64) return joined_of<64, true>(a, st);
         return joined_of<96, true>(a, st);
