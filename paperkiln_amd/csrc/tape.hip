@@ -822,9 +822,13 @@ Var embedding_of(const Var& table, const std::shared_ptr<Buffer>& ids, Tensor ro
     return record(std::move(rows), {table}, [ids](Variable* self) {
         const Var& t = self->parents[0];
         if (!t->requires_grad) return;
-        // a model's embedding is the last node of a pass: the sums held until then go with it
-        std::vector<HeldSum> held = held_sums();
-        if (k_embedding_bwd(self->grad, static_cast<const int*>(ids->p), t->ensure_grad(), held.data(), static_cast<int>(held.size())))
+        // a model's embedding is the last node of a pass: the sums held until then go with it, but for a table of one row that is a
+        // norm's weight as well and must not meet itself in one launch
+        bool again = false;
+        for (const auto& s : pending().sums) again = again || s.w.get() == t.get();
+        std::vector<HeldSum> held;
+        if (!again) held = held_sums();
+        if (k_embedding_bwd(self->grad, static_cast<const int*>(ids->p), t->ensure_grad(), again ? nullptr : held.data(), static_cast<int>(held.size())))
             pending().sums.clear();
     });
 }

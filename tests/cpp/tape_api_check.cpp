@@ -257,6 +257,37 @@ void shared_gradient_case(int dtype, const char* name, double tol) {
     }
 }
 
+// A table of one row that is a norm's weight as well: its two gradients, of which one is held to the end of the pass, both arrive.
+void table_as_gain_case() {
+    std::printf("one row as embedding table and as norm weight\n");
+    const int T = 64, d = 1024;
+    const auto hw = draw(d, 47, 1.0);
+    std::vector<int> target(T);
+    for (int i = 0; i < T; ++i) target[i] = (13 * i + 5) % d;
+    auto tg = device_ints(target), ids = device_ints(std::vector<int>(T, 0));
+    auto leaf = [&] {
+        pk::Var w = pk::make_var(pk::upload(hw.data(), 1, d), true);
+        w->is_param = true;
+        return w;
+    };
+    auto pass = [&](const pk::Var& table, const pk::Var& gain) {
+        pk::backward(pk::ops::cross_entropy(pk::ops::rmsnorm(pk::ops::embedding(table, ids, T), gain), tg));
+    };
+    const pk::Var table = leaf(), gain = leaf(), both = leaf();
+    pass(table, gain);
+    pass(both, both);
+    const auto gt = host(table->grad), gg = host(gain->grad), gb = host(both->grad);
+    double w = 0.0, size_e = 0.0, size_g = 0.0;
+    for (int i = 0; i < d; ++i) {
+        w = std::fmax(w, std::fabs(static_cast<double>(gb[i]) - (static_cast<double>(gt[i]) + gg[i])));
+        size_e = std::fmax(size_e, std::fabs(gt[i]));
+        size_g = std::fmax(size_g, std::fabs(gg[i]));
+    }
+    check(size_e > 1e-4 && size_g > 1e-4, "neither gradient is zero", std::fmin(size_e, size_g));
+    // one of the two is added to the other's finished sum or the sum goes on from it: T + 1 roundings at most
+    check(w <= (T + 1) * 6e-8 * (size_e + size_g), "gradient = of the table + of the weight", w);
+}
+
 // r + x W with the add inside the product's epilogue (bf16) against the two ops it stands for; edge tiles in both
 // directions, and a contraction long enough for the two-wavefront-set form of the kernel.
 void linear_add_case(int dtype, const char* name, int T, int din, int dout, double tol) {
@@ -513,6 +544,7 @@ int main() {
     checkpoint_case();
     shared_gradient_case(PK_F32, "float32", 1e-6);
     shared_gradient_case(PK_BF16, "bfloat16 (the fused row kernel)", 1.0 / 128);
+    table_as_gain_case();
     linear_add_case(PK_F32, "float32 (product, then add)", 40, 24, 16, 1e-6);
     linear_add_case(PK_BF16, "bfloat16, edge tiles", 200, 72, 136, 1.0 / 128);
     linear_add_case(PK_BF16, "bfloat16, long contraction", 300, 1376, 64, 1.0 / 128);
