@@ -139,9 +139,11 @@ __device__ inline float add_products(bf16x8 x, bf16x8 y, float sum) {
 // rounded at delta's size four times instead of once, which dS, one bf16 operand there, does not show: errors of dQ and dK against
 // float64 are 1.63e-3 to 1.79e-3 of their norms and the same to four digits either way over 28 inputs, V with a mean of 30 standard
 // deviations among them. Not where P and dS keep all their bits (EXACT), nor at 128 columns, where it spilled 30 registers more; dQ not where
-// four wavefronts share the tiles (T 1661, 16 heads 21.5 us | 24.5), nor in the joined launch for sizes whose dQ by itself is not: where V is the
-// same in every row dS is zero and dQ the rounding of dP alone, two to three times as much from -delta (joined launch, from -delta | from zero, us:
-// T 470 x 8, 8 heads 20.1 | 20.4, T 1024 x 8 50.1 | 50.9, T 1661, 16 heads 45.5 | 46.4).
+// four wavefronts share the tiles (T 1661, 16 heads 21.5 us | 24.5), nor dQ or dK/dV in the joined launch for sizes whose launch of it alone is
+// another kernel, which subtracts delta at the end: where V is the same in every row dS is zero and dQ and dK are the rounding of dP alone, two to
+// four times as much from -delta (dK, T 150 x 4, 16 heads 1.9e-3 | 5.3e-4, alone 4.4e-4; T 64 x 31, 4 heads 3.1e-3 | 8.5e-4, alone 1.5e-3). Joined launch, from
+// -delta | from zero, us: dQ, T 470 x 8, 8 heads 20.1 | 20.4, T 1024 x 8 50.1 | 50.9, T 1661, 16 heads 45.5 | 46.4; dK/dV, T 470 x 8 19.1 | 19.5, T 923
+// x 7, 4 heads 29.4 | 30.1, T 150 x 4 9.5 | 9.6; 1.007 over 60 shapes, one by 4 % (subtracted behind dV's product 1.014, one by 7).
 template <int D, bool EXACT>
 constexpr bool FROM_DELTA = !EXACT && D == 64;
 
@@ -481,11 +483,13 @@ constexpr int dkdv_lds() {  // in uint16; LSE and delta of a tile's rows behind 
     constexpr int TILES = (QW > 1 ? 2 : 1) * KW * (2 * 32 * NB * (D + 8) + 128 * NB), RED = KW > 1 ? QW * KW * (D / 32) * (JOIN_BOTH<D> ? 4096 : 2048) : 0;
     return TILES > RED ? TILES : RED;
 }
-template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA>
+template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA, bool MINUS_DELTA = FROM_DELTA<D, EXACT>>
 __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, uint16_t* lds) {
     // a lane holds the row of O whose row of dO its wavefront has just written; or the chunks of O beside its chunks of dO
     static_assert(!OWN_DELTA || (QW == 1 && NB == 1) || (QW > 1 && (D == 32 || D == 64)), "a row's chunks are in 4 or 8 neighbouring lanes");
     constexpr bool BY_ROW = OWN_DELTA && QW == 1, BY_CHUNK = OWN_DELTA && QW > 1;
+    // where dP does not start from -delta: it is subtracted behind dV's product, or, where the kernel's other form starts from it, at once
+    constexpr bool LATE = !FROM_DELTA<D, EXACT>;
     constexpr int BNK = 32 * QW, BMQ = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int ROWC = 2 * BMQ * 2;                    // LSE and delta of a tile's rows, in uint16
     constexpr int TILE = 2 * BMQ * S + ROWC, NBUF = QW > 1 ? 2 : 1;
@@ -553,7 +557,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
         uint16_t* t = lds + (buf % NBUF * KW + kg) * TILE;
         mq.template store<true>(t, S, gt);
         mg.template store<true>(t + BMQ * S, S, gt);
-        float out = gt >= BMQ ? (FROM_DELTA<D, EXACT> ? -row_r : row_r) : EXACT ? -row_r : -row_r * LOG2E;
+        float out = gt >= BMQ ? (MINUS_DELTA ? -row_r : row_r) : EXACT ? -row_r : -row_r * LOG2E;
         if constexpr (BY_CHUNK) {
 #pragma unroll
             for (int i = 0; i < Mover<D, G, BMQ>::CPT; ++i) {
@@ -561,7 +565,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                 part += lane_moved<0xB1>(part);  // lane ^ 1
                 part += lane_moved<0x4E>(part);  // lane ^ 2
                 if (D == 64) part += lane_moved<0x141>(part);  // the other four of eight
-                if (gt % (D / 8) == 0) reinterpret_cast<float*>(t + 2 * BMQ * S)[BMQ + (gt + G * i) / (D / 8)] = FROM_DELTA<D, EXACT> ? -part : part;
+                if (gt % (D / 8) == 0) reinterpret_cast<float*>(t + 2 * BMQ * S)[BMQ + (gt + G * i) / (D / 8)] = MINUS_DELTA ? -part : part;
             }
             if (gt >= BMQ) return;
         }
@@ -571,7 +575,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) part = add_products(oreg[kk], lds_read8(t + BMQ * S + tile_row<D>(c32) * S + kk * 16 + g * 8), part);
             part = xhalf_sum(part);
-            if (g == 1) out = FROM_DELTA<D, EXACT> ? -part : part;
+            if (g == 1) out = MINUS_DELTA ? -part : part;
         }
         if (gt < 2 * BMQ) reinterpret_cast<float*>(t + 2 * BMQ * S)[gt] = out;
     };
@@ -604,7 +608,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
                 f32x4 dl = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (FROM_DELTA<D, EXACT>) dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
+                if (MINUS_DELTA) dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = dl[e];
             }
@@ -612,6 +616,15 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
             for (int kk = 0; kk < KK; ++kk) s = mfma32(lds_read8(Qs + (nb * 32 + tile_row<D>(c32)) * S + kk * 16 + g * 8), kreg[kk], s);
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) dp = mfma32(lds_read8(Gs + (nb * 32 + tile_row<D>(c32)) * S + kk * 16 + g * 8), vreg[kk], dp);
+            if (!MINUS_DELTA && !LATE) {
+                f32x4 dl[4];  // all asked for before any is used: one by one 1.015 over the 60 shapes
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) dl[qd] = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dp[qd * 4 + e] -= dl[qd][e];
+            }
             // lane = key kj; element r = query qlo + (r/4)*8 + 4g + r%4
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
@@ -627,9 +640,9 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
                 f32x4 dl = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (!FROM_DELTA<D, EXACT>) dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
+                if (LATE) dl = *reinterpret_cast<const f32x4*>(rows + BMQ + nb * 32 + qd * 8 + g * 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (FROM_DELTA<D, EXACT> ? dp[qd * 4 + e] : dp[qd * 4 + e] - dl[e]);
+                for (int e = 0; e < 4; ++e) dp[qd * 4 + e] = s[qd * 4 + e] * (LATE ? dp[qd * 4 + e] - dl[e] : dp[qd * 4 + e]);
             }
             accumulate_tr<D, EXACT ? BWD_PARTS : 1, true>(Qs, S, nb * 32, dp, acc + DB, lane);
         }
@@ -700,7 +713,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, in
 // ---- the same of wavefronts that own their rows (split_takes_joined) ----
 // dK/dV forms delta from the chunks of O beside those of dO while it moves a tile (up to 64 columns, whose chunks are in 4 or 8 neighbouring
 // lanes; above, it is read): a launch of delta before this one cost 4 us more, of 13 to 60.
-template <int D, bool EXACT, bool MINUS_DELTA>
+template <int D, bool EXACT, bool DQ_MINUS, bool DKDV_MINUS>
 __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     all_arguments(a);
     constexpr bool OWN_DELTA = D <= 64;
@@ -709,9 +722,9 @@ __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     const JoinedBlocks jb(a, 128);
     int rank, r, kvu;
     if (!jb.map(a, rank, r, kvu)) return;
-    if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA>(a, rank, r, kvu, lds);
+    if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA, DKDV_MINUS>(a, rank, r, kvu, lds);
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
-    dq_block<D, 4, 1, 2, EXACT, MINUS_DELTA>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    dq_block<D, 4, 1, 2, EXACT, DQ_MINUS>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of
@@ -1031,9 +1044,9 @@ bool split_takes_joined(const AttnArgs& a) {
     if (!a.causal && n > 8 && a.Hq > a.Hkv) return false;
     return u >= (n == 1 ? 80 : n <= 5 ? 150 : n <= 12 ? 200 : 232) && u <= (a.causal ? 420 : a.T <= 64 ? 380 : 400);
 }
-template <int D, bool EXACT, bool MINUS_DELTA = false>
+template <int D, bool EXACT, bool DQ_MINUS = false, bool DKDV_MINUS = false>
 int joined_of(const AttnArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL((split_joined<D, EXACT, MINUS_DELTA>), dim3(JoinedBlocks(a, 128).grid(a)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((split_joined<D, EXACT, DQ_MINUS, DKDV_MINUS>), dim3(JoinedBlocks(a, 128).grid(a)), dim3(256), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -1046,7 +1059,9 @@ int launch_split_joined(const AttnArgs& a_in, hipStream_t st) {
     const auto run = [&]() -> int {
         if (a.dk_dim == 64) {
             const Form alone = dq_form(a);
-            return alone == Form::NONE || alone == Form::FOUR ? joined_of<64, false>(a, st) : joined_of<64, false, true>(a, st);
+            const bool dkdv = split_takes_dkdv(a_in) || mfma_dkdv3_takes(a_in);
+            if (alone == Form::NONE || alone == Form::FOUR) return dkdv ? joined_of<64, false, false, true>(a, st) : joined_of<64, false>(a, st);
+            return dkdv ? joined_of<64, false, true, true>(a, st) : joined_of<64, false, true>(a, st);
         }
         if (a.dk_dim <= 32) return joined_of<32, true>(a, st);
         if (a.dk_dim <= 64) return joined_of<64, true>(a, st);
