@@ -279,10 +279,11 @@ __global__ __launch_bounds__(G::NTHR, 2) void gemm_bf16(GemmArgs g) {
 // loads have one slice of matrix work to hide behind, 512 clocks against a round trip of 1,500 - 2,000, and a loop
 // that spends four scalar instructions per matrix instruction on addresses and branches is bound by instruction
 // issue. Here the operand slices go from memory straight into LDS (buffer_load_dwordx4 ... lds: no staging
-// registers, no LDS stores, a lane outside the buffer writes zeros), into a ring of NS slots; the loads of slice
-// s + NS - 1 are issued before slice s is multiplied; a tile's buffer descriptors are formed once and the position
+// registers, no LDS stores, a lane outside the buffer writes zeros), into a ring of NS slots; a slot is asked for anew
+// as soon as its slice's last fragments are in registers; a tile's buffer descriptors are formed once and the position
 // in the contraction is the instruction's scalar offset (which the hardware counts in its range check); the slice
-// loop is unrolled over the ring, so every LDS address is a register formed once plus an immediate.
+// loop is unrolled over the ring, so every LDS address is a register formed once plus an immediate. The result leaves
+// through a strip of LDS beside the ring, so the next tile's slices keep coming meanwhile.
 //
 // One load instruction fills 1 KB of LDS lane after lane, so a lane's place in LDS is fixed and what varies is which
 // 16 bytes of memory it fetches. The tiles are therefore not padded but swizzled:
@@ -386,16 +387,30 @@ struct TileStore {
     static_assert(SR * CPR % G::NTHR == 0 && G::NTHR % CPR == 0, "whole stores per thread, one chunk column per thread");
     static constexpr int PER_PHASE = SR * CPR / G::NTHR;
     static constexpr int NST = PHASES * PER_PHASE;
-    static constexpr int CP = G::BN + EPC;  // strip pitch in elements: rows stay 16-byte aligned, writes conflict-free
-    static constexpr int BYTES = SR * CP * (CF32 ? 4 : 2);
+    static constexpr int BYTES = SR * CPR * 16;
+    // Place of column `col` of strip row `row`, in elements: rows are not padded (the strip lies beside the ring, and the two fill the
+    // LDS to the byte), chunks are dealt over the banks by the row instead, two lanes of a half-wavefront to a bank as padding has it.
+    __device__ static int at(int row, int col) { return row * G::BN + ((col / EPC) ^ (row & 31 & (CPR - 1))) * EPC + col % EPC; }
+};
+// LDS of a ring kernel: NS slots of one slice of both operands and, beside them, a strip of the result on its way out (or half of the
+// second wavefront set's sums).
+template <typename G, int NS>
+struct RingLds {
+    static constexpr int SLOT = (G::BM + G::BN) * BK * 2;
+    static constexpr int SUMS = G::KS == 1 ? 0 : G::WGM * G::WGN * 64 * (G::FM / 2) * G::FN * 64;
+    static constexpr int STRIP = TileStore<G, false>::BYTES > SUMS ? TileStore<G, false>::BYTES : SUMS;
+    static_assert(TileStore<G, true>::BYTES <= STRIP, "both result types' strips");
+    static constexpr int BYTES = NS * SLOT + STRIP;
+    static_assert(NS >= 2 && BYTES <= 160 * 1024, "the ring and the strip must fit the LDS");
+    static constexpr int PER_CU = BYTES <= 80 * 1024 ? 2 : 1;
 };
 
 // C = op(A) op(B), persistent: gridDim.x workgroups walk the virtual blocks v = blockIdx.x, + gridDim.x, ...
 // (virtual block -> (contraction slice, tile) as gemm_bf16 maps (blockIdx.z, blockIdx.x), XCD by XCD), and the ring
 // runs on across tile boundaries: the first slices of the next tile are on their way while the last ones of this tile
 // are multiplied and its result is stored, so a tile's first round trip to memory is paid once per workgroup.
-template <typename G, bool TA, bool TB, bool CF32, int NS, bool SPREAD, int EPI = 0>
-__global__ __launch_bounds__(G::NTHR, NS * (RingOp<TA, G::BM, G::NTHR / 64>::BYTES + RingOp<!TB, G::BN, G::NTHR / 64>::BYTES) <= 80 * 1024 ? 2 : 1)
+template <typename G, bool TA, bool TB, bool CF32, int NS, int EPI = 0>
+__global__ __launch_bounds__(G::NTHR, (RingLds<G, NS>::PER_CU))
 void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     static_assert(EPI == 0 || EPI == 3 || (G::KS == 1 && !CF32), "the head's epilogues: one wavefront set, bf16 result");
     constexpr bool GROUPED = EPI == 3;
@@ -410,14 +425,15 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     constexpr int SLOT = OA::BYTES + OB::BYTES, PERTOT = OA::PER + OB::PER;
     constexpr int BNC = GATE ? BN / 2 : BN;  // columns of C per tile
     constexpr int NST = EPI == 5 ? ST::NST / 2 * 3 : EPI == 6 ? ST::NST / 2 : EPI == 7 ? ST::NST * 2 : ST::NST;
-    static_assert(NS >= 2 && NS * SLOT <= 160 * 1024, "the ring must fit the LDS");
-    static_assert(ST::BYTES <= SLOT, "an epilogue strip must fit one ring slot");
+    using RL = RingLds<G, NS>;
+    static_assert(SLOT == RL::SLOT, "a slice of both operands");
     static_assert((NS - 2) * PERTOT + NST < 64, "memory operations in flight must fit the counter");
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * SLOT];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[RL::BYTES];
+    uint8_t* const strip = lds + NS * SLOT;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int KS = G::KS, NWQ = G::WGM * G::WGN, KPW = BK / 16 / KS;  // k-chunks of a slice per wavefront
     static_assert(KS == 1 || KS == 2, "one or two wavefront sets");
-    static_assert(KS == 1 || (FM % 2 == 0 && NWQ * 64 * (FM / 2) * FN * 64 <= SLOT), "half of the second set's sums per slot");
+    static_assert(KS == 1 || FM % 2 == 0, "half of the second set's sums at a time");
     const int ks = KS == 1 ? 0 : w / NWQ, wq = w - ks * NWQ;
     const int c32 = lane & 31, gh = lane >> 5, wm = wq / G::WGN, wn = wq % G::WGN;
 
@@ -556,20 +572,9 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             open();
         }
     };
-    auto fetch_pieces = [&](auto first, auto count) {  // pieces first .. first + count - 1
-        constexpr int F = decltype(first)::value, N = decltype(count)::value;
-        if constexpr (N > 0) {
-            fetch_piece(std::integral_constant<int, F>{});
-            if constexpr (N > 1) fetch_piece(std::integral_constant<int, F + 1>{});
-            if constexpr (N > 2) fetch_piece(std::integral_constant<int, F + 2>{});
-            if constexpr (N > 3) fetch_piece(std::integral_constant<int, F + 3>{});
-            static_assert(N <= 4, "at most four pieces per k-chunk");
-        }
-    };
     auto fetch = [&](int slot) {  // the whole slice at once (before the first slice is multiplied)
         fetch_begin(slot);
-        fetch_pieces(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
-        if constexpr (PERTOT > 4) fetch_pieces(std::integral_constant<int, 4>{}, std::integral_constant<int, PERTOT - 4>{});
+        static_for<0, PERTOT>([&](auto pc) { fetch_piece(pc); });
         fetch_end();
     };
 
@@ -706,7 +711,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
                 const u32x2 v = {pack_bf16(acc[i][j][qd * 4], acc[i][j][qd * 4 + 1]), pack_bf16(acc[i][j][qd * 4 + 2], acc[i][j][qd * 4 + 3])};
-                *reinterpret_cast<u32x2*>(cs + (wm * 32 + c32) * ST::CP + (wn * FN + j) * 32 + qd * 8 + gh * 4) = v;
+                *reinterpret_cast<u32x2*>(cs + ST::at(wm * 32 + c32, (wn * FN + j) * 32 + qd * 8 + gh * 4)) = v;
             }
     };
     // descriptor of a [M, ld] matrix from the tile's first element on, `cols` columns from there to the last row's end
@@ -716,7 +721,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
         return u32x4{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32) & 0xffffu, left > 0x7ffffff0 ? 0x7ffffff0u : static_cast<uint32_t>(left),
                      0x00020000u};
     };
-    auto store_gated = [&](uint8_t* strip, const Block& bl) {
+    auto store_gated = [&](const Block& bl) {
         constexpr int GPR = ST::CPR / 2;  // chunks of gate in a strip row; each with its chunk of up four further on
         static_assert(NTHR % GPR == 0 && ST::SR * GPR % NTHR == 0, "one chunk column per thread, whole rounds of rows");
         const int q = static_cast<int>(threadIdx.x) % GPR, cg = (q >> 2) * 8 + (q & 3), col = gated_column(cg);
@@ -731,8 +736,8 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
             for (int k = 0; k < ST::SR * GPR / NTHR; ++k) {
                 const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / GPR, trow = (srow >> 5) * FM * 32 + (srow & 31);
-                const u32x4 gate = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + cg * 8),
-                            up = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + cg * 8 + 32);
+                const u32x4 gate = *reinterpret_cast<const u32x4*>(cs + ST::at(srow, cg * 8)),
+                            up = *reinterpret_cast<const u32x4*>(cs + ST::at(srow, cg * 8 + 32));
                 u32x4 v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = pack_bf16(gated(lo(gate[e]), lo(up[e])), gated(hi(gate[e]), hi(up[e])));
@@ -746,7 +751,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             __syncthreads();
         }
     };
-    auto store_gated_grad = [&](uint8_t* strip, const Block& bl) {
+    auto store_gated_grad = [&](const Block& bl) {
         const u32x4 to_c = tile_rsrc(g.c, bl, 2 * g.N, 2 * g.N - bl.n0), gu = tile_rsrc(g.d, bl, 2 * g.N, 2 * g.N - bl.n0);
         const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint16_t*>(static_cast<const uint16_t*>(g.d) + static_cast<int64_t>(bl.m0) * 2 * g.N + bl.n0), 0, static_cast<int>(gu[2]), 0x00020000);
@@ -766,7 +771,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
             for (int k = 0; k < ST::PER_PHASE; ++k) {
                 const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / ST::CPR;
-                const u32x4 d = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + st_ch * 8);
+                const u32x4 d = *reinterpret_cast<const u32x4*>(cs + ST::at(srow, st_ch * 8));
                 u32x4 dg, du;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -782,8 +787,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             __syncthreads();
         }
     };
-    // the tile's result, through the ring slot `strip` (which every wavefront has finished reading)
-    auto store_result = [&](uint8_t* strip, const Block& bl) {
+    auto store_result = [&](const Block& bl) {  // the tile's result, through the strip
         if (KS == 2) {  // set 1 hands its sums to set 0, half of them at a time: [wavefront][16-byte group][lane]
             f32x4* red = reinterpret_cast<f32x4*>(strip) + wq * ((FM / 2) * FN * 4) * 64 + lane;
 #pragma unroll
@@ -840,11 +844,11 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                         const int row = (CF32 ? 0 : wm * 32) + c32, col = (wn * FN + j) * 32 + qd * 8 + gh * 4;
                         if (CF32) {
                             const f32x4 v = {acc[i][j][qd * 4], acc[i][j][qd * 4 + 1], acc[i][j][qd * 4 + 2], acc[i][j][qd * 4 + 3]};
-                            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(cs) + row * ST::CP + col) = v;
+                            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(cs) + ST::at(row, col)) = v;
                         } else {
                             const u32x2 v = {pack_bf16(acc[i][j][qd * 4], acc[i][j][qd * 4 + 1]),
                                              pack_bf16(acc[i][j][qd * 4 + 2], acc[i][j][qd * 4 + 3])};
-                            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(cs) + row * ST::CP + col) = v;
+                            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(cs) + ST::at(row, col)) = v;
                         }
                     }
             }
@@ -854,7 +858,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
             for (int k = 0; k < ST::PER_PHASE; ++k) {
                 const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / ST::CPR;
-                u32x4 v = *reinterpret_cast<const u32x4*>(cs + srow * ST::CP + st_ch * ST::EPC);
+                u32x4 v = *reinterpret_cast<const u32x4*>(cs + ST::at(srow, st_ch * ST::EPC));
                 uint32_t off = coff[k];
                 if (GROUPED) {  // the row pitch is the problem's
                     const int trow = CF32 ? srow : (srow >> 5) * FM * 32 + (srow & 31);
@@ -882,71 +886,96 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     };
 
     // ---- the stream ----
+    // Rotated by a k-chunk: a chunk's matrix instructions run while the next chunk's fragments are read, and a slice's last chunk runs
+    // behind the barrier that hands out the next slice, whose first fragments are read meanwhile and whose slot's successor is asked
+    // for (half of its loads there, half beside the next slice's first chunk). Left to itself the compiler reads a chunk's fragments
+    // right in front of its matrix instructions, and a barrier drains both wavefronts of a SIMD. Microseconds so | now, whole launches:
+    // 4096^3 115 | 103, [32000, 512] over 4096 137 | 132, [4096, 512] over 32000 134 | 124, the head's first pass over 4096 x 32000 x 512
+    // 134 | 126, [8192, 1536] over 512 20.1 | 19.5. What is left is the loads' way into LDS and the clock: without them 4096^3 takes 82,
+    // with operands of zeros (no lower clock) 77, without the fragment reads 103 to 111. Not ahead: 256 x 256 tiles of four wavefronts,
+    // 128 x 128 each (half the fragment reads: level), slices of 32 in rings of 3 and 4 slots (117 | 107).
+    constexpr int NF = FM + FN, NM = FM * FN, HALF = PERTOT / 2;
+    static_assert(KPW % 2 == 0, "fragments of even and odd chunks in registers of their own");
+    bf16x8 fra[2][FM], frb[2][FN];
+    auto read_frag = [&](auto qc, auto kqc, const uint8_t* As) {  // fragment Q of chunk KQ, in the order the matrix instructions need them
+        constexpr int Q = decltype(qc)::value, KQ = decltype(kqc)::value, L = FM < FN ? FM : FN;
+        const uint8_t* Bs = As + OA::BYTES;
+        const int kk = ks * KPW + KQ;
+        if constexpr (Q < 2 * L && Q % 2 == 0)
+            frb[KQ & 1][Q / 2] = read_b(Bs, Q / 2, KQ, kk);
+        else if constexpr (Q < 2 * L)
+            fra[KQ & 1][Q / 2] = read_a(As, Q / 2, KQ, kk);
+        else if constexpr (FM > FN)
+            fra[KQ & 1][Q - L] = read_a(As, Q - L, KQ, kk);
+        else
+            frb[KQ & 1][Q - L] = read_b(Bs, Q - L, KQ, kk);
+    };
+    // the matrix instructions of chunk KQ, each behind a fragment of chunk KN (of the slice at `next`) and before a load of its share
+    auto chunk = [&](auto kqc, auto knc, const uint8_t* next, auto first, auto count) {
+        constexpr int KQ = decltype(kqc)::value, F = decltype(first)::value, N = decltype(count)::value;
+        static_for<0, NM>([&](auto mc) {
+            constexpr int Q = decltype(mc)::value, PERQ = (NF + NM - 1) / NM;
+            static_for<Q * PERQ, (Q + 1) * PERQ < NF ? (Q + 1) * PERQ : NF>([&](auto fc) { read_frag(fc, knc, next); });
+            acc[Q / FN][Q % FN] = mfma32(frb[KQ & 1][Q % FN], fra[KQ & 1][Q / FN], acc[Q / FN][Q % FN]);
+            static_for<F + Q * N / NM, F + (Q + 1) * N / NM>([&](auto pc) { fetch_piece(pc); });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    const auto keep_here = []() { asm volatile("" ::: "memory"); };  // reads above are not to move behind the branch below
     open();
     {
         int slot = 0;
         for (int s = 0; s < NS - 1; ++s) fetch(slot++);
     }
+    fetch_begin(NS - 1);
+    static_for<0, HALF>([&](auto pc) { fetch_piece(pc); });
     Block cb;  // compute side: the block in hand
     int cv = next_block(static_cast<int>(blockIdx.x), cb);
     int c_slice = 0, c_nslices = (cb.k_end - cb.k_begin + BK - 1) / BK;
-    int since_store = NS;  // waits since the last tile's stores were issued; below NS - 1 they are still counted
+    int since_store = NS;  // waits since the last tile's stores were issued; below NS - 2 they are still counted
     zero_acc();
+    wait_loads<(NS - 2) * PERTOT + HALF>();
+    barrier();
+    static_for<0, NF>([&](auto fc) { read_frag(fc, std::integral_constant<int, 0>{}, lds); });
     for (;;) {
         bool done = false;
 #pragma unroll
         for (int u = 0; u < NS; ++u) {
-            // Slice in hand landed: everything this wavefront issued after that slice's loads may still be in flight
-            // -- the loads of NS - 2 later slices and, for the NS - 1 slices asked for before the last tile's
-            // stores, those stores (memory operations complete in order).
-            if (since_store < NS - 1)
+            const uint8_t* const slice = lds + u * SLOT;
+            // the second half of the loads that the slice before began
+            chunk(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, slice, std::integral_constant<int, HALF>{},
+                  std::integral_constant<int, PERTOT - HALF>{});
+            keep_here();
+            fetch_end();
+            static_for<1, KPW - 1>([&](auto kc) {
+                constexpr int KQ = decltype(kc)::value;
+                chunk(kc, std::integral_constant<int, KQ + 1>{}, slice, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+            });
+            // The next slice landed: everything this wavefront issued after that slice's loads may still be in flight -- the loads of
+            // NS - 2 later slices and, for the slices asked for before the last tile's stores, those stores (memory operations
+            // complete in order). This slice's last fragments are in registers, so behind the barrier its slot is free.
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (NS > 2 && since_store < NS - 2)
                 wait_loads<(NS - 2) * PERTOT + NST>();
             else
                 wait_loads<(NS - 2) * PERTOT>();
             since_store = min(since_store + 1, NS);
-            barrier();                       // ... for every wavefront, and all have read the slice before
-            fetch_begin((u + NS - 1) % NS);  // slice + NS - 1 of the stream goes into the slot the slice before leaves
-            const uint8_t* As = lds + u * SLOT;
-            const uint8_t* Bs = As + OA::BYTES;
-            constexpr int SP = SPREAD ? KPW : 0;
-            constexpr int PPK = SP == 0 ? 0 : (PERTOT + SP - 1) / SP;  // loads dropped behind each k-chunk's matrix instructions
-            if constexpr (SP == 0) {
-                fetch_pieces(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
-                if constexpr (PERTOT > 4) fetch_pieces(std::integral_constant<int, 4>{}, std::integral_constant<int, PERTOT - 4>{});
-            }
-            auto chunk = [&](auto kqc) {
-                constexpr int KQ = decltype(kqc)::value;
-                const int kk = ks * KPW + KQ;
-                bf16x8 fa[FM], fbb[FN];
-#pragma unroll
-                for (int i = 0; i < FM; ++i) fa[i] = read_a(As, i, KQ, kk);
-#pragma unroll
-                for (int j = 0; j < FN; ++j) fbb[j] = read_b(Bs, j, KQ, kk);
-#pragma unroll
-                for (int i = 0; i < FM; ++i)
-#pragma unroll
-                    for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(fbb[j], fa[i], acc[i][j]);
-                constexpr int F = KQ * PPK, N = SP == 0 || F >= PERTOT ? 0 : (F + PPK <= PERTOT ? PPK : PERTOT - F);
-                fetch_pieces(std::integral_constant<int, F>{}, std::integral_constant<int, (N > 4 ? 4 : N)>{});
-                if constexpr (N > 4) fetch_pieces(std::integral_constant<int, F + 4>{}, std::integral_constant<int, N - 4>{});
-            };
-            chunk(std::integral_constant<int, 0>{});
-            if constexpr (KPW > 1) chunk(std::integral_constant<int, 1>{});
-            if constexpr (KPW > 2) chunk(std::integral_constant<int, 2>{});
-            if constexpr (KPW > 3) chunk(std::integral_constant<int, 3>{});
-            fetch_end();
+            barrier();
+            fetch_begin(u);
+            chunk(std::integral_constant<int, KPW - 1>{}, std::integral_constant<int, 0>{}, lds + (u + 1) % NS * SLOT, std::integral_constant<int, 0>{},
+                  std::integral_constant<int, HALF>{});
+            keep_here();
             if (++c_slice == c_nslices) {  // wavefront-uniform
                 if constexpr (EPI == 1) {
-                    head_stats(cb);  // nothing goes through the slot, and no store joins the count of loads in flight
+                    head_stats(cb);
                 } else {
                     if constexpr (EPI == 2 || EPI == 4) head_dlogits(cb);
-                    barrier();  // every wavefront has read slot u: it takes the result on its way out
                     if constexpr (GATE)
-                        store_gated(lds + u * SLOT, cb);
+                        store_gated(cb);
                     else if constexpr (GATE_GRAD)
-                        store_gated_grad(lds + u * SLOT, cb);
+                        store_gated_grad(cb);
                     else
-                        store_result(lds + u * SLOT, cb);
+                        store_result(cb);
                     since_store = 0;
                 }
                 cv = next_block(cv + stride, cb);
@@ -1034,12 +1063,12 @@ void launch_form(bool tA, bool tB, const GemmArgs& g, dim3 grid, hipStream_t st)
     if (tA && !tB) hipLaunchKernelGGL((gemm_bf16<G, true, false, CF32>), grid, dim3(G::NTHR), 0, st, g);
     if (tA && tB) hipLaunchKernelGGL((gemm_bf16<G, true, true, CF32>), grid, dim3(G::NTHR), 0, st, g);
 }
-template <typename G, bool CF32, int NS, bool SPREAD>
+template <typename G, bool CF32, int NS>
 void launch_ring_form(bool tA, bool tB, const GemmArgs& g, dim3 grid, hipStream_t st) {
-    if (!tA && !tB) hipLaunchKernelGGL((gemm_ring<G, false, false, CF32, NS, SPREAD>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
-    if (!tA && tB) hipLaunchKernelGGL((gemm_ring<G, false, true, CF32, NS, SPREAD>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
-    if (tA && !tB) hipLaunchKernelGGL((gemm_ring<G, true, false, CF32, NS, SPREAD>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
-    if (tA && tB) hipLaunchKernelGGL((gemm_ring<G, true, true, CF32, NS, SPREAD>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
+    if (!tA && !tB) hipLaunchKernelGGL((gemm_ring<G, false, false, CF32, NS>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
+    if (!tA && tB) hipLaunchKernelGGL((gemm_ring<G, false, true, CF32, NS>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
+    if (tA && !tB) hipLaunchKernelGGL((gemm_ring<G, true, false, CF32, NS>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
+    if (tA && tB) hipLaunchKernelGGL((gemm_ring<G, true, true, CF32, NS>), grid, dim3(G::NTHR), 0, st, g, HeadArgs{}, GroupArgs{});
 }
 int cu_count() {
     static const int n = [] {
@@ -1057,27 +1086,13 @@ void launch_ring(bool tA, bool tB, GemmArgs g, int S, bool c_f32, hipStream_t st
     g.tiles_n = (g.N + G::BN - 1) / G::BN;
     g.splits = S;
     // persistent: as many workgroups as the chip holds at once (a multiple of 8, one XCD's share each), or fewer
-    constexpr int NW = G::NTHR / 64;
-    constexpr int RING = NS * (RingOp<false, G::BM, NW>::BYTES + RingOp<false, G::BN, NW>::BYTES);  // same for every form
     const int64_t vblocks = (static_cast<int64_t>(g.tiles_m) * g.tiles_n * S + 7) / 8 * 8;
-    const int64_t slots = static_cast<int64_t>(cu_count()) / 8 * 8 * (RING <= 80 * 1024 ? 2 : 1);
+    const int64_t slots = static_cast<int64_t>(cu_count()) / 8 * 8 * RingLds<G, NS>::PER_CU;
     const unsigned gx = static_cast<unsigned>(std::min(vblocks, slots));
-    // When a slice's loads are issued. Spread behind the matrix instructions of the slice in hand they cost no issue
-    // time of their own, but the last of them then leaves late: a ring of two slots has only the rest of that slice
-    // to cover its latency, which pays where tiles change often (a short contraction, or the large tile whose slices
-    // take long) and costs 10 % in the steady state of a long one; three and more slots always have the slack.
-    const bool spread = NS > 2 || G::BM > 128 || std::min(g.K, g.k_per_split) <= 768;
-    if constexpr (NS > 2 || (G::BM > 128)) {
-        if (c_f32)
-            launch_ring_form<G, true, NS, true>(tA, tB, g, dim3(gx), st);
-        else
-            launch_ring_form<G, false, NS, true>(tA, tB, g, dim3(gx), st);
-    } else {
-        if (c_f32 && spread) launch_ring_form<G, true, NS, true>(tA, tB, g, dim3(gx), st);
-        if (c_f32 && !spread) launch_ring_form<G, true, NS, false>(tA, tB, g, dim3(gx), st);
-        if (!c_f32 && spread) launch_ring_form<G, false, NS, true>(tA, tB, g, dim3(gx), st);
-        if (!c_f32 && !spread) launch_ring_form<G, false, NS, false>(tA, tB, g, dim3(gx), st);
-    }
+    if (c_f32)
+        launch_ring_form<G, true, NS>(tA, tB, g, dim3(gx), st);
+    else
+        launch_ring_form<G, false, NS>(tA, tB, g, dim3(gx), st);
     hip_check(hipGetLastError(), "gemm_ring launch");
 }
 template <typename G>
@@ -1262,7 +1277,7 @@ void launch_head(GemmArgs g, const HeadArgs& hd, hipStream_t st) {
     const int64_t vblocks = static_cast<int64_t>((g.tiles_m * g.tiles_n + 7) / 8 * 8);
     const int64_t slots = cu_count() / 8 * 8 * (G::BM > 128 ? 1 : 2);
     const unsigned gx = static_cast<unsigned>(std::min<int64_t>(vblocks, slots));
-    hipLaunchKernelGGL((gemm_ring<G, false, true, false, 2, true, EPI>), dim3(gx), dim3(G::NTHR), 0, st, g, hd, GroupArgs{});
+    hipLaunchKernelGGL((gemm_ring<G, false, true, false, 2, EPI>), dim3(gx), dim3(G::NTHR), 0, st, g, hd, GroupArgs{});
     hip_check(hipGetLastError(), "gemm_ring (head) launch");
 }
 }  // namespace
@@ -1336,7 +1351,7 @@ void launch_gated_form(GemmArgs g, hipStream_t st) {
     g.tiles_m = (g.M + G::BM - 1) / G::BM;
     g.tiles_n = (g.N + BNC - 1) / BNC;
     const int64_t vblocks = (static_cast<int64_t>(g.tiles_m) * g.tiles_n + 7) / 8 * 8, slots = cu_count() / 8 * 8 * (G::BM > 128 ? 1 : 2);
-    hipLaunchKernelGGL((gemm_ring<G, false, TB, false, 2, true, EPI>), dim3(static_cast<unsigned>(std::min(vblocks, slots))), dim3(G::NTHR), 0,
+    hipLaunchKernelGGL((gemm_ring<G, false, TB, false, 2, EPI>), dim3(static_cast<unsigned>(std::min(vblocks, slots))), dim3(G::NTHR), 0,
                        st, g, HeadArgs{}, GroupArgs{});
     hip_check(hipGetLastError(), "gemm_ring (gated) launch");
 }
@@ -1474,7 +1489,7 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
         g.k_per_split = kps;
         g.part_stride = elements;
         const int64_t vblocks = (static_cast<int64_t>(tiles) * S + 7) / 8 * 8;
-        hipLaunchKernelGGL((gemm_ring<GeoSmallK2, true, false, true, 4, true, 3>),
+        hipLaunchKernelGGL((gemm_ring<GeoSmallK2, true, false, true, 4, 3>),
                            dim3(static_cast<unsigned>(std::min<int64_t>(vblocks, cu_count() / 8 * 8))), dim3(GeoSmallK2::NTHR), 0, st, g, HeadArgs{}, gr);
         hip_check(hipGetLastError(), "gemm_ring (grouped) launch");
         hipLaunchKernelGGL(sum_group, dim3(static_cast<unsigned>(std::min<int64_t>((elements / 4 + 255) / 256, 4096))), dim3(256), 0, st,
@@ -1485,11 +1500,11 @@ bool gemm_mfma_grouped_tn(const GroupedProduct* ps, int count, int64_t K, hipStr
     const int64_t vblocks = (static_cast<int64_t>(tiles) + 7) / 8 * 8;
     if (tiles <= cu_count()) {
         const unsigned gx = static_cast<unsigned>(std::min<int64_t>(vblocks, cu_count() / 8 * 8));
-        hipLaunchKernelGGL((gemm_ring<GeoSmallK2, true, false, true, 4, true, 3>), dim3(gx), dim3(GeoSmallK2::NTHR), 0, st, g,
+        hipLaunchKernelGGL((gemm_ring<GeoSmallK2, true, false, true, 4, 3>), dim3(gx), dim3(GeoSmallK2::NTHR), 0, st, g,
                            HeadArgs{}, gr);
     } else {
         const unsigned gx = static_cast<unsigned>(std::min<int64_t>(vblocks, cu_count() / 8 * 8 * 2));
-        hipLaunchKernelGGL((gemm_ring<GeoSmall, true, false, true, 2, false, 3>), dim3(gx), dim3(GeoSmall::NTHR), 0, st, g,
+        hipLaunchKernelGGL((gemm_ring<GeoSmall, true, false, true, 2, 3>), dim3(gx), dim3(GeoSmall::NTHR), 0, st, g,
                            HeadArgs{}, gr);
     }
     hip_check(hipGetLastError(), "gemm_ring (grouped) launch");

@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "pk_internal.h"
 
 namespace pk {
@@ -250,6 +252,14 @@ __device__ inline void dma_piece(uint32_t lds_byte, uint32_t off, u32x4 rsrc, ui
     static_assert(J >= 0 && J < 4, "immediate offsets below 4096");
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen offset:%4 lds" ::"s"(lds_byte), "v"(off),
                  "s"(rsrc), "s"(soff), "n"(J * 1024));
+}
+// f(integral_constant B), ..., f(integral_constant E - 1)
+template <int B, int E, typename F>
+__device__ inline void static_for(F&& f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
 }
 template <int N>
 __device__ inline void wait_loads() {
