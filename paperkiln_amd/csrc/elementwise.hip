@@ -859,6 +859,13 @@ __global__ void rope_inplace_k(T* x, const int* pos, RopeFreq freq, int d, int h
     }
 }
 
+__global__ void rope_table_k(RopeFreq freq, int pairs, int64_t positions, float2* table) {
+    const int64_t i = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x;
+    if (i >= positions * pairs) return;
+    const float th = static_cast<float>(static_cast<int>(i / pairs)) * freq.f[i % pairs];
+    table[i] = make_float2(cosf(th), sinf(th));
+}
+
 template <typename T>
 __global__ void emb_fwd(const float* table, const int* ids, T* y, int64_t n, int d) {
     for (int64_t i = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x; i < n * d; i += static_cast<int64_t>(gridDim.x) * NT)
@@ -1572,16 +1579,26 @@ void k_rmsnorm_bwd(const Tensor& dy, const Tensor& x, const float* rinv, const T
     }
 }
 namespace {
-RopeFreq rope_freq(const Tensor& x, float theta, int d, int head_dim) {
-    if (x.cols != 3 * d) throw std::runtime_error("apply_rope: cols must be divisible by 3");
-    if (head_dim % 2 != 0 || head_dim > d) throw std::runtime_error("apply_rope: head_dim must be even and <= d");
+RopeFreq rope_freq(float theta, int head_dim) {
     if (head_dim > 2 * ROPE_MAX_PAIRS) throw std::runtime_error("apply_rope: head_dim above 256 is not supported");
     RopeFreq freq;
     for (int dim = 0; dim < head_dim; dim += 2)  // ops.cpp:499-500
         freq.f[dim >> 1] = 1.0f / std::pow(theta, static_cast<float>(dim) / static_cast<float>(head_dim));
     return freq;
 }
+RopeFreq rope_freq(const Tensor& x, float theta, int d, int head_dim) {
+    if (x.cols != 3 * d) throw std::runtime_error("apply_rope: cols must be divisible by 3");
+    if (head_dim % 2 != 0 || head_dim > d) throw std::runtime_error("apply_rope: head_dim must be even and <= d");
+    return rope_freq(theta, head_dim);
+}
 }  // namespace
+void k_rope_table(float theta, int head_dim, int64_t positions, float* table) {
+    const int64_t all = positions * (head_dim / 2);
+    if (all == 0) return;  // no pairs
+    hipLaunchKernelGGL(rope_table_k, dim3(static_cast<unsigned>((all + NT - 1) / NT)), dim3(NT), 0, tape_stream(), rope_freq(theta, head_dim),
+                       head_dim / 2, positions, reinterpret_cast<float2*>(table));
+    post();
+}
 void k_rope(const Tensor& x, const int* pos, float theta, int d, int head_dim, int rot_heads, bool inverse,
             const Tensor& y) {
     const RopeFreq freq = rope_freq(x, theta, d, head_dim);

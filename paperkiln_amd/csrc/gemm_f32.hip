@@ -29,7 +29,8 @@ struct Job {
 };
 // What becomes of a tile. GATE: B is [gate | up], N columns each, and a tile is the same columns of both: C = silu(gate) up, and both
 // of them to gu if it is given. GATE_GRAD: the product is C's gradient d for the gate and up in gu: C is [M, 2 N] and gets theirs.
-enum class End { PLAIN, GATE, GATE_GRAD };
+// TURN: C is a [q | k | v] projection whose q and k turn by their positions (a lane's partner of a pair is its neighbour).
+enum class End { PLAIN, GATE, GATE_GRAD, TURN };
 // One product's numbers are found at one place, several products' only once the workgroup knows whose tile it has: a second
 // round trip to the arguments, 0.4 to 0.8 us of the 3.5 to 8 that a small product takes.
 template <int MAX>
@@ -85,7 +86,7 @@ __device__ inline int bytes_of(int rows, int cols, int64_t ld) { return static_c
 // sums, of every other step of a chunk, so that four wavefronts' chains of additions, with which a sum's error grows, are as short
 // as eight wavefronts' (at the sizes named below no slower: 4.69 us | 4.68, 3.78 | 3.80, 5.72 | 5.75, 5.87 | 5.88 with one | two).
 template <bool TA, bool TB, int MB, int NB, int KW, int SUMS, int MAX, End END>
-__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta) {
+__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta, const Turn turn) {
     constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB;
     constexpr int HALF = END == End::GATE ? NB / 2 : NB, TN = 16 * HALF;  // blocks of columns of C
     constexpr int ITEMS = (MB * HALF + KW - 1) / KW;                      // blocks that a wavefront adds up and stores
@@ -165,11 +166,19 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
     // gradients 27.0 -> 25.3): held over the loop those blocks cost it registers (28.0).
     const float* const add = jobs.job[j].addend ? jobs.job[j].addend : beta != 0.0f ? jobs.job[j].c : nullptr;
     const int64_t ldc = jobs.job[j].ldc;
-    f32x4 met[EARLY ? ITEMS : 1][END == End::GATE_GRAD ? 2 : 1];
-    auto meet = [&](int x, int y, f32x4 (&v)[END == End::GATE_GRAD ? 2 : 1]) {
+    constexpr bool MEETS = END == End::GATE_GRAD || END == End::TURN;  // two numbers an element
+    f32x4 met[EARLY ? ITEMS : 1][MEETS ? 2 : 1];
+    const int base = END == End::TURN ? m0 - quotient(m0, turn.seq_len) * turn.seq_len : 0;
+    auto meet = [&](int x, int y, f32x4 (&v)[MEETS ? 2 : 1]) {
         const int n = min(n0 + y * 16 + l16, N - 1);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+            if constexpr (END == End::TURN) {
+                const int pair = max(turned_pair(turn, n), 0), at = turned_position<TM>(turn, base, x * 16 + 4 * grp + r);
+                const float2 cs = *reinterpret_cast<const float2*>(turn.table + (static_cast<int64_t>(at) * (turn.head_dim / 2) + pair) * 2);
+                v[0][r] = cs.x, v[1][r] = cs.y;
+                continue;
+            }
             const int64_t o = min(m0 + x * 16 + 4 * grp + r, M - 1) * ldc + n;
             if constexpr (END == End::GATE_GRAD)
                 v[0][r] = jobs.job[j].gu[o], v[1][r] = jobs.job[j].gu[o + N];
@@ -178,7 +187,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
         }
     };
     if constexpr (EARLY)
-        if (END == End::GATE_GRAD || add)
+        if (MEETS || add)
 #pragma unroll
             for (int q = 0; q < ITEMS; ++q) {
                 const int g = min(q * KW + kw, MB * HALF - 1);
@@ -199,8 +208,16 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
         if (i + u < mine) multiply(u);
 
     float* const out = jobs.job[j].c;
-    auto store = [&](int x, int y, f32x4 v, const f32x4 (&e)[END == End::GATE_GRAD ? 2 : 1]) {
+    auto store = [&](int x, int y, f32x4 v, const f32x4 (&e)[MEETS ? 2 : 1]) {
         const int n = n0 + y * 16 + l16;
+        if constexpr (END == End::TURN) {
+            const bool turns = turned_pair(turn, n) >= 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float w = lane_moved<0xB1>(v[r]), t = l16 & 1 ? w * e[1][r] + v[r] * e[0][r] : v[r] * e[0][r] - w * e[1][r];
+                v[r] = turns ? t : v[r];
+            }
+        }
         if (n >= N) return;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -210,7 +227,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
                 if constexpr (END == End::GATE_GRAD)
                     gated_grad(e[0][r], e[1][r], v[r], out[o], out[o + N]);
                 else
-                    out[o] = add ? e[0][r] + v[r] : v[r];
+                    out[o] = END != End::TURN && add ? e[0][r] + v[r] : v[r];
             }
         }
     };
@@ -251,7 +268,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
                 store_gated(g / HALF, g % HALF, s, up);
             } else {
                 if constexpr (!EARLY)
-                    if (END == End::GATE_GRAD || add) meet(g / HALF, g % HALF, met[0]);
+                    if (MEETS || add) meet(g / HALF, g % HALF, met[0]);
                 store(g / HALF, g % HALF, s, met[EARLY ? g0 / KW : 0]);
             }
         }
@@ -259,7 +276,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 }
 
 template <bool TA, bool TB, int MB, int NB, int KW, End END, int SUMS = 1, int MAX>
-void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
+void launch(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn) {
     constexpr int TM = 16 * MB, TN = 16 * (END == End::GATE ? NB / 2 : NB);
     int tiles = 0;
     for (int j = 0; j < jobs.count; ++j) {
@@ -268,7 +285,7 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
     }
     for (int j = jobs.count; j <= MAX; ++j) jobs.first[j] = tiles;
     hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, SUMS, MAX, END>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
-                       tiles, beta);
+                       tiles, beta, turn);
     hip_check(hipGetLastError(), "gemm_f32");
 }
 
@@ -286,7 +303,7 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st) {
 //   contractions of more tiles than that are over sooner as 16 x 32, for which the last round is half as long (1000 x 576 x
 //   192: 7.7 us against 9.4, 256 x 1376 x 256: 5.8 against 6.8; with B transposed, whose rows those tiles read twice, they are not).
 template <bool TA, bool TB, End END, int MAX>
-void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st) {
+void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn = {}) {
     int64_t tiles = 0;
     int longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
@@ -294,25 +311,26 @@ void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st) {
         longest = std::max(longest, jobs.job[j].K);
     }
     if (tiles > 640 && (!TA || longest < 256))
-        launch<TA, TB, 4, 4, 4, END>(jobs, beta, st);
+        launch<TA, TB, 4, 4, 4, END>(jobs, beta, st, turn);
     else if (TA && longest >= 256 && tiles > 768)
-        launch<TA, TB, 2, 4, 4, END>(jobs, beta, st);
+        launch<TA, TB, 2, 4, 4, END>(jobs, beta, st, turn);
     else if (TA && longest >= 256 && tiles > 320 && tiles <= 512)
-        launch<TA, TB, 2, 4, 8, END>(jobs, beta, st);
+        launch<TA, TB, 2, 4, 8, END>(jobs, beta, st, turn);
     else if (tiles <= 64 && END != End::GATE)
-        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END, 2>(jobs, beta, st);
+        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END, 2>(jobs, beta, st, turn);
     else if (tiles <= 128)
-        launch<TA, TB, 1, 2, 4, END, 2>(jobs, beta, st);
+        launch<TA, TB, 1, 2, 4, END, 2>(jobs, beta, st, turn);
     else if (!TA && !TB && tiles > 256 && longest <= 256)
-        launch<TA, TB, 1, 2, 4, END>(jobs, beta, st);
+        launch<TA, TB, 1, 2, 4, END>(jobs, beta, st, turn);
     else if (tiles <= 256 && longest >= 256)
-        launch<TA, TB, 2, 2, 8, END>(jobs, beta, st);
+        launch<TA, TB, 2, 2, 8, END>(jobs, beta, st, turn);
     else
-        launch<TA, TB, 2, 2, 4, END>(jobs, beta, st);
+        launch<TA, TB, 2, 2, 4, END>(jobs, beta, st, turn);
 }
 
 template <int MAX>
-bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st, End end = End::PLAIN, float* gu = nullptr) {
+bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st, End end = End::PLAIN, float* gu = nullptr,
+              const Turn& turn = {}) {
     Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
@@ -338,6 +356,7 @@ bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
     if constexpr (MAX == 1) {
         if (end == End::GATE) launch_by_size<false, false, End::GATE>(jobs, beta, st);
         if (end == End::GATE_GRAD) launch_by_size<false, true, End::GATE_GRAD>(jobs, beta, st);
+        if (end == End::TURN) launch_by_size<false, false, End::TURN>(jobs, beta, st, turn);
         if (end != End::PLAIN) return true;
     }
     if (tA)
@@ -362,6 +381,11 @@ bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t
 bool gemm_f32_gated_grad(const float* dy, const float* w, const float* gu, float* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
     const F32Product p{dy, K, w, K, dgu, 2 * N, nullptr, M, N, K};
     return multiply<1>(&p, 1, false, true, 0.0f, st, End::GATE_GRAD, const_cast<float*>(gu));
+}
+bool gemm_f32_turned(const float* x, const float* w, float* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st) {
+    const int64_t N = 3 * static_cast<int64_t>(turn.d);
+    const F32Product p{x, K, w, N, y, N, nullptr, M, N, K};
+    return turn.d % 2 == 0 && turn.head_dim % 2 == 0 && multiply<1>(&p, 1, false, false, 0.0f, st, End::TURN, nullptr, turn);
 }
 
 }  // namespace pk

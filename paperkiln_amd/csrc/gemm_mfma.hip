@@ -81,6 +81,7 @@ struct HeadArgs {
     const float* row_inv;  // pass 2: [M], 1 / sum_j exp(z_j - row_max)
     float gscale;          // pass 2
     int vocab;             // EPI 4: columns from here to N only pad the matrix; their dlogits are 0
+    Turn turn;             // EPI 8
 };
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -417,6 +418,8 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     // A gated product's ends. 5, 6: B is [gate | up], N columns each; C = silu(gate) up, and (5) both of them to D, [M, 2 N]. 7: the
     // product is the gradient of C for the gate and up in D; C is [M, 2 N] and gets theirs.
     constexpr bool GATE = EPI == 5 || EPI == 6, GATE_GRAD = EPI == 7;
+    // 8: C is a [q | k | v] projection whose q and k turn by their positions.
+    constexpr bool TURN = EPI == 8;
     static_assert(!GATE || (!TB && G::FN == 2), "a wavefront holds a block of gate and one of up");
     constexpr int BM = G::BM, BN = G::BN, NTHR = G::NTHR, FM = G::FM, FN = G::FN, NW = NTHR / 64;
     using OA = RingOp<TA, BM, NW>;
@@ -787,6 +790,44 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
             __syncthreads();
         }
     };
+    // The product counts as it is stored, rounded. Cosines and sines of all chunks' four pairs are asked for before the first store, behind
+    // which they would wait.
+    auto store_turned = [&](const Block& bl) {
+        const u32x4 to_c = tile_rsrc(g.c, bl, g.N, g.N - bl.n0);
+        const int col = bl.n0 + st_ch * 8, pair = max(turned_pair(hd.turn, col), 0), base = bl.m0 - quotient(bl.m0, hd.turn.seq_len) * hd.turn.seq_len;
+        const bool turns = turned_pair(hd.turn, col) >= 0;
+        const uint32_t mask = col < g.N ? 0u : OUTSIDE;
+        uint16_t* const cs = reinterpret_cast<uint16_t*>(strip);
+        f32x4 by[FM][ST::PER_PHASE][2];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int k = 0; k < ST::PER_PHASE; ++k) {
+                const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / ST::CPR;
+                const int at = turned_position<BM>(hd.turn, base, (srow >> 5) * FM * 32 + (srow & 31) + i * 32);
+                const f32x4* const p = reinterpret_cast<const f32x4*>(hd.turn.table + (static_cast<int64_t>(at) * (hd.turn.head_dim / 2) + pair) * 2);
+                by[i][k][0] = p[0], by[i][k][1] = p[1];
+            }
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            write_strip(cs, i);
+            __syncthreads();
+            const uint32_t soff = static_cast<uint32_t>(i * 32) * g.N * 2u;
+#pragma unroll
+            for (int k = 0; k < ST::PER_PHASE; ++k) {
+                const int srow = (static_cast<int>(threadIdx.x) + k * NTHR) / ST::CPR;
+                u32x4 v = *reinterpret_cast<const u32x4*>(cs + ST::at(srow, st_ch * 8));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float x0 = lo(v[e]), x1 = hi(v[e]), c = by[i][k][e / 2][e % 2 * 2], s = by[i][k][e / 2][e % 2 * 2 + 1];
+                    const uint32_t t = pack_bf16(x0 * c - x1 * s, x0 * s + x1 * c);
+                    v[e] = turns ? t : v[e];
+                }
+                store16(v, coff[k] | mask, to_c, soff);
+            }
+            __syncthreads();
+        }
+    };
     auto store_result = [&](const Block& bl) {  // the tile's result, through the strip
         if (KS == 2) {  // set 1 hands its sums to set 0, half of them at a time: [wavefront][16-byte group][lane]
             f32x4* red = reinterpret_cast<f32x4*>(strip) + wq * ((FM / 2) * FN * 4) * 64 + lane;
@@ -974,6 +1015,8 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                         store_gated(cb);
                     else if constexpr (GATE_GRAD)
                         store_gated_grad(cb);
+                    else if (TURN && (cb.n0 < hd.turn.cols || (cb.n0 < hd.turn.d + hd.turn.cols && cb.n0 + BN > hd.turn.d)))
+                        store_turned(cb);
                     else
                         store_result(cb);
                     since_store = 0;
@@ -1387,6 +1430,30 @@ bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* d
     g.d = gu;
     g.ldc = 2 * N;
     large ? launch_gated_form<GeoLarge, true, 7>(g, st) : launch_gated_form<GeoSmall, true, 7>(g, st);
+    return true;
+}
+
+// ---- RoPE inside the q|k|v product ----
+// On its way out the product turns q and k by the cosines and sines of a table, which a pass of its own over q and k would form anew (8192 x
+// 1536 x 512: 19.4 us and 5.0 | 21.6, first head or all 8; a model of 6 such layers with checkpointing, whose step makes 12, all heads,
+// 3.84 -> 3.75 ms a step). The small kernels ask for a lane's cosines behind the first chunks (fp32, 512 x 384 x 128: 4.8 us and 3.0 | 5.0).
+// Tiles of 128 x 128; not the 256 x 256 ones, which start at 512 tiles of q|k|v and whose ends have no registers left.
+bool gemm_mfma_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st) {
+    const int64_t N = 3 * static_cast<int64_t>(turn.d);
+    if (g_force_geo < 0 && gemm_small_is_ahead(false, false, M, N, K) && gemm_small_turned(x, w, y, M, K, turn, st)) return true;
+    if (turn.d % 8 || turn.head_dim % 8 || turn.cols % 8 || !takes(x, false, K, w, false, N, M, N, K) || !aligned16(y) || !aligned16(turn.table)) return false;
+    const Plan p = make_plan(false, false, M, N, K, K, N, N);
+    if (g_force_geo >= 0 || p.S != 1 || p.ring != 6 || M * N * 2 >= (int64_t{1} << 31) - 4096) return false;
+    GemmArgs g = gemm_args(x, K, w, N, M, N, K);
+    g.c = y;
+    g.tiles_m = (g.M + GeoSmall::BM - 1) / GeoSmall::BM;
+    g.tiles_n = (g.N + GeoSmall::BN - 1) / GeoSmall::BN;
+    HeadArgs hd{};
+    hd.turn = turn;
+    const int64_t vblocks = (static_cast<int64_t>(g.tiles_m) * g.tiles_n + 7) / 8 * 8, slots = cu_count() / 8 * 8 * RingLds<GeoSmall, 2>::PER_CU;
+    hipLaunchKernelGGL((gemm_ring<GeoSmall, false, false, false, 2, 8>), dim3(static_cast<unsigned>(std::min(vblocks, slots))), dim3(GeoSmall::NTHR), 0,
+                       st, g, hd, GroupArgs{});
+    hip_check(hipGetLastError(), "gemm_ring (turned) launch");
     return true;
 }
 

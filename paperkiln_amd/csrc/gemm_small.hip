@@ -23,7 +23,7 @@ struct Job {
     uint16_t* gu;  // as in gemm_f32.hip
     int lda, ldb, ldc, M, N, K;
 };
-enum class End { PLAIN, GATE, GATE_GRAD };
+enum class End { PLAIN, GATE, GATE_GRAD, TURN };
 // as in gemm_f32.hip: one product's numbers are found without a second round trip to the arguments (512 x 384 x 128 4.2 -> 3.3 us,
 // 512 x 128 x 344 4.7 -> 3.6, 2048 x 128 x 128 4.0 -> 3.4)
 template <int MAX>
@@ -73,7 +73,7 @@ struct Chunk {
 };
 
 template <bool TA, bool TB, bool CF32, int KW, int MAX, End END>
-__global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs, const int tiles, const int accumulate) {
+__global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs, const int tiles, const int accumulate, const Turn turn) {
     constexpr int BUFS = 4, NC = END == End::GATE ? 2 : 1;  // NC: columns of gate and of up, or of one matrix
     // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
     const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -142,6 +142,15 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
     const void* const add = jobs.job[j].addend ? jobs.job[j].addend : accumulate ? jobs.job[j].c : nullptr;
     const int64_t ldc = jobs.job[j].ldc;
     u32x2 met[RPW];
+    const int pair = END == End::TURN ? turned_pair(turn, n0 + 2 * l16) : -1;
+    if constexpr (END == End::TURN) {
+        const int base = m0 - quotient(m0, turn.seq_len) * turn.seq_len;
+#pragma unroll
+        for (int q = 0; q < RPW; ++q) {
+            const int row = kw * RPW + q, at = turned_position<32>(turn, base, 2 * (4 * grp + (row & 3)) + (row >> 2));
+            if (pair >= 0) met[q] = *reinterpret_cast<const u32x2*>(turn.table + (static_cast<int64_t>(at) * (turn.head_dim / 2) + pair) * 2);
+        }
+    }
     if (END == End::GATE_GRAD || (END == End::PLAIN && add))
 #pragma unroll
         for (int q = 0; q < RPW; ++q) {
@@ -214,6 +223,13 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o + N) = pack_bf16(du[0], du[1]);
             continue;
         }
+        if constexpr (END == End::TURN) {
+            if (pair >= 0) {
+                const float c = __uint_as_float(met[q][0]), s = __uint_as_float(met[q][1]), t = s0 * c - s1 * s;
+                s1 = s0 * s + s1 * c;
+                s0 = t;
+            }
+        }
         if (CF32) {
             f32x2 v = {s0, s1};
             if (add) v[0] += __uint_as_float(met[q][0]), v[1] += __uint_as_float(met[q][1]);
@@ -229,7 +245,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
 }
 
 template <bool TA, bool TB, bool CF32, End END = End::PLAIN, int MAX>
-void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st) {
+void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st, const Turn& turn = {}) {
     int tiles = 0, longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
         jobs.first[j] = tiles;
@@ -240,9 +256,9 @@ void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st) {
     const dim3 grid((tiles + 7) / 8 * 8);
     // eight wavefronts where each still has a few chunks and two workgroups fit every CU
     if (longest >= 512 && tiles <= 1024)
-        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 8, MAX, END>), grid, dim3(512), 0, st, jobs, tiles, accumulate ? 1 : 0);
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 8, MAX, END>), grid, dim3(512), 0, st, jobs, tiles, accumulate ? 1 : 0, turn);
     else
-        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 4, MAX, END>), grid, dim3(256), 0, st, jobs, tiles, accumulate ? 1 : 0);
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 4, MAX, END>), grid, dim3(256), 0, st, jobs, tiles, accumulate ? 1 : 0, turn);
     hip_check(hipGetLastError(), "gemm_small");
 }
 
@@ -265,7 +281,7 @@ bool gemm_small_is_ahead(bool tA, bool tB, int64_t M, int64_t N, int64_t K) {
 namespace {
 template <int MAX>
 bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st, End end = End::PLAIN,
-              void* gu = nullptr) {
+              void* gu = nullptr, const Turn& turn = {}) {
     Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
@@ -293,6 +309,7 @@ bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, 
     if constexpr (MAX == 1) {
         if (end == End::GATE) launch<false, false, false, End::GATE>(jobs, acc, st);
         if (end == End::GATE_GRAD) launch<false, true, false, End::GATE_GRAD>(jobs, acc, st);
+        if (end == End::TURN) launch<false, false, false, End::TURN>(jobs, acc, st, turn);
         if (end != End::PLAIN) return true;
     }
     if (tA)
@@ -316,6 +333,11 @@ bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M
 bool gemm_small_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
     const SmallProduct p{dy, K, w, K, dgu, 2 * N, nullptr, M, N, K};
     return multiply<1>(&p, 1, false, true, PK_BF16, 0.0f, st, End::GATE_GRAD, const_cast<void*>(gu));
+}
+bool gemm_small_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st) {
+    const int64_t N = 3 * static_cast<int64_t>(turn.d);
+    const SmallProduct p{x, K, w, N, y, N, nullptr, M, N, K};
+    return turn.d % 2 == 0 && turn.head_dim % 2 == 0 && multiply<1>(&p, 1, false, false, PK_BF16, 0.0f, st, End::TURN, nullptr, turn);
 }
 
 }  // namespace pk

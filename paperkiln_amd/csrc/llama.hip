@@ -172,6 +172,17 @@ struct Model {
     // zero_grad, the clip norm and the optimiser step are then one launch each, not one per parameter.
     Tensor pslab, gslab, mslab, vslab;
     SlabReader reader;
+    // Cosines and sines of RoPE's angles for every position that a sequence of this model has had, laid out once like the weights.
+    std::shared_ptr<Buffer> turns;
+    int64_t turned_positions = 0;
+    void turn_positions(int64_t seq_len) {
+        if (seq_len <= turned_positions) return;
+        const int dk = cfg.d / cfg.n_heads;
+        auto table = std::make_shared<Buffer>(sizeof(float) * seq_len * std::max(dk / 2 * 2, 2));
+        k_rope_table(cfg.rope_theta, dk, seq_len, static_cast<float*>(table->p));
+        turns = std::move(table);
+        turned_positions = seq_len;
+    }
     long t = 0;
     // Pinned staging for what a pass sends up (ids, targets, positions): one host copy and asynchronous transfers
     // instead of three transfers from pageable memory with a wait each. Written only between passes (a pass ends
@@ -274,8 +285,7 @@ struct Model {
     Var block_forward(const Block& b, const Var& x, const std::shared_ptr<Buffer>& pos, int64_t seq_len) const {
         const int dk = cfg.d / cfg.n_heads;
         Var h = ops::rmsnorm(x, b.ln1_w);
-        Var qkv = ops::linear3(h, b.q, b.k, b.v);
-        qkv = ops::apply_rope(qkv, pos, cfg.rope_theta, dk, cfg.rope_all_heads ? cfg.n_heads : 1, /*in_place=*/true);
+        Var qkv = ops::linear3_rope(h, b.q, b.k, b.v, pos, cfg.rope_theta, dk, cfg.rope_all_heads ? cfg.n_heads : 1, turns, seq_len == 0 ? x->data.rows : seq_len);
         const float sc = 1.0f / std::sqrt(static_cast<float>(dk));
         Var x1 = ops::linear_add(ops::attention_qkv(qkv, cfg.n_heads, sc, seq_len, true, cfg.window, cfg.sinks), b.o, x);
         Var h2 = ops::rmsnorm(x1, b.ln2_w);
@@ -494,6 +504,7 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
             prepare_shadow(b.down);
         }
         prepare_shadow(m->embed);
+        m->turn_positions(sl);
         const size_t base = dev_live_bytes();  // the allocator's host-side counters: nothing to wait for
         dev_reset_peak();
         const size_t live0 = live_variables();

@@ -285,6 +285,21 @@ __device__ inline void gated_grad(float g, float u, float d, float& dg, float& d
 // n / d where neither is negative: a division of signed numbers is a third longer, and a workgroup divides three to five times before its first load
 __host__ __device__ inline int quotient(int n, int d) { return static_cast<int>(static_cast<unsigned>(n) / static_cast<unsigned>(d)); }
 
+// Places in a product's Turn (tensor.h). The pair of a head that column c begins (or is in), -1 for one that stays as it is:
+template <typename T>
+__device__ inline int turned_pair(const T& t, int c) {
+    const int w = c >= t.d ? c - t.d : c;
+    if (c >= 2 * t.d || w >= t.cols) return -1;
+    return (w - quotient(w, t.head_dim) * t.head_dim) >> 1;
+}
+// the position of the row `off` (below SPAN) past one of position `base`
+template <int SPAN, typename T>
+__device__ inline int turned_position(const T& t, int base, int off) {
+    const int p = base + off;
+    if (t.seq_len >= SPAN) return p >= t.seq_len ? p - t.seq_len : p;
+    return p - quotient(p, t.seq_len) * t.seq_len;
+}
+
 // The arguments lie in six lines of memory, and the first look at each is 600 clocks. Asked for where they are used they are two to four such
 // waits one after the other before a workgroup's first load; here they are one.
 // us, as they are used | at once: T 512 x 16, 8 heads of 64 forward 13.6 | 13.4, backward 36.1 | 33.8; T 1024 x 8 20.5 | 19.9, 51.6 | 48.8; T 128, 4 heads

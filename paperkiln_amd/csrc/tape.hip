@@ -605,14 +605,14 @@ void cat_gradients(const Var& x, const std::vector<Var>& Ws, const Tensor& dy) {
 // gate/up projections) as ONE GEMM against the column-wise concatenation of their weights, which
 // is kept as a compute-dtype copy like any other shadow. Backward is one GEMM for dX and one for
 // all the weight gradients, whose column blocks are scattered to the separate gradient tensors.
-Var linear_cat(const Var& x, const std::vector<Var>& Ws) {
+static Var linear_cat_by(const Var& x, const std::vector<Var>& Ws, const std::function<bool(const Tensor& W, const Tensor& y)>& product) {
     if (Ws.empty() || Ws.size() > 4) throw std::runtime_error("linear_cat: 1 to 4 weights");
     const int64_t N = x->data.rows, d = Ws[0]->data.cols;
     for (const Var& W : Ws)
         if (W->data.cols != d || W->data.rows != x->data.cols) shape_fail("matmul: inner dimensions disagree");
     const int n = static_cast<int>(Ws.size());
     Tensor y = Tensor::make(N, n * d, x->data.dtype);
-    gemm(x->data, false, shadow_cat(Ws), false, y.ptr(), y.dtype, N, n * d, n * d, 0.0f);
+    if (!product || !product(shadow_cat(Ws), y)) gemm(x->data, false, shadow_cat(Ws), false, y.ptr(), y.dtype, N, n * d, n * d, 0.0f);
     std::vector<Var> parents{x};
     parents.insert(parents.end(), Ws.begin(), Ws.end());
     return record(std::move(y), std::move(parents), [](Variable* self) {
@@ -620,6 +620,7 @@ Var linear_cat(const Var& x, const std::vector<Var>& Ws) {
     });
 }
 
+Var linear_cat(const Var& x, const std::vector<Var>& Ws) { return linear_cat_by(x, Ws, nullptr); }
 Var linear3(const Var& x, const Var& Wq, const Var& Wk, const Var& Wv) { return linear_cat(x, {Wq, Wk, Wv}); }
 
 Var add(const Var& a, const Var& b) {
@@ -786,21 +787,43 @@ Var rmsnorm(const Var& x, const Var& w) {
     });
 }
 
+// The node of a rotation that has been applied where qkv lies, a projection nobody else reads (a Linear's backward needs its input and
+// weight, not its output): the node shares the storage; the backward turns this node's gradient back in place and passes it on whole.
+static Var rope_in_place(const Var& qkv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads, int d) {
+    return record(Tensor(qkv->data), {qkv}, [pos, theta, head_dim, rot_heads, d](Variable* self) {
+        const Var& x = self->parents[0];
+        if (!x->requires_grad) return;
+        k_rope_inplace(self->own_grad(), static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, true);
+        x->accumulate_owned(std::move(self->grad));
+        self->grad = Tensor();
+    });
+}
+
+Var linear3_rope(const Var& x, const Var& Wq, const Var& Wk, const Var& Wv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads,
+                 const std::shared_ptr<Buffer>& table, int64_t seq_len) {
+    const int64_t M = x->data.rows, K = x->data.cols;
+    const int d = static_cast<int>(Wq->data.cols);
+    if (rot_heads < 1 || static_cast<int64_t>(rot_heads) * head_dim > d) throw std::runtime_error("apply_rope: head_dim must be even and <= d");
+    bool turned = false;
+    const Var qkv = linear_cat_by(x, {Wq, Wk, Wv}, [&](const Tensor& W, const Tensor& y) {
+        if (gemm_backend() == 0 || W.dtype != y.dtype || seq_len > (1 << 30)) return false;
+        const Turn turn{static_cast<const float*>(table->p), static_cast<int>(seq_len), d, head_dim, rot_heads * head_dim};
+        turned = y.dtype == PK_BF16 ? gemm_mfma_turned(x->data.ptr(), W.ptr(), y.ptr(), M, K, turn, tape_stream())
+                                    : gemm_f32_is_ahead(false, M, 3 * d, K) &&
+                                          gemm_f32_turned(static_cast<const float*>(x->data.ptr()), static_cast<const float*>(W.ptr()),
+                                                          static_cast<float*>(y.ptr()), M, K, turn, tape_stream());
+        return turned;
+    });
+    if (!turned) return apply_rope(qkv, pos, theta, head_dim, rot_heads, /*in_place=*/true);
+    return rope_in_place(qkv, pos, theta, head_dim, rot_heads, d);
+}
+
 Var apply_rope(const Var& qkv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads, bool in_place) {
     if (qkv->data.cols % 3 != 0) shape_fail("apply_rope: cols must be divisible by 3");
     const int d = static_cast<int>(qkv->data.cols / 3);
     if (in_place) {
-        // The caller hands over a projection nobody else reads (a Linear's backward needs its input and weight, not
-        // its output): the rotation is applied where the data lies and the node shares the storage; the backward
-        // turns this node's gradient back in place and passes it on whole.
         k_rope_inplace(qkv->data, static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, false);
-        return record(Tensor(qkv->data), {qkv}, [pos, theta, head_dim, rot_heads, d](Variable* self) {
-            const Var& x = self->parents[0];
-            if (!x->requires_grad) return;
-            k_rope_inplace(self->own_grad(), static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, true);
-            x->accumulate_owned(std::move(self->grad));
-            self->grad = Tensor();
-        });
+        return rope_in_place(qkv, pos, theta, head_dim, rot_heads, d);
     }
     Tensor y = Tensor::make(qkv->data.rows, qkv->data.cols, qkv->data.dtype);
     k_rope(qkv->data, static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, false, y);

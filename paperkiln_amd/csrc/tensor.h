@@ -50,6 +50,14 @@ void k_add_held(const HeldSum* held, int count);  // no two with the same dw
 void k_rope(const Tensor& x, const int* pos, float theta, int d, int head_dim, int rot_heads, bool inverse,
             const Tensor& y);
 void k_rope_inplace(const Tensor& x, const int* pos, float theta, int d, int head_dim, int rot_heads, bool inverse);
+// table[p][i] = cosine and sine of position p's angle for pair i of a head, the ones that k_rope forms
+void k_rope_table(float theta, int head_dim, int64_t positions, float* table);
+// How a product that is a fused [rows, 3 d] projection turns its q and k thirds on the way out; row r has position r % seq_len.
+struct Turn {
+    const float* table;  // [seq_len or more][head_dim / 2] pairs of k_rope_table
+    int seq_len, d, head_dim;
+    int cols;  // the first so many columns of the q and of the k third turn
+};
 void k_embedding_fwd(const Tensor& table_f32, const int* ids, const Tensor& y);       // ops.cpp:329-337
 // scatter-add, ops.cpp:338-347; held sums (no two with the same dw) may ride along: true if they did
 bool k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable_f32, const HeldSum* held = nullptr, int count = 0);
@@ -169,6 +177,11 @@ bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M
 bool gemm_small_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
 bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
 bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
+// y [M, 3 d] = x w (x [M, K], w [K, 3 d], row-major without gaps) with q and k turned, y of the operands' type. False, with nothing
+// done, for what they do not take.
+bool gemm_f32_turned(const float* x, const float* w, float* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st);
+bool gemm_small_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st);
+bool gemm_mfma_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st);
 int64_t gemm_head_spans(int64_t M, int64_t N);
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,

@@ -85,6 +85,34 @@ def test_fp32_gated_product_in_its_projections(d, ff, tokens, seq):
     test_fp32_training_on_ragged_sizes(130, d, ff, tokens, seq)
 
 
+@pytest.mark.parametrize("all_heads", [False, True])
+@pytest.mark.parametrize("dtype,d,heads,tokens,seq", [
+    ("fp32", 64, 2, 33, 11), ("fp32", 96, 3, 77, 0), ("fp32", 128, 4, 516, 129), ("fp32", 192, 3, 300, 30), ("fp32", 256, 4, 1025, 205),
+    ("fp32", 24, 2, 70, 7), ("bf16", 64, 2, 33, 11), ("bf16", 128, 4, 516, 129), ("bf16", 24, 2, 70, 7), ("bf16", 256, 4, 2050, 410),
+    ("bf16", 320, 5, 2112, 33), ("bf16", 512, 8, 2048, 127 + 1), ("bf16", 512, 16, 1400, 100), ("bf16", 384, 3, 3001, 3001)])
+def test_rope_in_the_projection(dtype, d, heads, tokens, seq, all_heads):
+    """q and k turned on their way out of the q|k|v product, from a table, against the pass of its own beside the library's product: tiles of
+    16 to 128 rows of sequences shorter and longer than one, thirds that end inside a tile, head sizes that are no multiple of 8, and a
+    second pass with longer sequences than the table has."""
+    m = Llama(vocab=130, d=d, n_layers=1, n_heads=heads, d_ff=2 * d, compute_dtype=dtype, rope_all_heads=all_heads, seed=8)
+    toks = synth.randint(3, tokens + 1, 130)
+    tol = 1e-5 if dtype == "fp32" else 2e-2
+    before = blockops.set_gemm_backend(0)
+    try:
+        for sl in (seq, tokens):
+            blockops.set_gemm_backend(0)
+            want_loss, _ = m.loss_backward(toks[:-1], toks[1:], sl)
+            want = m.grads()
+            blockops.set_gemm_backend(1)
+            for ck in (False, True):
+                loss, _ = m.loss_backward(toks[:-1], toks[1:], sl, checkpoint=ck)
+                assert abs(loss - want_loss) < (1e-5 if dtype == "fp32" else 1e-3)
+                assert rel(m.grads(), want) < tol
+    finally:
+        blockops.set_gemm_backend(before)
+        m.close()
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("vocab,d,ff,layers", [(130, 64, 176, 8), (37, 12, 20, 1), (37, 6, 10, 1)])
 def test_optimiser_step_writes_the_copies(vocab, d, ff, layers, dtype):
