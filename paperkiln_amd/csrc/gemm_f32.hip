@@ -85,9 +85,16 @@ __device__ inline int bytes_of(int rows, int cols, int64_t ld) { return static_c
 // A workgroup's tile is MB x NB blocks of 16 x 16; its KW wavefronts split the contraction chunk by chunk. SUMS 2: a wavefront has two
 // sums, of every other step of a chunk, so that four wavefronts' chains of additions, with which a sum's error grows, are as short
 // as eight wavefronts' (at the sizes named below no slower: 4.69 us | 4.68, 3.78 | 3.80, 5.72 | 5.75, 5.87 | 5.88 with one | two).
-template <bool TA, bool TB, int MB, int NB, int KW, int SUMS, int MAX, End END>
-__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta, const Turn turn) {
-    constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= 4 ? 3 : 2, TM = 16 * MB;
+//
+// NORM: A's rows count normalised (Norm in tensor.h). A wavefront adds up the squares of what it loads of them and multiplies it by the
+// norm's weight; the rows' sums meet where the tiles' do, and every workgroup of a row of tiles writes its share of the normalised rows'
+// columns, of a short contraction out of the registers they still lie in. A launch of its own was 2.8 us and the wait for it, of a chain of 44
+// launches in a small model's step (512 x 384 x 128: 2.8 and 5.0 us | 5.6; gate and up, 512 x 688 x 128: 2.8 and 5.4 | 6.2, as 32 x 32: what
+// every workgroup adds is a microsecond, and of 16 x 32 there are two rounds, 7.2). The step: 3.75 -> 3.67 ms for 16.
+template <bool TA, bool TB, int MB, int NB, int KW, int SUMS, int MAX, End END, bool NORM>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, const int tiles, const float beta, const Turn turn, const Norm norm) {
+    static_assert(!NORM || (!TA && MAX == 1 && MB <= 2 && NB <= 2), "rows of one A, small tiles");
+    constexpr int KC = MB * NB <= 4 ? 32 : 16, BUFS = MB * NB <= (NORM ? 2 : 4) ? 3 : 2, TM = 16 * MB;
     constexpr int HALF = END == End::GATE ? NB / 2 : NB, TN = 16 * HALF;  // blocks of columns of C
     constexpr int ITEMS = (MB * HALF + KW - 1) / KW;                      // blocks that a wavefront adds up and stores
     constexpr bool EARLY = END != End::GATE && ITEMS == 1;
@@ -125,15 +132,22 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 #pragma unroll
     for (int i = 0; i < NB; ++i) ob[i] = static_cast<int>(TB ? col[i] * ldb + 4 * grp : 4 * grp * ldb + col[i]) * 4;
     float fa[BUFS][MB][KC / 4], fb[BUFS][NB][KC / 4];
+    float fw[NORM ? BUFS : 1][1][KC / 4], squares[MB];
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(NORM ? norm.w : a), 0, K * 4, 0x00020000);
+    const int ow[1] = {16 * grp};
+#pragma unroll
+    for (int x = 0; x < MB; ++x) squares[x] = 0.0f;
     const int chunks = (K + KC - 1) / KC;
     auto load = [&](int chunk, int buf) {
         const int over = max((chunk + 1) * KC - K, 0), k0 = chunk * KC - over;
         if (over == 0) {
             load_chunk<TA, MB, KC>(ra, jobs.job[j].lda, oa, k0, fa[buf]);
             load_chunk<!TB, NB, KC>(rb, jobs.job[j].ldb, ob, k0, fb[buf]);
+            if constexpr (NORM) load_chunk<false, 1, KC>(rw, 0, ow, k0, fw[buf]);
         } else if (K >= KC) {  // the last chunk, moved back to end where the contraction does: its first steps are done already
             load_chunk<TA, MB, KC>(ra, jobs.job[j].lda, oa, k0, fa[buf]);
             load_chunk<!TB, NB, KC>(rb, jobs.job[j].ldb, ob, k0, fb[buf]);
+            if constexpr (NORM) load_chunk<false, 1, KC>(rw, 0, ow, k0, fw[buf]);
 #pragma unroll
             for (int s = 0; s < KC / 4; ++s) {
                 const bool done = 4 * grp + 4 * (s & ~3) + (s & 3) < over;
@@ -145,9 +159,18 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
         } else {
             load_short<TA, MB, KC>(a, lda, row, 4 * grp, K, fa[buf]);
             load_short<!TB, NB, KC>(b, ldb, col, 4 * grp, K, fb[buf]);
+            if constexpr (NORM) load_chunk<false, 1, KC>(rw, 0, ow, 0, fw[buf]);  // zeros past the end
         }
     };
     auto multiply = [&](int buf) {
+        if constexpr (NORM)
+#pragma unroll
+            for (int s = 0; s < KC / 4; ++s)
+#pragma unroll
+                for (int x = 0; x < MB; ++x) {
+                    squares[x] = fmaf(fa[buf][x][s], fa[buf][x][s], squares[x]);
+                    fa[buf][x][s] *= fw[buf][0][s];
+                }
 #pragma unroll
         for (int s = 0; s < KC / 4; ++s)
 #pragma unroll
@@ -252,7 +275,61 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
     for (int x = 0; x < MB; ++x)
 #pragma unroll
         for (int y = 0; y < NB; ++y) part[kw][x * NB + y][lane] = SUMS > 1 ? acc[0][x][y] + acc[SUMS - 1][x][y] : acc[0][x][y];
+    __shared__ float of_row[NORM ? KW : 1][NORM ? TM : 1];
+    if constexpr (NORM)
+#pragma unroll
+        for (int x = 0; x < MB; ++x) {  // a row's other steps are 16, 32 and 48 lanes on
+            float q = squares[x];
+            q += __shfl_xor(q, 16);
+            q += __shfl_xor(q, 32);
+            if (grp == 0) of_row[kw][x * 16 + l16] = q;
+        }
     __syncthreads();
+    float inverse[MB];  // 1 / rms of row l16 of a block
+    if constexpr (NORM) {
+#pragma unroll
+        for (int x = 0; x < MB; ++x) {
+            float q = of_row[0][x * 16 + l16];
+#pragma unroll
+            for (int k = 1; k < KW; ++k) q += of_row[k][x * 16 + l16];
+            inverse[x] = 1.0f / sqrtf(q / static_cast<float>(K) + norm.eps);
+        }
+        if (norm.y) {  // column tile c writes chunks c, c + tn, ...: of a short contraction out of the registers they still lie in
+            const int at_col = t - jobs.first[j] - at_row * tn;
+            float* const y = static_cast<float*>(norm.y);
+#pragma unroll
+            for (int x = 0; x < MB; ++x) {
+                const int m = m0 + x * 16 + l16;
+                if (at_col == 0 && kw == 0 && grp == 0 && m < M) norm.rinv[m] = inverse[x];
+            }
+            if (chunks <= BUFS * KW && K % KC == 0) {
+#pragma unroll
+                for (int u = 0; u < BUFS; ++u) {
+                    const int c = kw + u * KW;
+                    if (c >= chunks || c - quotient(c, tn) * tn != at_col) continue;
+#pragma unroll
+                    for (int x = 0; x < MB; ++x) {
+                        const int m = m0 + x * 16 + l16;
+#pragma unroll
+                        for (int s = 0; s < KC / 4; s += 4) {
+                            const f32x4 v = {fa[u][x][s], fa[u][x][s + 1], fa[u][x][s + 2], fa[u][x][s + 3]};
+                            if (m < M) *reinterpret_cast<f32x4*>(y + static_cast<int64_t>(m) * K + c * KC + 4 * grp + 4 * s) = v * inverse[x];
+                        }
+                    }
+                }
+            } else {
+                for (int c = at_col; c < chunks; c += tn)
+#pragma unroll
+                    for (int x = 0; x < MB; ++x) {
+                        const int m = m0 + x * 16 + l16, k = c * KC + 4 * (kw * 4 + grp);
+                        if (m < M && 4 * (kw * 4 + grp) < KC && k < K) {
+                            const f32x4 v = *reinterpret_cast<const f32x4*>(a + m * lda + k), w = *reinterpret_cast<const f32x4*>(norm.w + k);
+                            *reinterpret_cast<f32x4*>(y + static_cast<int64_t>(m) * K + k) = v * w * inverse[x];
+                        }
+                    }
+            }
+        }
+    }
 #pragma unroll
     for (int g0 = 0; g0 < MB * HALF; g0 += KW) {
         const int g = g0 + kw;
@@ -261,10 +338,17 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
             f32x4 s = part[0][at][lane];
 #pragma unroll
             for (int k = 1; k < KW; ++k) s += part[k][at][lane];
+            f32x4 by;
+            if constexpr (NORM) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) by[r] = __shfl(g < HALF ? inverse[0] : inverse[MB - 1], 4 * grp + r);
+                s *= by;
+            }
             if constexpr (END == End::GATE) {
                 f32x4 up = part[0][at + HALF][lane];
 #pragma unroll
                 for (int k = 1; k < KW; ++k) up += part[k][at + HALF][lane];
+                if constexpr (NORM) up *= by;
                 store_gated(g / HALF, g % HALF, s, up);
             } else {
                 if constexpr (!EARLY)
@@ -276,7 +360,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f32_k(const Jobs<MAX> jobs, c
 }
 
 template <bool TA, bool TB, int MB, int NB, int KW, End END, int SUMS = 1, int MAX>
-void launch(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn) {
+void launch(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn, const Norm* norm) {
     constexpr int TM = 16 * MB, TN = 16 * (END == End::GATE ? NB / 2 : NB);
     int tiles = 0;
     for (int j = 0; j < jobs.count; ++j) {
@@ -284,8 +368,14 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn) {
         tiles += ((jobs.job[j].M + TM - 1) / TM) * ((jobs.job[j].N + TN - 1) / TN);
     }
     for (int j = jobs.count; j <= MAX; ++j) jobs.first[j] = tiles;
-    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, SUMS, MAX, END>), dim3((tiles + 7) / 8 * 8), dim3(64 * KW), 0, st, jobs,
-                       tiles, beta, turn);
+    const dim3 grid((tiles + 7) / 8 * 8), block(64 * KW);
+    if constexpr (MAX == 1 && MB <= 2 && NB <= 2 && (END == End::GATE || END == End::TURN))
+        if (norm) {
+            hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, SUMS, MAX, END, true>), grid, block, 0, st, jobs, tiles, beta, turn, *norm);
+            hip_check(hipGetLastError(), "gemm_f32");
+            return;
+        }
+    hipLaunchKernelGGL((gemm_f32_k<TA, TB, MB, NB, KW, SUMS, MAX, END, false>), grid, block, 0, st, jobs, tiles, beta, turn, Norm{});
     hip_check(hipGetLastError(), "gemm_f32");
 }
 
@@ -303,7 +393,7 @@ void launch(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn) {
 //   contractions of more tiles than that are over sooner as 16 x 32, for which the last round is half as long (1000 x 576 x
 //   192: 7.7 us against 9.4, 256 x 1376 x 256: 5.8 against 6.8; with B transposed, whose rows those tiles read twice, they are not).
 template <bool TA, bool TB, End END, int MAX>
-void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn = {}) {
+void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& turn = {}, const Norm* norm = nullptr) {
     int64_t tiles = 0;
     int longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
@@ -311,26 +401,26 @@ void launch_by_size(Jobs<MAX>& jobs, float beta, hipStream_t st, const Turn& tur
         longest = std::max(longest, jobs.job[j].K);
     }
     if (tiles > 640 && (!TA || longest < 256))
-        launch<TA, TB, 4, 4, 4, END>(jobs, beta, st, turn);
+        launch<TA, TB, 4, 4, 4, END>(jobs, beta, st, turn, norm);
     else if (TA && longest >= 256 && tiles > 768)
-        launch<TA, TB, 2, 4, 4, END>(jobs, beta, st, turn);
+        launch<TA, TB, 2, 4, 4, END>(jobs, beta, st, turn, norm);
     else if (TA && longest >= 256 && tiles > 320 && tiles <= 512)
-        launch<TA, TB, 2, 4, 8, END>(jobs, beta, st, turn);
+        launch<TA, TB, 2, 4, 8, END>(jobs, beta, st, turn, norm);
     else if (tiles <= 64 && END != End::GATE)
-        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END, 2>(jobs, beta, st, turn);
+        launch<TA, TB, 1, END == End::GATE ? 2 : 1, 4, END, 2>(jobs, beta, st, turn, norm);
     else if (tiles <= 128)
-        launch<TA, TB, 1, 2, 4, END, 2>(jobs, beta, st, turn);
-    else if (!TA && !TB && tiles > 256 && longest <= 256)
-        launch<TA, TB, 1, 2, 4, END>(jobs, beta, st, turn);
+        launch<TA, TB, 1, 2, 4, END, 2>(jobs, beta, st, turn, norm);
+    else if (!TA && !TB && !norm && tiles > 256 && longest <= 256)
+        launch<TA, TB, 1, 2, 4, END>(jobs, beta, st, turn, norm);
     else if (tiles <= 256 && longest >= 256)
-        launch<TA, TB, 2, 2, 8, END>(jobs, beta, st, turn);
+        launch<TA, TB, 2, 2, 8, END>(jobs, beta, st, turn, norm);
     else
-        launch<TA, TB, 2, 2, 4, END>(jobs, beta, st, turn);
+        launch<TA, TB, 2, 2, 4, END>(jobs, beta, st, turn, norm);
 }
 
 template <int MAX>
 bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st, End end = End::PLAIN, float* gu = nullptr,
-              const Turn& turn = {}) {
+              const Turn& turn = {}, const Norm* norm = nullptr) {
     Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
@@ -354,9 +444,9 @@ bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
         jobs.job[j].K = static_cast<int>(p.K);
     }
     if constexpr (MAX == 1) {
-        if (end == End::GATE) launch_by_size<false, false, End::GATE>(jobs, beta, st);
+        if (end == End::GATE) launch_by_size<false, false, End::GATE>(jobs, beta, st, turn, norm);
         if (end == End::GATE_GRAD) launch_by_size<false, true, End::GATE_GRAD>(jobs, beta, st);
-        if (end == End::TURN) launch_by_size<false, false, End::TURN>(jobs, beta, st, turn);
+        if (end == End::TURN) launch_by_size<false, false, End::TURN>(jobs, beta, st, turn, norm);
         if (end != End::PLAIN) return true;
     }
     if (tA)
@@ -368,24 +458,30 @@ bool multiply(const F32Product* ps, int count, bool tA, bool tB, float beta, hip
     return true;
 }
 
+// The normalised rows are written 16 bytes at a time. Not in the 64 x 64 tiles of more than 640 of 32 x 32, which have no registers for it.
+bool norm_fits(const float* x, int64_t M, int64_t columns, int64_t K, const Norm* norm) {
+    const auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    return !norm || (((M + 31) / 32) * ((columns + 31) / 32) <= 640 && K % 4 == 0 && at16(x) && at16(norm->w) && at16(norm->y));
+}
+
 }  // namespace
 
 bool gemm_f32(const F32Product* ps, int count, bool tA, bool tB, float beta, hipStream_t st) {
     if (count < 1 || count > 8 || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
     return count == 1 ? multiply<1>(ps, count, tA, tB, beta, st) : multiply<8>(ps, count, tA, tB, beta, st);
 }
-bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t M, int64_t N, int64_t K, hipStream_t st, const Norm* norm) {
     const F32Product p{x, K, w, 2 * N, h, N, nullptr, M, N, K};
-    return multiply<1>(&p, 1, false, false, 0.0f, st, End::GATE, gu);
+    return norm_fits(x, M, 2 * N, K, norm) && multiply<1>(&p, 1, false, false, 0.0f, st, End::GATE, gu, {}, norm);
 }
 bool gemm_f32_gated_grad(const float* dy, const float* w, const float* gu, float* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
     const F32Product p{dy, K, w, K, dgu, 2 * N, nullptr, M, N, K};
     return multiply<1>(&p, 1, false, true, 0.0f, st, End::GATE_GRAD, const_cast<float*>(gu));
 }
-bool gemm_f32_turned(const float* x, const float* w, float* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st) {
+bool gemm_f32_turned(const float* x, const float* w, float* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st, const Norm* norm) {
     const int64_t N = 3 * static_cast<int64_t>(turn.d);
     const F32Product p{x, K, w, N, y, N, nullptr, M, N, K};
-    return turn.d % 2 == 0 && turn.head_dim % 2 == 0 && multiply<1>(&p, 1, false, false, 0.0f, st, End::TURN, nullptr, turn);
+    return turn.d % 2 == 0 && turn.head_dim % 2 == 0 && norm_fits(x, M, N, K, norm) && multiply<1>(&p, 1, false, false, 0.0f, st, End::TURN, nullptr, turn, norm);
 }
 
 }  // namespace pk

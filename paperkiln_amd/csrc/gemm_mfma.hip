@@ -1406,8 +1406,9 @@ bool gated_plan(bool tB, int64_t M, int64_t cols, int64_t K, int64_t ldb, int64_
 }
 }  // namespace
 // h = silu(x gate) .* (x up) for w = [gate | up], N columns each; [x gate | x up] to gu unless that is null.
-bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st) {
-    if (g_force_geo < 0 && gemm_small_is_ahead(false, false, M, 2 * N, K) && gemm_small_gated(x, w, gu, h, M, N, K, st)) return true;
+bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st, const Norm* norm) {
+    if (g_force_geo < 0 && gemm_small_is_ahead(false, false, M, 2 * N, K) && gemm_small_gated(x, w, gu, h, M, N, K, st, norm)) return true;
+    if (norm) return false;
     bool large;
     if (N % 8 || !takes(x, false, K, w, false, 2 * N, M, 2 * N, K) || !aligned16(h) || !aligned16(gu) || !gated_plan(false, M, 2 * N, K, 2 * N, 2 * N, large))
         return false;
@@ -1438,9 +1439,10 @@ bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* d
 // 1536 x 512: 19.4 us and 5.0 | 21.6, first head or all 8; a model of 6 such layers with checkpointing, whose step makes 12, all heads,
 // 3.84 -> 3.75 ms a step). The small kernels ask for a lane's cosines behind the first chunks (fp32, 512 x 384 x 128: 4.8 us and 3.0 | 5.0).
 // Tiles of 128 x 128; not the 256 x 256 ones, which start at 512 tiles of q|k|v and whose ends have no registers left.
-bool gemm_mfma_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st) {
+bool gemm_mfma_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st, const Norm* norm) {
     const int64_t N = 3 * static_cast<int64_t>(turn.d);
-    if (g_force_geo < 0 && gemm_small_is_ahead(false, false, M, N, K) && gemm_small_turned(x, w, y, M, K, turn, st)) return true;
+    if (g_force_geo < 0 && gemm_small_is_ahead(false, false, M, N, K) && gemm_small_turned(x, w, y, M, K, turn, st, norm)) return true;
+    if (norm) return false;
     if (turn.d % 8 || turn.head_dim % 8 || turn.cols % 8 || !takes(x, false, K, w, false, N, M, N, K) || !aligned16(y) || !aligned16(turn.table)) return false;
     const Plan p = make_plan(false, false, M, N, K, K, N, N);
     if (g_force_geo >= 0 || p.S != 1 || p.ring != 6 || M * N * 2 >= (int64_t{1} << 31) - 4096) return false;

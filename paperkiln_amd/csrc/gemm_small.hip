@@ -72,8 +72,12 @@ struct Chunk {
     }
 };
 
-template <bool TA, bool TB, bool CF32, int KW, int MAX, End END>
-__global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs, const int tiles, const int accumulate, const Turn turn) {
+// NORM: A's rows count normalised, as in gemm_f32.hip; the product of a row and the norm's weight is rounded where the normalised row would be.
+// (512 x 384 x 128: 3.1 us of its own and 3.6 | 4.4; gate and up, 512 x 688 x 128: 3.1 and 4.1 | 5.1. A step of a bf16 model of 4 layers of
+// width 256 with checkpointing, 512 tokens: 9.1 -> 8.5 ms for 12.)
+template <bool TA, bool TB, bool CF32, int KW, int MAX, End END, bool NORM>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs, const int tiles, const int accumulate, const Turn turn, const Norm norm) {
+    static_assert(!NORM || (!TA && MAX == 1), "rows of one A");
     constexpr int BUFS = 4, NC = END == End::GATE ? 2 : 1;  // NC: columns of gate and of up, or of one matrix
     // every XCD takes a contiguous range of the tiles: neighbours share operand rows or columns in its L2
     const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -109,11 +113,20 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
 
     Chunk<TA> fa[BUFS];
     Chunk<!TB> fb[BUFS][NC];
+    f32x4 fw[NORM ? BUFS : 1][2];
+    float squares[2] = {0.0f, 0.0f};
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(norm.w), 0, K * 4, 0x00020000);
     const int chunks = (K + KC - 1) / KC;
     auto load = [&](int chunk, int buf) {
         // the last chunk of a contraction that is no multiple is moved back to end where that does: its first steps are done
         const int over = max((chunk + 1) * KC - K, 0), k0 = chunk * KC - over;
         fa[buf].load(ra, oa, k0, lda);
+        if constexpr (NORM)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, 32 * grp + 16 * h, k0 * 4, 0);
+                fw[buf][h] = *reinterpret_cast<const f32x4*>(&v);
+            }
 #pragma unroll
         for (int c = 0; c < NC; ++c) fb[buf][c].load(rb, oc[c], k0, ldb);
         if (over > 0) {
@@ -123,6 +136,15 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
         }
     };
     auto multiply = [&](int buf) {
+        if constexpr (NORM)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = __uint_as_float(fa[buf].raw[b][e] << 16), hi = __uint_as_float(fa[buf].raw[b][e] & 0xffff0000u);
+                    squares[b] = fmaf(hi, hi, fmaf(lo, lo, squares[b]));
+                    fa[buf].raw[b][e] = pack_bf16(lo * fw[buf][e / 2][e % 2 * 2], hi * fw[buf][e / 2][e % 2 * 2 + 1]);
+                }
         const bf16x8 a0 = fa[buf].block(0), a1 = fa[buf].block(1);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -185,7 +207,41 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
         for (int x = 0; x < 2; ++x)
 #pragma unroll
             for (int y = 0; y < 2; ++y) part[kw][c][x][y][lane] = acc[c][x][y];
+    __shared__ float of_row[NORM ? KW : 1][NORM ? 32 : 1];
+    if constexpr (NORM)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {  // a row's other steps are 16, 32 and 48 lanes on
+            float q = squares[b];
+            q += __shfl_xor(q, 16);
+            q += __shfl_xor(q, 32);
+            if (grp == 0) of_row[kw][2 * l16 + b] = q;
+        }
     __syncthreads();
+    auto inverse = [&](int r) {  // 1 / rms of the tile's row r
+        float q = of_row[0][NORM ? r : 0];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) q += of_row[NORM ? k : 0][NORM ? r : 0];
+        return 1.0f / sqrtf(q / static_cast<float>(K) + norm.eps);
+    };
+    if constexpr (NORM)
+        if (norm.y) {
+            const int at_col = t - jobs.first[j] - at_row * tn, share = (quotient(K + 3, 4) + tn - 1) / tn * 4, c0 = at_col * share, n = min(share, K - c0);
+            const int r = static_cast<int>(threadIdx.x) % 32, m = m0 + r;
+            if (m < M && (n > 0 || at_col == 0)) {
+                const float by = inverse(r);
+                if (at_col == 0 && static_cast<int>(threadIdx.x) < 32) norm.rinv[m] = by;
+                uint16_t* const y = static_cast<uint16_t*>(norm.y) + static_cast<int64_t>(m) * K + c0;
+                const uint16_t* const x = jobs.job[j].a + static_cast<int64_t>(m) * lda + c0;
+                for (int c = static_cast<int>(threadIdx.x) / 32 * 4; c < n; c += 64 * KW / 32 * 4) {
+                    u32x2 v = *reinterpret_cast<const u32x2*>(x + c);
+                    const f32x4 w = *reinterpret_cast<const f32x4*>(norm.w + c0 + c);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        v[e] = pack_bf16(__uint_as_float(v[e] << 16) * by * w[2 * e], __uint_as_float(v[e] & 0xffff0000u) * by * w[2 * e + 1]);
+                    *reinterpret_cast<u32x2*>(y + c) = v;
+                }
+            }
+        }
     const int n = n0 + 2 * l16;
     if (n >= N) return;
 #pragma unroll
@@ -198,6 +254,8 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
             return s;
         };
         float s0 = sum(0, 0), s1 = sum(0, 1);
+        float by = 1.0f;
+        if constexpr (NORM) by = inverse(2 * (4 * grp + r) + x), s0 *= by, s1 *= by;
         const int m = m0 + 2 * (4 * grp + r) + x;
         if (m >= M) continue;
         const int64_t o = m * ldc + n;
@@ -205,7 +263,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
         const auto lo = [](uint32_t v) { return __uint_as_float(v << 16); };
         const auto hi = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
         if constexpr (END == End::GATE) {
-            const uint32_t gate = pack_bf16(s0, s1), up = pack_bf16(sum(1, 0), sum(1, 1));
+            const uint32_t gate = pack_bf16(s0, s1), up = NORM ? pack_bf16(sum(1, 0) * by, sum(1, 1) * by) : pack_bf16(sum(1, 0), sum(1, 1));
             *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(jobs.job[j].c) + o) =
                 pack_bf16(gated(lo(gate), lo(up)), gated(hi(gate), hi(up)));
             if (uint16_t* const gu = jobs.job[j].gu) {
@@ -245,7 +303,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_small_k(const Jobs<MAX> jobs,
 }
 
 template <bool TA, bool TB, bool CF32, End END = End::PLAIN, int MAX>
-void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st, const Turn& turn = {}) {
+void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st, const Turn& turn = {}, const Norm* norm = nullptr) {
     int tiles = 0, longest = 0;
     for (int j = 0; j < jobs.count; ++j) {
         jobs.first[j] = tiles;
@@ -255,10 +313,19 @@ void launch(Jobs<MAX>& jobs, bool accumulate, hipStream_t st, const Turn& turn =
     for (int j = jobs.count; j <= MAX; ++j) jobs.first[j] = tiles;
     const dim3 grid((tiles + 7) / 8 * 8);
     // eight wavefronts where each still has a few chunks and two workgroups fit every CU
-    if (longest >= 512 && tiles <= 1024)
-        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 8, MAX, END>), grid, dim3(512), 0, st, jobs, tiles, accumulate ? 1 : 0, turn);
+    const bool eight = longest >= 512 && tiles <= 1024;
+    const auto start = [&](auto kw, auto normed, const Norm& n) {
+        constexpr int KW = decltype(kw)::value;
+        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, KW, MAX, END, decltype(normed)::value>), grid, dim3(64 * KW), 0, st, jobs, tiles, accumulate ? 1 : 0,
+                           turn, n);
+    };
+    const auto by_length = [&](auto normed, const Norm& n) {
+        eight ? start(std::integral_constant<int, 8>{}, normed, n) : start(std::integral_constant<int, 4>{}, normed, n);
+    };
+    if constexpr (MAX == 1 && (END == End::GATE || END == End::TURN))
+        norm ? by_length(std::true_type{}, *norm) : by_length(std::false_type{}, Norm{});
     else
-        hipLaunchKernelGGL((gemm_small_k<TA, TB, CF32, 4, MAX, END>), grid, dim3(256), 0, st, jobs, tiles, accumulate ? 1 : 0, turn);
+        by_length(std::false_type{}, Norm{});
     hip_check(hipGetLastError(), "gemm_small");
 }
 
@@ -281,7 +348,7 @@ bool gemm_small_is_ahead(bool tA, bool tB, int64_t M, int64_t N, int64_t K) {
 namespace {
 template <int MAX>
 bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st, End end = End::PLAIN,
-              void* gu = nullptr, const Turn& turn = {}) {
+              void* gu = nullptr, const Turn& turn = {}, const Norm* norm = nullptr) {
     Jobs<MAX> jobs{};
     jobs.count = count;
     for (int j = 0; j < count; ++j) {
@@ -307,9 +374,9 @@ bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, 
     }
     const bool f32 = c_dtype == PK_F32, acc = beta != 0.0f;
     if constexpr (MAX == 1) {
-        if (end == End::GATE) launch<false, false, false, End::GATE>(jobs, acc, st);
+        if (end == End::GATE) launch<false, false, false, End::GATE>(jobs, acc, st, turn, norm);
         if (end == End::GATE_GRAD) launch<false, true, false, End::GATE_GRAD>(jobs, acc, st);
-        if (end == End::TURN) launch<false, false, false, End::TURN>(jobs, acc, st, turn);
+        if (end == End::TURN) launch<false, false, false, End::TURN>(jobs, acc, st, turn, norm);
         if (end != End::PLAIN) return true;
     }
     if (tA)
@@ -320,24 +387,30 @@ bool multiply(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, 
         f32 ? launch<false, false, true>(jobs, acc, st) : launch<false, false, false>(jobs, acc, st);
     return true;
 }
+// the normalised rows are written four columns at a time
+bool norm_fits(const void* x, int64_t K, const Norm* norm) {
+    const auto at = [](const void* p, int a) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
+    return !norm || (K % 4 == 0 && K <= 4096 && at(x, 8) && at(norm->w, 16) && at(norm->y, 8));
+}
 }  // namespace
 
 bool gemm_small(const SmallProduct* ps, int count, bool tA, bool tB, int c_dtype, float beta, hipStream_t st) {
     if (count < 1 || count > 8 || (tA && tB) || (beta != 0.0f && beta != 1.0f)) return false;
     return count == 1 ? multiply<1>(ps, count, tA, tB, c_dtype, beta, st) : multiply<8>(ps, count, tA, tB, c_dtype, beta, st);
 }
-bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st, const Norm* norm) {
     const SmallProduct p{x, K, w, 2 * N, h, N, nullptr, M, N, K};
-    return multiply<1>(&p, 1, false, false, PK_BF16, 0.0f, st, End::GATE, gu);
+    return norm_fits(x, K, norm) && multiply<1>(&p, 1, false, false, PK_BF16, 0.0f, st, End::GATE, gu, {}, norm);
 }
 bool gemm_small_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st) {
     const SmallProduct p{dy, K, w, K, dgu, 2 * N, nullptr, M, N, K};
     return multiply<1>(&p, 1, false, true, PK_BF16, 0.0f, st, End::GATE_GRAD, const_cast<void*>(gu));
 }
-bool gemm_small_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st) {
+bool gemm_small_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st, const Norm* norm) {
     const int64_t N = 3 * static_cast<int64_t>(turn.d);
     const SmallProduct p{x, K, w, N, y, N, nullptr, M, N, K};
-    return turn.d % 2 == 0 && turn.head_dim % 2 == 0 && multiply<1>(&p, 1, false, false, PK_BF16, 0.0f, st, End::TURN, nullptr, turn);
+    return turn.d % 2 == 0 && turn.head_dim % 2 == 0 && norm_fits(x, K, norm) &&
+           multiply<1>(&p, 1, false, false, PK_BF16, 0.0f, st, End::TURN, nullptr, turn, norm);
 }
 
 }  // namespace pk

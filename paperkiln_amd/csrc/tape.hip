@@ -719,51 +719,7 @@ Var silu_mul_cat(const Var& gu) {
     return record(std::move(y), {gu}, silu_mul_cat_backward);
 }
 
-Var gated_mlp(const Var& x, const Var& gate, const Var& up, const Var& down, const Var& r, bool result_needed) {
-    const int64_t N = x->data.rows, ff = gate->data.cols, in = x->data.cols;
-    const int dtype = x->data.dtype;
-    if (gate->data.rows != in || up->data.rows != in || up->data.cols != ff || down->data.rows != ff)
-        shape_fail("matmul: inner dimensions disagree");
-    if (r->data.rows != N || r->data.cols != down->data.cols || r->data.dtype != dtype) shape_fail("add: shape mismatch");
-    // gate and up are kept where a backward pass will ask for them
-    const bool keep = grad_enabled() && (x->requires_grad || gate->requires_grad || up->requires_grad);
-    const Tensor& Wgu = shadow_cat({gate, up});
-    Tensor h = Tensor::make(N, ff, dtype), gu;
-    if (keep) gu = Tensor::make(N, 2 * ff, dtype);
-    const auto in_product = [&] {
-        if (gemm_backend() == 0 || Wgu.dtype != dtype) return false;
-        if (dtype == PK_BF16) return gemm_mfma_gated(x->data.ptr(), Wgu.ptr(), keep ? gu.ptr() : nullptr, h.ptr(), N, ff, in, tape_stream());
-        return gemm_f32_is_ahead(false, N, 2 * ff, in) &&
-               gemm_f32_gated(static_cast<const float*>(x->data.ptr()), static_cast<const float*>(Wgu.ptr()),
-                              keep ? static_cast<float*>(gu.ptr()) : nullptr, static_cast<float*>(h.ptr()), N, ff, in, tape_stream());
-    };
-    if (!in_product()) {
-        if (!keep) gu = Tensor::make(N, 2 * ff, dtype);
-        gemm(x->data, false, Wgu, false, gu.ptr(), dtype, N, 2 * ff, 2 * ff, 0.0f);
-        k_silu_mul_cat_fwd(gu, h);
-    }
-    Tensor y = Tensor::make(N, down->data.cols, dtype);
-    if (result_needed || !grad_enabled()) add_product(r->data, h, shadow_of(down), y);
-
-    // three nodes, as the ops by themselves would leave them
-    Var both;
-    if (keep)
-        both = record(std::move(gu), {x, gate, up}, [](Variable* self) {
-            cat_gradients(self->parents[0], {self->parents[1], self->parents[2]}, self->grad);
-        });
-    Var gated = keep ? record(std::move(h), {both}, silu_mul_cat_backward) : make_var(std::move(h), false);
-    return record(std::move(y), {gated, down, r}, [](Variable* self) {
-        const Var& gated = self->parents[0];
-        if (gated->requires_grad && !gated_gradient_in_product(self->grad, self->parents[1], gated->parents[0])) product_gradient(self);
-        product_weight_gradients(self);
-    });
-}
-
-Var rmsnorm(const Var& x, const Var& w) {
-    if (w->data.rows != 1 || w->data.cols != x->data.cols) shape_fail("rmsnorm: w must be [1, cols(x)]");
-    auto rinv = std::make_shared<Buffer>(sizeof(float) * x->data.rows);
-    Tensor y = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
-    k_rmsnorm_fwd(x->data, w->data, 1e-5f, y, static_cast<float*>(rinv->p));
+static Var norm_node(Tensor y, const Var& x, const Var& w, const std::shared_ptr<Buffer>& rinv) {
     return record(std::move(y), {x, w}, [rinv](Variable* self) {
         const Var& x = self->parents[0];
         const Var& w = self->parents[1];
@@ -786,6 +742,98 @@ Var rmsnorm(const Var& x, const Var& w) {
         }
     });
 }
+static void check_norm(const Var& x, const Var& w);
+// A normalised matrix that the product reading it may form itself: its node, whose rows are there once either has (or nowhere, where no
+// backward pass will ask for them and the product formed them).
+struct NormAhead {
+    Var x, w, h;
+    std::shared_ptr<Buffer> rinv;
+    Norm norm{};
+    NormAhead(const Var& x_, const Var& w_) : x(x_), w(w_) {
+        check_norm(x, w);
+        Tensor y;
+        y.rows = x->data.rows, y.cols = x->data.cols, y.dtype = x->data.dtype;
+        norm.w = static_cast<const float*>(w->data.ptr());
+        norm.eps = 1e-5f;
+        if (grad_enabled()) {
+            y = Tensor::make(y.rows, y.cols, y.dtype);
+            rinv = std::make_shared<Buffer>(sizeof(float) * y.rows);
+            norm.y = y.ptr();
+            norm.rinv = static_cast<float*>(rinv->p);
+        }
+        h = norm_node(std::move(y), x, w, rinv);
+    }
+    void by_itself() {
+        if (h->data.empty()) {
+            h->data = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
+            rinv = std::make_shared<Buffer>(sizeof(float) * x->data.rows);
+        }
+        k_rmsnorm_fwd(x->data, w->data, norm.eps, h->data, static_cast<float*>(rinv->p));
+    }
+};
+static Var gated_mlp_of(const Var& x, const Var& gate, const Var& up, const Var& down, const Var& r, bool result_needed, NormAhead* ahead) {
+    const int64_t N = x->data.rows, ff = gate->data.cols, in = x->data.cols;
+    const int dtype = x->data.dtype;
+    if (gate->data.rows != in || up->data.rows != in || up->data.cols != ff || down->data.rows != ff)
+        shape_fail("matmul: inner dimensions disagree");
+    if (r->data.rows != N || r->data.cols != down->data.cols || r->data.dtype != dtype) shape_fail("add: shape mismatch");
+    // gate and up are kept where a backward pass will ask for them
+    const bool keep = grad_enabled() && (x->requires_grad || gate->requires_grad || up->requires_grad);
+    const Tensor& Wgu = shadow_cat({gate, up});
+    Tensor h = Tensor::make(N, ff, dtype), gu;
+    if (keep) gu = Tensor::make(N, 2 * ff, dtype);
+    const auto in_product = [&](const Tensor& from, const Norm* norm) {
+        if (gemm_backend() == 0 || Wgu.dtype != dtype) return false;
+        if (dtype == PK_BF16) return gemm_mfma_gated(from.ptr(), Wgu.ptr(), keep ? gu.ptr() : nullptr, h.ptr(), N, ff, in, tape_stream(), norm);
+        return gemm_f32_is_ahead(false, N, 2 * ff, in) &&
+               gemm_f32_gated(static_cast<const float*>(from.ptr()), static_cast<const float*>(Wgu.ptr()),
+                              keep ? static_cast<float*>(gu.ptr()) : nullptr, static_cast<float*>(h.ptr()), N, ff, in, tape_stream(), norm);
+    };
+    bool formed = ahead && in_product(ahead->x->data, &ahead->norm);
+    if (!formed) {
+        if (ahead) ahead->by_itself();
+        formed = in_product(x->data, nullptr);
+    }
+    if (!formed) {
+        if (!keep) gu = Tensor::make(N, 2 * ff, dtype);
+        gemm(x->data, false, Wgu, false, gu.ptr(), dtype, N, 2 * ff, 2 * ff, 0.0f);
+        k_silu_mul_cat_fwd(gu, h);
+    }
+    Tensor y = Tensor::make(N, down->data.cols, dtype);
+    if (result_needed || !grad_enabled()) add_product(r->data, h, shadow_of(down), y);
+
+    // three nodes, as the ops by themselves would leave them
+    Var both;
+    if (keep)
+        both = record(std::move(gu), {x, gate, up}, [](Variable* self) {
+            cat_gradients(self->parents[0], {self->parents[1], self->parents[2]}, self->grad);
+        });
+    Var gated = keep ? record(std::move(h), {both}, silu_mul_cat_backward) : make_var(std::move(h), false);
+    return record(std::move(y), {gated, down, r}, [](Variable* self) {
+        const Var& gated = self->parents[0];
+        if (gated->requires_grad && !gated_gradient_in_product(self->grad, self->parents[1], gated->parents[0])) product_gradient(self);
+        product_weight_gradients(self);
+    });
+}
+
+Var gated_mlp(const Var& x, const Var& gate, const Var& up, const Var& down, const Var& r, bool result_needed) {
+    return gated_mlp_of(x, gate, up, down, r, result_needed, nullptr);
+}
+Var rms_gated_mlp(const Var& x, const Var& norm_w, const Var& gate, const Var& up, const Var& down, bool result_needed) {
+    NormAhead ahead(x, norm_w);
+    return gated_mlp_of(ahead.h, gate, up, down, x, result_needed, &ahead);
+}
+
+static void check_norm(const Var& x, const Var& w) {
+    if (w->data.rows != 1 || w->data.cols != x->data.cols) shape_fail("rmsnorm: w must be [1, cols(x)]");
+}
+Var rmsnorm(const Var& x, const Var& w) {
+    check_norm(x, w);
+    auto rinv = std::make_shared<Buffer>(sizeof(float) * x->data.rows);
+    Tensor y = Tensor::make(x->data.rows, x->data.cols, x->data.dtype);
+    k_rmsnorm_fwd(x->data, w->data, 1e-5f, y, static_cast<float*>(rinv->p));
+    return norm_node(std::move(y), x, w, rinv);
+}
 
 // The node of a rotation that has been applied where qkv lies, a projection nobody else reads (a Linear's backward needs its input and
 // weight, not its output): the node shares the storage; the backward turns this node's gradient back in place and passes it on whole.
@@ -799,19 +847,26 @@ static Var rope_in_place(const Var& qkv, const std::shared_ptr<Buffer>& pos, flo
     });
 }
 
-Var linear3_rope(const Var& x, const Var& Wq, const Var& Wk, const Var& Wv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads,
-                 const std::shared_ptr<Buffer>& table, int64_t seq_len) {
+Var rms_linear3_rope(const Var& x, const Var& norm_w, const Var& Wq, const Var& Wk, const Var& Wv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim,
+                     int rot_heads, const std::shared_ptr<Buffer>& table, int64_t seq_len) {
     const int64_t M = x->data.rows, K = x->data.cols;
     const int d = static_cast<int>(Wq->data.cols);
     if (rot_heads < 1 || static_cast<int64_t>(rot_heads) * head_dim > d) throw std::runtime_error("apply_rope: head_dim must be even and <= d");
+    NormAhead ahead(x, norm_w);
     bool turned = false;
-    const Var qkv = linear_cat_by(x, {Wq, Wk, Wv}, [&](const Tensor& W, const Tensor& y) {
-        if (gemm_backend() == 0 || W.dtype != y.dtype || seq_len > (1 << 30)) return false;
+    const Var qkv = linear_cat_by(ahead.h, {Wq, Wk, Wv}, [&](const Tensor& W, const Tensor& y) {
         const Turn turn{static_cast<const float*>(table->p), static_cast<int>(seq_len), d, head_dim, rot_heads * head_dim};
-        turned = y.dtype == PK_BF16 ? gemm_mfma_turned(x->data.ptr(), W.ptr(), y.ptr(), M, K, turn, tape_stream())
-                                    : gemm_f32_is_ahead(false, M, 3 * d, K) &&
-                                          gemm_f32_turned(static_cast<const float*>(x->data.ptr()), static_cast<const float*>(W.ptr()),
-                                                          static_cast<float*>(y.ptr()), M, K, turn, tape_stream());
+        const auto in_product = [&](const Tensor& from, const Norm* norm) {
+            if (gemm_backend() == 0 || W.dtype != y.dtype || seq_len > (1 << 30)) return false;
+            if (y.dtype == PK_BF16) return gemm_mfma_turned(from.ptr(), W.ptr(), y.ptr(), M, K, turn, tape_stream(), norm);
+            return gemm_f32_is_ahead(false, M, 3 * d, K) && gemm_f32_turned(static_cast<const float*>(from.ptr()), static_cast<const float*>(W.ptr()),
+                                                                            static_cast<float*>(y.ptr()), M, K, turn, tape_stream(), norm);
+        };
+        turned = in_product(x->data, &ahead.norm);
+        if (!turned) {
+            ahead.by_itself();
+            turned = in_product(ahead.h->data, nullptr);
+        }
         return turned;
     });
     if (!turned) return apply_rope(qkv, pos, theta, head_dim, rot_heads, /*in_place=*/true);

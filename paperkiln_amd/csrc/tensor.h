@@ -105,6 +105,15 @@ struct AdamWPart {
 bool k_adamw_parts(const Tensor& p, const Tensor& g, const Tensor& m, const Tensor& v, const std::vector<AdamWPart>& parts, float lr,
                    float b1, float b2, float eps, float wd, float c1, float c2, const Clip& clip);
 
+// How a product of x's normalised rows forms them itself (k_rmsnorm_fwd): x comes as it is, w [K] goes into it, 1 / rms of a row into the
+// sums. The normalised rows (x's type) go to y and 1 / rms to rinv, where a backward pass will ask for them; both may be null.
+struct Norm {
+    const float* w;
+    float eps;
+    void* y;
+    float* rinv;
+};
+
 // C[M,N] (+)= op(A) . op(B), row-major, bf16 or fp32 operands, fp32 accumulate
 // (device::gemm, src/device.cpp:91-125). C may be a column slice of a wider
 // matrix (ldc). beta is 0 or 1.
@@ -171,17 +180,17 @@ bool gemm_f32_held_is_ahead(int64_t M, int64_t N, int64_t K);      // the same f
 // SwiGLU inside the products beside it, row-major without gaps. *_gated: h [M, N] = silu(x gate) .* (x up) for x [M, K] and
 // w = [gate | up] [K, 2 N], and [x gate | x up] to gu unless that is null. *_gated_grad: d = dy w^T (dy [M, K], w [N, K]) is
 // the gradient of silu(gate) .* up; that of gu = [gate | up] goes to dgu. False, with nothing done, for what they do not take.
-bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_f32_gated(const float* x, const float* w, float* gu, float* h, int64_t M, int64_t N, int64_t K, hipStream_t st, const Norm* norm = nullptr);
 bool gemm_f32_gated_grad(const float* dy, const float* w, const float* gu, float* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
-bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_small_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st, const Norm* norm = nullptr);
 bool gemm_small_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
-bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_mfma_gated(const void* x, const void* w, void* gu, void* h, int64_t M, int64_t N, int64_t K, hipStream_t st, const Norm* norm = nullptr);
 bool gemm_mfma_gated_grad(const void* dy, const void* w, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K, hipStream_t st);
 // y [M, 3 d] = x w (x [M, K], w [K, 3 d], row-major without gaps) with q and k turned, y of the operands' type. False, with nothing
 // done, for what they do not take.
-bool gemm_f32_turned(const float* x, const float* w, float* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st);
-bool gemm_small_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st);
-bool gemm_mfma_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st);
+bool gemm_f32_turned(const float* x, const float* w, float* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st, const Norm* norm = nullptr);
+bool gemm_small_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st, const Norm* norm = nullptr);
+bool gemm_mfma_turned(const void* x, const void* w, void* y, int64_t M, int64_t K, const Turn& turn, hipStream_t st, const Norm* norm = nullptr);
 int64_t gemm_head_spans(int64_t M, int64_t N);
 bool gemm_head_takes(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 bool gemm_head_rows(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const int* target,

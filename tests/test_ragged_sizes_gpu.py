@@ -89,11 +89,14 @@ def test_fp32_gated_product_in_its_projections(d, ff, tokens, seq):
 @pytest.mark.parametrize("dtype,d,heads,tokens,seq", [
     ("fp32", 64, 2, 33, 11), ("fp32", 96, 3, 77, 0), ("fp32", 128, 4, 516, 129), ("fp32", 192, 3, 300, 30), ("fp32", 256, 4, 1025, 205),
     ("fp32", 24, 2, 70, 7), ("bf16", 64, 2, 33, 11), ("bf16", 128, 4, 516, 129), ("bf16", 24, 2, 70, 7), ("bf16", 256, 4, 2050, 410),
-    ("bf16", 320, 5, 2112, 33), ("bf16", 512, 8, 2048, 127 + 1), ("bf16", 512, 16, 1400, 100), ("bf16", 384, 3, 3001, 3001)])
-def test_rope_in_the_projection(dtype, d, heads, tokens, seq, all_heads):
-    """q and k turned on their way out of the q|k|v product, from a table, against the pass of its own beside the library's product: tiles of
-    16 to 128 rows of sequences shorter and longer than one, thirds that end inside a tile, head sizes that are no multiple of 8, and a
-    second pass with longer sequences than the table has."""
+    ("bf16", 320, 5, 2112, 33), ("bf16", 512, 8, 2048, 128), ("bf16", 512, 16, 1400, 100), ("bf16", 384, 3, 3001, 3001),
+    ("fp32", 40, 5, 50, 10), ("fp32", 512, 8, 100, 25), ("fp32", 448, 7, 17, 17), ("fp32", 100, 5, 1100, 55), ("fp32", 128, 2, 1700, 85),
+    ("bf16", 40, 5, 50, 10), ("bf16", 100, 5, 1100, 55), ("bf16", 512, 8, 17, 17), ("bf16", 68, 1, 200, 40)])
+def test_norm_and_rope_in_the_projection(dtype, d, heads, tokens, seq, all_heads):
+    """Rows normalised where the q|k|v and gate|up products load them, kept and not kept, and q and k turned on their way out, from a table,
+    against the passes of their own beside the library's products: tiles of 16 to 128 rows of sequences shorter and longer than one, thirds
+    that end inside a tile, widths below a chunk of the contraction, beside one and past what a workgroup holds of it at once, head sizes that
+    are no multiple of 8, and a second pass with longer sequences than the table has."""
     m = Llama(vocab=130, d=d, n_layers=1, n_heads=heads, d_ff=2 * d, compute_dtype=dtype, rope_all_heads=all_heads, seed=8)
     toks = synth.randint(3, tokens + 1, 130)
     tol = 1e-5 if dtype == "fp32" else 2e-2
