@@ -1004,18 +1004,23 @@ __global__ void ce_rows(T* logits, const int* targets, float gscale, float* nll,
 // The same row operation for the chunked head (fp32 logits, vocabulary a multiple of 4 and at most
 // 32768): 1024 threads hold the whole row in registers, so the logits are read ONCE; the forward pass
 // writes nothing but the row's nll, the backward writes dlogits straight in the GEMM's operand type.
+// Rows of up to 2048 words are a wavefront's, four to a workgroup: nothing waits for another wavefront (512 rows of 512 words CE_SMALL).
 constexpr int CE_NT = 1024, CE_V4 = 8;  // 8 float4 per thread
-template <typename TOut, bool WRITE>
-__global__ __launch_bounds__(CE_NT) void ce_rows_reg(const float* logits, TOut* dl, const int* targets, float gscale,
-                                                     float* nll, int C, int64_t dl_ld) {
-    __shared__ float sh[CE_NT / 64];
-    const float* row = logits + static_cast<int64_t>(blockIdx.x) * C;
-    const int t = targets[blockIdx.x];
+template <typename TOut, bool WRITE, int ROW_NT>
+__global__ __launch_bounds__(ROW_NT > 256 ? ROW_NT : 256) void ce_rows_reg(const float* logits, TOut* dl, const int* targets, float gscale,
+                                                                           float* nll, int C, int64_t dl_ld, int64_t rows) {
+    static_assert(ROW_NT == 64 || ROW_NT == CE_NT, "a row to a wavefront or to a workgroup");
+    __shared__ float sh[ROW_NT / 64];
+    const int64_t r_ = ROW_NT == 64 ? blockIdx.x * static_cast<int64_t>(4) + (threadIdx.x >> 6) : blockIdx.x;
+    if (r_ >= rows) return;
+    const int tid = static_cast<int>(threadIdx.x) % ROW_NT;
+    const float* row = logits + r_ * C;
+    const int t = targets[r_];
     f32x4 v[CE_V4];
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < CE_V4; ++i) {
-        const int j = (threadIdx.x + i * CE_NT) * 4;
+        const int j = (tid + i * ROW_NT) * 4;
         if (j < C) {
             v[i] = *reinterpret_cast<const f32x4*>(row + j);
             mx = fmaxf(fmaxf(mx, fmaxf(v[i][0], v[i][1])), fmaxf(v[i][2], v[i][3]));
@@ -1026,18 +1031,19 @@ __global__ __launch_bounds__(CE_NT) void ce_rows_reg(const float* logits, TOut* 
             const float y = __shfl_xor(x, o);
             x = is_max ? fmaxf(x, y) : x + y;
         }
+        if constexpr (ROW_NT == 64) return x;
         __syncthreads();  // sh is reused
         if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
         __syncthreads();
         float r = sh[0];
-        for (int w = 1; w < CE_NT / 64; ++w) r = is_max ? fmaxf(r, sh[w]) : r + sh[w];
+        for (int w = 1; w < ROW_NT / 64; ++w) r = is_max ? fmaxf(r, sh[w]) : r + sh[w];
         return r;
     };
     mx = reduce(mx, true);
     float z = 0.0f;
 #pragma unroll
     for (int i = 0; i < CE_V4; ++i) {
-        const int j = (threadIdx.x + i * CE_NT) * 4;
+        const int j = (tid + i * ROW_NT) * 4;
         if (j < C) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -1050,16 +1056,16 @@ __global__ __launch_bounds__(CE_NT) void ce_rows_reg(const float* logits, TOut* 
     const float inv = 1.0f / z;
 #pragma unroll
     for (int i = 0; i < CE_V4; ++i) {
-        const int j = (threadIdx.x + i * CE_NT) * 4;
+        const int j = (tid + i * ROW_NT) * 4;
         if (j < C) {
-            if (t >= j && t < j + 4) nll[blockIdx.x] = -logf(fmaxf(v[i][t - j] * inv, 1e-12f));
+            if (t >= j && t < j + 4) nll[r_] = -logf(fmaxf(v[i][t - j] * inv, 1e-12f));
             if (WRITE) {
                 float o[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[e] = (v[i][e] * inv - (j + e == t ? 1.0f : 0.0f)) * gscale;
                 // dl may be the logits buffer itself (bf16 rows written over the fp32 row they came from):
                 // every thread of the row has its logits in registers since before the first reduction
-                TOut* dst = dl + static_cast<int64_t>(blockIdx.x) * dl_ld + j;
+                TOut* dst = dl + r_ * dl_ld + j;
                 if (sizeof(TOut) == 4) {
                     f32x4 w = {o[0], o[1], o[2], o[3]};
                     *reinterpret_cast<f32x4*>(dst) = w;
@@ -1108,8 +1114,18 @@ __global__ __launch_bounds__(1024) void mean_f32_k(const float* x, int64_t n, fl
         if (pinned) *pinned = mean;
     }
 }
+// the sum of a workgroup's NT values, one barrier (a tree in LDS has eight, a microsecond of a small launch)
+__device__ inline double block_sum(double s, double (&sh)[NT / 64]) {
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = sh[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) s += sh[w];
+    return s;
+}
 __global__ void sumsq_part(const float* x, int64_t n, double* part) {
-    __shared__ double sh[NT];
+    __shared__ double sh[NT / 64];
     double s = 0.0;
     if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {  // 16 bytes a lane, four chains of additions
         const int64_t n4 = n / 4;
@@ -1128,33 +1144,27 @@ __global__ void sumsq_part(const float* x, int64_t n, double* part) {
         for (int64_t i = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * NT)
             s += static_cast<double>(x[i]) * x[i];
     }
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = NT / 2; o >= 1; o >>= 1) {
-        if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    s = block_sum(s, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 // The clip of ops::clip_grad_norm (src/ops.cpp:1047-1062) from the partial sums of squares: the norm in double, what the
 // gradients are to be multiplied by, and the norm itself for the host (pinned memory). It stays on the device: the
 // optimizer step behind it reads it there, where a copy to the host and back between the two left the GPU idle for 35 to
 // 50 us a step.
-__device__ float clip_of(const double* part, int n, float max_norm, double (&sh)[NT], float* norm) {
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += NT) s += part[i];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = NT / 2; o >= 1; o >>= 1) {
-        if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-        __syncthreads();
+__device__ float clip_of(const double* part, int n, float max_norm, double (&sh)[NT / 64], float* norm) {
+    double q[SUMSQ_MAX_PARTS / NT];  // all on their way together
+#pragma unroll
+    for (int k = 0; k < SUMSQ_MAX_PARTS / NT; ++k) {
+        const int i = threadIdx.x + k * NT;
+        q[k] = i < n ? part[i] : 0.0;
     }
-    const double total = sqrt(sh[0]), limit = static_cast<double>(max_norm);
+    const double total = sqrt(block_sum((q[0] + q[1]) + (q[2] + q[3]), sh)), limit = static_cast<double>(max_norm);
     if (norm && threadIdx.x == 0) *norm = static_cast<float>(total);
     return total > limit && total > 0.0 ? static_cast<float>(limit / total) : 1.0f;
 }
+static_assert(SUMSQ_MAX_PARTS == 4 * NT, "four partial sums a thread");
 __global__ void clip_factor_k(const double* part, int n, float max_norm, float* factor, float* norm_out) {
-    __shared__ double sh[NT];
+    __shared__ double sh[NT / 64];
     const float f = clip_of(part, n, max_norm, sh, norm_out);
     if (threadIdx.x == 0) *factor = f;
 }
@@ -1197,24 +1207,26 @@ struct AdamWParts {
 };
 //
 // OWN_CLIP: every workgroup forms the clip's factor from the partial sums itself, block 0 writes the norm. Up to 1024 workgroups that costs
-// less than a launch before this one (0.46 M parameters: 2.8 us and the gap between two against 1 us).
+// less than a launch before this one (0.46 M parameters: 2.8 us and the gap between two against 1 us); what a thread updates is on its way meanwhile.
 template <typename TY, bool OWN_CLIP>
 __global__ void adamw_parts_k(AdamWParts ps, float* p, float* g, float* m, float* v, float lr, float b1, float b2, float eps, float wd,
                               float c1, float c2, Clip cl) {
-    float own = 1.0f;
-    if constexpr (OWN_CLIP) {
-        __shared__ double sh[NT];
-        own = clip_of(cl.part_dev, cl.n, cl.max_norm, sh, blockIdx.x == 0 ? cl.norm_pinned : nullptr);
-    }
     const int block = static_cast<int>(blockIdx.x);
     const int j = __builtin_popcountll(__builtin_amdgcn_ballot_w64(block >= ps.begin[threadIdx.x & 63])) - 1;
     const AdamWParts::Part part = ps.part[j];
     const int e = ((block - ps.begin[j]) * NT + static_cast<int>(threadIdx.x)) * 4;
-    if (e >= part.count) return;
-    const float gs = OWN_CLIP ? own : cl.factor ? *cl.factor : 1.0f;
-    const int64_t i = part.at + e;
+    const bool mine = e < part.count;
+    const int64_t i = part.at + (mine ? e : 0);
     auto at = [&](float* s) -> f32x4& { return *reinterpret_cast<f32x4*>(s + i); };
     f32x4 gi = at(g), mi = at(m), vi = at(v), pi = at(p);
+    float gs;
+    if constexpr (OWN_CLIP) {
+        __shared__ double sh[NT / 64];
+        gs = clip_of(cl.part_dev, cl.n, cl.max_norm, sh, blockIdx.x == 0 ? cl.norm_pinned : nullptr);
+    } else {
+        gs = cl.factor ? *cl.factor : 1.0f;
+    }
+    if (!mine) return;
     if (gs != 1.0f) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) gi[k] *= gs;
@@ -1684,16 +1696,21 @@ bool k_ce_rows_once(const Tensor& logits, const int* targets, float gscale, floa
     if (dl_ld == 0) dl_ld = C;
     if (logits.dtype != PK_F32 || C % 4 != 0 || C > CE_NT * CE_V4 * 4) return false;  // caller takes the generic kernel
     const float* src = static_cast<const float*>(logits.ptr());
-    if (!dl) {
-        hipLaunchKernelGGL((ce_rows_reg<float, false>), dim3(logits.rows), dim3(CE_NT), 0, tape_stream(), src,
-                           static_cast<float*>(nullptr), targets, gscale, nll_rows, C, dl_ld);
-    } else if (dl->dtype == PK_F32) {
-        hipLaunchKernelGGL((ce_rows_reg<float, true>), dim3(logits.rows), dim3(CE_NT), 0, tape_stream(), src,
-                           static_cast<float*>(dl->ptr()), targets, gscale, nll_rows, C, dl_ld);
-    } else {
-        hipLaunchKernelGGL((ce_rows_reg<uint16_t, true>), dim3(logits.rows), dim3(CE_NT), 0, tape_stream(), src,
-                           static_cast<uint16_t*>(dl->ptr()), targets, gscale, nll_rows, C, dl_ld);
-    }
+    const auto launch = [&](auto* out, auto write, auto row_threads) {
+        using TOut = std::remove_pointer_t<decltype(out)>;
+        constexpr int ROW_NT = decltype(row_threads)::value;
+        hipLaunchKernelGGL((ce_rows_reg<TOut, decltype(write)::value, ROW_NT>), dim3(static_cast<unsigned>(ROW_NT == 64 ? (logits.rows + 3) / 4 : logits.rows)),
+                           dim3(ROW_NT == 64 ? 256 : ROW_NT), 0, tape_stream(), src, out, targets, gscale, nll_rows, C, dl_ld, logits.rows);
+    };
+    const auto by_length = [&](auto* out, auto write) {
+        C <= 64 * CE_V4 * 4 ? launch(out, write, std::integral_constant<int, 64>{}) : launch(out, write, std::integral_constant<int, CE_NT>{});
+    };
+    if (!dl)
+        by_length(static_cast<float*>(nullptr), std::false_type{});
+    else if (dl->dtype == PK_F32)
+        by_length(static_cast<float*>(dl->ptr()), std::true_type{});
+    else
+        by_length(static_cast<uint16_t*>(dl->ptr()), std::true_type{});
     post();
     return true;
 }
@@ -1714,7 +1731,7 @@ double k_sum_f32_to_host(const float* x, int64_t n) {
 }
 int k_sumsq_parts(const Tensor& g, double* part_dev) {
     if (g.dtype != PK_F32) throw std::runtime_error("clip_grad_norm: gradients must be fp32");
-    const int nb = static_cast<int>(std::min<int64_t>((g.numel() + NT - 1) / NT, SUMSQ_MAX_PARTS));
+    const int nb = static_cast<int>(std::min<int64_t>((g.numel() + 4 * NT - 1) / (4 * NT), SUMSQ_MAX_PARTS));
     hipLaunchKernelGGL(sumsq_part, dim3(nb), dim3(NT), 0, tape_stream(), static_cast<const float*>(g.ptr()), g.numel(),
                        part_dev);
     post();
