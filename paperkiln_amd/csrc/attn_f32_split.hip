@@ -132,10 +132,10 @@ __device__ inline void accumulate_tr32(const float* tile, const f32x16& c, f32x1
 }
 
 // a quad of a lane's output row
-__device__ inline void store_quad(void* base, int64_t row_off, int db, int qd, int g, const f32x4& v, float sc, int dk) {
+__device__ inline void store_quad(void* base, int64_t row_off, int db, int qd, int g, const f32x4& v, float sc, int dk, const TurnRow& turn = {}) {
     const int col = 32 * db + 8 * qd + 4 * g;
     const f32x4 o = {v[0] * sc, v[1] * sc, v[2] * sc, v[3] * sc};
-    if (col < dk) *reinterpret_cast<f32x4*>(static_cast<float*>(base) + row_off + col) = o;
+    if (col < dk) *reinterpret_cast<f32x4*>(static_cast<float*>(base) + row_off + col) = turn.quad(o, col, dk);
 }
 
 // Both tensors of a wavefront's next tile on their way together, or one behind the other's product. Where chains are a tile or two, as in
@@ -251,7 +251,7 @@ constexpr int dq_lds() {  // floats
     constexpr int TILE = 2 * 32 * (D + 4), RED = KW * (D / 32) * 1024;
     return KW * TILE > RED ? KW * TILE : RED;
 }
-template <int D, int KW, bool BOTH>
+template <int D, int KW, bool BOTH, bool TURN = false>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float* lds) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P;
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -325,7 +325,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int id, float
     __syncthreads();  // every wavefront has read its last tile
     const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
     join_shares<DB, KW, 1>(acc, lds, kg, lane, no_weights, [&](int db, int qd, const f32x4 (&v)[1]) {
-        if (qi < a.T) store_quad(a.dq, ro, db, qd, g, v[0], a.scale, dk);
+        if (qi < a.T) store_quad(a.dq, ro, db, qd, g, v[0], a.scale, dk, turn_row<TURN>(a, h, qi));
     });
 }
 template <int D, int KW>
@@ -350,7 +350,7 @@ constexpr int dkdv_lds() {  // floats
     constexpr int TILE = 2 * 32 * (D + 4) + 64, RED = 2 * KW * (D / 32) * 1024;
     return (K_IN_LDS<D> + V_IN_LDS<D>) * 32 * (D + 4) + (KW * TILE > RED ? KW * TILE : RED);
 }
-template <int D, int KW, bool OWN_DELTA>
+template <int D, int KW, bool OWN_DELTA, bool TURN = false>
 __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     constexpr int DB = D / 32, P = D + 4, TILE = 2 * 32 * P + 64;
     constexpr bool BOTH = D == 32 && OWN_DELTA;
@@ -508,7 +508,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int id, float* lds) {
     void* const dst_v = scratch ? room : a.dv;
     void* const dst_k = scratch ? room : a.dk;
     join_shares<2 * DB, KW, 1>(acc, lds + KVB, kg, lane, no_weights, [&](int n, int qd, const f32x4 (&v)[1]) {
-        if (mine) store_quad(n < DB ? dst_v : dst_k, n < DB ? rv : rk, n < DB ? n : n - DB, qd, g, v[0], n < DB ? 1.0f : a.scale, dk);
+        if (mine) store_quad(n < DB ? dst_v : dst_k, n < DB ? rv : rk, n < DB ? n : n - DB, qd, g, v[0], n < DB ? 1.0f : a.scale, dk, n < DB ? TurnRow() : turn_row<TURN>(a, hk, kj));
     });
 }
 template <int D, int KW>
@@ -521,16 +521,16 @@ __global__ __launch_bounds__(64 * KW, D <= 32 && KW == 4 ? 3 : D <= 64 ? 2 : 1) 
 // ---- dK, dV and dQ in one launch ----
 // Two launches of a handful of workgroups each, the second waiting for the first one's delta, are two round trips to memory with
 // most CUs idle. Here blocks 0 .. dkdv_ids - 1 are the dK/dV launch's, which forms its own delta, and the others the dQ launch's.
-template <int D>
+template <int D, bool TURN>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_split_bwd(AttnArgs a, int dkdv_ids) {
     all_arguments(a);
     constexpr int Q = dq_lds<D, 4>(), K = dkdv_lds<D, 4>();
     __shared__ __attribute__((aligned(16))) float lds[Q > K ? Q : K];
     const int id = static_cast<int>(blockIdx.x);
     if (id < dkdv_ids)
-        dkdv_block<D, 4, true>(a, id, lds);
+        dkdv_block<D, 4, true, TURN>(a, id, lds);
     else
-        dq_block<D, 4, D == 32>(a, 1, id - dkdv_ids, lds);
+        dq_block<D, 4, D == 32, TURN>(a, 1, id - dkdv_ids, lds);
 }
 
 // A block's tiles split between four or eight wavefronts, or not this kernel.
@@ -617,7 +617,11 @@ void run_dkdv(const AttnArgs& a, hipStream_t st) {
 
 template <int D>
 void run_bwd(const OneLaunch& l, hipStream_t st) {
-    hipLaunchKernelGGL(f32_split_bwd<D>, dim3(l.dkdv_ids + l.dq_ids), dim3(256), 0, st, l.a, l.dkdv_ids);
+    const dim3 grid(l.dkdv_ids + l.dq_ids);
+    if (l.a.turn)
+        hipLaunchKernelGGL((f32_split_bwd<D, true>), grid, dim3(256), 0, st, l.a, l.dkdv_ids);
+    else
+        hipLaunchKernelGGL((f32_split_bwd<D, false>), grid, dim3(256), 0, st, l.a, l.dkdv_ids);
 }
 
 }  // namespace

@@ -80,13 +80,13 @@ __device__ inline bf16x8 tr_operand(const uint16_t* plane, int row0, int db, int
 }
 // store_block of attn_split.h in this column order, fp32
 template <int D>
-__device__ inline void store_block32(void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
+__device__ inline void store_block32(void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk, const TurnRow& turn = {}) {
     float* row = static_cast<float*>(base) + row_off;
 #pragma unroll
     for (int qd = 0; qd < 4; ++qd) {
         const int col = tr_col0<D>(db, qd, g);
         const f32x4 v = {acc[qd * 4] * sc, acc[qd * 4 + 1] * sc, acc[qd * 4 + 2] * sc, acc[qd * 4 + 3] * sc};
-        if (col < dk) *reinterpret_cast<f32x4*>(row + col) = v;
+        if (col < dk) *reinterpret_cast<f32x4*>(row + col) = turn.quad(v, col, dk);
     }
 }
 
@@ -580,7 +580,7 @@ constexpr int dq_lds() {  // in uint16
     constexpr int TILES = BUFS<D, QW, KW> * KW * 6 * Mover3<D, 64 * QW>::PLANE, RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
     return TILES > RED ? TILES : RED;
 }
-template <int D, int QW, int KW, bool ALL, int N>
+template <int D, int QW, int KW, bool ALL, bool TURN, int N>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h, int hk, int qblk, uint16_t (&lds)[N]) {
     constexpr int BM = 32 * QW, DB = D / 32, G = 64 * QW, NBUF = BUFS<D, QW, KW>;
     constexpr int PLANE = Mover3<D, G>::PLANE, TILE = 6 * PLANE;
@@ -675,7 +675,7 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
         const int64_t ro = b * a.dq_sb + h * a.dq_sh + qe * a.dq_st;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
-            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, ge, acc[db], sc, dk);
+            if (KW == 1 || db % KW == kg) store_block32<D>(a.dq, ro, db, ge, acc[db], sc, dk, turn_row<TURN>(a, h, qe));
     }
 }
 template <int D, int QW, int KW>
@@ -683,7 +683,7 @@ __global__ __launch_bounds__(64 * QW * KW, D <= 64 ? 2 : 1) void x3_dq(AttnArgs 
     all_arguments(a);
     __shared__ __attribute__((aligned(16))) uint16_t lds[dq_lds<D, QW, KW>()];
     int b, h, hk, qblk;
-    if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW, false>(a, fuse_delta, b, h, hk, qblk, lds);
+    if (map_query_block(a, (a.T + 32 * QW - 1) / (32 * QW), b, h, hk, qblk)) dq_block<D, QW, KW, false, false>(a, fuse_delta, b, h, hk, qblk, lds);
 }
 
 // The two products of a step that need no other go to two sets of wavefronts, as in the other dK/dV kernels: with both
@@ -713,7 +713,7 @@ __device__ inline f32x16 get_tile(const float* buf, int lane) {
 // 4096 x 4: 337 -> 323). At 128 columns there is one wavefront to a SIMD and both do it at the end of the first phase (1777; 1872).
 template <int D, int QW>
 constexpr int DKDV_TILE = 6 * Mover3<D, 64 * QW>::PLANE + 128;  // in uint16; LSE and delta of a tile's rows behind it
-template <int D, int QW, bool ALL, int N>
+template <int D, int QW, bool ALL, bool TURN, int N>
 __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, uint16_t (&lds)[N], float* pbuf) {
     constexpr int BNK = 32 * QW, DB = D / 32, G = 64 * QW;
     constexpr bool APART = D < 128;
@@ -866,7 +866,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                                                                        : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
         void* const dst = scratch ? room : role == 0 ? a.dv : a.dk;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) store_block32<D>(dst, row, db, g, acc[db], sc, dk);
+        for (int db = 0; db < DB; ++db) store_block32<D>(dst, row, db, g, acc[db], sc, dk, role == 0 ? TurnRow() : turn_row<TURN>(a, hk, kj));
     }
 }
 template <int D, int QW>
@@ -879,11 +879,11 @@ __global__ __launch_bounds__(128 * QW, 2) void x3_dkdv(AttnArgs a) {
     // block 0 of every unit first: without a band it is seen by every query, with one it owns the sink keys
     if (a.causal && nblk > 1 ? xcd_map_block_major(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu)
                              : xcd_map(nblk, a.head_split, a.Hkv * a.B, blk, rr, kvu))
-        dkdv_block<D, QW, false>(a, blk, rr, kvu, lds, pbuf);
+        dkdv_block<D, QW, false, false>(a, blk, rr, kvu, lds, pbuf);
 }
 
 // ---- dK, dV and dQ in one launch, delta read (f32x3_takes_bwd) ----
-template <int D, bool ALL>
+template <int D, bool ALL, bool TURN>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
     all_arguments(a);
     constexpr int Q = dq_lds<D, 2, 2>(), K = 2 * DKDV_TILE<D, 2>, N = Q > K + 4096 ? Q : K + 4096;
@@ -891,9 +891,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void x3_bwd(AttnArgs a) {
     const JoinedBlocks jb(a, 64);
     int rank, r, kvu;
     if (!jb.map(a, rank, r, kvu)) return;
-    if (r < a.head_split) return dkdv_block<D, 2, ALL>(a, rank, r, kvu, lds, reinterpret_cast<float*>(lds + K));
+    if (r < a.head_split) return dkdv_block<D, 2, ALL, TURN>(a, rank, r, kvu, lds, reinterpret_cast<float*>(lds + K));
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
-    dq_block<D, 2, 2, ALL>(a, 0, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    dq_block<D, 2, 2, ALL, TURN>(a, 0, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // ---- dQ above 64 columns: the same two phases ----
@@ -1089,6 +1089,13 @@ int run_dkdv(const AttnArgs& a_in, hipStream_t st) {
     return a.head_split > 1 ? launch_gqa_reduce(a, st) : a.tail ? launch_sink_tail_reduce(a, st) : PK_OK;
 }
 
+template <int D, bool ALL>
+void launch_x3_bwd(const AttnArgs& a, dim3 grid, hipStream_t st) {
+    if (a.turn)
+        hipLaunchKernelGGL((x3_bwd<D, ALL, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((x3_bwd<D, ALL, false>), grid, dim3(256), 0, st, a);
+}
 template <int D>
 int run_bwd(const AttnArgs& a_in, hipStream_t st) {
     AttnArgs a = a_in;
@@ -1097,9 +1104,9 @@ int run_bwd(const AttnArgs& a_in, hipStream_t st) {
     if (const int rc = launch_row_delta(a, false, st)) return rc;
     const dim3 grid(JoinedBlocks(a, 64).grid(a));
     if (f32x3_bwd_keeps_all(a_in))
-        hipLaunchKernelGGL((x3_bwd<D, true>), grid, dim3(256), 0, st, a);
+        launch_x3_bwd<D, true>(a, grid, st);
     else
-        hipLaunchKernelGGL((x3_bwd<D, false>), grid, dim3(256), 0, st, a);
+        launch_x3_bwd<D, false>(a, grid, st);
     PK_HIP(hipGetLastError());
     return a.head_split > 1 ? launch_gqa_reduce(a, st) : PK_OK;
 }

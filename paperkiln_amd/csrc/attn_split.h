@@ -96,26 +96,50 @@ __device__ inline const T* head_of(const void* base, int64_t sb, int b, int64_t 
     return p;
 }
 
+// A gradient's row on its way out: turned back by its position's cosines and sines where the arguments say so (AttnArgs::turn). A launch of
+// its own that did this reads and writes dQ and dK again: 3 to 5 us of a layer's backward pass, against 0.3 to 2.5 of the launch here (8 x 1024
+// tokens, 8 heads of 64, bf16: 56.3 -> 58.9 and one of 5.1 less). The others keep kernels without it: the registers that its test takes are 0.5 to
+// 0.8 % of those too.
+struct TurnRow {
+    const float* at = nullptr;
+    bool on = false;
+    TurnRow() = default;
+    __device__ TurnRow(const AttnArgs& a, int head, int row) : at(a.turn + static_cast<int64_t>(row) * a.dk_dim), on(head < a.turn_heads) {}
+    // columns col .. col + 3 (a multiple of 4)
+    __device__ f32x4 quad(f32x4 v, int col, int dk) const {
+        if (!on) return v;
+        const f32x4 t = *reinterpret_cast<const f32x4*>(at + min(col, dk - 4));
+        return f32x4{v[0] * t[0] + v[1] * t[1], v[1] * t[0] - v[0] * t[1], v[2] * t[2] + v[3] * t[3], v[3] * t[2] - v[2] * t[3]};
+    }
+};
+template <bool TURN>
+__device__ inline TurnRow turn_row(const AttnArgs& a, int head, int row) {
+    if constexpr (TURN)
+        return TurnRow(a, head, row);
+    else
+        return TurnRow();
+}
+
 // One 32 x 32 accumulator block (lane = row of the output, natural column order) scaled and written; columns past dk are
 // not. Both lanes of a pair (c, c + 32) hold the same row and must be active.
-__device__ inline void store_block(bool f32, void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk) {
+__device__ inline void store_block(bool f32, void* base, int64_t row_off, int db, int g, const f32x16& acc, float sc, int dk, const TurnRow& turn = {}) {
     if (f32) {
         float* row = static_cast<float*>(base) + row_off;
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
             const int col = 32 * db + 8 * qd + 4 * g;
             const f32x4 v = {acc[qd * 4] * sc, acc[qd * 4 + 1] * sc, acc[qd * 4 + 2] * sc, acc[qd * 4 + 3] * sc};
-            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = v;
+            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = turn.quad(v, col, dk);
         }
     } else {
         uint16_t* row = static_cast<uint16_t*>(base) + row_off;
 #pragma unroll
         for (int qp = 0; qp < 2; ++qp) {
-            const int lo = qp * 8, hi = qp * 8 + 4;
-            const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo] * sc, acc[lo + 1] * sc),
-                                                             pack_bf16(acc[hi] * sc, acc[hi + 1] * sc), false, false);
-            const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[lo + 2] * sc, acc[lo + 3] * sc),
-                                                             pack_bf16(acc[hi + 2] * sc, acc[hi + 3] * sc), false, false);
+            const int lo = qp * 8, hi = qp * 8 + 4, at = 32 * db + 16 * qp + 4 * g;
+            const f32x4 x = turn.quad(f32x4{acc[lo] * sc, acc[lo + 1] * sc, acc[lo + 2] * sc, acc[lo + 3] * sc}, at, dk),
+                        y = turn.quad(f32x4{acc[hi] * sc, acc[hi + 1] * sc, acc[hi + 2] * sc, acc[hi + 3] * sc}, at + 8, dk);
+            const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(x[0], x[1]), pack_bf16(y[0], y[1]), false, false);
+            const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(x[2], x[3]), pack_bf16(y[2], y[3]), false, false);
             const u32x4 v = {r0[0], r1[0], r0[1], r1[1]};
             const int col = 32 * db + 8 * (2 * qp + g);
             if (col < dk) *reinterpret_cast<u32x4*>(row + col) = v;
@@ -124,18 +148,22 @@ __device__ inline void store_block(bool f32, void* base, int64_t row_off, int db
 }
 
 // Quads qd and qd + 1 (even, odd) of such a block
-__device__ inline void store_half(bool f32, void* base, int64_t row_off, int db, int qd, int g, const f32x4 (&v)[2], float sc, int dk) {
+__device__ inline void store_half(bool f32, void* base, int64_t row_off, int db, int qd, int g, const f32x4 (&v)[2], float sc, int dk,
+                                  const TurnRow& turn = {}) {
     if (f32) {
         float* row = static_cast<float*>(base) + row_off;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int col = 32 * db + 8 * (qd + q) + 4 * g;
             const f32x4 o = {v[q][0] * sc, v[q][1] * sc, v[q][2] * sc, v[q][3] * sc};
-            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = o;
+            if (col < dk) *reinterpret_cast<f32x4*>(row + col) = turn.quad(o, col, dk);
         }
     } else {
-        const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(v[0][0] * sc, v[0][1] * sc), pack_bf16(v[1][0] * sc, v[1][1] * sc), false, false);
-        const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(v[0][2] * sc, v[0][3] * sc), pack_bf16(v[1][2] * sc, v[1][3] * sc), false, false);
+        const int at = 32 * db + 8 * qd + 4 * g;
+        const f32x4 x = turn.quad(f32x4{v[0][0] * sc, v[0][1] * sc, v[0][2] * sc, v[0][3] * sc}, at, dk),
+                    y = turn.quad(f32x4{v[1][0] * sc, v[1][1] * sc, v[1][2] * sc, v[1][3] * sc}, at + 8, dk);
+        const auto r0 = __builtin_amdgcn_permlane32_swap(pack_bf16(x[0], x[1]), pack_bf16(y[0], y[1]), false, false);
+        const auto r1 = __builtin_amdgcn_permlane32_swap(pack_bf16(x[2], x[3]), pack_bf16(y[2], y[3]), false, false);
         const u32x4 o = {r0[0], r1[0], r0[1], r1[1]};
         const int col = 32 * db + 8 * (qd + g);
         if (col < dk) *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(base) + row_off + col) = o;

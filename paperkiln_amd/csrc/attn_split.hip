@@ -353,7 +353,7 @@ constexpr int dq_lds() {  // in uint16
     constexpr int TILES = (QW > 1 ? 2 : 1) * KW * 2 * 32 * NB * (D + 8), RED = KW > 1 ? QW * KW * (D / 32) * 2048 : 0;
     return TILES > RED ? TILES : RED;
 }
-template <int D, int QW, int KW, int NB, bool EXACT, bool MINUS_DELTA = FROM_DELTA<D, EXACT> && (QW > 1 || KW == 8)>
+template <int D, int QW, int KW, int NB, bool EXACT, bool MINUS_DELTA = FROM_DELTA<D, EXACT> && (QW > 1 || KW == 8), bool TURN = false>
 __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h, int hk, int qblk, uint16_t* lds) {
     constexpr int BM = 32 * QW, BN = 32 * NB, KK = D / 16, DB = D / 32, G = 64 * QW, S = D + 8;
     constexpr int TILE = 2 * BN * S, NBUF = QW > 1 ? 2 : 1;
@@ -445,11 +445,11 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
     const int64_t ro = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
     if constexpr (KW > 1)
         join_shares<DB, KW, 2>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane, no_weights, [&](int db, int qd, const f32x4 (&v)[2]) {
-            if (qi < a.T) store_half(a.grad_f32 != 0, a.dq, ro, db, qd, g, v, a.scale, dk);
+            if (qi < a.T) store_half(a.grad_f32 != 0, a.dq, ro, db, qd, g, v, a.scale, dk, turn_row<TURN>(a, h, qi));
         });
     else if (qi < a.T)
 #pragma unroll
-        for (int db = 0; db < DB; ++db) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk);
+        for (int db = 0; db < DB; ++db) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk, turn_row<TURN>(a, h, qi));
 }
 template <int D, int QW, int KW, int NB, bool EXACT>
 __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
@@ -483,7 +483,7 @@ constexpr int dkdv_lds() {  // in uint16; LSE and delta of a tile's rows behind 
     constexpr int TILES = (QW > 1 ? 2 : 1) * KW * (2 * 32 * NB * (D + 8) + 128 * NB), RED = KW > 1 ? QW * KW * (D / 32) * (JOIN_BOTH<D> ? 4096 : 2048) : 0;
     return TILES > RED ? TILES : RED;
 }
-template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA, bool MINUS_DELTA = FROM_DELTA<D, EXACT>>
+template <int D, int QW, int KW, int NB, bool EXACT, bool OWN_DELTA, bool MINUS_DELTA = FROM_DELTA<D, EXACT>, bool TURN = false>
 __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, uint16_t* lds) {
     // a lane holds the row of O whose row of dO its wavefront has just written; or the chunks of O beside its chunks of dO
     static_assert(!OWN_DELTA || (QW == 1 && NB == 1) || (QW > 1 && (D == 32 || D == 64)), "a row's chunks are in 4 or 8 neighbouring lanes");
@@ -673,7 +673,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
             if (n0 > 0) __syncthreads();
             join_shares<N, KW, 2>(acc + n0, reinterpret_cast<float*>(lds) + qg * KW * N * 1024, kg, lane, no_weights, [&](int n, int qd, const f32x4 (&v)[2]) {
                 const bool is_v = n0 + n < DB;
-                if (mine) store_half(f32, is_v ? dst_v : dst_k, is_v ? rv : rk, is_v ? n : n0 + n - DB, qd, g, v, is_v ? 1.0f : a.scale, dk);
+                if (mine) store_half(f32, is_v ? dst_v : dst_k, is_v ? rv : rk, is_v ? n : n0 + n - DB, qd, g, v, is_v ? 1.0f : a.scale, dk, is_v ? TurnRow() : turn_row<TURN>(a, hk, kj));
             });
         }
     } else if (mine) {
@@ -682,7 +682,7 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
             if (n < DB)
                 store_block(f32, dst_v, rv, n, g, acc[n], 1.0f, dk);
             else
-                store_block(f32, dst_k, rk, n - DB, g, acc[n], a.scale, dk);
+                store_block(f32, dst_k, rk, n - DB, g, acc[n], a.scale, dk, turn_row<TURN>(a, hk, kj));
         }
     }
 }
@@ -696,7 +696,7 @@ __global__ __launch_bounds__(64 * QW * KW, OCC) void split_dkdv(AttnArgs a) {
 
 // ---- dK, dV and dQ in one launch, as in attn_f32_split.hip ----
 // Blocks 0 .. dkdv_ids - 1 are the dK/dV launch's, which forms its own delta, and the others the dQ launch's.
-template <int D, bool EXACT>
+template <int D, bool EXACT, bool TURN>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, int dkdv_ids) {
     all_arguments(a);
     constexpr int Q = dq_lds<D, 1, 4, 1>(), K = dkdv_lds<D, 1, 4, 1>();
@@ -704,16 +704,16 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void split_bwd(AttnArgs a, in
     const int id = static_cast<int>(blockIdx.x);
     int blk, rr, kvu, b, h, hk, qblk;
     if (id < dkdv_ids) {
-        if (map_key_block(a, 32, blk, rr, kvu, id)) dkdv_block<D, 1, 4, 1, EXACT, true>(a, blk, rr, kvu, lds);
+        if (map_key_block(a, 32, blk, rr, kvu, id)) dkdv_block<D, 1, 4, 1, EXACT, true, FROM_DELTA<D, EXACT>, TURN>(a, blk, rr, kvu, lds);
     } else if (map_query_block(a, (a.T + 31) / 32, b, h, hk, qblk, id - dkdv_ids)) {
-        dq_block<D, 1, 4, 1, EXACT>(a, 1, b, h, hk, qblk, lds);
+        dq_block<D, 1, 4, 1, EXACT, false, TURN>(a, 1, b, h, hk, qblk, lds);
     }
 }
 
 // ---- the same of wavefronts that own their rows (split_takes_joined) ----
 // dK/dV forms delta from the chunks of O beside those of dO while it moves a tile (up to 64 columns, whose chunks are in 4 or 8 neighbouring
 // lanes; above, it is read): a launch of delta before this one cost 4 us more, of 13 to 60.
-template <int D, bool EXACT, bool DQ_MINUS, bool DKDV_MINUS>
+template <int D, bool EXACT, bool DQ_MINUS, bool DKDV_MINUS, bool TURN>
 __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     all_arguments(a);
     constexpr bool OWN_DELTA = D <= 64;
@@ -722,9 +722,9 @@ __global__ __launch_bounds__(256, 2) void split_joined(AttnArgs a) {
     const JoinedBlocks jb(a, 128);
     int rank, r, kvu;
     if (!jb.map(a, rank, r, kvu)) return;
-    if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA, DKDV_MINUS>(a, rank, r, kvu, lds);
+    if (r < a.head_split) return dkdv_block<D, 4, 1, 2, EXACT, OWN_DELTA, DKDV_MINUS, TURN>(a, rank, r, kvu, lds);
     const int b = quotient(kvu, a.Hkv), hk = kvu - b * a.Hkv;
-    dq_block<D, 4, 1, 2, EXACT, DQ_MINUS>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
+    dq_block<D, 4, 1, 2, EXACT, DQ_MINUS, TURN>(a, OWN_DELTA, b, hk * (jb.each - a.head_split) + r - a.head_split, hk, jb.ranks - 1 - rank, lds);
 }
 
 // How a launch shares its work out: four wavefronts with 32 rows each (WIDE; in tiles of 32, SHORT) or two (HALF), or one block of
@@ -950,7 +950,11 @@ int dkdv_of(const AttnArgs& a, Form f, hipStream_t st) {
 }
 template <int D, bool EXACT>
 int bwd_of(const OneLaunch& l, hipStream_t st) {
-    hipLaunchKernelGGL((split_bwd<D, EXACT>), dim3(l.dkdv_ids + l.dq_ids), dim3(256), 0, st, l.a, l.dkdv_ids);
+    const dim3 grid(l.dkdv_ids + l.dq_ids);
+    if (l.a.turn)
+        hipLaunchKernelGGL((split_bwd<D, EXACT, true>), grid, dim3(256), 0, st, l.a, l.dkdv_ids);
+    else
+        hipLaunchKernelGGL((split_bwd<D, EXACT, false>), grid, dim3(256), 0, st, l.a, l.dkdv_ids);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -1046,7 +1050,11 @@ bool split_takes_joined(const AttnArgs& a) {
 }
 template <int D, bool EXACT, bool DQ_MINUS = false, bool DKDV_MINUS = false>
 int joined_of(const AttnArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL((split_joined<D, EXACT, DQ_MINUS, DKDV_MINUS>), dim3(JoinedBlocks(a, 128).grid(a)), dim3(256), 0, st, a);
+    const dim3 grid(JoinedBlocks(a, 128).grid(a));
+    if (a.turn)
+        hipLaunchKernelGGL((split_joined<D, EXACT, DQ_MINUS, DKDV_MINUS, true>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((split_joined<D, EXACT, DQ_MINUS, DKDV_MINUS, false>), grid, dim3(256), 0, st, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }

@@ -135,7 +135,16 @@ size_t part_bytes(const pk_attn_shape* s) {
 
 int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k, const pk_tensor4* v,
                const pk_tensor4* o, const float* lse, const pk_tensor4* d_o, const pk_tensor4* dq, const pk_tensor4* dk,
-               const pk_tensor4* dv, void* workspace, size_t workspace_bytes, int stages, bool split_heads, void* stream);
+               const pk_tensor4* dv, void* workspace, size_t workspace_bytes, int stages, bool split_heads, void* stream, TurnBack* back = nullptr);
+
+// Whether the kernels that a whole backward goes to turn dQ and dK back on their way out (AttnArgs::turn): the joined ones of wavefronts that
+// own or share their tiles, but not where partial rows are added up behind them.
+bool bwd_turns(const AttnArgs& a, bool bf16) {
+    if (a.in_place || a.Hq != a.Hkv || (a.window > 0 && a.sinks > 0) || a.dk_dim % 4) return false;
+    if (bf16 ? !split_serves(a) : !f32_mfma_supported(a)) return false;
+    const Bwd form = bf16 ? bwd_of_bf16(a) : bwd_of_f32(a);
+    return form != Bwd::APART && form != Bwd::JOINED;
+}
 
 // The bytes from the first element of a tensor to past its last.
 struct Extent {
@@ -267,7 +276,7 @@ namespace {
 
 int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k, const pk_tensor4* v,
                const pk_tensor4* o, const float* lse, const pk_tensor4* d_o, const pk_tensor4* dq, const pk_tensor4* dk,
-               const pk_tensor4* dv, void* workspace, size_t workspace_bytes, int stages, bool split_heads, void* stream) {
+               const pk_tensor4* dv, void* workspace, size_t workspace_bytes, int stages, bool split_heads, void* stream, TurnBack* back) {
     if (int rc = check_shape(s, "pk_attn_bwd")) return rc;
     if (stages <= 0 || (stages & ~PK_BWD_ALL))
         return fail(PK_ERR_ARGUMENT, "pk_attn_bwd_stages: stages must be a non-empty subset of PK_BWD_ALL");
@@ -304,6 +313,11 @@ int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
         else if (s->dtype == PK_BF16 ? split_serves(a) && bf16_deals_heads(a) : f32_mfma_supported(a) && f32_deals_heads(a))
             return fail(PK_ERR_WORKSPACE, "pk_attn_bwd: the dK/dV kernel of these tensors needs partial sums that its shape was not given");
     }
+    if (back && stages == PK_BWD_ALL && bwd_turns(a, s->dtype == PK_BF16)) {
+        a.turn = back->table;
+        a.turn_heads = back->heads;
+        back->turned = true;
+    }
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (s->dtype == PK_BF16 && split_serves(a)) return launch_mfma_bwd(a, stages, st);
     if (s->dtype == PK_F32 && f32_mfma_supported(a)) return launch_f32_mfma_bwd(a, stages, st);
@@ -311,4 +325,11 @@ int bwd_stages(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k,
 }
 
 }  // namespace
+
+int attn_bwd_turned(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k, const pk_tensor4* v, const pk_tensor4* o, const float* lse,
+                    const pk_tensor4* d_o, const pk_tensor4* dq, const pk_tensor4* dk, const pk_tensor4* dv, void* workspace, size_t workspace_bytes,
+                    TurnBack& back, void* stream) {
+    back.turned = false;
+    return bwd_stages(s, q, k, v, o, lse, d_o, dq, dk, dv, workspace, workspace_bytes, PK_BWD_ALL, true, stream, &back);
+}
 }  // namespace pk

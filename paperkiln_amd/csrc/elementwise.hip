@@ -1004,7 +1004,7 @@ __global__ void ce_rows(T* logits, const int* targets, float gscale, float* nll,
 // The same row operation for the chunked head (fp32 logits, vocabulary a multiple of 4 and at most
 // 32768): 1024 threads hold the whole row in registers, so the logits are read ONCE; the forward pass
 // writes nothing but the row's nll, the backward writes dlogits straight in the GEMM's operand type.
-// Rows of up to 2048 words are a wavefront's, four to a workgroup: nothing waits for another wavefront (512 rows of 512 words CE_SMALL).
+// Rows of up to 2048 words are a wavefront's, four to a workgroup: nothing waits for another wavefront (512 rows of 512 words 7.1 -> 4.6 us).
 constexpr int CE_NT = 1024, CE_V4 = 8;  // 8 float4 per thread
 template <typename TOut, bool WRITE, int ROW_NT>
 __global__ __launch_bounds__(ROW_NT > 256 ? ROW_NT : 256) void ce_rows_reg(const float* logits, TOut* dl, const int* targets, float gscale,

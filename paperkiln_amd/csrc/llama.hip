@@ -284,9 +284,11 @@ struct Model {
     // concat_cols nodes of :47-53 are one attention node reading heads in place.
     Var block_forward(const Block& b, const Var& x, const std::shared_ptr<Buffer>& pos, int64_t seq_len) const {
         const int dk = cfg.d / cfg.n_heads;
-        Var qkv = ops::rms_linear3_rope(x, b.ln1_w, b.q, b.k, b.v, pos, cfg.rope_theta, dk, cfg.rope_all_heads ? cfg.n_heads : 1, turns, seq_len == 0 ? x->data.rows : seq_len);
+        std::shared_ptr<ops::Turned> turned;
+        Var qkv = ops::rms_linear3_rope(x, b.ln1_w, b.q, b.k, b.v, pos, cfg.rope_theta, dk, cfg.rope_all_heads ? cfg.n_heads : 1, turns,
+                                        seq_len == 0 ? x->data.rows : seq_len, turned);
         const float sc = 1.0f / std::sqrt(static_cast<float>(dk));
-        Var x1 = ops::linear_add(ops::attention_qkv(qkv, cfg.n_heads, sc, seq_len, true, cfg.window, cfg.sinks), b.o, x);
+        Var x1 = ops::linear_add(ops::attention_turned(qkv, turned, cfg.n_heads, sc, seq_len, true, cfg.window, cfg.sinks), b.o, x);
         // re-run at backward time, the block's own output is not needed again (the gradient arrives from outside): the
         // down projection is recorded but not multiplied
         return ops::rms_gated_mlp(x1, b.ln2_w, b.gate, b.up, b.down, !recomputing());

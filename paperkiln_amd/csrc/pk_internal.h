@@ -54,6 +54,10 @@ struct AttnArgs {
     int grad_f32; // dq/dk/dv element type: 1 = fp32, 0 = bf16
     int in_place; // O (bwd: a gradient) lies where an input does, or between its rows
     float scale;
+    // bwd, where bwd_turns says so: dQ and dK of the first turn_heads heads are turned back by their rows' positions on the way out, row p of
+    // `turn` holding dk_dim / 2 pairs of cosine and sine (k_rope_table); null: they are not
+    const float* turn;
+    int turn_heads;
 };
 
 // Visible-set test shared by every kernel: the reference's two ranges
@@ -218,6 +222,15 @@ Bwd bwd_of_bf16(const AttnArgs& a);
 Bwd bwd_of_f32(const AttnArgs& a);
 // The same of a shape with aligned rows, as a number; -1 for one that the scalar kernels take. For tests.
 extern "C" int pk_bwd_of_shape(const pk_attn_shape* s);
+// The backward of tensors that RoPE turned, with its rotation undone in the same launch where the kernels do that (`turned`).
+struct TurnBack {
+    const float* table;
+    int heads;
+    bool turned;
+};
+int attn_bwd_turned(const pk_attn_shape* s, const pk_tensor4* q, const pk_tensor4* k, const pk_tensor4* v, const pk_tensor4* o, const float* lse,
+                    const pk_tensor4* d_o, const pk_tensor4* dq, const pk_tensor4* dk, const pk_tensor4* dv, void* workspace, size_t workspace_bytes,
+                    TurnBack& back, void* stream);
 bool bf16_deals_heads(const AttnArgs& a);  // its dK/dV kernel for this launch uses a.head_split and a.part
 int launch_mfma_dkdv2(const AttnArgs& a, hipStream_t st);
 bool joined_takes_bwd(const AttnArgs& a);  // attn_bwd_dkdv2.hip: dQ (with delta) and dK/dV in one launch, head_dim 128

@@ -1,6 +1,7 @@
 // Host side of the device-resident tape: see tape.h. Plain C++ driving the
 // kernels of elementwise.hip and the attention entry points of the C ABI.
 #include "tape.h"
+#include "pk_internal.h"
 
 #include <algorithm>
 #include <cmath>
@@ -837,18 +838,21 @@ Var rmsnorm(const Var& x, const Var& w) {
 
 // The node of a rotation that has been applied where qkv lies, a projection nobody else reads (a Linear's backward needs its input and
 // weight, not its output): the node shares the storage; the backward turns this node's gradient back in place and passes it on whole.
-static Var rope_in_place(const Var& qkv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads, int d) {
-    return record(Tensor(qkv->data), {qkv}, [pos, theta, head_dim, rot_heads, d](Variable* self) {
+static Var rope_in_place(const Var& qkv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads, int d,
+                         const std::shared_ptr<Turned>& turned = nullptr) {
+    return record(Tensor(qkv->data), {qkv}, [pos, theta, head_dim, rot_heads, d, turned](Variable* self) {
         const Var& x = self->parents[0];
         if (!x->requires_grad) return;
-        k_rope_inplace(self->own_grad(), static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, true);
+        if (!turned || !turned->gradient_is_back)
+            k_rope_inplace(self->own_grad(), static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, true);
+        if (turned) turned->gradient_is_back = false;
         x->accumulate_owned(std::move(self->grad));
         self->grad = Tensor();
     });
 }
 
 Var rms_linear3_rope(const Var& x, const Var& norm_w, const Var& Wq, const Var& Wk, const Var& Wv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim,
-                     int rot_heads, const std::shared_ptr<Buffer>& table, int64_t seq_len) {
+                     int rot_heads, const std::shared_ptr<Buffer>& table, int64_t seq_len, std::shared_ptr<Turned>& turned_by) {
     const int64_t M = x->data.rows, K = x->data.cols;
     const int d = static_cast<int>(Wq->data.cols);
     if (rot_heads < 1 || static_cast<int64_t>(rot_heads) * head_dim > d) throw std::runtime_error("apply_rope: head_dim must be even and <= d");
@@ -869,8 +873,11 @@ Var rms_linear3_rope(const Var& x, const Var& norm_w, const Var& Wq, const Var& 
         }
         return turned;
     });
-    if (!turned) return apply_rope(qkv, pos, theta, head_dim, rot_heads, /*in_place=*/true);
-    return rope_in_place(qkv, pos, theta, head_dim, rot_heads, d);
+    if (!turned) k_rope_inplace(qkv->data, static_cast<const int*>(pos->p), theta, d, head_dim, rot_heads, false);
+    turned_by = std::make_shared<Turned>();
+    turned_by->table = table;
+    turned_by->heads = rot_heads;
+    return rope_in_place(qkv, pos, theta, head_dim, rot_heads, d, turned_by);
 }
 
 Var apply_rope(const Var& qkv, const std::shared_ptr<Buffer>& pos, float theta, int head_dim, int rot_heads, bool in_place) {
@@ -938,6 +945,9 @@ pk_attn_shape shape_of(const AttnGeom& g, int dtype) {
 }  // namespace
 
 Var attention_qkv(const Var& qkv, int n_heads, float scale, int64_t seq_len, bool causal, int window, int sinks) {
+    return attention_turned(qkv, nullptr, n_heads, scale, seq_len, causal, window, sinks);
+}
+Var attention_turned(const Var& qkv, const std::shared_ptr<Turned>& turned, int n_heads, float scale, int64_t seq_len, bool causal, int window, int sinks) {
     const int64_t N = qkv->data.rows, d3 = qkv->data.cols;
     if (d3 % 3 != 0 || (d3 / 3) % n_heads != 0) shape_fail("fused_attention: shape mismatch");
     const int64_t d = d3 / 3, sl = seq_len == 0 ? N : seq_len;
@@ -952,7 +962,7 @@ Var attention_qkv(const Var& qkv, int n_heads, float scale, int64_t seq_len, boo
                      v4 = view4(qkv->data.ptr(), 2 * d, es, sl * d3, d3, g.dk), o4 = view4(o.ptr(), 0, es, sl * d, d, g.dk);
     attn_check(pk_attn_fwd(&sh, &q4, &k4, &v4, &o4, static_cast<float*>(lse->p), tape_stream()));
     // The node keeps O (its own data) and LSE; P is rebuilt from Q, K and LSE in backward.
-    return record(std::move(o), {qkv}, [g, lse](Variable* self) {
+    return record(std::move(o), {qkv}, [g, lse, turned](Variable* self) {
         const Var& qkv = self->parents[0];
         if (!qkv->requires_grad) return;
         const int64_t N = qkv->data.rows, d3 = qkv->data.cols, d = d3 / 3, sl = g.T;
@@ -966,8 +976,15 @@ Var attention_qkv(const Var& qkv, int n_heads, float scale, int64_t seq_len, boo
                          o4 = view4(self->data.ptr(), 0, es, sl * d, d, g.dk), g4 = view4(self->grad.ptr(), 0, es, sl * d, d, g.dk),
                          dq4 = view4(dqkv.ptr(), 0, es, sl * d3, d3, g.dk), dk4 = view4(dqkv.ptr(), d, es, sl * d3, d3, g.dk),
                          dv4 = view4(dqkv.ptr(), 2 * d, es, sl * d3, d3, g.dk);
-        attn_check(pk_attn_bwd(&sh, &q4, &k4, &v4, &o4, static_cast<const float*>(lse->p), &g4, &dq4, &dk4, &dv4, ws.p,
-                               ws.bytes, tape_stream()));
+        if (turned && qkv->grad.empty()) {
+            TurnBack back{static_cast<const float*>(turned->table->p), turned->heads, false};
+            attn_check(attn_bwd_turned(&sh, &q4, &k4, &v4, &o4, static_cast<const float*>(lse->p), &g4, &dq4, &dk4, &dv4, ws.p, ws.bytes, back,
+                                       tape_stream()));
+            turned->gradient_is_back = back.turned;
+        } else {
+            attn_check(pk_attn_bwd(&sh, &q4, &k4, &v4, &o4, static_cast<const float*>(lse->p), &g4, &dq4, &dk4, &dv4, ws.p,
+                                   ws.bytes, tape_stream()));
+        }
         qkv->accumulate_owned(std::move(dqkv));
     });
 }

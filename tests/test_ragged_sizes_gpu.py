@@ -116,6 +116,24 @@ def test_norm_and_rope_in_the_projection(dtype, d, heads, tokens, seq, all_heads
         m.close()
 
 
+@pytest.mark.parametrize("all_heads", [False, True])
+@pytest.mark.parametrize("dtype,d,heads,tokens,seq", [
+    ("fp32", 64, 2, 33, 11), ("fp32", 40, 5, 50, 10), ("fp32", 192, 2, 1030, 515), ("fp32", 256, 2, 1538, 769), ("bf16", 64, 2, 33, 11),
+    ("bf16", 80, 1, 70, 35), ("bf16", 96, 1, 700, 350), ("bf16", 192, 2, 1030, 515), ("bf16", 512, 8, 4084, 1021), ("bf16", 768, 8, 4000, 500)])
+def test_rope_undone_in_attention_backward(dtype, d, heads, tokens, seq, all_heads):
+    """dQ and dK turned back where the attention kernels write them against a pass of its own, which a window with sinks has: a window of all
+    keys but the first and one sink see what causal attention sees. Where bf16 gradients are rounded differs: P, dS, dQ or dK and the turned
+    ones, 2 ^ -9 each of a norm."""
+    toks = synth.randint(3, tokens + 1, 130)
+    got = []
+    for window, sinks in ((seq - 1, 1), (0, 0)):
+        m = Llama(vocab=130, d=d, n_layers=1, n_heads=heads, d_ff=2 * d, compute_dtype=dtype, rope_all_heads=all_heads, window=window, sinks=sinks, seed=8)
+        got.append((m.loss_backward(toks[:-1], toks[1:], seq)[0], m.grads()))
+        m.close()
+    assert abs(got[0][0] - got[1][0]) < (1e-5 if dtype == "fp32" else 1e-3)
+    assert rel(got[1][1], got[0][1]) < (1e-5 if dtype == "fp32" else 4 * 2.0 ** -9)
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("vocab,d,ff,layers", [(130, 64, 176, 8), (37, 12, 20, 1), (37, 6, 10, 1)])
 def test_optimiser_step_writes_the_copies(vocab, d, ff, layers, dtype):
