@@ -382,6 +382,17 @@ __device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weig
                         store4g<true>(a.part, row * D + TrMap<D>::col0(db, qd, g), acc[db][qd * 4] * sc, acc[db][qd * 4 + 1] * sc,
                                       acc[db][qd * 4 + 2] * sc, acc[db][qd * 4 + 3] * sc);
             }
+        } else if (!GF32 && chunk < 0) {  // (no tile is read any more)
+            using Rows = RowStrip<D>;
+            static_assert(NTHR / 64 * Rows::ELEMS <= 6 * BMQ * S, "the wavefronts' strips");
+            uint16_t* const strip = Qs[0] + static_cast<int>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * Rows::ELEMS;
+            const int k1 = kj - c32, from = piece ? a.sinks - k1 : 0;
+            const int64_t st = rl == 0 ? a.dv_st : a.dk_st;
+            const float sc = rl == 0 ? 1.0f : a.scale;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) store_acc_bf16<D>(Rows::row(strip, c32), db, g, acc[db], sc);
+            Rows::out(strip, static_cast<uint16_t*>(rl == 0 ? a.dv : a.dk) + (rl == 0 ? b * a.dv_sb + hk * a.dv_sh : b * a.dk_sb + hk * a.dk_sh) + k1 * st, st, from,
+                      a.T - k1, lane);
         } else if (kj < a.T && chunk < 0 && !(piece && kj < a.sinks)) {
             void* dst = rl == 0 ? a.dv : a.dk;
             const int64_t ob = rl == 0 ? b * a.dv_sb + hk * a.dv_sh + kj * a.dv_st
@@ -389,10 +400,6 @@ __device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weig
             const float sc = rl == 0 ? 1.0f : a.scale;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
-                if (!GF32) {
-                    store_acc_bf16<D>(static_cast<uint16_t*>(dst) + ob, db, g, acc[db], sc);
-                    continue;
-                }
 #pragma unroll
                 for (int qd = 0; qd < 4; ++qd)
                     store4g<GF32>(dst, ob + TrMap<D>::col0(db, qd, g), acc[db][qd * 4] * sc, acc[db][qd * 4 + 1] * sc,

@@ -541,8 +541,20 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
             const int kj = kj0 + 32 * kb;
-            if (kj >= a.T) continue;
             const float sc = rl == 0 ? 1.0f : a.scale;
+            if (!GF32 && hs == 1) {
+                using Rows = RowStrip<D>;
+                static_assert(4 * Rows::ELEMS <= 3 * BMQ * S, "the wavefronts' strips");
+                uint16_t* const strip = Qs[0] + w * Rows::ELEMS;
+                const int k1 = kw0 + 32 * kb;
+                const int64_t st = rl == 0 ? a.dv_st : a.dk_st;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) store_acc_bf16<D>(Rows::row(strip, c32), db, g, acc[kb][db], sc);
+                Rows::out(strip, static_cast<uint16_t*>(rl == 0 ? a.dv : a.dk) + (rl == 0 ? b * a.dv_sb + hk * a.dv_sh : b * a.dk_sb + hk * a.dk_sh) + k1 * st, st, 0,
+                          a.T - k1, lane);
+                continue;
+            }
+            if (kj >= a.T) continue;
             if (hs > 1) {  // fp32 partial sums of this split, rows of pitch D
                 float* prow = a.part + ((static_cast<size_t>(kvu) * hs + rr) * 2 + (rl == 0 ? 1 : 0)) * a.T * D +
                               static_cast<size_t>(kj) * D;
@@ -559,10 +571,6 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
                                        : b * a.dk_sb + hk * a.dk_sh + kj * a.dk_st;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
-                if (!GF32) {
-                    store_acc_bf16<D>(static_cast<uint16_t*>(dst) + ob, db, g, acc[kb][db], sc);
-                    continue;
-                }
 #pragma unroll
                 for (int qd = 0; qd < 4; ++qd)
                     store4g<GF32>(dst, ob + TrMap<D>::col0(db, qd, g), acc[kb][db][qd * 4] * sc, acc[kb][db][qd * 4 + 1] * sc,
@@ -574,9 +582,9 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
             run_role(std::integral_constant<int, 0>{});
         else
             run_role(std::integral_constant<int, 1>{});
-        // No barrier here: after the last barrier of the step loop nobody reads the rings any more, the stores above
-        // touch no LDS, and a barrier would make every wavefront wait for its stores to be acknowledged before the
-        // next pass may ask for its rows.
+        // After the last barrier of the step loop nobody reads the rings any more, but whole rows leave through them, where the next pass's first
+        // tiles go; the other forms' stores touch no LDS, and a barrier would only make every wavefront wait for them.
+        if (!GF32 && hs == 1 && pass + 1 < npass) __syncthreads();
     }
 }
 

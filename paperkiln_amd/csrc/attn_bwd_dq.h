@@ -191,7 +191,15 @@ __device__ inline void dq_block(const AttnArgs& a, int b, int h, int hk, int qbl
         t = tn;
     }
 
-    if (qi < a.T) {
+    if constexpr (!GF32 && NW <= 4) {  // (no tile is read any more; eight wavefronts' rows would not fit)
+        using Rows = RowStrip<D>;
+        static_assert(NW * Rows::ELEMS <= DQ_LDS<D, NW>, "the wavefronts' strips");
+        uint16_t* const strip = lds + w * Rows::ELEMS;
+        const int q1 = qi - c32;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) store_acc_bf16<D>(Rows::row(strip, c32), db, g, dq_acc[db], a.scale);
+        Rows::out(strip, static_cast<uint16_t*>(a.dq) + b * a.dq_sb + h * a.dq_sh + q1 * a.dq_st, a.dq_st, 0, a.T - q1, lane);
+    } else if (qi < a.T) {
         const int64_t ob = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {

@@ -482,6 +482,7 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
             __syncthreads();
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in the ring after the pass
+        if (!GF32) __syncthreads();  // of any wavefront: it takes the results' strips
 
         // the last matrix instructions may still be writing the accumulators
         asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
@@ -491,15 +492,20 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
             for (int db = 0; db < DB; ++db) asm volatile("" : "+a"(acc[qb][db]));
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-            const int qi = qw + qb * 32 + c32;
+            const int q1 = qw + qb * 32, qi = q1 + c32;
+            if constexpr (!GF32) {
+                using Rows = RowStrip<D>;
+                static_assert(4 * Rows::ELEMS <= RING * BN * S, "the wavefronts' strips");
+                uint16_t* const strip = Kt[0] + w * Rows::ELEMS;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) store_acc_bf16<D>(Rows::row(strip, c32), db, g, acc[qb][db], a.scale);
+                Rows::out(strip, static_cast<uint16_t*>(a.dq) + b * a.dq_sb + h * a.dq_sh + q1 * a.dq_st, a.dq_st, 0, a.T - q1, lane);
+                continue;
+            }
             if (qi >= a.T) continue;
             const int64_t ob = b * a.dq_sb + h * a.dq_sh + qi * a.dq_st;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
-                if (!GF32) {
-                    store_acc_bf16<D>(static_cast<uint16_t*>(a.dq) + ob, db, g, acc[qb][db], a.scale);
-                    continue;
-                }
 #pragma unroll
                 for (int qd = 0; qd < 4; ++qd)
                     store4q<GF32>(a.dq, ob + TrMap<D>::col0(db, qd, g), acc[qb][db][qd * 4] * a.scale,
@@ -507,10 +513,10 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
                                   acc[qb][db][qd * 4 + 3] * a.scale);
             }
         }
-        // No barrier here: every wavefront passed the barrier of the last iteration after its last read of the ring,
-        // the stores above touch no LDS, and the next pass meets its own barriers before anybody reads what another
-        // wavefront wrote. A barrier would also make each wavefront wait for its dQ stores to be acknowledged before
-        // the next pass may ask for its rows.
+        // bf16: the next pass's rows land where the strips are. fp32 needs no barrier: every wavefront passed that of the last iteration after its
+        // last read of the ring, its stores touch no LDS, and the next pass meets its own barriers before anybody reads what another wavefront
+        // wrote.
+        if (!GF32 && pass + 1 < npass) __syncthreads();
     }
 }
 

@@ -324,17 +324,19 @@ __global__ __launch_bounds__(64 * NW, OCC) void mfma_fwd(AttnArgs a) {
         t = tn;
     }
 
-    // Epilogue: O = acc / l, LSE = m*scale + ln(l) (natural log, scaled units).
+    // Epilogue: O = acc / l, LSE = m*scale + ln(l) (natural log, scaled units). No tile is read any more.
+    using Rows = RowStrip<D>;
+    static_assert(NW <= 8 && 4 * Rows::ELEMS <= 2 * BN * C::KS, "four wavefronts' strips in either tensor's buffers");
+    uint16_t* const strip = (w < 4 ? Kbuf[0] : Vbuf[0]) + (w & 3) * Rows::ELEMS;
 #pragma unroll
     for (int qb = 0; qb < NQ; ++qb) {
-        const int qi = q0 + (w * NQ + qb) * 32 + c32;
+        const int q1 = q0 + (w * NQ + qb) * 32, qi = q1 + c32;
         const float lt = xhalf_sum(l[qb]);
-        if (qi >= a.T) continue;
         const float inv = 1.0f / lt;
-        uint16_t* orow = static_cast<uint16_t*>(a.o) + b * a.o_sb + h * a.o_sh + qi * a.o_st;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) store_acc_bf16_natural(orow, db, g, acc_o[qb][db], inv);
-        if (g == 0)
+        for (int db = 0; db < DB; ++db) store_acc_bf16_natural(Rows::row(strip, c32), db, g, acc_o[qb][db], inv);
+        Rows::out(strip, static_cast<uint16_t*>(a.o) + b * a.o_sb + h * a.o_sh + q1 * a.o_st, a.o_st, 0, a.T - q1, lane);
+        if (qi < a.T && g == 0)
             a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = m[qb] * a.scale + logf(lt);
     }
     __syncthreads();  // the next pass refills the tile buffers

@@ -867,3 +867,30 @@ def test_lines_between_split_and_unsplit_chains(case, dk):
     B, T, Hq, Hkv, causal, window, sinks = case
     e = errors(*run_attention(B, T, Hq, Hkv, dk, torch.bfloat16, causal, window, sinks))
     assert e[0] < 5e-3 and e[1] < 1e-5 and max(e[2:4]) < 5e-3 and e[4] < 2e-5, e
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("case", [(1, 1, 1, 1, True, 0, 0), (2, 33, 3, 3, False, 0, 0), (3, 300, 5, 5, True, 0, 0), (16, 512, 8, 8, True, 0, 0), (6, 777, 12, 12, False, 0, 0),
+                                  (1, 1501, 16, 16, True, 16, 3), (2, 2048, 16, 4, True, 256, 4), (3, 1025, 16, 16, True, 0, 0), (2, 3001, 16, 4, True, 0, 0),
+                                  (4, 2000, 16, 16, True, 100, 0)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_bf16_rows_of_whole_lines_and_of_others(case, dk):
+    """Results whose rows are whole lines of memory and the same results as rows that begin and end inside one, with another's data on either side: the
+    same bits, and nothing written beside them. Against float64 as elsewhere: P, dS, O and the gradients rounded to 2 ^ -9 each."""
+    B, T, Hq, Hkv, causal, window, sinks = case
+    gen = torch.Generator(device="cuda").manual_seed(T + dk)
+    draw = lambda h: torch.randn((B, T, h, dk), generator=gen, device="cuda").bfloat16()  # noqa: E731
+    q, k, v, d_o = draw(Hq), draw(Hkv), draw(Hkv), draw(Hq)
+    scale = float(np.float32(1.0 / np.sqrt(dk)))
+    o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
+    got = (o, lse) + ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks)
+    assert max(errors(got, exact_attention(q, k, v, d_o, scale, causal, window, sinks))) < 1e-2
+    room = [torch.full((B, T, h, dk + 16), 7.0, device="cuda", dtype=torch.bfloat16) for h in (Hq, Hq, Hkv, Hkv)]
+    inside = [r[..., 8:-8] for r in room]
+    t4, by = ops._t4, ctypes.byref
+    _lib.check(_lib.lib().pk_attn_fwd(by(ops._shape(q, k, scale, causal, window, sinks)), by(t4(q)), by(t4(k)), by(t4(v)), by(t4(inside[0])),
+                                      ctypes.c_void_p(lse.data_ptr()), ops._stream()))
+    ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks,
+                 out=(*inside[1:], torch.empty(ops.bwd_workspace_bytes(q, k, window=window, sinks=sinks), dtype=torch.uint8, device="cuda")))
+    for r, i, g in zip(room, inside, (got[0],) + got[2:]):
+        assert torch.equal(i, g)
+        assert bool((r[..., :8] == 7.0).all()) and bool((r[..., -8:] == 7.0).all())
