@@ -338,9 +338,20 @@ __global__ __launch_bounds__(64 * QW * KW, 2) void split_fwd(AttnArgs a) {
         });
         m = mt, l = lt;
     }
+    bool stored = KW > 1;
+    if constexpr (KW == 1 && WHOLE_ROWS<D, EXACT>)
+        if (dk == D) {
+            using Rows = RowStrip<D>;
+            static_assert(QW * Rows::ELEMS <= NBUF * KW * TILE, "the wavefronts' strips");
+            uint16_t* const strip = lds + qg * Rows::ELEMS;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) store_block(false, strip, c32 * Rows::S, db, g, acc[db], 1.0f / l, D);
+            Rows::out(strip, static_cast<uint16_t*>(a.o) + b * a.o_sb + h * a.o_sh + qlo * a.o_st, a.o_st, 0, a.T - qlo, lane);
+            stored = true;
+        }
     if (qi < a.T) {
         const float inv = 1.0f / l;
-        if (KW == 1)
+        if (!stored)
 #pragma unroll
             for (int db = 0; db < DB; ++db) store_block(false, a.o, ro, db, g, acc[db], inv, dk);
         if (g == 0 && kg == 0) a.lse[(static_cast<int64_t>(b) * a.Hq + h) * a.T + qi] = m * a.scale + logf(l);
@@ -447,9 +458,21 @@ __device__ inline void dq_block(const AttnArgs& a, int fuse_delta, int b, int h,
         join_shares<DB, KW, 2>(acc, reinterpret_cast<float*>(lds) + qg * KW * DB * 1024, kg, lane, no_weights, [&](int db, int qd, const f32x4 (&v)[2]) {
             if (qi < a.T) store_half(a.grad_f32 != 0, a.dq, ro, db, qd, g, v, a.scale, dk, turn_row<TURN>(a, h, qi));
         });
-    else if (qi < a.T)
+    else {
+        if constexpr (WHOLE_ROWS<D, EXACT>)
+            if (dk == D && !a.grad_f32) {
+                using Rows = RowStrip<D>;
+                static_assert(QW * Rows::ELEMS <= NBUF * KW * TILE, "the wavefronts' strips");
+                uint16_t* const strip = lds + qg * Rows::ELEMS;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk, turn_row<TURN>(a, h, qi));
+                for (int db = 0; db < DB; ++db)
+                    store_block(false, strip, c32 * Rows::S, db, g, acc[db], a.scale, D, turn_row<TURN>(a, h, min(qi, a.T - 1)));
+                return Rows::out(strip, static_cast<uint16_t*>(a.dq) + b * a.dq_sb + h * a.dq_sh + qlo * a.dq_st, a.dq_st, 0, a.T - qlo, lane);
+            }
+        if (qi < a.T)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) store_block(a.grad_f32 != 0, a.dq, ro, db, g, acc[db], a.scale, dk, turn_row<TURN>(a, h, qi));
+    }
 }
 template <int D, int QW, int KW, int NB, bool EXACT>
 __global__ __launch_bounds__(64 * QW * KW, 2) void split_dq(AttnArgs a, int fuse_delta) {
@@ -676,7 +699,22 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                 if (mine) store_half(f32, is_v ? dst_v : dst_k, is_v ? rv : rk, is_v ? n : n0 + n - DB, qd, g, v, is_v ? 1.0f : a.scale, dk, is_v ? TurnRow() : turn_row<TURN>(a, hk, kj));
             });
         }
-    } else if (mine) {
+    } else {
+        if constexpr (WHOLE_ROWS<D, EXACT>)
+            if (dk == D && !a.grad_f32 && hs == 1 && tl.nch == 0) {
+                using Rows = RowStrip<D>;
+                static_assert(QW * Rows::ELEMS <= NBUF * KW * TILE, "the wavefronts' strips");
+                uint16_t* const strip = lds + qg * Rows::ELEMS;
+                const int k1 = kj - c32;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) store_block(false, strip, c32 * Rows::S, db, g, acc[db], 1.0f, D);
+                Rows::out(strip, static_cast<uint16_t*>(a.dv) + b * a.dv_sb + hk * a.dv_sh + k1 * a.dv_st, a.dv_st, 0, a.T - k1, lane);
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+                    store_block(false, strip, c32 * Rows::S, db, g, acc[DB + db], a.scale, D, turn_row<TURN>(a, hk, min(kj, a.T - 1)));
+                return Rows::out(strip, static_cast<uint16_t*>(a.dk) + b * a.dk_sb + hk * a.dk_sh + k1 * a.dk_st, a.dk_st, 0, a.T - k1, lane);
+            }
+        if (!mine) return;
 #pragma unroll
         for (int n = 0; n < 2 * DB; ++n) {
             if (n < DB)
