@@ -239,11 +239,11 @@ __device__ inline F8 ld8(const float* p, int64_t e) {
 }
 __device__ inline void st8(uint16_t* p, int64_t e, const F8& x) {
     const u32x4 r = {pack_bf16(x.v[0], x.v[1]), pack_bf16(x.v[2], x.v[3]), pack_bf16(x.v[4], x.v[5]), pack_bf16(x.v[6], x.v[7])};
-    *reinterpret_cast<u32x4*>(p + e) = r;
+    store_through(reinterpret_cast<u32x4*>(p + e), r);
 }
 __device__ inline void st8(float* p, int64_t e, const F8& x) {
-    *reinterpret_cast<f32x4*>(p + e) = f32x4{x.v[0], x.v[1], x.v[2], x.v[3]};
-    *reinterpret_cast<f32x4*>(p + e + 4) = f32x4{x.v[4], x.v[5], x.v[6], x.v[7]};
+    store_through(reinterpret_cast<f32x4*>(p + e), f32x4{x.v[0], x.v[1], x.v[2], x.v[3]});
+    store_through(reinterpret_cast<f32x4*>(p + e + 4), f32x4{x.v[4], x.v[5], x.v[6], x.v[7]});
 }
 #define PK_EW8_LOOP(i, n8) \
     for (int64_t i = blockIdx.x * static_cast<int64_t>(NT) + threadIdx.x; i < (n8); i += static_cast<int64_t>(gridDim.x) * NT)
@@ -1230,7 +1230,7 @@ __global__ void adamw_parts_k(AdamWParts ps, float* p, float* g, float* m, float
     if (gs != 1.0f) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) gi[k] *= gs;
-        at(g) = gi;
+        store_through(&at(g), gi);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1238,20 +1238,19 @@ __global__ void adamw_parts_k(AdamWParts ps, float* p, float* g, float* m, float
         adamw_one(pk, gi[k], mk, vk, lr, b1, b2, eps, wd, c1, c2);
         pi[k] = pk, mi[k] = mk, vi[k] = vk;
     }
-    at(m) = mi;
-    at(v) = vi;
-    at(p) = pi;
+    store_through(&at(m), mi);
+    store_through(&at(v), vi);
+    store_through(&at(p), pi);
     if (!part.copy) return;
     const int r = e / part.cols, c = e - r * part.cols;
     TY* const to = static_cast<TY*>(part.copy) + static_cast<int64_t>(r) * part.ld + part.off + c;
     if constexpr (std::is_same<TY, float>::value) {
-        *reinterpret_cast<f32x4*>(to) = pi;
+        store_through(reinterpret_cast<f32x4*>(to), pi);
     } else {
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
         uint16_t four[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) stf(four, k, pi[k]);
-        *reinterpret_cast<u32x2*>(to) = u32x2{four[0] | static_cast<uint32_t>(four[1]) << 16, four[2] | static_cast<uint32_t>(four[3]) << 16};
+        store_through(reinterpret_cast<u32x2*>(to), u32x2{four[0] | static_cast<uint32_t>(four[1]) << 16, four[2] | static_cast<uint32_t>(four[3]) << 16});
     }
 }
 // What a training pass begins with, in one launch: its gradients cleared, and the host's n words fetched from pinned memory (first,
@@ -1269,7 +1268,7 @@ __global__ void begin_pass_rows(f32x4* clear, int64_t n4, const int* pinned, int
     const int row = static_cast<int>(first) / d4, c = (static_cast<int>(first) - row * d4) * 4;
     const int id = first < quads ? pinned[row] : 0;  // quads threads or more are launched
     for (int64_t i = first; i < n; i += stride) to[i] = pinned[i];
-    for (int64_t i = first; i < n4; i += stride) clear[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t i = first; i < n4; i += stride) store_through(clear + i, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
     if (first >= quads) return;
     const f32x4 v = *reinterpret_cast<const f32x4*>(table + static_cast<int64_t>(id) * (d4 * 4) + c);
 #pragma unroll
