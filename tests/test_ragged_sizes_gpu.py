@@ -869,11 +869,12 @@ def test_lines_between_split_and_unsplit_chains(case, dk):
     assert e[0] < 5e-3 and e[1] < 1e-5 and max(e[2:4]) < 5e-3 and e[4] < 2e-5, e
 
 
+@pytest.mark.parametrize("grad", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
 @pytest.mark.parametrize("dk", [64, 128])
 @pytest.mark.parametrize("case", [(1, 1, 1, 1, True, 0, 0), (2, 33, 3, 3, False, 0, 0), (3, 300, 5, 5, True, 0, 0), (16, 512, 8, 8, True, 0, 0), (6, 777, 12, 12, False, 0, 0),
                                   (1, 1501, 16, 16, True, 16, 3), (2, 2048, 16, 4, True, 256, 4), (3, 1025, 16, 16, True, 0, 0), (2, 3001, 16, 4, True, 0, 0),
-                                  (4, 2000, 16, 16, True, 100, 0)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
-def test_bf16_rows_of_whole_lines_and_of_others(case, dk):
+                                  (4, 2000, 16, 16, True, 100, 0), (2, 1000, 16, 4, True, 0, 0), (4, 512, 14, 2, True, 0, 0)], ids=lambda c: "B%d_T%d_H%d_%d_c%d_w%d_s%d" % c)
+def test_bf16_rows_of_whole_lines_and_of_others(case, dk, grad):
     """Results whose rows are whole lines of memory and the same results as rows that begin and end inside one, with another's data on either side: the
     same bits, and nothing written beside them. Against float64 as elsewhere: P, dS, O and the gradients rounded to 2 ^ -9 each."""
     B, T, Hq, Hkv, causal, window, sinks = case
@@ -882,15 +883,15 @@ def test_bf16_rows_of_whole_lines_and_of_others(case, dk):
     q, k, v, d_o = draw(Hq), draw(Hkv), draw(Hkv), draw(Hq)
     scale = float(np.float32(1.0 / np.sqrt(dk)))
     o, lse = ops.attn_fwd(q, k, v, scale, causal, window, sinks)
-    got = (o, lse) + ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks)
+    got = (o, lse) + ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, grad_dtype=grad)
     assert max(errors(got, exact_attention(q, k, v, d_o, scale, causal, window, sinks))) < 1e-2
-    room = [torch.full((B, T, h, dk + 16), 7.0, device="cuda", dtype=torch.bfloat16) for h in (Hq, Hq, Hkv, Hkv)]
+    room = [torch.full((B, T, h, dk + 16), 7.0, device="cuda", dtype=t) for h, t in ((Hq, torch.bfloat16), (Hq, grad), (Hkv, grad), (Hkv, grad))]
     inside = [r[..., 8:-8] for r in room]
     t4, by = ops._t4, ctypes.byref
     _lib.check(_lib.lib().pk_attn_fwd(by(ops._shape(q, k, scale, causal, window, sinks)), by(t4(q)), by(t4(k)), by(t4(v)), by(t4(inside[0])),
                                       ctypes.c_void_p(lse.data_ptr()), ops._stream()))
-    ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks,
-                 out=(*inside[1:], torch.empty(ops.bwd_workspace_bytes(q, k, window=window, sinks=sinks), dtype=torch.uint8, device="cuda")))
+    ops.attn_bwd(q, k, v, o, lse, d_o, scale, causal, window, sinks, grad,
+                 (*inside[1:], torch.empty(ops.bwd_workspace_bytes(q, k, grad, window, sinks), dtype=torch.uint8, device="cuda")))
     for r, i, g in zip(room, inside, (got[0],) + got[2:]):
         assert torch.equal(i, g)
         assert bool((r[..., :8] == 7.0).all()) and bool((r[..., -8:] == 7.0).all())
