@@ -372,16 +372,11 @@ __device__ inline void dkdv2_blocks(const AttnArgs& a, Ring<D, BMQ>& tiles, Weig
                                   acc[db][qd * 4 + 2] * sc, acc[db][qd * 4 + 3] * sc);
         }
         if (JOINED && hs > 1) {  // partial sums of this share of the heads, for launch_gqa_reduce
-            if (kj < a.T) {
-                const int64_t row = ((static_cast<int64_t>(kvu) * hs + rr) * 2 + (rl == 0 ? 1 : 0)) * a.T + kj;
-                const float sc = rl == 0 ? 1.0f : a.scale;
-#pragma unroll
-                for (int db = 0; db < DB; ++db)
-#pragma unroll
-                    for (int qd = 0; qd < 4; ++qd)
-                        store4g<true>(a.part, row * D + TrMap<D>::col0(db, qd, g), acc[db][qd * 4] * sc, acc[db][qd * 4 + 1] * sc,
-                                      acc[db][qd * 4 + 2] * sc, acc[db][qd * 4 + 3] * sc);
-            }
+            static_assert(!JOINED || NTHR / 64 * LineStrip<64>::FLOATS * 2 <= 6 * BMQ * S, "the wavefronts' strips");
+            float* const strip = reinterpret_cast<float*>(Qs[0]) + static_cast<int>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * LineStrip<64>::FLOATS;
+            const int k1 = kj - c32;
+            const int64_t row = ((static_cast<int64_t>(kvu) * hs + rr) * 2 + (rl == 0 ? 1 : 0)) * a.T + k1;
+            store_rows_f32<D>(strip, a.part + row * D, D, a.T - k1, acc, rl == 0 ? 1.0f : a.scale, lane);
         } else if (!GF32 && chunk < 0) {  // (no tile is read any more)
             using Rows = RowStrip<D>;
             static_assert(NTHR / 64 * Rows::ELEMS <= 6 * BMQ * S, "the wavefronts' strips");

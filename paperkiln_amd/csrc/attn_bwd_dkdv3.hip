@@ -556,27 +556,10 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
             }
             if (hs > 1) {  // fp32 partial sums of this split, rows of pitch D
                 float* pbase = a.part + ((static_cast<size_t>(kvu) * hs + rr) * 2 + (rl == 0 ? 1 : 0)) * a.T * D;
-                if constexpr (D == 64) {
-                    static_assert(4 * LineStrip::FLOATS * 2 <= 3 * BMQ * S, "the wavefronts' strips");
-                    float* const strip = reinterpret_cast<float*>(Qs[0]) + w * LineStrip::FLOATS;
-                    const int k1 = kw0 + 32 * kb;
-#pragma unroll
-                    for (int db = 0; db < DB; ++db) {
-#pragma unroll
-                        for (int qd = 0; qd < 4; ++qd)
-                            LineStrip::put(strip, c32, qd, g, f32x4{acc[kb][db][qd * 4] * sc, acc[kb][db][qd * 4 + 1] * sc, acc[kb][db][qd * 4 + 2] * sc, acc[kb][db][qd * 4 + 3] * sc});
-                        LineStrip::out(strip, pbase + static_cast<int64_t>(k1) * D + db * 32, D, a.T - k1, lane);
-                    }
-                    continue;
-                }
-                if (kj >= a.T) continue;
-                float* prow = pbase + static_cast<size_t>(kj) * D;
-#pragma unroll
-                for (int db = 0; db < DB; ++db)
-#pragma unroll
-                    for (int qd = 0; qd < 4; ++qd)
-                        store4g<true>(prow, TrMap<D>::col0(db, qd, g), acc[kb][db][qd * 4] * sc, acc[kb][db][qd * 4 + 1] * sc,
-                                      acc[kb][db][qd * 4 + 2] * sc, acc[kb][db][qd * 4 + 3] * sc);
+                static_assert(2 * LineStrip<64>::FLOATS * 2 <= 3 * BMQ * S, "two wavefronts' strips in either tensor's ring");
+                float* const strip = reinterpret_cast<float*>(w < 2 ? Qs[0] : dOs[0]) + (w & 1) * LineStrip<64>::FLOATS;
+                const int k1 = kw0 + 32 * kb;
+                store_rows_f32<D>(strip, pbase + static_cast<int64_t>(k1) * D, D, a.T - k1, acc[kb], sc, lane);
                 continue;
             }
             if (kj >= a.T) continue;
@@ -598,7 +581,7 @@ __global__ __launch_bounds__(256, 1) void mfma_dkdv3(AttnArgs a) {
             run_role(std::integral_constant<int, 1>{});
         // After the last barrier of the step loop nobody reads the rings any more, but whole rows leave through them, where the next pass's first
         // tiles go; the other forms' stores touch no LDS, and a barrier would only make every wavefront wait for them.
-        if (((!GF32 && hs == 1) || (D == 64 && hs > 1)) && pass + 1 < npass) __syncthreads();
+        if ((!GF32 || hs > 1) && pass + 1 < npass) __syncthreads();
     }
 }
 

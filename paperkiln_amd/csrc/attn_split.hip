@@ -716,8 +716,9 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
             }
         if constexpr (WHOLE_ROWS<D, EXACT> && !TURN)
             if (dk == D && tl.nch == 0) {  // fp32: a share's partial sums, or the gradients
-                static_assert(QW * LineStrip::FLOATS * 2 <= NBUF * KW * TILE, "the wavefronts' strips");
-                float* const strip = reinterpret_cast<float*>(lds) + qg * LineStrip::FLOATS;
+                using Lines = LineStrip<>;
+                static_assert(QW * Lines::FLOATS * 2 <= NBUF * KW * TILE, "the wavefronts' strips");
+                float* const strip = reinterpret_cast<float*>(lds) + qg * Lines::FLOATS;
                 const int k1 = kj - c32;
 #pragma unroll
                 for (int n = 0; n < 2 * DB; ++n) {
@@ -725,12 +726,12 @@ __device__ inline void dkdv_block(const AttnArgs& a, int blk, int rr, int kvu, u
                     const float sc = is_v ? 1.0f : a.scale;
 #pragma unroll
                     for (int qd = 0; qd < 4; ++qd)
-                        LineStrip::put(strip, c32, qd, g, f32x4{acc[n][qd * 4] * sc, acc[n][qd * 4 + 1] * sc, acc[n][qd * 4 + 2] * sc, acc[n][qd * 4 + 3] * sc});
+                        Lines::put(strip, c32, 8 * qd + 4 * g, f32x4{acc[n][qd * 4] * sc, acc[n][qd * 4 + 1] * sc, acc[n][qd * 4 + 2] * sc, acc[n][qd * 4 + 3] * sc});
                     float* const to = parts  ? a.part + ((static_cast<int64_t>(kvu) * hs + rr) * 2 + (is_v ? 1 : 0)) * a.T * D
                                       : is_v ? static_cast<float*>(a.dv) + b * a.dv_sb + hk * a.dv_sh
                                              : static_cast<float*>(a.dk) + b * a.dk_sb + hk * a.dk_sh;
                     const int64_t st = parts ? D : is_v ? a.dv_st : a.dk_st;
-                    LineStrip::out(strip, to + k1 * st + (is_v ? n : n - DB) * 32, st, a.T - k1, lane);
+                    Lines::out(strip, to + k1 * st + (is_v ? n : n - DB) * 32, st, a.T - k1, lane);
                 }
                 return;
             }

@@ -194,22 +194,25 @@ struct RowStrip {
         asm volatile("" ::: "memory");
     }
 };
-// The same of fp32, 32 columns at a time: a line of memory to a row where the rows begin on one (partial sums of a group's shares: backward of T 512 x 4, 14 heads
-// on 2 28.4 -> 23.6 us, 1000 x 2, 16 on 4 40.2 -> 37.1, 2048 x 4, 14 on 2 143.7 -> 141.4).
+// The same of fp32, W columns at a time: whole lines of memory to a row where the rows begin on one (partial sums of a group's shares: backward of T 512 x 4, 14 heads
+// on 2 28.4 -> 23.6 us, 1000 x 2, 16 on 4 40.2 -> 37.1, 2048 x 4, 14 on 2 143.7 -> 141.4; of 128 columns, 3001, 32 on 8 300 -> 290, 2048 x 4, 16 on 2 301 ->
+// 283).
+template <int W = 32>
 struct LineStrip {
-    static constexpr int P = 36, FLOATS = 32 * P;
-    // columns 8 qd + 4 g .. of row r
-    __device__ static void put(float* strip, int r, int qd, int g, f32x4 v) { *reinterpret_cast<f32x4*>(strip + r * P + 8 * qd + 4 * g) = v; }
+    static constexpr int P = W + 4, FLOATS = 32 * P;
+    __device__ static void put(float* strip, int r, int col, f32x4 v) { *reinterpret_cast<f32x4*>(strip + r * P + col) = v; }
     __device__ static void out(const float* strip, float* base, int64_t st, int to, int lane) {
+        constexpr int CPR = W / 4, RPI = 64 / CPR;  // 16-byte chunks of a row, rows per instruction
         asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();  // the rows are other lanes'
         const bool lines = ((reinterpret_cast<uintptr_t>(base) | static_cast<uintptr_t>(st * 4)) & 127) == 0;
-        const int r0 = lane >> 3, c = (lane & 7) * 4;
+        const int r0 = lane / CPR, c = lane % CPR * 4;
         float* p = base + r0 * st + c;
 #pragma unroll
-        for (int k = 0; k < 4; ++k, p += 8 * st) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(strip + (r0 + 8 * k) * P + c);
-            if (r0 + 8 * k >= to) continue;
+        for (int k = 0; k < 32 / RPI; ++k, p += RPI * st) {
+            const int r = r0 + k * RPI;
+            const f32x4 v = *reinterpret_cast<const f32x4*>(strip + r * P + c);
+            if (r >= to) continue;
             if (lines)
                 store_through(reinterpret_cast<f32x4*>(p), v);
             else
@@ -219,6 +222,24 @@ struct LineStrip {
         asm volatile("" ::: "memory");
     }
 };
+// 32 rows of accumulators in the column order of TrMap<D>, times sc, through a strip of 64 columns
+template <int D>
+__device__ inline void store_rows_f32(float* strip, float* base, int64_t st, int to, const f32x16 (&acc)[D / 32], float sc, int lane) {
+    using Lines = LineStrip<64>;
+    const int g = lane >> 5, c32 = lane & 31;
+#pragma unroll
+    for (int half = 0; half < D / 64; ++half) {
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+                if (TrMap<D>::col0(db, qd, 0) / 64 != half) continue;
+                Lines::put(strip, c32, TrMap<D>::col0(db, qd, g) - 64 * half,
+                           f32x4{acc[db][qd * 4] * sc, acc[db][qd * 4 + 1] * sc, acc[db][qd * 4 + 2] * sc, acc[db][qd * 4 + 3] * sc});
+            }
+        Lines::out(strip, base + 64 * half, st, to, lane);
+    }
+}
 
 // Where row r of a tile sits in LDS when the tile serves both 16-byte row reads and transposing reads at a pitch
 // 4 banks past a multiple of 64. For head_dim 128 rows keep their order (the column permutation above does the
