@@ -378,7 +378,7 @@ __device__ inline void store16(u32x4 v, uint32_t off, u32x4 rsrc, uint32_t soff)
     // back while nothing multiplies. Rows leave a strip as whole lines, so nothing is written twice. 8192 x 1536 x 512 17.6 -> 15.9 us, 8192 x 512 x 512
     // 8.0 -> 7.4, 8192 x 1376 x 512 17.0 -> 15.0, fp32 results 32000 x 512 x 4096 131.9 -> 129.1 and 512 x 2752 x 8192 34.8 -> 33.6, 4096 ^ 3 103.5 ->
     // 102.3. Not nt, which keeps the last-level cache from holding the lines as well: a little more of this, and 5 to 9 % of the kernels that read them next.
-    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen sc1\n\ts_nop 0" ::"v"(v), "v"(off), "s"(rsrc), "s"(soff) : "memory");
+    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen sc1\n\ts_nop 1" ::"v"(v), "v"(off), "s"(rsrc), "s"(soff) : "memory");
 }
 // What a workgroup stores per tile, for the count of memory operations in flight: FM strips of all WGM * 32 rows
 // (bf16) or FM * WGM strips of 32 rows (fp32, whose wider rows would not fit a ring slot otherwise), each

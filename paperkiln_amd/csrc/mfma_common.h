@@ -158,9 +158,9 @@ __device__ inline void store_acc_bf16(uint16_t* row, int db, int g, const f32x16
 // AdamW over 35 M parameters 174.3 -> 172.9, over 0.46 M 6.9 -> 5.9). Not for lines that several stores fill, which would go out once for each, nor for nt, which
 // also keeps them from the last-level cache, where the next kernel looks.
 // Invisible to the compiler's count of memory operations in flight, whose waits are the longer for it; the data registers may be overwritten by the
-// very next instruction, which a 16-byte store does not allow: one idle state.
-__device__ inline void store_through(u32x4* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory"); }
-__device__ inline void store_through(f32x4* p, f32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory"); }
+// next two instructions, which a 16-byte store does not allow: two idle states.
+__device__ inline void store_through(u32x4* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory"); }
+__device__ inline void store_through(f32x4* p, f32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory"); }
 __device__ inline void store_through(u32x2* p, u32x2 v) { asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory"); }
 // A wavefront's 32 finished rows of D bf16 on their way out, through a strip of LDS of its own: a lane holds pieces of one row, so stored from the
 // registers a line of memory arrives in 4 to 8 writes of 16 or 32 bytes. From the strip (store_acc_bf16 to row(): a pitch of 16 bytes past the row, so neither
