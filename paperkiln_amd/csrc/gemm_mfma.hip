@@ -373,7 +373,7 @@ __device__ inline void lane_offsets_masked(uint32_t (&off)[O::PER], const uint32
 }
 __device__ inline void store16(u32x4 v, uint32_t off, u32x4 rsrc, uint32_t soff) {
     // invisible to the compiler's count of memory operations in flight, like the loads above; the data registers
-    // may be overwritten by the very next instruction, which a 16-byte store does not allow: one idle state
+    // may be overwritten by the next two instructions, which a 16-byte store does not allow: two idle states
     // sc1, agent scope: an XCD's L2 passes the line on at once instead of holding it until the kernel's end, when eight L2s of 4 MB would be written
     // back while nothing multiplies. Rows leave a strip as whole lines, so nothing is written twice. 8192 x 1536 x 512 17.6 -> 15.9 us, 8192 x 512 x 512
     // 8.0 -> 7.4, 8192 x 1376 x 512 17.0 -> 15.0, fp32 results 32000 x 512 x 4096 131.9 -> 129.1 and 512 x 2752 x 8192 34.8 -> 33.6, 4096 ^ 3 103.5 ->
