@@ -769,17 +769,28 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
         const u32x4 to_c = tile_rsrc(g.c, bl, 2 * g.N, 2 * g.N - bl.n0), gu = tile_rsrc(g.d, bl, 2 * g.N, 2 * g.N - bl.n0);
         const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint16_t*>(static_cast<const uint16_t*>(g.d) + static_cast<int64_t>(bl.m0) * 2 * g.N + bl.n0), 0, static_cast<int>(gu[2]), 0x00020000);
+        const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(static_cast<uint16_t*>(g.c) + static_cast<int64_t>(bl.m0) * 2 * g.N + bl.n0, 0,
+                                                                            static_cast<int>(to_c[2]), 0x00020000);
         const uint32_t mask = bl.n0 + st_ch * 8 < g.N ? 0u : OUTSIDE;
         uint16_t* const cs = reinterpret_cast<uint16_t*>(strip);
+        // Gate and up of as many strips as the registers hold are on their way before the first store, and the compiler counts the stores: waits for
+        // loads are none for stores (8192 x 1376 x 512 38.8 -> 37.6 us).
+        constexpr int AHEAD = BM > 128 ? 1 : FM;
+        u32x4 gate[AHEAD][ST::PER_PHASE], up[AHEAD][ST::PER_PHASE];
+        const auto ask = [&](int i) {
+            const uint32_t soff = static_cast<uint32_t>(i * 32) * g.N * 4u, up_at = soff + g.N * 2u;
+#pragma unroll
+            for (int k = 0; k < ST::PER_PHASE; ++k) {
+                gate[i % AHEAD][k] = __builtin_amdgcn_raw_buffer_load_b128(from, static_cast<int>(coff[k] | mask), static_cast<int>(soff), 0);
+                up[i % AHEAD][k] = __builtin_amdgcn_raw_buffer_load_b128(from, static_cast<int>(coff[k] | mask), static_cast<int>(up_at), 0);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD - 1; ++i) ask(i);
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const uint32_t soff = static_cast<uint32_t>(i * 32) * g.N * 4u, up_at = soff + g.N * 2u;
-            u32x4 gate[ST::PER_PHASE], up[ST::PER_PHASE];  // on their way while the strip is written
-#pragma unroll
-            for (int k = 0; k < ST::PER_PHASE; ++k) {
-                gate[k] = __builtin_amdgcn_raw_buffer_load_b128(from, static_cast<int>(coff[k] | mask), static_cast<int>(soff), 0);
-                up[k] = __builtin_amdgcn_raw_buffer_load_b128(from, static_cast<int>(coff[k] | mask), static_cast<int>(up_at), 0);
-            }
+            if (i + AHEAD - 1 < FM) ask(i + AHEAD - 1);
             write_strip(cs, i);
             __syncthreads();
 #pragma unroll
@@ -790,13 +801,13 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float a[2], b[2];
-                    gated_grad(lo(gate[k][e]), lo(up[k][e]), lo(d[e]), a[0], b[0]);
-                    gated_grad(hi(gate[k][e]), hi(up[k][e]), hi(d[e]), a[1], b[1]);
+                    gated_grad(lo(gate[i % AHEAD][k][e]), lo(up[i % AHEAD][k][e]), lo(d[e]), a[0], b[0]);
+                    gated_grad(hi(gate[i % AHEAD][k][e]), hi(up[i % AHEAD][k][e]), hi(d[e]), a[1], b[1]);
                     dg[e] = pack_bf16(a[0], a[1]);
                     du[e] = pack_bf16(b[0], b[1]);
                 }
-                store16(dg, coff[k] | mask, to_c, soff);
-                store16(du, coff[k] | mask, to_c, up_at);
+                store16_counted(dg, coff[k] | mask, to, soff);
+                store16_counted(du, coff[k] | mask, to, up_at);
             }
             __syncthreads();
         }
