@@ -509,12 +509,24 @@ int pk_llama_loss_backward(void* h, const int* host_ids, const int* host_targets
         dev_reset_peak();
         const size_t live0 = live_variables();
         Tensor rows = Tensor::make(n, m->cfg.d, compute_dtype());
-        if (!k_begin_pass(m->gslab, st, static_cast<int*>(sent->p), 3 * n, m->embed->data, rows))
+        // The head's product writes the embedding's whole gradient before anything is added to it, so that part of the slab, its first, is not
+        // cleared before: a 32000 x 512 table's 65 MB written once and read once less (this launch 22.2 -> 15.3 us, the head's two products
+        // [32000, 512] over 4096 rows 117 -> 112.5 each).
+        const Variable& em = *m->embed;
+        const bool head_writes = fused_head && do_backward && grad_enabled() && em.requires_grad && em.is_param && em.grad.buf == m->gslab.buf &&
+                                 em.grad.off_bytes == m->gslab.off_bytes;
+        Tensor clear = m->gslab;
+        if (head_writes) {
+            const int64_t written = std::min(clear.cols, (em.data.numel() + 63) / 64 * 64);
+            clear.off_bytes += written * static_cast<int64_t>(sizeof(float));
+            clear.cols -= written;
+        }
+        if (!k_begin_pass(clear, st, static_cast<int*>(sent->p), 3 * n, m->embed->data, rows))
             k_embedding_fwd(m->embed->data, static_cast<const int*>(ids->p), rows);
         Var hid = m->hidden(ops::embedding_of(m->embed, ids, std::move(rows)), pos_dev, seq_len);
         // the loss comes back into the pinned staging's spare word; one wait behind the last kernel ends the pass
         float* hl = reinterpret_cast<float*>(st + 3 * n);
-        Var l = fused_head ? ops::linear_cross_entropy_to(hid, m->embed, tg, m->head_chunk_rows, do_backward != 0, hl)
+        Var l = fused_head ? ops::linear_cross_entropy_to(hid, m->embed, tg, m->head_chunk_rows, do_backward != 0, hl, head_writes)
                            : ops::cross_entropy(ops::matmul_nt(hid, m->embed), tg);
         hid.reset();
         // the allocator's counters move when the host allocates and frees, not when the GPU gets there: no wait here

@@ -12,9 +12,11 @@ struct ShadowCopy {
 };
 std::vector<ShadowCopy> shadow_copies();
 namespace ops {
-// ops::embedding of rows already gathered, and ops::linear_cross_entropy as the root of a pass with its value to pinned host memory as well
+// ops::embedding of rows already gathered, and ops::linear_cross_entropy as the root of a pass with its value to pinned host memory as well, which
+// writes E's gradient instead of adding to it where that has not been cleared (dE_unset)
 Var embedding_of(const Var& table, const std::shared_ptr<Buffer>& ids, Tensor rows);
-Var linear_cross_entropy_to(const Var& h, const Var& E, const std::shared_ptr<Buffer>& targets, int64_t chunk_rows, bool loss_is_root, float* pinned);
+Var linear_cross_entropy_to(const Var& h, const Var& E, const std::shared_ptr<Buffer>& targets, int64_t chunk_rows, bool loss_is_root, float* pinned,
+                            bool dE_unset = false);
 // What a rotated projection's node and the attention that alone reads it share: the attention's backward turns dQ and dK back on their way out
 // where its kernels do that, and the node then passes its gradient on as it is.
 struct Turned {

@@ -1083,7 +1083,7 @@ Var linear_cross_entropy(const Var& h, const Var& E, const std::shared_ptr<Buffe
     return linear_cross_entropy_to(h, E, targets, chunk_rows, loss_is_root, nullptr);
 }
 Var linear_cross_entropy_to(const Var& h, const Var& E, const std::shared_ptr<Buffer>& targets, int64_t chunk_rows, bool loss_is_root,
-                            float* pinned) {
+                            float* pinned, bool dE_unset) {
     const int64_t N = h->data.rows, V = E->data.rows, d = h->data.cols;
     if (d != E->data.cols) shape_fail("matmul: inner dimensions disagree");
     const int* tg = static_cast<const int*>(targets->p);
@@ -1168,7 +1168,7 @@ Var linear_cross_entropy_to(const Var& h, const Var& E, const std::shared_ptr<Bu
             gemm(dl, false, Ek, false, static_cast<char*>(dh1.ptr()) + r0 * d * hes, dh1.dtype, rows, d, d, 0.0f, dl_ld);
         }
         dl.cols = V;
-        if (want_dE) gemm(dl, true, hview, false, dE1.ptr(), PK_F32, V, d, d, r0 == 0 && !dE_in_place ? 0.0f : 1.0f, dl_ld);
+        if (want_dE) gemm(dl, true, hview, false, dE1.ptr(), PK_F32, V, d, d, r0 == 0 && (!dE_in_place || dE_unset) ? 0.0f : 1.0f, dl_ld);
     }
     Tensor out = Tensor::make(1, 1, PK_F32), one = Tensor::make(1, 1, PK_F32);  // one: backward() hands it over whole
     k_mean_f32(static_cast<const float*>(nll.p), N, out, &one, pinned);  // the loss stays on the device: no wait in mid-step

@@ -895,3 +895,36 @@ def test_bf16_rows_of_whole_lines_and_of_others(case, dk, grad):
     for r, i, g in zip(room, inside, (got[0],) + got[2:]):
         assert torch.equal(i, g)
         assert bool((r[..., :8] == 7.0).all()) and bool((r[..., -8:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("vocab,d,ff,tokens,chunk,fused", [(130, 64, 176, 64, 0, True), (37, 12, 20, 30, 7, True), (1001, 256, 700, 700, 256, True),
+                                                           (5, 8, 10, 3, 0, True), (504, 512, 1376, 4100, 0, True), (130, 64, 176, 64, 0, False)])
+def test_nothing_is_left_of_the_gradients_before(dtype, vocab, d, ff, tokens, chunk, fused):
+    """A pass on a model whose last pass left NaN in every gradient, with and without a pass forward alone between them, against the same pass
+    on a new model: the head's product writes the embedding's gradient where it is the first to, whole and beside words that no token has."""
+    toks = [synth.randint(s, tokens + 1, vocab) for s in (3, 4)]
+
+    def new():
+        m = Llama(vocab=vocab, d=d, n_layers=1, n_heads=2, d_ff=ff, compute_dtype=dtype, seed=8)
+        if chunk:
+            m.set_head_chunk(chunk)
+        return m
+
+    m, other = new(), new()
+    params = other.params()
+    other.loss_backward(toks[1][:-1], toks[1][1:], 0, fused_head=fused)
+    want = other.grads()
+    other.close()
+    for forward_between in (False, True):
+        m.set_params({k: np.full_like(v, np.nan) for k, v in params.items()})
+        m.loss_backward(toks[0][:-1], toks[0][1:], 0, fused_head=fused)
+        assert all(np.isnan(g).any() for g in m.grads().values())
+        m.set_params(params)
+        if forward_between:
+            m.loss_backward(toks[0][:-1], toks[0][1:], 0, backward=False, fused_head=fused)
+            assert all((g == 0).all() for g in m.grads().values())
+        m.loss_backward(toks[1][:-1], toks[1][1:], 0, fused_head=fused)
+        for k, g in m.grads().items():
+            assert np.array_equal(g, want[k]), k
+    m.close()
