@@ -177,3 +177,41 @@ def test_no_unspaced_register_hazard_around_asm_matrix_instructions(src, tmp_pat
     assert "v_mfma_f32_32x32x16_bf16" in text
     found = scan(str(out))
     assert not found, "\n".join(found[:20])
+
+
+def stores_overwritten(path):
+    """16-byte stores whose data a vector instruction writes less than two issue slots later. The store reads its registers after it issues, and the
+    hardware does not wait (measured, through a buffer with its scalar offset in a register: the last dword of some lanes was the next value's)."""
+    found = []
+    for kern, (ins, _) in parse(path).items():
+        for k, w in enumerate(ins):
+            if not w.op.endswith("store_dwordx4") or w.op.startswith("scratch"):
+                continue
+            ops = [x.strip() for x in w.text.partition(" ")[2].split(",")]
+            data, slots, j = _regs(ops[0] if w.op.startswith("buffer") else ops[1]), 0, k + 1
+            while j < len(ins) and slots < 2:
+                if ins[j].vw & data:
+                    found.append(f"{kern}: {w.line}: {w.text}  ->  {ins[j].line}: {ins[j].text}")
+                slots += ins[j].slots
+                j += 1
+    return found
+
+
+def test_stores_keep_their_data(tmp_path):
+    """The GEMM and the strips' users: stores from asm statements bring idle states of their own, and those the compiler places are followed by some."""
+    case, good = tmp_path / "case.s", "buffer_store_dwordx4 v[4:7], v1, s[0:3], s5 offen sc1\ns_nop 1\nv_mov_b32 v7, v2"
+    for body, bad in ((good, 0), (good.replace("s_nop 1", "s_nop 0"), 1), (good.replace("buffer_store_dwordx4 v[4:7], v1, s[0:3], s5 offen", "global_store_dwordx4 v[8:9], v[4:7], off")
+                                                                          .replace("s_nop 1\n", ""), 1)):
+        case.write_text("_Zcase:\n" + body + "\ns_endpgm\n")
+        assert len(stores_overwritten(str(case))) == bad
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not found")
+    jobs = {src: tmp_path / (src + ".s") for src in ("gemm_mfma.hip", "elementwise.hip", "attn_split.hip")}
+    running = [subprocess.Popen([hipcc, *FLAGS, os.path.join(CSRC, src), "-o", str(out)], stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+               for src, out in jobs.items()]
+    assert [p.wait() for p in running] == [0] * len(running)
+    for src, out in jobs.items():
+        assert "store_dwordx4" in out.read_text(), src
+        found = stores_overwritten(str(out))
+        assert not found, "\n".join(found[:20])
