@@ -917,9 +917,13 @@ __global__ void __launch_bounds__(EMB_NT) emb_bwd_runs(const T* dy, const int* s
 
 // The same sums without the sort, for a batch of ids that a workgroup can look through itself: block p leaves if an
 // earlier row has row p's id, and otherwise lists the later rows that have it, in ascending order (each wavefront its own
-// quarter of them), and adds them up. A sort of a few hundred ids is four launches that take 15 us on an idle chip.
+// quarter of them), and adds them up, two columns a thread, so that a long list's loads are as many in flight as the sort's kernel has. A
+// workgroup looks at all ids in front of it and behind it, four to a load; they are in the first cache after the first one.
 // Workgroups n, n + 1, ... take the held sums, `per` to each: a launch of their own is 2.5 us and what lies between two.
-constexpr int EMB_SCAN_MAX = 4096;
+// bf16 rows of 512 columns, 8192 ids of 32000, by the sort's seven launches and the held sums' own | here: 61 | 33 us; with the gather, ids drawn
+// evenly 98 | 80, by frequency (1 / rank) 213 | 107; 6000 ids 93 | 71 and 150 | 91; of 500, 128 columns 81 | 56 and 159 | 81. Up to 4096 ids, which
+// came here one at a time before: 101 -> 79 by frequency, the rest level. Work grows with the square of the ids: the line is where it was measured to.
+constexpr int EMB_SCAN_MAX = 8192;
 template <typename T>
 __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, float* dtable, int n, int d, ColSums sums, int per) {
     static_assert(NT == 256, "16 columns x 16 groups of parts");
@@ -928,43 +932,79 @@ __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, 
         const int at = blockIdx.x - n, job = at / per;
         return colsum_block<16>(sums.job[job], at - job * per, sh);
     }
-    __shared__ uint16_t rows[NT / 64][EMB_SCAN_MAX / (NT / 64) + 64];
+    __shared__ uint16_t rows[NT / 64][EMB_SCAN_MAX / (NT / 64) + 256];
     __shared__ int count[NT / 64];
-    const int p = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int id = ids[p];
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const int p = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, id = ids[p];
+    // the four ids from q on (a multiple of 4), those of [from, to) among them: a bit each where it is this one
+    const bool wide = (reinterpret_cast<uintptr_t>(ids) & 15) == 0;
+    const auto matches = [&](int q, int from, int to) -> uint32_t {
+        i32x4 v{};
+        if (wide && q + 4 <= n) {
+            v = *reinterpret_cast<const i32x4*>(ids + q);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = q + e < n ? ids[q + e] : 0;
+        }
+        uint32_t hit = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hit |= (v[e] == id && q + e >= from && q + e < to ? 1u : 0u) << e;
+        return hit;
+    };
     bool seen = false;
 #pragma unroll 4
-    for (int q = threadIdx.x; q < p; q += NT) seen = seen | (ids[q] == id);
+    for (int q = threadIdx.x * 4; q < p; q += NT * 4) seen = seen | (matches(q, 0, p) != 0);
     if (__syncthreads_or(seen)) return;
-    const int quarter = ((n - p + NT - 1) / NT) * 64;  // of the rows p .. n - 1, in whole wavefronts
-    const int lo = p + wv * quarter, hi = min(lo + quarter, n);
+    const int first = p & ~3, quarter = ((n - first + 4 * NT - 1) / (4 * NT)) * 256;  // of the rows first .. n - 1, in whole loads of a wavefront
+    const int lo = first + wv * quarter, hi = min(lo + quarter, n);
+    const uint64_t below = (uint64_t{1} << lane) - 1;
     int c = 0;
-#pragma unroll 4
-    for (int q0 = lo; q0 < hi; q0 += 64) {
-        const bool hit = q0 + lane < hi && ids[q0 + lane] == id;
-        const uint64_t m = __ballot(hit);
-        if (hit) rows[wv][c + __popcll(m & ((uint64_t{1} << lane) - 1))] = static_cast<uint16_t>(q0 + lane);
-        c += __popcll(m);
+#pragma unroll 2
+    for (int q0 = lo; q0 < hi; q0 += 256) {
+        const uint32_t hit = matches(q0 + lane * 4, p, hi);
+        int at = c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint64_t m = __ballot(hit >> e & 1);
+            at += __popcll(m & below);
+            c += __popcll(m);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (hit >> e & 1) rows[wv][at++] = static_cast<uint16_t>(q0 + lane * 4 + e);
     }
     if (lane == 0) count[wv] = c;
     __syncthreads();
-    for (int col = threadIdx.x; col < d; col += NT) {
-        float* dst = dtable + static_cast<int64_t>(id) * d + col;
-        float acc = *dst;
+    const auto add = [&](int col, auto cols) {  // the list's rows of columns col, col + NT, ...
+        constexpr int COLS = decltype(cols)::value;
+        float* const dst = dtable + static_cast<int64_t>(id) * d + col;
+        float acc[COLS];
+#pragma unroll
+        for (int k = 0; k < COLS; ++k) acc[k] = dst[k * NT];
         for (int w = 0; w < NT / 64; ++w) {
             const int end = count[w];
             int r = 0;
             for (; r + EMB_ROWS <= end; r += EMB_ROWS) {
-                float v[EMB_ROWS];
+                float v[EMB_ROWS][COLS];
 #pragma unroll
-                for (int u = 0; u < EMB_ROWS; ++u) v[u] = ldf(dy, static_cast<int64_t>(rows[w][r + u]) * d + col);
+                for (int u = 0; u < EMB_ROWS; ++u)
 #pragma unroll
-                for (int u = 0; u < EMB_ROWS; ++u) acc += v[u];
+                    for (int k = 0; k < COLS; ++k) v[u][k] = ldf(dy, static_cast<int64_t>(rows[w][r + u]) * d + col + k * NT);
+#pragma unroll
+                for (int u = 0; u < EMB_ROWS; ++u)
+#pragma unroll
+                    for (int k = 0; k < COLS; ++k) acc[k] += v[u][k];
             }
-            for (; r < end; ++r) acc += ldf(dy, static_cast<int64_t>(rows[w][r]) * d + col);
+            for (; r < end; ++r)
+#pragma unroll
+                for (int k = 0; k < COLS; ++k) acc[k] += ldf(dy, static_cast<int64_t>(rows[w][r]) * d + col + k * NT);
         }
-        *dst = acc;
-    }
+#pragma unroll
+        for (int k = 0; k < COLS; ++k) dst[k * NT] = acc[k];
+    };
+    int col = threadIdx.x;
+    for (; col + NT < d; col += 2 * NT) add(col, std::integral_constant<int, 2>{});
+    if (col < d) add(col, std::integral_constant<int, 1>{});
 }
 
 __device__ inline float block_reduce(float x, bool is_max, float* sh) {
