@@ -371,14 +371,19 @@ __device__ inline void lane_offsets_masked(uint32_t (&off)[O::PER], const uint32
         off[j] = ok ? whole[j] : OUTSIDE;
     }
 }
+template <bool SPILLED = false>
 __device__ inline void store16(u32x4 v, uint32_t off, u32x4 rsrc, uint32_t soff) {
     // invisible to the compiler's count of memory operations in flight, like the loads above; the data registers
-    // may be overwritten by the next two instructions, which a 16-byte store does not allow: two idle states
+    // may be overwritten by the next two instructions, which a 16-byte store does not allow: two idle states behind it. SPILLED: five in front of
+    // it, for scalars that a vector instruction has just written (dma_piece).
     // sc1, agent scope: an XCD's L2 passes the line on at once instead of holding it until the kernel's end, when eight L2s of 4 MB would be written
     // back while nothing multiplies. Rows leave a strip as whole lines, so nothing is written twice. 8192 x 1536 x 512 17.6 -> 15.9 us, 8192 x 512 x 512
     // 8.0 -> 7.4, 8192 x 1376 x 512 17.0 -> 15.0, fp32 results 32000 x 512 x 4096 131.9 -> 129.1 and 512 x 2752 x 8192 34.8 -> 33.6, 4096 ^ 3 103.5 ->
     // 102.3. Not nt, which keeps the last-level cache from holding the lines as well: a little more of this, and 5 to 9 % of the kernels that read them next.
-    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen sc1\n\ts_nop 1" ::"v"(v), "v"(off), "s"(rsrc), "s"(soff) : "memory");
+    if constexpr (SPILLED)
+        asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, %3 offen sc1\n\ts_nop 1" ::"v"(v), "v"(off), "s"(rsrc), "s"(soff) : "memory");
+    else
+        asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen sc1\n\ts_nop 1" ::"v"(v), "v"(off), "s"(rsrc), "s"(soff) : "memory");
 }
 // The same where the compiler counts it, between loads whose waits are not to be waits for the stores as well. The compiler leaves the idle states
 // out where the scalar offset is a register: without them the last dword of some lanes was the next value's (256 x 256 tiles).
@@ -426,6 +431,7 @@ __global__ __launch_bounds__(G::NTHR, (RingLds<G, NS>::PER_CU))
 void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     static_assert(EPI == 0 || EPI == 3 || (G::KS == 1 && !CF32), "the head's epilogues: one wavefront set, bf16 result");
     constexpr bool GROUPED = EPI == 3;
+    constexpr bool SPILLED = EPI == 1 || EPI == 2 || EPI == 4;  // 56 to 81 scalars of the head's passes lie in vector registers
     // A gated product's ends. 5, 6: B is [gate | up], N columns each; C = silu(gate) up, and (5) both of them to D, [M, 2 N]. 7: the
     // product is the gradient of C for the gate and up in D; C is [M, 2 N] and gets theirs.
     constexpr bool GATE = EPI == 5 || EPI == 6, GATE_GRAD = EPI == 7;
@@ -571,10 +577,10 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
     auto fetch_piece = [&](auto qc) {
         constexpr int Q = decltype(qc)::value;
         if constexpr (Q < OA::PER) {
-            dma_piece<Q>(f_la, f_ca ? offa_c[Q] : offa[Q], da.rsrc, f_sa);
+            dma_piece<Q, SPILLED ? 3 : 0>(f_la, f_ca ? offa_c[Q] : offa[Q], da.rsrc, f_sa);
         } else if constexpr (Q < PERTOT) {
             constexpr int J = Q - OA::PER;
-            dma_piece<J>(f_lb, f_cb ? offb_c[J] : offb[J], db.rsrc, f_sb);
+            dma_piece<J, SPILLED ? 3 : 0>(f_lb, f_cb ? offb_c[J] : offb[J], db.rsrc, f_sb);
         }
     };
     auto fetch_end = [&]() {
@@ -957,7 +963,7 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                     if (q + AHEAD < ST::NST) ask(q + AHEAD);
                     store16_counted(v, place(k), crs_c, strip_at(ph));
                 } else {
-                    store16(v, place(k), crs, strip_at(ph));
+                    store16<SPILLED>(v, place(k), crs, strip_at(ph));
                 }
             }
             __syncthreads();

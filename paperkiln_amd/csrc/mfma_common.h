@@ -304,42 +304,20 @@ constexpr uint32_t OUTSIDE = 0x80000000u, PAST_END = 0x40000000u;
 // Descriptors start this far before the tile, so that a lane offset minus the instruction's immediate (below 4096)
 // never goes negative.
 constexpr int BIAS = 4096;
-// PER consecutive 1 KB pieces of LDS from `lds_byte` on, lane offsets off[j] (already less j KB), scalar offset soff.
-// m0 is set and used inside the one statement; the compiler never keeps a value of its own in m0 across other code.
-template <int PER>
-__device__ inline void dma_group(uint32_t lds_byte, const uint32_t (&off)[PER], u32x4 rsrc, uint32_t soff) {
-    static_assert(PER == 1 || PER == 2 || PER == 4, "groups of one, two or four pieces");
-    if constexpr (PER == 1)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(off[0]),
-                     "s"(rsrc), "s"(soff)
-                     : "memory");
-    else if constexpr (PER == 2)
-        asm volatile(
-            "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-            "buffer_load_dwordx4 %1, %3, %4 offen lds\n\t"
-            "buffer_load_dwordx4 %2, %3, %4 offen offset:1024 lds" ::"s"(lds_byte),
-            "v"(off[0]), "v"(off[1]), "s"(rsrc), "s"(soff)
-            : "memory");
-    else
-        asm volatile(
-            "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-            "buffer_load_dwordx4 %1, %5, %6 offen lds\n\t"
-            "buffer_load_dwordx4 %2, %5, %6 offen offset:1024 lds\n\t"
-            "buffer_load_dwordx4 %3, %5, %6 offen offset:2048 lds\n\t"
-            "buffer_load_dwordx4 %4, %5, %6 offen offset:3072 lds" ::"s"(lds_byte),
-            "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(rsrc), "s"(soff)
-            : "memory");
-}
-// One piece of such a group on its own: the J-th 1 KB from `lds_byte` on (lane offset already less J KB), for kernels
-// that drop their loads one by one between other instructions. No "memory" clobber: the compiler may move its own LDS
-// reads across the statement (it keeps its place among the other volatile statements, the waits and barriers that
-// guard the slot it fills), which a clobber would forbid -- every piece would then fence the fragment reads of the
+// The J-th 1 KB of LDS from `lds_byte` on (lane offset already less J KB), for kernels that drop their loads one by one between other
+// instructions. m0 is set and used inside the one statement; the compiler never keeps a value of its own in m0 across other code.
+// A memory instruction sees a scalar that a vector instruction has written (the compiler brings spilled ones back that way) only five issue
+// slots later, and the compiler keeps no such distance in front of a statement. IDLE: more idle states than the one that m0 needs; with three the
+// statement stands anywhere. Kernels whose scalars are spilled take them; for the others, whose products they make 1 to 3 % longer (8192 x 512 over
+// 1536 17.35 -> 17.8 us, 4096 ^ 3 108.5 -> 109.8), the assembly is searched for such reads by a test.
+// No "memory" clobber: the compiler may move its own LDS reads across the statement (it keeps its place among the other volatile statements, the
+// waits and barriers that guard the slot it fills), which a clobber would forbid -- every piece would then fence the fragment reads of the
 // chunk after it from the matrix instructions of the chunk before.
-template <int J>
+template <int J, int IDLE = 0>
 __device__ inline void dma_piece(uint32_t lds_byte, uint32_t off, u32x4 rsrc, uint32_t soff) {
     static_assert(J >= 0 && J < 4, "immediate offsets below 4096");
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen offset:%4 lds" ::"s"(lds_byte), "v"(off),
-                 "s"(rsrc), "s"(soff), "n"(J * 1024));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop %5\n\tbuffer_load_dwordx4 %1, %2, %3 offen offset:%4 lds" ::"s"(lds_byte), "v"(off),
+                 "s"(rsrc), "s"(soff), "n"(J * 1024), "n"(IDLE));
 }
 // f(integral_constant B), ..., f(integral_constant E - 1)
 template <int B, int E, typename F>

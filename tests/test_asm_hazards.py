@@ -10,12 +10,15 @@ them and the vector instructions around them. Two of those distances are not enf
     a register that a matrix instruction wrote less than its pass count + 3 issue slots earlier (8 passes for v_mfma_f32_32x32x16_bf16) sees the old contents. A
     matrix instruction in between counts as 8 slots: it cannot enter the pipe before the writer has left it.
 
+  * a memory instruction that reads, as its descriptor, offset or base, a scalar register which a vector instruction (the lane read that brings
+    a spilled scalar back) wrote less than 5 issue slots earlier sees the old contents; of memory instructions in asm statements;
+
   * a vector instruction that WRITES a register which a matrix instruction issued less than 11 slots earlier is still
     going to write (write after write), or which a matrix instruction issued less than 7 slots earlier still reads as
     its C operand from ordinary registers (write after read: the 8-pass instruction reads C over its passes), would
     corrupt that instruction's result or input.
 
-This test compiles the two kernels to assembly and checks these distances on every path of the control-flow graph
+These tests compile the kernels to assembly and check these distances on every path of the control-flow graph
 that the assembler text shows: fall-through over labels, taken branches and loop back-edges (the tail of a loop body
 is followed by its head)."""
 import os
@@ -33,7 +36,9 @@ RAW_VALU_TO_MFMA = 2    # idle or unrelated issue slots wanted between a vector 
 RAW_MFMA_TO_OTHER = 11  # 8 passes + 3
 WAW_MFMA_TO_VALU = 11   # a vector write to a register a matrix instruction is still going to write
 WAR_SRCC_TO_VALU = 7    # a vector write to a register a matrix instruction still reads as its C operand
+VALU_SGPR_TO_VMEM = 5   # a vector write of a scalar register and the memory instruction that reads it
 MFMA_SLOTS = 8          # a matrix instruction in between enters the pipe only when the one before it has left it
+ASM_MEMORY = ["gemm_mfma.hip", "elementwise.hip", "attn_split.hip", "attn_fwd_mfma.hip", "attn_bwd_mfma.hip", "attn_bwd_dkdv2.hip", "attn_bwd_dkdv3.hip", "attn_bwd_dq3.hip"]
 HORIZON = max(RAW_MFMA_TO_OTHER, WAW_MFMA_TO_VALU, WAR_SRCC_TO_VALU, RAW_VALU_TO_MFMA)
 
 
@@ -197,21 +202,83 @@ def stores_overwritten(path):
     return found
 
 
-def test_stores_keep_their_data(tmp_path):
-    """The GEMM and the strips' users: stores from asm statements bring idle states of their own, and those the compiler places are followed by some."""
+@pytest.fixture(scope="module")
+def assembly(tmp_path_factory):
+    """{source: its assembly} of every source with memory instructions in asm statements"""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not found")
+    out = tmp_path_factory.mktemp("asm")
+    jobs = {src: str(out / (src + ".s")) for src in ASM_MEMORY}
+    running = [subprocess.Popen([hipcc, *FLAGS, os.path.join(CSRC, src), "-o", to], stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+               for src, to in jobs.items()]
+    assert [p.wait() for p in running] == [0] * len(running)
+    return jobs
+
+
+def test_stores_keep_their_data(tmp_path, assembly):
+    """Stores from asm statements bring idle states of their own, and those the compiler places are followed by some."""
     case, good = tmp_path / "case.s", "buffer_store_dwordx4 v[4:7], v1, s[0:3], s5 offen sc1\ns_nop 1\nv_mov_b32 v7, v2"
     for body, bad in ((good, 0), (good.replace("s_nop 1", "s_nop 0"), 1), (good.replace("buffer_store_dwordx4 v[4:7], v1, s[0:3], s5 offen", "global_store_dwordx4 v[8:9], v[4:7], off")
                                                                           .replace("s_nop 1\n", ""), 1)):
         case.write_text("_Zcase:\n" + body + "\ns_endpgm\n")
         assert len(stores_overwritten(str(case))) == bad
-    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    if not os.path.exists(hipcc):
-        pytest.skip("hipcc not found")
-    jobs = {src: tmp_path / (src + ".s") for src in ("gemm_mfma.hip", "elementwise.hip", "attn_split.hip")}
-    running = [subprocess.Popen([hipcc, *FLAGS, os.path.join(CSRC, src), "-o", str(out)], stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
-               for src, out in jobs.items()]
-    assert [p.wait() for p in running] == [0] * len(running)
-    for src, out in jobs.items():
-        assert "store_dwordx4" in out.read_text(), src
-        found = stores_overwritten(str(out))
+    for src, out in assembly.items():
+        assert "store_dwordx4" in open(out).read(), src
+        found = stores_overwritten(out)
+        assert not found, "\n".join(found[:20])
+
+
+def _scalars(tok):
+    """scalar registers named by an operand"""
+    regs = set()
+    for lo, hi, one in re.findall(r"(?<![\w.\[])s(?:\[(\d+):(\d+)\]|(\d+)(?!\w))", tok):
+        regs |= set(range(int(lo), int(hi) + 1)) if lo else {int(one)}
+    return regs
+
+
+def scalars_read_early(path):
+    """Memory instructions that read a scalar register less than five issue slots after a vector instruction (a lane read back from where it was
+    spilled, say) has written it: they see what it held before. The compiler keeps the distance for its own instructions, not for those in
+    asm statements. A scalar instruction's write in between counts instead."""
+    found = []
+    for kern, (ins, labels) in parse(path).items():
+        preds, by_vector, by_scalar = [[] for _ in ins], [], []
+        for j, i in enumerate(ins):
+            if i.falls_through and j + 1 < len(ins):
+                preds[j + 1].append(j)
+            if i.target in labels and labels[i.target] < len(ins):
+                preds[labels[i.target]].append(j)
+            ops = i.text.partition(" ")[2].split(",")
+            second = re.match(r"v_(add|sub|subrev|addc|subb|subbrev)_co|v_div_scale|v_mad_[iu]64", i.op)
+            wrote = _scalars(ops[0]) | (_scalars(ops[1]) if second else set())
+            by_vector.append(wrote if i.op.startswith("v_") else set())
+            by_scalar.append(wrote if i.op.startswith("s_") else set())
+        for k, r in enumerate(ins):
+            if not r.op.startswith(("buffer_", "global_", "scratch_", "flat_")):
+                continue
+            stack, seen = [(j, 0, frozenset(_scalars(r.text.partition(" ")[2]))) for j in preds[k]], set()
+            while stack:
+                j, dist, regs = stack.pop()
+                if dist >= VALU_SGPR_TO_VMEM or not regs or (j, dist, regs) in seen:
+                    continue
+                seen.add((j, dist, regs))
+                if by_vector[j] & regs:
+                    found.append(f"{kern}: {ins[j].line}: {ins[j].text}  ->  {r.line}: {r.text}  (distance {dist})")
+                regs = regs - by_vector[j] - by_scalar[j]
+                stack.extend((jj, dist + ins[j].slots, regs) for jj in preds[j])
+    return found
+
+
+def test_memory_instructions_see_their_scalars(tmp_path, assembly):
+    case = tmp_path / "case.s"
+    load = "s_mov_b32 m0, s0\ns_nop 0\nbuffer_load_dwordx4 v1, s[4:7], s98 offen lds"
+    for body, bad in (("v_readlane_b32 s7, v162, 9\n" + load, 1), ("v_readlane_b32 s98, v162, 9\n" + load, 1), ("v_readlane_b32 s8, v162, 9\n" + load, 0),
+                      ("v_readlane_b32 s7, v162, 9\n" + load.replace("s_nop 0", "s_nop 3"), 0), ("v_readlane_b32 s7, v162, 9\n" + load.replace("s_nop 0", "s_nop 2"), 1),
+                      ("v_readlane_b32 s7, v162, 9\ns_mov_b32 s7, s9\n" + load, 0), ("v_sub_co_u32_e64 v8, s[98:99], s85, 1\n" + load, 1),
+                      (f".LBB0_1:\n{load}\nv_readlane_b32 s4, v162, 9\ns_cbranch_scc1 .LBB0_1", 1)):
+        case.write_text("_Zcase:\n" + body + "\ns_endpgm\n")
+        assert len(scalars_read_early(str(case))) == bad, body
+    for src, out in assembly.items():
+        found = scalars_read_early(out)
         assert not found, "\n".join(found[:20])

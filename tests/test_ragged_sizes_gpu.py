@@ -37,10 +37,11 @@ def test_bf16_training_on_a_ragged_token_count(tokens, seq):
 
 
 @pytest.mark.parametrize("vocab,d,ff,layers,tokens,seq", [(301, 64, 176, 2, 77, 11), (1001, 128, 344, 1, 693, 77),
-                                                          (12345, 256, 688, 1, 2600, 650), (17, 64, 176, 1, 64, 0)])
+                                                          (12345, 256, 688, 1, 2600, 650), (17, 64, 176, 1, 64, 0),
+                                                          (3122, 512, 1368, 1, 2924, 34), (20001, 512, 1368, 1, 4100, 820)])
 def test_bf16_training_with_any_vocabulary(vocab, d, ff, layers, tokens, seq):
     """The tied head's cross-entropy inside its product, with a vocabulary padded to a multiple of 8 (small and large
-    tiles), and the weight gradients of few tokens in one launch. Against the library GEMM, same operands."""
+    tiles, several rounds of each), and the weight gradients of few tokens in one launch. Against the library GEMM, same operands."""
     m = Llama(vocab=vocab, d=d, n_layers=layers, n_heads=d // 32, d_ff=ff, compute_dtype="bf16", seed=8)
     toks = synth.randint(3, tokens + 1, vocab)
     toks[:4] = vocab - 1  # the last word is used, as input and as target
