@@ -921,8 +921,12 @@ __global__ void __launch_bounds__(EMB_NT) emb_bwd_runs(const T* dy, const int* s
 // workgroup looks at all ids in front of it and behind it, four to a load; they are in the first cache after the first one.
 // Workgroups n, n + 1, ... take the held sums, `per` to each: a launch of their own is 2.5 us and what lies between two.
 // bf16 rows of 512 columns, 8192 ids of 32000, by the sort's seven launches and the held sums' own | here: 61 | 33 us; with the gather, ids drawn
-// evenly 98 | 80, by frequency (1 / rank) 213 | 107; 6000 ids 93 | 71 and 150 | 91; of 500, 128 columns 81 | 56 and 159 | 81. Up to 4096 ids, which
-// came here one at a time before: 101 -> 79 by frequency, the rest level. Work grows with the square of the ids: the line is where it was measured to.
+// evenly 98 | 80, by frequency (1 / rank) 213 | 107; 6000 ids 93 | 71 and 150 | 91; of 500, 128 columns 81 | 56 and 159 | 81.
+// Where it is the sort's turn (bf16, ids of 32000 drawn evenly, by frequency, half of them one, all of them one; us, sort | here):
+//   ids      work grows with their square: 8192, 64 columns 31 102 442 860 | 25 29 125 244, 512 columns 46 147 642 1516 | 27 34 241 428; 12288, 64 columns
+//            34 137 638 1260 | 61 44 184 365, 512 columns 55 211 992 2138 | 65 64 358 634, where ids drawn evenly are behind.
+//   columns  512 at a time, one after the other, of an id that the sort deals to d / 64 workgroups: 4097 ids, 512 columns 36 76 241 451 | 13 21 83 175, 1024 columns 45 78 238 449
+//            | 14 40 235 474, 1025 columns 48 87 279 450 | 21 60 299 642, 2048 columns 60 101 284 447 | 18 109 464 938. Up to 4096 ids all widths came here before as well.
 constexpr int EMB_SCAN_MAX = 8192;
 template <typename T>
 __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, float* dtable, int n, int d, ColSums sums, int per) {
@@ -936,15 +940,15 @@ __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, 
     __shared__ int count[NT / 64];
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     const int p = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, id = ids[p];
-    // the four ids from q on (a multiple of 4), those of [from, to) among them: a bit each where it is this one
     const bool wide = (reinterpret_cast<uintptr_t>(ids) & 15) == 0;
+    // of the four ids from q on (a multiple of 4; a wavefront's are neighbours), those of [from, to): a bit each where it is this one
     const auto matches = [&](int q, int from, int to) -> uint32_t {
-        i32x4 v{};
-        if (wide && q + 4 <= n) {
+        i32x4 v;
+        if (wide && __builtin_amdgcn_readfirstlane(q - lane * 4) + 256 <= n) {
             v = *reinterpret_cast<const i32x4*>(ids + q);
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = q + e < n ? ids[q + e] : 0;
+            for (int e = 0; e < 4; ++e) v[e] = ids[min(q + e, n - 1)];
         }
         uint32_t hit = 0;
 #pragma unroll
@@ -975,6 +979,7 @@ __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, 
     }
     if (lane == 0) count[wv] = c;
     __syncthreads();
+    const uint32_t pitch = d;  // (of a signed number a row's address is twice the scalar instructions, a tenth of a long list's time)
     const auto add = [&](int col, auto cols) {  // the list's rows of columns col, col + NT, ...
         constexpr int COLS = decltype(cols)::value;
         float* const dst = dtable + static_cast<int64_t>(id) * d + col;
@@ -989,7 +994,7 @@ __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, 
 #pragma unroll
                 for (int u = 0; u < EMB_ROWS; ++u)
 #pragma unroll
-                    for (int k = 0; k < COLS; ++k) v[u][k] = ldf(dy, static_cast<int64_t>(rows[w][r + u]) * d + col + k * NT);
+                    for (int k = 0; k < COLS; ++k) v[u][k] = ldf(dy, static_cast<int64_t>(uint64_t{rows[w][r + u]} * pitch) + col + k * NT);
 #pragma unroll
                 for (int u = 0; u < EMB_ROWS; ++u)
 #pragma unroll
@@ -997,7 +1002,7 @@ __global__ void __launch_bounds__(NT) emb_bwd_scan(const T* dy, const int* ids, 
             }
             for (; r < end; ++r)
 #pragma unroll
-                for (int k = 0; k < COLS; ++k) acc[k] += ldf(dy, static_cast<int64_t>(rows[w][r]) * d + col + k * NT);
+                for (int k = 0; k < COLS; ++k) acc[k] += ldf(dy, static_cast<int64_t>(uint64_t{rows[w][r]} * pitch) + col + k * NT);
         }
 #pragma unroll
         for (int k = 0; k < COLS; ++k) dst[k * NT] = acc[k];
@@ -1692,11 +1697,12 @@ void k_embedding_fwd(const Tensor& table, const int* ids, const Tensor& y) {
                                                 y.rows, static_cast<int>(y.cols)));
     post();
 }
+extern "C" int pk_embedding_scans(int64_t n, int64_t d) { return n <= 4096 || (n <= EMB_SCAN_MAX && d <= 1024); }
 bool k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable, const HeldSum* held, int count) {
     if (dy.rows > (1 << 30)) shape_fail("embedding: more than 2^30 rows");
     const int n = static_cast<int>(dy.rows), d = static_cast<int>(dy.cols);
     const hipStream_t st = tape_stream();
-    if (n <= EMB_SCAN_MAX) {
+    if (pk_embedding_scans(n, d)) {
         ColSums sums{};
         int per = 1;
         const bool with = held && count <= ColSums::MAX;

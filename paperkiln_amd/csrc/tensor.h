@@ -61,6 +61,8 @@ struct Turn {
 void k_embedding_fwd(const Tensor& table_f32, const int* ids, const Tensor& y);       // ops.cpp:329-337
 // scatter-add, ops.cpp:338-347; held sums (no two with the same dw) may ride along: true if they did
 bool k_embedding_bwd(const Tensor& dy, const int* ids, const Tensor& dtable_f32, const HeldSum* held = nullptr, int count = 0);
+// Whether n rows of d columns go without the sort, by workgroups that look through all ids. For tests.
+extern "C" int pk_embedding_scans(int64_t n, int64_t d);
 // Row-wise softmax cross-entropy on a block of logits (ops.cpp:350-376): writes
 // dlogits = (P - onehot) * gscale in place and the per-row nll (fp32) with the
 // reference's max(p, 1e-12) clamp.

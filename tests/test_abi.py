@@ -169,3 +169,10 @@ F32_LAUNCHES = [
 def test_which_launches_a_whole_backward_takes(dtype, form, shape):
     """dQ and dK/dV go into one launch where that is ahead of two, or of the blocks of 32 rows that share one as well."""
     assert BWD_FORMS[_lib.lib().pk_bwd_of_shape(ctypes.byref(_lib.AttnShape(*shape, 1.0, dtype, dtype)))] == form
+
+
+@pytest.mark.parametrize("n,d,scans", [(1, 64, 1), (4096, 1024, 1), (4096, 4096, 1), (4097, 512, 1), (4097, 1024, 1), (4097, 1025, 0), (8192, 512, 1), (8192, 1024, 1),
+                                       (8192, 2048, 0), (8193, 64, 0), (1 << 20, 512, 0)])
+def test_which_embedding_gradients_go_without_the_sort(n, d, scans):
+    """Workgroups that look through all ids and take a row's columns 512 at a time: as far as they are ahead of the sort, in ids and in columns."""
+    assert _lib.lib().pk_embedding_scans(ctypes.c_int64(n), ctypes.c_int64(d)) == scans

@@ -931,10 +931,11 @@ def test_nothing_is_left_of_the_gradients_before(dtype, vocab, d, ff, tokens, ch
     m.close()
 
 
-@pytest.mark.parametrize("n,vocab,d", [(1, 3, 5), (3, 1, 700), (1023, 40, 33), (4097, 5000, 64), (8191, 32000, 513), (8192, 7, 130), (8192, 1, 1025), (8193, 300, 64)])
+@pytest.mark.parametrize("n,vocab,d", [(1, 3, 5), (3, 1, 700), (1023, 40, 33), (4097, 5000, 64), (8191, 32000, 513), (8192, 7, 130), (8192, 1, 1025), (8193, 300, 64),
+                                       (4097, 3, 1024), (4097, 2, 1025), (4095, 3, 1300), (8190, 4, 1024), (257, 40, 700)])
 def test_embedding_gradient_of_ids_looked_through(n, vocab, d):
     """Up to 8192 ids are looked through by every workgroup, four to a load: counts that are no multiple of four, one beside the sort's, ids that all
-    rows share or none, columns short of one and of two a thread, and ids that do not begin on 16 bytes. A row's sum is formed in row order: the bits
+    rows share or none, columns short of one and of two a thread and beside the sort's, and ids that do not begin on 16 bytes. A row's sum is formed in row order: the bits
     of the same additions one after the other."""
     rng = np.random.RandomState(n + d)
     ids, dy = rng.randint(0, vocab, n).astype(np.int32), rng.randn(n, d).astype(np.float32)
