@@ -490,6 +490,8 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
         for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
             for (int db = 0; db < DB; ++db) asm volatile("" : "+a"(acc[qb][db]));
+        int at = lane;  // places in a strip are formed here and not kept over the passes: there are no registers for them
+        if constexpr (!GF32) asm volatile("" : "+v"(at));
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
             const int q1 = qw + qb * 32, qi = q1 + c32;
@@ -498,8 +500,8 @@ __global__ __launch_bounds__(256, 1) void mfma_dq3(AttnArgs a) {
                 static_assert(4 * Rows::ELEMS <= RING * BN * S, "the wavefronts' strips");
                 uint16_t* const strip = Kt[0] + w * Rows::ELEMS;
 #pragma unroll
-                for (int db = 0; db < DB; ++db) store_acc_bf16<D>(Rows::row(strip, c32), db, g, acc[qb][db], a.scale);
-                Rows::out(strip, static_cast<uint16_t*>(a.dq) + b * a.dq_sb + h * a.dq_sh + q1 * a.dq_st, a.dq_st, 0, a.T - q1, lane);
+                for (int db = 0; db < DB; ++db) store_acc_bf16<D>(Rows::row(strip, at & 31), db, at >> 5, acc[qb][db], a.scale);
+                Rows::out(strip, static_cast<uint16_t*>(a.dq) + b * a.dq_sb + h * a.dq_sh + q1 * a.dq_st, a.dq_st, 0, a.T - q1, at);
                 continue;
             }
             if (qi >= a.T) continue;

@@ -1071,6 +1071,9 @@ void gemm_ring(GemmArgs g, HeadArgs hd, GroupArgs gr) {
                         store_result(cb);
                     since_store = 0;
                 }
+                // the next slice's first fragments once more, not kept over the end of a tile whose gate and up take their registers
+                if constexpr (GATE_GRAD && BM > 128)
+                    static_for<0, NF>([&](auto fc) { read_frag(fc, std::integral_constant<int, 0>{}, lds + (u + 1) % NS * SLOT); });
                 cv = next_block(cv + stride, cb);
                 if (cv >= V) {
                     done = true;
