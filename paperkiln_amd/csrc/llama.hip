@@ -180,6 +180,8 @@ struct Model {
         const int dk = cfg.d / cfg.n_heads;
         auto table = std::make_shared<Buffer>(sizeof(float) * seq_len * std::max(dk / 2 * 2, 2));
         k_rope_table(cfg.rope_theta, dk, seq_len, static_cast<float*>(table->p));
+        // Waited for, once per growth: a pass that fails behind this one leaves the table to the next, which may be on another stream.
+        hip_check(hipStreamSynchronize(tape_stream()), "hipStreamSynchronize");
         turns = std::move(table);
         turned_positions = seq_len;
     }

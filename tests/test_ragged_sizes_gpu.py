@@ -136,6 +136,22 @@ def test_rope_undone_in_attention_backward(dtype, d, heads, tokens, seq, all_hea
 
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_rope_table_of_passes_on_several_streams(dtype):
+    """The table of cosines and sines grows with the longest sequence yet, on whichever stream that pass runs, and serves shorter ones behind it on others: the
+    bits of models that have had no other pass."""
+    cfg = dict(vocab=130, d=64, n_layers=1, n_heads=2, d_ff=128, compute_dtype=dtype, rope_all_heads=True, seed=8)
+    toks = synth.randint(3, 321, 130)
+    m, streams = Llama(**cfg), [torch.cuda.Stream() for _ in range(3)]
+    for i, seq in enumerate((16, 64, 32, 320, 160, 80)):
+        got = m.loss_backward(toks[:320], toks[1:], seq, stream=streams[i % 3].cuda_stream)[0], m.grads()
+        fresh = Llama(**cfg)
+        assert fresh.loss_backward(toks[:320], toks[1:], seq)[0] == got[0]
+        assert all(np.array_equal(g, got[1][k]) for k, g in fresh.grads().items())
+        fresh.close()
+    m.close()
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("vocab,d,ff,layers", [(130, 64, 176, 8), (37, 12, 20, 1), (37, 6, 10, 1)])
 def test_optimiser_step_writes_the_copies(vocab, d, ff, layers, dtype):
     """AdamW with the products' copies of the parameters written in the same pass: more parameters than one launch takes, sizes
