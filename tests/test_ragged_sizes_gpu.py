@@ -135,6 +135,56 @@ def test_rope_undone_in_attention_backward(dtype, d, heads, tokens, seq, all_hea
     assert rel(got[1][1], got[0][1]) < (1e-5 if dtype == "fp32" else 4 * 2.0 ** -9)
 
 
+def exact_block_model(params, toks, seq, heads, rot_heads, window):
+    """Loss and gradients in float64 of a Llama of one block (llama.cpp:25-89) whose attention sees the last `window` keys."""
+    P = {k: torch.from_numpy(v).cuda().double().requires_grad_() for k, v in params.items()}
+    W = {k.split(".")[-2]: v for k, v in P.items()}
+    x, y = (torch.from_numpy(t.astype(np.int64)).cuda() for t in (toks[:-1], toks[1:]))
+    E = W["embed_tokens"]
+    n, d = len(x), E.shape[1]
+    dk = d // heads
+    norm = lambda t, w: t * w.reshape(1, -1) / torch.sqrt((t * t).mean(1, keepdim=True) + 1e-5)  # noqa: E731
+    angle = (torch.arange(n, device="cuda") % seq)[:, None] / 10000.0 ** (torch.arange(0, dk, 2, device="cuda").double() / dk)
+    c, s = torch.cos(angle)[:, None], torch.sin(angle)[:, None]
+
+    def turn(t):  # [n, heads, dk], the first rot_heads of them
+        a, b = t[:, :rot_heads, 0::2], t[:, :rot_heads, 1::2]
+        return torch.cat([torch.stack([a * c - b * s, a * s + b * c], -1).reshape(n, rot_heads, dk), t[:, rot_heads:]], 1)
+
+    h = E[x]
+    u = norm(h, W["input_layernorm"])
+    q, k, v = ((u @ W[w]).reshape(n, heads, dk) for w in ("q_proj", "k_proj", "v_proj"))
+    q, k, v = (t.reshape(-1, seq, heads, dk).transpose(1, 2).contiguous() for t in (turn(q), turn(k), v))
+    i, j = torch.arange(seq, device="cuda")[:, None], torch.arange(seq, device="cuda")[None, :]
+    scores = (q @ k.transpose(2, 3).contiguous() / dk ** 0.5).masked_fill((j > i) | (j + window <= i), float("-inf"))
+    h = h + (torch.softmax(scores, -1) @ v).transpose(1, 2).reshape(n, d) @ W["o_proj"]
+    u = norm(h, W["post_attention_layernorm"])
+    h = h + (torch.nn.functional.silu(u @ W["gate_proj"]) * (u @ W["up_proj"])) @ W["down_proj"]
+    loss = torch.nn.functional.cross_entropy(norm(h, W["norm"]) @ E.T, y)
+    loss.backward()
+    return float(loss), {k: t.grad.cpu().numpy() for k, t in P.items()}
+
+
+@pytest.mark.parametrize("all_heads", [False, True])
+@pytest.mark.parametrize("dtype,d,heads,tokens,seq,window,form", [
+    ("fp32", 64, 2, 33, 11, 4, "F32_SPLIT"), ("fp32", 96, 1, 700, 350, 64, "F32_SPLIT"), ("fp32", 256, 2, 1538, 769, 200, "F32_PARTS_ALL"),
+    ("fp32", 512, 8, 4084, 1021, 128, "F32_PARTS"), ("bf16", 64, 2, 33, 11, 4, "SPLIT"), ("bf16", 80, 1, 70, 35, 9, "SPLIT"),
+    ("bf16", 128, 2, 2000, 250, 30, "SPLIT"), ("bf16", 256, 2, 1538, 769, 200, "SPLIT"), ("bf16", 512, 8, 4084, 1021, 128, "SPLIT_JOINED"),
+    ("bf16", 768, 8, 4000, 500, 100, "SPLIT_JOINED")])
+def test_rope_undone_under_a_band(dtype, d, heads, tokens, seq, window, form, all_heads):
+    """dQ and dK turned back where the attention kernels write them, under a band without sinks, against float64. bf16: some twenty tensors of a pass are
+    rounded, each by 2 ^ -9 of a norm at most; fp32: a chain of sums of up to 4084 terms, sqrt(4084) 2 ^ -24 = 4e-6 each."""
+    assert bwd_form((tokens // seq, seq, heads, heads, 1, window, 0), d // heads, torch.float32 if dtype == "fp32" else torch.bfloat16) == form
+    m = Llama(vocab=130, d=d, n_layers=1, n_heads=heads, d_ff=2 * d, compute_dtype=dtype, rope_all_heads=all_heads, window=window, seed=8)
+    toks = synth.randint(3, tokens + 1, 130)
+    loss, _ = m.loss_backward(toks[:-1], toks[1:], seq)
+    want_loss, want = exact_block_model(m.params(), toks, seq, heads, heads if all_heads else 1, window)
+    assert abs(loss - want_loss) < (1e-5 if dtype == "fp32" else 1e-3)
+    got = m.grads()
+    assert rel(got, {k: g.reshape(got[k].shape) for k, g in want.items()}) < (2e-5 if dtype == "fp32" else 20 * 2.0 ** -9)
+    m.close()
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 def test_rope_table_of_passes_on_several_streams(dtype):
     """The table of cosines and sines grows with the longest sequence yet, on whichever stream that pass runs, and serves shorter ones behind it on others: the
