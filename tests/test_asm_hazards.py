@@ -282,3 +282,12 @@ def test_memory_instructions_see_their_scalars(tmp_path, assembly):
     for src, out in assembly.items():
         found = scalars_read_early(out)
         assert not found, "\n".join(found[:20])
+
+
+@pytest.mark.parametrize("src,kernel,most", [("gemm_mfma.hip", "gemm_ring", 1), ("attn_bwd_dq3.hip", "mfma_dq3", 11), ("attn_bwd_dkdv3.hip", "mfma_dkdv3", 0),
+                                             ("attn_bwd_dkdv2.hip", "mfma_dkdv2", 0), ("attn_fwd_mfma.hip", "mfma_fwd", 0)])
+def test_loops_keep_their_vector_registers(assembly, src, kernel, most):
+    """Loops whose loads in flight are counted by hand: a spilled register's load is one more to wait for, between the matrix instructions. Forms of a
+    kernel that have some spill no more than the fp32 gradients' dQ does beside its loop (11), a 256 x 256 product of two transposed operands one."""
+    spilled = {n: int(c) for n, c in re.findall(r"\.name: +(_Z\w+)\n(?:(?!\.name: +_Z)[^\n]*\n)*? +\.vgpr_spill_count: +(\d+)", open(assembly[src]).read()) if kernel in n}
+    assert spilled and max(spilled.values()) <= most, {n: c for n, c in spilled.items() if c > most}
